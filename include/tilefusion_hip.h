@@ -111,6 +111,9 @@ uint64_t tf_pattern_hash(int M, const int *Ap, const int *Ai);
 /* A wrapped matrix has no host arrays to fingerprint, so its pattern is not checked unless the
  * caller, who knows the host copy, provides the fingerprint here (0 = unknown again). */
 tf_status tf_csr_set_pattern_hash(tf_csr *a, uint64_t hash);
+/* The owner of a wrapped matrix promises not to change its arrays any more: executors then keep what they derive from its
+ * values (the rows in a schedule's order) from call to call, as they do for an uploaded matrix. */
+tf_status tf_csr_set_constant(tf_csr *a);
 void tf_csr_free(tf_csr *a);
 
 tf_status tf_dense_upload(int M, int N, const float *host, tf_dense **out);
@@ -279,6 +282,8 @@ typedef struct {
      read most -- the rows of the hot partitions first, then by falling number of reads -- instead of at their own
      index.  Invisible to the caller (results identical); 0 = do so, -1 = rows at their own index. */
   int place_intermediate;
+  /* tf_pattern_hash(L, Ap, Ai), for a caller that has it already; 0 = computed (a pass over the pattern). */
+  uint64_t pattern_hash;
 } tf_inspect_opts;
 
 typedef struct tf_schedule tf_schedule;
@@ -293,6 +298,9 @@ typedef struct tf_schedule tf_schedule;
  * unfused remainder), re-derived for one workgroup's LDS instead of a CPU cache. */
 tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *opts,
                      tf_schedule **out);
+/* A schedule for one product Y = A * X with up to N columns (tf_spmm_scheduled): every row in the remainder lists.
+ * pattern_hash as in tf_inspect_opts. */
+tf_status tf_inspect_spmm(int L, int M, const int *Ap, const int *Ai, int N, uint64_t pattern_hash, tf_schedule **out);
 void tf_schedule_free(tf_schedule *s);
 
 typedef struct {
@@ -407,10 +415,12 @@ enum {
                            another -- which measured as fast on the R-MAT configuration (2.32 ms
                            against 2.35 ms: the gathers and the GEMM's operand traffic meet in the
                            same memory system), so it is not the default */
-  TF_RELU = 4u,          /* tf_gcn_two_layers: ReLU between the layers */
-  TF_FUSE_LAYERS = 8u    /* tf_gcn_two_layers: run the second schedule's two-layer tiles (one launch, the hidden
+  TF_RELU = 4u,          /* tf_gcn_two_layers: ReLU between the layers; tf_gemm_spmm, tf_spmm_scheduled: ReLU of the result */
+  TF_FUSE_LAYERS = 8u,   /* tf_gcn_two_layers: run the second schedule's two-layer tiles (one launch, the hidden
                            layer never leaves LDS), or fail with TF_EUNSUPPORTED if it has none; without this flag
                            each layer is one tf_gemm_spmm (see tf_gcn_two_layers)                            */
+  TF_C_TRANSPOSED = 16u  /* tf_gemm_spmm, tf_gcn_two_layers, tf_gemm_ex: the weights are stored outputs x inputs (N x K), as
+                           torch stores a layer's                                                            */
 };
 
 /* D = A * (B * C), A and B sparse.  Stands in for
@@ -458,13 +468,19 @@ tf_status tf_gcn_two_layers(const tf_csr *A, const tf_dense *X, const tf_dense *
 /* Unfused building blocks, the reference's in-process baselines:
  * Y = A * X   (swiftware::sparse::spmmCsrParallel<float>, fusion/src/SpMM_SpMM.cpp:37-55) */
 tf_status tf_spmm(const tf_csr *A, const tf_dense *X, tf_dense *Y, unsigned flags, void *stream);
-/* Y = X * W   (the cblas_sgemm call at fusion/gcn/GCN_Layer_MKL_Forward_Utils.h:1144).
- * K % 8 == 0, N % 32 == 0 and N <= 256 go straight to the MFMA kernel; any other shape is padded / cut into column
- * panels in a workspace the library keeps per device.  The workspace only grows: a call whose buffers fit is
- * asynchronous on `stream` like every other; the first call with a larger shape frees and allocates (which waits for
- * the device, and is refused with TF_EUNSUPPORTED while `stream` is being captured).  Calls with such shapes on one
- * device share that workspace: keep them on one stream, or order them with events. */
+/* The same with a schedule of tf_inspect_spmm on A's pattern, for this N or more: rows are dealt out by length, long rows cut
+ * among workgroups, so that a graph with hub rows does not wait for the one lane group that has the longest (R-MAT, 2^17
+ * nodes, N = 64: 1.23 ms without, 0.06 ms with).  Asynchronous on `stream`, one call at a time per schedule. */
+tf_status tf_spmm_scheduled(const tf_csr *A, const tf_dense *X, tf_dense *Y, tf_schedule *schedule, unsigned flags, void *stream);
+/* Y = X * W   (the cblas_sgemm call at fusion/gcn/GCN_Layer_MKL_Forward_Utils.h:1144), any shape. */
 tf_status tf_gemm(const tf_dense *X, const tf_dense *W, tf_dense *Y, void *stream);
+/* The same with W stored N x K (TF_C_TRANSPOSED), and with Y = 0 wherever `mask` (of Y's shape, may be null) is zero
+ * or less: the step back through a ReLU whose output is `mask`. */
+tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *Y, const tf_dense *mask, unsigned flags, void *stream);
+/* Y (N x K) = G^T * X with G M x N and X M x K: the gradient of a layer's weights.  `workspace`: device memory of
+ * tf_weight_grad_workspace(M, N, K) bytes, in use until the call's work on `stream` is done. */
+tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream);
+size_t tf_weight_grad_workspace(int M, int N, int K);
 
 /* D = A * (B * C), A and B sparse, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the

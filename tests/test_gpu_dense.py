@@ -1,0 +1,121 @@
+"""The dense products beside the executors (Y = X W in any shape and storage of W, the gradient of a layer's weights) and the
+scheduled row product, at the sizes where their kernels change hands or have remainders, against float64."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+pytestmark = pytest.mark.gpu
+RELU, C_TRANSPOSED = 4, 16
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def rel(got, want):
+    return float(np.abs(got - want).max() / max(np.abs(want).max(), 1e-30))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (15, 16, 3), (17, 33, 16), (64, 500, 32), (3000, 500, 32), (3000, 7, 41), (1000, 300, 64),
+                                   (70000, 20, 7), (5000, 251, 130), (40000, 64, 300), (777, 1433, 64)])
+@pytest.mark.parametrize("w_t", [False, True])
+def test_gemm_of_any_shape(gpu, tf, M, K, N, w_t):
+    say(f"gemm {M} x {K} x {N} w_t={w_t}")
+    rng = np.random.default_rng(M + 7 * K + 13 * N)
+    X, W, m = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    Xd, Wd = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if w_t else W)
+    want = X.astype(np.float64) @ W.astype(np.float64)
+    for mask in (None, m):
+        Y = tf.DenseMatrix.from_numpy(np.full((M, N), np.nan, np.float32))
+        md = tf.DenseMatrix.from_numpy(mask) if mask is not None else None
+        assert tf.lib().tf_gemm_ex(Xd.h, Wd.h, Y.h, md.h if md else None, C_TRANSPOSED if w_t else 0, None) == 0
+        tf.device_synchronize()
+        ref = want if mask is None else np.where(mask > 0, want, 0.0)
+        assert rel(Y.to_numpy(), ref) <= 1e-5, (mask is not None)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 7, 5), (33, 32, 128), (3000, 7, 32), (3000, 32, 500), (10000, 64, 300), (5001, 33, 161),
+                                   (100000, 64, 128), (20011, 130, 31), (64, 300, 97)])
+def test_weight_gradient(gpu, tf, M, N, K):
+    say(f"weight gradient {M} rows, {N} x {K}")
+    rng = np.random.default_rng(M + N + K)
+    G, X = rng.uniform(-1, 1, (M, N)).astype(np.float32), rng.uniform(0, 1, (M, K)).astype(np.float32)
+    Gd, Xd, Y = tf.DenseMatrix.from_numpy(G), tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(np.full((N, K), np.nan, np.float32))
+    lib = tf.lib()
+    ws = tf.DenseMatrix(1, lib.tf_weight_grad_workspace(M, N, K) // 4)
+    for _ in range(2):
+        assert lib.tf_weight_grad(Gd.h, Xd.h, Y.h, C.c_void_p(ws.device_ptr()), None) == 0
+    tf.device_synchronize()
+    assert rel(Y.to_numpy(), G.astype(np.float64).T @ X.astype(np.float64)) <= 1e-5
+
+
+@pytest.mark.parametrize("N", [1, 3, 4, 7, 16, 40, 64, 100, 128, 257])
+@pytest.mark.parametrize("relu", [False, True])
+def test_scheduled_row_product(gpu, tf, N, relu):
+    """Hub rows of one and of several chunks, rows without entries, rows of up to 32 entries."""
+    say(f"scheduled spmm N={N} relu={relu}")
+    rng = np.random.default_rng(N)
+    M = 4000
+    A = sp.random(M, M, density=3.0 / M, random_state=5, format="lil", dtype=np.float32)
+    for r, n in ((0, 33), (1, 900), (2000, 1024), (2001, 1025), (3999, 3500)):
+        A[r, :] = 0
+        A[r, rng.choice(M, n, replace=False)] = rng.uniform(-1, 1, n)
+    A = sp.csr_matrix(A, dtype=np.float32)
+    A.sort_indices()
+    X = rng.uniform(-1, 1, (M, N)).astype(np.float32)
+    Ah = tf.CsrMatrix.from_scipy(A).to_device()
+    lib = tf.lib()
+    s = C.c_void_p()
+    assert lib.tf_inspect_spmm(M, M, Ah._pp, Ah._pi, N, 0, C.byref(s)) == 0
+    try:
+        Xd, Y = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(np.full((M, N), np.nan, np.float32))
+        want = A.astype(np.float64) @ X.astype(np.float64)
+        for flags in (RELU if relu else 0, 1 | (RELU if relu else 0)):  # then D += A X
+            assert lib.tf_spmm_scheduled(Ah.h, Xd.h, Y.h, s, flags, None) == 0
+            tf.device_synchronize()
+            ref = want if not flags & 1 else (np.maximum(want, 0) if relu else want) + want
+            assert rel(Y.to_numpy(), np.maximum(ref, 0) if relu else ref) <= 1e-5, flags
+    finally:
+        lib.tf_schedule_free(s)
+
+
+@pytest.mark.parametrize("K,N", [(30, 7), (500, 32), (251, 47), (64, 300), (300, 128), (32, 1)])
+def test_layer_that_fuses_nothing_in_any_width(gpu, tf, K, N):
+    """GeMM-SpMM on a graph: K and N as they come, either storage of the weights, accumulation, a ReLU of the result."""
+    say(f"unfused layer K={K} N={N}")
+    A = tf.workloads.rmat(12, 4096 * 8, seed=3)
+    M = A.shape[0]
+    rng = np.random.default_rng(K + N)
+    X, W, D0 = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    Xd = tf.DenseMatrix.from_numpy(X)
+    want = A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))
+    for flags in (0, 1, RELU, C_TRANSPOSED, 1 | RELU | C_TRANSPOSED):
+        Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if flags & C_TRANSPOSED else W)
+        D = tf.DenseMatrix.from_numpy(D0)
+        assert tf.lib().tf_gemm_spmm(Ah.to_device().h, Xd.h, Wd.h, D.h, S.h, flags, None) == 0
+        tf.device_synchronize()
+        ref = want + D0 if flags & 1 else want
+        assert rel(D.to_numpy(), np.maximum(ref, 0) if flags & RELU else ref) <= 1e-5, flags
+
+
+@pytest.mark.parametrize("K,N", [(64, 64), (30, 40)])
+def test_fused_layer_with_transposed_weights(gpu, tf, K, N):
+    """The same flags where rows fuse (a band), through the padded copies and the transposing one."""
+    say(f"fused layer K={K} N={N}")
+    A = tf.workloads.banded_random(3000, 32, 16, seed=9)
+    M = A.shape[0]
+    rng = np.random.default_rng(K)
+    X, W = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    want = A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))
+    for flags in (0, C_TRANSPOSED, C_TRANSPOSED | RELU):
+        Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if flags & C_TRANSPOSED else W)
+        D = tf.DenseMatrix(M, N)
+        assert tf.lib().tf_gemm_spmm(Ah.to_device().h, tf.DenseMatrix.from_numpy(X).h, Wd.h, D.h, S.h, flags, None) == 0
+        tf.device_synchronize()
+        assert rel(D.to_numpy(), np.maximum(want, 0) if flags & RELU else want) <= 1e-5, flags

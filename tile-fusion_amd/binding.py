@@ -97,6 +97,7 @@ SIGNATURES = {
     "tf_csr_wrap_device": (C.c_int, [C.c_int, C.c_int, C.c_int, _VP, _VP, _VP, C.POINTER(_VP)]),
     "tf_pattern_hash": (C.c_uint64, [C.c_int, _PI, _PI]),
     "tf_csr_set_pattern_hash": (C.c_int, [_VP, C.c_uint64]),
+    "tf_csr_set_constant": (C.c_int, [_VP]),
     "tf_csr_free": (None, [_VP]),
     "tf_dense_upload": (C.c_int, [C.c_int, C.c_int, _PF, C.POINTER(_VP)]),
     "tf_dense_alloc": (C.c_int, [C.c_int, C.c_int, C.POINTER(_VP)]),
@@ -113,6 +114,7 @@ SIGNATURES = {
     "tf_reorder_partition": (C.c_int, [C.c_int, _PI, _PI, C.c_int, C.c_int, _PI, _PI]),
     "tf_permute_csr": (C.c_int, [C.c_int, _PI, _PI, _PF, _PI, C.POINTER(_PI), C.POINTER(_PI), C.POINTER(_PF)]),
     "tf_inspect": (C.c_int, [C.c_int, C.c_int, _PI, _PI, C.POINTER(InspectOpts), C.POINTER(_VP)]),
+    "tf_inspect_spmm": (C.c_int, [C.c_int, C.c_int, _PI, _PI, C.c_int, C.c_uint64, C.POINTER(_VP)]),
     "tf_schedule_free": (None, [_VP]),
     "tf_schedule_get_info": (C.c_int, [_VP, C.POINTER(ScheduleInfo)]),
     "tf_schedule_get_view": (C.c_int, [_VP, C.POINTER(ScheduleView)]),
@@ -126,7 +128,11 @@ SIGNATURES = {
     "tf_gemm_spmm": (C.c_int, [_VP, _VP, _VP, _VP, _VP, C.c_uint, _VP]),
     "tf_gcn_two_layers": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, C.c_uint, _VP]),
     "tf_spmm": (C.c_int, [_VP, _VP, _VP, C.c_uint, _VP]),
+    "tf_spmm_scheduled": (C.c_int, [_VP, _VP, _VP, _VP, C.c_uint, _VP]),
     "tf_gemm": (C.c_int, [_VP, _VP, _VP, _VP]),
+    "tf_gemm_ex": (C.c_int, [_VP, _VP, _VP, _VP, C.c_uint, _VP]),
+    "tf_weight_grad": (C.c_int, [_VP, _VP, _VP, _VP, _VP]),
+    "tf_weight_grad_workspace": (C.c_size_t, [C.c_int, C.c_int, C.c_int]),
     "tf_calibrate_issue": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float)]),
 }
 

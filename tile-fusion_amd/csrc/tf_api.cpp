@@ -34,6 +34,7 @@ namespace tf {
 
 struct DeviceSchedule {
   int device = -1;
+  char *arena = nullptr;  // one allocation for the lists and the workspace, which the pointers below name parts of
   TileDesc *tiles = nullptr;
   int *fused_ids = nullptr;
   int *win = nullptr;
@@ -44,7 +45,8 @@ struct DeviceSchedule {
   int *step_ptr = nullptr;
   int *fused_rec = nullptr;
   LongChunk *long_chunks = nullptr;
-  LongRow *long_rows = nullptr;
+  LongRow *long_rows = nullptr;  // the rows that partial sums are added up for: of several chunks, or of segments
+  int n_long_rows = 0;
   LongRow *seg_groups = nullptr;
   float *inter = nullptr;    // M x N intermediate, only if some tile writes back
   float *partial = nullptr;  // n_long_chunks (or segments) x N
@@ -88,16 +90,17 @@ hipError_t launch_fused_spmm_spmm_window(const TileDesc *, const int *, int, con
 hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, const int *, const int *,
                                            const float *, int, const float *, const int *, const int *,
                                            const float *, int, float *, int, int, int, int, hipStream_t);
-hipError_t launch_spmm_rows(const int *, int, const int *, const int *, const float *, const float *,
-                            float *, int, int, int, int, hipStream_t, int compact = 0, int coalesced_pairs = 0, int flagged = 0);
+hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
+hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
+hipError_t launch_gemm_direct(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const float *, int, hipStream_t);
+WeightGradPlan plan_weight_grad(int, int, int, int);
+hipError_t launch_weight_grad(const WeightGradPlan &, const float *, int, const float *, int, int, float *, float *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
 hipError_t launch_march_fill(const int *, const int *, const float *, const float *, int *, size_t, hipStream_t);
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
                                         const float *, float *, float *, int, int, int, int, int, int, int, hipStream_t);
 hipError_t launch_scatter_values(const int *, const int *, const float *, float *, int, hipStream_t);
-hipError_t launch_seg_reduce(const LongRow *, int, const int *, const float *, float *, int, int, hipStream_t);
-hipError_t launch_long_rows(const LongChunk *, int, const LongRow *, int, const int *, const float *,
-                            const float *, float *, float *, int, int, hipStream_t);
+hipError_t launch_seg_reduce(const LongRow *, int, const int *, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_fused_gemm_spmm(const TileDesc *, int, const int *, const float *, const float *,
                                   int, int, const int *, const int *, const float *, float *,
                                   float *, int, int, int, int, int, hipStream_t);
@@ -107,6 +110,7 @@ hipError_t launch_fused_gemm_spmm_stream(const TileDesc *, int, const int *, con
 hipError_t launch_gemm(const float *, const float *, float *, const int *, int, int, int, int, hipStream_t, int y_by_position = 0);
 hipError_t launch_fill(float *, size_t, float, hipStream_t);
 hipError_t launch_pad(const float *, int, int, float *, int, int, hipStream_t);
+hipError_t launch_transpose_pad(const float *, int, int, int, int, float *, int, int, hipStream_t);
 hipError_t launch_copy_cols(const float *, int, int, int, int, float *, int, int, int, int, int, hipStream_t);
 hipError_t launch_relu(float *, size_t, hipStream_t);
 hipError_t launch_fused_gcn2(const Tile2 *, int, const float *, const float *, const float *, int, int, int, const int *, const int *,
@@ -152,14 +156,7 @@ int default_compute_units() {
 
 void release_device_schedule(DeviceSchedule *d) {
   if (!d) return;
-  (void)hipFree(d->tiles); (void)hipFree(d->fused_ids); (void)hipFree(d->win); (void)hipFree(d->rem_rows); (void)hipFree(d->zero_rows); (void)hipFree(d->plain_rows);
-  (void)hipFree(d->long_chunks); (void)hipFree(d->long_rows); (void)hipFree(d->seg_groups);
-  (void)hipFree(d->seg_ptr); (void)hipFree(d->ent_src); (void)hipFree(d->ent_pos); (void)hipFree(d->seg_col); (void)hipFree(d->lrow_seg); (void)hipFree(d->seg_val);
-  (void)hipFree(d->step_begin); (void)hipFree(d->step_ptr); (void)hipFree(d->fused_rec);
-  (void)hipFree(d->inter); (void)hipFree(d->partial); (void)hipFree(d->Bpad); (void)hipFree(d->Cpad); (void)hipFree(d->Cpanel); (void)hipFree(d->Dpanel); (void)hipFree(d->hidden); (void)hipFree(d->l2_tiles);
-  (void)hipFree(d->rem_ptr); (void)hipFree(d->rem_col); (void)hipFree(d->rem_src); (void)hipFree(d->rem_val);
-  (void)hipFree(d->m_runs); (void)hipFree(d->m_row_ptr); (void)hipFree(d->m_load_ptr); (void)hipFree(d->m_load);
-  (void)hipFree(d->m_row_out); (void)hipFree(d->m_ell_off); (void)hipFree(d->m_ell_src); (void)hipFree(d->m_ell); (void)hipFree(d->m_trash);
+  (void)hipFree(d->arena); (void)hipFree(d->Cpad); (void)hipFree(d->hidden);
   if (d->side) (void)hipStreamDestroy(d->side);
   if (d->fork) (void)hipEventDestroy(d->fork);
   if (d->join) (void)hipEventDestroy(d->join);
@@ -169,13 +166,51 @@ void release_device_schedule(DeviceSchedule *d) {
   delete d;
 }
 
-template <class T> static tf_status upload_vec(const std::vector<T> &v, T **out) {
-  *out = nullptr;
-  if (v.empty()) return TF_OK;
-  TF_HIP(hipMalloc(reinterpret_cast<void **>(out), v.size() * sizeof(T)));
-  TF_HIP(hipMemcpy(*out, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-  return TF_OK;
-}
+// The parts of a schedule's arena: lists to be copied there and workspace to be reserved, collected first and then made with
+// one allocation; lists of up to 64 KB, which come first, travel in one copy.  (An allocation, its release and a small copy
+// each cost tens of microseconds: a schedule has up to thirty arrays.)
+class ArenaParts {
+ public:
+  template <class T> void list(const std::vector<T> &v, T **out) {
+    *out = nullptr;
+    if (!v.empty()) add(v.data(), v.size() * sizeof(T), out);
+  }
+  template <class T> void reserve(size_t n, T **out) { add(nullptr, std::max<size_t>(n, 1) * sizeof(T), out); }
+  tf_status make(char **arena) {
+    std::stable_partition(parts_.begin(), parts_.end(), [](const Part &p) { return small(p); });
+    size_t total = 0, packed = 0;
+    for (Part &p : parts_) {  // (the large ones start where an allocation of their own would: at a page)
+      const size_t align = p.bytes >= ((size_t)2 << 20) ? (size_t)2 << 20 : 256;
+      p.at = (total + align - 1) / align * align;
+      total = p.at + p.bytes;
+      if (small(p)) packed = total;
+    }
+    if (total == 0) return TF_OK;
+    TF_HIP(hipMalloc(reinterpret_cast<void **>(arena), total));
+    std::vector<char> stage(packed);
+    for (const Part &p : parts_) {
+      *p.out = *arena + p.at;
+      if (small(p)) std::memcpy(stage.data() + p.at, p.data, p.bytes);
+    }
+    if (packed > 0) TF_HIP(hipMemcpy(*arena, stage.data(), packed, hipMemcpyHostToDevice));
+    for (const Part &p : parts_)
+      if (p.data && !small(p)) TF_HIP(hipMemcpy(*arena + p.at, p.data, p.bytes, hipMemcpyHostToDevice));
+    return TF_OK;
+  }
+
+ private:
+  struct Part { const void *data; size_t bytes, at; void **out; };
+  static bool small(const Part &p) { return p.data && p.bytes <= 65536; }
+  template <class T> void add(const void *data, size_t bytes, T **out) { parts_.push_back({data, bytes, 0, reinterpret_cast<void **>(out)}); }
+  std::vector<Part> parts_;
+};
+
+// A GeMM-SpMM schedule in which nothing fuses is a GEMM into the intermediate and row products out of it, for which K
+// and N are what the caller has.  (Tiles take K in steps of 8 and N in steps of 32: padded copies, column panels.)
+static bool untiled(const tf_schedule *s) { return s->opts.op == TF_OP_GEMM_SPMM && s->launch_tiles.empty(); }
+// Floats from one row of the intermediate to the next: a multiple of 4, so that every lane's columns of a row are one
+// aligned load.
+static int inter_ld(const tf_schedule *s) { return untiled(s) ? (s->user_N + 3) / 4 * 4 : s->opts.N; }
 
 // Device copies of the schedule arrays and the workspace, made on first use.
 static tf_status ensure_device(tf_schedule *s) {
@@ -191,78 +226,76 @@ static tf_status ensure_device(tf_schedule *s) {
   auto *d = new (std::nothrow) DeviceSchedule();
   if (!d) return fail(TF_ENOMEM, "out of host memory");
   d->device = dev;
-  tf_status rc = TF_OK;
+  ArenaParts parts;
+  const std::vector<float> trash(64, 0.f);
+  std::vector<LongChunk> chunks;
+  std::vector<LongRow> summed;  // the rows that partial sums are added up for
   if (s->march) {  // nothing but the run lists is needed on the device
-    rc = upload_vec(s->march_runs, &d->m_runs);
-    if (!rc) rc = upload_vec(s->march_row_ptr, &d->m_row_ptr);
-    if (!rc) rc = upload_vec(s->march_load_ptr, &d->m_load_ptr);
-    if (!rc) rc = upload_vec(s->march_load, &d->m_load);
-    if (!rc) rc = upload_vec(s->march_row_out, &d->m_row_out);
-    if (!rc) rc = upload_vec(s->march_ell_off, &d->m_ell_off);
-    if (!rc) rc = upload_vec(s->march_ell_src, &d->m_ell_src);
-    if (!rc) {
-      hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->m_ell), s->march_ell_off.size() * 2 * sizeof(int));
-      if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&d->m_trash), 64 * sizeof(float));
-      if (e == hipSuccess) e = hipMemset(d->m_trash, 0, 64 * sizeof(float));
-      if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(ELL rows)");
+    parts.list(s->march_runs, &d->m_runs);
+    parts.list(s->march_row_ptr, &d->m_row_ptr);
+    parts.list(s->march_load_ptr, &d->m_load_ptr);
+    parts.list(s->march_load, &d->m_load);
+    parts.list(s->march_row_out, &d->m_row_out);
+    parts.list(s->march_ell_off, &d->m_ell_off);
+    parts.list(s->march_ell_src, &d->m_ell_src);
+    parts.reserve(s->march_ell_off.size() * 2, &d->m_ell);
+    parts.list(trash, &d->m_trash);
+  } else {
+    parts.list(s->launch_tiles, &d->tiles);
+    parts.list(s->l2_tiles, &d->l2_tiles);
+    parts.list(s->fused_ids, &d->fused_ids);
+    parts.list(s->win, &d->win);
+    parts.list(s->rem_rows, &d->rem_rows);
+    parts.list(s->zero_rows, &d->zero_rows);
+    parts.list(s->plain_rows, &d->plain_rows);
+    parts.list(s->launch_step, &d->step_begin);
+    parts.list(s->step_ptr, &d->step_ptr);
+    parts.list(s->fused_rec, &d->fused_rec);
+    if (!s->rem_ptr.empty()) {
+      parts.list(s->rem_ptr, &d->rem_ptr);
+      parts.list(s->rem_col, &d->rem_col);
+      parts.list(s->rem_src, &d->rem_src);
+      parts.reserve(s->rem_src.size(), &d->rem_val);
     }
-    if (rc) { release_device_schedule(d); return rc; }
-    s->dev = d;
-    return TF_OK;
-  }
-  rc = upload_vec(s->launch_tiles, &d->tiles);
-  if (!rc) rc = upload_vec(s->l2_tiles, &d->l2_tiles);
-  if (!rc) rc = upload_vec(s->fused_ids, &d->fused_ids);
-  if (!rc) rc = upload_vec(s->win, &d->win);
-  if (!rc) rc = upload_vec(s->rem_rows, &d->rem_rows);
-  if (!rc) rc = upload_vec(s->zero_rows, &d->zero_rows);
-  if (!rc) rc = upload_vec(s->plain_rows, &d->plain_rows);
-  if (!rc) rc = upload_vec(s->launch_step, &d->step_begin);
-  if (!rc) rc = upload_vec(s->step_ptr, &d->step_ptr);
-  if (!rc) rc = upload_vec(s->fused_rec, &d->fused_rec);
-  if (!rc && !s->rem_ptr.empty()) {
-    rc = upload_vec(s->rem_ptr, &d->rem_ptr);
-    if (!rc) rc = upload_vec(s->rem_col, &d->rem_col);
-    if (!rc) rc = upload_vec(s->rem_src, &d->rem_src);
-    if (!rc) {
-      hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->rem_val), std::max<size_t>(s->rem_src.size(), 1) * sizeof(float));
-      if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(reordered rows)");
+    const size_t N = (size_t)std::max(s->opts.N, s->user_N);
+    size_t slots = 0;  // partial sums
+    if (!s->long_chunks.empty()) {
+      // The chunk of a row that has no other goes straight to the row of the result (slot -1); only rows of several
+      // chunks need partial sums and the launch that adds them up.
+      chunks = s->long_chunks;
+      for (const LongRow &lr : s->long_rows) {
+        if (lr.count == 1) { chunks[lr.first].slot = -1; continue; }
+        summed.push_back({lr.row, (int)slots, lr.count, 0});
+        for (int c = 0; c < lr.count; ++c) chunks[lr.first + c].slot = (int)slots++;
+      }
+      // longest first: what starts last should end soon
+      std::stable_sort(chunks.begin(), chunks.end(), [](const LongChunk &a, const LongChunk &b) { return a.k_end - a.k_begin > b.k_end - b.k_begin; });
+      parts.list(chunks, &d->long_chunks);
+    } else {
+      summed = s->long_rows;
     }
-  }
-  if (!rc) rc = upload_vec(s->long_chunks, &d->long_chunks);
-  if (!rc) rc = upload_vec(s->long_rows, &d->long_rows);
-  if (!rc && s->long_part) {
-    rc = upload_vec(s->seg_ptr, &d->seg_ptr);
-    if (!rc) rc = upload_vec(s->ent_src, &d->ent_src);
-    if (!rc) rc = upload_vec(s->ent_pos, &d->ent_pos);
-    if (!rc) rc = upload_vec(s->seg_col, &d->seg_col);
-    if (!rc) rc = upload_vec(s->lrow_seg, &d->lrow_seg);
-    if (!rc) rc = upload_vec(s->seg_groups, &d->seg_groups);
-    if (!rc) {
-      hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->seg_val), std::max<size_t>(s->seg_src.size(), 1) * sizeof(float));
-      if (e == hipSuccess)
-        e = hipMalloc(reinterpret_cast<void **>(&d->partial), (s->seg_ptr.size() - 1 + s->seg_groups.size()) * (size_t)s->opts.N * sizeof(float));
-      if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(long-row segments)");
+    parts.list(summed, &d->long_rows);
+    d->n_long_rows = (int)summed.size();
+    if (s->long_part) {
+      parts.list(s->seg_ptr, &d->seg_ptr);
+      parts.list(s->ent_src, &d->ent_src);
+      parts.list(s->ent_pos, &d->ent_pos);
+      parts.list(s->seg_col, &d->seg_col);
+      parts.list(s->lrow_seg, &d->lrow_seg);
+      parts.list(s->seg_groups, &d->seg_groups);
+      parts.reserve(s->seg_src.size(), &d->seg_val);
+      slots = s->seg_ptr.size() - 1 + s->seg_groups.size();
     }
+    if (slots > 0) parts.reserve(slots * N, &d->partial);
+    if (s->n_writeback_rows > 0) parts.reserve((size_t)s->M * inter_ld(s), &d->inter);
+    const bool tiled = s->opts.op == TF_OP_GEMM_SPMM && !s->launch_tiles.empty();
+    if (tiled && s->user_N != s->opts.N) {
+      parts.reserve((size_t)s->opts.K * s->opts.N, &d->Cpanel);
+      parts.reserve((size_t)s->L * s->opts.N, &d->Dpanel);
+    }
+    if (tiled && s->user_K != s->opts.K) parts.reserve((size_t)s->M * s->opts.K, &d->Bpad);
   }
-  if (!rc && s->n_writeback_rows > 0) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->inter), (size_t)s->M * s->opts.N * sizeof(float));
-    if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(intermediate)");
-  }
-  if (!rc && s->opts.op == TF_OP_GEMM_SPMM && s->user_N != s->opts.N) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->Cpanel), (size_t)s->opts.K * s->opts.N * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&d->Dpanel), (size_t)s->L * s->opts.N * sizeof(float));
-    if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(column panels)");
-  }
-  if (!rc && s->opts.op == TF_OP_GEMM_SPMM && s->user_K != s->opts.K) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->Bpad), (size_t)s->M * s->opts.K * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&d->Cpad), (size_t)s->opts.K * s->opts.N * sizeof(float));
-    if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(padded operands)");
-  }
-  if (!rc && !s->long_chunks.empty()) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->partial), s->long_chunks.size() * (size_t)s->opts.N * sizeof(float));
-    if (e != hipSuccess) rc = hip_fail(e, "hipMalloc(partials)");
-  }
+  tf_status rc = parts.make(&d->arena);
   if (!rc && s->long_part && s->plain_hot > 0) {
     hipError_t e = hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d->fork, hipEventDisableTiming);
@@ -316,59 +349,84 @@ static tf_status ensure_segment_values(const tf_csr *A, tf_schedule *s, hipStrea
   d->seg_val_serial = A->serial;
   return TF_OK;
 }
-static tf_status run_hot_segments(tf_schedule *s, hipStream_t st) {
+// What the row products of a call read and write: T (row stride ldt) the intermediate or, for a rows-only schedule, the
+// operand itself; N columns.
+struct Remainder {
+  const float *T;
+  int ldt, N, rows;  // rows of T
+  float *D;
+  int accumulate, relu;
+};
+static tf_status run_hot_segments(tf_schedule *s, const Remainder &r, hipStream_t st) {
   DeviceSchedule *d = s->dev;
-  TF_PHASE(s, "spmm_rows_kernel (hot long-row segments)", st,
-           launch_spmm_rows(nullptr, 8 * s->seg_per_xcd, d->seg_ptr, d->seg_col, d->seg_val, d->inter, d->partial, s->opts.N, 0, -1, 1, st, /*compact=*/0, /*coalesced_pairs=*/1));
+  RowsArgs a;
+  a.n_rows = 8 * s->seg_per_xcd;
+  a.Ap = d->seg_ptr; a.Ai = d->seg_col; a.Ax = d->seg_val;
+  a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = d->partial; a.ldy = r.N; a.N = r.N;
+  a.streaming = 1;
+  RowsHow how;
+  how.xcd_chunk_rows = -1;
+  TF_PHASE(s, "spmm_rows_kernel (hot long-row segments)", st, launch_spmm_rows(a, how, st));
   return TF_OK;
 }
 
 // Second-op rows that no tile fused: served from the intermediate in HBM.  hot_on_side: the hot
 // long-row segments were launched on the side stream already and are joined here.
-static tf_status run_remainder(const tf_csr *A, tf_dense *D, tf_schedule *s, int accumulate, bool hot_on_side, hipStream_t st) {
+static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
   DeviceSchedule *d = s->dev;
-  const int N = s->opts.N;
-  if (!s->zero_rows.empty() && !accumulate)  // (D += 0 needs nothing)
-    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), D->d, N, st));
+  const int N = r.N;
+  if (!s->zero_rows.empty() && !r.accumulate)  // (D += 0 needs nothing)
+    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, N, st));
+  RowsArgs a;
+  a.n_rows = (int)s->rem_rows.size();
+  a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
+  a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = N; a.N = N;
+  a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = 1;
+  RowsHow how;
+  how.xcd_chunk_rows = s->xcd_chunk_rows;
+  a.chunks = d->long_chunks;
+  a.n_chunks = (unsigned)s->long_chunks.size();
+  a.chunk_Ai = A->i; a.chunk_Ax = A->x; a.partial = d->partial;
   if (!s->rem_rows.empty() && !s->rem_ptr.empty()) {
     // The rows in the order of the list, entries side by side -- the reference's reordered adjacency
     // (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653; executor at
-    // GCN_Layer_MKL_Forward_Utils.h:294-373).  The values are copied on the first call with an uploaded
-    // matrix, whose device arrays never change, and on every call with a wrapped one.
+    // GCN_Layer_MKL_Forward_Utils.h:294-373).  The values are copied on the first call with a matrix whose
+    // device arrays never change, and on every call with any other.
     if (!(A->serial != 0 && d->rem_val_serial == A->serial))
       TF_PHASE(s, "gather_values_kernel", st, launch_gather_values(d->rem_src, A->x, d->rem_val, (int)s->rem_src.size(), st));
     d->rem_val_serial = A->serial;
-    TF_PHASE(s, "spmm_rows_kernel (short remainder rows)", st,
-             launch_spmm_rows(d->rem_rows, (int)s->rem_rows.size(), d->rem_ptr, d->rem_col, d->rem_val, d->inter, D->d, N, accumulate,
-                              s->xcd_chunk_rows, /*streaming=*/1, st, /*compact=*/1, /*coalesced_pairs=*/0, s->rem_flagged ? 1 : 0));
-  } else if (!s->rem_rows.empty()) {
-    // identity list: no indirection needed
-    TF_PHASE(s, "spmm_rows_kernel (short remainder rows)", st,
-             launch_spmm_rows(s->rem_identity ? nullptr : d->rem_rows, (int)s->rem_rows.size(), A->p, A->i,
-                              A->x, d->inter, D->d, N, accumulate, s->xcd_chunk_rows, /*streaming=*/1, st));
+    a.rows = d->rem_rows;
+    a.Ap = d->rem_ptr; a.Ai = d->rem_col; a.Ax = d->rem_val;
+    a.compact = 1;
+    how.flagged = s->rem_flagged ? 1 : 0;
+  } else if (!s->rem_identity) {
+    a.rows = d->rem_rows;
   }
+  // one launch, the long rows' workgroups first
+  if (a.n_rows > 0 || a.n_chunks > 0)
+    TF_PHASE(s, a.n_chunks > 0 ? "spmm_rows_kernel (short and long remainder rows)" : "spmm_rows_kernel (short remainder rows)", st, launch_spmm_rows(a, how, st));
   if (s->long_part) {
     const int n_hot = 8 * s->seg_per_xcd, n_seg = (int)s->seg_ptr.size() - 1;
     if (!hot_on_side) {
       if (tf_status rc = ensure_segment_values(A, s, st)) return rc;
-      if (tf_status rc = run_hot_segments(s, st)) return rc;
+      if (tf_status rc = run_hot_segments(s, r, st)) return rc;
     }
-    TF_PHASE(s, "spmm_rows_kernel (cold long-row segments)", st,
-             launch_spmm_rows(nullptr, n_seg - n_hot, d->seg_ptr + n_hot, d->seg_col, d->seg_val, d->inter,
-                              d->partial + (size_t)n_hot * N, N, 0, 0, 1, st));
+    RowsArgs c;
+    c.n_rows = n_seg - n_hot;
+    c.Ap = d->seg_ptr + n_hot; c.Ai = d->seg_col; c.Ax = d->seg_val;
+    c.X = r.T; c.ldx = r.ldt; c.x_rows = r.rows; c.Y = d->partial + (size_t)n_hot * N; c.ldy = N; c.N = N;
+    c.streaming = 1;
+    TF_PHASE(s, "spmm_rows_kernel (cold long-row segments)", st, launch_spmm_rows(c, RowsHow(), st));
     if (hot_on_side) TF_HIP(hipStreamWaitEvent(st, d->join, 0));
     // groups of segments of the rows with many (into their own slots of `partial`), then the rows
     if (!s->seg_groups.empty())
       TF_PHASE(s, "long_seg_reduce_kernel (groups)", st,
-               launch_seg_reduce(d->seg_groups, (int)s->seg_groups.size(), d->lrow_seg, d->partial, d->partial, N, 0, st));
+               launch_seg_reduce(d->seg_groups, (int)s->seg_groups.size(), d->lrow_seg, d->partial, d->partial, N, N, 0, 0, st));
     TF_PHASE(s, "long_seg_reduce_kernel (rows)", st,
-             launch_seg_reduce(d->long_rows, (int)s->long_rows.size(), d->lrow_seg, d->partial, D->d, N, accumulate, st));
+             launch_seg_reduce(d->long_rows, d->n_long_rows, d->lrow_seg, d->partial, r.D, N, N, r.accumulate, r.relu, st));
+  } else if (d->n_long_rows > 0) {
+    TF_PHASE(s, "long_row_reduce_kernel", st, launch_long_row_reduce(d->long_rows, d->n_long_rows, d->partial, r.D, N, N, r.accumulate, r.relu, st));
   }
-  if (!s->long_chunks.empty())
-    TF_PHASE(s, "spmm_long_chunk_kernel + long_row_reduce_kernel", st,
-             launch_long_rows(d->long_chunks, (int)s->long_chunks.size(), d->long_rows,
-                              (int)s->long_rows.size(), A->i, A->x, d->inter, d->partial, D->d, N,
-                              accumulate, st));
   return TF_OK;
 }
 
@@ -402,13 +460,6 @@ tf_status scratch_of_current_device(float **out) {
   *out = g_scratch_ptr[dev];
   return TF_OK;
 }
-
-// tf_gemm's buffers for shapes off the MFMA kernel's fast path: padded X, a panel of W, a panel of Y.
-struct GemmWorkspace {
-  float *buf[3] = {nullptr, nullptr, nullptr};
-  size_t floats[3] = {0, 0, 0};
-};
-GemmWorkspace g_gemm_ws[kMaxDevices];
 
 }  // namespace
 
@@ -542,6 +593,9 @@ extern "C" tf_status tf_event_elapsed_ms(void *start, void *stop, float *ms) {
   return TF_OK;
 }
 
+// a matrix whose device arrays never change has a number of its own
+static std::atomic<unsigned long long> g_next_serial{1};
+
 // ---- operands ----------------------------------------------------------------------
 
 extern "C" tf_status tf_csr_upload(int M, int N, const int *Ap, const int *Ai, const float *Ax,
@@ -559,8 +613,7 @@ extern "C" tf_status tf_csr_upload(int M, int N, const int *Ap, const int *Ai, c
   auto *a = new (std::nothrow) tf_csr();
   if (!a) return fail(TF_ENOMEM, "out of host memory");
   a->M = M; a->N = N; a->nnz = nnz; a->owns = true;
-  static std::atomic<unsigned long long> next_serial{1};
-  a->serial = next_serial.fetch_add(1);
+  a->serial = g_next_serial.fetch_add(1);
   a->hash = tf_pattern_hash(M, Ap, Ai);
   hipError_t e = hipMalloc(reinterpret_cast<void **>(&a->p), (size_t)(M + 1) * sizeof(int));
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&a->i), (size_t)std::max(nnz, 1) * sizeof(int));
@@ -590,6 +643,12 @@ extern "C" tf_status tf_csr_wrap_device(int M, int N, int nnz, const int *dAp, c
 extern "C" tf_status tf_csr_set_pattern_hash(tf_csr *a, uint64_t hash) {
   if (!a) return fail(TF_EINVAL, "tf_csr_set_pattern_hash: null argument");
   a->hash = hash;
+  return TF_OK;
+}
+
+extern "C" tf_status tf_csr_set_constant(tf_csr *a) {
+  if (!a) return fail(TF_EINVAL, "tf_csr_set_constant: null argument");
+  a->serial = g_next_serial.fetch_add(1);
   return TF_OK;
 }
 
@@ -664,17 +723,24 @@ extern "C" void tf_dense_free(tf_dense *d) {
 
 // ---- executors -----------------------------------------------------------------------
 
-static tf_status check_common(const char *who, const tf_csr *A, const tf_dense *C, const tf_dense *D,
-                              const tf_schedule *s, int op) {
-  if (!A || !C || !D || !s) return fail(TF_EINVAL, "%s: null argument", who);
-  if (s->opts.op != op) return fail(TF_ESCHEDULE, "%s: schedule was built for the other operation", who);
+static tf_status check_pattern(const char *who, const tf_csr *A, const tf_schedule *s) {
   if (A->M != s->L || A->N != s->M || A->nnz != s->nnz)
     return fail(TF_ESCHEDULE, "%s: schedule was built for a %d x %d pattern with %lld entries, A is %d x %d with %d",
                 who, s->L, s->M, s->nnz, A->M, A->N, A->nnz);
   if (A->hash && A->hash != s->pattern_hash)
     return fail(TF_ESCHEDULE, "%s: A has the shape and entry count the schedule was built for, but another sparsity pattern", who);
-  if (C->N != s->user_N || D->N != s->user_N)
-    return fail(TF_ESCHEDULE, "%s: schedule was built for N = %d, C has %d and D has %d columns", who, s->user_N, C->N, D->N);
+  return TF_OK;
+}
+
+static tf_status check_common(const char *who, const tf_csr *A, const tf_dense *C, const tf_dense *D,
+                              const tf_schedule *s, int op, bool c_transposed = false) {
+  if (!A || !C || !D || !s) return fail(TF_EINVAL, "%s: null argument", who);
+  if (s->rows_only) return fail(TF_ESCHEDULE, "%s: the schedule is one of tf_inspect_spmm", who);
+  if (s->opts.op != op) return fail(TF_ESCHEDULE, "%s: schedule was built for the other operation", who);
+  if (tf_status rc = check_pattern(who, A, s)) return rc;
+  const int cn = c_transposed ? C->M : C->N;
+  if (cn != s->user_N || D->N != s->user_N)
+    return fail(TF_ESCHEDULE, "%s: schedule was built for N = %d, C has %d and D has %d columns", who, s->user_N, cn, D->N);
   if (D->M != A->M) return fail(TF_EINVAL, "%s: D has %d rows, A has %d", who, D->M, A->M);
   return TF_OK;
 }
@@ -745,60 +811,79 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
                                         s->windowed ? s->lds_bytes_general : s->lds_bytes, acc, st));
   if (!s->plain_rows.empty()) {  // intermediate rows of tiles that fuse nothing
     const bool all = (int)s->plain_rows.size() == s->M;
-    TF_PHASE(s, "spmm_rows_kernel (intermediate rows)", st,
-             tf::launch_spmm_rows(all ? nullptr : d->plain_rows, (int)s->plain_rows.size(), B->p, B->i, B->x,
-                                  C->d, d->inter, s->opts.N, 0, s->xcd_chunk_rows, tf::inter_streams(s), st));
+    tf::RowsArgs a;
+    a.rows = all ? nullptr : d->plain_rows;
+    a.n_rows = (int)s->plain_rows.size();
+    a.Ap = B->p; a.Ai = B->i; a.Ax = B->x;
+    a.X = C->d; a.ldx = s->opts.N; a.x_rows = C->M; a.Y = d->inter; a.ldy = s->opts.N; a.N = s->opts.N;
+    a.streaming = tf::inter_streams(s);
+    tf::RowsHow how;
+    how.xcd_chunk_rows = s->xcd_chunk_rows;
+    TF_PHASE(s, "spmm_rows_kernel (intermediate rows)", st, tf::launch_spmm_rows(a, how, st));
   }
-  return tf::run_remainder(A, D, s, acc, false, st);
+  return tf::run_remainder(A, s, tf::Remainder{d->inter, s->opts.N, s->opts.N, s->M, D->d, acc, 0}, false, st);
 }
 
-// One pass of a GeMM-SpMM schedule: D (L x opts.N, dense) = A * (Bd * Cd) with Bd L' x opts.K and Cd opts.K x opts.N
-// as the kernels take them.
-// relu_in: Bd holds a layer's output before its activation; only for schedules that relu_on_load_ok() accepts.
-static tf_status gemm_spmm_pass(const tf_csr *A, const float *Bd, const float *Cd, tf_dense *D, tf_schedule *s, int acc,
-                                unsigned flags, hipStream_t st, int relu_in = 0) {
+// W as the row GEMM takes it: row-major K x N with N a multiple of 32 up to 256, K of 8, small enough for LDS.
+static bool row_gemm_takes(int K, int N) { return K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072; }
+
+// What a GeMM-SpMM pass reads and writes: B (M x K), C (K x N, or N x K with c_t) and D (L x N).
+struct GemmPass {
+  const float *B, *C;
+  int c_t, K, N;
+  float *D;
+  int accumulate;
+  int relu_in;  // B holds a layer's output before its activation; only for schedules that relu_on_load_ok() accepts
+  int relu;     // the rows of D that the row kernels write go through a ReLU
+};
+
+// One pass of a GeMM-SpMM schedule: D = A * (B * C), K and N as the schedule's kernels take them (any when nothing fuses).
+static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass &g, unsigned flags, hipStream_t st) {
   tf::DeviceSchedule *d = s->dev;
-  const int n_launch = (int)s->launch_tiles.size();
+  const int n_launch = (int)s->launch_tiles.size(), ldt = tf::inter_ld(s);
   if (n_launch > 0) {
     if (s->gemm_stream)
       TF_PHASE(s, "fused_gemm_spmm_stream_kernel", st,
                tf::launch_fused_gemm_spmm_stream(d->tiles, n_launch, d->step_begin, d->step_ptr,
-                                                 d->fused_rec, Bd, Cd, s->opts.K, s->opts.N, s->ring_rows,
-                                                 A->i, A->x, D->d, d->inter, s->lds_bytes, acc, st, relu_in));
+                                                 d->fused_rec, g.B, g.C, g.K, g.N, s->ring_rows,
+                                                 A->i, A->x, g.D, d->inter, s->lds_bytes, g.accumulate, st, g.relu_in));
     else
       TF_PHASE(s, s->gemm_regw ? "fused_gemm_spmm_regw_kernel" : "fused_gemm_spmm_kernel", st,
-               tf::launch_fused_gemm_spmm(d->tiles, n_launch, d->fused_ids, Bd, Cd,
-                                          s->opts.K, s->gemm_kc, A->p, A->i, A->x, D->d, d->inter,
-                                          s->opts.N, s->lds_bytes, acc, s->opts.compute_units, s->gemm_regw ? 1 : 0, st));
+               tf::launch_fused_gemm_spmm(d->tiles, n_launch, d->fused_ids, g.B, g.C,
+                                          g.K, s->gemm_kc, A->p, A->i, A->x, g.D, d->inter,
+                                          g.N, s->lds_bytes, g.accumulate, s->opts.compute_units, s->gemm_regw ? 1 : 0, st));
   }
   // Column-partitioned long rows read the most-read ("hot") intermediate rows only through their
   // hot segments.  Those rows are produced first; on request (TF_SECOND_STREAM) the hot segments
   // then run on a second stream beside the rest of the GEMM and are joined before the rows' sums.
   const bool overlap = d->side && s->plain_hot > 0 && (flags & TF_SECOND_STREAM);
+  const tf::Remainder rem{d->inter, ldt, g.N, s->M, g.D, g.accumulate, g.relu};
   if (!s->plain_rows.empty()) {  // intermediate rows of tiles that fuse nothing
     const int n_plain = (int)s->plain_rows.size();
     const int placed = s->t_pos.empty() ? 0 : 1;  // the intermediate's rows stored in the order of the list
     const bool all = n_plain == s->M && s->plain_hot == 0 && !placed;
+    const bool row_gemm = !g.c_t && ldt == g.N && row_gemm_takes(g.K, g.N);
+    auto gemm = [&](int first, int count) {
+      const int *rows = all ? nullptr : d->plain_rows + first;
+      float *Y = d->inter + (placed ? (size_t)first * ldt : 0);
+      return row_gemm ? tf::launch_gemm(g.B, g.C, Y, rows, count, g.K, g.N, s->opts.compute_units, st, placed)
+                      : tf::launch_gemm_direct(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, nullptr, s->opts.compute_units, st);
+    };
     if (overlap) {
-      TF_PHASE(s, "gemm_rows_kernel (hot rows)", st,
-               tf::launch_gemm(Bd, Cd, d->inter, d->plain_rows, s->plain_hot, s->opts.K, s->opts.N, s->opts.compute_units, st, placed));
+      TF_PHASE(s, "gemm_rows_kernel (hot rows)", st, gemm(0, s->plain_hot));
       // the regrouped values (of the hot and of the cold segments) before the fork: the cold segments run on
       // this stream and are not ordered after anything the side stream does until the join
       if (tf_status rc2 = tf::ensure_segment_values(A, s, st)) return rc2;
       TF_HIP(hipEventRecord(d->fork, st));
       TF_HIP(hipStreamWaitEvent(d->side, d->fork, 0));
-      if (tf_status rc2 = tf::run_hot_segments(s, d->side)) return rc2;
+      if (tf_status rc2 = tf::run_hot_segments(s, rem, d->side)) return rc2;
       TF_HIP(hipEventRecord(d->join, d->side));
-      if (n_plain > s->plain_hot)
-        TF_PHASE(s, "gemm_rows_kernel (other rows)", st,
-                 tf::launch_gemm(Bd, Cd, d->inter + (placed ? (size_t)s->plain_hot * s->opts.N : 0), d->plain_rows + s->plain_hot,
-                                 n_plain - s->plain_hot, s->opts.K, s->opts.N, s->opts.compute_units, st, placed));
+      if (n_plain > s->plain_hot) TF_PHASE(s, "gemm_rows_kernel (other rows)", st, gemm(s->plain_hot, n_plain - s->plain_hot));
     } else {
-      TF_PHASE(s, "gemm_rows_kernel", st,
-               tf::launch_gemm(Bd, Cd, d->inter, all ? nullptr : d->plain_rows, n_plain, s->opts.K, s->opts.N, s->opts.compute_units, st, placed));
+      TF_PHASE(s, row_gemm ? "gemm_rows_kernel" : "gemm_direct_kernel", st, gemm(0, n_plain));
     }
   }
-  return tf::run_remainder(A, D, s, acc, overlap && !s->plain_rows.empty(), st);
+  return tf::run_remainder(A, s, rem, overlap && !s->plain_rows.empty(), st);
 }
 
 
@@ -810,46 +895,55 @@ static bool relu_on_load_ok(const tf_schedule *s) {
 
 static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_dense *C, tf_dense *D,
                                 tf_schedule *s, unsigned flags, void *stream, int relu_in) {
-  tf_status rc = check_common("tf_gemm_spmm", A, C, D, s, TF_OP_GEMM_SPMM);
+  const int c_t = (flags & TF_C_TRANSPOSED) ? 1 : 0, relu = (flags & TF_RELU) ? 1 : 0;
+  tf_status rc = check_common("tf_gemm_spmm", A, C, D, s, TF_OP_GEMM_SPMM, c_t != 0);
   if (rc) return rc;
   if (!B) return fail(TF_EINVAL, "tf_gemm_spmm: B is null");
   if (B->M != A->N) return fail(TF_EINVAL, "tf_gemm_spmm: B has %d rows, A has %d columns", B->M, A->N);
-  if (B->N != s->user_K || C->M != s->user_K)
-    return fail(TF_ESCHEDULE, "tf_gemm_spmm: schedule was built for K = %d, B has %d columns and C has %d rows", s->user_K, B->N, C->M);
+  const int c_k = c_t ? C->N : C->M;
+  if (B->N != s->user_K || c_k != s->user_K)
+    return fail(TF_ESCHEDULE, "tf_gemm_spmm: schedule was built for K = %d, B has %d columns and C has %d rows", s->user_K, B->N, c_k);
   rc = tf::ensure_device(s);
   if (rc) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int acc = (flags & TF_ACCUMULATE) ? 1 : 0;
   tf::DeviceSchedule *d = s->dev;
   d->prof_n = 0;
+  if (relu_in && !relu_on_load_ok(s)) return fail(TF_EINVAL, "tf_gemm_spmm: internal error, activation on load with a schedule that cannot apply it");
+  if (tf::untiled(s)) return gemm_spmm_pass(A, s, GemmPass{B->d, C->d, c_t, s->user_K, s->user_N, D->d, acc, 0, relu}, flags, st);
+  // Tiles take K in steps of 8 and N in steps of 32: zero-padded copies of B and C where the caller's differ.
   const float *Bd = B->d, *Cd = C->d;
   const bool panels = s->user_N != s->opts.N;
-  if (s->user_K != s->opts.K) {  // zero-padded copies with K rounded up to 8 (the kernels' k step)
+  if (s->user_K != s->opts.K) {
     TF_PHASE(s, "pad_kernel (B)", st, tf::launch_pad(B->d, B->M, B->N, d->Bpad, B->M, s->opts.K, st));
     Bd = d->Bpad;
-    if (!panels) {
-      TF_PHASE(s, "pad_kernel (C)", st, tf::launch_pad(C->d, C->M, C->N, d->Cpad, s->opts.K, C->N, st));
-      Cd = d->Cpad;
+  }
+  if (!panels && (c_t || s->user_K != s->opts.K)) {
+    if (!d->Cpad) TF_HIP(hipMalloc(reinterpret_cast<void **>(&d->Cpad), (size_t)s->opts.K * s->opts.N * sizeof(float)));
+    if (c_t) TF_PHASE(s, "transpose_pad_kernel (C)", st, tf::launch_transpose_pad(C->d, C->M, C->N, 0, s->user_N, d->Cpad, s->opts.K, s->opts.N, st));
+    else TF_PHASE(s, "pad_kernel (C)", st, tf::launch_pad(C->d, C->M, C->N, d->Cpad, s->opts.K, C->N, st));
+    Cd = d->Cpad;
+  }
+  if (!panels) {
+    rc = gemm_spmm_pass(A, s, GemmPass{Bd, Cd, 0, s->opts.K, s->opts.N, D->d, acc, relu_in, 0}, flags, st);
+  } else {
+    // A width the MFMA kernels do not take: one pass per column panel of opts.N columns.  The panel of C is
+    // copied out (zero columns past N, zero rows past K), the pass writes a dense L x opts.N panel of D,
+    // and its columns are copied (or added, with TF_ACCUMULATE) into the caller's D.
+    for (int q = 0; q < s->n_panels; ++q) {
+      const int c0 = q * s->opts.N, w = std::min(s->opts.N, s->user_N - c0);
+      if (c_t)
+        TF_PHASE(s, "transpose_pad_kernel (panel of C)", st, tf::launch_transpose_pad(C->d, C->M, C->N, c0, w, d->Cpanel, s->opts.K, s->opts.N, st));
+      else
+        TF_PHASE(s, "copy_cols_kernel (panel of C)", st,
+                 tf::launch_copy_cols(C->d, C->M, C->N, c0, w, d->Cpanel, s->opts.K, s->opts.N, 0, s->opts.N, 0, st));
+      if (tf_status rc2 = gemm_spmm_pass(A, s, GemmPass{Bd, d->Cpanel, 0, s->opts.K, s->opts.N, d->Dpanel, 0, 0, 0}, flags, st)) return rc2;
+      TF_PHASE(s, "copy_cols_kernel (panel of D)", st,
+               tf::launch_copy_cols(d->Dpanel, D->M, s->opts.N, 0, w, D->d, D->M, D->N, c0, w, acc, st));
     }
   }
-  if (relu_in && !relu_on_load_ok(s)) return fail(TF_EINVAL, "tf_gemm_spmm: internal error, activation on load with a schedule that cannot apply it");
-  if (!panels) return gemm_spmm_pass(A, Bd, Cd, D, s, acc, flags, st, relu_in);
-  // A width the MFMA kernels do not take: one pass per column panel of opts.N columns.  The panel of C is
-  // copied out (zero columns past N, zero rows past K), the pass writes a dense L x opts.N panel of D,
-  // and its columns are copied (or added, with TF_ACCUMULATE) into the caller's D.
-  tf_dense panel = *D;
-  panel.d = d->Dpanel;
-  panel.N = s->opts.N;
-  panel.owns = false;
-  for (int q = 0; q < s->n_panels; ++q) {
-    const int c0 = q * s->opts.N, w = std::min(s->opts.N, s->user_N - c0);
-    TF_PHASE(s, "copy_cols_kernel (panel of C)", st,
-             tf::launch_copy_cols(C->d, C->M, C->N, c0, w, d->Cpanel, s->opts.K, s->opts.N, 0, s->opts.N, 0, st));
-    if (tf_status rc2 = gemm_spmm_pass(A, Bd, d->Cpanel, &panel, s, 0, flags, st)) return rc2;
-    TF_PHASE(s, "copy_cols_kernel (panel of D)", st,
-             tf::launch_copy_cols(d->Dpanel, D->M, s->opts.N, 0, w, D->d, D->M, D->N, c0, w, acc, st));
-  }
-  return TF_OK;
+  if (!rc && relu) TF_PHASE(s, "relu_kernel", st, tf::launch_relu(D->d, (size_t)D->M * D->N, st));
+  return rc;
 }
 
 extern "C" tf_status tf_gemm_spmm(const tf_csr *A, const tf_dense *B, const tf_dense *C, tf_dense *D,
@@ -861,8 +955,9 @@ extern "C" tf_status tf_gcn_two_layers(const tf_csr *A, const tf_dense *X, const
                                        tf_schedule *s1, tf_schedule *s2, tf_dense *hidden, unsigned flags, void *stream) {
   if (!A || !X || !W1 || !W2 || !D || !s1 || !s2) return fail(TF_EINVAL, "tf_gcn_two_layers: null argument");
   if (A->M != A->N) return fail(TF_EINVAL, "tf_gcn_two_layers: A must be square (it is %d x %d)", A->M, A->N);
-  const int H = W1->N;
-  if (W2->M != H) return fail(TF_EINVAL, "tf_gcn_two_layers: W1 has %d columns, W2 has %d rows", H, W2->M);
+  const bool w_t = (flags & TF_C_TRANSPOSED) != 0;  // both weights as torch stores a layer's: outputs x inputs
+  const int H = w_t ? W1->M : W1->N, w1_k = w_t ? W1->N : W1->M, w2_k = w_t ? W2->N : W2->M, w2_n = w_t ? W2->M : W2->N;
+  if (w2_k != H) return fail(TF_EINVAL, "tf_gcn_two_layers: W1 has %d columns, W2 has %d rows", H, w2_k);
   if (hidden && (hidden->M != A->M || hidden->N != H))
     return fail(TF_EINVAL, "tf_gcn_two_layers: hidden is %d x %d, expected %d x %d", hidden->M, hidden->N, A->M, H);
   // every check of shape and schedule before anything is allocated or run
@@ -872,15 +967,15 @@ extern "C" tf_status tf_gcn_two_layers(const tf_csr *A, const tf_dense *X, const
     return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the schedules were built for %d x %d and %d x %d patterns, A is %d x %d", s1->L, s1->M, s2->L, s2->M, A->M, A->N);
   if (s1->user_N != H) return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the first schedule was built for N = %d, W1 has %d columns", s1->user_N, H);
   if (s2->user_K != H) return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the second schedule was built for K = %d, the hidden layer has %d columns", s2->user_K, H);
-  if (X->M != A->N || X->N != s1->user_K || W1->M != s1->user_K)
-    return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the first schedule was built for K = %d, X is %d x %d and W1 has %d rows", s1->user_K, X->M, X->N, W1->M);
-  if (W2->N != s2->user_N || D->N != s2->user_N || D->M != A->M)
-    return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the second schedule was built for N = %d, W2 has %d columns and D is %d x %d", s2->user_N, W2->N, D->M, D->N);
+  if (X->M != A->N || X->N != s1->user_K || w1_k != s1->user_K)
+    return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the first schedule was built for K = %d, X is %d x %d and W1 has %d rows", s1->user_K, X->M, X->N, w1_k);
+  if (w2_n != s2->user_N || D->N != s2->user_N || D->M != A->M)
+    return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the second schedule was built for N = %d, W2 has %d columns and D is %d x %d", s2->user_N, w2_n, D->M, D->N);
   // On request (TF_FUSE_LAYERS): one launch with the hidden layer in LDS, every tile of the second schedule's two-layer
   // tiles carrying its rows through both layers (fused_gcn2_kernel).  Not the default: a tile recomputes its
   // neighbours' halo rows in both GEMMs and runs its four phases one after the other, which on the banded 262,144-row
   // pattern (K = H = N = 128) takes 0.63 ms against 0.31 ms for the two streamed launches of the composed path.
-  const bool fuse_ok = !hidden && !s2->l2_tiles.empty() && s2->user_N == s2->opts.N && s1->user_K == s1->opts.K && s1->user_K <= 256;
+  const bool fuse_ok = !hidden && !w_t && !s2->l2_tiles.empty() && s2->user_N == s2->opts.N && s1->user_K == s1->opts.K && s1->user_K <= 256;
   if ((flags & TF_FUSE_LAYERS) && !fuse_ok)
     return fail(TF_EUNSUPPORTED, "tf_gcn_two_layers: TF_FUSE_LAYERS needs a second schedule with two-layer tiles (tf_schedule_info.two_layer_tiles: "
                 "a banded pattern, widths of 32, 64 or 128), K a multiple of 8 up to 256 and no `hidden` argument");
@@ -913,14 +1008,15 @@ extern "C" tf_status tf_gcn_two_layers(const tf_csr *A, const tf_dense *X, const
       return fail(TF_ESCHEDULE, "tf_gcn_two_layers: the second schedule's hidden-layer buffer holds %zu floats, %zu are needed", s2->dev->hidden_floats, need);
     h.d = s2->dev->hidden;
   }
-  // first layer (its schedule is checked against X and W1 there), activation, second layer.  The activation is a
-  // launch of its own over the hidden layer -- unless that layer stays inside the library and the second schedule
+  // first layer (its schedule is checked against X and W1 there), activation, second layer.  The activation is part of
+  // the first layer's row products where nothing fuses and a launch of its own over the hidden layer where tiles do --
+  // unless that layer stays inside the library and the second schedule
   // streams all its rows: then the second layer's producers apply it to the hidden rows as they read them
   // (262,144-row band, K = H = N = 128: the pass over the hidden layer took 41 of the call's 343 us).
-  if (tf_status rc = tf_gemm_spmm(A, X, W1, &h, s1, flags & TF_SECOND_STREAM, stream)) return rc;
   const bool relu = (flags & TF_RELU) != 0, on_load = relu && !hidden && relu_on_load_ok(s2);
-  if (relu && !on_load) TF_HIP(tf::launch_relu(h.d, (size_t)h.M * h.N, static_cast<hipStream_t>(stream)));
-  return gemm_spmm_impl(A, &h, W2, D, s2, flags & (TF_ACCUMULATE | TF_SECOND_STREAM), stream, on_load ? 1 : 0);
+  const unsigned common = flags & (TF_SECOND_STREAM | TF_C_TRANSPOSED);
+  if (tf_status rc = tf_gemm_spmm(A, X, W1, &h, s1, common | (relu && !on_load ? TF_RELU : 0u), stream)) return rc;
+  return gemm_spmm_impl(A, &h, W2, D, s2, common | (flags & TF_ACCUMULATE), stream, on_load ? 1 : 0);
 }
 
 // ---- benchmark aid: per-launch times of the last executor call -------------------------
@@ -945,6 +1041,15 @@ extern "C" tf_status tf_schedule_get_profile(tf_schedule *s, tf_profile *out) {
     full.n = d->prof_n;
   }
   return tf::emit_out("tf_schedule_get_profile", out, full, TF_SIZE_THROUGH(tf_profile, ms));
+}
+
+// Y = A X for every row of A in order.
+static tf::RowsArgs all_rows(const tf_csr *A, const float *X, float *Y, int N) {
+  tf::RowsArgs a;
+  a.n_rows = A->M;
+  a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
+  a.X = X; a.ldx = N; a.x_rows = A->N; a.Y = Y; a.ldy = N; a.N = N;
+  return a;
 }
 
 // ---- an executor that allocates nothing ----------------------------------------------------
@@ -972,8 +1077,11 @@ extern "C" tf_status tf_spmm_spmm_noalloc(const tf_csr *A, const tf_csr *B, cons
   hipStream_t st = static_cast<hipStream_t>(stream);
   // every intermediate row is overwritten (rows without entries with zeros), so nothing of the
   // previous call's contents is read
-  TF_HIP(tf::launch_spmm_rows(nullptr, B->M, B->p, B->i, B->x, C->d, T, C->N, 0, 0, /*streaming=*/0, st));
-  TF_HIP(tf::launch_spmm_rows(nullptr, A->M, A->p, A->i, A->x, T, D->d, C->N, (flags & TF_ACCUMULATE) ? 1 : 0, 0, /*streaming=*/1, st));
+  tf::RowsArgs first = all_rows(B, C->d, T, C->N), second = all_rows(A, T, D->d, C->N);
+  second.streaming = 1;
+  second.accumulate = (flags & TF_ACCUMULATE) ? 1 : 0;
+  TF_HIP(tf::launch_spmm_rows(first, tf::RowsHow(), st));
+  TF_HIP(tf::launch_spmm_rows(second, tf::RowsHow(), st));
   return TF_OK;
 }
 
@@ -981,55 +1089,54 @@ extern "C" tf_status tf_spmm(const tf_csr *A, const tf_dense *X, tf_dense *Y, un
   if (!A || !X || !Y) return fail(TF_EINVAL, "tf_spmm: null argument");
   if (X->M != A->N || Y->M != A->M || X->N != Y->N)
     return fail(TF_EINVAL, "tf_spmm: shapes A %d x %d, X %d x %d, Y %d x %d", A->M, A->N, X->M, X->N, Y->M, Y->N);
-  TF_HIP(tf::launch_spmm_rows(nullptr, A->M, A->p, A->i, A->x, X->d, Y->d, X->N,
-                              (flags & TF_ACCUMULATE) ? 1 : 0, 0, /*streaming=*/1, static_cast<hipStream_t>(stream)));
+  tf::RowsArgs a = all_rows(A, X->d, Y->d, X->N);
+  a.streaming = 1;
+  a.accumulate = (flags & TF_ACCUMULATE) ? 1 : 0;
+  TF_HIP(tf::launch_spmm_rows(a, tf::RowsHow(), static_cast<hipStream_t>(stream)));
   return TF_OK;
 }
 
+extern "C" tf_status tf_spmm_scheduled(const tf_csr *A, const tf_dense *X, tf_dense *Y, tf_schedule *s, unsigned flags, void *stream) {
+  if (!A || !X || !Y || !s) return fail(TF_EINVAL, "tf_spmm_scheduled: null argument");
+  if (!s->rows_only) return fail(TF_ESCHEDULE, "tf_spmm_scheduled: the schedule is not one of tf_inspect_spmm");
+  if (tf_status rc = check_pattern("tf_spmm_scheduled", A, s)) return rc;
+  if (X->M != A->N || Y->M != A->M || X->N != Y->N || X->N > s->user_N)
+    return fail(TF_EINVAL, "tf_spmm_scheduled: shapes A %d x %d, X %d x %d, Y %d x %d, schedule for N up to %d", A->M, A->N, X->M, X->N, Y->M, Y->N, s->user_N);
+  if (tf_status rc = tf::ensure_device(s)) return rc;
+  s->dev->prof_n = 0;
+  return tf::run_remainder(A, s, tf::Remainder{X->d, X->N, X->N, X->M, Y->d, (flags & TF_ACCUMULATE) ? 1 : 0, (flags & TF_RELU) ? 1 : 0}, false,
+                           static_cast<hipStream_t>(stream));
+}
+
 extern "C" tf_status tf_gemm(const tf_dense *X, const tf_dense *W, tf_dense *Y, void *stream) {
+  return tf_gemm_ex(X, W, Y, nullptr, 0, stream);
+}
+
+extern "C" tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *Y, const tf_dense *mask, unsigned flags, void *stream) {
   if (!X || !W || !Y) return fail(TF_EINVAL, "tf_gemm: null argument");
-  if (X->N != W->M || Y->M != X->M || Y->N != W->N)
-    return fail(TF_EINVAL, "tf_gemm: shapes X %d x %d, W %d x %d, Y %d x %d", X->M, X->N, W->M, W->N, Y->M, Y->N);
-  const int K = X->N, N = W->N, M = X->M;
+  const bool w_t = (flags & TF_C_TRANSPOSED) != 0;
+  const int K = X->N, N = Y->N, M = X->M;
+  if ((w_t ? W->N : W->M) != K || (w_t ? W->M : W->N) != N || Y->M != M)
+    return fail(TF_EINVAL, "tf_gemm: shapes X %d x %d, W %d x %d%s, Y %d x %d", X->M, X->N, W->M, W->N, w_t ? " (transposed)" : "", Y->M, Y->N);
+  if (mask && (mask->M != M || mask->N != N)) return fail(TF_EINVAL, "tf_gemm: mask is %d x %d, Y is %d x %d", mask->M, mask->N, M, N);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (K <= 0 || N <= 0 || M <= 0) return fail(TF_EINVAL, "tf_gemm: empty operand");
-  if (K % 8 == 0 && N % 32 == 0 && N <= 256) {
-    TF_HIP(tf::launch_gemm(X->d, W->d, Y->d, nullptr, M, K, N, tf::default_compute_units(), st));
-    return TF_OK;
-  }
-  // Shapes the MFMA kernel does not take: K padded to 8 with zeros and N cut into equal panels of 32 .. 256 columns,
-  // in a workspace this library keeps per device.  It only ever grows: a call whose buffers fit allocates
-  // nothing and does not wait for the stream; a call that needs more frees and allocates (which waits for
-  // the device) and is refused while `st` is being captured into a graph.
-  const int Kp = (K + 7) / 8 * 8, n_panels = (N + 255) / 256, Wd = ((N + n_panels - 1) / n_panels + 31) / 32 * 32;
-  const size_t need[3] = {Kp != K ? (size_t)M * Kp : 0, (size_t)Kp * Wd, (size_t)M * Wd};
-  int dev = 0;
-  TF_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices) return fail(TF_EUNSUPPORTED, "tf_gemm: device ordinal %d is beyond the %d this library keeps workspaces for", dev, kMaxDevices);
-  static std::mutex mu;
-  std::lock_guard<std::mutex> lock(mu);
-  GemmWorkspace &ws = g_gemm_ws[dev];
-  for (int q = 0; q < 3; ++q) {
-    if (need[q] <= ws.floats[q]) continue;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
-      return fail(TF_EUNSUPPORTED, "tf_gemm: this shape needs a larger workspace than the library holds, which cannot be allocated while the "
-                  "stream is being captured; call it once with this shape outside the capture first");
-    (void)hipGetLastError();
-    (void)hipFree(ws.buf[q]);  // (waits for work that may still use it)
-    ws.buf[q] = nullptr;
-    ws.floats[q] = 0;
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&ws.buf[q]), need[q] * sizeof(float));
-    if (e != hipSuccess) return tf::hip_fail(e, "hipMalloc(tf_gemm workspace)");
-    ws.floats[q] = need[q];
-  }
-  float *Xp = need[0] ? ws.buf[0] : nullptr, *Wp = ws.buf[1], *Yp = ws.buf[2];
-  if (Xp) TF_HIP(tf::launch_pad(X->d, M, K, Xp, M, Kp, st));
-  for (int q = 0; q < n_panels; ++q) {
-    const int c0 = q * Wd, w = std::min(Wd, N - c0);
-    TF_HIP(tf::launch_copy_cols(W->d, K, N, c0, w, Wp, Kp, Wd, 0, Wd, 0, st));
-    TF_HIP(tf::launch_gemm(Xp ? Xp : X->d, Wp, Yp, nullptr, M, Kp, Wd, tf::default_compute_units(), st));
-    TF_HIP(tf::launch_copy_cols(Yp, M, Wd, 0, w, Y->d, M, N, c0, w, 0, st));
-  }
+  if (!w_t && !mask && row_gemm_takes(K, N))
+    TF_HIP(tf::launch_gemm(X->d, W->d, Y->d, nullptr, M, K, N, tf::default_compute_units(), st, 0));
+  else
+    TF_HIP(tf::launch_gemm_direct(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, mask ? mask->d : nullptr, tf::default_compute_units(), st));
+  return TF_OK;
+}
+
+extern "C" size_t tf_weight_grad_workspace(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return tf::plan_weight_grad(M, N, K, tf::default_compute_units()).partial_floats * sizeof(float);
+}
+
+extern "C" tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream) {
+  if (!G || !X || !Y || !workspace) return fail(TF_EINVAL, "tf_weight_grad: null argument");
+  if (G->M != X->M || Y->M != G->N || Y->N != X->N)
+    return fail(TF_EINVAL, "tf_weight_grad: shapes G %d x %d, X %d x %d, Y %d x %d", G->M, G->N, X->M, X->N, Y->M, Y->N);
+  const tf::WeightGradPlan p = tf::plan_weight_grad(G->M, G->N, X->N, tf::default_compute_units());
+  TF_HIP(tf::launch_weight_grad(p, G->d, G->N, X->d, X->N, G->M, workspace, Y->d, static_cast<hipStream_t>(stream)));
   return TF_OK;
 }

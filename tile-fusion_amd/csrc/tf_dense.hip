@@ -1,0 +1,325 @@
+// Dense products beside the two executors: Y = X W for any K, N and either storage of W, and the gradient of a
+// layer's weights, Y = G^T X, a product of small size summed over all rows.  Written for gfx950, fp32 MFMA.
+#include <hip/hip_runtime.h>
+#include <algorithm>
+
+#include "tf_internal.h"
+#include "tf_device.h"
+
+namespace tf {
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // (rows of K floats start at any multiple of 4 bytes)
+typedef float acc16 __attribute__((ext_vector_type(16)));
+typedef float acc4 __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------------------------
+// Y[q, :N] = X[rows[q], :K] * W, W stored K x N or (WT) N x K as torch stores a layer's weights, any K and N.
+// A wavefront owns 16 rows and 16 CB columns of v_mfma_f32_16x16x4_f32; KW wavefronts of a workgroup share a row
+// tile and take every KW-th step of 16 values of k each (their sums are added through LDS in a fixed order), so that
+// a product of few rows still fills the device: 3,000 rows x 500 x 32 are 376 workgroups whose wavefronts have 8
+// steps each, where one 32-row block per wavefront with all of K is 94 wavefronts of 250 MFMAs in a chain
+// (13.2 us; 3 us here).  X and W come straight from global memory -- the wavefronts of a workgroup read the same W, which L1
+// serves -- with k permuted inside a step the same way for both operands: lane (j, h) holds k = 16 s + 4 h + t for
+// MFMA t, one 16-byte load of X, and of W when it is stored N x K.  Columns are dealt to lanes CB at a time
+// (column CB j + cb to column block cb), so that a K x N stored W is loaded, and Y stored, CB floats per lane.
+// mask (of Y's shape, or null): Y = 0 where mask <= 0, the derivative of a ReLU whose output is mask.
+// ---------------------------------------------------------------------------------
+template <int CB> struct cvec { float v[CB]; };
+
+template <int CB, int KW, bool WT>
+__global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
+                                                          float *__restrict__ Y, int ldy, const int *__restrict__ rows,
+                                                          int y_by_row, int n_rows, int K, int N,
+                                                          const float *__restrict__ mask) {
+  constexpr int RT = 4 / KW;  // row tiles per workgroup
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
+  const int kw = wave % KW, rt = wave / KW;
+  const int row0 = (blockIdx.x * RT + rt) * 16, col0 = blockIdx.y * 16 * CB + CB * j;
+  const int q = min(row0 + j, n_rows - 1);
+  const float *xp = X + (size_t)(rows ? rows[q] : q) * ldx + 4 * h;
+  const float *wp[CB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const int c = min(col0 + cb, N - 1);
+    wp[cb] = WT ? W + (size_t)c * K + 4 * h : W + (size_t)(4 * h) * N + c;
+  }
+  const bool whole = col0 + CB <= N;  // this lane's CB columns exist
+  acc4 acc[CB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) acc[cb] = 0.f;
+  struct operands { f4v a, b[CB]; };
+  auto load = [&](int s) __attribute__((always_inline)) {
+    operands o;
+    o.a = *reinterpret_cast<const f4u *>(xp + 16 * s);
+    if constexpr (WT) {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) o.b[cb] = *reinterpret_cast<const f4u *>(wp[cb] + 16 * s);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const size_t at = (size_t)(16 * s + t) * N;
+        if (whole) {
+          const cvec<CB> w = *reinterpret_cast<const cvec<CB> *>(wp[0] + at);
+#pragma unroll
+          for (int cb = 0; cb < CB; ++cb) o.b[cb][t] = w.v[cb];
+        } else {
+#pragma unroll
+          for (int cb = 0; cb < CB; ++cb) o.b[cb][t] = wp[cb][at];
+        }
+      }
+    }
+    return o;
+  };
+  auto multiply = [&](const operands &o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[t], o.b[cb][t], acc[cb], 0, 0, 0);
+  };
+  const int full = K / 16;
+  if (kw < full) {
+    operands cur = load(kw);
+    for (int s = kw; s < full; s += KW) {
+      const operands nxt = load(min(s + KW, full - 1));
+      multiply(cur);
+      cur = nxt;
+    }
+  }
+  if (K % 16 != 0 && full % KW == kw) {  // the last step: values of k past K are zeros in both operands
+    operands o;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bool in = 16 * full + 4 * h + t < K;
+      o.a[t] = in ? xp[16 * full + t] : 0.f;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) o.b[cb][t] = in ? (WT ? wp[cb][16 * full + t] : wp[cb][(size_t)(16 * full + t) * N]) : 0.f;
+    }
+    multiply(o);
+  }
+  if constexpr (KW > 1) {
+    __shared__ acc4 part[RT][KW - 1][CB][64];
+    if (kw > 0) {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) part[rt][kw - 1][cb][lane] = acc[cb];
+    }
+    __syncthreads();
+    if (kw > 0) return;
+#pragma unroll
+    for (int w = 0; w < KW - 1; ++w)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) acc[cb] += part[rt][w][cb][lane];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {  // register r of lane (j, h): row 4 h + r of the tile
+    const int x = row0 + 4 * h + r;
+    if (x >= n_rows) continue;
+    const size_t at = (size_t)(rows && y_by_row ? rows[x] : x) * ldy + col0;
+    if (whole) {
+      cvec<CB> out;
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) out.v[cb] = acc[cb][r];
+      if (mask) {
+        const cvec<CB> m = *reinterpret_cast<const cvec<CB> *>(mask + at);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) out.v[cb] = m.v[cb] <= 0.f ? 0.f : out.v[cb];
+      }
+      *reinterpret_cast<cvec<CB> *>(Y + at) = out;
+    } else {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+        if (col0 + cb < N) Y[at + cb] = mask && mask[at + cb] <= 0.f ? 0.f : acc[cb][r];
+    }
+  }
+}
+
+// X: n_rows x K, row stride ldx (or the rows of X that `rows` lists); Y: row q of it at q * ldy, or at rows[q] * ldy when
+// y_by_row is set.  wt: W is N x K.
+hipError_t launch_gemm_direct(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
+                              int n_rows, int K, int N, const float *mask, int compute_units, hipStream_t st) {
+  if (n_rows <= 0) return hipSuccess;
+  // Column blocks per wavefront: as many as the width has (up to four: X is then read once per 64 columns), fewer
+  // where that leaves compute units without a workgroup.  Wavefronts per row tile: one when the row tiles fill the
+  // device eight wavefronts deep, else the steps of k are shared out.
+  const long long rt = (n_rows + 15) / 16;
+  int cb = N > 32 ? 4 : N > 16 ? 2 : 1;
+  while (cb > 1 && rt * ((N + 16 * cb - 1) / (16 * cb)) < compute_units) cb /= 2;
+  const long long tiles = rt * ((N + 16 * cb - 1) / (16 * cb));
+  const int kw = tiles >= 8LL * compute_units || K <= 32 ? 1 : tiles >= 4LL * compute_units || K <= 64 ? 2 : 4;
+  const dim3 grid((unsigned)((rt + 4 / kw - 1) / (4 / kw)), (unsigned)((N + 16 * cb - 1) / (16 * cb)));
+#define CALL3(CB_, KW_, WT_) \
+  hipLaunchKernelGGL((gemm_direct_kernel<CB_, KW_, WT_>), grid, dim3(256), 0, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, mask)
+#define CALL2(CB_, KW_) do { if (wt) { CALL3(CB_, KW_, true); } else { CALL3(CB_, KW_, false); } } while (0)
+#define CALL(CB_) do { if (kw == 1) { CALL2(CB_, 1); } else if (kw == 2) { CALL2(CB_, 2); } else { CALL2(CB_, 4); } } while (0)
+  if (cb == 4) CALL(4); else if (cb == 2) CALL(2); else CALL(1);
+#undef CALL
+#undef CALL2
+#undef CALL3
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------
+// Y[n, k] = sum over m < M of G[m, n] * X[m, k]: the gradient of a layer's weights.  Both operands are read once, in
+// whole rows; a wavefront holds a 32 NB x 32 KB tile of Y (v_mfma_f32_32x32x2_f32: lane (j, h) supplies row m + h of
+// both operands) and sums its share of the rows, the four wavefronts of a workgroup are added through LDS, and
+// weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.  Column NB j + nb of G belongs to
+// column block nb (and KB j + kb of X to kb), so that a lane loads adjacent columns; a lane whose columns would
+// reach past the last one works on the last NB (KB) instead, which writes some values of Y twice, the same.
+// Bound: the rows of X and G from HBM, or fp32 MFMA when 2 N K / 4 (N + K) exceeds 31 FLOP per byte.
+// ---------------------------------------------------------------------------------
+constexpr int kWgUnroll = 4;  // pairs of rows in flight per wavefront
+
+template <int NB, int KB>
+__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__restrict__ G, int N, const float *__restrict__ X,
+                                                             int K, int M, int rows_per_group, int k_chunks,
+                                                             float *__restrict__ partial) {
+  constexpr int T = NB * KB;
+  __shared__ acc16 red[2][T][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 32, h = lane / 32;
+  const int nc = blockIdx.y / k_chunks, kc = blockIdx.y % k_chunks;
+  const float *gp = G + min(nc * 32 * NB + NB * j, N - NB);
+  const float *xp = X + min(kc * 32 * KB + KB * j, K - KB);
+  const int m_end = min(M, (int)(blockIdx.x + 1) * rows_per_group);
+  acc16 acc[NB][KB];
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int b = 0; b < KB; ++b) acc[a][b] = 0.f;
+  struct operands { cvec<NB> g[kWgUnroll]; cvec<KB> x[kWgUnroll]; };
+  auto load = [&](int m0) __attribute__((always_inline)) {
+    operands o;
+#pragma unroll
+    for (int u = 0; u < kWgUnroll; ++u) {
+      const size_t m = min(m0 + 2 * u + h, M - 1);
+      o.g[u] = *reinterpret_cast<const cvec<NB> *>(gp + m * N);
+      o.x[u] = *reinterpret_cast<const cvec<KB> *>(xp + m * K);
+    }
+    return o;
+  };
+  auto multiply = [&](const operands &o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kWgUnroll; ++u)
+#pragma unroll
+      for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int b = 0; b < KB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.g[u].v[a], o.x[u].v[b], acc[a][b], 0, 0, 0);
+  };
+  constexpr int S = 2 * kWgUnroll;  // rows per step
+  int m = blockIdx.x * rows_per_group + wave * S;
+  if (m < m_end) {
+    operands cur = load(m);
+    for (; m + S <= m_end; m += 4 * S) {
+      const operands nxt = load(m + 4 * S < m_end ? m + 4 * S : m);
+      multiply(cur);
+      cur = nxt;
+    }
+    if (m < m_end) {  // rows past the group's last one are zeros in both operands
+#pragma unroll
+      for (int u = 0; u < kWgUnroll; ++u)
+        if (m + 2 * u + h >= m_end) {
+#pragma unroll
+          for (int a = 0; a < NB; ++a) cur.g[u].v[a] = 0.f;
+#pragma unroll
+          for (int b = 0; b < KB; ++b) cur.x[u].v[b] = 0.f;
+        }
+      multiply(cur);
+    }
+  }
+#pragma unroll
+  for (int half = 2; half >= 1; half /= 2) {
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int b = 0; b < KB; ++b) red[wave - half][a * KB + b][lane] = acc[a][b];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int b = 0; b < KB; ++b) acc[a][b] += red[wave][a * KB + b][lane];
+    }
+    __syncthreads();
+  }
+  if (wave == 0) {  // partial[group][chunk][tile][register][lane]
+    float *out = partial + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * (T * 1024) + lane;
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int b = 0; b < KB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[((a * KB + b) * 16 + r) * 64] = acc[a][b][r];
+  }
+}
+
+// Adds the groups' tiles: one workgroup per register of a tile, the groups dealt to its four wavefronts.
+__global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float *__restrict__ partial, int groups, int chunks,
+                                                                 int k_chunks, int NB, int KB, int N, int K,
+                                                                 float *__restrict__ Y) {
+  __shared__ float red[3][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 32, h = lane / 32;
+  const int T = NB * KB, chunk = blockIdx.y, reg = blockIdx.x;
+  const float *p = partial + (size_t)chunk * (T * 1024) + reg * 64 + lane;
+  const size_t stride = (size_t)chunks * (T * 1024);
+  float s = 0.f;
+  int g = wave;
+  for (; g + 12 < groups; g += 16) {
+    const float a = p[(size_t)g * stride], b = p[(size_t)(g + 4) * stride], c = p[(size_t)(g + 8) * stride], d = p[(size_t)(g + 12) * stride];
+    s += (a + b) + (c + d);
+  }
+  for (; g < groups; g += 4) s += p[(size_t)g * stride];
+  if (wave > 0) red[wave - 1][lane] = s;
+  __syncthreads();
+  if (wave > 0) return;
+  s += red[0][lane];
+  s += red[1][lane];
+  s += red[2][lane];
+  const int r = reg % 16, kb = (reg / 16) % KB, nb = reg / 16 / KB;
+  const int i = 8 * (r / 4) + 4 * h + r % 4;  // row of the 32 x 32 block that register r of lane (j, h) holds
+  const int n = min(chunk / k_chunks * 32 * NB + NB * i, N - NB) + nb, k = min(chunk % k_chunks * 32 * KB + KB * j, K - KB) + kb;
+  Y[(size_t)n * K + k] = s;
+}
+
+// How launch_weight_grad cuts the product: chunks of Y, groups of rows.
+WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
+  WeightGradPlan p;
+  p.nb = N > 32 ? 2 : 1;
+  p.n_chunks = (N + 32 * p.nb - 1) / (32 * p.nb);
+  // the width of X in the fewest chunks of at most 160 columns, evenly (300 = 2 x 160, 128 = 1 x 128, 500 = 4 x 128)
+  p.k_chunks = (K + 159) / 160;
+  p.kb = std::max(1, std::min(5, (K + 32 * p.k_chunks - 1) / (32 * p.k_chunks)));
+  if (p.kb > K) p.kb = 1;
+  p.k_chunks = (K + 32 * p.kb - 1) / (32 * p.kb);
+  const int chunks = p.n_chunks * p.k_chunks;
+  // two workgroups per compute unit; a group has 32 rows or more (one step of its four wavefronts)
+  const int want = std::max(1, 2 * compute_units / chunks);
+  p.rows_per_group = std::max(32, (((M + want - 1) / want) + 31) / 32 * 32);
+  p.groups = (M + p.rows_per_group - 1) / p.rows_per_group;
+  p.partial_floats = (size_t)p.groups * chunks * p.nb * p.kb * 1024;
+  return p;
+}
+
+hipError_t launch_weight_grad(const WeightGradPlan &p, const float *G, int N, const float *X, int K, int M, float *partial, float *Y, hipStream_t st) {
+  const int chunks = p.n_chunks * p.k_chunks;
+  const dim3 grid(p.groups, chunks);
+#define CALL2(NB_, KB_) \
+  hipLaunchKernelGGL((weight_grad_kernel<NB_, KB_>), grid, dim3(256), 0, st, G, N, X, K, M, p.rows_per_group, p.k_chunks, partial)
+#define CALL(NB_)                                                                  \
+  do {                                                                             \
+    switch (p.kb) {                                                                \
+      case 1: CALL2(NB_, 1); break; case 2: CALL2(NB_, 2); break; case 3: CALL2(NB_, 3); break; \
+      case 4: CALL2(NB_, 4); break; default: CALL2(NB_, 5); break;                 \
+    }                                                                              \
+  } while (0)
+  if (p.nb == 2) CALL(2); else CALL(1);
+#undef CALL
+#undef CALL2
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3(p.nb * p.kb * 16, chunks), dim3(256), 0, st, partial, p.groups, chunks, p.k_chunks,
+                     p.nb, p.kb, N, K, Y);
+  return hipGetLastError();
+}
+
+}  // namespace tf

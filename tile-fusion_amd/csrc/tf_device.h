@@ -87,25 +87,6 @@ template <int V> struct GlobalRows {
   __device__ __forceinline__ fvec<V> load(int row) const {
     return *reinterpret_cast<const fvec<V> *>(base + (size_t)row * ld + coff);
   }
-  // A column index whose top bit is set names a row the schedule expects no second reader to find in L2
-  // ("cold"): it is fetched with a streaming load, so that it does not push a row with readers out.
-  __device__ __forceinline__ fvec<V> load_flagged(int c) const {
-    const float *p = base + (size_t)(c & INT_MAX) * ld + coff;
-    fvec<V> r;
-    if (c < 0) {
-      if constexpr (V == 1) {
-        r.v[0] = __builtin_nontemporal_load(p);
-      } else {
-        typedef float fv __attribute__((ext_vector_type(V)));
-        const fv x = __builtin_nontemporal_load(reinterpret_cast<const fv *>(p));
-#pragma unroll
-        for (int u = 0; u < V; ++u) r.v[u] = x[u];
-      }
-    } else {
-      r = *reinterpret_cast<const fvec<V> *>(p);
-    }
-    return r;
-  }
 };
 template <int V> struct LdsRows {
   const float *base;  // slab; row r of the intermediate is at (r - first) * ld

@@ -96,8 +96,8 @@ extern "C" uint64_t tf_pattern_hash(int M, const int *Ap, const int *Ai) {
   return h ? h : 1;
 }
 
-extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
-                                const tf_inspect_opts *user, tf_schedule **out) {
+// rows_only: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, bool rows_only, tf_schedule **out) {
   if (!out) return tf::fail(TF_EINVAL, "tf_inspect: out is null");
   *out = nullptr;
   if (L <= 0 || M <= 0 || !Ap || !user) return tf::fail(TF_EINVAL, "tf_inspect: bad L/M/Ap/opts");
@@ -132,7 +132,7 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
     n_panels = (o.N + 255) / 256;
     o.N = ((o.N + n_panels - 1) / n_panels + 31) / 32 * 32;
   }
-  if ((long long)std::max(L, M) * o.N > INT_MAX)  // (the width the kernels see: a panel's, when N is cut into panels)
+  if (!rows_only && (long long)std::max(L, M) * o.N > INT_MAX)  // (the width the kernels see: a panel's, when N is cut into panels)
     return tf::fail(TF_EUNSUPPORTED, "tf_inspect: rows*N exceeds int32 indexing");
   // The MFMA kernels walk k in steps of 8: a K that is not a multiple of 8 is rounded up here and
   // the executor pads B's columns and C's rows with zeros into its workspace on every call.
@@ -182,7 +182,7 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
   // (the register-W tile kernel also keeps 16 bytes per fused row behind the slab)
   const int row_bytes = gemm_regw ? (o.N + 4) * 4 + 16 : o.N * 4;
   const int p_max = (o.lds_budget_bytes - staging) / row_bytes;
-  if (p_max < 8)
+  if (p_max < 8 && !rows_only)
     return tf::fail(TF_EINVAL, "tf_inspect: LDS budget %d holds only %d intermediate rows of N=%d behind %d bytes of staging",
                     o.lds_budget_bytes, std::max(p_max, 0), o.N, staging);
   if (o.strip_cols <= 0) o.strip_cols = 32;
@@ -211,10 +211,11 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
     S->L = L;
     S->M = M;
     S->nnz = nnz;
-    S->pattern_hash = tf_pattern_hash(L, Ap, Ai);
+    S->pattern_hash = given.pattern_hash ? given.pattern_hash : tf_pattern_hash(L, Ap, Ai);
     S->gemm_kc = gemm_kc;
     S->user_K = user_K;
     S->user_N = user_N;
+    S->rows_only = rows_only;
     S->n_panels = n_panels;
     S->gemm_regw = gemm_regw;
     S->gemm_stream = gemm_stream;
@@ -365,7 +366,7 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
     auto never = [&](int i) { return reach_hi(i) - reach_lo(i) > p_max; };
 
     int slab_rows = windowed ? S->slab_rows : 0;
-    int s = windowed ? M : 0;
+    int s = windowed || rows_only ? M : 0;
 
     // ---- streamed runs (GeMM-SpMM, C in registers) ----------------------------------------
     // One run per compute unit.  A run produces the rows [prod_begin, prod_end) in steps of 64
@@ -497,7 +498,8 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
     std::vector<char> need(M, 0);
     for (int i = 0; i < L; ++i) {
       if (fused[i]) { S->fused_nnz += Ap[i + 1] - Ap[i]; continue; }
-      for (int k = Ap[i]; k < Ap[i + 1]; ++k) need[Ai[k]] = 1;
+      if (!rows_only)
+        for (int k = Ap[i]; k < Ap[i + 1]; ++k) need[Ai[k]] = 1;
       const int len = Ap[i + 1] - Ap[i];
       if (len > o.long_row_nnz) {
         tf::LongRow lr{i, (int)S->long_chunks.size(), 0, 0};
@@ -685,11 +687,15 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
       // not simply all rows in order gets its rows stored side by side in list order, so that a
       // workgroup reads one stretch of columns and values instead of one stretch per row.
       if (!S->rem_identity && !S->rem_rows.empty() && o.reorder_adjacency >= 0) {
-        S->rem_ptr.reserve(S->rem_rows.size() + 1);
-        S->rem_ptr.push_back(0);
-        for (int i : S->rem_rows) {
-          for (int k = Ap[i]; k < Ap[i + 1]; ++k) { S->rem_col.push_back(Ai[k]); S->rem_src.push_back(k); }
-          S->rem_ptr.push_back((int)S->rem_col.size());
+        S->rem_ptr.resize(S->rem_rows.size() + 1);
+        S->rem_ptr[0] = 0;
+        for (size_t q = 0; q < S->rem_rows.size(); ++q) S->rem_ptr[q + 1] = S->rem_ptr[q] + Ap[S->rem_rows[q] + 1] - Ap[S->rem_rows[q]];
+        S->rem_col.resize(S->rem_ptr.back());
+        S->rem_src.resize(S->rem_ptr.back());
+        for (size_t q = 0; q < S->rem_rows.size(); ++q) {
+          const int k0 = Ap[S->rem_rows[q]], n = S->rem_ptr[q + 1] - S->rem_ptr[q];
+          std::copy(Ai + k0, Ai + k0 + n, S->rem_col.begin() + S->rem_ptr[q]);
+          std::iota(S->rem_src.begin() + S->rem_ptr[q], S->rem_src.begin() + S->rem_ptr[q + 1], k0);
         }
         // Gathers that are not expected to find their row in L2 are marked (top bit of the column): the row kernel
         // fetches those with streaming loads, so that they do not push out the rows that have readers.  On a
@@ -733,16 +739,14 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
     S->xcd_chunk_rows = o.xcd_chunk_rows;
 
     // Tiles that fuse nothing are not launched as tiles: the intermediate rows they own go to
-    // the row kernels (plain SpMM / GEMM), and only those some remainder row reads.  A GEMM
-    // whose weight does not fit LDS has no row-list form; such tiles stay tiles.
-    const bool plain_ok = o.op == TF_OP_SPMM_SPMM || (long long)o.K * o.N * 4 <= 131072;
+    // the row kernels (plain SpMM / GEMM), and only those some remainder row reads.
     for (auto &t : S->tiles) {
       int a = -1, b = -1, cnt = 0;
       for (int r = t.own_begin; r < t.own_end; ++r)
         if (need[r]) { if (a < 0) a = r; b = r + 1; ++cnt; }
       if (a >= 0) { t.wb_begin = a; t.wb_end = b; }
       const bool fuses = t.cons_end > t.cons_begin;
-      if (fuses || !plain_ok) {
+      if (fuses) {
         S->launch_tiles.push_back(t);
         if (gemm_stream) S->launch_step.push_back(S->tile_step[&t - S->tiles.data()]);
         if (a >= 0) S->n_writeback_rows += b - a;
@@ -807,6 +811,11 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
         (o.K == 32 || o.K == 64 || o.K == 128) && (o.N == 32 || o.N == 64 || o.N == 128))
       build_two_layer_tiles(S, M, Ap, Ai, o.K, o.N, o.compute_units);
 
+    if (rows_only) {
+      *out = S;
+      return TF_OK;
+    }
+
     // MultiDimensionalSet-layout view (Fusion_Inspector.h:959-1010).
     const int nt = (int)S->tiles.size();
     std::vector<int> rem_all;
@@ -857,6 +866,19 @@ extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai,
   }
   *out = S;
   return TF_OK;
+}
+
+extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, tf_schedule **out) {
+  return inspect(L, M, Ap, Ai, user, false, out);
+}
+
+extern "C" tf_status tf_inspect_spmm(int L, int M, const int *Ap, const int *Ai, int N, uint64_t pattern_hash, tf_schedule **out) {
+  tf_inspect_opts o{};
+  o.struct_size = sizeof(o);
+  o.op = TF_OP_SPMM_SPMM;
+  o.N = N;
+  o.pattern_hash = pattern_hash;
+  return inspect(L, M, Ap, Ai, &o, true, out);
 }
 
 extern "C" void tf_schedule_free(tf_schedule *s) {

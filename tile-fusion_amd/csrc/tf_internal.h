@@ -46,6 +46,39 @@ static_assert(sizeof(Tile2) == 32, "Tile2 is read as two int4 by the kernel");
 constexpr int kTile2Pad = 4;                 // floats behind every slab row (tf_gcn2.hip: kG2Pad)
 constexpr int kTile2StageFloats = 2 * 64 * 36;  // the two staging buffers of X (tf_gcn2.hip: kG2StageFloats)
 
+// Operands of the row kernel (tf_rows.hip).  Y[i,:] (+)= sum over row r's entries of Ax[k] * X[Ai[k],:], i = rows[q] (q without
+// a list), r = q with `compact`, else i.
+struct RowsArgs {
+  const int *rows = nullptr;
+  int n_rows = 0;
+  const int *Ap = nullptr, *Ai = nullptr;
+  const float *Ax = nullptr, *X = nullptr;
+  int ldx = 0;
+  unsigned x_rows = 0;  // rows of X
+  float *Y = nullptr;
+  int ldy = 0, N = 0;
+  int accumulate = 0, streaming = 0, compact = 0, relu = 0;
+  // chunks of long rows, a workgroup each; slot < 0: the row's only chunk, which goes straight to Y
+  // (their k_begin and k_end count in chunk_Ai and chunk_Ax, the matrix' own arrays)
+  const LongChunk *chunks = nullptr;
+  unsigned n_chunks = 0;
+  const int *chunk_Ai = nullptr;
+  const float *chunk_Ax = nullptr;
+  float *partial = nullptr;
+  unsigned chunk_blocks = 0;          // set by the launcher
+  int n_blocks = 0, per_xcd = 0;  // set by the launcher
+};
+struct RowsHow {
+  int xcd_chunk_rows = 0;   // how row blocks are dealt to the XCDs (tf_inspect_opts.xcd_chunk_rows)
+  int flagged = 0;          // columns carry the "cold" mark
+};
+
+// How launch_weight_grad cuts Y = G^T X (tf_dense.hip).
+struct WeightGradPlan {
+  int nb, kb, n_chunks, k_chunks, rows_per_group, groups;
+  size_t partial_floats;
+};
+
 struct DeviceSchedule;  // device copies + workspace, defined in tf_api.cpp
 
 // Marching runs: LDS layout and list format shared by the inspector, the validator and the kernel.
@@ -80,6 +113,7 @@ struct tf_schedule {
   int user_K = 0;             // K as given; opts.K is K rounded up to a multiple of 8 (what the kernels see)
   int user_N = 0;             // N as given; GeMM-SpMM with a width the MFMA kernels do not take (N % 32, N > 256) runs
   int n_panels = 1;           // as n_panels column panels of opts.N columns each, the last one zero-padded
+  bool rows_only = false;     // a schedule of tf_inspect_spmm: one product, every row in the remainder lists
   int gemm_kc = 0;            // rows of C staged in LDS per step (GeMM-SpMM)
   bool gemm_regw = false;     // GeMM-SpMM tiles keep C in registers (no staging; slab rows padded)
   int slab_ld = 0;            // floats between two slab rows of the general / GeMM-SpMM tile kernels

@@ -444,93 +444,6 @@ __global__ __launch_bounds__(kW64Block) void fused_spmm_spmm_window64_kernel(
   }
 }
 
-// ---------------------------------------------------------------------------------
-// Row-wise SpMM  Y[i,:] = sum_k Ax[k] * X[Ai[k],:]  for i = rows[q] (or i = q when rows
-// is null).  Serves the unfused remainder (X = the intermediate in HBM), producer rows
-// that no tile fuses, and tf_spmm.  One lane group per row and small, short-lived
-// workgroups: what hides the gather latency is the number of rows in flight.
-// ---------------------------------------------------------------------------------
-template <int V, int LPR, bool COAL, bool FLAG = false>
-__global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
-    const int *__restrict__ rows, int n_rows, int n_blocks, int per_xcd, const int *__restrict__ Ap,
-    const int *__restrict__ Ai, const float *__restrict__ Ax, const float *__restrict__ X, int ldx,
-    float *__restrict__ Y, int N, int accumulate, int streaming, int compact) {
-  constexpr int G = kBlock / LPR;
-  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
-  const int b = xcd_contiguous(blockIdx.x, per_xcd);
-  if (b >= n_blocks) return;
-  const int q = b * G + group;
-  if (q >= n_rows) return;  // whole lane groups leave together
-  const int i = rows ? rows[q] : q;
-  // compact: the CSR arrays hold the listed rows only, in the order of the list (the reference's
-  // reordered adjacency: consumer rows stored in schedule order), so row q of them is row rows[q] of Y
-  const int r = compact ? q : i;
-  const int kb = Ap[r], ke = Ap[r + 1];
-  for (int c0 = 0; c0 < N; c0 += LPR * V) {
-    const int coff = c0 + glane * V;
-    const bool ok = coff < N;
-    const GlobalRows<V> src{X, ldx, ok ? coff : 0};
-    fvec<V> acc = vzero<V>();
-    if (accumulate && ok) acc = *reinterpret_cast<const fvec<V> *>(Y + (size_t)i * N + coff);
-    // COAL: the group's lanes load the pairs of up to LPR entries with one coalesced request and hand
-    // them round by shuffles -- one round trip for the pairs of a long row or segment instead of one
-    // per eight entries (hot long-row segments of the R-MAT step, 22 entries on average: 0.86 -> 0.74
-    // ms).  Rows of a few entries, and segments whose gathers all miss L2, are served as well or
-    // better by every lane reading the pairs itself (cold segments 0.27 -> 0.29 ms).
-    // FLAG: column indices carry the schedule's "cold" mark in their top bit (see GlobalRows::load_flagged)
-    if constexpr (COAL) row_dot<V, LPR, GlobalRows<V>, FLAG>(Ai, Ax, kb, ke, glane, ok, src, acc);
-    else row_dot_direct<V, LPR, GlobalRows<V>, FLAG>(Ai, Ax, kb, ke, ok, src, acc);
-    if (ok) {
-      if (streaming) store_streaming<V>(Y + (size_t)i * N + coff, acc);
-      else *reinterpret_cast<fvec<V> *>(Y + (size_t)i * N + coff) = acc;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------
-// Long remainder rows.  One workgroup per chunk of a row: lane groups take LPR-entry
-// segments round-robin, partial sums are combined across the groups through LDS in a
-// fixed order, and the chunk's result goes to partial[slot].  A second kernel adds a
-// row's chunks in order, so the result does not depend on scheduling.
-// ---------------------------------------------------------------------------------
-template <int V, int LPR>
-__global__ __launch_bounds__(kBlock) void spmm_long_chunk_kernel(
-    const LongChunk *__restrict__ chunks, const int *__restrict__ Ai, const float *__restrict__ Ax,
-    const float *__restrict__ X, int ldx, float *__restrict__ partial, int N) {
-  constexpr int G = kBlock / LPR;
-  __shared__ __align__(16) float red[G * LPR * V];
-  const LongChunk ch = chunks[blockIdx.x];
-  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
-  for (int c0 = 0; c0 < N; c0 += LPR * V) {
-    const int coff = c0 + glane * V;
-    const bool ok = coff < N;
-    const GlobalRows<V> src{X, ldx, ok ? coff : 0};
-    fvec<V> acc = vzero<V>();
-    for (int k0 = ch.k_begin + group * LPR; k0 < ch.k_end; k0 += G * LPR)
-      row_dot<V, LPR>(Ai, Ax, k0, min(ch.k_end, k0 + LPR), glane, ok, src, acc);
-    *reinterpret_cast<fvec<V> *>(red + (group * LPR + glane) * V) = acc;
-    __syncthreads();
-    if (group == 0 && ok) {
-      fvec<V> sum = vzero<V>();
-      for (int g = 0; g < G; ++g) vadd<V>(*reinterpret_cast<const fvec<V> *>(red + (g * LPR + glane) * V), sum);
-      *reinterpret_cast<fvec<V> *>(partial + (size_t)ch.slot * N + coff) = sum;
-    }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void long_row_reduce_kernel(const LongRow *__restrict__ rows,
-                                                                 const float *__restrict__ partial,
-                                                                 float *__restrict__ Y, int N,
-                                                                 int accumulate) {
-  const LongRow lr = rows[blockIdx.x];
-  for (int c = threadIdx.x; c < N; c += kBlock) {
-    float s = accumulate ? Y[(size_t)lr.row * N + c] : 0.f;
-    for (int p = 0; p < lr.count; ++p) s += partial[(size_t)(lr.first + p) * N + c];
-    Y[(size_t)lr.row * N + c] = s;
-  }
-}
-
 // out[i] = val[src[i]]: the values of the rows of a list, in the order of the list.
 __global__ void gather_values_kernel(const int *__restrict__ src, const float *__restrict__ val, float *__restrict__ out, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = val[src[i]];
@@ -538,40 +451,10 @@ __global__ void gather_values_kernel(const int *__restrict__ src, const float *_
 
 // Column-partitioned long rows: out[pos[i]] = val[src[i]] puts the values of A into the order of
 // the regrouped entries (src ascending: the reads walk A's array once, the writes fall into
-// nine ascending streams), and Y[row] (+)= the row's segment sums, added in the order of its list.
+// nine ascending streams).
 __global__ void scatter_values_kernel(const int *__restrict__ src, const int *__restrict__ pos,
                                       const float *__restrict__ val, float *__restrict__ out, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[pos[i]] = val[src[i]];
-}
-
-// One lane group per long row, every lane four adjacent columns; the partial rows of eight
-// segments are requested before the first is added.
-template <int V, int LPR>
-__global__ __launch_bounds__(kBlock) void long_seg_reduce_kernel(const LongRow *__restrict__ rows, int n_long,
-                                                                 const int *__restrict__ seg_of,
-                                                                 const float *partial, float *Y, int N,
-                                                                 int accumulate) {  // (Y may be `partial` itself: other rows)
-  constexpr int G = kBlock / LPR;
-  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
-  const int q = blockIdx.x * G + group;
-  if (q >= n_long) return;
-  const LongRow lr = rows[q];
-  for (int c0 = 0; c0 < N; c0 += LPR * V) {
-    const int coff = c0 + glane * V;
-    if (coff >= N) continue;
-    fvec<V> acc = vzero<V>();
-    if (accumulate) acc = *reinterpret_cast<const fvec<V> *>(Y + (size_t)lr.row * N + coff);
-    for (int p0 = 0; p0 < lr.count; p0 += 8) {
-      fvec<V> x[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u < lr.count) x[u] = *reinterpret_cast<const fvec<V> *>(partial + (size_t)seg_of[lr.first + p0 + u] * N + coff);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u < lr.count) vadd<V>(x[u], acc);
-    }
-    *reinterpret_cast<fvec<V> *>(Y + (size_t)lr.row * N + coff) = acc;
-  }
 }
 
 // dst (rows x ld_dst) = src (src_rows x ld_src) in its top left corner, zeros elsewhere.
@@ -581,6 +464,16 @@ __global__ void pad_kernel(const float *__restrict__ src, int src_rows, int ld_s
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     const int r = (int)(i / ld_dst), c = (int)(i % ld_dst);
     dst[i] = (r < src_rows && c < ld_src) ? src[(size_t)r * ld_src + c] : 0.f;
+  }
+}
+
+// dst (rows x cols) = the transpose of the rows [row0, row0 + n_rows) of src (ld_src columns) in its top left corner, zeros
+// elsewhere: a layer's weights as torch stores them (outputs x inputs) for kernels that take K x N.
+__global__ void transpose_pad_kernel(const float *__restrict__ src, int ld_src, int row0, int n_rows, float *__restrict__ dst, int rows,
+                                     int cols) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows * cols; i += gridDim.x * blockDim.x) {
+    const int k = i / cols, n = i % cols;
+    dst[i] = (n < n_rows && k < ld_src) ? src[(size_t)(row0 + n) * ld_src + k] : 0.f;
   }
 }
 
@@ -1865,9 +1758,6 @@ inline bool xcd_remap_on() {
 }
 inline int per_xcd_of(int n) { return xcd_remap_on() ? (n + kXcds - 1) / kXcds : 0; }
 inline int grid_of(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
-// The same for chunks of `bpc` items per XCD turn (see xcd_contiguous).
-inline int chunk_bpc(int n, int bpc) { return !xcd_remap_on() ? 0 : (bpc <= 0 || bpc * kXcds >= n) ? (n + kXcds - 1) / kXcds : bpc; }
-inline int grid_chunked(int n, int bpc) { return bpc <= 0 ? grid_of(n) : (n + bpc * kXcds - 1) / (bpc * kXcds) * (bpc * kXcds); }
 
 template <class F> hipError_t allow_lds(F kernel, int bytes) {
   if (bytes <= 65536) return hipSuccess;
@@ -1967,54 +1857,9 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *tiles, const int *win
   return err != hipSuccess ? err : hipGetLastError();
 }
 
-hipError_t launch_spmm_rows(const int *rows, int n_rows, const int *Ap, const int *Ai, const float *Ax,
-                            const float *X, float *Y, int N, int accumulate, int xcd_chunk_rows,
-                            int streaming, hipStream_t st, int compact, int coalesced_pairs, int flagged) {
-  if (n_rows <= 0) return hipSuccess;
-  const Shape s = pick_shape(N);
-  if (flagged && s.V != 4) return hipErrorInvalidValue;  // (schedules mark columns only when N is a multiple of 4)
-  const int G = kBlock / s.LPR;
-  const int n_blocks = (n_rows + G - 1) / G;
-  // 0: workgroup b takes block b; > 0: chunks of rows per XCD turn; < 0: one contiguous run per XCD
-  const int bpc = xcd_chunk_rows == 0 ? 0 : chunk_bpc(n_blocks, xcd_chunk_rows > 0 ? std::max(1, xcd_chunk_rows / G) : 0);
-#define CALL3(V_, L_, COAL_, FLAG_)                                                                                   \
-  hipLaunchKernelGGL((spmm_rows_kernel<V_, L_, COAL_, FLAG_>), dim3(grid_chunked(n_blocks, bpc)), dim3(kBlock), 0, st, \
-                     rows, n_rows, n_blocks, bpc, Ap, Ai, Ax, X, N, Y, N, accumulate, streaming, compact)
-#define CALL2(V_, L_, COAL_) CALL3(V_, L_, COAL_, false)
-#define CALL(V_, L_) do { if (coalesced_pairs) { CALL2(V_, L_, true); } else { CALL2(V_, L_, false); } } while (0)
-#define CALLF(L_) do { if (coalesced_pairs) { CALL3(4, L_, true, true); } else { CALL3(4, L_, false, true); } } while (0)
-  if (flagged) {
-    if (s.LPR == 8) { CALLF(8); } else if (s.LPR == 16) { CALLF(16); } else if (s.LPR == 32) { CALLF(32); } else { CALLF(64); }
-    return hipGetLastError();
-  }
-  TF_DISPATCH_VL(s.V, s.LPR, CALL);
-#undef CALL
-#undef CALL2
-#undef CALL3
-#undef CALLF
-  return hipGetLastError();
-}
-
-hipError_t launch_long_rows(const LongChunk *chunks, int n_chunks, const LongRow *rows, int n_long,
-                            const int *Ai, const float *Ax, const float *X, float *partial, float *Y,
-                            int N, int accumulate, hipStream_t st) {
-  if (n_chunks <= 0) return hipSuccess;
-  const Shape s = pick_shape(N);
-#define CALL(V_, L_)                                                                          \
-  hipLaunchKernelGGL((spmm_long_chunk_kernel<V_, L_>), dim3(n_chunks), dim3(kBlock), 0, st,   \
-                     chunks, Ai, Ax, X, N, partial, N)
-  TF_DISPATCH_VL(s.V, s.LPR, CALL);
-#undef CALL
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(long_row_reduce_kernel, dim3(n_long), dim3(kBlock), 0, st, rows, partial, Y, N,
-                     accumulate);
-  return hipGetLastError();
-}
-
 // Long rows regrouped by column partition.  The executor runs the hot segments (an eighth per
 // XCD, in XCD order) on the row kernel with one contiguous run of segments per XCD and the cold
-// ones round-robin; these two put A's values into segment order and add up a row's segments.
+// ones round-robin; this puts A's values into segment order.
 hipError_t launch_scatter_values(const int *ent_src, const int *ent_pos, const float *Ax, float *seg_val, int n_entries,
                                  hipStream_t st) {
   if (n_entries <= 0) return hipSuccess;
@@ -2027,21 +1872,6 @@ hipError_t launch_gather_values(const int *src, const float *Ax, float *out, int
   if (n <= 0) return hipSuccess;
   const int blocks = std::min((n + kBlock - 1) / kBlock, 65536);
   hipLaunchKernelGGL(gather_values_kernel, dim3(blocks), dim3(kBlock), 0, st, src, Ax, out, n);
-  return hipGetLastError();
-}
-
-// Y[rows[q].row] (+)= the sums in partial[seg_of[first .. first + count)], in that order (Y may be
-// `partial` itself for the groups of segments of rows with many).
-hipError_t launch_seg_reduce(const LongRow *rows, int n_rows, const int *seg_of, const float *partial, float *Y, int N,
-                             int accumulate, hipStream_t st) {
-  if (n_rows <= 0) return hipSuccess;
-  const Shape s = pick_shape(N);
-  const int G = kBlock / s.LPR;
-#define CALL(V_, L_)                                                                                                \
-  hipLaunchKernelGGL((long_seg_reduce_kernel<V_, L_>), dim3((n_rows + G - 1) / G), dim3(kBlock), 0, st, rows, n_rows, \
-                     seg_of, partial, Y, N, accumulate)
-  TF_DISPATCH_VL(s.V, s.LPR, CALL);
-#undef CALL
   return hipGetLastError();
 }
 
@@ -2195,6 +2025,12 @@ hipError_t launch_pad(const float *src, int src_rows, int ld_src, float *dst, in
   if (n == 0) return hipSuccess;
   const int blocks = (int)std::min<size_t>((n + kBlock - 1) / kBlock, 65536);
   hipLaunchKernelGGL(pad_kernel, dim3(blocks), dim3(kBlock), 0, st, src, src_rows, ld_src, dst, rows, ld_dst);
+  return hipGetLastError();
+}
+
+hipError_t launch_transpose_pad(const float *src, int src_rows, int ld_src, int row0, int n_rows, float *dst, int rows, int cols, hipStream_t st) {
+  if (row0 < 0 || row0 + n_rows > src_rows || (long long)rows * cols > INT_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(transpose_pad_kernel, dim3(std::min((rows * cols + 255) / 256, 1024)), dim3(256), 0, st, src, ld_src, row0, n_rows, dst, rows, cols);
   return hipGetLastError();
 }
 

@@ -1,0 +1,386 @@
+// Row-wise SpMM  Y[i,:] = sum_k Ax[k] * X[Ai[k],:]  for gfx950: the unfused remainder of a schedule (X = the
+// intermediate in HBM), producer rows that no tile fuses, tf_spmm, and the reduction of long rows' partial sums.
+// One lane group of LPR lanes owns one row, a lane V adjacent columns of it; the stored entries are walked in CSR
+// order with one fma per element, as in the reference's AVX2 kernels
+// (fusion/src/SpMM_SpMM_vectorized.cpp:892-936).  Small, short-lived workgroups: what hides the gather latency is
+// the number of rows in flight.
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include <cstdlib>
+#include <utility>
+
+#include "tf_internal.h"
+#include "tf_device.h"
+
+namespace tf {
+
+namespace {
+
+// V floats at any multiple of four bytes: rows of N columns start anywhere when N is not a multiple of 4.
+typedef float f4 __attribute__((ext_vector_type(4)));
+template <int V> struct at4 { typedef float type __attribute__((ext_vector_type(V), aligned(4))); };
+template <> struct at4<1> { typedef float type; };
+
+template <int V> __device__ __forceinline__ fvec<V> load_any(const float *p) {
+  fvec<V> r;
+  const typename at4<V>::type x = *reinterpret_cast<const typename at4<V>::type *>(p);
+  if constexpr (V == 1) r.v[0] = x;
+  else {
+#pragma unroll
+    for (int u = 0; u < V; ++u) r.v[u] = x[u];
+  }
+  return r;
+}
+template <int V> __device__ __forceinline__ void store_any(float *p, const fvec<V> &v, bool streaming) {
+  typename at4<V>::type x;
+  if constexpr (V == 1) x = v.v[0];
+  else {
+#pragma unroll
+    for (int u = 0; u < V; ++u) x[u] = v.v[u];
+  }
+  // (written out: the compiler makes one store of the two branches and drops the hint)
+  if (streaming && V == 4) asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(p), "v"(x) : "memory");
+  else if (streaming && V == 1) asm volatile("global_store_dword %0, %1, off nt" ::"v"(p), "v"(x) : "memory");
+  else *reinterpret_cast<typename at4<V>::type *>(p) = x;
+}
+
+template <int V> struct RowsOf {
+  const float *__restrict__ base;
+  int ld;    // row stride in floats
+  int coff;  // this lane's first column
+  __device__ __forceinline__ fvec<V> load(int row) const { return load_any<V>(base + (size_t)row * ld + coff); }
+  // A column index whose top bit is set names a row the schedule expects no second reader to find in L2
+  // ("cold"): it is fetched with a streaming load, so that it does not push a row with readers out.
+  __device__ __forceinline__ fvec<V> load_flagged(int c) const {
+    const float *p = base + (size_t)(c & INT_MAX) * ld + coff;
+    if (c < 0) {
+      fvec<V> r;
+      const typename at4<V>::type x = __builtin_nontemporal_load(reinterpret_cast<const typename at4<V>::type *>(p));
+      if constexpr (V == 1) r.v[0] = x;
+      else {
+#pragma unroll
+        for (int u = 0; u < V; ++u) r.v[u] = x[u];
+      }
+      return r;
+    }
+    return load_any<V>(p);
+  }
+};
+
+// ---- the walk over a row's entries with the pairs handed round by DPP ----------------------------------
+//
+// Each lane loads one (column, value) pair of up to E = min(LPR, 16) consecutive entries (E = 4 for groups of 4 and 8 lanes),
+// turns the column into the row's byte offset, and the other lanes of the group get both through a DPP broadcast that is
+// the operand of the instruction that needs it: an entry costs one v_add_u32 (its gather's offset), one gather and four
+// v_fmac_f32.  When every lane reads the pairs itself, the redundant copies are a third of what L1 returns, and every
+// entry of a batch has a branch around its load.  Entries past a row's end take an offset past the end of X, for which a
+// buffer load returns zeros without a memory access: no branches, and fma(0, 0, acc) leaves the sum as it is.  X may have up
+// to 2 GB (32-bit offsets).
+template <int E, int L> struct group_bcast;  // lane L of the 16 (E = 16), of the quad (E = 4), of the pair (E = 2)
+#define TF_GROUP_BCAST(E_, CTRL)                                                                                       \
+  template <int L> struct group_bcast<E_, L> {                                                                         \
+    static __device__ __forceinline__ unsigned add(unsigned off, unsigned lane_off) {                                  \
+      unsigned r;                                                                                                      \
+      asm("s_nop 1\n\tv_add_u32_dpp %0, %1, %2 " CTRL(3) " row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(off), "v"(lane_off), "n"(L), "n"(L + 2)); \
+      return r;                                                                                                        \
+    }                                                                                                                  \
+    static __device__ __forceinline__ void fma(float val, const f4 &x, fvec<4> &acc) {                                 \
+      asm("s_nop 1\n\t"                                                                                                \
+          "v_fmac_f32_dpp %0, %4, %5 " CTRL(9) " row_mask:0xf bank_mask:0xf\n\t"                                       \
+          "v_fmac_f32_dpp %1, %4, %6 " CTRL(9) " row_mask:0xf bank_mask:0xf\n\t"                                       \
+          "v_fmac_f32_dpp %2, %4, %7 " CTRL(9) " row_mask:0xf bank_mask:0xf\n\t"                                       \
+          "v_fmac_f32_dpp %3, %4, %8 " CTRL(9) " row_mask:0xf bank_mask:0xf"                                           \
+          : "+v"(acc.v[0]), "+v"(acc.v[1]), "+v"(acc.v[2]), "+v"(acc.v[3])                                             \
+          : "v"(val), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "n"(L), "n"(L + 2));                                 \
+    }                                                                                                                  \
+  }
+#define TF_ROW16(N_) "row_newbcast:%" #N_
+#define TF_QUAD(N_) "quad_perm:[%" #N_ ",%" #N_ ",%" #N_ ",%" #N_ "]"
+TF_GROUP_BCAST(16, TF_ROW16);
+TF_GROUP_BCAST(4, TF_QUAD);
+#undef TF_GROUP_BCAST
+// (a pair's other pair in the quad is another row's)
+template <int L> struct group_bcast<2, L> {
+  static __device__ __forceinline__ unsigned add(unsigned off, unsigned lane_off) {
+    unsigned r;
+    asm("s_nop 1\n\tv_add_u32_dpp %0, %1, %2 quad_perm:[%3,%3,%4,%4] row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(off), "v"(lane_off), "n"(L), "n"(L + 2));
+    return r;
+  }
+  static __device__ __forceinline__ void fma(float val, const f4 &x, fvec<4> &acc) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 quad_perm:[%9,%9,%10,%10] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %6 quad_perm:[%9,%9,%10,%10] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %7 quad_perm:[%9,%9,%10,%10] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %8 quad_perm:[%9,%9,%10,%10] row_mask:0xf bank_mask:0xf"
+        : "+v"(acc.v[0]), "+v"(acc.v[1]), "+v"(acc.v[2]), "+v"(acc.v[3])
+        : "v"(val), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "n"(L), "n"(L + 2));
+  }
+};
+
+__device__ __forceinline__ f4 buffer_gather(__amdgpu_buffer_rsrc_t x, unsigned off) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(x, (int)off, 0, 0);
+  return f4{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
+}
+
+// B entries, the pairs of entry u in lane (FIRST + u) % E of set (FIRST + u) / E.
+template <int E, int FIRST, int B, int SETS>
+__device__ __forceinline__ void dpp_batch(__amdgpu_buffer_rsrc_t X, const unsigned (&off)[SETS], const float (&val)[SETS], unsigned lane_off, fvec<4> &acc) {
+  f4 x[B];
+  [&]<int... U>(std::integer_sequence<int, U...>) __attribute__((always_inline)) {
+    ((x[U] = buffer_gather(X, group_bcast<E, (FIRST + U) % E>::add(off[(FIRST + U) / E], lane_off))), ...);
+    (group_bcast<E, (FIRST + U) % E>::fma(val[(FIRST + U) / E], x[U], acc), ...);
+  }(std::make_integer_sequence<int, B>{});
+}
+
+template <int LPR>
+__device__ __forceinline__ void row_dot_dpp(const int *__restrict__ idx, const float *__restrict__ val, int kb, int ke, int glane,
+                                            __amdgpu_buffer_rsrc_t X, unsigned row_bytes, unsigned lane_off, fvec<4> &acc) {
+  constexpr int E = LPR >= 16 ? 16 : LPR >= 4 ? 4 : 2, SETS = E == 16 ? 1 : 8 / E, STEP = E * SETS;
+  const int mine = glane % E;
+  for (int k0 = kb; k0 < ke; k0 += STEP) {
+    unsigned off[SETS];
+    float v[SETS];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      const int k = k0 + s * E + mine;
+      off[s] = 0x80000000u;
+      v[s] = 0.f;
+      if (k < ke) { off[s] = (unsigned)idx[k] * row_bytes; v[s] = val[k]; }
+    }
+    // (a branch of the wavefront: taken when some row of it has that many entries left)
+    if (__ballot(ke - k0 > 4)) dpp_batch<E, 0, 8>(X, off, v, lane_off, acc);
+    else dpp_batch<E, 0, 4>(X, off, v, lane_off, acc);
+    if constexpr (STEP == 16) {
+      if (__ballot(ke - k0 > 12)) dpp_batch<E, 8, 8>(X, off, v, lane_off, acc);
+      else if (__ballot(ke - k0 > 8)) dpp_batch<E, 8, 4>(X, off, v, lane_off, acc);
+    }
+  }
+}
+
+template <int V> __device__ __forceinline__ void relu_of(fvec<V> &v) {
+#pragma unroll
+  for (int u = 0; u < V; ++u) v.v[u] = v.v[u] < 0.f ? 0.f : v.v[u];  // (a NaN stays one)
+}
+
+// What one lane stores of a row of N columns: its V columns, or the last V when they reach past the end (two
+// lanes of a group then store some of the same values).
+template <int V> __device__ __forceinline__ int clamp_col(int c, int N) { return V == 1 ? min(c, N - 1) : min(c, N - V); }
+
+}  // namespace
+
+// ---------------------------------------------------------------------------------
+// The workgroups of a launch: first chunk_blocks for the chunks of long rows (a workgroup each; a multiple of 8,
+// those past n_chunks have nothing to do), so that the longest work starts first, then the rows.
+//
+// Chunks: the lane groups take eight entries of the chunk at a time, in turn, partial sums are combined inside a wavefront by shuffles
+// and across the wavefronts through LDS, in a fixed order.  The only chunk of a row (slot < 0) goes straight to Y, a chunk of
+// a row with several to partial[slot], which long_row_reduce_kernel adds up in order.
+//
+// How a row's entries are walked: kDpp (above), the default; kDirect, every lane reads the pairs itself, for rows of fewer
+// than four columns and for X beyond 2 GB; kMarked, the same with the schedule's "cold" mark in the columns' top bit.
+// ---------------------------------------------------------------------------------
+enum { kDirect, kMarked, kDpp };
+template <int V, int LPR, int WALK, bool CHUNKS>
+__global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
+  constexpr int G = kBlock / LPR;
+  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
+  __amdgpu_buffer_rsrc_t xr;
+  if constexpr (WALK == kDpp) xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X), 0, (int)(a.x_rows * a.ldx * 4u), 0x00020000);
+  if constexpr (CHUNKS) {
+    if (blockIdx.x < a.chunk_blocks) {
+      if (blockIdx.x >= a.n_chunks) return;
+      constexpr int kWaves = kBlock / 64, GW = 64 / LPR;  // lane groups of a wavefront
+      __shared__ fvec<V> red[kWaves][LPR];
+      const LongChunk ch = a.chunks[blockIdx.x];
+      const int wave = threadIdx.x / 64;
+      for (int c0 = 0; c0 < a.N; c0 += LPR * V) {
+        const int col = c0 + glane * V;
+        const bool ok = col < a.N;
+        const int coff = clamp_col<V>(col, a.N);
+        const RowsOf<V> src{a.X, a.ldx, coff};
+        fvec<V> acc = vzero<V>();
+        // (the direct walk: the other one beside it takes more than the 64 registers of eight wavefronts per SIMD)
+        for (int k0 = ch.k_begin + group * 8; k0 < ch.k_end; k0 += G * 8)
+          row_dot_direct<V, LPR>(a.chunk_Ai, a.chunk_Ax, k0, min(ch.k_end, k0 + 8), ok, src, acc);
+        if constexpr (GW > 1) {
+#pragma unroll
+          for (int d = LPR; d < 64; d *= 2)
+#pragma unroll
+            for (int u = 0; u < V; ++u) acc.v[u] += __shfl_xor(acc.v[u], d, 64);
+        }
+        if (wave > 0 && threadIdx.x % 64 < LPR) red[wave][glane] = acc;
+        __syncthreads();
+        if (group == 0 && ok) {
+#pragma unroll
+          for (int w = 1; w < kWaves; ++w) vadd<V>(red[w][glane], acc);
+          if (ch.slot < 0) {
+            float *y = a.Y + (size_t)ch.row * a.ldy + coff;
+            if (a.accumulate) vadd<V>(load_any<V>(y), acc);
+            if (a.relu) relu_of<V>(acc);
+            store_any<V>(y, acc, a.streaming);
+          } else {
+            store_any<V>(a.partial + (size_t)ch.slot * a.N + coff, acc, false);
+          }
+        }
+        __syncthreads();
+      }
+      return;
+    }
+  }
+  // The workgroups live for a microsecond or two: the arguments are all requested at once here, not one after the other
+  // where they are first used, and a listed row's place in Y is not waited for before its entries are.
+  asm volatile("" ::"s"(a.rows), "s"(a.Ap), "s"(a.Ai), "s"(a.Ax), "s"(a.X), "s"(a.Y), "s"(a.ldx), "s"(a.ldy), "s"(a.N), "s"(a.n_rows),
+               "s"(a.accumulate), "s"(a.streaming), "s"(a.compact), "s"(a.relu), "s"(a.n_blocks), "s"(a.per_xcd));
+  const int b = xcd_contiguous(CHUNKS ? blockIdx.x - a.chunk_blocks : blockIdx.x, a.per_xcd);
+  if (b >= a.n_blocks) return;
+  const int q = b * G + group;
+  if (q >= a.n_rows) return;  // whole lane groups leave together
+  // compact: the CSR arrays hold the listed rows only, in the order of the list (the reference's
+  // reordered adjacency: consumer rows stored in schedule order), so row q of them is row rows[q] of Y
+  int r = q, i = q;
+  if (a.rows) {
+    i = a.rows[q];
+    if (!a.compact) r = i;
+  }
+  const int kb = a.Ap[r], ke = a.Ap[r + 1];
+  for (int c0 = 0; c0 < a.N; c0 += LPR * V) {
+    const int col = c0 + glane * V;
+    const bool ok = col < a.N;
+    const int coff = clamp_col<V>(col, a.N);
+    const RowsOf<V> src{a.X, a.ldx, coff};
+    float *y = a.Y + (size_t)i * a.ldy + coff;
+    fvec<V> acc = vzero<V>();
+    if (a.accumulate && ok) acc = load_any<V>(y);
+    if constexpr (WALK == kDpp) row_dot_dpp<LPR>(a.Ai, a.Ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
+    else row_dot_direct<V, LPR, RowsOf<V>, WALK == kMarked>(a.Ai, a.Ax, kb, ke, ok, src, acc);
+    if (ok) {
+      if (a.relu) relu_of<V>(acc);
+      store_any<V>(y, acc, a.streaming);
+    }
+  }
+}
+
+// The rows with several chunks: Y[row] (+)= their partial sums, in order.
+__global__ __launch_bounds__(kBlock) void long_row_reduce_kernel(const LongRow *__restrict__ rows, const float *__restrict__ partial,
+                                                                 float *__restrict__ Y, int ldy, int N, int accumulate, int relu) {
+  const LongRow lr = rows[blockIdx.x];
+  for (int c = threadIdx.x; c < N; c += kBlock) {
+    float s = accumulate ? Y[(size_t)lr.row * ldy + c] : 0.f;
+    for (int p = 0; p < lr.count; ++p) s += partial[(size_t)(lr.first + p) * N + c];
+    Y[(size_t)lr.row * ldy + c] = relu && s < 0.f ? 0.f : s;
+  }
+}
+
+// One lane group per long row, every lane four adjacent columns; the partial rows of eight
+// segments are requested before the first is added.  (Y may be `partial` itself: other rows.)
+template <int V, int LPR>
+__global__ __launch_bounds__(kBlock) void long_seg_reduce_kernel(const LongRow *__restrict__ rows, int n_long,
+                                                                 const int *__restrict__ seg_of, const float *partial, float *Y,
+                                                                 int ldy, int N, int accumulate, int relu) {
+  constexpr int G = kBlock / LPR;
+  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
+  const int q = blockIdx.x * G + group;
+  if (q >= n_long) return;
+  const LongRow lr = rows[q];
+  for (int c0 = 0; c0 < N; c0 += LPR * V) {
+    if (c0 + glane * V >= N) continue;
+    const int coff = clamp_col<V>(c0 + glane * V, N);
+    float *y = Y + (size_t)lr.row * ldy + coff;
+    fvec<V> acc = vzero<V>();
+    if (accumulate) acc = load_any<V>(y);
+    for (int p0 = 0; p0 < lr.count; p0 += 8) {
+      fvec<V> x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u < lr.count) x[u] = load_any<V>(partial + (size_t)seg_of[lr.first + p0 + u] * N + coff);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u < lr.count) vadd<V>(x[u], acc);
+    }
+    if (relu) relu_of<V>(acc);
+    store_any<V>(y, acc, false);
+  }
+}
+
+// ---- launchers ----------------------------------------------------------------------
+
+namespace {
+
+// Lanes a row of N columns takes: V = 4 columns each (any N of four or more: a lane whose columns would reach past the
+// row's end takes the last four), one each for narrower rows.  With accumulation into a row longer than the 256 columns of
+// one pass, a last lane of a later pass must not fall back into columns the pass before has added to.
+struct RowShape { int V, LPR; };
+RowShape row_shape(int N, int accumulate) {
+  const int V = N < 4 || (accumulate && N > 256 && N % 4 != 0) ? 1 : 4;
+  int LPR = V == 1 ? (N < 4 ? 4 : 64) : 2;
+  if (V == 4)
+    while (LPR * 4 < N && LPR < 64) LPR *= 2;
+  return {V, LPR};
+}
+
+inline bool xcd_remap_on() {
+  static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
+  return on;
+}
+
+#define TF_DISPATCH_ROWS(S_, CALL)                                              \
+  do {                                                                          \
+    if (S_.V == 1) { if (S_.LPR == 4) { CALL(1, 4); } else { CALL(1, 64); } }   \
+    else if (S_.LPR == 2) { CALL(4, 2); } else if (S_.LPR == 4) { CALL(4, 4); } \
+    else if (S_.LPR == 8) { CALL(4, 8); } else if (S_.LPR == 16) { CALL(4, 16); } \
+    else if (S_.LPR == 32) { CALL(4, 32); } else { CALL(4, 64); }               \
+  } while (0)
+
+}  // namespace
+
+hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
+  if (a.n_rows <= 0 && a.n_chunks <= 0) return hipSuccess;
+  RowShape s = row_shape(a.N, a.accumulate);
+  a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
+  const int G = kBlock / s.LPR;
+  a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
+  // 0: workgroup b takes block b; > 0: chunks of rows per XCD turn; < 0: one contiguous run per XCD
+  const int n = a.n_blocks, want = how.xcd_chunk_rows > 0 ? std::max(1, how.xcd_chunk_rows / G) : 0;
+  a.per_xcd = how.xcd_chunk_rows == 0 || !xcd_remap_on() ? 0 : (want <= 0 || want * kXcds >= n) ? (n + kXcds - 1) / kXcds : want;
+  const int per = std::max(a.per_xcd, 1) * kXcds;
+  const dim3 grid(a.chunk_blocks + (n + per - 1) / per * per);
+#define CALL3(V_, L_, WALK_, CH_) hipLaunchKernelGGL((spmm_rows_kernel<V_, L_, WALK_, CH_>), grid, dim3(kBlock), 0, st, a)
+#define CALL2(V_, L_, WALK_) do { if (a.n_chunks > 0) { CALL3(V_, L_, WALK_, true); } else { CALL3(V_, L_, WALK_, false); } } while (0)
+#define CALLP(V_, L_) do { if constexpr (V_ == 4) { CALL2(V_, L_, kDpp); } } while (0)
+#define CALLD(V_, L_) CALL2(V_, L_, kDirect)
+#define CALLM(V_, L_) CALL2(V_, L_, kMarked)
+  if (how.flagged) TF_DISPATCH_ROWS(s, CALLM);
+  else if (s.V == 4 && (unsigned long long)a.x_rows * a.ldx * 4 <= 0x80000000ull) TF_DISPATCH_ROWS(s, CALLP);
+  else TF_DISPATCH_ROWS(s, CALLD);
+#undef CALLP
+#undef CALLD
+#undef CALLM
+#undef CALL2
+#undef CALL3
+  return hipGetLastError();
+}
+
+hipError_t launch_long_row_reduce(const LongRow *rows, int n_rows, const float *partial, float *Y, int ldy, int N, int accumulate,
+                                  int relu, hipStream_t st) {
+  if (n_rows <= 0) return hipSuccess;
+  hipLaunchKernelGGL(long_row_reduce_kernel, dim3(n_rows), dim3(kBlock), 0, st, rows, partial, Y, ldy, N, accumulate, relu);
+  return hipGetLastError();
+}
+
+// Y[rows[q].row] (+)= the sums in partial[seg_of[first .. first + count)], in that order (Y may be
+// `partial` itself for the groups of segments of rows with many).
+hipError_t launch_seg_reduce(const LongRow *rows, int n_rows, const int *seg_of, const float *partial, float *Y, int ldy, int N,
+                             int accumulate, int relu, hipStream_t st) {
+  if (n_rows <= 0) return hipSuccess;
+  const RowShape s = row_shape(N, accumulate);
+  const int G = kBlock / s.LPR;
+#define CALL(V_, L_)                                                                                                \
+  hipLaunchKernelGGL((long_seg_reduce_kernel<V_, L_>), dim3((n_rows + G - 1) / G), dim3(kBlock), 0, st, rows, n_rows, \
+                     seg_of, partial, Y, ldy, N, accumulate, relu)
+  TF_DISPATCH_ROWS(s, CALL);
+#undef CALL
+  return hipGetLastError();
+}
+
+}  // namespace tf
