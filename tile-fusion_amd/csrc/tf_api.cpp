@@ -92,7 +92,7 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
                                            const float *, int, float *, int, int, int, int, hipStream_t);
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
 hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
-hipError_t launch_gemm_direct(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const float *, int, hipStream_t);
+hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const float *, int, hipStream_t);
 WeightGradPlan plan_weight_grad(int, int, int, int);
 hipError_t launch_weight_grad(const WeightGradPlan &, const float *, int, const float *, int, int, float *, float *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
@@ -824,8 +824,12 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
   return tf::run_remainder(A, s, tf::Remainder{d->inter, s->opts.N, s->opts.N, s->M, D->d, acc, 0}, false, st);
 }
 
-// W as the row GEMM takes it: row-major K x N with N a multiple of 32 up to 256, K of 8, small enough for LDS.
-static bool row_gemm_takes(int K, int N) { return K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072; }
+// W as the row GEMM takes it: row-major K x N with N a multiple of 32 up to 256, K of 8, small enough for LDS.  Its 32-row
+// blocks on two wavefronts per SIMD need 256 rows per compute unit to be the faster kernel (128 x 128: 23 us at 32,000 rows
+// where launch_gemm_any takes 19, 27 at 64,000 where that takes 29, 20 at 4,000 where that takes 6).
+static bool row_gemm_takes(long long rows, int K, int N, int compute_units) {
+  return rows >= 256LL * compute_units && K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072;
+}
 
 // What a GeMM-SpMM pass reads and writes: B (M x K), C (K x N, or N x K with c_t) and D (L x N).
 struct GemmPass {
@@ -862,12 +866,12 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
     const int n_plain = (int)s->plain_rows.size();
     const int placed = s->t_pos.empty() ? 0 : 1;  // the intermediate's rows stored in the order of the list
     const bool all = n_plain == s->M && s->plain_hot == 0 && !placed;
-    const bool row_gemm = !g.c_t && ldt == g.N && row_gemm_takes(g.K, g.N);
+    const bool row_gemm = !g.c_t && ldt == g.N && row_gemm_takes(n_plain, g.K, g.N, s->opts.compute_units);
     auto gemm = [&](int first, int count) {
       const int *rows = all ? nullptr : d->plain_rows + first;
       float *Y = d->inter + (placed ? (size_t)first * ldt : 0);
       return row_gemm ? tf::launch_gemm(g.B, g.C, Y, rows, count, g.K, g.N, s->opts.compute_units, st, placed)
-                      : tf::launch_gemm_direct(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, nullptr, s->opts.compute_units, st);
+                      : tf::launch_gemm_any(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, nullptr, s->opts.compute_units, st);
     };
     if (overlap) {
       TF_PHASE(s, "gemm_rows_kernel (hot rows)", st, gemm(0, s->plain_hot));
@@ -880,7 +884,7 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
       TF_HIP(hipEventRecord(d->join, d->side));
       if (n_plain > s->plain_hot) TF_PHASE(s, "gemm_rows_kernel (other rows)", st, gemm(s->plain_hot, n_plain - s->plain_hot));
     } else {
-      TF_PHASE(s, row_gemm ? "gemm_rows_kernel" : "gemm_direct_kernel", st, gemm(0, n_plain));
+      TF_PHASE(s, row_gemm ? "gemm_rows_kernel" : "gemm_panel_kernel", st, gemm(0, n_plain));
     }
   }
   return tf::run_remainder(A, s, rem, overlap && !s->plain_rows.empty(), st);
@@ -1120,10 +1124,10 @@ extern "C" tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *
     return fail(TF_EINVAL, "tf_gemm: shapes X %d x %d, W %d x %d%s, Y %d x %d", X->M, X->N, W->M, W->N, w_t ? " (transposed)" : "", Y->M, Y->N);
   if (mask && (mask->M != M || mask->N != N)) return fail(TF_EINVAL, "tf_gemm: mask is %d x %d, Y is %d x %d", mask->M, mask->N, M, N);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (!w_t && !mask && row_gemm_takes(K, N))
+  if (!w_t && !mask && row_gemm_takes(M, K, N, tf::default_compute_units()))
     TF_HIP(tf::launch_gemm(X->d, W->d, Y->d, nullptr, M, K, N, tf::default_compute_units(), st, 0));
   else
-    TF_HIP(tf::launch_gemm_direct(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, mask ? mask->d : nullptr, tf::default_compute_units(), st));
+    TF_HIP(tf::launch_gemm_any(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, mask ? mask->d : nullptr, tf::default_compute_units(), st));
   return TF_OK;
 }
 

@@ -2,6 +2,7 @@
 // layer's weights, Y = G^T X, a product of small size summed over all rows.  Written for gfx950, fp32 MFMA.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <climits>
 
 #include "tf_internal.h"
 #include "tf_device.h"
@@ -133,11 +134,208 @@ __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restric
   }
 }
 
+// ---------------------------------------------------------------------------------
+// The same product for many rows: W (a panel of 16 V Q columns of it) in LDS, once per workgroup, row-major and padded with zeros
+// to whole steps of k and whole panels, whichever way it is stored; every wavefront walks its own run of 16-row blocks
+// with no barrier, its rows of X requested a group of kGemmAhead steps ahead (the first group before W is staged).
+// Column block (v, q) of lane j is column 16 V q + V j + v: a lane reads V adjacent values of W per k and stores V adjacent columns of
+// Y, sixteen lanes side by side.  Sixteen wavefronts per compute unit (up to 128 registers each), so that a SIMD has
+// three others to feed its matrix core while one waits: 131,072 x 300 x 64 takes 62 us (139 us with
+// every row tile reading W from L2; 33 us and 39 us for a padded copy of X in 32-row blocks).
+// Bound: X and Y from HBM for up to 64 columns, fp32 MFMA beyond.
+// ---------------------------------------------------------------------------------
+constexpr int kGemmAhead = 4;  // steps of 16 values of k per group of operands
+
+template <int V, int Q, bool WT>
+__global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
+                                                          float *__restrict__ Y, int ldy, const int *__restrict__ rows,
+                                                          int y_by_row, int n_rows, int K, int N,
+                                                          const float *__restrict__ mask) {
+  extern __shared__ __align__(16) float wlds[];
+  constexpr int P = 16 * V * Q, A = kGemmAhead;  // columns of the panel
+  const int waves = blockDim.x / 64, wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
+  const int panel0 = blockIdx.y * P, S = (K + 15) / 16, G = (S + A - 1) / A;
+  const int n_blocks = (n_rows + 15) / 16, total_waves = gridDim.x * waves, gw = blockIdx.x * waves + wave;
+  const int b0 = (int)((long long)gw * n_blocks / total_waves), b1 = (int)((long long)(gw + 1) * n_blocks / total_waves);
+  const int groups = (b1 - b0) * G;
+  struct operands { f4v a[A]; };
+  // The operands of group gi (block b0 + gi / G, steps A (gi % G) ..); groups past the last are the last again.
+  int gi_next = 0, g_next = 0, b_next = b0;
+  const float *xp = X;
+  auto row_of = [&](int b) {
+    const int q = min(b * 16 + j, n_rows - 1);
+    return X + (size_t)(rows ? rows[q] : q) * ldx + 4 * h;
+  };
+  auto load_next = [&]() __attribute__((always_inline)) {
+    operands o;
+#pragma unroll
+    for (int u = 0; u < A; ++u) {
+      const int s = min(g_next * A + u, S - 1);
+      if (16 * s + 16 <= K) {
+        o.a[u] = *reinterpret_cast<const f4u *>(xp + 16 * s);
+      } else if (K % 4 == 0) {
+        o.a[u] = 0.f;
+        if (16 * s + 4 * h < K) o.a[u] = *reinterpret_cast<const f4u *>(xp + 16 * s);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o.a[u][t] = 16 * s + 4 * h + t < K ? xp[16 * s + t] : 0.f;
+      }
+    }
+    if (++gi_next < groups && ++g_next == G) {
+      g_next = 0;
+      xp = row_of(++b_next);
+    }
+    return o;
+  };
+  operands cur, nxt;
+  if (groups > 0) {
+    xp = row_of(b0);
+    cur = load_next();
+  }
+  // W into LDS: a column's sixteen values of one step per thread and item, all requested before the first is stored
+  for (int it = threadIdx.x; it < S * P; it += blockDim.x) {
+    const int n = it % P, s = it / P, c = min(panel0 + n, N - 1);
+    const bool in = panel0 + n < N;
+    f4v v[4];
+    if (16 * s + 16 <= K) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if constexpr (WT) v[u] = *reinterpret_cast<const f4u *>(W + (size_t)c * K + 16 * s + 4 * u);
+        else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[u][t] = W[(size_t)(16 * s + 4 * u + t) * N + c];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int k = 16 * s + 4 * u + t;
+          v[u][t] = k < K ? (WT ? W[(size_t)c * K + k] : W[(size_t)k * N + c]) : 0.f;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) wlds[(16 * s + 4 * u + t) * P + n] = in ? v[u][t] : 0.f;
+  }
+  __syncthreads();
+  acc4 acc[Q][V];
+  const float *wl = wlds + 4 * h * P + V * j;
+  auto run = [&](int g, const operands &o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < A; ++u) {
+      const int s = g * A + u;
+      if (s >= S) break;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float *w = wl + (16 * s + t) * P;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          typedef float wv __attribute__((ext_vector_type(V)));
+          wv b;
+          if constexpr (V == 1) b[0] = w[16 * q]; else b = *reinterpret_cast<const wv *>(w + 16 * V * q);
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[q][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[u][t], b[v], acc[q][v], 0, 0, 0);
+        }
+      }
+    }
+  };
+  auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int x = b * 16 + 4 * h + r;
+      if (x >= n_rows) continue;
+      const size_t row = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int c = panel0 + 16 * V * q + V * j;
+        float *y = Y + row + c;
+        if (c + V <= N) {
+          cvec<V> out;
+#pragma unroll
+          for (int v = 0; v < V; ++v) out.v[v] = acc[q][v][r];
+          if (mask) {
+            const cvec<V> m = *reinterpret_cast<const cvec<V> *>(mask + row + c);
+#pragma unroll
+            for (int v = 0; v < V; ++v) out.v[v] = m.v[v] <= 0.f ? 0.f : out.v[v];
+          }
+          *reinterpret_cast<cvec<V> *>(y) = out;
+        } else {
+#pragma unroll
+          for (int v = 0; v < V; ++v)
+            if (c + v < N) y[v] = mask && mask[row + c + v] <= 0.f ? 0.f : acc[q][v][r];
+        }
+      }
+    }
+  };
+  int b = b0, g = 0;
+  auto step = [&](const operands &o) __attribute__((always_inline)) {
+    if (g == 0) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[q][v] = 0.f;
+    }
+    run(g, o);
+    if (++g == G) {
+      store(b++);
+      g = 0;
+    }
+  };
+  for (int gi = 0; gi < groups; gi += 2) {
+    nxt = load_next();
+    step(cur);
+    if (gi + 1 < groups) {
+      cur = load_next();
+      step(nxt);
+    }
+  }
+}
+
 // X: n_rows x K, row stride ldx (or the rows of X that `rows` lists); Y: row q of it at q * ldy, or at rows[q] * ldy when
 // y_by_row is set.  wt: W is N x K.
-hipError_t launch_gemm_direct(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
-                              int n_rows, int K, int N, const float *mask, int compute_units, hipStream_t st) {
+hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
+                           int n_rows, int K, int N, const float *mask, int compute_units, hipStream_t st) {
   if (n_rows <= 0) return hipSuccess;
+  // Which kernel (us, this one / one 16-row tile per wavefront, at 4,000 / 16,000 / 32,000 / 64,000 rows): copying W to LDS
+  // takes 5 us before the first product, the other kernel reads it from L2 for every row tile: 128 x 128 10.4 / 5.9,
+  // 11.9 / 13.8, 19.4 / 24.1, 29 / 41; 64 x 64 5.3 / 4.1, 5.8 / 6.0, 8.9 / 9.0, 12.9 / 15.4; 500 x 32 13.3 / 6.6,
+  // 15.6 / 12.3, 25.4 / 21.2, 39 / 54; 40 x 7 4.9 / 4.1, 4.9 / 4.3, 6.7 / 4.2, 8.5 / 5.2.  Widths are cut into panels that
+  // fit LDS (X is read once per panel).
+  const long long lds_k = (long long)(K + 15) / 16 * 16 * 4;  // bytes per column
+  int unit = N <= 16 ? 16 : N <= 32 ? 32 : N <= 64 ? 64 : N <= 96 ? 96 : 128;
+  if (N > 128) {  // equal panels
+    const int n_panels = (N + 127) / 128, w = (N + n_panels - 1) / n_panels;
+    unit = w <= 96 ? 96 : 128;
+  }
+  while (unit > 16 && lds_k * unit > 163840) unit = unit == 96 ? 64 : unit / 2;
+  const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 160LL * compute_units : 48LL * compute_units;
+  if (n_rows >= from && lds_k * unit <= 163840) {
+    const int panels = (N + unit - 1) / unit, lds = (int)(lds_k * unit), n_blocks = (n_rows + 15) / 16;
+    const int waves = n_blocks >= 16 * compute_units ? 16 : n_blocks >= 8 * compute_units ? 8 : 4;
+    const dim3 grid(std::max(1, std::min(compute_units / std::min(panels, 2), (n_blocks + waves - 1) / waves)), panels);
+    hipError_t err = hipSuccess;
+#define CALLP2(V_, Q_, WT_)                                                                                                    \
+  do {                                                                                                                         \
+    if (lds > 65536)                                                                                                           \
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_panel_kernel<V_, Q_, WT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+    if (err == hipSuccess)                                                                                                     \
+      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, mask); \
+  } while (0)
+#define CALLP(V_, Q_) do { if (wt) { CALLP2(V_, Q_, true); } else { CALLP2(V_, Q_, false); } } while (0)
+    switch (unit) {
+      case 16: CALLP(1, 1); break;
+      case 32: CALLP(2, 1); break;
+      case 64: CALLP(4, 1); break;
+      case 96: CALLP(2, 3); break;
+      default: CALLP(4, 2); break;
+    }
+#undef CALLP
+#undef CALLP2
+    return err != hipSuccess ? err : hipGetLastError();
+  }
   // Column blocks per wavefront: as many as the width has (up to four: X is then read once per 64 columns), fewer
   // where that leaves compute units without a workgroup.  Wavefronts per row tile: one when the row tiles fill the
   // device eight wavefronts deep, else the steps of k are shared out.
