@@ -1,0 +1,56 @@
+"""SpMM-SpMM of any width: windowed tiles with a ragged last strip (aligned and unaligned rows, a last strip of fewer than four
+columns, accumulation), and the patterns that run as two row products instead of in tiles or marching runs, bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import oracle_spmm_spmm, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N", [4, 5, 7, 20, 29, 31, 33, 60, 63, 65, 66, 68, 77, 127, 129, 140, 257])
+@pytest.mark.parametrize("rows", [700, 20000])
+def test_windowed_tiles_of_any_width(gpu, tf, orc, N, rows):
+    say(f"window N={N} rows={rows}")
+    A = tf.workloads.banded_random(rows, 32, 11, seed=N)
+    C = tf.workloads.uniform((rows, N), 2)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_SPMM_SPMM, N=N, inner=Ah)
+    S.validate()
+    assert S.info()["windowed"] and S.info()["wide_strips"] == 1
+    want = oracle_spmm_spmm(orc, A, A, C)
+    Cd, D = tf.DenseMatrix.from_numpy(C), tf.DenseMatrix.from_numpy(np.full((rows, N), np.nan, np.float32))
+    tf.spmm_spmm(Ah, Ah, Cd, D, S)
+    tf.device_synchronize()
+    assert np.array_equal(D.to_numpy(), want)
+    tf.spmm_spmm(Ah, Ah, Cd, D, S, accumulate=True)
+    tf.device_synchronize()
+    assert np.abs(D.to_numpy() - 2 * want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("pattern,N", [("grid2d", 24), ("grid2d", 64), ("grid3d", 64), ("grid3d", 77), ("box3d", 64), ("box3d", 3), ("hub", 40)])
+@pytest.mark.parametrize("other_inner", [False, True])
+def test_two_row_products(gpu, tf, orc, pattern, N, other_inner):
+    say(f"two products {pattern} N={N} other_inner={other_inner}")
+    w = tf.workloads
+    if pattern == "hub":
+        A = w.rmat(11, 2048 * 8, seed=4)
+    else:
+        A = {"grid2d": lambda: w.laplacian_2d(70, 45), "grid3d": lambda: w.laplacian_3d(17), "box3d": lambda: w.box_stencil_3d(15)}[pattern]()
+    B = A.copy()
+    if other_inner:
+        B.data = np.random.default_rng(1).uniform(-1, 1, B.nnz).astype(np.float32)
+    C = w.uniform((A.shape[0], N), 5)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    Bh = tf.CsrMatrix.from_scipy(B) if other_inner else Ah
+    S = tf.inspector(Ah, op=tf.OP_SPMM_SPMM, N=N, inner=Bh)
+    D = tf.DenseMatrix(A.shape[0], N)
+    S.set_profiling(True)
+    tf.spmm_spmm(Ah, Bh, tf.DenseMatrix.from_numpy(C), D, S)
+    tf.device_synchronize()
+    assert [n.split("_kernel")[0] for n, _ in S.profile() if n.startswith(("spmm_rows", "fused"))] == ["spmm_rows"] * 2
+    want = oracle_spmm_spmm(orc, A, B, C)
+    if pattern == "hub":
+        assert np.abs(D.to_numpy() - want).max() <= 1e-5 * np.abs(want).max()
+    else:
+        assert np.array_equal(D.to_numpy(), want)

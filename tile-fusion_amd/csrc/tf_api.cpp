@@ -230,7 +230,9 @@ static tf_status ensure_device(tf_schedule *s) {
   const std::vector<float> trash(64, 0.f);
   std::vector<LongChunk> chunks;
   std::vector<LongRow> summed;  // the rows that partial sums are added up for
-  if (s->march) {  // nothing but the run lists is needed on the device
+  if (s->two_passes) {  // (the lists are the other schedule's)
+    parts.reserve((size_t)s->M * s->opts.N, &d->inter);
+  } else if (s->march) {  // nothing but the run lists is needed on the device
     parts.list(s->march_runs, &d->m_runs);
     parts.list(s->march_row_ptr, &d->m_row_ptr);
     parts.list(s->march_load_ptr, &d->m_load_ptr);
@@ -356,6 +358,7 @@ struct Remainder {
   int ldt, N, rows;  // rows of T
   float *D;
   int accumulate, relu;
+  int streaming = 1;  // D is not read again by this library
 };
 static tf_status run_hot_segments(tf_schedule *s, const Remainder &r, hipStream_t st) {
   DeviceSchedule *d = s->dev;
@@ -381,7 +384,7 @@ static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder 
   a.n_rows = (int)s->rem_rows.size();
   a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
   a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = N; a.N = N;
-  a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = 1;
+  a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
   RowsHow how;
   how.xcd_chunk_rows = s->xcd_chunk_rows;
   a.chunks = d->long_chunks;
@@ -745,6 +748,15 @@ static tf_status check_common(const char *who, const tf_csr *A, const tf_dense *
   return TF_OK;
 }
 
+// Y = A X for every row of A in order.
+static tf::RowsArgs all_rows(const tf_csr *A, const float *X, float *Y, int N) {
+  tf::RowsArgs a;
+  a.n_rows = A->M;
+  a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
+  a.X = X; a.ldx = N; a.x_rows = A->N; a.Y = Y; a.ldy = N; a.N = N;
+  return a;
+}
+
 extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_dense *C, tf_dense *D,
                                   tf_schedule *s, unsigned flags, void *stream) {
   tf_status rc = check_common("tf_spmm_spmm", A, C, D, s, TF_OP_SPMM_SPMM);
@@ -759,9 +771,27 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
   tf::DeviceSchedule *d = s->dev;
   d->prof_n = 0;
   const int n_launch = (int)s->launch_tiles.size();
+  if (s->march && (B->nnz != s->inner_nnz || B->N != s->opts.inner_cols || (B->hash && B->hash != s->inner_hash)))
+    return fail(TF_ESCHEDULE, "tf_spmm_spmm: the schedule's runs were built on another inner pattern than B's");
+  if (s->two_passes) {
+    tf_schedule *rows = s->two_passes;
+    if ((rc = tf::ensure_device(rows))) return rc;
+    rows->profiling = s->profiling;
+    rows->dev->prof_n = 0;
+    const int N = s->opts.N;
+    // (the lists hold A's columns: they serve B when it has A's pattern)
+    const bool same = B == A || (B->p == A->p && B->i == A->i && B->x == A->x) || (B->hash && B->hash == s->pattern_hash);
+    if (same) {
+      rc = tf::run_remainder(B, rows, tf::Remainder{C->d, N, N, C->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
+    } else {
+      tf::RowsArgs a = all_rows(B, C->d, d->inter, N);
+      a.streaming = tf::inter_streams(s);
+      TF_PHASE(rows, "spmm_rows_kernel (intermediate rows)", st, tf::launch_spmm_rows(a, tf::RowsHow(), st));
+    }
+    if (rc) return rc;
+    return tf::run_remainder(A, rows, tf::Remainder{d->inter, N, N, s->M, D->d, acc, 0}, false, st);
+  }
   if (s->march) {
-    if (B->nnz != s->inner_nnz || B->N != s->opts.inner_cols || (B->hash && B->hash != s->inner_hash))
-      return fail(TF_ESCHEDULE, "tf_spmm_spmm: the schedule's runs were built on another inner pattern than B's");
     // The values in the order of the runs' ELL rows (the reference's reordered adjacency,
     // createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653): filled in on the first call with
     // uploaded matrices, whose device arrays never change, and on every call with wrapped ones.
@@ -1036,7 +1066,7 @@ extern "C" tf_status tf_schedule_get_profile(tf_schedule *s, tf_profile *out) {
   tf_profile full;
   std::memset(&full, 0, sizeof(full));
   if (s->dev && s->profiling) {
-    tf::DeviceSchedule *d = s->dev;
+    tf::DeviceSchedule *d = s->two_passes ? s->two_passes->dev : s->dev;
     for (int q = 0; q < d->prof_n; ++q) {
       TF_HIP(hipEventSynchronize(d->prof_ev[q][1]));
       TF_HIP(hipEventElapsedTime(&full.ms[q], d->prof_ev[q][0], d->prof_ev[q][1]));
@@ -1045,15 +1075,6 @@ extern "C" tf_status tf_schedule_get_profile(tf_schedule *s, tf_profile *out) {
     full.n = d->prof_n;
   }
   return tf::emit_out("tf_schedule_get_profile", out, full, TF_SIZE_THROUGH(tf_profile, ms));
-}
-
-// Y = A X for every row of A in order.
-static tf::RowsArgs all_rows(const tf_csr *A, const float *X, float *Y, int N) {
-  tf::RowsArgs a;
-  a.n_rows = A->M;
-  a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
-  a.X = X; a.ldx = N; a.x_rows = A->N; a.Y = Y; a.ldy = N; a.N = N;
-  return a;
 }
 
 // ---- an executor that allocates nothing ----------------------------------------------------

@@ -96,6 +96,35 @@ extern "C" uint64_t tf_pattern_hash(int M, const int *Ap, const int *Ai) {
   return h ? h : 1;
 }
 
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, bool rows_only, tf_schedule **out);
+
+// Which SpMM-SpMM schedules the executor runs as two row products instead of in their tiles, when the caller has not asked
+// for tiles of its own.
+//  * Tiles that gather C from L2 (no window in LDS): always.  A tile's rows wait for its slab between two barriers, the row
+//    kernel's do not: 16 entries in a band of 32, 50,000 rows, N = 16 / 24 / 48: 16.5 / 16.7 / 24.5 us in tiles, 10.7 /
+//    15.2 / 21.2 us as two products; 300 x 300 grid, N = 32: 48 and 19 us.
+//  * Marching runs with few rows to march over: a run walks at least two planes before its first row and the device
+//    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 18 us, 110,592 rows 33 / 39 us,
+//    2^21 rows 341 / 599 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
+//    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
+static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given, const int *Ap, const int *Ai) {
+  if (S->opts.op != TF_OP_SPMM_SPMM || S->windowed) return TF_OK;
+  bool want;
+  if (S->march)
+    want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 88000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
+  else
+    want = !S->launch_tiles.empty() && given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0;
+  if (!want) return TF_OK;
+  tf_inspect_opts o{};
+  o.struct_size = sizeof(o);
+  o.op = TF_OP_SPMM_SPMM;
+  o.N = S->opts.N;
+  o.xcd_chunk_rows = given.xcd_chunk_rows;
+  o.reorder_adjacency = given.reorder_adjacency;
+  o.pattern_hash = S->pattern_hash;
+  return inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes);
+}
+
 // rows_only: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.
 static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, bool rows_only, tf_schedule **out) {
   if (!out) return tf::fail(TF_EINVAL, "tf_inspect: out is null");
@@ -193,7 +222,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
   // (measured faster than the lane-group kernel from 1,024 to 2^20 rows of a band, so it is the
   // default wherever it applies)
   // (the kernel addresses the CSR arrays with 32-bit byte offsets and loads four entries at a time)
-  const bool want_wide = have_inner && o.N % 64 == 0 && o.inner_Ap[M] >= 4 && nnz >= 4 && o.inner_Ap[M] < (1 << 30) && nnz < (1 << 30) &&
+  // (any width of four columns and more; multiples of 32 that are not multiples of 64 have strips of their own)
+  const bool want_wide = have_inner && o.N >= 4 && (o.N % 64 == 0 || o.N % 32 != 0) && o.inner_Ap[M] >= 4 && nnz >= 4 && o.inner_Ap[M] < (1 << 30) && nnz < (1 << 30) &&
                          (o.wide_strips > 0 || (o.wide_strips == 0 && user->strip_cols <= 0 && user->lds_budget_bytes <= 0 &&
                                               user->tile_rows <= 0));
   int r_cap = o.tile_rows > 0 ? o.tile_rows : ceil_div(M, 2 * o.compute_units);
@@ -250,25 +280,38 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // unit: long matrices).  Narrow strips: 32 or 64 columns, the tile's entries staged in LDS
     // as well, two workgroups per compute unit.
     bool windowed = false, win_wide = false;
+    // column extent of every row of the inner matrix (INT_MAX / 0 for an empty row: no constraint)
+    std::vector<int> blo, bhi;
+    bool inner_ok = false;
+    if (want_wide || want_window) {
+      const int *Bp = o.inner_Ap, *Bi = o.inner_Ai;
+      inner_ok = Bp[0] == 0;
+      if (inner_ok && Bp == Ap && Bi == Ai && L == M && M == o.inner_cols) {
+        blo = lo; bhi = hi;
+        for (int r = 0; r < M; ++r)
+          if (Bp[r] == Bp[r + 1]) { blo[r] = INT_MAX; bhi[r] = 0; }
+      } else {
+        blo.resize(M); bhi.resize(M);
+        for (int r = 0; r < M && inner_ok; ++r) {
+          int a = INT_MAX, b = -1;
+          if (Bp[r + 1] < Bp[r]) { inner_ok = false; break; }
+          for (int k = Bp[r]; k < Bp[r + 1]; ++k) {
+            const int c = Bi[k];
+            if (c < 0 || c >= o.inner_cols) { inner_ok = false; break; }
+            a = std::min(a, c);
+            b = std::max(b, c);
+          }
+          blo[r] = a;
+          bhi[r] = b + 1;
+        }
+      }
+    }
     auto build_window = [&](bool wide, int wide_cap = 0) {
       const int *Bp = o.inner_Ap, *Bi = o.inner_Ai;
       const int SW = wide ? 64 : o.strip_cols;
       const int budget = wide ? (user->lds_budget_bytes > 0 ? user->lds_budget_bytes : kMaxLds) : o.lds_budget_bytes;
       const int cap = wide ? (wide_cap > 0 ? wide_cap : user->tile_rows > 0 ? user->tile_rows : std::max(64, ceil_div(M, o.compute_units))) : r_cap;
-      std::vector<int> blo(M), bhi(M);
-      bool ok = (Bp[0] == 0);
-      for (int r = 0; r < M && ok; ++r) {
-        int a = INT_MAX, b = -1;
-        if (Bp[r + 1] < Bp[r]) { ok = false; break; }
-        for (int k = Bp[r]; k < Bp[r + 1]; ++k) {
-          const int c = Bi[k];
-          if (c < 0 || c >= o.inner_cols) { ok = false; break; }
-          a = std::min(a, c);
-          b = std::max(b, c);
-        }
-        blo[r] = a;      // INT_MAX / 0 for an empty row: no constraint
-        bhi[r] = b + 1;
-      }
+      bool ok = inner_ok;
       auto a16 = [](long long x) { return (x + 15) / 16 * 16; };
       auto lds_of = [&](int P, int R, long long nz, int Wc) {
         if (wide) return a16(4LL * (P + 1)) + a16(4LL * (R + 1)) + 4LL * SW * ((long long)Wc + P);
@@ -350,6 +393,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // ---- marching runs (stencils on 3D grids: no range of consecutive rows holds a row's dependences) ----
     if (!windowed && have_inner && o.march >= 0) {
       if (tf::build_march(S, M, Ap, Ai, o.inner_Ap, o.inner_Ai, o, given)) {
+        if (tf_status rc = choose_two_passes(S, given, Ap, Ai)) { tf_schedule_free(S); return rc; }
         *out = S;
         return TF_OK;
       }
@@ -679,8 +723,14 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         }
       }
       for (int i : S->rem_rows) byc[cls(i)].push_back(i);
-      S->rem_rows.clear();
-      for (auto &v : byc) S->rem_rows.insert(S->rem_rows.end(), v.begin(), v.end());
+      // (a product of its own whose rows are nearly all of one class -- a stencil and its boundary -- stays in order too: the
+      // list costs its rows an indirection and the entries a copy; 27 points, 40^3, N = 16: 21.1 us through a list, 19.1 without)
+      size_t most = 0;
+      for (auto &v : byc) most = std::max(most, v.size());
+      if (!(rows_only && most * 8 >= S->rem_rows.size() * 7)) {
+        S->rem_rows.clear();
+        for (auto &v : byc) S->rem_rows.insert(S->rem_rows.end(), v.begin(), v.end());
+      }
       S->rem_identity = (int)S->rem_rows.size() == L;
       for (int q = 0; q < L && S->rem_identity; ++q) S->rem_identity = (S->rem_rows[q] == q);
       // Reordered adjacency (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653): a list that is
@@ -815,6 +865,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       *out = S;
       return TF_OK;
     }
+    if (tf_status rc = choose_two_passes(S, given, Ap, Ai)) { tf_schedule_free(S); return rc; }
 
     // MultiDimensionalSet-layout view (Fusion_Inspector.h:959-1010).
     const int nt = (int)S->tiles.size();
@@ -883,6 +934,7 @@ extern "C" tf_status tf_inspect_spmm(int L, int M, const int *Ap, const int *Ai,
 
 extern "C" void tf_schedule_free(tf_schedule *s) {
   if (!s) return;
+  tf_schedule_free(s->two_passes);
   tf::release_device_schedule(s->dev);
   delete s;
 }
@@ -930,7 +982,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   }
   long long ws = 0;
   if (s->march) ws += (long long)s->march_ell_off.size() * 16;  // ELL rows with values, their offsets and sources
-  if (s->n_writeback_rows > 0) ws += (long long)s->M * s->opts.N * 4;
+  if (s->n_writeback_rows > 0 || s->two_passes) ws += (long long)s->M * s->opts.N * 4;
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
   if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1 + (long long)s->seg_groups.size()) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C

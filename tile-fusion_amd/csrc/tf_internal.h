@@ -113,6 +113,9 @@ struct tf_schedule {
   int user_K = 0;             // K as given; opts.K is K rounded up to a multiple of 8 (what the kernels see)
   int user_N = 0;             // N as given; GeMM-SpMM with a width the MFMA kernels do not take (N % 32, N > 256) runs
   int n_panels = 1;           // as n_panels column panels of opts.N columns each, the last one zero-padded
+  // SpMM-SpMM: where it is faster than the tiles (see choose_two_passes in tf_inspector.cpp) the executor runs two row
+  // products through an intermediate in HBM, by this schedule of tf_inspect_spmm on A's pattern.
+  tf_schedule *two_passes = nullptr;
   bool rows_only = false;     // a schedule of tf_inspect_spmm: one product, every row in the remainder lists
   int gemm_kc = 0;            // rows of C staged in LDS per step (GeMM-SpMM)
   bool gemm_regw = false;     // GeMM-SpMM tiles keep C in registers (no staging; slab rows padded)

@@ -334,7 +334,12 @@ __device__ __forceinline__ fvec<4> row_dot_quad_regs(const QuadEntries &first, c
   return acc;
 }
 
-template <bool ACC>
+// RAGGED: N is not a multiple of 64.  In the last strip a lane whose four columns reach past N works on the last four
+// instead (some columns of the window, the slab and D are then written twice, with the same values) and lanes wholly
+// past N store nothing; rows that do not start at 16 bytes (N % 4) reach LDS through registers.  Half a strip of idle
+// lanes is cheaper than leaving the tile: 50,000 rows of 16 in a band of 32, N = 77: 170 us in tiles whose C comes from
+// L2, 35 us as two row-kernel passes, 20 us here.
+template <bool ACC, bool RAGGED>
 __global__ __launch_bounds__(kW64Block) void fused_spmm_spmm_window64_kernel(
     const TileDesc *__restrict__ tiles, const int2 *__restrict__ win, int n_tiles, int per_xcd,
     const int *__restrict__ Bp, const int *__restrict__ Bi, const float *__restrict__ Bx, int nnzB,
@@ -358,11 +363,28 @@ __global__ __launch_bounds__(kW64Block) void fused_spmm_spmm_window64_kernel(
   // a wavefront moves 64 units of 16 bytes, i.e. four window rows, to consecutive LDS addresses.
   const int wave = tid / 64, lane = tid % 64;
   auto stage_window = [&](int c0, int first_wave, int n_waves) {
+    if (RAGGED && N % 4 != 0) {
+      constexpr int U = 8;  // requests in flight per wavefront
+      for (int u0 = (wave - first_wave) * 64; u0 < n4; u0 += U * n_waves * 64) {
+        float4u x[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          const int u = min(u0 + k * n_waves * 64 + lane, n4 - 1);
+          x[k] = *reinterpret_cast<const float4u *>(C + (size_t)(w.x + u / 16) * N + min(c0 + (u % 16) * 4, N - 4));
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          const int u = u0 + k * n_waves * 64 + lane;
+          if (u < n4) *reinterpret_cast<fvec<4> *>(Cbuf + u * 4) = fvec<4>{x[k][0], x[k][1], x[k][2], x[k][3]};
+        }
+      }
+      return;
+    }
     for (int u0 = (wave - first_wave) * 64; u0 < n4; u0 += n_waves * 64) {
       const int u = u0 + lane;
       if (u < n4)
         __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void *)(C + (size_t)(w.x + u / 16) * N + c0 + (u % 16) * 4),
+            (const __attribute__((address_space(1))) void *)(C + (size_t)(w.x + u / 16) * N + (RAGGED ? min(c0 + (u % 16) * 4, N - 4) : c0 + (u % 16) * 4)),
             (__attribute__((address_space(3))) void *)(Cbuf + u0 * 4), 16, 0, 0);
     }
   };
@@ -414,24 +436,33 @@ __global__ __launch_bounds__(kW64Block) void fused_spmm_spmm_window64_kernel(
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else {
       if (R > 0) ea = fetchA(group);
-      float *dst = D + (size_t)(t.own_begin + group) * N + c0 + glane * 4;
+      const bool mine = !RAGGED || c0 + glane * 4 < N;  // this lane has columns in the strip
+      float *dst = D + (size_t)(t.own_begin + group) * N + (RAGGED ? min(c0 + glane * 4, N - 4) : c0 + glane * 4);
       const size_t round_stride = (size_t)g2 * N;
+      auto row_out = [&](const QuadEntries &e) __attribute__((always_inline)) {
+        fvec<4> acc = vzero<4>();
+        if constexpr (ACC && RAGGED) {
+          const float4u x = *reinterpret_cast<const float4u *>(dst);
+          acc = fvec<4>{x[0], x[1], x[2], x[3]};
+        } else if constexpr (ACC) {
+          acc = *reinterpret_cast<const fvec<4> *>(dst);
+        }
+        acc = row_dot_quad_regs<EXACT>(e, Ai, Ax, e.kb, e.ke, nnzA, offA, tbase, q, acc);
+        if constexpr (RAGGED) {
+          if (ACC && N - c0 < 4) {  // the strip's only lane: its other columns have been added to in the strip before
+            for (int u = 4 - (N - c0); u < 4 && mine; ++u) dst[u] = acc.v[u];
+          } else if (mine) __builtin_nontemporal_store(float4u{acc.v[0], acc.v[1], acc.v[2], acc.v[3]}, reinterpret_cast<float4u *>(dst));
+        } else {
+          store_streaming<4>(dst, acc);
+        }
+        dst += round_stride;
+      };
       for (int i = group; i < R; i += 2 * g2) {
         eb = fetchA(i + g2);
-        {
-          fvec<4> acc = vzero<4>();
-          if constexpr (ACC) acc = *reinterpret_cast<const fvec<4> *>(dst);
-          store_streaming<4>(dst, row_dot_quad_regs<EXACT>(ea, Ai, Ax, ea.kb, ea.ke, nnzA, offA, tbase, q, acc));
-          dst += round_stride;
-        }
+        row_out(ea);
         if (i + g2 >= R) break;
         ea = fetchA(i + 2 * g2);
-        {
-          fvec<4> acc = vzero<4>();
-          if constexpr (ACC) acc = *reinterpret_cast<const fvec<4> *>(dst);
-          store_streaming<4>(dst, row_dot_quad_regs<EXACT>(eb, Ai, Ax, eb.kb, eb.ke, nnzA, offA, tbase, q, acc));
-          dst += round_stride;
-        }
+        row_out(eb);
       }
     }
     lds_barrier();  // slab consumed, next window (if any) in LDS
@@ -1843,16 +1874,20 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *tiles, const int *win
   // wavefronts that fetch the next strip's window during the second product: two are enough for one
   // more strip of one tile per compute unit, four keep up when tiles or strips queue
   const int n_loaders = (n_tiles > compute_units || N > 2 * kW64Strip) ? 4 : 2;
-  if (N % kW64Strip != 0 || nnzA < 4 || nnzB < 4 || nnzA >= (1 << 30) || nnzB >= (1 << 30)) return hipErrorInvalidValue;
+  if (N < 4 || nnzA < 4 || nnzB < 4 || nnzA >= (1 << 30) || nnzB >= (1 << 30)) return hipErrorInvalidValue;
   const int per = per_xcd_of(n_tiles);
   const int2 *w2 = reinterpret_cast<const int2 *>(win);
   hipError_t err;
-#define CALL64(ACC_)                                                                                    \
-  err = allow_lds(fused_spmm_spmm_window64_kernel<ACC_>, lds_bytes);                                    \
+#define CALL64(ACC_, RAG_)                                                                              \
+  err = allow_lds(fused_spmm_spmm_window64_kernel<ACC_, RAG_>, lds_bytes);                              \
   if (err == hipSuccess)                                                                                \
-    hipLaunchKernelGGL((fused_spmm_spmm_window64_kernel<ACC_>), dim3(grid_of(n_tiles)), dim3(kW64Block), \
+    hipLaunchKernelGGL((fused_spmm_spmm_window64_kernel<ACC_, RAG_>), dim3(grid_of(n_tiles)), dim3(kW64Block), \
                        lds_bytes, st, tiles, w2, n_tiles, per, Bp, Bi, Bx, nnzB, C, Ap, Ai, Ax, nnzA, D, N, n_loaders)
-  if (accumulate) { CALL64(true); } else { CALL64(false); }
+  if (N % kW64Strip == 0) {
+    if (accumulate) { CALL64(true, false); } else { CALL64(false, false); }
+  } else {
+    if (accumulate) { CALL64(true, true); } else { CALL64(false, true); }
+  }
 #undef CALL64
   return err != hipSuccess ? err : hipGetLastError();
 }
