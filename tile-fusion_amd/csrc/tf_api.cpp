@@ -92,7 +92,7 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
                                            const float *, int, float *, int, int, int, int, hipStream_t);
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
 hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
-hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const float *, int, hipStream_t);
+hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const GemmOut &, int, hipStream_t);
 WeightGradPlan plan_weight_grad(int, int, int, int);
 hipError_t launch_weight_grad(const WeightGradPlan &, const float *, int, const float *, int, int, float *, float *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
@@ -207,7 +207,7 @@ class ArenaParts {
 
 // A GeMM-SpMM schedule in which nothing fuses is a GEMM into the intermediate and row products out of it, for which K
 // and N are what the caller has.  (Tiles take K in steps of 8 and N in steps of 32: padded copies, column panels.)
-static bool untiled(const tf_schedule *s) { return s->opts.op == TF_OP_GEMM_SPMM && s->launch_tiles.empty(); }
+static bool untiled(const tf_schedule *s) { return s->opts.op == TF_OP_GEMM_SPMM && (s->launch_tiles.empty() || s->two_passes); }
 // Floats from one row of the intermediate to the next: a multiple of 4, so that every lane's columns of a row are one
 // aligned load.
 static int inter_ld(const tf_schedule *s) { return untiled(s) ? (s->user_N + 3) / 4 * 4 : s->opts.N; }
@@ -231,7 +231,8 @@ static tf_status ensure_device(tf_schedule *s) {
   std::vector<LongChunk> chunks;
   std::vector<LongRow> summed;  // the rows that partial sums are added up for
   if (s->two_passes) {  // (the lists are the other schedule's)
-    parts.reserve((size_t)s->M * s->opts.N, &d->inter);
+    parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
+    parts.list(s->l2_tiles, &d->l2_tiles);
   } else if (s->march) {  // nothing but the run lists is needed on the device
     parts.list(s->march_runs, &d->m_runs);
     parts.list(s->march_row_ptr, &d->m_row_ptr);
@@ -901,7 +902,7 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
       const int *rows = all ? nullptr : d->plain_rows + first;
       float *Y = d->inter + (placed ? (size_t)first * ldt : 0);
       return row_gemm ? tf::launch_gemm(g.B, g.C, Y, rows, count, g.K, g.N, s->opts.compute_units, st, placed)
-                      : tf::launch_gemm_any(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, nullptr, s->opts.compute_units, st);
+                      : tf::launch_gemm_any(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, tf::GemmOut(), s->opts.compute_units, st);
     };
     if (overlap) {
       TF_PHASE(s, "gemm_rows_kernel (hot rows)", st, gemm(0, s->plain_hot));
@@ -924,7 +925,7 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
 // A schedule whose every intermediate row is produced by the streamed kernel straight from B (no padded copy, no
 // column panels, no rows left to the row GEMM) can apply an activation to B as it is read.
 static bool relu_on_load_ok(const tf_schedule *s) {
-  return s->gemm_stream && s->plain_rows.empty() && s->user_K == s->opts.K && s->user_N == s->opts.N && !s->launch_tiles.empty();
+  return s->gemm_stream && !s->two_passes && s->plain_rows.empty() && s->user_K == s->opts.K && s->user_N == s->opts.N && !s->launch_tiles.empty();
 }
 
 static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_dense *C, tf_dense *D,
@@ -944,6 +945,31 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
   tf::DeviceSchedule *d = s->dev;
   d->prof_n = 0;
   if (relu_in && !relu_on_load_ok(s)) return fail(TF_EINVAL, "tf_gemm_spmm: internal error, activation on load with a schedule that cannot apply it");
+  if (s->two_passes) {
+    tf_schedule *rows = s->two_passes;
+    if ((rc = tf::ensure_device(rows))) return rc;
+    rows->profiling = s->profiling;
+    rows->dev->prof_n = 0;
+    const int K = s->user_K, N = s->user_N, cus = s->opts.compute_units;
+    if (s->spmm_first) {
+      rc = tf::run_remainder(A, rows, tf::Remainder{B->d, K, K, B->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
+      if (rc) return rc;
+      tf::GemmOut how;
+      how.accumulate = acc;
+      how.relu = relu;
+      if (!c_t && !acc && !relu && row_gemm_takes(s->L, K, N, cus))
+        TF_PHASE(rows, "gemm_rows_kernel", st, tf::launch_gemm(d->inter, C->d, D->d, nullptr, s->L, K, N, cus, st, 0));
+      else
+        TF_PHASE(rows, "gemm_panel_kernel", st, tf::launch_gemm_any(d->inter, K, C->d, c_t, D->d, N, nullptr, 0, s->L, K, N, how, cus, st));
+      return TF_OK;
+    }
+    const int ldt = tf::inter_ld(s);
+    if (!c_t && ldt == N && row_gemm_takes(s->M, K, N, cus))
+      TF_PHASE(rows, "gemm_rows_kernel", st, tf::launch_gemm(B->d, C->d, d->inter, nullptr, s->M, K, N, cus, st, 0));
+    else
+      TF_PHASE(rows, "gemm_panel_kernel", st, tf::launch_gemm_any(B->d, K, C->d, c_t, d->inter, ldt, nullptr, 0, s->M, K, N, tf::GemmOut(), cus, st));
+    return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, relu}, false, st);
+  }
   if (tf::untiled(s)) return gemm_spmm_pass(A, s, GemmPass{B->d, C->d, c_t, s->user_K, s->user_N, D->d, acc, 0, relu}, flags, st);
   // Tiles take K in steps of 8 and N in steps of 32: zero-padded copies of B and C where the caller's differ.
   const float *Bd = B->d, *Cd = C->d;
@@ -1066,7 +1092,7 @@ extern "C" tf_status tf_schedule_get_profile(tf_schedule *s, tf_profile *out) {
   tf_profile full;
   std::memset(&full, 0, sizeof(full));
   if (s->dev && s->profiling) {
-    tf::DeviceSchedule *d = s->two_passes ? s->two_passes->dev : s->dev;
+    tf::DeviceSchedule *d = s->dev->prof_n == 0 && s->two_passes && s->two_passes->dev ? s->two_passes->dev : s->dev;
     for (int q = 0; q < d->prof_n; ++q) {
       TF_HIP(hipEventSynchronize(d->prof_ev[q][1]));
       TF_HIP(hipEventElapsedTime(&full.ms[q], d->prof_ev[q][0], d->prof_ev[q][1]));
@@ -1147,8 +1173,11 @@ extern "C" tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (!w_t && !mask && row_gemm_takes(M, K, N, tf::default_compute_units()))
     TF_HIP(tf::launch_gemm(X->d, W->d, Y->d, nullptr, M, K, N, tf::default_compute_units(), st, 0));
-  else
-    TF_HIP(tf::launch_gemm_any(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, mask ? mask->d : nullptr, tf::default_compute_units(), st));
+  else {
+    tf::GemmOut how;
+    how.mask = mask ? mask->d : nullptr;
+    TF_HIP(tf::launch_gemm_any(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, how, tf::default_compute_units(), st));
+  }
   return TF_OK;
 }
 

@@ -24,15 +24,45 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 // serves -- with k permuted inside a step the same way for both operands: lane (j, h) holds k = 16 s + 4 h + t for
 // MFMA t, one 16-byte load of X, and of W when it is stored N x K.  Columns are dealt to lanes CB at a time
 // (column CB j + cb to column block cb), so that a K x N stored W is loaded, and Y stored, CB floats per lane.
-// mask (of Y's shape, or null): Y = 0 where mask <= 0, the derivative of a ReLU whose output is mask.
 // ---------------------------------------------------------------------------------
 template <int CB> struct cvec { float v[CB]; };
+
+// The values v of CB adjacent columns at Y + at, the first `columns` of them existing ones.
+template <int CB> __device__ __forceinline__ void gemm_store(float *__restrict__ Y, size_t at, cvec<CB> v, int columns, const GemmOut &how) {
+  auto finish = [&](float x, size_t i) __attribute__((always_inline)) {
+    if (how.accumulate) x += Y[i];
+    if (how.mask) x = how.mask[i] <= 0.f ? 0.f : x;
+    if (how.relu) x = x < 0.f ? 0.f : x;
+    return x;
+  };
+  if (columns >= CB) {
+    if (how.accumulate || how.mask || how.relu) {
+      cvec<CB> m;
+      if (how.mask) m = *reinterpret_cast<const cvec<CB> *>(how.mask + at);
+      if (how.accumulate) {
+        const cvec<CB> y = *reinterpret_cast<const cvec<CB> *>(Y + at);
+#pragma unroll
+        for (int c = 0; c < CB; ++c) v.v[c] += y.v[c];
+      }
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        if (how.mask) v.v[c] = m.v[c] <= 0.f ? 0.f : v.v[c];
+        if (how.relu) v.v[c] = v.v[c] < 0.f ? 0.f : v.v[c];
+      }
+    }
+    *reinterpret_cast<cvec<CB> *>(Y + at) = v;
+  } else {
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+      if (c < columns) Y[at + c] = finish(v.v[c], at + c);
+  }
+}
 
 template <int CB, int KW, bool WT>
 __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
                                                           float *__restrict__ Y, int ldy, const int *__restrict__ rows,
                                                           int y_by_row, int n_rows, int K, int N,
-                                                          const float *__restrict__ mask) {
+                                                          const GemmOut out_how) {
   constexpr int RT = 4 / KW;  // row tiles per workgroup
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
   const int kw = wave % KW, rt = wave / KW;
@@ -116,21 +146,10 @@ __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restric
     const int x = row0 + 4 * h + r;
     if (x >= n_rows) continue;
     const size_t at = (size_t)(rows && y_by_row ? rows[x] : x) * ldy + col0;
-    if (whole) {
-      cvec<CB> out;
+    cvec<CB> out;
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) out.v[cb] = acc[cb][r];
-      if (mask) {
-        const cvec<CB> m = *reinterpret_cast<const cvec<CB> *>(mask + at);
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) out.v[cb] = m.v[cb] <= 0.f ? 0.f : out.v[cb];
-      }
-      *reinterpret_cast<cvec<CB> *>(Y + at) = out;
-    } else {
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb)
-        if (col0 + cb < N) Y[at + cb] = mask && mask[at + cb] <= 0.f ? 0.f : acc[cb][r];
-    }
+    for (int cb = 0; cb < CB; ++cb) out.v[cb] = acc[cb][r];
+    gemm_store<CB>(Y, at, out, N - col0, out_how);
   }
 }
 
@@ -150,7 +169,7 @@ template <int V, int Q, bool WT>
 __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
                                                           float *__restrict__ Y, int ldy, const int *__restrict__ rows,
                                                           int y_by_row, int n_rows, int K, int N,
-                                                          const float *__restrict__ mask) {
+                                                          const GemmOut out_how) {
   extern __shared__ __align__(16) float wlds[];
   constexpr int P = 16 * V * Q, A = kGemmAhead;  // columns of the panel
   const int waves = blockDim.x / 64, wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
@@ -251,22 +270,10 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         const int c = panel0 + 16 * V * q + V * j;
-        float *y = Y + row + c;
-        if (c + V <= N) {
-          cvec<V> out;
+        cvec<V> out;
 #pragma unroll
-          for (int v = 0; v < V; ++v) out.v[v] = acc[q][v][r];
-          if (mask) {
-            const cvec<V> m = *reinterpret_cast<const cvec<V> *>(mask + row + c);
-#pragma unroll
-            for (int v = 0; v < V; ++v) out.v[v] = m.v[v] <= 0.f ? 0.f : out.v[v];
-          }
-          *reinterpret_cast<cvec<V> *>(y) = out;
-        } else {
-#pragma unroll
-          for (int v = 0; v < V; ++v)
-            if (c + v < N) y[v] = mask && mask[row + c + v] <= 0.f ? 0.f : acc[q][v][r];
-        }
+        for (int v = 0; v < V; ++v) out.v[v] = acc[q][v][r];
+        gemm_store<V>(Y, row + c, out, N - c, out_how);
       }
     }
   };
@@ -297,7 +304,7 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 // X: n_rows x K, row stride ldx (or the rows of X that `rows` lists); Y: row q of it at q * ldy, or at rows[q] * ldy when
 // y_by_row is set.  wt: W is N x K.
 hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
-                           int n_rows, int K, int N, const float *mask, int compute_units, hipStream_t st) {
+                           int n_rows, int K, int N, const GemmOut &how, int compute_units, hipStream_t st) {
   if (n_rows <= 0) return hipSuccess;
   // Which kernel (us, this one / one 16-row tile per wavefront, at 4,000 / 16,000 / 32,000 / 64,000 rows): copying W to LDS
   // takes 5 us before the first product, the other kernel reads it from L2 for every row tile: 128 x 128 10.4 / 5.9,
@@ -322,7 +329,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     if (lds > 65536)                                                                                                           \
       err = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_panel_kernel<V_, Q_, WT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
     if (err == hipSuccess)                                                                                                     \
-      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, mask); \
+      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how); \
   } while (0)
 #define CALLP(V_, Q_) do { if (wt) { CALLP2(V_, Q_, true); } else { CALLP2(V_, Q_, false); } } while (0)
     switch (unit) {
@@ -346,7 +353,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   const int kw = tiles >= 8LL * compute_units || K <= 32 ? 1 : tiles >= 4LL * compute_units || K <= 64 ? 2 : 4;
   const dim3 grid((unsigned)((rt + 4 / kw - 1) / (4 / kw)), (unsigned)((N + 16 * cb - 1) / (16 * cb)));
 #define CALL3(CB_, KW_, WT_) \
-  hipLaunchKernelGGL((gemm_direct_kernel<CB_, KW_, WT_>), grid, dim3(256), 0, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, mask)
+  hipLaunchKernelGGL((gemm_direct_kernel<CB_, KW_, WT_>), grid, dim3(256), 0, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how)
 #define CALL2(CB_, KW_) do { if (wt) { CALL3(CB_, KW_, true); } else { CALL3(CB_, KW_, false); } } while (0)
 #define CALL(CB_) do { if (kw == 1) { CALL2(CB_, 1); } else if (kw == 2) { CALL2(CB_, 2); } else { CALL2(CB_, 4); } } while (0)
   if (cb == 4) CALL(4); else if (cb == 2) CALL(2); else CALL(1);

@@ -107,10 +107,30 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 18 us, 110,592 rows 33 / 39 us,
 //    2^21 rows 341 / 599 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
 //    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
+//
+// GeMM-SpMM, where the tiles' cost is the GEMM and its copies:
+//  * as (A B) C where K is two thirds of N or less: the gathers are K columns wide instead of N.  K = 32, N = 128: 700 x 700
+//    grid 219 us -> 118 us, 262,144 rows of 16 in a band of 32 (streamed tiles) 86 -> 64 us.
+//  * as A (B C) where the tiles need padded copies of B or column panels of D (262,144-row band, 250 x 32: 327 us, as two
+//    products 96; 134 x 106: 330 / 208), do not hold C in registers (300 x 128: 960 / 298), fuse only a part of the rows (64 x
+//    64 grid, 128 x 128: 30 / 12), or are not streamed: short matrices, 4,096 rows of the grid with 64 x 64 11.2 / 9.2 us, 5,000 rows of a
+//    band with 128 x 128 20 / 16, 20,000 rows 32 / 32.  With 64 x 64 such tiles win from some 8,000 rows on (20,000: 13.8 / 16.0).
 static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given, const int *Ap, const int *Ai) {
-  if (S->opts.op != TF_OP_SPMM_SPMM || S->windowed) return TF_OK;
+  if (S->windowed) return TF_OK;
   bool want;
-  if (S->march)
+  int N = S->opts.N;
+  if (S->opts.op == TF_OP_GEMM_SPMM) {
+    const int K = S->user_K;
+    N = S->user_N;
+    if (given.tile_rows > 0 || given.lds_budget_bytes > 0 || given.max_redundancy > 0.f || given.long_row_nnz > 0 || given.long_row_partition != 0 ||
+        given.hot_partition_bytes != 0 || given.short_row_hot_bytes != 0)
+      return TF_OK;
+    S->spmm_first = 3LL * K <= 2LL * N;
+    const bool tiled = !S->launch_tiles.empty();
+    const bool padded = K != S->opts.K || N != S->opts.N, partly = (long long)S->fused_ids.size() * 8 < 7LL * S->L;
+    want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || (!S->gemm_stream && ((long long)K * N > 64 * 64 || S->M < 8000))));
+    if (S->spmm_first) N = K;
+  } else if (S->march)
     want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 88000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
   else
     want = !S->launch_tiles.empty() && given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0;
@@ -118,7 +138,8 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
   tf_inspect_opts o{};
   o.struct_size = sizeof(o);
   o.op = TF_OP_SPMM_SPMM;
-  o.N = S->opts.N;
+  o.N = N;
+  o.compute_units = S->opts.compute_units;
   o.xcd_chunk_rows = given.xcd_chunk_rows;
   o.reorder_adjacency = given.reorder_adjacency;
   o.pattern_hash = S->pattern_hash;
@@ -982,7 +1003,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   }
   long long ws = 0;
   if (s->march) ws += (long long)s->march_ell_off.size() * 16;  // ELL rows with values, their offsets and sources
-  if (s->n_writeback_rows > 0 || s->two_passes) ws += (long long)s->M * s->opts.N * 4;
+  if (s->n_writeback_rows > 0 || s->two_passes) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
   if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1 + (long long)s->seg_groups.size()) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C

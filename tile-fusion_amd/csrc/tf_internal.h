@@ -73,6 +73,13 @@ struct RowsHow {
   int flagged = 0;          // columns carry the "cold" mark
 };
 
+// What becomes of a dense product's values on their way to Y (tf_dense.hip).
+struct GemmOut {
+  const float *mask = nullptr;  // of Y's shape: 0 where it is zero or less (the derivative of a ReLU whose output it is)
+  int accumulate = 0;           // Y += the product
+  int relu = 0;
+};
+
 // How launch_weight_grad cuts Y = G^T X (tf_dense.hip).
 struct WeightGradPlan {
   int nb, kb, n_chunks, k_chunks, rows_per_group, groups;
@@ -113,9 +120,10 @@ struct tf_schedule {
   int user_K = 0;             // K as given; opts.K is K rounded up to a multiple of 8 (what the kernels see)
   int user_N = 0;             // N as given; GeMM-SpMM with a width the MFMA kernels do not take (N % 32, N > 256) runs
   int n_panels = 1;           // as n_panels column panels of opts.N columns each, the last one zero-padded
-  // SpMM-SpMM: where it is faster than the tiles (see choose_two_passes in tf_inspector.cpp) the executor runs two row
-  // products through an intermediate in HBM, by this schedule of tf_inspect_spmm on A's pattern.
+  // Where it is faster than the tiles (see choose_two_passes in tf_inspector.cpp) the executor runs two products through an
+  // intermediate in HBM, A's by this schedule of tf_inspect_spmm.  spmm_first (GeMM-SpMM): as (A B) C.
   tf_schedule *two_passes = nullptr;
+  bool spmm_first = false;
   bool rows_only = false;     // a schedule of tf_inspect_spmm: one product, every row in the remainder lists
   int gemm_kc = 0;            // rows of C staged in LDS per step (GeMM-SpMM)
   bool gemm_regw = false;     // GeMM-SpMM tiles keep C in registers (no staging; slab rows padded)
