@@ -54,3 +54,18 @@ def test_two_row_products(gpu, tf, orc, pattern, N, other_inner):
         assert np.abs(D.to_numpy() - want).max() <= 1e-5 * np.abs(want).max()
     else:
         assert np.array_equal(D.to_numpy(), want)
+
+
+@pytest.mark.parametrize("N", [97, 100, 128, 52, 64])
+def test_column_slices(gpu, tf, orc, N):
+    """Graphs of the sizes at which the row kernel deals column slices to the XCDs (row counts that are no multiple of its blocks)."""
+    say(f"column slices N={N}")
+    n = 30011
+    A = tf.workloads.erdos_renyi_gcn(n, 3.0, seed=N)
+    C = tf.workloads.uniform((n, N), 7)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_SPMM_SPMM, N=N, inner=Ah)
+    D = tf.DenseMatrix(n, N)
+    tf.spmm_spmm(Ah, Ah, tf.DenseMatrix.from_numpy(C), D, S)
+    tf.device_synchronize()
+    assert np.array_equal(D.to_numpy(), oracle_spmm_spmm(orc, A, A, C))

@@ -209,8 +209,12 @@ class ArenaParts {
 // and N are what the caller has.  (Tiles take K in steps of 8 and N in steps of 32: padded copies, column panels.)
 static bool untiled(const tf_schedule *s) { return s->opts.op == TF_OP_GEMM_SPMM && (s->launch_tiles.empty() || s->two_passes); }
 // Floats from one row of the intermediate to the next: a multiple of 4, so that every lane's columns of a row are one
-// aligned load.
-static int inter_ld(const tf_schedule *s) { return untiled(s) ? (s->user_N + 3) / 4 * 4 : s->opts.N; }
+// aligned load, and whole cache lines where the row kernel then works in column slices (slices_for in tf_rows.hip).
+static int inter_ld(const tf_schedule *s) {
+  if (!untiled(s) && !s->two_passes) return s->opts.N;
+  const int N = s->user_N;
+  return N > 96 && N < 128 && s->M >= 16000 && s->M <= 131072 ? 128 : (N + 3) / 4 * 4;
+}
 
 // Device copies of the schedule arrays and the workspace, made on first use.
 static tf_status ensure_device(tf_schedule *s) {
@@ -360,6 +364,7 @@ struct Remainder {
   float *D;
   int accumulate, relu;
   int streaming = 1;  // D is not read again by this library
+  int ldd = 0;        // floats from one row of D to the next (0: N)
 };
 static tf_status run_hot_segments(tf_schedule *s, const Remainder &r, hipStream_t st) {
   DeviceSchedule *d = s->dev;
@@ -378,13 +383,13 @@ static tf_status run_hot_segments(tf_schedule *s, const Remainder &r, hipStream_
 // long-row segments were launched on the side stream already and are joined here.
 static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
   DeviceSchedule *d = s->dev;
-  const int N = r.N;
+  const int N = r.N, ldd = r.ldd > 0 ? r.ldd : r.N;
   if (!s->zero_rows.empty() && !r.accumulate)  // (D += 0 needs nothing)
-    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, N, st));
+    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, ldd, st));
   RowsArgs a;
   a.n_rows = (int)s->rem_rows.size();
   a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
-  a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = N; a.N = N;
+  a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = ldd; a.N = N;
   a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
   RowsHow how;
   how.xcd_chunk_rows = s->xcd_chunk_rows;
@@ -427,9 +432,9 @@ static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder 
       TF_PHASE(s, "long_seg_reduce_kernel (groups)", st,
                launch_seg_reduce(d->seg_groups, (int)s->seg_groups.size(), d->lrow_seg, d->partial, d->partial, N, N, 0, 0, st));
     TF_PHASE(s, "long_seg_reduce_kernel (rows)", st,
-             launch_seg_reduce(d->long_rows, d->n_long_rows, d->lrow_seg, d->partial, r.D, N, N, r.accumulate, r.relu, st));
+             launch_seg_reduce(d->long_rows, d->n_long_rows, d->lrow_seg, d->partial, r.D, ldd, N, r.accumulate, r.relu, st));
   } else if (d->n_long_rows > 0) {
-    TF_PHASE(s, "long_row_reduce_kernel", st, launch_long_row_reduce(d->long_rows, d->n_long_rows, d->partial, r.D, N, N, r.accumulate, r.relu, st));
+    TF_PHASE(s, "long_row_reduce_kernel", st, launch_long_row_reduce(d->long_rows, d->n_long_rows, d->partial, r.D, ldd, N, r.accumulate, r.relu, st));
   }
   return TF_OK;
 }
@@ -779,18 +784,21 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     if ((rc = tf::ensure_device(rows))) return rc;
     rows->profiling = s->profiling;
     rows->dev->prof_n = 0;
-    const int N = s->opts.N;
+    const int N = s->opts.N, ldt = tf::inter_ld(s);
     // (the lists hold A's columns: they serve B when it has A's pattern)
     const bool same = B == A || (B->p == A->p && B->i == A->i && B->x == A->x) || (B->hash && B->hash == s->pattern_hash);
     if (same) {
-      rc = tf::run_remainder(B, rows, tf::Remainder{C->d, N, N, C->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
+      tf::Remainder first{C->d, N, N, C->M, d->inter, 0, 0, tf::inter_streams(s)};
+      first.ldd = ldt;
+      rc = tf::run_remainder(B, rows, first, false, st);
     } else {
       tf::RowsArgs a = all_rows(B, C->d, d->inter, N);
+      a.ldy = ldt;
       a.streaming = tf::inter_streams(s);
       TF_PHASE(rows, "spmm_rows_kernel (intermediate rows)", st, tf::launch_spmm_rows(a, tf::RowsHow(), st));
     }
     if (rc) return rc;
-    return tf::run_remainder(A, rows, tf::Remainder{d->inter, N, N, s->M, D->d, acc, 0}, false, st);
+    return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, 0}, false, st);
   }
   if (s->march) {
     // The values in the order of the runs' ELL rows (the reference's reordered adjacency,

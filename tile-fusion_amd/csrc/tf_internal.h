@@ -66,7 +66,7 @@ struct RowsArgs {
   const float *chunk_Ax = nullptr;
   float *partial = nullptr;
   unsigned chunk_blocks = 0;          // set by the launcher
-  int n_blocks = 0, per_xcd = 0;  // set by the launcher
+  int n_blocks = 0, per_xcd = 0, slices = 1;  // set by the launcher
 };
 struct RowsHow {
   int xcd_chunk_rows = 0;   // how row blocks are dealt to the XCDs (tf_inspect_opts.xcd_chunk_rows)

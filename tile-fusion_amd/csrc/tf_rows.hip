@@ -177,6 +177,9 @@ template <int V> __device__ __forceinline__ int clamp_col(int c, int N) { return
 // and across the wavefronts through LDS, in a fixed order.  The only chunk of a row (slot < 0) goes straight to Y, a chunk of
 // a row with several to partial[slot], which long_row_reduce_kernel adds up in order.
 //
+// Column slices (slices > 1): workgroup b works on the columns [4 LPR s, 4 LPR (s + 1)) of its rows with s = b mod 8 mod
+// slices, so that an XCD gathers from one slice of X, `slices` times smaller than X; see slices_for.
+//
 // How a row's entries are walked: kDpp (above), the default; kDirect, every lane reads the pairs itself, for rows of fewer
 // than four columns and for X beyond 2 GB; kMarked, the same with the schedule's "cold" mark in the columns' top bit.
 // ---------------------------------------------------------------------------------
@@ -231,8 +234,16 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
   // The workgroups live for a microsecond or two: the arguments are all requested at once here, not one after the other
   // where they are first used, and a listed row's place in Y is not waited for before its entries are.
   asm volatile("" ::"s"(a.rows), "s"(a.Ap), "s"(a.Ai), "s"(a.Ax), "s"(a.X), "s"(a.Y), "s"(a.ldx), "s"(a.ldy), "s"(a.N), "s"(a.n_rows),
-               "s"(a.accumulate), "s"(a.streaming), "s"(a.compact), "s"(a.relu), "s"(a.n_blocks), "s"(a.per_xcd));
-  const int b = xcd_contiguous(CHUNKS ? blockIdx.x - a.chunk_blocks : blockIdx.x, a.per_xcd);
+               "s"(a.accumulate), "s"(a.streaming), "s"(a.compact), "s"(a.relu), "s"(a.n_blocks), "s"(a.per_xcd), "s"(a.slices));
+  int b = CHUNKS ? blockIdx.x - a.chunk_blocks : blockIdx.x, c_begin = 0, c_end = a.N;
+  if (a.slices > 1) {
+    const int xcd = b % kXcds;
+    b = b / kXcds * (kXcds / a.slices) + xcd / a.slices;
+    c_begin = xcd % a.slices * (LPR * V);
+    c_end = min(a.N, c_begin + LPR * V);
+  } else {
+    b = xcd_contiguous(b, a.per_xcd);
+  }
   if (b >= a.n_blocks) return;
   const int q = b * G + group;
   if (q >= a.n_rows) return;  // whole lane groups leave together
@@ -244,7 +255,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
     if (!a.compact) r = i;
   }
   const int kb = a.Ap[r], ke = a.Ap[r + 1];
-  for (int c0 = 0; c0 < a.N; c0 += LPR * V) {
+  for (int c0 = c_begin; c0 < c_end; c0 += LPR * V) {
     const int col = c0 + glane * V;
     const bool ok = col < a.N;
     const int coff = clamp_col<V>(col, a.N);
@@ -319,6 +330,19 @@ RowShape row_shape(int N, int accumulate) {
   return {V, LPR};
 }
 
+// Slices of 32 columns, a cache line each, where a slice is a few times an XCD's L2 and X is not: gathers that came out of
+// the Infinity Cache then hit.  One product of an Erdos-Renyi graph (10 - 12 entries a row), whole rows / slices: N = 128,
+// 10,000 rows 6.4 / 6.4 us, 20,000 14.5 / 10.1, 50,000 46 / 34, 100,000 83 / 75, 200,000 170 / 171; N = 64, 50,000 rows 21 / 19,
+// 100,000 41 / 39, and not on stencils (16 / 16.5).  Rows that do not start at a line would share lines between slices
+// (N = 100, 50,000 rows: 41 / 65).
+int slices_for(const RowsArgs &a) {
+  if (a.ldx % 32 != 0 || (reinterpret_cast<uintptr_t>(a.X) & 127u)) return 1;
+  const long long bytes = (long long)a.x_rows * a.ldx * 4;
+  if (a.N > 96 && a.N <= 128 && a.x_rows >= 16000 && bytes <= (64LL << 20)) return 4;
+  if (a.N > 48 && a.N <= 64 && a.compact && a.x_rows >= 24000 && bytes <= (40LL << 20)) return 2;
+  return 1;
+}
+
 inline bool xcd_remap_on() {
   static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
   return on;
@@ -335,23 +359,32 @@ inline bool xcd_remap_on() {
 }  // namespace
 
 hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
+
   if (a.n_rows <= 0 && a.n_chunks <= 0) return hipSuccess;
   RowShape s = row_shape(a.N, a.accumulate);
   a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
+  a.slices = s.V == 4 && !how.flagged && a.n_chunks == 0 && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
+  if (a.slices > 1) s.LPR = 8;
   const int G = kBlock / s.LPR;
   a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
   // 0: workgroup b takes block b; > 0: chunks of rows per XCD turn; < 0: one contiguous run per XCD
   const int n = a.n_blocks, want = how.xcd_chunk_rows > 0 ? std::max(1, how.xcd_chunk_rows / G) : 0;
   a.per_xcd = how.xcd_chunk_rows == 0 || !xcd_remap_on() ? 0 : (want <= 0 || want * kXcds >= n) ? (n + kXcds - 1) / kXcds : want;
   const int per = std::max(a.per_xcd, 1) * kXcds;
-  const dim3 grid(a.chunk_blocks + (n + per - 1) / per * per);
+  const int turns = kXcds / a.slices;  // row blocks per eight workgroups
+  const dim3 grid(a.chunk_blocks + (a.slices > 1 ? (n + turns - 1) / turns * kXcds : (n + per - 1) / per * per));
 #define CALL3(V_, L_, WALK_, CH_) hipLaunchKernelGGL((spmm_rows_kernel<V_, L_, WALK_, CH_>), grid, dim3(kBlock), 0, st, a)
 #define CALL2(V_, L_, WALK_) do { if (a.n_chunks > 0) { CALL3(V_, L_, WALK_, true); } else { CALL3(V_, L_, WALK_, false); } } while (0)
 #define CALLP(V_, L_) do { if constexpr (V_ == 4) { CALL2(V_, L_, kDpp); } } while (0)
 #define CALLD(V_, L_) CALL2(V_, L_, kDirect)
 #define CALLM(V_, L_) CALL2(V_, L_, kMarked)
+  // The DPP walk pays where L1 or L2 serves the gathers (27 points, 80^3, N = 64: 154 -> 116 us; R-MAT 2^20, N = 32: 311 -> 284)
+  // and costs a little where the Infinity Cache does, rows in no order and X beyond 48 MB (Erdos-Renyi, 200,000 rows,
+  // N = 64 / 100: 85.2 -> 87.0, 159.5 -> 162.3).
+  const unsigned long long x_bytes = (unsigned long long)a.x_rows * a.ldx * 4;
+  const bool far_gathers = a.compact && a.N >= 64 && x_bytes > (48ull << 20);
   if (how.flagged) TF_DISPATCH_ROWS(s, CALLM);
-  else if (s.V == 4 && (unsigned long long)a.x_rows * a.ldx * 4 <= 0x80000000ull) TF_DISPATCH_ROWS(s, CALLP);
+  else if (s.V == 4 && x_bytes <= 0x80000000ull && !far_gathers) TF_DISPATCH_ROWS(s, CALLP);
   else TF_DISPATCH_ROWS(s, CALLD);
 #undef CALLP
 #undef CALLD

@@ -63,7 +63,7 @@ struct Adjacency : torch::CustomClassHolder {
   uint64_t hash = 0;
   tf_csr *csr = nullptr;
   std::map<std::pair<int, int>, tf_schedule *> gemm_schedules;  // (K, N)
-  std::map<int, tf_schedule *> row_schedules;                   // N, rounded up to a power of two from 128 on
+  std::map<int, tf_schedule *> row_schedules;                   // N, rounded up to a power of two from 32 on
   c10::intrusive_ptr<Adjacency> transposed;                     // null: not built yet, or `symmetric`
   bool symmetric = false;
   std::mutex mutex;
@@ -89,7 +89,7 @@ struct Adjacency : torch::CustomClassHolder {
     return s;
   }
   tf_schedule *row_schedule(int width) {
-    int N = 128;
+    int N = 32;
     while (N < width) N *= 2;
     tf_schedule *&s = row_schedules[N];
     if (!s) check(tf_inspect_spmm(rows, cols, Ap.data(), Ai.data(), N, hash, &s));
