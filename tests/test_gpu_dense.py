@@ -119,3 +119,40 @@ def test_fused_layer_with_transposed_weights(gpu, tf, K, N):
         assert tf.lib().tf_gemm_spmm(Ah.to_device().h, tf.DenseMatrix.from_numpy(X).h, Wd.h, D.h, S.h, flags, None) == 0
         tf.device_synchronize()
         assert rel(D.to_numpy(), np.maximum(want, 0) if flags & RELU else want) <= 1e-5, flags
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 4, 1), (500, 30, 30), (4096, 64, 64), (4096, 5, 130), (3000, 128, 7), (2000, 100, 129), (23999, 33, 17), (24001, 30, 30),
+                                   (24500, 64, 96), (30000, 7, 16), (25000, 61, 64)])
+@pytest.mark.parametrize("listed", [False, True])
+def test_layer_in_one_launch(gpu, tf, M, K, N, listed):
+    """(A B) C in one kernel: rows in order and in lists (two length classes, rows without entries), either storage of the weights,
+    accumulation and a ReLU of the result."""
+    say(f"one launch M={M} {K}x{N} listed={listed}")
+    rng = np.random.default_rng(M + K + N)
+    if listed:
+        A = tf.workloads.erdos_renyi_gcn(M, 8.0, seed=3)
+        if M > 100:
+            keep = np.ones(M)
+            keep[rng.integers(0, M, M // 3)] = 0.0
+            A = sp.csr_matrix(sp.diags(keep) @ A)
+            A.eliminate_zeros()
+        A = sp.csr_matrix(A, dtype=np.float32)
+    else:
+        A = sp.csr_matrix(sp.diags([1.0, -2.0, 3.0], [-1, 0, 2], shape=(M, M)), dtype=np.float32)
+    A.sort_indices()
+    X, W, D0 = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    S.validate()
+    want = A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))
+    Xd = tf.DenseMatrix.from_numpy(X)
+    S.set_profiling(True)
+    for flags in (0, C_TRANSPOSED, 1, RELU, 1 | RELU | C_TRANSPOSED):
+        Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if flags & C_TRANSPOSED else W)
+        D = tf.DenseMatrix.from_numpy(D0)
+        assert tf.lib().tf_gemm_spmm(Ah.to_device().h, Xd.h, Wd.h, D.h, S.h, flags, None) == 0
+        tf.device_synchronize()
+        if flags == 0:
+            assert "spmm_gemm_kernel" in [n for n, _ in S.profile()]
+        ref = want + D0 if flags & 1 else want
+        assert rel(D.to_numpy(), np.maximum(ref, 0) if flags & RELU else ref) <= 1e-5, flags

@@ -91,6 +91,7 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
                                            const float *, int, const float *, const int *, const int *,
                                            const float *, int, float *, int, int, int, int, hipStream_t);
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
+hipError_t launch_spmm_gemm(const RowsArgs &, const float *, int, int, const GemmOut &, hipStream_t);
 hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const GemmOut &, int, hipStream_t);
 WeightGradPlan plan_weight_grad(int, int, int, int);
@@ -379,19 +380,14 @@ static tf_status run_hot_segments(tf_schedule *s, const Remainder &r, hipStream_
   return TF_OK;
 }
 
-// Second-op rows that no tile fused: served from the intermediate in HBM.  hot_on_side: the hot
-// long-row segments were launched on the side stream already and are joined here.
-static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
+// The row kernel's operands for the remainder rows and the chunks of the long ones.
+static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder &r, hipStream_t st, RowsArgs &a, RowsHow &how) {
   DeviceSchedule *d = s->dev;
   const int N = r.N, ldd = r.ldd > 0 ? r.ldd : r.N;
-  if (!s->zero_rows.empty() && !r.accumulate)  // (D += 0 needs nothing)
-    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, ldd, st));
-  RowsArgs a;
   a.n_rows = (int)s->rem_rows.size();
   a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
   a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = ldd; a.N = N;
   a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
-  RowsHow how;
   how.xcd_chunk_rows = s->xcd_chunk_rows;
   a.chunks = d->long_chunks;
   a.n_chunks = (unsigned)s->long_chunks.size();
@@ -411,6 +407,21 @@ static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder 
   } else if (!s->rem_identity) {
     a.rows = d->rem_rows;
   }
+  return TF_OK;
+}
+
+// Second-op rows that no tile fused: served from the intermediate in HBM.  hot_on_side: the hot
+// long-row segments were launched on the side stream already and are joined here.
+static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
+  DeviceSchedule *d = s->dev;
+  const int N = r.N, ldd = r.ldd > 0 ? r.ldd : r.N;
+  if (!s->zero_rows.empty() && !r.accumulate)  // (D += 0 needs nothing)
+    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, ldd, st));
+  else if (!s->zero_rows.empty() && r.relu)    // (but for the ReLU, of all of D: a second one changes nothing)
+    TF_PHASE(s, "relu_kernel", st, launch_relu(r.D, (size_t)s->L * ldd, st));
+  RowsArgs a;
+  RowsHow how;
+  if (tf_status rc = remainder_rows(A, s, r, st, a, how)) return rc;
   // one launch, the long rows' workgroups first
   if (a.n_rows > 0 || a.n_chunks > 0)
     TF_PHASE(s, a.n_chunks > 0 ? "spmm_rows_kernel (short and long remainder rows)" : "spmm_rows_kernel (short remainder rows)", st, launch_spmm_rows(a, how, st));
@@ -960,11 +971,22 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
     rows->dev->prof_n = 0;
     const int K = s->user_K, N = s->user_N, cus = s->opts.compute_units;
     if (s->spmm_first) {
-      rc = tf::run_remainder(A, rows, tf::Remainder{B->d, K, K, B->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
-      if (rc) return rc;
       tf::GemmOut how;
       how.accumulate = acc;
       how.relu = relu;
+      // (rows without entries would need a ReLU of what D holds; B within the kernel's 32-bit offsets)
+      if (s->one_launch && !(acc && relu && !rows->zero_rows.empty()) && (unsigned long long)B->M * K * 4 <= 0x80000000ull) {
+        if (!rows->zero_rows.empty() && !acc)
+          TF_PHASE(rows, "zero_rows_kernel (rows without entries)", st, tf::launch_zero_rows(rows->dev->zero_rows, (int)rows->zero_rows.size(), D->d, N, st));
+        tf::RowsArgs a;
+        tf::RowsHow rows_how;
+        if ((rc = tf::remainder_rows(A, rows, tf::Remainder{B->d, K, K, B->M, D->d, 0, 0}, st, a, rows_how))) return rc;
+        a.ldy = N;
+        TF_PHASE(rows, "spmm_gemm_kernel", st, tf::launch_spmm_gemm(a, C->d, c_t, N, how, st));
+        return TF_OK;
+      }
+      rc = tf::run_remainder(A, rows, tf::Remainder{B->d, K, K, B->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
+      if (rc) return rc;
       if (!c_t && !acc && !relu && row_gemm_takes(s->L, K, N, cus))
         TF_PHASE(rows, "gemm_rows_kernel", st, tf::launch_gemm(d->inter, C->d, D->d, nullptr, s->L, K, N, cus, st, 0));
       else

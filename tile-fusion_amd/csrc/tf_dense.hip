@@ -9,10 +9,7 @@
 
 namespace tf {
 
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // (rows of K floats start at any multiple of 4 bytes)
 typedef float acc16 __attribute__((ext_vector_type(16)));
-typedef float acc4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------
 // Y[q, :N] = X[rows[q], :K] * W, W stored K x N or (WT) N x K as torch stores a layer's weights, any K and N.
@@ -25,39 +22,6 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 // MFMA t, one 16-byte load of X, and of W when it is stored N x K.  Columns are dealt to lanes CB at a time
 // (column CB j + cb to column block cb), so that a K x N stored W is loaded, and Y stored, CB floats per lane.
 // ---------------------------------------------------------------------------------
-template <int CB> struct cvec { float v[CB]; };
-
-// The values v of CB adjacent columns at Y + at, the first `columns` of them existing ones.
-template <int CB> __device__ __forceinline__ void gemm_store(float *__restrict__ Y, size_t at, cvec<CB> v, int columns, const GemmOut &how) {
-  auto finish = [&](float x, size_t i) __attribute__((always_inline)) {
-    if (how.accumulate) x += Y[i];
-    if (how.mask) x = how.mask[i] <= 0.f ? 0.f : x;
-    if (how.relu) x = x < 0.f ? 0.f : x;
-    return x;
-  };
-  if (columns >= CB) {
-    if (how.accumulate || how.mask || how.relu) {
-      cvec<CB> m;
-      if (how.mask) m = *reinterpret_cast<const cvec<CB> *>(how.mask + at);
-      if (how.accumulate) {
-        const cvec<CB> y = *reinterpret_cast<const cvec<CB> *>(Y + at);
-#pragma unroll
-        for (int c = 0; c < CB; ++c) v.v[c] += y.v[c];
-      }
-#pragma unroll
-      for (int c = 0; c < CB; ++c) {
-        if (how.mask) v.v[c] = m.v[c] <= 0.f ? 0.f : v.v[c];
-        if (how.relu) v.v[c] = v.v[c] < 0.f ? 0.f : v.v[c];
-      }
-    }
-    *reinterpret_cast<cvec<CB> *>(Y + at) = v;
-  } else {
-#pragma unroll
-    for (int c = 0; c < CB; ++c)
-      if (c < columns) Y[at + c] = finish(v.v[c], at + c);
-  }
-}
-
 template <int CB, int KW, bool WT>
 __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
                                                           float *__restrict__ Y, int ldy, const int *__restrict__ rows,

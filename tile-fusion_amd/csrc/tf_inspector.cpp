@@ -108,13 +108,19 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    2^21 rows 341 / 599 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
 //    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
 //
-// GeMM-SpMM, where the tiles' cost is the GEMM and its copies:
-//  * as (A B) C where K is two thirds of N or less: the gathers are K columns wide instead of N.  K = 32, N = 128: 700 x 700
-//    grid 219 us -> 118 us, 262,144 rows of 16 in a band of 32 (streamed tiles) 86 -> 64 us.
-//  * as A (B C) where the tiles need padded copies of B or column panels of D (262,144-row band, 250 x 32: 327 us, as two
+// GeMM-SpMM:
+//  * as (A B) C in one launch (spmm_gemm_kernel) where no row has its sum from several workgroups and K is narrow.  Under 24,000
+//    rows the second launch and the chain of loads count (us, one launch / GEMM and row product or tiles): 64 x 64 grid, 64 x 64 5.2 /
+//    9.0, 128 x 128 8.1 / 11.6; Erdos-Renyi 8,000 rows 64 x 64 6.2 / 12.1, 128 x 64 9.1 / 14.1, 100 x 16 7.4 / 8.8, 250 x 32 16.5 / 11.6;
+//    20,000 rows 64 x 64 10.2 / 20.1, 128 x 128 30 / 36, 200 x 128 47 / 43, 100 x 16 14.0 / 11.9.  With more rows the intermediate's
+//    trip does, as long as W's trips from L2 do not: 200,000 rows 64 x 64 93 / 113, 700 x 700 grid 30 x 30 52 / 78, 64 x 64
+//    127 / 136, 128 x 128 408 / 316; streamed tiles stay the faster way at 64 x 64 (262,144-row band 79 / 60).
+//  * as (A B) C in two launches where K is two thirds of N or less: the gathers are K columns wide instead of N.  K = 32, N = 128: 700 x 700
+//    grid 219 us -> 118 us (136 in one launch), 262,144 rows of 16 in a band of 32 (streamed tiles) 86 -> 64 us.
+//  * as A (B C) where tiles need padded copies of B or column panels of D (262,144-row band, 250 x 32: 327 us, as two
 //    products 96; 134 x 106: 330 / 208), do not hold C in registers (300 x 128: 960 / 298), fuse only a part of the rows (64 x
-//    64 grid, 128 x 128: 30 / 12), or are not streamed: short matrices, 4,096 rows of the grid with 64 x 64 11.2 / 9.2 us, 5,000 rows of a
-//    band with 128 x 128 20 / 16, 20,000 rows 32 / 32.  With 64 x 64 such tiles win from some 8,000 rows on (20,000: 13.8 / 16.0).
+//    64 grid, 128 x 128: 30 / 12), or are not streamed: short matrices, 5,000 rows of a
+//    band with 128 x 128 20 / 16, 20,000 rows 32 / 32.
 static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given, const int *Ap, const int *Ai) {
   if (S->windowed) return TF_OK;
   bool want;
@@ -125,15 +131,19 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     if (given.tile_rows > 0 || given.lds_budget_bytes > 0 || given.max_redundancy > 0.f || given.long_row_nnz > 0 || given.long_row_partition != 0 ||
         given.hot_partition_bytes != 0 || given.short_row_hot_bytes != 0)
       return TF_OK;
-    S->spmm_first = 3LL * K <= 2LL * N;
+    const long long M = S->L, work = M * K;
     const bool tiled = !S->launch_tiles.empty();
     const bool padded = K != S->opts.K || N != S->opts.N, partly = (long long)S->fused_ids.size() * 8 < 7LL * S->L;
-    want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || (!S->gemm_stream && ((long long)K * N > 64 * 64 || S->M < 8000))));
+    const bool streamed = tiled && S->gemm_stream && !padded && !partly;
+    S->one_launch = K >= 4 && (M < 24000 ? (K <= 128 && (K <= 2 * N || M < 10000)) || (K <= 2 * N && work <= 2000000)
+                                         : K <= 64 && K <= N && (N <= 64 || M <= 150000) && !(streamed && K > 32));
+    S->spmm_first = S->one_launch || 3LL * K <= 2LL * N;
+    want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || !S->gemm_stream));
     if (S->spmm_first) N = K;
   } else if (S->march)
     want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 88000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
   else
-    want = !S->launch_tiles.empty() && given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0;
+    want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;
   if (!want) return TF_OK;
   tf_inspect_opts o{};
   o.struct_size = sizeof(o);
@@ -143,7 +153,20 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
   o.xcd_chunk_rows = given.xcd_chunk_rows;
   o.reorder_adjacency = given.reorder_adjacency;
   o.pattern_hash = S->pattern_hash;
-  return inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes);
+  if (tf_status rc = inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes)) return rc;
+  const tf_schedule *rows = S->two_passes;
+  if (S->one_launch && (!rows->long_chunks.empty() || rows->long_part || rows->rem_flagged)) {
+    // hub rows: another order of the products, or the schedule's own (a GEMM of the rows that are read, placed by reads)
+    S->one_launch = false;
+    if (3LL * S->user_K > 2LL * S->user_N) {
+      S->spmm_first = false;
+      if (S->launch_tiles.empty()) {
+        tf_schedule_free(S->two_passes);
+        S->two_passes = nullptr;
+      }
+    }
+  }
+  return TF_OK;
 }
 
 // rows_only: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.

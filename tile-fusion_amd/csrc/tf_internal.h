@@ -124,6 +124,7 @@ struct tf_schedule {
   // intermediate in HBM, A's by this schedule of tf_inspect_spmm.  spmm_first (GeMM-SpMM): as (A B) C.
   tf_schedule *two_passes = nullptr;
   bool spmm_first = false;
+  bool one_launch = false;    // ... in one kernel that multiplies the rows of A B by C in LDS (spmm_gemm_kernel)
   bool rows_only = false;     // a schedule of tf_inspect_spmm: one product, every row in the remainder lists
   int gemm_kc = 0;            // rows of C staged in LDS per step (GeMM-SpMM)
   bool gemm_regw = false;     // GeMM-SpMM tiles keep C in registers (no staging; slab rows padded)

@@ -272,6 +272,112 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------
+// Y = (A X) W in one launch: the rows of A X, K columns wide, are gathered as in spmm_rows_kernel into LDS, R of them a
+// workgroup, and multiplied by W (K x N, or N x K with WT) on v_mfma_f32_16x16x4_f32; neither intermediate nor second
+// launch.  In the product a wavefront owns 16 rows and 16 V columns (column V j + v of its panel is column block v's lane j).
+// R = 16, for few rows: what counts is the chain of dependent loads, so the four wavefronts share the columns and W's first
+// four steps are requested before the gathers.  R = 64, for many rows of up to 32 columns of X: what counts is L2, so W is
+// read once per 64 rows and seven workgroups share a compute unit, one gathering while another multiplies.  See
+// one_launch in tf_api.cpp for where this is the faster way.
+// ---------------------------------------------------------------------------------
+template <int LPR, int R, int V, bool WT>
+__global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(const RowsArgs a, const float *__restrict__ W, int N, const GemmOut how) {
+  extern __shared__ __align__(16) float slab[];
+  constexpr int G = kBlock / LPR, RT = R / 16, CW = 4 / RT;  // lane groups; row tiles; wavefronts side by side in columns
+  const int K = a.N, ld = (K + 15) / 16 * 16 + 4;            // (four floats behind a row: its reads start in other banks)
+  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X), 0, (int)(a.x_rows * a.ldx * 4u), 0x00020000);
+  const int q0 = blockIdx.x * R;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
+  const int rt = wave % RT, S = (K + 15) / 16, full = K / 16;
+  const int first_col = wave / RT * 16 * V + V * j;
+  const float *sp = slab + (rt * 16 + j) * ld + 4 * h;
+  struct panel { f4v b[V]; };
+  // step s of W for this lane's columns (32-bit offsets: W is far smaller than 4 GB)
+  auto load = [&](int col0, int s) __attribute__((always_inline)) {
+    panel o;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const unsigned c = min(col0 + v, N - 1), k0 = 16 * s + 4 * h;
+      if (s < full) {
+        if constexpr (WT) o.b[v] = *reinterpret_cast<const f4u *>(W + (c * (unsigned)K + k0));
+        else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) o.b[v][t] = W[(k0 + t) * (unsigned)N + c];
+        }
+      } else {  // values of k past K
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o.b[v][t] = k0 + t < (unsigned)K ? W[WT ? c * (unsigned)K + k0 + t : (k0 + t) * (unsigned)N + c] : 0.f;
+      }
+    }
+    return o;
+  };
+  constexpr int AHEAD = R == 16 ? 4 : 1;  // steps of W requested ahead
+  panel w[AHEAD];
+  if (R == 16 && first_col < N) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) w[u] = load(first_col, min(u, S - 1));
+  }
+  for (int r = group; r < R; r += G) {
+    const int q = q0 + r;
+    int kb = 0, ke = 0;
+    if (q < a.n_rows) {
+      const int row = a.rows && !a.compact ? a.rows[q] : q;
+      kb = a.Ap[row];
+      ke = a.Ap[row + 1];
+    }
+    for (int c0 = 0; c0 < K; c0 += LPR * 4) {
+      const int col = c0 + glane * 4, coff = clamp_col<4>(col, K);
+      fvec<4> acc = vzero<4>();
+      row_dot_dpp<LPR>(a.Ai, a.Ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
+      if (col < K) {
+        float *s = slab + r * ld + coff;
+        if (K % 4 == 0) *reinterpret_cast<fvec<4> *>(s) = acc;
+        else { s[0] = acc.v[0]; s[1] = acc.v[1]; s[2] = acc.v[2]; s[3] = acc.v[3]; }
+      }
+    }
+    if (glane < ld - 4 - K) slab[r * ld + K + glane] = 0.f;  // (up to 15 columns that fill the last step of k)
+    if (LPR < 16)
+      for (int c = glane + LPR; c < ld - 4 - K; c += LPR) slab[r * ld + K + c] = 0.f;
+  }
+  __syncthreads();
+  for (int col0 = first_col; col0 - V * j < N; col0 += CW * 16 * V) {
+    acc4 acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = 0.f;
+    if (R != 16 || col0 != first_col) {
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) w[u] = load(col0, min(u, S - 1));
+    }
+    for (int s0 = 0; s0 < S; s0 += AHEAD) {
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const int s = s0 + u;
+        if (s >= S) break;
+        const panel cur = w[u];
+        if (s + AHEAD < S) w[u] = load(col0, s + AHEAD);
+        const f4v x = *reinterpret_cast<const f4v *>(sp + 16 * s);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t], cur.b[v][t], acc[v], 0, 0, 0);
+      }
+    }
+    if (col0 < N) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int q = q0 + rt * 16 + 4 * h + r;
+        if (q >= a.n_rows) continue;
+        cvec<V> out;
+#pragma unroll
+        for (int v = 0; v < V; ++v) out.v[v] = acc[v][r];
+        gemm_store<V>(a.Y, (size_t)(a.rows ? a.rows[q] : q) * a.ldy + col0, out, N - col0, how);
+      }
+    }
+  }
+}
+
 // The rows with several chunks: Y[row] (+)= their partial sums, in order.
 __global__ __launch_bounds__(kBlock) void long_row_reduce_kernel(const LongRow *__restrict__ rows, const float *__restrict__ partial,
                                                                  float *__restrict__ Y, int ldy, int N, int accumulate, int relu) {
@@ -392,6 +498,34 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
 #undef CALL2
 #undef CALL3
   return hipGetLastError();
+}
+
+// Y = (A X) W for the rows of `a` (a.N = K the columns of X, a.ldy that of Y): K from 4 up, X of up to 2 GB, no long rows.
+hipError_t launch_spmm_gemm(const RowsArgs &a, const float *W, int wt, int N, const GemmOut &how, hipStream_t st) {
+  if (a.n_rows <= 0) return hipSuccess;
+  if (a.N < 4 || a.n_chunks > 0 || (unsigned long long)a.x_rows * a.ldx * 4 > 0x80000000ull) return hipErrorInvalidValue;
+  const RowShape s = row_shape(a.N, 0);
+  const int R = a.n_rows < 24000 ? 16 : 64, lds = R * ((a.N + 15) / 16 * 16 + 4) * 4;
+  const dim3 grid((a.n_rows + R - 1) / R);
+  hipError_t err = hipSuccess;
+#define CALL3(L_, R_, V_, WT_)                                                                                                         \
+  do {                                                                                                                                 \
+    if (lds > 65536)                                                                                                                   \
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_gemm_kernel<L_, R_, V_, WT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+    if (err == hipSuccess) hipLaunchKernelGGL((spmm_gemm_kernel<L_, R_, V_, WT_>), grid, dim3(kBlock), lds, st, a, W, N, how);         \
+  } while (0)
+#define CALL2(L_, R_, V_) do { if (wt) { CALL3(L_, R_, V_, true); } else { CALL3(L_, R_, V_, false); } } while (0)
+#define CALL(V__, L_)                                                                                                   \
+  do {                                                                                                                  \
+    if constexpr (V__ == 4) {                                                                                           \
+      if (R == 16) { if (N > 64) { CALL2(L_, 16, 2); } else { CALL2(L_, 16, 1); } } else if (N > 16) { CALL2(L_, 64, 2); } else { CALL2(L_, 64, 1); } \
+    }                                                                                                                   \
+  } while (0)
+  TF_DISPATCH_ROWS(s, CALL);
+#undef CALL
+#undef CALL2
+#undef CALL3
+  return err != hipSuccess ? err : hipGetLastError();
 }
 
 hipError_t launch_long_row_reduce(const LongRow *rows, int n_rows, const float *partial, float *Y, int ldy, int N, int accumulate,
