@@ -81,6 +81,34 @@ def test_scheduled_row_product(gpu, tf, N, relu):
         lib.tf_schedule_free(s)
 
 
+@pytest.mark.parametrize("N", [1, 3, 30, 64, 128, 260])
+@pytest.mark.parametrize("empty", [0.3, 0.9])
+def test_rows_without_entries(gpu, tf, N, empty):
+    """Fewer and more rows without entries than with, cleared by the row product's own launch; with accumulation untouched but for
+    a ReLU."""
+    say(f"empty rows N={N} {empty}")
+    rng = np.random.default_rng(N)
+    M = 17000
+    A = sp.csr_matrix(sp.diags((rng.random(M) >= empty).astype(np.float32)) @ tf.workloads.erdos_renyi_gcn(M, 9.0, seed=1), dtype=np.float32)
+    A.eliminate_zeros()
+    X, D0 = (rng.uniform(-1, 1, (M, N)).astype(np.float32) for _ in range(2))
+    Ah = tf.CsrMatrix.from_scipy(A).to_device()
+    lib = tf.lib()
+    s = C.c_void_p()
+    assert lib.tf_inspect_spmm(M, M, Ah._pp, Ah._pi, N, 0, C.byref(s)) == 0
+    try:
+        Xd = tf.DenseMatrix.from_numpy(X)
+        want = A.astype(np.float64) @ X.astype(np.float64)
+        for flags in (0, RELU, 1, 1 | RELU):
+            Y = tf.DenseMatrix.from_numpy(D0 if flags & 1 else np.full((M, N), np.nan, np.float32))
+            assert lib.tf_spmm_scheduled(Ah.h, Xd.h, Y.h, s, flags, None) == 0
+            tf.device_synchronize()
+            ref = want + D0 if flags & 1 else want
+            assert rel(Y.to_numpy(), np.maximum(ref, 0) if flags & RELU else ref) <= 1e-5, flags
+    finally:
+        lib.tf_schedule_free(s)
+
+
 @pytest.mark.parametrize("K,N", [(30, 7), (500, 32), (251, 47), (64, 300), (300, 128), (32, 1)])
 def test_layer_that_fuses_nothing_in_any_width(gpu, tf, K, N):
     """GeMM-SpMM on a graph: K and N as they come, either storage of the weights, accumulation, a ReLU of the result."""

@@ -116,7 +116,6 @@ hipError_t launch_copy_cols(const float *, int, int, int, int, float *, int, int
 hipError_t launch_relu(float *, size_t, hipStream_t);
 hipError_t launch_fused_gcn2(const Tile2 *, int, const float *, const float *, const float *, int, int, int, const int *, const int *,
                              const float *, float *, int, int, int, hipStream_t);
-hipError_t launch_zero_rows(const int *, int, float *, int, hipStream_t);
 hipError_t launch_xcd_probe(int *, int, hipStream_t);
 hipError_t launch_issue_probe(float *, int, int, int, int, hipStream_t);
 
@@ -389,6 +388,8 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
   a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = ldd; a.N = N;
   a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
   how.xcd_chunk_rows = s->xcd_chunk_rows;
+  a.zero_rows = d->zero_rows;
+  a.n_zero = r.accumulate && !r.relu ? 0 : (int)s->zero_rows.size();  // (D += 0 needs nothing)
   a.chunks = d->long_chunks;
   a.n_chunks = (unsigned)s->long_chunks.size();
   a.chunk_Ai = A->i; a.chunk_Ax = A->x; a.partial = d->partial;
@@ -415,10 +416,6 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
 static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
   DeviceSchedule *d = s->dev;
   const int N = r.N, ldd = r.ldd > 0 ? r.ldd : r.N;
-  if (!s->zero_rows.empty() && !r.accumulate)  // (D += 0 needs nothing)
-    TF_PHASE(s, "zero_rows_kernel (rows without entries)", st, launch_zero_rows(d->zero_rows, (int)s->zero_rows.size(), r.D, ldd, st));
-  else if (!s->zero_rows.empty() && r.relu)    // (but for the ReLU, of all of D: a second one changes nothing)
-    TF_PHASE(s, "relu_kernel", st, launch_relu(r.D, (size_t)s->L * ldd, st));
   RowsArgs a;
   RowsHow how;
   if (tf_status rc = remainder_rows(A, s, r, st, a, how)) return rc;
@@ -974,13 +971,10 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
       tf::GemmOut how;
       how.accumulate = acc;
       how.relu = relu;
-      // (rows without entries would need a ReLU of what D holds; B within the kernel's 32-bit offsets)
-      if (s->one_launch && !(acc && relu && !rows->zero_rows.empty()) && (unsigned long long)B->M * K * 4 <= 0x80000000ull) {
-        if (!rows->zero_rows.empty() && !acc)
-          TF_PHASE(rows, "zero_rows_kernel (rows without entries)", st, tf::launch_zero_rows(rows->dev->zero_rows, (int)rows->zero_rows.size(), D->d, N, st));
+      if (s->one_launch && (unsigned long long)B->M * K * 4 <= 0x80000000ull) {  // (the kernel's 32-bit offsets into B)
         tf::RowsArgs a;
         tf::RowsHow rows_how;
-        if ((rc = tf::remainder_rows(A, rows, tf::Remainder{B->d, K, K, B->M, D->d, 0, 0}, st, a, rows_how))) return rc;
+        if ((rc = tf::remainder_rows(A, rows, tf::Remainder{B->d, K, K, B->M, D->d, acc, relu}, st, a, rows_how))) return rc;
         a.ldy = N;
         TF_PHASE(rows, "spmm_gemm_kernel", st, tf::launch_spmm_gemm(a, C->d, c_t, N, how, st));
         return TF_OK;

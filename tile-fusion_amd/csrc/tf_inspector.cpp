@@ -612,20 +612,26 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     {
       long long long_nnz = 0;
       for (const auto &lr : S->long_rows) long_nnz += Ap[lr.row + 1] - Ap[lr.row];
+      // (narrower rows are not worth partial sums of their own: 2^20 nodes, N = 32 / 48 / 64, chunks 242 / 432 / 550 us, partitions
+      // 294 / 438 / 472)
       const bool want = o.long_row_partition > 0 ||
-                        (o.long_row_partition == 0 && long_nnz >= (1 << 20) && (long long)M * o.N * 4 > (64LL << 20));
+                        (o.long_row_partition == 0 && long_nnz >= (1 << 20) && (long long)M * o.N * 4 > (64LL << 20) && o.N >= 56);
       // (three times an L2's 4 MB measured best on the R-MAT graph: 2.68 ms per step with 4 MB, 2.54 with 12 or
       // 16 MB, 2.60 with 32 MB -- the reads inside a partition are skewed too, and its hottest rows are what stays)
       const int part_rows = std::max(64, (o.hot_partition_bytes > 0 ? o.hot_partition_bytes : (12 << 20)) / (o.N * 4));
       // Regrouped rows pay for their partial sums (a row of 4N bytes written and read again per group): with the
       // threshold left to the library, rows of up to 64 entries stay whole rows of the row kernel (measured on the
       // 2^21-node R-MAT step, thresholds 32 / 40 / 48 / 64 / 96: 2.04 / 1.97 / 1.97 / 1.96 / 1.97 ms).
-      if (want && user->long_row_nnz <= 0 && S->long_chunks.size() < (size_t)INT_MAX) {
-        constexpr int kPartitionedFrom = 64;
+      // In chunks, a workgroup per row of a few dozen entries is the dearer way once there are rows enough to fill the chip by
+      // themselves.  R-MAT graphs, rows of up to 32 / 64 / 128 entries kept whole: 2^16 nodes, N = 8 / 64, 25.9 / 25.8 / 36.7 and 37.4 / 36.1 / 38.3 us,
+      // 2^17 nodes 37 / 40.7 / 47.3 and 56 / 52.9 / 52.4, 2^18 nodes 64 / 61 / 70 and 107 / 104 / 96, 2^20 nodes 196 / 194 / 178 and
+      // 555 / 556 / 555 (N = 32: 279 / 270 / 242).
+      const int whole = want ? 64 : L >= 200000 && o.N >= 16 ? 128 : L >= 100000 && o.N >= 48 ? 64 : 32;
+      if (user->long_row_nnz <= 0 && whole > o.long_row_nnz && S->long_chunks.size() < (size_t)INT_MAX) {
         std::vector<tf::LongRow> keep_rows;
         std::vector<tf::LongChunk> keep_chunks;
         for (const auto &lr : S->long_rows) {
-          if (Ap[lr.row + 1] - Ap[lr.row] <= kPartitionedFrom) { S->rem_rows.push_back(lr.row); continue; }
+          if (Ap[lr.row + 1] - Ap[lr.row] <= whole) { S->rem_rows.push_back(lr.row); continue; }
           tf::LongRow nr{lr.row, (int)keep_chunks.size(), lr.count, 0};
           for (int c = 0; c < lr.count; ++c) {
             tf::LongChunk ch = S->long_chunks[lr.first + c];
@@ -637,7 +643,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         S->long_rows.swap(keep_rows);
         S->long_chunks.swap(keep_chunks);
         std::sort(S->rem_rows.begin(), S->rem_rows.end());
-        S->opts.long_row_nnz = o.long_row_nnz = kPartitionedFrom;
+        S->opts.long_row_nnz = o.long_row_nnz = whole;
         long_nnz = 0;
         for (const auto &lr : S->long_rows) long_nnz += Ap[lr.row + 1] - Ap[lr.row];
       }
@@ -746,19 +752,32 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // Remainder rows of similar length go together: a lane group walks a row alone, so a
     // workgroup is as slow as its longest row.  Order is kept inside a length class, and a
     // matrix whose rows all fall in one class keeps its order entirely.
+    // Where the order has no locality to keep (entries a long way from the diagonal on average), the rows go by falling length:
+    // the row product of an R-MAT graph of 2^18 nodes, N = 40 / 64 / 128: 117 / 121 / 195 -> 109 / 115 / 188 us, 2^20 nodes 354 / 434 / 819
+    // -> 323 / 408 / 790.
     {
       auto cls = [&](int i) {
         const int len = Ap[i + 1] - Ap[i];
         return len <= 8 ? 0 : len <= 32 ? 1 : len <= 128 ? 2 : len <= 512 ? 3 : 4;
       };
+      auto scattered = [&] {  // (65,536 rows are looked at)
+        const size_t n = S->rem_rows.size(), step = n / 65536 + 1;
+        double far = 0;
+        long long entries = 0;
+        for (size_t q = 0; q < n; q += step) {
+          const int i = S->rem_rows[q];
+          for (int k = Ap[i]; k < Ap[i + 1]; ++k) far += std::abs(Ai[k] - (double)i * M / L);
+          entries += Ap[i + 1] - Ap[i];
+        }
+        return far * 8 > (double)M * entries;
+      };
       std::vector<int> byc[5];
-      // Rows without entries, when they are many (half of the nodes of an R-MAT graph are isolated), leave
-      // the list: a row of zeros needs no lane group and no row pointers, a fill kernel over the rows'
-      // own list writes it (the row kernel of the 2^21-node R-MAT step: 0.69 -> 0.50 ms, the fill 0.12 ms).
+      // Rows without entries, when they are many (half of the nodes of an R-MAT graph are isolated), leave the list: a row of
+      // zeros needs no lane group of its own and no row pointers, the row kernels clear it beside their other work.
       {
         size_t n_empty = 0;
         for (int i : S->rem_rows) n_empty += Ap[i + 1] == Ap[i];
-        if (n_empty >= 4096 && n_empty * 8 >= S->rem_rows.size()) {
+        if (n_empty >= 4096 && n_empty * 8 >= S->rem_rows.size() && n_empty < S->rem_rows.size()) {
           std::vector<int> keep;
           keep.reserve(S->rem_rows.size() - n_empty);
           S->zero_rows.reserve(n_empty);
@@ -772,8 +791,16 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       size_t most = 0;
       for (auto &v : byc) most = std::max(most, v.size());
       if (!(rows_only && most * 8 >= S->rem_rows.size() * 7)) {
-        S->rem_rows.clear();
-        for (auto &v : byc) S->rem_rows.insert(S->rem_rows.end(), v.begin(), v.end());
+        if (scattered()) {
+          std::vector<int> at(o.long_row_nnz + 2, 0);  // (no remainder row is longer)
+          const std::vector<int> rows(S->rem_rows);
+          for (int i : rows) ++at[o.long_row_nnz - (Ap[i + 1] - Ap[i]) + 1];
+          for (int len = 0; len <= o.long_row_nnz; ++len) at[len + 1] += at[len];
+          for (int i : rows) S->rem_rows[at[o.long_row_nnz - (Ap[i + 1] - Ap[i])]++] = i;
+        } else {
+          S->rem_rows.clear();
+          for (auto &v : byc) S->rem_rows.insert(S->rem_rows.end(), v.begin(), v.end());
+        }
       }
       S->rem_identity = (int)S->rem_rows.size() == L;
       for (int q = 0; q < L && S->rem_identity; ++q) S->rem_identity = (S->rem_rows[q] == q);

@@ -58,6 +58,9 @@ struct RowsArgs {
   float *Y = nullptr;
   int ldy = 0, N = 0;
   int accumulate = 0, streaming = 0, compact = 0, relu = 0;
+  // rows of Y without entries that are not among n_rows: cleared on the way (n_zero > 0 needs n_rows > 0)
+  const int *zero_rows = nullptr;
+  int n_zero = 0;
   // chunks of long rows, a workgroup each; slot < 0: the row's only chunk, which goes straight to Y
   // (their k_begin and k_end count in chunk_Ai and chunk_Ax, the matrix' own arrays)
   const LongChunk *chunks = nullptr;

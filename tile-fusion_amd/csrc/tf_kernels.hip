@@ -521,17 +521,6 @@ __global__ void copy_cols_kernel(const float *__restrict__ src, int src_rows, in
   }
 }
 
-// Rows of zeros: Y[rows[q], :] = 0 (second-op rows without entries), V floats per thread.
-template <int V>
-__global__ void zero_rows_kernel(const int *__restrict__ rows, size_t units, float *__restrict__ Y, int N) {
-  const int per_row = N / V;
-  for (size_t u = blockIdx.x * (size_t)blockDim.x + threadIdx.x; u < units; u += (size_t)gridDim.x * blockDim.x) {
-    const size_t q = u / per_row;
-    const int c = (int)(u - q * per_row) * V;
-    store_streaming<V>(Y + (size_t)rows[q] * N + c, vzero<V>());  // (plain stores: this launch 5 % faster, the next one 5 % slower)
-  }
-}
-
 // p = max(p, 0) over n values: four per thread, and the up to three values behind the last four one each.
 __global__ void relu_kernel(float *__restrict__ p, size_t n) {
   const size_t n4 = n / 4;
@@ -2066,15 +2055,6 @@ hipError_t launch_pad(const float *src, int src_rows, int ld_src, float *dst, in
 hipError_t launch_transpose_pad(const float *src, int src_rows, int ld_src, int row0, int n_rows, float *dst, int rows, int cols, hipStream_t st) {
   if (row0 < 0 || row0 + n_rows > src_rows || (long long)rows * cols > INT_MAX) return hipErrorInvalidValue;
   hipLaunchKernelGGL(transpose_pad_kernel, dim3(std::min((rows * cols + 255) / 256, 1024)), dim3(256), 0, st, src, ld_src, row0, n_rows, dst, rows, cols);
-  return hipGetLastError();
-}
-
-hipError_t launch_zero_rows(const int *rows, int n_rows, float *Y, int N, hipStream_t st) {
-  if (n_rows <= 0) return hipSuccess;
-  const size_t units = (size_t)n_rows * (N % 4 == 0 ? N / 4 : N);
-  const unsigned blocks = (unsigned)std::min<size_t>((units + 255) / 256, 1u << 20);
-  if (N % 4 == 0) hipLaunchKernelGGL((zero_rows_kernel<4>), dim3(blocks), dim3(256), 0, st, rows, units, Y, N);
-  else hipLaunchKernelGGL((zero_rows_kernel<1>), dim3(blocks), dim3(256), 0, st, rows, units, Y, N);
   return hipGetLastError();
 }
 
