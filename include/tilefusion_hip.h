@@ -478,7 +478,7 @@ tf_status tf_gemm(const tf_dense *X, const tf_dense *W, tf_dense *Y, void *strea
  * or less: the step back through a ReLU whose output is `mask`. */
 tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *Y, const tf_dense *mask, unsigned flags, void *stream);
 /* Y (N x K) = G^T * X with G M x N and X M x K: the gradient of a layer's weights.  `workspace`: device memory of
- * tf_weight_grad_workspace(M, N, K) bytes, in use until the call's work on `stream` is done. */
+ * tf_weight_grad_workspace(M, N, K) bytes (null where that is 0), in use until the call's work on `stream` is done. */
 tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream);
 size_t tf_weight_grad_workspace(int M, int N, int K);
 

@@ -146,10 +146,15 @@ static tf_status hip_fail(hipError_t e, const char *what) {
   } while (0)
 
 int default_compute_units() {
+  static std::atomic<int> known[64];  // per device, once asked for
   int dev = 0, cu = 0;
-  if (hipGetDevice(&dev) == hipSuccess &&
-      hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cu > 0)
-    return cu;
+  if (hipGetDevice(&dev) == hipSuccess) {
+    if (dev >= 0 && dev < 64 && (cu = known[dev].load(std::memory_order_relaxed)) > 0) return cu;
+    if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cu > 0) {
+      if (dev >= 0 && dev < 64) known[dev].store(cu, std::memory_order_relaxed);
+      return cu;
+    }
+  }
   (void)hipGetLastError();
   return 256;
 }
@@ -1211,10 +1216,11 @@ extern "C" size_t tf_weight_grad_workspace(int M, int N, int K) {
 }
 
 extern "C" tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream) {
-  if (!G || !X || !Y || !workspace) return fail(TF_EINVAL, "tf_weight_grad: null argument");
+  if (!G || !X || !Y) return fail(TF_EINVAL, "tf_weight_grad: null argument");
   if (G->M != X->M || Y->M != G->N || Y->N != X->N)
     return fail(TF_EINVAL, "tf_weight_grad: shapes G %d x %d, X %d x %d, Y %d x %d", G->M, G->N, X->M, X->N, Y->M, Y->N);
   const tf::WeightGradPlan p = tf::plan_weight_grad(G->M, G->N, X->N, tf::default_compute_units());
+  if (p.partial_floats && !workspace) return fail(TF_EINVAL, "tf_weight_grad: %zu bytes of workspace needed", p.partial_floats * sizeof(float));
   TF_HIP(tf::launch_weight_grad(p, G->d, G->N, X->d, X->N, G->M, workspace, Y->d, static_cast<hipStream_t>(stream)));
   return TF_OK;
 }

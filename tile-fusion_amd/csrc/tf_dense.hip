@@ -17,7 +17,7 @@ typedef float acc16 __attribute__((ext_vector_type(16)));
 // tile and take every KW-th step of 16 values of k each (their sums are added through LDS in a fixed order), so that
 // a product of few rows still fills the device: 3,000 rows x 500 x 32 are 376 workgroups whose wavefronts have 8
 // steps each, where one 32-row block per wavefront with all of K is 94 wavefronts of 250 MFMAs in a chain
-// (13.2 us; 3 us here).  X and W come straight from global memory -- the wavefronts of a workgroup read the same W, which L1
+// (13.2 us; 6.9 us here).  X and W come straight from global memory -- the wavefronts of a workgroup read the same W, which L1
 // serves -- with k permuted inside a step the same way for both operands: lane (j, h) holds k = 16 s + 4 h + t for
 // MFMA t, one 16-byte load of X, and of W when it is stored N x K.  Columns are dealt to lanes CB at a time
 // (column CB j + cb to column block cb), so that a K x N stored W is loaded, and Y stored, CB floats per lane.
@@ -337,6 +337,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // Bound: the rows of X and G from HBM, or fp32 MFMA when 2 N K / 4 (N + K) exceeds 31 FLOP per byte.
 // ---------------------------------------------------------------------------------
 constexpr int kWgUnroll = 4;  // pairs of rows in flight per wavefront
+constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel
 
 template <int NB, int KB>
 __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__restrict__ G, int N, const float *__restrict__ X,
@@ -450,9 +451,59 @@ __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float *__
   Y[(size_t)n * K + k] = s;
 }
 
+// The same for few rows in one launch: a workgroup of sixteen wavefronts per 16 x 16 tile of Y (v_mfma_f32_16x16x4_f32, so that
+// there are tiles enough) and no partial sums in memory.  What counts is the chain of loads: a wavefront keeps sixteen steps of four
+// rows in flight, eight being multiplied and the next eight on their way.  Two launches / this one, us: 7 x 32,
+// 1,000 rows 6.3 / 3.8, 4,096 7.2 / 8.0, 8,192 9.8 / 14; 32 x 500, 3,000 rows 12.0 / 9.0; 128 x 512, 4,096 rows 20.9 / 11.2 -- and a launch less for
+// the host, which is what a small model waits for.
+__global__ __launch_bounds__(1024, 4) void weight_grad_few_kernel(const float *__restrict__ G, int N, const float *__restrict__ X, int K, int M,
+                                                                  int k_tiles, float *__restrict__ Y) {
+  constexpr int W = 16, U = 8;
+  __shared__ float red[W][4][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
+  const int n0 = blockIdx.x / k_tiles * 16, k0 = blockIdx.x % k_tiles * 16;
+  // rows past the last one lie past the end of both buffers: their loads return zeros
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(G), 0, M * N * 4, 0x00020000),
+                               xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(X), 0, M * K * 4, 0x00020000);
+  unsigned g_off = ((4 * wave + h) * N + min(n0 + j, N - 1)) * 4u, x_off = ((4 * wave + h) * K + min(k0 + j, K - 1)) * 4u;
+  acc4 acc = 0.f;
+  struct operands { float g[U], x[U]; };
+  auto load = [&]() __attribute__((always_inline)) {
+    operands o;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      o.g[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gr, (int)g_off, 0, 0));
+      o.x[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)x_off, 0, 0));
+      g_off += 4 * W * 4u * N;
+      x_off += 4 * W * 4u * K;
+    }
+    return o;
+  };
+  operands cur = load();
+  for (int m0 = 4 * wave; m0 < M; m0 += 4 * W * U) {
+    const operands nxt = load();
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.g[u], cur.x[u], acc, 0, 0, 0);
+    cur = nxt;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc[r];
+  __syncthreads();
+  if (wave >= 4) return;
+  float s = red[0][wave][lane];  // wavefront r adds up register r
+#pragma unroll
+  for (int w = 1; w < W; ++w) s += red[w][wave][lane];
+  const int n = n0 + 4 * h + wave, k = k0 + j;
+  if (n < N && k < K) Y[(size_t)n * K + k] = s;
+}
+
 // How launch_weight_grad cuts the product: chunks of Y, groups of rows.
 WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
   WeightGradPlan p;
+  // (some more tiles than compute units; 32-bit offsets, with a thousand rows past the end)
+  p.few = M <= kWgFewRows && ((N + 15) / 16) * ((K + 15) / 16) <= 2 * compute_units && std::max(N, K) <= 16384;
+  p.partial_floats = 0;
+  if (p.few) return p;
   p.nb = N > 32 ? 2 : 1;
   p.n_chunks = (N + 32 * p.nb - 1) / (32 * p.nb);
   // the width of X in the fewest chunks of at most 160 columns, evenly (300 = 2 x 160, 128 = 1 x 128, 500 = 4 x 128)
@@ -470,6 +521,11 @@ WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
 }
 
 hipError_t launch_weight_grad(const WeightGradPlan &p, const float *G, int N, const float *X, int K, int M, float *partial, float *Y, hipStream_t st) {
+  if (p.few) {
+    const int k_tiles = (K + 15) / 16, n_tiles = (N + 15) / 16;
+    hipLaunchKernelGGL(weight_grad_few_kernel, dim3(k_tiles * n_tiles), dim3(1024), 0, st, G, N, X, K, M, k_tiles, Y);
+    return hipGetLastError();
+  }
   const int chunks = p.n_chunks * p.k_chunks;
   const dim3 grid(p.groups, chunks);
 #define CALL2(NB_, KB_) \

@@ -257,9 +257,10 @@ Tensor weight_grad(const Tensor &t, const Tensor &x_) {
   c10::OptionalDeviceGuard guard(t.device());
   const int M = (int)t.size(0), N = (int)t.size(1), K = (int)x.size(1);
   Tensor out = at::empty({N, K}, t.options());
-  Tensor ws = at::empty({(int64_t)(tf_weight_grad_workspace(M, N, K) / sizeof(float))}, t.options());
+  const int64_t floats = (int64_t)(tf_weight_grad_workspace(M, N, K) / sizeof(float));
+  const Tensor ws = floats > 0 ? at::empty({floats}, t.options()) : Tensor();
   Dense tb(t), xb(x), ob(out);
-  check(tf_weight_grad(tb, xb, ob, ws.data_ptr<float>(), stream_of(t)));
+  check(tf_weight_grad(tb, xb, ob, floats > 0 ? ws.data_ptr<float>() : nullptr, stream_of(t)));
   return out;
 }
 
