@@ -91,7 +91,7 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
                                            const float *, int, const float *, const int *, const int *,
                                            const float *, int, float *, int, int, int, int, hipStream_t);
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
-hipError_t launch_spmm_gemm(const RowsArgs &, const float *, int, int, const GemmOut &, hipStream_t);
+hipError_t launch_spmm_gemm(RowsArgs, const RowsHow &, const float *, int, int, const GemmOut &, hipStream_t);
 hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const GemmOut &, int, hipStream_t);
 WeightGradPlan plan_weight_grad(int, int, int, int);
@@ -392,7 +392,7 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
   a.Ap = A->p; a.Ai = A->i; a.Ax = A->x;
   a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = ldd; a.N = N;
   a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
-  how.xcd_chunk_rows = s->xcd_chunk_rows;
+  how.xcd_chunk_rows = s->row_deal;
   a.zero_rows = d->zero_rows;
   a.n_zero = r.accumulate && !r.relu ? 0 : (int)s->zero_rows.size();  // (D += 0 needs nothing)
   a.chunks = d->long_chunks;
@@ -981,7 +981,7 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
         tf::RowsHow rows_how;
         if ((rc = tf::remainder_rows(A, rows, tf::Remainder{B->d, K, K, B->M, D->d, acc, relu}, st, a, rows_how))) return rc;
         a.ldy = N;
-        TF_PHASE(rows, "spmm_gemm_kernel", st, tf::launch_spmm_gemm(a, C->d, c_t, N, how, st));
+        TF_PHASE(rows, "spmm_gemm_kernel", st, tf::launch_spmm_gemm(a, rows_how, C->d, c_t, N, how, st));
         return TF_OK;
       }
       rc = tf::run_remainder(A, rows, tf::Remainder{B->d, K, K, B->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);

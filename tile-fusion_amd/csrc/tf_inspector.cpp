@@ -104,8 +104,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    kernel's do not: 16 entries in a band of 32, 50,000 rows, N = 16 / 24 / 48: 16.5 / 16.7 / 24.5 us in tiles, 10.7 /
 //    15.2 / 21.2 us as two products; 300 x 300 grid, N = 32: 48 and 19 us.
 //  * Marching runs with few rows to march over: a run walks at least two planes before its first row and the device
-//    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 18 us, 110,592 rows 33 / 39 us,
-//    2^21 rows 341 / 599 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
+//    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 13 us, 110,592 rows 34 / 28 us,
+//    216,000 rows 48 / 50 us (N = 128: 97 / 121), 2^21 rows 341 / 610 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
 //    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
 //
 // GeMM-SpMM:
@@ -141,7 +141,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || !S->gemm_stream));
     if (S->spmm_first) N = K;
   } else if (S->march)
-    want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 88000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
+    want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
   else
     want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;
   if (!want) return TF_OK;
@@ -786,12 +786,13 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         }
       }
       for (int i : S->rem_rows) byc[cls(i)].push_back(i);
-      // (a product of its own whose rows are nearly all of one class -- a stencil and its boundary -- stays in order too: the
+      // (a product of all rows whose rows are nearly all of one class -- a stencil and its boundary -- stays in order too: the
       // list costs its rows an indirection and the entries a copy; 27 points, 40^3, N = 16: 21.1 us through a list, 19.1 without)
       size_t most = 0;
       for (auto &v : byc) most = std::max(most, v.size());
-      if (!(rows_only && most * 8 >= S->rem_rows.size() * 7)) {
-        if (scattered()) {
+      const bool far = scattered();
+      if (!((int)S->rem_rows.size() == L && most * 8 >= S->rem_rows.size() * 7)) {
+        if (far) {
           std::vector<int> at(o.long_row_nnz + 2, 0);  // (no remainder row is longer)
           const std::vector<int> rows(S->rem_rows);
           for (int i : rows) ++at[o.long_row_nnz - (Ap[i + 1] - Ap[i]) + 1];
@@ -804,6 +805,18 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       }
       S->rem_identity = (int)S->rem_rows.size() == L;
       for (int q = 0; q < L && S->rem_identity; ++q) S->rem_identity = (S->rem_rows[q] == q);
+      // A product of all rows in order, of a matrix with locality: one contiguous run of rows per XCD, so that a row of X is
+      // gathered into one L2, not into all eight -- where no XCD's run has much more work than the others'.  Two products, workgroups dealt
+      // to the XCDs in turn / a run each: 7 points, 60^3, N = 32, 44 / 30 us, 30 x 40 x 50, N = 64, 30.5 / 18; 27 points, 24^3, N = 32, 13.1 / 10.8, 60^3
+      // 85 / 75; 5 points, 900^2, N = 32, 120 / 95.  Past 100 MB of X the runs' planes outgrow the Infinity Cache together, and turns of
+      // 512 rows are better: 7 points, 110^3, N = 32, 293 / 252 / 231 in turns.
+      S->row_deal = o.xcd_chunk_rows;
+      if (S->rem_identity && !far && o.xcd_chunk_rows == 0) {
+        constexpr int kXcds = 8;
+        long long most_work = 0;
+        for (int x = 0; x < kXcds; ++x) most_work = std::max<long long>(most_work, Ap[(x + 1LL) * L / kXcds] - Ap[(long long)x * L / kXcds]);
+        if (most_work * kXcds * 100 <= 115LL * nnz) S->row_deal = (long long)M * o.N * 4 <= (100LL << 20) ? -1 : 512;
+      }
       // Reordered adjacency (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653): a list that is
       // not simply all rows in order gets its rows stored side by side in list order, so that a
       // workgroup reads one stretch of columns and values instead of one stretch per row.

@@ -163,6 +163,7 @@ struct tf_schedule {
   bool rem_flagged = false;  // rem_col carries the "cold" mark in the top bit of some columns (short_row_hot_bytes)
   int rem_hot_rows = 0;      // intermediate rows left unmarked
   int xcd_chunk_rows = 0;           // rows per XCD turn of the row kernels (0: one contiguous run per XCD)
+  int row_deal = 0;  // how the row kernels deal their rows to the XCDs: xcd_chunk_rows where given, else the inspector's choice
   std::vector<tf::LongChunk> long_chunks;
   std::vector<tf::LongRow> long_rows;
   // Long rows cut by column instead (long_part): the most-read intermediate rows are dealt to 8

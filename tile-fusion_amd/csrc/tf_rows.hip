@@ -309,7 +309,9 @@ __global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(cons
   const int K = a.N, ld = (K + 15) / 16 * 16 + 4;            // (four floats behind a row: its reads start in other banks)
   const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X), 0, (int)(a.x_rows * a.ldx * 4u), 0x00020000);
-  const int q0 = blockIdx.x * R;
+  const int block = xcd_contiguous(blockIdx.x, a.per_xcd);
+  if (block >= a.n_blocks) return;
+  const int q0 = block * R;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
   const int rt = wave % RT, S = (K + 15) / 16, full = K / 16;
   const int first_col = wave / RT * 16 * V + V * j;
@@ -481,6 +483,15 @@ inline bool xcd_remap_on() {
   return on;
 }
 
+// How a.n_blocks workgroups of `rows` rows are dealt to the XCDs -- 0: workgroup b takes block b; > 0: chunks of rows per XCD turn;
+// < 0: one contiguous run per XCD -- and the workgroups to launch for it.
+int deal_to_xcds(RowsArgs &a, int xcd_chunk_rows, int rows) {
+  const int n = a.n_blocks, want = xcd_chunk_rows > 0 ? std::max(1, xcd_chunk_rows / rows) : 0;
+  a.per_xcd = xcd_chunk_rows == 0 || !xcd_remap_on() ? 0 : (want <= 0 || want * kXcds >= n) ? (n + kXcds - 1) / kXcds : want;
+  const int per = std::max(a.per_xcd, 1) * kXcds;
+  return (n + per - 1) / per * per;
+}
+
 #define TF_DISPATCH_ROWS(S_, CALL)                                              \
   do {                                                                          \
     if (S_.V == 1) { if (S_.LPR == 4) { CALL(1, 4); } else { CALL(1, 64); } }   \
@@ -500,12 +511,9 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   if (a.slices > 1) s.LPR = 8;
   const int G = kBlock / s.LPR;
   a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
-  // 0: workgroup b takes block b; > 0: chunks of rows per XCD turn; < 0: one contiguous run per XCD
-  const int n = a.n_blocks, want = how.xcd_chunk_rows > 0 ? std::max(1, how.xcd_chunk_rows / G) : 0;
-  a.per_xcd = how.xcd_chunk_rows == 0 || !xcd_remap_on() ? 0 : (want <= 0 || want * kXcds >= n) ? (n + kXcds - 1) / kXcds : want;
-  const int per = std::max(a.per_xcd, 1) * kXcds;
+  const int blocks = deal_to_xcds(a, how.xcd_chunk_rows, G);
   const int turns = kXcds / a.slices;  // row blocks per eight workgroups
-  const dim3 grid(a.chunk_blocks + (a.slices > 1 ? (n + turns - 1) / turns * kXcds : (n + per - 1) / per * per));
+  const dim3 grid(a.chunk_blocks + (a.slices > 1 ? (a.n_blocks + turns - 1) / turns * kXcds : blocks));
 #define CALL3(V_, L_, WALK_, CH_) hipLaunchKernelGGL((spmm_rows_kernel<V_, L_, WALK_, CH_>), grid, dim3(kBlock), 0, st, a)
 #define CALL2(V_, L_, WALK_) do { if (a.n_chunks > 0) { CALL3(V_, L_, WALK_, true); } else { CALL3(V_, L_, WALK_, false); } } while (0)
 #define CALLP(V_, L_) do { if constexpr (V_ == 4) { CALL2(V_, L_, kDpp); } } while (0)
@@ -528,12 +536,13 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
 }
 
 // Y = (A X) W for the rows of `a` (a.N = K the columns of X, a.ldy that of Y): K from 4 up, X of up to 2 GB, no long rows.
-hipError_t launch_spmm_gemm(const RowsArgs &a, const float *W, int wt, int N, const GemmOut &how, hipStream_t st) {
+hipError_t launch_spmm_gemm(RowsArgs a, const RowsHow &rows, const float *W, int wt, int N, const GemmOut &how, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
   if (a.N < 4 || a.n_chunks > 0 || (unsigned long long)a.x_rows * a.ldx * 4 > 0x80000000ull) return hipErrorInvalidValue;
   const RowShape s = row_shape(a.N, 0);
   const int R = a.n_rows < 24000 ? 16 : 64, lds = R * ((a.N + 15) / 16 * 16 + 4) * 4;
-  const dim3 grid((a.n_rows + R - 1) / R);
+  a.n_blocks = (a.n_rows + R - 1) / R;
+  const dim3 grid(deal_to_xcds(a, rows.xcd_chunk_rows, R));
   hipError_t err = hipSuccess;
 #define CALL3(L_, R_, V_, WT_)                                                                                                         \
   do {                                                                                                                                 \
