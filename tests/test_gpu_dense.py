@@ -36,6 +36,48 @@ def test_gemm_of_any_shape(gpu, tf, M, K, N, w_t):
         assert rel(Y.to_numpy(), ref) <= 1e-5, (mask is not None)
 
 
+@pytest.mark.parametrize("M,K,N", [(13001, 4, 33), (12999, 17, 64), (20481, 18, 17), (13007, 19, 129), (13001, 66, 97), (262145, 131, 35), (40000, 100, 100),
+                                   (13000, 5, 257)])
+def test_gemm_panel_edges(gpu, tf, M, K, N):
+    """W in LDS: steps of k that end after one to four values, a last lane whose columns overlap its neighbour's, rows and panels
+    that end early; non-finite values beside the edges stay where they are."""
+    say(f"gemm panel {M} x {K} x {N}")
+    rng = np.random.default_rng(M + K + N)
+    X, W = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    X[M - 2, K - 1] = np.inf
+    m = rng.uniform(-1, 1, (M, N)).astype(np.float32)
+    Xd, md = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(m)
+    with np.errstate(invalid="ignore"):
+        want = X.astype(np.float64) @ W.astype(np.float64)
+    ok = np.arange(M) != M - 2
+    for w_t in (False, True):
+        Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if w_t else W)
+        for mask in (None, md):
+            Y = tf.DenseMatrix.from_numpy(np.full((M, N), np.nan, np.float32))
+            assert tf.lib().tf_gemm_ex(Xd.h, Wd.h, Y.h, mask.h if mask else None, C_TRANSPOSED if w_t else 0, None) == 0
+            tf.device_synchronize()
+            got, ref = Y.to_numpy(), want if mask is None else np.where(m > 0, want, 0.0)
+            assert rel(got[ok], ref[ok]) <= 1e-5
+            assert np.array_equal(np.isinf(got[~ok]), np.isinf(ref[~ok]))
+
+
+@pytest.mark.parametrize("K,N", [(129, 33), (64, 100), (18, 128)])
+def test_gemm_of_listed_rows(gpu, tf, K, N):
+    """The rows an R-MAT graph reads, gathered by the product itself and stored in the order of their reads."""
+    say(f"listed rows {K} x {N}")
+    A = tf.workloads.rmat(15, 8 << 15, seed=5)
+    M = A.shape[0]
+    rng = np.random.default_rng(K)
+    X, W = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    D = tf.DenseMatrix(M, N)
+    Xd, Wd = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(W)
+    assert tf.lib().tf_gemm_spmm(Ah.to_device().h, Xd.h, Wd.h, D.h, S.h, 0, None) == 0
+    tf.device_synchronize()
+    assert rel(D.to_numpy(), A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))) <= 1e-5
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 7, 5), (33, 32, 128), (3000, 7, 32), (3000, 32, 500), (10000, 64, 300), (5001, 33, 161),
                                    (100000, 64, 128), (20011, 130, 31), (64, 300, 97), (4096, 65, 33), (4097, 31, 30)])
 def test_weight_gradient(gpu, tf, M, N, K):

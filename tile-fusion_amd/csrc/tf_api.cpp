@@ -877,10 +877,11 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
 }
 
 // W as the row GEMM takes it: row-major K x N with N a multiple of 32 up to 256, K of 8, small enough for LDS.  Its 32-row
-// blocks on two wavefronts per SIMD need 256 rows per compute unit to be the faster kernel (128 x 128: 23 us at 32,000 rows
-// where launch_gemm_any takes 19, 27 at 64,000 where that takes 29, 20 at 4,000 where that takes 6).
+// blocks on two wavefronts per SIMD are the faster kernel from 1,024 rows per compute unit on, the other one balances fewer better (us,
+// 64 x 128 / 128 x 64 / 128 x 128, this one and launch_gemm_any: 100,000 rows 34 25 52 and 26 24 42, 131,072 rows 30 26 46 and 28 26 44, 262,144 rows
+// 52 46 82 and 55 50 82).
 static bool row_gemm_takes(long long rows, int K, int N, int compute_units) {
-  return rows >= 256LL * compute_units && K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072;
+  return rows >= 1024LL * compute_units && K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072;
 }
 
 // What a GeMM-SpMM pass reads and writes: B (M x K), C (K x N, or N x K with c_t) and D (L x N).

@@ -123,13 +123,21 @@ __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restric
 // with no barrier, its rows of X requested a group of kGemmAhead steps ahead (the first group before W is staged).
 // Column block (v, q) of lane j is column 16 V q + V j + v: a lane reads V adjacent values of W per k and stores V adjacent columns of
 // Y, sixteen lanes side by side.  Sixteen wavefronts per compute unit (up to 128 registers each), so that a SIMD has
-// three others to feed its matrix core while one waits: 131,072 x 300 x 64 takes 62 us (139 us with
+// three others to feed its matrix core while one waits: 131,072 x 300 x 64 takes 54 us (139 us with
 // every row tile reading W from L2; 33 us and 39 us for a padded copy of X in 32-row blocks).
 // Bound: X and Y from HBM for up to 64 columns, fp32 MFMA beyond.
 // ---------------------------------------------------------------------------------
 constexpr int kGemmAhead = 4;  // steps of 16 values of k per group of operands
 
-template <int V, int Q, bool WT>
+// Rows in order and values as they are; with zeros where the mask is zero or less; rows of a list, values as they are; all else.
+enum { kPlain, kMasked, kListed, kAnyOut };
+
+// The loop has no load or store under a condition, so that a wait for a group of operands leaves younger requests and the
+// stores before them in flight: rows past the last one are the last one again and store its values once more, a lane whose
+// V columns reach past the last one works on the last V, and the last step's values of k past K are cleared in registers.
+// (Conditions around them, us: 262,144 x 64 x 64 37, 128 x 64 58, 64 x 128 61; without 29, 50, 55;
+// 30,000 x 300 x 64 23.0, 100 x 83 15.8; without 18.3, 13.1.)
+template <int V, int Q, bool WT, int OUT>
 __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
                                                           float *__restrict__ Y, int ldy, const int *__restrict__ rows,
                                                           int y_by_row, int n_rows, int K, int N,
@@ -140,45 +148,31 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
   const int panel0 = blockIdx.y * P, S = (K + 15) / 16, G = (S + A - 1) / A;
   const int n_blocks = (n_rows + 15) / 16, total_waves = gridDim.x * waves, gw = blockIdx.x * waves + wave;
   const int b0 = (int)((long long)gw * n_blocks / total_waves), b1 = (int)((long long)(gw + 1) * n_blocks / total_waves);
-  const int groups = (b1 - b0) * G;
+  auto column = [&](int n) { return OUT == kAnyOut ? min(panel0 + n, N - 1) : min(panel0 + n - n % V, N - V) + n % V; };  // of W
   struct operands { f4v a[A]; };
-  // The operands of group gi (block b0 + gi / G, steps A (gi % G) ..); groups past the last are the last again.
-  int gi_next = 0, g_next = 0, b_next = b0;
-  const float *xp = X;
-  auto row_of = [&](int b) {
-    const int q = min(b * 16 + j, n_rows - 1);
-    return X + (size_t)(rows ? rows[q] : q) * ldx + 4 * h;
+  auto row_index = [&](int b) __attribute__((always_inline)) {
+    const int q = min(min(b, b1 - 1) * 16 + j, n_rows - 1);
+    if constexpr (OUT == kPlain || OUT == kMasked) return q;
+    else if constexpr (OUT == kListed) return rows[q];
+    else return rows ? rows[q] : q;
   };
-  auto load_next = [&]() __attribute__((always_inline)) {
+  auto load = [&](const float *xp, int g) __attribute__((always_inline)) {
     operands o;
 #pragma unroll
-    for (int u = 0; u < A; ++u) {
-      const int s = min(g_next * A + u, S - 1);
-      if (16 * s + 16 <= K) {
-        o.a[u] = *reinterpret_cast<const f4u *>(xp + 16 * s);
-      } else if (K % 4 == 0) {
-        o.a[u] = 0.f;
-        if (16 * s + 4 * h < K) o.a[u] = *reinterpret_cast<const f4u *>(xp + 16 * s);
-      } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) o.a[u][t] = 16 * s + 4 * h + t < K ? xp[16 * s + t] : 0.f;
-      }
-    }
-    if (++gi_next < groups && ++g_next == G) {
-      g_next = 0;
-      xp = row_of(++b_next);
-    }
+    for (int u = 0; u < A; ++u) o.a[u] = *reinterpret_cast<const f4u *>(xp + min(16 * (g * A + u) + 4 * h, K - 4));
     return o;
   };
-  operands cur, nxt;
-  if (groups > 0) {
-    xp = row_of(b0);
-    cur = load_next();
+  const float *xp = X;
+  operands cur;
+  int next_row = 0;  // of this lane in the block after the next one to begin
+  if (b0 < b1) {
+    xp = X + (size_t)row_index(b0) * ldx;
+    next_row = row_index(b0 + 1);
+    cur = load(xp, 0);
   }
   // W into LDS: a column's sixteen values of one step per thread and item, all requested before the first is stored
   for (int it = threadIdx.x; it < S * P; it += blockDim.x) {
-    const int n = it % P, s = it / P, c = min(panel0 + n, N - 1);
-    const bool in = panel0 + n < N;
+    const int n = it % P, s = it / P, c = column(n);
     f4v v[4];
     if (16 * s + 16 <= K) {
 #pragma unroll
@@ -201,66 +195,98 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) wlds[(16 * s + 4 * u + t) * P + n] = in ? v[u][t] : 0.f;
+      for (int t = 0; t < 4; ++t) wlds[(16 * s + 4 * u + t) * P + n] = v[u][t];
   }
   __syncthreads();
   acc4 acc[Q][V];
   const float *wl = wlds + 4 * h * P + V * j;
-  auto run = [&](int g, const operands &o) __attribute__((always_inline)) {
+  auto step = [&](int s, const f4v &a) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < A; ++u) {
-      const int s = g * A + u;
-      if (s >= S) break;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float *w = wl + (16 * s + t) * P;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          typedef float wv __attribute__((ext_vector_type(V)));
-          wv b;
-          if constexpr (V == 1) b[0] = w[16 * q]; else b = *reinterpret_cast<const wv *>(w + 16 * V * q);
-#pragma unroll
-          for (int v = 0; v < V; ++v) acc[q][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[u][t], b[v], acc[q][v], 0, 0, 0);
-        }
-      }
-    }
-  };
-  auto store = [&](int b) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int x = b * 16 + 4 * h + r;
-      if (x >= n_rows) continue;
-      const size_t row = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
+    for (int t = 0; t < 4; ++t) {
+      const float *w = wl + (16 * s + t) * P;
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        const int c = panel0 + 16 * V * q + V * j;
-        cvec<V> out;
+        typedef float wv __attribute__((ext_vector_type(V)));
+        wv b;
+        if constexpr (V == 1) b[0] = w[16 * q]; else b = *reinterpret_cast<const wv *>(w + 16 * V * q);
 #pragma unroll
-        for (int v = 0; v < V; ++v) out.v[v] = acc[q][v][r];
-        gemm_store<V>(Y, row + c, out, N - c, out_how);
+        for (int v = 0; v < V; ++v) acc[q][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[v], acc[q][v], 0, 0, 0);
       }
     }
   };
-  int b = b0, g = 0;
-  auto step = [&](const operands &o) __attribute__((always_inline)) {
-    if (g == 0) {
+  auto run = [&](int g, const operands &o) __attribute__((always_inline)) {
+    if (16 * A * (g + 1) <= K) {
 #pragma unroll
-      for (int q = 0; q < Q; ++q)
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc[q][v] = 0.f;
+      for (int u = 0; u < A; ++u) step(g * A + u, o.a[u]);
+      return;
     }
-    run(g, o);
-    if (++g == G) {
-      store(b++);
-      g = 0;
+#pragma unroll
+    for (int u = 0; u < A; ++u) {
+      const int s = g * A + u, at = 16 * s + 4 * h, d = at - min(at, K - 4);
+      if (s >= S) break;
+      // the step's values are d places behind those that were loaded, zeros follow
+      f4v v = o.a[u];
+      v = d & 1 ? f4v{v[1], v[2], v[3], 0.f} : v;
+      v = d & 2 ? f4v{v[2], v[3], 0.f, 0.f} : v;
+      v = d >= 4 ? f4v{0.f, 0.f, 0.f, 0.f} : v;
+      step(s, v);
     }
   };
-  for (int gi = 0; gi < groups; gi += 2) {
-    nxt = load_next();
-    step(cur);
-    if (gi + 1 < groups) {
-      cur = load_next();
-      step(nxt);
+  for (int b = b0; b < b1; ++b) {
+    const float *xn = X + (size_t)next_row * ldx;
+    next_row = row_index(b + 2);
+    int y_row[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int x = min(b * 16 + 4 * h + r, n_rows - 1);
+      if constexpr (OUT == kListed) y_row[r] = rows[x]; else y_row[r] = x;
+      if (OUT == kListed && !y_by_row) y_row[r] = x;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[q][v] = 0.f;
+    for (int g = 0; g < G; ++g) {
+      operands nxt = load(g + 1 < G ? xp : xn, g + 1 < G ? g + 1 : 0);
+      run(g, cur);
+      cur = nxt;
+    }
+    xp = xn;
+    if constexpr (OUT == kAnyOut) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int x = b * 16 + 4 * h + r;
+        if (x >= n_rows) continue;
+        const size_t row = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const int c = panel0 + 16 * V * q + V * j;
+          cvec<V> out;
+#pragma unroll
+          for (int v = 0; v < V; ++v) out.v[v] = acc[q][v][r];
+          gemm_store<V>(Y, row + c, out, N - c, out_how);
+        }
+      }
+    } else {
+      size_t at[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) at[r] = (size_t)y_row[r] * ldy;
+      cvec<V> m[4][Q];
+      if constexpr (OUT == kMasked) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) m[r][q] = *reinterpret_cast<const cvec<V> *>(out_how.mask + at[r] + min(panel0 + 16 * V * q + V * j, N - V));
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          cvec<V> out;
+#pragma unroll
+          for (int v = 0; v < V; ++v) out.v[v] = OUT == kMasked && m[r][q].v[v] <= 0.f ? 0.f : acc[q][v][r];
+          *reinterpret_cast<cvec<V> *>(Y + at[r] + min(panel0 + 16 * V * q + V * j, N - V)) = out;
+        }
     }
   }
 }
@@ -270,11 +296,10 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
                            int n_rows, int K, int N, const GemmOut &how, int compute_units, hipStream_t st) {
   if (n_rows <= 0) return hipSuccess;
-  // Which kernel (us, this one / one 16-row tile per wavefront, at 4,000 / 16,000 / 32,000 / 64,000 rows): copying W to LDS
-  // takes 5 us before the first product, the other kernel reads it from L2 for every row tile: 128 x 128 10.4 / 5.9,
-  // 11.9 / 13.8, 19.4 / 24.1, 29 / 41; 64 x 64 5.3 / 4.1, 5.8 / 6.0, 8.9 / 9.0, 12.9 / 15.4; 500 x 32 13.3 / 6.6,
-  // 15.6 / 12.3, 25.4 / 21.2, 39 / 54; 40 x 7 4.9 / 4.1, 4.9 / 4.3, 6.7 / 4.2, 8.5 / 5.2.  Widths are cut into panels that
-  // fit LDS (X is read once per panel).
+  // Which kernel (us, this one / one 16-row tile per wavefront, at 8,000 / 16,000 / 30,000 rows): copying W to LDS
+  // takes some 4 us before the first product, the other kernel reads it from L2 for every row tile, by single values where W is
+  // K x N.  128 x 128 9.3 / 8.1 (K x N: 9.3 / 11.6), 11.0 / 13.8, 16.8 / 23; 64 x 64 5.0 / 4.6 (5.0 / 5.7), 5.0 / 6.0, 6.7 / 9.0; 500 x 32, 30,000 rows
+  // 17.6 / 20.8; 40 x 7 6.7 / 4.2.  Widths are cut into panels that fit LDS (X is read once per panel).
   const long long lds_k = (long long)(K + 15) / 16 * 16 * 4;  // bytes per column
   int unit = N <= 16 ? 16 : N <= 32 ? 32 : N <= 64 ? 64 : N <= 96 ? 96 : 128;
   if (N > 128) {  // equal panels
@@ -282,19 +307,22 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     unit = w <= 96 ? 96 : 128;
   }
   while (unit > 16 && lds_k * unit > 163840) unit = unit == 96 ? 64 : unit / 2;
-  const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 160LL * compute_units : 48LL * compute_units;
-  if (n_rows >= from && lds_k * unit <= 163840) {
+  const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 80LL * compute_units : (wt ? 48LL : 24LL) * compute_units;
+  if (n_rows >= from && lds_k * unit <= 163840 && K >= 4) {
     const int panels = (N + unit - 1) / unit, lds = (int)(lds_k * unit), n_blocks = (n_rows + 15) / 16;
     const int waves = n_blocks >= 16 * compute_units ? 16 : n_blocks >= 8 * compute_units ? 8 : 4;
     const dim3 grid(std::max(1, std::min(compute_units / std::min(panels, 2), (n_blocks + waves - 1) / waves)), panels);
     hipError_t err = hipSuccess;
-#define CALLP2(V_, Q_, WT_)                                                                                                    \
+    const int out = how.accumulate || how.relu || N < 4 || (rows && how.mask) ? kAnyOut : rows ? kListed : how.mask ? kMasked : kPlain;
+#define CALLP3(V_, Q_, WT_, OUT_)                                                                                              \
   do {                                                                                                                         \
     if (lds > 65536)                                                                                                           \
-      err = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_panel_kernel<V_, Q_, WT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_panel_kernel<V_, Q_, WT_, OUT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
     if (err == hipSuccess)                                                                                                     \
-      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how); \
+      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_, OUT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how); \
   } while (0)
+#define CALLP2(V_, Q_, WT_)                                                                                                    \
+  do { if (out == kPlain) { CALLP3(V_, Q_, WT_, kPlain); } else if (out == kMasked) { CALLP3(V_, Q_, WT_, kMasked); } else if (out == kListed) { CALLP3(V_, Q_, WT_, kListed); } else { CALLP3(V_, Q_, WT_, kAnyOut); } } while (0)
 #define CALLP(V_, Q_) do { if (wt) { CALLP2(V_, Q_, true); } else { CALLP2(V_, Q_, false); } } while (0)
     switch (unit) {
       case 16: CALLP(1, 1); break;
@@ -305,6 +333,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     }
 #undef CALLP
 #undef CALLP2
+#undef CALLP3
     return err != hipSuccess ? err : hipGetLastError();
   }
   // Column blocks per wavefront: as many as the width has (up to four: X is then read once per 64 columns), fewer
