@@ -46,7 +46,9 @@ struct DeviceSchedule {
   int *fused_rec = nullptr;
   LongChunk *long_chunks = nullptr;
   LongRow *long_rows = nullptr;  // the rows that partial sums are added up for: of several chunks, or of segments
-  int n_long_rows = 0;
+  int n_long_rows = 0, n_big_rows = 0;  // of segments: those with groups of them come first
+  int *chunk_long = nullptr;     // per chunk: which of long_rows it belongs to, -1 when it is its row's only one
+  unsigned *arrived = nullptr;   // per row of several chunks: how many of them are done
   LongRow *seg_groups = nullptr;
   float *inter = nullptr;    // M x N intermediate, only if some tile writes back
   float *partial = nullptr;  // n_long_chunks (or segments) x N
@@ -92,7 +94,6 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
                                            const float *, int, float *, int, int, int, int, hipStream_t);
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
 hipError_t launch_spmm_gemm(RowsArgs, const RowsHow &, const float *, int, int, const GemmOut &, hipStream_t);
-hipError_t launch_long_row_reduce(const LongRow *, int, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const GemmOut &, int, hipStream_t);
 WeightGradPlan plan_weight_grad(int, int, int, int);
 hipError_t launch_weight_grad(const WeightGradPlan &, const float *, int, const float *, int, int, float *, float *, hipStream_t);
@@ -101,7 +102,7 @@ hipError_t launch_march_fill(const int *, const int *, const float *, const floa
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
                                         const float *, float *, float *, int, int, int, int, int, int, int, hipStream_t);
 hipError_t launch_scatter_values(const int *, const int *, const float *, float *, int, hipStream_t);
-hipError_t launch_seg_reduce(const LongRow *, int, const int *, const float *, float *, int, int, int, int, hipStream_t);
+hipError_t launch_seg_reduce(const LongRow *, int, int, const LongRow *, int, const int *, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_fused_gemm_spmm(const TileDesc *, int, const int *, const float *, const float *,
                                   int, int, const int *, const int *, const float *, float *,
                                   float *, int, int, int, int, int, hipStream_t);
@@ -239,6 +240,8 @@ static tf_status ensure_device(tf_schedule *s) {
   const std::vector<float> trash(64, 0.f);
   std::vector<LongChunk> chunks;
   std::vector<LongRow> summed;  // the rows that partial sums are added up for
+  std::vector<int> chunk_long;
+  std::vector<unsigned> arrived;
   if (s->two_passes) {  // (the lists are the other schedule's)
     parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
     parts.list(s->l2_tiles, &d->l2_tiles);
@@ -283,8 +286,16 @@ static tf_status ensure_device(tf_schedule *s) {
       // longest first: what starts last should end soon
       std::stable_sort(chunks.begin(), chunks.end(), [](const LongChunk &a, const LongChunk &b) { return a.k_end - a.k_begin > b.k_end - b.k_begin; });
       parts.list(chunks, &d->long_chunks);
+      std::vector<int> of_slot(slots);
+      for (size_t r = 0; r < summed.size(); ++r) std::fill_n(of_slot.begin() + summed[r].first, summed[r].count, (int)r);
+      for (const LongChunk &c : chunks) chunk_long.push_back(c.slot < 0 ? -1 : of_slot[c.slot]);
+      parts.list(chunk_long, &d->chunk_long);
+      arrived.assign(summed.size(), 0);
+      parts.list(arrived, &d->arrived);
     } else {
       summed = s->long_rows;
+      const int n_seg = (int)s->seg_ptr.size() - 1;
+      d->n_big_rows = (int)(std::stable_partition(summed.begin(), summed.end(), [&](const LongRow &lr) { return lr.count > 0 && s->lrow_seg[lr.first] >= n_seg; }) - summed.begin());
     }
     parts.list(summed, &d->long_rows);
     d->n_long_rows = (int)summed.size();
@@ -296,7 +307,7 @@ static tf_status ensure_device(tf_schedule *s) {
       parts.list(s->lrow_seg, &d->lrow_seg);
       parts.list(s->seg_groups, &d->seg_groups);
       parts.reserve(s->seg_src.size(), &d->seg_val);
-      slots = s->seg_ptr.size() - 1 + s->seg_groups.size();
+      slots = s->seg_ptr.size() - 1;
     }
     if (slots > 0) parts.reserve(slots * N, &d->partial);
     if (s->n_writeback_rows > 0) parts.reserve((size_t)s->M * inter_ld(s), &d->inter);
@@ -398,6 +409,7 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
   a.chunks = d->long_chunks;
   a.n_chunks = (unsigned)s->long_chunks.size();
   a.chunk_Ai = A->i; a.chunk_Ax = A->x; a.partial = d->partial;
+  a.chunk_long = d->chunk_long; a.long_rows = d->long_rows; a.arrived = d->arrived;
   if (!s->rem_rows.empty() && !s->rem_ptr.empty()) {
     // The rows in the order of the list, entries side by side -- the reference's reordered adjacency
     // (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653; executor at
@@ -440,14 +452,8 @@ static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder 
     c.streaming = 1;
     TF_PHASE(s, "spmm_rows_kernel (cold long-row segments)", st, launch_spmm_rows(c, RowsHow(), st));
     if (hot_on_side) TF_HIP(hipStreamWaitEvent(st, d->join, 0));
-    // groups of segments of the rows with many (into their own slots of `partial`), then the rows
-    if (!s->seg_groups.empty())
-      TF_PHASE(s, "long_seg_reduce_kernel (groups)", st,
-               launch_seg_reduce(d->seg_groups, (int)s->seg_groups.size(), d->lrow_seg, d->partial, d->partial, N, N, 0, 0, st));
-    TF_PHASE(s, "long_seg_reduce_kernel (rows)", st,
-             launch_seg_reduce(d->long_rows, d->n_long_rows, d->lrow_seg, d->partial, r.D, ldd, N, r.accumulate, r.relu, st));
-  } else if (d->n_long_rows > 0) {
-    TF_PHASE(s, "long_row_reduce_kernel", st, launch_long_row_reduce(d->long_rows, d->n_long_rows, d->partial, r.D, ldd, N, r.accumulate, r.relu, st));
+    TF_PHASE(s, "long_seg_reduce_kernel", st,
+             launch_seg_reduce(d->long_rows, d->n_long_rows, d->n_big_rows, d->seg_groups, n_seg, d->lrow_seg, d->partial, r.D, ldd, N, r.accumulate, r.relu, st));
   }
   return TF_OK;
 }

@@ -783,8 +783,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         const int len = Ap[i + 1] - Ap[i];
         return len <= 8 ? 0 : len <= 32 ? 1 : len <= 128 ? 2 : len <= 512 ? 3 : 4;
       };
-      auto scattered = [&] {  // (65,536 rows are looked at)
-        const size_t n = S->rem_rows.size(), step = n / 65536 + 1;
+      auto scattered = [&] {  // (some 8,192 rows are looked at)
+        const size_t n = S->rem_rows.size(), step = n / 8192 + 1;
         double far = 0;
         long long entries = 0;
         for (size_t q = 0; q < n; q += step) {
@@ -1091,7 +1091,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   if (s->march) ws += (long long)s->march_ell_off.size() * 16;  // ELL rows with values, their offsets and sources
   if (s->n_writeback_rows > 0 || s->two_passes) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
-  if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1 + (long long)s->seg_groups.size()) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
+  if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C
   if (s->user_N != s->opts.N) ws += ((long long)s->L + s->opts.K) * s->opts.N * 4;  // one column panel of D and of C
   ws += (long long)s->rem_ptr.size() * 4 + (long long)s->rem_col.size() * 12;       // remainder rows in list order

@@ -68,6 +68,10 @@ struct RowsArgs {
   const int *chunk_Ai = nullptr;
   const float *chunk_Ax = nullptr;
   float *partial = nullptr;
+  // rows of several chunks: which of long_rows a chunk belongs to (-1: its row has no other), and how many of each have arrived
+  const int *chunk_long = nullptr;
+  const LongRow *long_rows = nullptr;
+  unsigned *arrived = nullptr;
   unsigned chunk_blocks = 0;          // set by the launcher
   int n_blocks = 0, per_xcd = 0, slices = 1;  // set by the launcher
 };

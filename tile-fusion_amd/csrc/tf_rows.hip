@@ -195,7 +195,9 @@ template <int V> __device__ __forceinline__ int clamp_col(int c, int N) { return
 //
 // Chunks: the lane groups take eight entries of the chunk at a time, in turn, partial sums are combined inside a wavefront by shuffles
 // and across the wavefronts through LDS, in a fixed order.  The only chunk of a row (slot < 0) goes straight to Y, a chunk of
-// a row with several to partial[slot], which long_row_reduce_kernel adds up in order.
+// a row with several to partial[slot]; the last of a row's chunks to arrive adds them up in order (a launch of its own for that: 5 us
+// after each of the four products of a training step of 345).  The last one sets
+// the counter back to zero.
 //
 // Column slices (slices > 1): workgroup b works on the columns [4 LPR s, 4 LPR (s + 1)) of its rows with s = b mod 8 mod
 // slices, so that an XCD gathers from one slice of X, `slices` times smaller than X; see slices_for.
@@ -243,10 +245,30 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
             if (a.relu) relu_of<V>(acc);
             store_any<V>(y, acc, a.streaming);
           } else {
-            store_any<V>(a.partial + (size_t)ch.slot * a.N + coff, acc, false);
+            float *p = a.partial + (size_t)ch.slot * a.N + coff;
+#pragma unroll
+            for (int u = 0; u < V; ++u) __hip_atomic_store(p + u, acc.v[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
         }
         __syncthreads();
+      }
+      if (ch.slot >= 0) {
+        __shared__ int last;
+        const LongRow lr = a.long_rows[a.chunk_long[blockIdx.x]];
+        // (the sums are stored past this XCD's L2 and have to be there before the chunk counts as done; a fence would write back all of L2 and
+        // made the launch 40 -> 74 us)
+        if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (threadIdx.x == 0)
+          last = __hip_atomic_fetch_add(a.arrived + a.chunk_long[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)lr.count - 1;
+        __syncthreads();
+        if (!last) return;
+        if (threadIdx.x == 0) __hip_atomic_store(a.arrived + a.chunk_long[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int c = threadIdx.x; c < a.N; c += kBlock) {
+          float *y = a.Y + (size_t)lr.row * a.ldy + c;
+          float s = a.accumulate ? *y : 0.f;
+          for (int p = 0; p < lr.count; ++p) s += __hip_atomic_load(a.partial + (size_t)(lr.first + p) * a.N + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          *y = a.relu && s < 0.f ? 0.f : s;
+        }
       }
       return;
     }
@@ -407,42 +429,60 @@ __global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(cons
   }
 }
 
-// The rows with several chunks: Y[row] (+)= their partial sums, in order.
-__global__ __launch_bounds__(kBlock) void long_row_reduce_kernel(const LongRow *__restrict__ rows, const float *__restrict__ partial,
-                                                                 float *__restrict__ Y, int ldy, int N, int accumulate, int relu) {
-  const LongRow lr = rows[blockIdx.x];
-  for (int c = threadIdx.x; c < N; c += kBlock) {
-    float s = accumulate ? Y[(size_t)lr.row * ldy + c] : 0.f;
-    for (int p = 0; p < lr.count; ++p) s += partial[(size_t)(lr.first + p) * N + c];
-    Y[(size_t)lr.row * ldy + c] = relu && s < 0.f ? 0.f : s;
-  }
-}
-
-// One lane group per long row, every lane four adjacent columns; the partial rows of eight
-// segments are requested before the first is added.  (Y may be `partial` itself: other rows.)
+// Y[row] (+)= the sums in partial[seg_of[first .. first + count)] of the long rows' segments, in order.  The rows from n_big on have a
+// lane group each, every lane four adjacent columns, the partial rows of eight segments requested before the first is added.
+// The first n_big rows have groups of segments (slots from n_seg on name them): a workgroup each, a group of segments per lane
+// group at a time, the groups' sums added in order through LDS.  (The groups in a launch before the rows': 37 us for both on a
+// 2^18-node R-MAT graph, N = 128; 25 us in one.)
+constexpr int kSegBlock = kBlock;
 template <int V, int LPR>
-__global__ __launch_bounds__(kBlock) void long_seg_reduce_kernel(const LongRow *__restrict__ rows, int n_long,
-                                                                 const int *__restrict__ seg_of, const float *partial, float *Y,
-                                                                 int ldy, int N, int accumulate, int relu) {
-  constexpr int G = kBlock / LPR;
+__global__ __launch_bounds__(kSegBlock) void long_seg_reduce_kernel(const LongRow *__restrict__ rows, int n_long, int n_big,
+                                                                    const LongRow *__restrict__ groups, int n_seg,
+                                                                    const int *__restrict__ seg_of, const float *__restrict__ partial,
+                                                                    float *__restrict__ Y, int ldy, int N, int accumulate, int relu) {
+  constexpr int G = kSegBlock / LPR;
+  __shared__ fvec<V> red[G][LPR];
   const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
-  const int q = blockIdx.x * G + group;
-  if (q >= n_long) return;
-  const LongRow lr = rows[q];
-  for (int c0 = 0; c0 < N; c0 += LPR * V) {
-    if (c0 + glane * V >= N) continue;
-    const int coff = clamp_col<V>(c0 + glane * V, N);
-    float *y = Y + (size_t)lr.row * ldy + coff;
-    fvec<V> acc = vzero<V>();
-    if (accumulate) acc = load_any<V>(y);
-    for (int p0 = 0; p0 < lr.count; p0 += 8) {
+  auto add_up = [&](int first, int count, int coff, fvec<V> &acc) __attribute__((always_inline)) {
+    for (int p0 = 0; p0 < count; p0 += 8) {
       fvec<V> x[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (p0 + u < lr.count) x[u] = load_any<V>(partial + (size_t)seg_of[lr.first + p0 + u] * N + coff);
+        if (p0 + u < count) x[u] = load_any<V>(partial + (size_t)seg_of[first + p0 + u] * N + coff);
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (p0 + u < lr.count) vadd<V>(x[u], acc);
+        if (p0 + u < count) vadd<V>(x[u], acc);
+    }
+  };
+  const bool big = (int)blockIdx.x < n_big;
+  const int q = big ? blockIdx.x : n_big + (blockIdx.x - n_big) * G + group;
+  if (q >= n_long) return;
+  const LongRow lr = rows[q];
+  const int g_first = big ? seg_of[lr.first] - n_seg : 0;
+  for (int c0 = 0; c0 < N; c0 += LPR * V) {
+    const bool ok = c0 + glane * V < N;
+    const int coff = clamp_col<V>(c0 + glane * V, N);
+    float *y = Y + (size_t)lr.row * ldy + coff;
+    fvec<V> acc = vzero<V>();
+    if (big) {
+      if (accumulate && group == 0 && ok) acc = load_any<V>(y);
+      for (int g0 = 0; g0 < lr.count; g0 += G) {
+        fvec<V> s = vzero<V>();
+        if (g0 + group < lr.count) {
+          const LongRow g = groups[g_first + g0 + group];
+          add_up(g.first, g.count, coff, s);
+        }
+        red[group][glane] = s;
+        __syncthreads();
+        if (group == 0)
+          for (int t = 0; t < G && g0 + t < lr.count; ++t) vadd<V>(red[t][glane], acc);
+        __syncthreads();
+      }
+      if (group > 0 || !ok) continue;
+    } else {
+      if (!ok) continue;
+      if (accumulate) acc = load_any<V>(y);
+      add_up(lr.first, lr.count, coff, acc);
     }
     if (relu) relu_of<V>(acc);
     store_any<V>(y, acc, false);
@@ -564,23 +604,15 @@ hipError_t launch_spmm_gemm(RowsArgs a, const RowsHow &rows, const float *W, int
   return err != hipSuccess ? err : hipGetLastError();
 }
 
-hipError_t launch_long_row_reduce(const LongRow *rows, int n_rows, const float *partial, float *Y, int ldy, int N, int accumulate,
-                                  int relu, hipStream_t st) {
-  if (n_rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(long_row_reduce_kernel, dim3(n_rows), dim3(kBlock), 0, st, rows, partial, Y, ldy, N, accumulate, relu);
-  return hipGetLastError();
-}
-
-// Y[rows[q].row] (+)= the sums in partial[seg_of[first .. first + count)], in that order (Y may be
-// `partial` itself for the groups of segments of rows with many).
-hipError_t launch_seg_reduce(const LongRow *rows, int n_rows, const int *seg_of, const float *partial, float *Y, int ldy, int N,
-                             int accumulate, int relu, hipStream_t st) {
+// The long rows' sums of their segments' partial sums; the rows with groups of segments come first.
+hipError_t launch_seg_reduce(const LongRow *rows, int n_rows, int n_big, const LongRow *groups, int n_seg, const int *seg_of, const float *partial,
+                             float *Y, int ldy, int N, int accumulate, int relu, hipStream_t st) {
   if (n_rows <= 0) return hipSuccess;
   const RowShape s = row_shape(N, accumulate);
-  const int G = kBlock / s.LPR;
-#define CALL(V_, L_)                                                                                                \
-  hipLaunchKernelGGL((long_seg_reduce_kernel<V_, L_>), dim3((n_rows + G - 1) / G), dim3(kBlock), 0, st, rows, n_rows, \
-                     seg_of, partial, Y, ldy, N, accumulate, relu)
+  const int G = kSegBlock / s.LPR;
+#define CALL(V_, L_)                                                                                                                       \
+  hipLaunchKernelGGL((long_seg_reduce_kernel<V_, L_>), dim3(n_big + (n_rows - n_big + G - 1) / G), dim3(kSegBlock), 0, st, rows, n_rows, n_big, \
+                     groups, n_seg, seg_of, partial, Y, ldy, N, accumulate, relu)
   TF_DISPATCH_ROWS(s, CALL);
 #undef CALL
   return hipGetLastError();
