@@ -1,0 +1,69 @@
+// Rules of dispatch, checked on the host: which lane of which workgroup stores which column.  Compiled with the host
+// sources by tests/test_host_rules.py; each argument names a check; exits 0 when all of them hold.
+#include <cstdarg>
+#include <cstdio>
+#include <cstring>
+#include <vector>
+#include "tf_internal.h"
+#include "tf_rows.h"
+namespace tf {
+static char g_err[512];
+tf_status fail(tf_status code, const char *fmt, ...) { va_list ap; va_start(ap, fmt); vsnprintf(g_err, sizeof g_err, fmt, ap); va_end(ap); return code; }
+int default_compute_units() { return 256; }
+void release_device_schedule(DeviceSchedule *) {}
+}  // namespace tf
+
+// Every column of a row is stored, and one that is added to is stored in one pass of one workgroup only: in a pass all lanes of a
+// row load Y before one of them stores.  As in spmm_rows_kernel, over all widths and the strides and sizes that slices look at.
+static int column_owners() {
+  int bad = 0, sliced = 0;
+  for (int accumulate = 0; accumulate < 2; ++accumulate)
+    for (int N = 1; N <= 600; ++N)
+      for (int pad = 0; pad < 2; ++pad)
+        for (int compact = 0; compact < 2; ++compact)
+          for (unsigned rows : {100u, 16000u, 30000u, 70000u, 131072u, 200000u}) {
+            tf::RowsArgs a;
+            a.X = reinterpret_cast<const float *>(1 << 20);
+            a.ldx = pad ? (N + 31) / 32 * 32 : N;
+            a.x_rows = rows;
+            a.N = N;
+            a.compact = compact;
+            a.accumulate = accumulate;
+            tf::RowShape s = tf::row_shape(N, accumulate);
+            a.slices = s.V == 4 ? tf::slices_for(a) : 1;
+            if (a.slices > 1) { s.LPR = tf::kSliceCols / 4; ++sliced; }
+            std::vector<int> passes(N, 0), last(N, -1);
+            int pass = 0;
+            for (int slice = 0; slice < a.slices; ++slice) {
+              const int c_begin = a.slices > 1 ? slice * s.LPR * s.V : 0;
+              const int c_end = a.slices > 1 ? (N < c_begin + s.LPR * s.V ? N : c_begin + s.LPR * s.V) : N;
+              for (int c0 = c_begin; c0 < c_end; c0 += s.LPR * s.V, ++pass)
+                for (int lane = 0; lane < s.LPR; ++lane) {
+                  const int col = c0 + lane * s.V;
+                  if (col >= N) continue;
+                  const int at = s.V == 1 ? tf::clamp_col<1>(col, N) : tf::clamp_col<4>(col, N);
+                  for (int u = 0; u < s.V; ++u) {
+                    if (at + u < 0 || at + u >= N) { printf("N %d: column %d stored\n", N, at + u); ++bad; continue; }
+                    if (last[at + u] != pass) { last[at + u] = pass; ++passes[at + u]; }
+                  }
+                }
+            }
+            for (int c = 0; c < N; ++c)
+              if (passes[c] < 1 || (accumulate && passes[c] > 1)) {
+                printf("N %d rows %u slices %d accumulate %d: column %d in %d passes\n", N, rows, a.slices, accumulate, c, passes[c]);
+                ++bad;
+              }
+          }
+  if (!sliced) { printf("no slices anywhere\n"); ++bad; }
+  return bad;
+}
+
+int main(int argc, char **argv) {
+  int bad = 0;
+  for (int k = 1; k < argc; ++k) {
+    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : 1;
+    printf("%s: bad %d\n", argv[k], b);
+    bad += b;
+  }
+  return bad != 0;
+}

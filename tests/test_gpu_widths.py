@@ -69,3 +69,34 @@ def test_column_slices(gpu, tf, orc, N):
     tf.spmm_spmm(Ah, Ah, tf.DenseMatrix.from_numpy(C), D, S)
     tf.device_synchronize()
     assert np.array_equal(D.to_numpy(), oracle_spmm_spmm(orc, A, A, C))
+
+
+@pytest.mark.parametrize("N", [97, 98, 99, 100, 128, 49, 64])
+@pytest.mark.parametrize("op", ["spmm", "gemm"])
+def test_column_slices_accumulate(gpu, tf, N, op):
+    """D += A (B C) at those sizes: every column of D is added to once, whichever workgroups store it.  Whole numbers, so that the
+    sums are exact in fp32 in any order: entries and operands of 1 to 4, below 2^24 altogether."""
+    say(f"column slices accumulate N={N} {op}")
+    n, K = 30011, 2 * N
+    rng = np.random.default_rng(N)
+    A = tf.workloads.erdos_renyi_gcn(n, 3.0, seed=N)
+    A.data = rng.integers(1, 3, A.nnz).astype(np.float32)
+    D0 = rng.integers(-4, 5, (n, N)).astype(np.float32)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    D = tf.DenseMatrix.from_numpy(D0)
+    A64 = A.astype(np.float64)
+    if op == "spmm":
+        C = rng.integers(-4, 5, (n, N)).astype(np.float32)
+        S = tf.inspector(Ah, op=tf.OP_SPMM_SPMM, N=N, inner=Ah)
+        step = A64 @ (A64 @ C.astype(np.float64))
+        operands = (Ah, tf.DenseMatrix.from_numpy(C))
+    else:
+        B, C = (rng.integers(-2, 3, s).astype(np.float32) for s in ((n, K), (K, N)))
+        S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+        step = A64 @ (B.astype(np.float64) @ C.astype(np.float64))
+        operands = (tf.DenseMatrix.from_numpy(B), tf.DenseMatrix.from_numpy(C))
+    assert np.abs(D0).max() + 2 * np.abs(step).max() < 2 ** 24
+    for k in (1, 2):
+        (tf.spmm_spmm if op == "spmm" else tf.gemm_spmm)(Ah, *operands, D, S, accumulate=True)
+        tf.device_synchronize()
+        assert np.array_equal(D.to_numpy(), D0 + k * step), k

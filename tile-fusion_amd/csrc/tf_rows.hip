@@ -11,6 +11,7 @@
 
 #include "tf_internal.h"
 #include "tf_device.h"
+#include "tf_rows.h"
 
 namespace tf {
 
@@ -182,10 +183,6 @@ __device__ __forceinline__ void clear_rows(const RowsArgs &a, int q, int glane, 
     }
   }
 }
-
-// What one lane stores of a row of N columns: its V columns, or the last V when they reach past the end (two
-// lanes of a group then store some of the same values).
-template <int V> __device__ __forceinline__ int clamp_col(int c, int N) { return V == 1 ? min(c, N - 1) : min(c, N - V); }
 
 }  // namespace
 
@@ -493,31 +490,6 @@ __global__ __launch_bounds__(kSegBlock) void long_seg_reduce_kernel(const LongRo
 
 namespace {
 
-// Lanes a row of N columns takes: V = 4 columns each (any N of four or more: a lane whose columns would reach past the
-// row's end takes the last four), one each for narrower rows.  With accumulation into a row longer than the 256 columns of
-// one pass, a last lane of a later pass must not fall back into columns the pass before has added to.
-struct RowShape { int V, LPR; };
-RowShape row_shape(int N, int accumulate) {
-  const int V = N < 4 || (accumulate && N > 256 && N % 4 != 0) ? 1 : 4;
-  int LPR = V == 1 ? (N < 4 ? 4 : 64) : 2;
-  if (V == 4)
-    while (LPR * 4 < N && LPR < 64) LPR *= 2;
-  return {V, LPR};
-}
-
-// Slices of 32 columns, a cache line each, where a slice is a few times an XCD's L2 and X is not: gathers that came out of
-// the Infinity Cache then hit.  One product of an Erdos-Renyi graph (10 - 12 entries a row), whole rows / slices: N = 128,
-// 10,000 rows 6.4 / 6.4 us, 20,000 14.5 / 10.1, 50,000 46 / 34, 100,000 83 / 75, 200,000 170 / 171; N = 64, 50,000 rows 21 / 19,
-// 100,000 41 / 39, and not on stencils (16 / 16.5).  Rows that do not start at a line would share lines between slices
-// (N = 100, 50,000 rows: 41 / 65).
-int slices_for(const RowsArgs &a) {
-  if (a.ldx % 32 != 0 || (reinterpret_cast<uintptr_t>(a.X) & 127u)) return 1;
-  const long long bytes = (long long)a.x_rows * a.ldx * 4;
-  if (a.N > 96 && a.N <= 128 && a.x_rows >= 16000 && bytes <= (64LL << 20)) return 4;
-  if (a.N > 48 && a.N <= 64 && a.compact && a.x_rows >= 24000 && bytes <= (40LL << 20)) return 2;
-  return 1;
-}
-
 inline bool xcd_remap_on() {
   static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
   return on;
@@ -548,7 +520,7 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   RowShape s = row_shape(a.N, a.accumulate);
   a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
   a.slices = s.V == 4 && !how.flagged && a.n_chunks == 0 && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
-  if (a.slices > 1) s.LPR = 8;
+  if (a.slices > 1) s.LPR = kSliceCols / 4;
   const int G = kBlock / s.LPR;
   a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
   const int blocks = deal_to_xcds(a, how.xcd_chunk_rows, G);
