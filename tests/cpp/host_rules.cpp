@@ -1,4 +1,4 @@
-// Rules of dispatch, checked on the host: which lane of which workgroup stores which column.  Compiled with the host
+// Rules of dispatch, checked on the host: which lane of which workgroup stores which column, what fits LDS.  Compiled with the host
 // sources by tests/test_host_rules.py; each argument names a check; exits 0 when all of them hold.
 #include <cstdarg>
 #include <cstdio>
@@ -58,10 +58,41 @@ static int column_owners() {
   return bad;
 }
 
+// Layers that run in one launch: the rows of A B that a workgroup holds fit its LDS, at every K; wider ones are inspected into something
+// else and accepted all the same.
+static int one_launch_fits() {
+  int bad = 0, taken = 0, beyond = 0;
+  for (int M : {1, 17, 500, 786, 4096, 9999, 23999, 24000, 30000}) {
+    std::vector<int> p(M + 1), i;
+    for (int r = 0; r < M; ++r) {
+      for (int c = r > 0 ? r - 1 : 0; c <= r + 1 && c < M; ++c) i.push_back(c);
+      p[r + 1] = (int)i.size();
+    }
+    for (int K : {4, 30, 64, 128, 250, 1000, 2543, 2544, 2545, 2560, 3000, 5000})
+      for (int N : {2, 64, 128, 700, 1273, 2000, 2600}) {
+        if ((long long)M * K > 4000000) continue;
+        tf_inspect_opts o{};
+        o.struct_size = sizeof(o);
+        o.op = TF_OP_GEMM_SPMM;
+        o.K = K;
+        o.N = N;
+        tf_schedule *s = nullptr;
+        if (tf_inspect(M, M, p.data(), i.data(), &o, &s)) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; continue; }
+        const int lds = s->one_launch ? (s->two_passes->rem_rows.size() < 24000 ? 16 : 64) * ((K + 15) / 16 * 16 + 4) * 4 : 0;
+        if (lds > 163840) { printf("M %d K %d N %d: one launch with %d bytes of LDS\n", M, K, N, lds); ++bad; }
+        taken += s->one_launch;
+        beyond += K > 2544 && K <= 2 * N && (long long)M * K <= 2000000;
+        tf_schedule_free(s);
+      }
+  }
+  if (!taken || !beyond) { printf("one launch %d times, %d sizes beyond it\n", taken, beyond); ++bad; }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
-    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : 1;
+    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

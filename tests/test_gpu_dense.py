@@ -226,3 +226,24 @@ def test_layer_in_one_launch(gpu, tf, M, K, N, listed):
             assert "spmm_gemm_kernel" in [n for n, _ in S.profile()]
         ref = want + D0 if flags & 1 else want
         assert rel(D.to_numpy(), np.maximum(ref, 0) if flags & RELU else ref) <= 1e-5, flags
+
+
+@pytest.mark.parametrize("M,K,N", [(500, 2544, 1273), (500, 2545, 1273), (500, 3000, 2000), (60, 6001, 3001)])
+def test_layer_of_few_rows_and_wide_features(gpu, tf, M, K, N):
+    """Up to the K whose rows fill LDS in one launch, and beyond it."""
+    say(f"few rows M={M} {K}x{N}")
+    rng = np.random.default_rng(K)
+    A = sp.csr_matrix(sp.diags([1.0, -2.0, 3.0], [-1, 0, 2], shape=(M, M)), dtype=np.float32)
+    X, W, D0 = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    S.set_profiling(True)
+    want = A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))
+    for flags in (0, 1 | RELU | C_TRANSPOSED):
+        Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if flags & C_TRANSPOSED else W)
+        D = tf.DenseMatrix.from_numpy(D0)
+        assert tf.lib().tf_gemm_spmm(Ah.to_device().h, tf.DenseMatrix.from_numpy(X).h, Wd.h, D.h, S.h, flags, None) == 0
+        tf.device_synchronize()
+        ref = np.maximum(want + D0, 0) if flags else want
+        assert rel(D.to_numpy(), ref) <= 1e-5, flags
+        assert ("spmm_gemm_kernel" in [n for n, _ in S.profile()]) == (K <= 2544)

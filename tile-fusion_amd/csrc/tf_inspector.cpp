@@ -18,10 +18,11 @@
 #include <cstring>
 
 #include "tf_internal.h"
+#include "tf_rows.h"
+
+using tf::kMaxLds;
 
 namespace {
-
-constexpr int kMaxLds = 163840;  // LDS per workgroup on gfx950
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
@@ -135,8 +136,9 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     const bool tiled = !S->launch_tiles.empty();
     const bool padded = K != S->opts.K || N != S->opts.N, partly = (long long)S->fused_ids.size() * 8 < 7LL * S->L;
     const bool streamed = tiled && S->gemm_stream && !padded && !partly;
-    S->one_launch = K >= 4 && (M < 24000 ? (K <= 128 && (K <= 2 * N || M < 10000)) || (K <= 2 * N && work <= 2000000)
-                                         : K <= 64 && K <= N && (N <= 64 || M <= 150000) && !(streamed && K > 32));
+    S->one_launch = tf::spmm_gemm_fits(S->L, K, N) &&
+                    (M < 24000 ? (K <= 128 && (K <= 2 * N || M < 10000)) || (K <= 2 * N && work <= 2000000)
+                               : K <= 64 && K <= N && (N <= 64 || M <= 150000) && !(streamed && K > 32));
     S->spmm_first = S->one_launch || 3LL * K <= 2LL * N;
     want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || !S->gemm_stream));
     if (S->spmm_first) N = K;

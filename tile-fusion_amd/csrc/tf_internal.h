@@ -13,6 +13,8 @@
 
 namespace tf {
 
+constexpr int kMaxLds = 163840;  // LDS per workgroup on gfx950
+
 // One fused tile = one workgroup.  The workgroup computes intermediate rows
 // [prod_begin, prod_end) into LDS, stores rows [wb_begin, wb_end) of them to the
 // intermediate in HBM (the ones remainder rows will read), then computes the

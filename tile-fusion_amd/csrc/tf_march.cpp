@@ -27,8 +27,6 @@ namespace tf {
 
 namespace {
 
-constexpr int kMaxLds = 163840;
-
 // The grid a pattern was generated on, from the distances between a row and its columns: a
 // 7-point-like stencil on nx x ny x nz points, x fastest, has the distances 1, nx and nx*ny; a
 // 5-point-like stencil on nx x n points the distances 1 and nx (a grid of nx x 1 x n: the runs then

@@ -1,6 +1,8 @@
 // How the row kernels (tf_rows.hip) deal a row's columns to lanes and XCDs.  Host rules without a HIP header, so that a
 // test can enumerate which lane stores which column.
 #pragma once
+#include <climits>
+
 #include "tf_internal.h"
 
 namespace tf {
@@ -37,6 +39,15 @@ inline int slices_for(const RowsArgs &a) {
   else if (a.N > 48 && a.N <= 64 && a.compact && a.x_rows >= 24000 && bytes <= (40LL << 20)) slices = 2;
   if (a.accumulate && a.N - 4 < (slices - 1) * kSliceCols) slices = 1;
   return slices;
+}
+
+// spmm_gemm_kernel: rows of A X a workgroup holds in LDS, and the LDS they take (K columns in steps of 16, four floats behind
+// each row).
+constexpr int spmm_gemm_rows(int n_rows) { return n_rows < 24000 ? 16 : 64; }
+constexpr long long spmm_gemm_lds(int n_rows, int K) { return spmm_gemm_rows(n_rows) * (((long long)K + 15) / 16 * 16 + 4) * 4; }
+// Sixteen rows of up to 2,544 columns fit the LDS of a compute unit; W's entries are counted in 32 bits.
+constexpr bool spmm_gemm_fits(int n_rows, int K, int N) {
+  return K >= 4 && spmm_gemm_lds(n_rows, K) <= kMaxLds && (long long)K * N <= UINT_MAX;
 }
 
 }  // namespace tf

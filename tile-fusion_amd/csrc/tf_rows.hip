@@ -547,12 +547,13 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Y = (A X) W for the rows of `a` (a.N = K the columns of X, a.ldy that of Y): K from 4 up, X of up to 2 GB, no long rows.
+// Y = (A X) W for the rows of `a` (a.N = K the columns of X, a.ldy that of Y): K and N as spmm_gemm_fits says, X of up to 2 GB, no
+// long rows.
 hipError_t launch_spmm_gemm(RowsArgs a, const RowsHow &rows, const float *W, int wt, int N, const GemmOut &how, hipStream_t st) {
   if (a.n_rows <= 0) return hipSuccess;
-  if (a.N < 4 || a.n_chunks > 0 || (unsigned long long)a.x_rows * a.ldx * 4 > 0x80000000ull) return hipErrorInvalidValue;
+  if (!spmm_gemm_fits(a.n_rows, a.N, N) || a.n_chunks > 0 || (unsigned long long)a.x_rows * a.ldx * 4 > 0x80000000ull) return hipErrorInvalidValue;
   const RowShape s = row_shape(a.N, 0);
-  const int R = a.n_rows < 24000 ? 16 : 64, lds = R * ((a.N + 15) / 16 * 16 + 4) * 4;
+  const int R = spmm_gemm_rows(a.n_rows), lds = (int)spmm_gemm_lds(a.n_rows, a.N);
   a.n_blocks = (a.n_rows + R - 1) / R;
   const dim3 grid(deal_to_xcds(a, rows.xcd_chunk_rows, R));
   hipError_t err = hipSuccess;
