@@ -89,10 +89,43 @@ static int one_launch_fits() {
   return bad;
 }
 
+// The row products of a schedule have room for partial sums of the width they run at, also on a band with hub rows, where the order of
+// the products is chosen again.
+static int partial_sums() {
+  int bad = 0, again = 0;
+  for (int M : {3000, 9000, 30000}) {
+    std::vector<int> p(1, 0), i;
+    for (int r = 0; r < M; ++r) {
+      if (r % 1000 == 500) for (int c = r % 2; c < M; c += 2) i.push_back(c);
+      else for (int c = r > 8 ? r - 8 : 0; c <= r + 8 && c < M; ++c) i.push_back(c);
+      p.push_back((int)i.size());
+    }
+    for (int K : {8, 30, 32, 64, 100, 128})
+      for (int N : {7, 32, 40, 64, 80, 96, 128, 140}) {
+        tf_inspect_opts o{};
+        o.struct_size = sizeof(o);
+        o.op = TF_OP_GEMM_SPMM;
+        o.K = K;
+        o.N = N;
+        tf_schedule *s = nullptr;
+        if (tf_inspect(M, M, p.data(), i.data(), &o, &s)) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; continue; }
+        if (const tf_schedule *rows = s->two_passes) {
+          const int width = s->spmm_first ? K : N;
+          if (rows->opts.N < width) { printf("M %d K %d N %d: partial sums of %d columns for a product of %d\n", M, K, N, rows->opts.N, width); ++bad; }
+          again += !s->spmm_first && K >= 4 && M < 10000 && N > K;
+        }
+        tf_schedule_free(s);
+      }
+  }
+  if (!again) { printf("the order is never chosen again\n"); ++bad; }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
-    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits() : 1;
+    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
+                  : !strcmp(argv[k], "partial_sums") ? partial_sums() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

@@ -247,3 +247,24 @@ def test_layer_of_few_rows_and_wide_features(gpu, tf, M, K, N):
         ref = np.maximum(want + D0, 0) if flags else want
         assert rel(D.to_numpy(), ref) <= 1e-5, flags
         assert ("spmm_gemm_kernel" in [n for n, _ in S.profile()]) == (K <= 2544)
+
+
+@pytest.mark.parametrize("K,N", [(64, 80), (30, 40), (128, 140), (128, 96)])
+def test_layer_on_a_band_with_hub_rows(gpu, tf, K, N):
+    """Rows of 1,500 entries (two chunks, whose sums are added up) among rows of 17, more columns behind the products than before them
+    and fewer."""
+    say(f"band with hubs {K}x{N}")
+    M = 3000
+    rng = np.random.default_rng(K + N)
+    A = sp.diags([1.0] * 17, list(range(-8, 9)), shape=(M, M), format="lil", dtype=np.float32)
+    for r in (500, 1500, 2500):
+        A[r, ::2] = 1.0
+    A = sp.csr_matrix(A, dtype=np.float32)
+    A.data = rng.uniform(-1, 1, A.nnz).astype(np.float32)
+    X, W = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    D = tf.DenseMatrix.from_numpy(np.full((M, N), np.nan, np.float32))
+    tf.gemm_spmm(Ah, tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(W), D, S)
+    tf.device_synchronize()
+    assert rel(D.to_numpy(), A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))) <= 1e-5

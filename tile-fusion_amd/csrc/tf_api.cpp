@@ -433,6 +433,8 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
 static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder &r, bool hot_on_side, hipStream_t st) {
   DeviceSchedule *d = s->dev;
   const int N = r.N, ldd = r.ldd > 0 ? r.ldd : r.N;
+  if (d->partial && N > std::max(s->opts.N, s->user_N))
+    return fail(TF_ESCHEDULE, "the schedule's partial sums have %d columns, the product has %d", std::max(s->opts.N, s->user_N), N);
   RowsArgs a;
   RowsHow how;
   if (tf_status rc = remainder_rows(A, s, r, st, a, how)) return rc;

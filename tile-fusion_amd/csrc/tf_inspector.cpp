@@ -162,10 +162,10 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     S->one_launch = false;
     if (3LL * S->user_K > 2LL * S->user_N) {
       S->spmm_first = false;
-      if (S->launch_tiles.empty()) {
-        tf_schedule_free(S->two_passes);
-        S->two_passes = nullptr;
-      }
+      tf_schedule_free(S->two_passes);
+      S->two_passes = nullptr;
+      o.N = S->user_N;  // (the lists and the room for partial sums are for the width that is gathered)
+      if (!S->launch_tiles.empty()) return inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes);
     }
   }
   return TF_OK;
