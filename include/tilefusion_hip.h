@@ -100,7 +100,8 @@ typedef struct tf_dense tf_dense;
 /* Copies a host CSR to the device.  Column indices need not be sorted. */
 tf_status tf_csr_upload(int M, int N, const int *Ap, const int *Ai, const float *Ax,
                         tf_csr **out);
-/* Wraps CSR arrays that already live in device memory; nothing is copied or owned. */
+/* Wraps CSR arrays that already live in device memory; nothing is copied or owned.  The values may change between calls: every
+ * call reads them where they are. */
 tf_status tf_csr_wrap_device(int M, int N, int nnz, const int *dAp, const int *dAi,
                              const float *dAx, tf_csr **out);
 /* 64-bit fingerprint of a sparsity pattern (row pointers and column indices, host arrays); never 0.
@@ -257,7 +258,7 @@ typedef struct {
   int march_tile_x, march_tile_y;
   /* Remainder rows (second-op rows served from the intermediate in HBM) are worked on in the order of
      a list (by length class).  0 / 1 = when that order is not simply all rows in order, the schedule
-     also keeps those rows' columns -- and the executor their values -- side by side in list order,
+     also keeps those rows' columns -- and, for a matrix whose arrays never change, their values -- side by side in list order,
      which is what the reference's reordered adjacency is to its executors (createReorderedAdj,
      fusion/gcn/SingleLayer/GCN_Single_Layer_SP_Demo_Utils.h:618-653, read by
      forwardForOneLayerFusedParallelSeparatedReorderedAdjVectorizedSP, GCN_Layer_MKL_Forward_Utils.h:294-373);

@@ -203,3 +203,26 @@ def test_two_layer_forward_op(gpu, tf):
     x, a1, a2 = x0.cuda().requires_grad_(), w1.cuda().requires_grad_(), w2.cuda().requires_grad_()
     torch.ops.sw_gcn.fusedGCN(adj, x, a1, a2, 8).backward(go.cuda())
     assert rel_err(x.grad, xd.grad.numpy()) <= TOL and rel_err(a1.grad, w1d.grad.numpy()) <= TOL and rel_err(a2.grad, w2d.grad.numpy()) <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pattern", ["rmat", "er", "grid"])
+def test_values_are_read_on_every_call(gpu, tf, pattern):
+    """A write that no version counter shows is honoured by the next forward pass: rows in lists, hub rows, rows in order."""
+    print(f"sw_gcn live values {pattern}", flush=True)
+    A = {"rmat": lambda: tf.workloads.rmat(13, 8 << 13, seed=3), "er": lambda: tf.workloads.erdos_renyi_gcn(30000, 8.0, seed=4),
+         "grid": lambda: tf.workloads.laplacian_2d(60)}[pattern]()
+    n = A.shape[0]
+    adj = csr_tensor(A, "cuda")
+    g = torch.Generator().manual_seed(1)
+    x, w1, w2 = torch.rand(n, 64, generator=g), torch.rand(64, 64, generator=g) - 0.5, torch.rand(40, 64, generator=g) - 0.5
+    xg, w1g, w2g = x.cuda(), w1.cuda(), w2.cuda()
+    for step in range(3):
+        B = A.astype(np.float64)
+        B.data = A.data * np.float64(1 + step)
+        adj.values().data.copy_(torch.tensor(B.data, dtype=torch.float32))
+        one = B @ (x.double().numpy() @ w1.double().numpy().T)
+        two = B @ (np.maximum(one, 0.0) @ w2.double().numpy().T)
+        assert rel_err(torch.ops.sw_gcn.fusedGeMMSpMM(adj, xg, w1g, [], 8), one) <= TOL, step
+        assert rel_err(torch.ops.sw_gcn.unfused_gcn_forward(adj, xg, w1g, 8), one) <= TOL, step
+        assert rel_err(torch.ops.sw_gcn.fusedGCN(adj, xg, w1g, w2g, 8), two) <= TOL, step

@@ -55,6 +55,7 @@ struct RowsArgs {
   int n_rows = 0;
   const int *Ap = nullptr, *Ai = nullptr;
   const float *Ax = nullptr, *X = nullptr;
+  const int *val_first = nullptr;  // with `compact`: where row q's values start in Ax (null: at Ap[q], as its columns in Ai)
   int ldx = 0;
   unsigned x_rows = 0;  // rows of X
   float *Y = nullptr;

@@ -27,7 +27,8 @@ inline RowShape row_shape(int N, int accumulate) {
 // the Infinity Cache then hit.  One product of an Erdos-Renyi graph (10 - 12 entries a row), whole rows / slices: N = 128,
 // 10,000 rows 6.4 / 6.4 us, 20,000 14.5 / 10.1, 50,000 46 / 34, 100,000 83 / 75, 200,000 170 / 171; N = 64, 50,000 rows 21 / 19,
 // 100,000 41 / 39, and not on stencils (16 / 16.5).  Rows that do not start at a line would share lines between slices
-// (N = 100, 50,000 rows: 41 / 65).
+// (N = 100, 50,000 rows: 41 / 65); values read in place cost a line a row and slice, more than two slices gain (N = 64, 100,000 rows:
+// 41.8 / 42.7).
 // The last slice's last lane may not reach back into the slice before it where Y is added to: workgroups of two XCDs would both
 // add to those columns, and one that loads after the other has stored adds twice.  (N = 97 .. 99: whole rows.)
 constexpr int kSliceCols = 32;
@@ -36,7 +37,7 @@ inline int slices_for(const RowsArgs &a) {
   const long long bytes = (long long)a.x_rows * a.ldx * 4;
   int slices = 1;
   if (a.N > 96 && a.N <= 128 && a.x_rows >= 16000 && bytes <= (64LL << 20)) slices = 4;
-  else if (a.N > 48 && a.N <= 64 && a.compact && a.x_rows >= 24000 && bytes <= (40LL << 20)) slices = 2;
+  else if (a.N > 48 && a.N <= 64 && a.compact && !a.val_first && a.x_rows >= 24000 && bytes <= (40LL << 20)) slices = 2;
   if (a.accumulate && a.N - 4 < (slices - 1) * kSliceCols) slices = 1;
   return slices;
 }

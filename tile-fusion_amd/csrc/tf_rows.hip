@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
   // The workgroups live for a microsecond or two: the arguments are all requested at once here, not one after the other
   // where they are first used, and a listed row's place in Y is not waited for before its entries are.
   asm volatile("" ::"s"(a.rows), "s"(a.Ap), "s"(a.Ai), "s"(a.Ax), "s"(a.X), "s"(a.Y), "s"(a.ldx), "s"(a.ldy), "s"(a.N), "s"(a.n_rows),
-               "s"(a.accumulate), "s"(a.streaming), "s"(a.compact), "s"(a.relu), "s"(a.n_blocks), "s"(a.per_xcd), "s"(a.slices), "s"(a.n_zero));
+               "s"(a.accumulate), "s"(a.streaming), "s"(a.compact), "s"(a.relu), "s"(a.n_blocks), "s"(a.per_xcd), "s"(a.slices), "s"(a.n_zero), "s"(a.val_first));
   int b = CHUNKS ? blockIdx.x - a.chunk_blocks : blockIdx.x, c_begin = 0, c_end = a.N;
   if (a.slices > 1) {
     const int xcd = b % kXcds;
@@ -294,6 +294,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
     if (!a.compact) r = i;
   }
   const int kb = a.Ap[r], ke = a.Ap[r + 1];
+  const float *ax = a.Ax;
+  if (a.val_first) ax += a.val_first[q] - kb;
   for (int c0 = c_begin; c0 < c_end; c0 += LPR * V) {
     const int col = c0 + glane * V;
     const bool ok = col < a.N;
@@ -302,8 +304,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
     float *y = a.Y + (size_t)i * a.ldy + coff;
     fvec<V> acc = vzero<V>();
     if (a.accumulate && ok) acc = load_any<V>(y);
-    if constexpr (WALK == kDpp) row_dot_dpp<LPR>(a.Ai, a.Ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
-    else row_dot_direct<V, LPR, RowsOf<V>, WALK == kMarked>(a.Ai, a.Ax, kb, ke, ok, src, acc);
+    if constexpr (WALK == kDpp) row_dot_dpp<LPR>(a.Ai, ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
+    else row_dot_direct<V, LPR, RowsOf<V>, WALK == kMarked>(a.Ai, ax, kb, ke, ok, src, acc);
     if (ok) {
       if (a.relu) relu_of<V>(acc);
       store_any<V>(y, acc, a.streaming);
@@ -364,15 +366,17 @@ __global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(cons
   for (int r = group; r < R; r += G) {
     const int q = q0 + r;
     int kb = 0, ke = 0;
+    const float *ax = a.Ax;
     if (q < a.n_rows) {
       const int row = a.rows && !a.compact ? a.rows[q] : q;
       kb = a.Ap[row];
       ke = a.Ap[row + 1];
+      if (a.val_first) ax += a.val_first[q] - kb;
     }
     for (int c0 = 0; c0 < K; c0 += LPR * 4) {
       const int col = c0 + glane * 4, coff = clamp_col<4>(col, K);
       fvec<4> acc = vzero<4>();
-      row_dot_dpp<LPR>(a.Ai, a.Ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
+      row_dot_dpp<LPR>(a.Ai, ax, kb, ke, glane, xr, a.ldx * 4u, coff * 4u, acc);
       if (col < K) {
         float *s = slab + r * ld + coff;
         if (K % 4 == 0) *reinterpret_cast<fvec<4> *>(s) = acc;

@@ -113,8 +113,8 @@ AdjacencyPtr make_adjacency(const Tensor &adj, const Tensor &crow, const Tensor 
     check(tf_csr_wrap_device(a->rows, a->cols, a->Ap[a->rows], crow.data_ptr<int>(), col.data_ptr<int>(), val.data_ptr<float>(), &a->csr));
     // the device arrays and the host pattern are copies of the same tensors: the executors may check schedules against it
     check(tf_csr_set_pattern_hash(a->csr, a->hash));
-    // (a change of the tensors changes their version counters, and with them the cache's key)
-    check(tf_csr_set_constant(a->csr));
+    // (the values are read on every call: writes that no version counter shows -- through .data, from another library's kernel,
+    // in the replay of a graph -- are honoured)
   }
   return a;
 }

@@ -32,6 +32,10 @@ Differences from the reference, all forced by where the data lives:
     [out, in] (gcn-e2e-training/FusedGCNModule.py:14-18; binding-project/src/Functions.cpp:228-290).
   * What is built once per adjacency (host pattern, schedules, transpose) is cached for the last 32 of them, keyed by
     the tensors' addresses and version counters: an in-place change of the values or indices makes a new entry.
+    The values themselves are read on every call, so that the forward pass honours writes that no version counter shows (through
+    ``.data``, by another library, in the replay of a graph).  The transpose for the backward pass, and whether the matrix is its
+    own transpose, are taken from the values once per entry: after such a write call ``clear_cache()`` before the next backward
+    pass of a matrix whose transpose changes with it.
 """
 import ctypes
 import os
