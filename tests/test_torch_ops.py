@@ -226,3 +226,77 @@ def test_values_are_read_on_every_call(gpu, tf, pattern):
         assert rel_err(torch.ops.sw_gcn.fusedGeMMSpMM(adj, xg, w1g, [], 8), one) <= TOL, step
         assert rel_err(torch.ops.sw_gcn.unfused_gcn_forward(adj, xg, w1g, 8), one) <= TOL, step
         assert rel_err(torch.ops.sw_gcn.fusedGCN(adj, xg, w1g, w2g, 8), two) <= TOL, step
+
+
+def _two_layers(n, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.rand(n, 48, generator=g), torch.rand(64, 48, generator=g) - 0.5, torch.rand(40, 64, generator=g) - 0.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pattern", ["rmat", "er"])
+def test_calls_on_several_streams_take_turns(gpu, tf, pattern):
+    """Calls that share an adjacency, and with it the schedules' partial sums and intermediates, run one after the other whatever
+    streams they are on: each finishes after the one before it, which waits behind a delay on its own stream."""
+    print(f"sw_gcn streams {pattern}", flush=True)
+    A = tf.workloads.rmat(13, 8 << 13, seed=5) if pattern == "rmat" else tf.workloads.erdos_renyi_gcn(9000, 8.0, seed=6)
+    n = A.shape[0]
+    x, w1, w2 = _two_layers(n, 3)
+    B = A.astype(np.float64)
+    one = B @ (x.double().numpy() @ w1.double().numpy().T)
+    two = B @ (np.maximum(one, 0.0) @ w2.double().numpy().T)
+    adj, xg, w1g, w2g = csr_tensor(A, "cuda"), x.cuda(), w1.cuda(), w2.cuda()
+    calls = [(lambda: torch.ops.sw_gcn.fusedGeMMSpMM(adj, xg, w1g, [], 8), one),
+             (lambda: torch.ops.sw_gcn.unfused_gcn_forward(adj, xg, w1g, 8), one),
+             (lambda: torch.ops.sw_gcn.fusedGCN(adj, xg, w1g, w2g, 8), two)]
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.default_stream(), torch.cuda.Stream()]
+    for call, want in calls:
+        torch.cuda.synchronize()
+        ends, outs = [], []
+        for k, s in enumerate(streams + streams):
+            with torch.cuda.stream(s):
+                if k % 2 == 0:
+                    torch.cuda._sleep(4000000)
+                outs.append(call())
+                e = torch.cuda.Event(enable_timing=True)
+                e.record()
+                ends.append(e)
+        torch.cuda.synchronize()
+        for o in outs:
+            assert rel_err(o, want) <= TOL
+        for before, after in zip(ends, ends[1:]):
+            assert before.elapsed_time(after) >= 0.0
+
+
+@pytest.mark.gpu
+def test_captured_calls_on_two_streams(gpu, tf):
+    """Two calls on one adjacency captured on a stream and one forked from it; the graph is replayed between eager calls."""
+    print("sw_gcn capture", flush=True)
+    A = tf.workloads.rmat(13, 8 << 13, seed=5)
+    n = A.shape[0]
+    x, w1, w2 = _two_layers(n, 4)
+    adj, xg, w1g, w2g = csr_tensor(A, "cuda"), x.cuda(), w1.cuda(), w2.cuda()
+    with torch.no_grad():
+        call = lambda: torch.ops.sw_gcn.fusedGCN(adj, xg, w1g, w2g, 8)
+        want = call().clone()
+        B = A.astype(np.float64)
+        assert rel_err(want, B @ (np.maximum(B @ (x.double().numpy() @ w1.double().numpy().T), 0.0) @ w2.double().numpy().T)) <= TOL
+        torch.cuda.synchronize()
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph):
+            cur = torch.cuda.current_stream()
+            first = call()
+            side.wait_stream(cur)
+            with torch.cuda.stream(side):
+                second = call()
+            third = call()
+            cur.wait_stream(side)
+        for _ in range(4):
+            for t in (first, second, third):
+                t.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            for t in (first, second, third):
+                assert torch.equal(t, want)
+            assert torch.equal(call(), want)
+            torch.cuda.synchronize()
