@@ -581,3 +581,46 @@ def test_executors_replay_from_a_graph(gpu, tf, orc):
     def check_ss(i):
         assert np.array_equal(D2.to_numpy(), oracle_spmm_spmm(orc, A, A, Cs[i])), i
     replay(lambda: tf.spmm_spmm(Ah, Ah, Cm, D2, S2, stream=st), fresh_c, check_ss)
+
+
+@pytest.mark.parametrize("K,N", [(64, 64), (128, 96), (100, 64)])
+def test_first_call_with_transposed_weights_can_be_captured(gpu, tf, K, N):
+    """Tiles that were warmed up with W as K x N are captured with W stored N x K (TF_C_TRANSPOSED): after a schedule's first call
+    no call allocates, so the capture succeeds; three replays with other features, eager calls in between."""
+    import ctypes as C
+    say(f"transposed weights under capture {K}x{N}")
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(sorted({line.split()[-1] for line in f if "libamdhip64.so" in line})[0])
+    A = tf.workloads.banded_random(30000, 32, 12, seed=77)
+    M = A.shape[0]
+    rng = np.random.default_rng(K)
+    Xs, W = [rng.uniform(-1, 1, (M, K)).astype(np.float32) for _ in range(3)], rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    Ah = tf.CsrMatrix.from_scipy(A).to_device()
+    S = tf.inspector(Ah, 1, op=tf.OP_GEMM_SPMM, N=N, K=K, max_redundancy=1.5)  # (an option given: tiles, not two products)
+    assert S.info()["n_fused_rows"] > 0 and S.info()["streamed"]
+    X, Wn, Wt = (tf.DenseMatrix.from_numpy(a) for a in (Xs[0], W, np.ascontiguousarray(W.T)))
+    D, E = tf.DenseMatrix(M, N), tf.DenseMatrix(M, N)
+    st = tf.Stream()
+    tf.gemm_spmm(Ah, X, Wn, E, S, stream=st)
+    st.synchronize()
+    graph, gexec = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(st.h, 0) == 0
+    try:
+        rc = tf.lib().tf_gemm_spmm(Ah.h, X.h, Wt.h, D.h, S.h, 16, st.h)
+    finally:
+        end = hip.hipStreamEndCapture(st.h, C.byref(graph))
+    assert rc == 0 and end == 0 and graph.value
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, C.c_size_t(0)) == 0
+    try:
+        for x in Xs:
+            X.copy_from(tf.DenseMatrix.from_numpy(x), stream=st)
+            D.fill(float("nan"), stream=st)
+            assert hip.hipGraphLaunch(gexec, st.h) == 0
+            tf.gemm_spmm(Ah, X, Wn, E, S, stream=st)
+            st.synchronize()
+            want = A.astype(np.float64) @ (x.astype(np.float64) @ W.astype(np.float64))
+            for got in (D, E):
+                assert np.abs(got.to_numpy() - want).max() <= 1e-5 * np.abs(want).max()
+    finally:
+        hip.hipGraphExecDestroy(gexec)
+        hip.hipGraphDestroy(graph)

@@ -63,8 +63,8 @@ struct DeviceSchedule {
   Tile2 *l2_tiles = nullptr; // two-layer tiles
   float *hidden = nullptr;   // tf_gcn_two_layers: the first layer's output, L x K of this (second-layer) schedule
   size_t hidden_floats = 0;
-  float *Bpad = nullptr;     // M x K' and K' x N copies of B and C, zero-padded, when K is not a multiple of 8
-  float *Cpad = nullptr;
+  float *Bpad = nullptr;     // M x K' copy of B, zero-padded, when K is not a multiple of 8
+  float *Cpad = nullptr;     // K' x N copy of C, zero-padded or from its transpose
   float *Cpanel = nullptr;   // K' x N and L x N: one column panel of C (zero-padded) and of D, when the caller's width is
   float *Dpanel = nullptr;   // not one the kernels take (user_N != N)
   // marching runs: the schedule's lists, and the ELL rows with the operands' values filled in
@@ -162,7 +162,7 @@ int default_compute_units() {
 
 void release_device_schedule(DeviceSchedule *d) {
   if (!d) return;
-  (void)hipFree(d->arena); (void)hipFree(d->Cpad); (void)hipFree(d->hidden);
+  (void)hipFree(d->arena); (void)hipFree(d->hidden);
   if (d->side) (void)hipStreamDestroy(d->side);
   if (d->fork) (void)hipEventDestroy(d->fork);
   if (d->join) (void)hipEventDestroy(d->join);
@@ -320,6 +320,8 @@ static tf_status ensure_device(tf_schedule *s) {
       parts.reserve((size_t)s->L * s->opts.N, &d->Dpanel);
     }
     if (tiled && s->user_K != s->opts.K) parts.reserve((size_t)s->M * s->opts.K, &d->Bpad);
+    // (also where K needs no padding: any call may come with TF_C_TRANSPOSED, and a captured one cannot allocate)
+    if (tiled && s->user_N == s->opts.N) parts.reserve((size_t)s->opts.K * s->opts.N, &d->Cpad);
   }
   tf_status rc = parts.make(&d->arena);
   if (!rc && s->long_part && s->plain_hot > 0) {
@@ -1026,7 +1028,6 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
     Bd = d->Bpad;
   }
   if (!panels && (c_t || s->user_K != s->opts.K)) {
-    if (!d->Cpad) TF_HIP(hipMalloc(reinterpret_cast<void **>(&d->Cpad), (size_t)s->opts.K * s->opts.N * sizeof(float)));
     if (c_t) TF_PHASE(s, "transpose_pad_kernel (C)", st, tf::launch_transpose_pad(C->d, C->M, C->N, 0, s->user_N, d->Cpad, s->opts.K, s->opts.N, st));
     else TF_PHASE(s, "pad_kernel (C)", st, tf::launch_pad(C->d, C->M, C->N, d->Cpad, s->opts.K, C->N, st));
     Cd = d->Cpad;

@@ -1095,6 +1095,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
   if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C
+  else if (s->user_N == s->opts.N && !s->launch_tiles.empty() && !s->two_passes) ws += (long long)s->opts.K * s->opts.N * 4;  // C from its transpose
   if (s->user_N != s->opts.N) ws += ((long long)s->L + s->opts.K) * s->opts.N * 4;  // one column panel of D and of C
   ws += (long long)s->rem_ptr.size() * 4 + (long long)s->rem_col.size() * 12;       // remainder rows in list order
   info->workspace_bytes = ws;
