@@ -624,3 +624,46 @@ def test_first_call_with_transposed_weights_can_be_captured(gpu, tf, K, N):
     finally:
         hip.hipGraphExecDestroy(gexec)
         hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("pattern", ["rmat", "stencil"])
+def test_values_of_a_captured_call_are_not_taken_for_written(gpu, tf, pattern):
+    """A call with another matrix of the same pattern is captured and never replayed: the next eager call with that matrix copies its
+    values itself (rows in lists and long rows by partition; marching runs)."""
+    import ctypes as C
+    say(f"values of a captured call {pattern}")
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(sorted({line.split()[-1] for line in f if "libamdhip64.so" in line})[0])
+    st = tf.Stream()
+    A1 = tf.workloads.rmat(13, 8 << 13, seed=9) if pattern == "rmat" else tf.workloads.laplacian_3d(20)
+    A2 = A1.copy()
+    A2.data = np.random.default_rng(1).uniform(-1, 1, A2.nnz).astype(np.float32)
+    M, N = A1.shape[0], 64
+    Xh = tf.workloads.uniform((M, N), 3)
+    X, D = tf.DenseMatrix.from_numpy(Xh), tf.DenseMatrix(M, N)
+    H1, H2 = (tf.CsrMatrix.from_scipy(A).to_device() for A in (A1, A2))
+    if pattern == "rmat":
+        W = tf.DenseMatrix.from_numpy(np.eye(N, dtype=np.float32))
+        S = tf.inspector(H1, 1, op=tf.OP_GEMM_SPMM, N=N, K=N, long_row_partition=1)
+        assert S.info()["long_row_hot_cols"] > 0
+        call = lambda H: tf.gemm_spmm(H, X, W, D, S, stream=st)
+        want = lambda A: A.astype(np.float64) @ Xh.astype(np.float64)
+    else:
+        S = tf.inspector(H1, 1, op=tf.OP_SPMM_SPMM, N=N, inner=H1, march=1)
+        assert S.info()["marched"]
+        call = lambda H: tf.spmm_spmm(H, H, X, D, S, stream=st)
+        want = lambda A: A.astype(np.float64) @ (A.astype(np.float64) @ Xh.astype(np.float64))
+    call(H1)
+    st.synchronize()
+    graph = C.c_void_p()
+    assert hip.hipStreamBeginCapture(st.h, 0) == 0
+    try:
+        call(H2)
+    finally:
+        assert hip.hipStreamEndCapture(st.h, C.byref(graph)) == 0
+    hip.hipGraphDestroy(graph)
+    for H, A in ((H2, A2), (H1, A1), (H2, A2)):
+        call(H)
+        st.synchronize()
+        ref = want(A)
+        assert np.abs(D.to_numpy() - ref).max() <= 1e-5 * np.abs(ref).max()

@@ -362,6 +362,14 @@ static hipError_t prof_end(tf_schedule *s, hipStream_t st) {
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// What to remember as the matrix whose values a call on `st` puts in a schedule's order: none when the call is being captured, for
+// nothing is written before the graph is launched, if it ever is.
+static unsigned long long written_now(hipStream_t st, unsigned long long serial) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (st && hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+  return status == hipStreamCaptureStatusNone ? serial : 0;
+}
+
 // The hot segments of column-partitioned long rows: segments of partition p are worked on by the
 // workgroups that land on XCD p.  The values in the order of the regrouped entries -- what the
 // reference's reordered adjacency (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653)
@@ -371,10 +379,9 @@ static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 // that both the hot and the cold launch are ordered after: the caller's, before a second stream forks.
 static tf_status ensure_segment_values(const tf_csr *A, tf_schedule *s, hipStream_t st) {
   DeviceSchedule *d = s->dev;
-  const bool have_values = A->serial != 0 && d->seg_val_serial == A->serial;
-  if (!have_values)
-    TF_PHASE(s, "scatter_values_kernel", st, launch_scatter_values(d->ent_src, d->ent_pos, A->x, d->seg_val, (int)s->seg_src.size(), st));
-  d->seg_val_serial = A->serial;
+  if (A->serial != 0 && d->seg_val_serial == A->serial) return TF_OK;
+  TF_PHASE(s, "scatter_values_kernel", st, launch_scatter_values(d->ent_src, d->ent_pos, A->x, d->seg_val, (int)s->seg_src.size(), st));
+  d->seg_val_serial = written_now(st, A->serial);
   return TF_OK;
 }
 // What the row products of a call read and write: T (row stride ldt) the intermediate or, for a rows-only schedule, the
@@ -426,9 +433,10 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
     if (A->serial == 0) {
       a.val_first = d->rem_first;
     } else {
-      if (d->rem_val_serial != A->serial)
+      if (d->rem_val_serial != A->serial) {
         TF_PHASE(s, "gather_values_kernel", st, launch_gather_values(d->rem_src, A->x, d->rem_val, (int)s->rem_src.size(), st));
-      d->rem_val_serial = A->serial;
+        d->rem_val_serial = written_now(st, A->serial);
+      }
       a.Ax = d->rem_val;
     }
     a.compact = 1;
@@ -837,10 +845,11 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     // createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653): filled in on the first call with
     // uploaded matrices, whose device arrays never change, and on every call with wrapped ones.
     const bool have = A->serial != 0 && B->serial != 0 && d->m_serial_a == A->serial && d->m_serial_b == B->serial;
-    if (!have)
+    if (!have) {
       TF_PHASE(s, "march_fill_kernel", st, tf::launch_march_fill(d->m_ell_off, d->m_ell_src, A->x, B->x, d->m_ell, s->march_ell_off.size(), st));
-    d->m_serial_a = A->serial;
-    d->m_serial_b = B->serial;
+      d->m_serial_a = tf::written_now(st, A->serial);
+      d->m_serial_b = tf::written_now(st, B->serial);
+    }
     TF_PHASE(s, "fused_spmm_spmm_march_kernel", st,
              tf::launch_fused_spmm_spmm_march(d->m_runs, (int)s->march_runs.size() / 2, d->m_row_ptr, d->m_load_ptr, d->m_load,
                                               d->m_row_out, d->m_ell, C->d, D->d, d->m_trash, s->opts.N, s->lds_bytes, s->march_tpg,
