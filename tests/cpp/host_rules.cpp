@@ -121,11 +121,52 @@ static int partial_sums() {
   return bad;
 }
 
+// Hub rows that end the choice of one launch are seen before its lists are made; rows near the lengths where lists differ are not
+// taken for them.  And columns out of range are refused by both inspectors, wherever in a row they stand.
+static int hubs_and_columns() {
+  int bad = 0;
+  const int M = 6000;
+  for (int longest : {31, 32, 33, 64, 65, 127, 128, 129, 1025})
+    for (int K : {64, 30})
+      for (int N : {64, 40, 20}) {
+        std::vector<int> p(1, 0), i;
+        for (int r = 0; r < M; ++r) {
+          const int len = r == 3000 ? longest : 3;
+          for (int k = 0; k < len; ++k) i.push_back((r + k * 3) % M);
+          p.push_back((int)i.size());
+        }
+        tf_inspect_opts o{};
+        o.struct_size = sizeof(o);
+        o.op = TF_OP_GEMM_SPMM;
+        o.K = K;
+        o.N = N;
+        tf_schedule *s = nullptr, *rows = nullptr;
+        if (tf_inspect(M, M, p.data(), i.data(), &o, &s) || tf_inspect_spmm(M, M, p.data(), i.data(), K, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
+        const bool cut = !rows->long_chunks.empty();
+        if (cut != (longest > 32) || (s->one_launch && cut) || (!cut && !s->one_launch) || (cut && s->spmm_first != (3 * K <= 2 * N)) ||
+            (s->two_passes && s->two_passes->opts.N < (s->spmm_first ? K : N))) {
+          printf("longest %d K %d N %d: one launch %d, (A B) C %d\n", longest, K, N, s->one_launch, s->spmm_first);
+          ++bad;
+        }
+        tf_schedule_free(s);
+        tf_schedule_free(rows);
+        for (int at : {0, 8999, 9000 + longest - 1, (int)i.size() - 1})
+          for (int c : {-1, INT_MIN, M, INT_MAX}) {
+            const int was = i[at];
+            i[at] = c;
+            if (tf_inspect(M, M, p.data(), i.data(), &o, &s) != TF_EINVAL || tf_inspect_spmm(M, M, p.data(), i.data(), N, 0, &rows) != TF_EINVAL) { printf("column %d accepted\n", c); ++bad; }
+            i[at] = was;
+          }
+      }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
     const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
-                  : !strcmp(argv[k], "partial_sums") ? partial_sums() : 1;
+                  : !strcmp(argv[k], "partial_sums") ? partial_sums()
+                  : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

@@ -97,7 +97,9 @@ extern "C" uint64_t tf_pattern_hash(int M, const int *Ap, const int *Ai) {
   return h ? h : 1;
 }
 
-static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, bool rows_only, tf_schedule **out);
+enum { kTiles, kRows, kRowsOfChecked };
+constexpr int kWholeRowMax = 128;  // rows of more entries are cut up, whatever the widths and row counts (unless the caller says otherwise)
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out);
 
 // Which SpMM-SpMM schedules the executor runs as two row products instead of in their tiles, when the caller has not asked
 // for tiles of its own.
@@ -141,6 +143,15 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
                                : K <= 64 && K <= N && (N <= 64 || M <= 150000) && !(streamed && K > 32));
     S->spmm_first = S->one_launch || 3LL * K <= 2LL * N;
     want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || !S->gemm_stream));
+    if (S->one_launch) {  // hub rows known before any list is made (see below)
+      int longest = 0;
+      for (int i = 0; i < S->L; ++i) longest = std::max(longest, Ap[i + 1] - Ap[i]);
+      if (longest > kWholeRowMax) {
+        S->one_launch = false;
+        S->spmm_first = 3LL * K <= 2LL * N;
+        want = S->spmm_first || tiled;
+      }
+    }
     if (S->spmm_first) N = K;
   } else if (S->march)
     want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
@@ -155,7 +166,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
   o.xcd_chunk_rows = given.xcd_chunk_rows;
   o.reorder_adjacency = given.reorder_adjacency;
   o.pattern_hash = S->pattern_hash;
-  if (tf_status rc = inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes)) return rc;
+  if (tf_status rc = inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes)) return rc;
   const tf_schedule *rows = S->two_passes;
   if (S->one_launch && (!rows->long_chunks.empty() || rows->long_part || rows->rem_flagged)) {
     // hub rows: another order of the products, or the schedule's own (a GEMM of the rows that are read, placed by reads)
@@ -165,14 +176,16 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
       tf_schedule_free(S->two_passes);
       S->two_passes = nullptr;
       o.N = S->user_N;  // (the lists and the room for partial sums are for the width that is gathered)
-      if (!S->launch_tiles.empty()) return inspect(S->L, S->M, Ap, Ai, &o, true, &S->two_passes);
+      if (!S->launch_tiles.empty()) return inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes);
     }
   }
   return TF_OK;
 }
 
-// rows_only: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.
-static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, bool rows_only, tf_schedule **out) {
+// kRows: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.  kRowsOfChecked: the same of a
+// pattern that an inspection under way has checked (a pass over the entries less: 2.5 of 14.5 ms at 100,000 rows of 16).
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out) {
+  const bool rows_only = what != kTiles;
   if (!out) return tf::fail(TF_EINVAL, "tf_inspect: out is null");
   *out = nullptr;
   if (L <= 0 || M <= 0 || !Ap || !user) return tf::fail(TF_EINVAL, "tf_inspect: bad L/M/Ap/opts");
@@ -299,19 +312,21 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     S->slab_ld = gemm_regw ? o.N + 4 : o.N;
 
     // Column extent of every second-op row (columns need not be sorted).
-    std::vector<int> lo(L), hi(L);
-    for (int i = 0; i < L; ++i) {
-      int a = INT_MAX, b = -1;
+    std::vector<int> lo(rows_only ? 0 : L), hi(rows_only ? 0 : L);
+    for (int i = 0; i < L && what != kRowsOfChecked; ++i) {
+      int a = INT_MAX, b = INT_MIN;
       for (int k = Ap[i]; k < Ap[i + 1]; ++k) {
-        const int c = Ai[k];
-        if (c < 0 || c >= M) {
-          delete S;
-          return tf::fail(TF_EINVAL, "tf_inspect: column %d out of range at row %d", c, i);
-        }
-        a = std::min(a, c);
-        b = std::max(b, c);
+        a = std::min(a, Ai[k]);
+        b = std::max(b, Ai[k]);
       }
-      if (b < 0) { a = std::min(i, M - 1); b = a - 1; }  // empty row: no dependence
+      if (Ap[i + 1] == Ap[i]) {  // empty row: no dependence
+        a = std::min(i, M - 1);
+        b = a - 1;
+      } else if (a < 0 || b >= M) {
+        delete S;
+        return tf::fail(TF_EINVAL, "tf_inspect: column %d out of range at row %d", a < 0 ? a : b, i);
+      }
+      if (rows_only) continue;
       lo[i] = a;
       hi[i] = b + 1;
     }
@@ -586,6 +601,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // worked on by a whole workgroup.
     const int chunk_nnz = std::max(o.long_row_nnz, 1024);
     std::vector<char> need(M, 0);
+    if (rows_only) S->rem_rows.reserve(L);
     for (int i = 0; i < L; ++i) {
       if (fused[i]) { S->fused_nnz += Ap[i + 1] - Ap[i]; continue; }
       if (!rows_only)
@@ -628,10 +644,11 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       // themselves.  R-MAT graphs, rows of up to 32 / 64 / 128 entries kept whole: 2^16 nodes, N = 8 / 64, 25.9 / 25.8 / 36.7 and 37.4 / 36.1 / 38.3 us,
       // 2^17 nodes 37 / 40.7 / 47.3 and 56 / 52.9 / 52.4, 2^18 nodes 64 / 61 / 70 and 107 / 104 / 96, 2^20 nodes 196 / 194 / 178 and
       // 555 / 556 / 555 (N = 32: 279 / 270 / 242).
-      const int whole = want ? 64 : L >= 200000 && o.N >= 16 ? 128 : L >= 100000 && o.N >= 48 ? 64 : 32;
+      const int whole = want ? 64 : L >= 200000 && o.N >= 16 ? kWholeRowMax : L >= 100000 && o.N >= 48 ? 64 : 32;
       if (user->long_row_nnz <= 0 && whole > o.long_row_nnz && S->long_chunks.size() < (size_t)INT_MAX) {
         std::vector<tf::LongRow> keep_rows;
         std::vector<tf::LongChunk> keep_chunks;
+        const size_t n_short = S->rem_rows.size();
         for (const auto &lr : S->long_rows) {
           if (Ap[lr.row + 1] - Ap[lr.row] <= whole) { S->rem_rows.push_back(lr.row); continue; }
           tf::LongRow nr{lr.row, (int)keep_chunks.size(), lr.count, 0};
@@ -644,7 +661,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         }
         S->long_rows.swap(keep_rows);
         S->long_chunks.swap(keep_chunks);
-        std::sort(S->rem_rows.begin(), S->rem_rows.end());
+        std::inplace_merge(S->rem_rows.begin(), S->rem_rows.begin() + n_short, S->rem_rows.end());
         S->opts.long_row_nnz = o.long_row_nnz = whole;
         long_nnz = 0;
         for (const auto &lr : S->long_rows) long_nnz += Ap[lr.row + 1] - Ap[lr.row];
@@ -796,7 +813,6 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         }
         return far * 8 > (double)M * entries;
       };
-      std::vector<int> byc[5];
       // Rows without entries, when they are many (half of the nodes of an R-MAT graph are isolated), leave the list: a row of
       // zeros needs no lane group of its own and no row pointers, the row kernels clear it beside their other work.
       {
@@ -810,11 +826,11 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
           S->rem_rows.swap(keep);
         }
       }
-      for (int i : S->rem_rows) byc[cls(i)].push_back(i);
+      size_t in_class[5] = {};
+      for (int i : S->rem_rows) ++in_class[cls(i)];
       // (a product of all rows whose rows are nearly all of one class -- a stencil and its boundary -- stays in order too: the
       // list costs its rows an indirection and the entries a copy; 27 points, 40^3, N = 16: 21.1 us through a list, 19.1 without)
-      size_t most = 0;
-      for (auto &v : byc) most = std::max(most, v.size());
+      const size_t most = *std::max_element(in_class, in_class + 5);
       const bool far = scattered();
       if (!((int)S->rem_rows.size() == L && most * 8 >= S->rem_rows.size() * 7)) {
         if (far) {
@@ -824,8 +840,10 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
           for (int len = 0; len <= o.long_row_nnz; ++len) at[len + 1] += at[len];
           for (int i : rows) S->rem_rows[at[o.long_row_nnz - (Ap[i + 1] - Ap[i])]++] = i;
         } else {
-          S->rem_rows.clear();
-          for (auto &v : byc) S->rem_rows.insert(S->rem_rows.end(), v.begin(), v.end());
+          size_t at[5] = {};
+          for (int c = 1; c < 5; ++c) at[c] = at[c - 1] + in_class[c - 1];
+          const std::vector<int> rows(S->rem_rows);
+          for (int i : rows) S->rem_rows[at[cls(i)]++] = i;
         }
       }
       S->rem_identity = (int)S->rem_rows.size() == L;
@@ -1029,7 +1047,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 }
 
 extern "C" tf_status tf_inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, tf_schedule **out) {
-  return inspect(L, M, Ap, Ai, user, false, out);
+  return inspect(L, M, Ap, Ai, user, kTiles, out);
 }
 
 extern "C" tf_status tf_inspect_spmm(int L, int M, const int *Ap, const int *Ai, int N, uint64_t pattern_hash, tf_schedule **out) {
@@ -1038,7 +1056,7 @@ extern "C" tf_status tf_inspect_spmm(int L, int M, const int *Ap, const int *Ai,
   o.op = TF_OP_SPMM_SPMM;
   o.N = N;
   o.pattern_hash = pattern_hash;
-  return inspect(L, M, Ap, Ai, &o, true, out);
+  return inspect(L, M, Ap, Ai, &o, kRows, out);
 }
 
 extern "C" void tf_schedule_free(tf_schedule *s) {
