@@ -668,21 +668,8 @@ __global__ __launch_bounds__(kBlock) void fused_gemm_spmm_kernel(
   }
 }
 
-// Plain GEMM  Y = X * W  (tf_gemm) when K*N is too large to keep W in LDS: 128 rows per
-// workgroup, W streamed through LDS in kc-row slices.
-template <int NB>
-__global__ __launch_bounds__(kBlock) void gemm_kernel(const float *__restrict__ X, const float *__restrict__ W,
-                                                      float *__restrict__ Y, int M, int K, int kc,
-                                                      int per_xcd, int n_blocks) {
-  extern __shared__ __align__(16) float lds[];
-  const int b = xcd_contiguous(blockIdx.x, per_xcd);
-  if (b >= n_blocks) return;
-  const int p0 = b * 128, p1 = min(M, p0 + 128);
-  tile_gemm<NB>(X, W, K, kc, p0, p1, lds, nullptr, Y, p0, p1);
-}
-
 // Row-list GEMM  Y[r,:] = X[r,:K] * W  for r = rows[q] (or r = q when rows is null):
-// intermediate rows that no tile fuses, and tf_gemm.  Persistent: W (K x N) is copied to
+// intermediate rows that no tile fuses, and tf_gemm, for many rows (row_gemm_takes in tf_api.cpp).  Persistent: W (K x N) is copied to
 // LDS once per workgroup, then every wavefront walks its own 32-row blocks with no
 // barrier at all; the rows of X for the next 32 values of k are already in flight
 // (16 bytes per lane and load, see tile_gemm for the k permutation) while the MFMAs of
@@ -1986,16 +1973,15 @@ hipError_t launch_fused_gemm_spmm_stream(const TileDesc *tiles, int n_tiles, con
 hipError_t launch_gemm(const float *X, const float *W, float *Y, const int *rows, int n_rows, int K,
                        int N, int compute_units, hipStream_t st, int y_by_position) {
   if (n_rows <= 0) return hipSuccess;
-  if (y_by_position && !rows) return hipErrorInvalidValue;
+  if ((y_by_position && !rows) || (long long)K * N * 4 > 131072) return hipErrorInvalidValue;
   const int NB = N / 32;
   hipError_t err = hipSuccess;
   const int w_bytes = K * N * 4;
-  if (w_bytes <= 131072) {
-    // W resident in LDS: persistent workgroups, as many per compute unit as the LDS allows
-    const int per_cu = 1;  // register use (accumulators + both operand pipelines) allows one 8-wave workgroup
-    const int nrb = (n_rows + 31) / 32;
-    const int grid = std::max(1, std::min(compute_units * per_cu, (nrb + kGemmBlock / 64 - 1) / (kGemmBlock / 64)));
-    const int lds = w_bytes + (rows ? (kGemmBlock / 64) * kGemmSeg * 32 * 4 : 0);  // + the wavefronts' row numbers
+  // W resident in LDS: persistent workgroups, as many per compute unit as the LDS allows
+  const int per_cu = 1;  // register use (accumulators + both operand pipelines) allows one 8-wave workgroup
+  const int nrb = (n_rows + 31) / 32;
+  const int grid = std::max(1, std::min(compute_units * per_cu, (nrb + kGemmBlock / 64 - 1) / (kGemmBlock / 64)));
+  const int lds = w_bytes + (rows ? (kGemmBlock / 64) * kGemmSeg * 32 * 4 : 0);  // + the wavefronts' row numbers
 #define CALL3(NB_, LIST_, G4C_, YPOS_)                                                              \
   err = allow_lds(gemm_rows_kernel<NB_, LIST_, G4C_, YPOS_>, lds);                                  \
   if (err == hipSuccess)                                                                            \
@@ -2013,24 +1999,10 @@ hipError_t launch_gemm(const float *X, const float *W, float *Y, const int *rows
     }                                                   \
   } while (0)
 #define CALL(NB_) do { if (rows && y_by_position) { CALL2(NB_, true, true); } else if (rows) { CALL2(NB_, true, false); } else { CALL2(NB_, false, false); } } while (0)
-    TF_DISPATCH_NB(NB, CALL);
+  TF_DISPATCH_NB(NB, CALL);
 #undef CALL
 #undef CALL2
 #undef CALL3
-    return err != hipSuccess ? err : hipGetLastError();
-  }
-  if (rows) return hipErrorInvalidValue;  // the streamed-W kernel takes contiguous rows only
-  const int kc = std::min(K, std::max(8, (32768 / (4 * N)) / 8 * 8));
-  const int blocks = (n_rows + 127) / 128;
-  const int per = per_xcd_of(blocks);
-  const int lds_bytes = kc * N * 4;
-#define CALL(NB_)                                                                               \
-  err = allow_lds(gemm_kernel<NB_>, lds_bytes);                                                 \
-  if (err == hipSuccess)                                                                        \
-    hipLaunchKernelGGL((gemm_kernel<NB_>), dim3(grid_of(blocks)), dim3(kBlock), lds_bytes, st, X, W, \
-                       Y, n_rows, K, kc, per, blocks)
-  TF_DISPATCH_NB(NB, CALL);
-#undef CALL
   return err != hipSuccess ? err : hipGetLastError();
 }
 
