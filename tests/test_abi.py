@@ -56,3 +56,18 @@ def test_cpp_header_compiles(tmp_path):
     r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", os.path.join(ROOT, "include"), str(src)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_default_build_without_torch():
+    """`make` builds the library, the API test program and the shim where python3 has no torch; `make torch` then says what is missing."""
+    import shutil
+    import subprocess
+    if shutil.which("make") is None:
+        pytest.skip("no make")
+    csrc = os.path.join(ROOT, "tile-fusion_amd", "csrc")
+    make = lambda *a: subprocess.run(["make", "-B", "-n", "-C", csrc, *a], capture_output=True, text=True, timeout=120)
+    with_torch, without = make("TORCH=/x/torch"), make("TORCH=")
+    assert with_torch.returncode == 0 and "-o %s" % os.path.join(ROOT, "tile-fusion_amd", "lib", "libtf_torch.so") in with_torch.stdout
+    assert without.returncode == 0 and "tf_torch.cpp" not in without.stdout and "libtilefusion_hip.so" in without.stdout
+    asked = make("TORCH=", "torch").stdout  # (the recipe's first line fails with TORCH empty)
+    assert asked.index('test -n ""') < asked.index("tf_torch.cpp") and "needs torch" in asked
