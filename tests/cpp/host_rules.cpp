@@ -78,6 +78,7 @@ static int one_launch_fits() {
         o.N = N;
         tf_schedule *s = nullptr;
         if (tf_inspect(M, M, p.data(), i.data(), &o, &s)) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; continue; }
+        if (tf_schedule_validate(s, M, M, p.data(), i.data())) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; }
         const int lds = s->one_launch ? (s->two_passes->rem_rows.size() < 24000 ? 16 : 64) * ((K + 15) / 16 * 16 + 4) * 4 : 0;
         if (lds > 163840) { printf("M %d K %d N %d: one launch with %d bytes of LDS\n", M, K, N, lds); ++bad; }
         taken += s->one_launch;
@@ -109,6 +110,7 @@ static int partial_sums() {
         o.N = N;
         tf_schedule *s = nullptr;
         if (tf_inspect(M, M, p.data(), i.data(), &o, &s)) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; continue; }
+        if (tf_schedule_validate(s, M, M, p.data(), i.data())) { printf("M %d K %d N %d: %s\n", M, K, N, tf::g_err); ++bad; }
         if (const tf_schedule *rows = s->two_passes) {
           const int width = s->spmm_first ? K : N;
           if (rows->opts.N < width) { printf("M %d K %d N %d: partial sums of %d columns for a product of %d\n", M, K, N, rows->opts.N, width); ++bad; }
@@ -142,6 +144,7 @@ static int hubs_and_columns() {
         o.N = N;
         tf_schedule *s = nullptr, *rows = nullptr;
         if (tf_inspect(M, M, p.data(), i.data(), &o, &s) || tf_inspect_spmm(M, M, p.data(), i.data(), K, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
+        if (tf_schedule_validate(s, M, M, p.data(), i.data()) || tf_schedule_validate(rows, M, M, p.data(), i.data())) { printf("%s\n", tf::g_err); ++bad; }
         const bool cut = !rows->long_chunks.empty();
         if (cut != (longest > 32) || (s->one_launch && cut) || (!cut && !s->one_launch) || (cut && s->spmm_first != (3 * K <= 2 * N)) ||
             (s->two_passes && s->two_passes->opts.N < (s->spmm_first ? K : N))) {

@@ -1141,6 +1141,18 @@ extern "C" tf_status tf_schedule_get_view(const tf_schedule *s, tf_schedule_view
   return tf::emit_out("tf_schedule_get_view", caller, full, TF_SIZE_THROUGH(tf_schedule_view, n_step_ptr));
 }
 
+// The row lists that a schedule of two products runs: every row once, room for partial sums of the width that is gathered, and in
+// one launch no row whose sum comes from several workgroups.
+static tf_status validate_two_passes(const tf_schedule *s, int L, int M, const int *Ap, const int *Ai) {
+  const tf_schedule *rows = s->two_passes;
+  if (!rows) return s->one_launch || s->spmm_first ? tf::fail(TF_ESCHEDULE, "(A B) C without row lists") : TF_OK;
+  const int width = s->opts.op == TF_OP_SPMM_SPMM ? s->opts.N : s->spmm_first ? s->user_K : s->user_N;
+  if (!rows->rows_only || rows->opts.N < width) return tf::fail(TF_ESCHEDULE, "two products: row lists for %d columns, %d are gathered", rows->opts.N, width);
+  if (s->one_launch && (!s->spmm_first || !rows->long_rows.empty() || rows->rem_flagged || !tf::spmm_gemm_fits((int)rows->rem_rows.size(), s->user_K, s->user_N)))
+    return tf::fail(TF_ESCHEDULE, "one launch: long or marked rows, or more LDS than there is");
+  return tf_schedule_validate(rows, L, M, Ap, Ai);
+}
+
 extern "C" tf_status tf_schedule_validate(const tf_schedule *s, int L, int M, const int *Ap,
                                           const int *Ai) {
   if (!s || !Ap) return tf::fail(TF_EINVAL, "tf_schedule_validate: null argument");
@@ -1149,9 +1161,10 @@ extern "C" tf_status tf_schedule_validate(const tf_schedule *s, int L, int M, co
                     s->L, s->M, s->nnz, L, M, Ap[L]);
   if (s->march)
     return tf::fail(TF_EINVAL, "tf_schedule_validate: marching runs are checked against both patterns: use tf_schedule_validate_inner");
+  if (tf_status rc = validate_two_passes(s, L, M, Ap, Ai)) return rc;
   const int row_bytes = (s->slab_ld > 0 ? s->slab_ld : s->opts.N) * 4 + (s->gemm_regw ? 16 : 0);
   std::vector<int> owner(M, -1), done(L, 0);
-  std::vector<char> stored(M, 0);
+  std::vector<char> stored(M, s->rows_only ? 1 : 0);  // (one product reads rows that the caller has)
   int prev_end = 0;
   for (size_t ti = 0; ti < s->tiles.size(); ++ti) {
     const auto &t = s->tiles[ti];
@@ -1207,7 +1220,7 @@ extern "C" tf_status tf_schedule_validate(const tf_schedule *s, int L, int M, co
           return tf::fail(TF_ESCHEDULE, "fused row %d reads intermediate row %d outside tile %zu [%d,%d)", i, Ai[k], ti, t.prod_begin, t.prod_end);
     }
   }
-  if (prev_end != M) return tf::fail(TF_ESCHEDULE, "owned rows end at %d, expected %d", prev_end, M);
+  if (prev_end != M && !s->rows_only) return tf::fail(TF_ESCHEDULE, "owned rows end at %d, expected %d", prev_end, M);
   auto check_rem = [&](int i) -> tf_status {
     if (i < 0 || i >= L) return tf::fail(TF_ESCHEDULE, "remainder row %d out of range", i);
     for (int k = Ap[i]; k < Ap[i + 1]; ++k)
@@ -1362,6 +1375,7 @@ extern "C" tf_status tf_schedule_validate_inner(const tf_schedule *s, int L, int
     if (inner_cols != s->opts.inner_cols || inner_Ap[M] != s->inner_nnz || tf_pattern_hash(M, inner_Ap, inner_Ai) != s->inner_hash ||
         tf_pattern_hash(L, Ap, Ai) != s->pattern_hash)
       return tf::fail(TF_ESCHEDULE, "the schedule's runs were built from another inner pattern");
+    if (tf_status rc = validate_two_passes(s, L, M, Ap, Ai)) return rc;
     return tf::validate_march(s, M, Ap, Ai, inner_Ap, inner_Ai);
   }
   if (tf_status rc = tf_schedule_validate(s, L, M, Ap, Ai)) return rc;
