@@ -58,6 +58,7 @@ struct DeviceSchedule {
   // the short remainder rows stored in the order of the row list: row pointers, columns, where each value (rem_first: each
   // row's first) comes from in A's array, and the values themselves (of the matrix rem_val_serial that does not change)
   int *rem_ptr = nullptr, *rem_col = nullptr, *rem_src = nullptr, *rem_first = nullptr;
+  bool rem_first_known = false;
   float *rem_val = nullptr;
   unsigned long long rem_val_serial = 0;
   Tile2 *l2_tiles = nullptr; // two-layer tiles
@@ -242,7 +243,6 @@ static tf_status ensure_device(tf_schedule *s) {
   std::vector<LongRow> summed;  // the rows that partial sums are added up for
   std::vector<int> chunk_long;
   std::vector<unsigned> arrived;
-  std::vector<int> rem_first;
   if (s->two_passes) {  // (the lists are the other schedule's)
     parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
     parts.list(s->l2_tiles, &d->l2_tiles);
@@ -272,8 +272,7 @@ static tf_status ensure_device(tf_schedule *s) {
       parts.list(s->rem_col, &d->rem_col);
       parts.list(s->rem_src, &d->rem_src);
       parts.reserve(s->rem_src.size(), &d->rem_val);
-      for (size_t q = 0; q < s->rem_rows.size(); ++q) rem_first.push_back(s->rem_ptr[q] < s->rem_ptr[q + 1] ? s->rem_src[s->rem_ptr[q]] : 0);
-      parts.list(rem_first, &d->rem_first);
+      parts.reserve(s->rem_rows.size(), &d->rem_first);
     }
     const size_t N = (size_t)std::max(s->opts.N, s->user_N);
     size_t slots = 0;  // partial sums
@@ -362,7 +361,7 @@ static hipError_t prof_end(tf_schedule *s, hipStream_t st) {
 
 static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// What to remember as the matrix whose values a call on `st` puts in a schedule's order: none when the call is being captured, for
+// What to remember as the matrix whose values a call on `st` puts in a schedule's order: none (0) when the call is being captured, for
 // nothing is written before the graph is launched, if it ever is.
 static unsigned long long written_now(hipStream_t st, unsigned long long serial) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -431,6 +430,11 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
     a.rows = d->rem_rows;
     a.Ap = d->rem_ptr; a.Ai = d->rem_col;
     if (A->serial == 0) {
+      if (!d->rem_first_known) {  // (a part of the pattern: the same for every matrix the schedule is run on)
+        TF_PHASE(s, "gather_values_kernel", st,
+                 launch_gather_values(d->rem_rows, reinterpret_cast<const float *>(A->p), reinterpret_cast<float *>(d->rem_first), a.n_rows, st));
+        d->rem_first_known = written_now(st, 1) != 0;
+      }
       a.val_first = d->rem_first;
     } else {
       if (d->rem_val_serial != A->serial) {
