@@ -52,7 +52,7 @@ struct DeviceSchedule {
   LongRow *seg_groups = nullptr;
   float *inter = nullptr;    // M x N intermediate, only if some tile writes back
   float *partial = nullptr;  // n_long_chunks (or segments) x N
-  int *seg_ptr = nullptr, *ent_src = nullptr, *ent_pos = nullptr, *seg_col = nullptr, *lrow_seg = nullptr;  // column-partitioned long rows
+  int *seg_ptr = nullptr, *seg_src = nullptr, *seg_col = nullptr, *lrow_seg = nullptr;  // column-partitioned long rows
   float *seg_val = nullptr;  // A's values in the order of the regrouped entries
   unsigned long long seg_val_serial = 0;  // the uploaded matrix they were taken from (0: none)
   // the short remainder rows stored in the order of the row list: row pointers, columns, where each value (rem_first: each
@@ -102,7 +102,6 @@ hipError_t launch_gather_values(const int *, const float *, float *, int, hipStr
 hipError_t launch_march_fill(const int *, const int *, const float *, const float *, int *, size_t, hipStream_t);
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
                                         const float *, float *, float *, int, int, int, int, int, int, int, hipStream_t);
-hipError_t launch_scatter_values(const int *, const int *, const float *, float *, int, hipStream_t);
 hipError_t launch_seg_reduce(const LongRow *, int, int, const LongRow *, int, const int *, const float *, float *, int, int, int, int, hipStream_t);
 hipError_t launch_fused_gemm_spmm(const TileDesc *, int, const int *, const float *, const float *,
                                   int, int, const int *, const int *, const float *, float *,
@@ -303,8 +302,7 @@ static tf_status ensure_device(tf_schedule *s) {
     d->n_long_rows = (int)summed.size();
     if (s->long_part) {
       parts.list(s->seg_ptr, &d->seg_ptr);
-      parts.list(s->ent_src, &d->ent_src);
-      parts.list(s->ent_pos, &d->ent_pos);
+      parts.list(s->seg_src, &d->seg_src);
       parts.list(s->seg_col, &d->seg_col);
       parts.list(s->lrow_seg, &d->lrow_seg);
       parts.list(s->seg_groups, &d->seg_groups);
@@ -379,7 +377,7 @@ static unsigned long long written_now(hipStream_t st, unsigned long long serial)
 static tf_status ensure_segment_values(const tf_csr *A, tf_schedule *s, hipStream_t st) {
   DeviceSchedule *d = s->dev;
   if (A->serial != 0 && d->seg_val_serial == A->serial) return TF_OK;
-  TF_PHASE(s, "scatter_values_kernel", st, launch_scatter_values(d->ent_src, d->ent_pos, A->x, d->seg_val, (int)s->seg_src.size(), st));
+  TF_PHASE(s, "gather_values_kernel", st, launch_gather_values(d->seg_src, A->x, d->seg_val, (int)s->seg_src.size(), st));
   d->seg_val_serial = written_now(st, A->serial);
   return TF_OK;
 }

@@ -753,18 +753,6 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
           }
           S->seg_col.resize(S->seg_src.size());
           for (size_t k = 0; k < S->seg_src.size(); ++k) S->seg_col[k] = Ai[S->seg_src[k]];
-          // the executor copies A's values into this order walking A's array once: pairs sorted by source
-          {
-            std::vector<int> pos_of((size_t)nnz);
-            for (size_t e = 0; e < S->seg_src.size(); ++e) pos_of[S->seg_src[e]] = (int)e;
-            S->ent_src.reserve(S->seg_src.size());
-            S->ent_pos.reserve(S->seg_src.size());
-            std::vector<int> lrows;
-            for (const auto &lr : S->long_rows) lrows.push_back(lr.row);
-            std::sort(lrows.begin(), lrows.end());
-            for (const int i : lrows)
-              for (int k = Ap[i]; k < Ap[i + 1]; ++k) { S->ent_src.push_back(k); S->ent_pos.push_back(pos_of[k]); }
-          }
           // A row adds up its segments' sums in a fixed order; a hub row has thousands of them, so
           // groups of up to 32 segments are summed first (into slots behind the segments').
           const int n_seg = (int)S->seg_ptr.size() - 1;

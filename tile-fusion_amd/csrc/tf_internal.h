@@ -183,7 +183,6 @@ struct tf_schedule {
   int hot_cols = 0;               // intermediate rows in the 8 partitions together
   std::vector<int> seg_ptr;       // [n_seg + 1] into seg_src/seg_col: partition 0's segments, 1's, ..., 7's, the cold ones
   std::vector<int> seg_src;       // per regrouped entry: its index in A's arrays
-  std::vector<int> ent_src, ent_pos;  // the same pairs (index in A's arrays, regrouped position) sorted by the former
   std::vector<int> seg_col;       // per regrouped entry: its column
   std::vector<int> lrow_seg;      // per long row (first, count of tf::LongRow): the partial-sum slots it adds up, in order:
                                   // segments, or for a row of more than 32 segments groups of up to 32 of them

@@ -475,17 +475,18 @@ __global__ __launch_bounds__(kW64Block) void fused_spmm_spmm_window64_kernel(
   }
 }
 
-// out[i] = val[src[i]]: the values of the rows of a list, in the order of the list.
+// out[i] = val[src[i]]: a matrix' values in the order of a schedule's lists.  Four entries a thread, their gathers in flight together
+// (src and out start at multiples of 16 bytes).
 __global__ void gather_values_kernel(const int *__restrict__ src, const float *__restrict__ val, float *__restrict__ out, int n) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = val[src[i]];
-}
-
-// Column-partitioned long rows: out[pos[i]] = val[src[i]] puts the values of A into the order of
-// the regrouped entries (src ascending: the reads walk A's array once, the writes fall into
-// nine ascending streams).
-__global__ void scatter_values_kernel(const int *__restrict__ src, const int *__restrict__ pos,
-                                      const float *__restrict__ val, float *__restrict__ out, int n) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[pos[i]] = val[src[i]];
+  for (unsigned i = 4 * (blockIdx.x * blockDim.x + threadIdx.x); i < (unsigned)n; i += 4 * gridDim.x * blockDim.x) {
+    if (i + 4 <= (unsigned)n) {
+      const int4 s = *reinterpret_cast<const int4 *>(src + i);
+      const float4 v = {val[s.x], val[s.y], val[s.z], val[s.w]};
+      *reinterpret_cast<float4 *>(out + i) = v;
+    } else {
+      for (unsigned k = i; k < (unsigned)n; ++k) out[k] = val[src[k]];
+    }
+  }
 }
 
 // dst (rows x ld_dst) = src (src_rows x ld_src) in its top left corner, zeros elsewhere.
@@ -1868,20 +1869,9 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *tiles, const int *win
   return err != hipSuccess ? err : hipGetLastError();
 }
 
-// Long rows regrouped by column partition.  The executor runs the hot segments (an eighth per
-// XCD, in XCD order) on the row kernel with one contiguous run of segments per XCD and the cold
-// ones round-robin; this puts A's values into segment order.
-hipError_t launch_scatter_values(const int *ent_src, const int *ent_pos, const float *Ax, float *seg_val, int n_entries,
-                                 hipStream_t st) {
-  if (n_entries <= 0) return hipSuccess;
-  const int blocks = std::min((n_entries + kBlock - 1) / kBlock, 65536);
-  hipLaunchKernelGGL(scatter_values_kernel, dim3(blocks), dim3(kBlock), 0, st, ent_src, ent_pos, Ax, seg_val, n_entries);
-  return hipGetLastError();
-}
-
 hipError_t launch_gather_values(const int *src, const float *Ax, float *out, int n, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  const int blocks = std::min((n + kBlock - 1) / kBlock, 65536);
+  const int blocks = std::min((n / 4 + kBlock) / kBlock, 65536);
   hipLaunchKernelGGL(gather_values_kernel, dim3(blocks), dim3(kBlock), 0, st, src, Ax, out, n);
   return hipGetLastError();
 }
