@@ -55,7 +55,7 @@ class Dense {
 };
 
 // Everything that is built once per adjacency matrix: the host copy of its pattern (the inspector runs on the host), the device CSR,
-// schedules per product and widths, its transpose.  `mutex` orders the calls that share the schedules' workspaces.
+// schedules per product and widths, its transpose.  Calls that share the schedules' workspaces take turns (Turn).
 struct Adjacency : torch::CustomClassHolder {
   std::vector<Tensor> keep;  // a wrapped matrix' arrays stay alive with it
   std::vector<int> Ap, Ai;
