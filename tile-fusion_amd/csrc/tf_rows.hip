@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
 // read once per 64 rows and seven workgroups share a compute unit, one gathering while another multiplies.  See
 // one_launch in tf_api.cpp for where this is the faster way.
 // ---------------------------------------------------------------------------------
-template <int LPR, int R, int V, bool WT>
+template <int LPR, int R, int V, bool WT, bool IN_PLACE>
 __global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(const RowsArgs a, const float *__restrict__ W, int N, const GemmOut how) {
   extern __shared__ __align__(16) float slab[];
   constexpr int G = kBlock / LPR, RT = R / 16, CW = 4 / RT;  // lane groups; row tiles; wavefronts side by side in columns
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kBlock, R == 16 ? 1 : 7) void spmm_gemm_kernel(cons
       const int row = a.rows && !a.compact ? a.rows[q] : q;
       kb = a.Ap[row];
       ke = a.Ap[row + 1];
-      if (a.val_first) ax += a.val_first[q] - kb;
+      if constexpr (IN_PLACE) ax += a.val_first[q] - kb;
     }
     for (int c0 = 0; c0 < K; c0 += LPR * 4) {
       const int col = c0 + glane * 4, coff = clamp_col<4>(col, K);
@@ -565,12 +565,13 @@ hipError_t launch_spmm_gemm(RowsArgs a, const RowsHow &rows, const float *W, int
   a.n_blocks = (a.n_rows + R - 1) / R;
   const dim3 grid(deal_to_xcds(a, rows.xcd_chunk_rows, R));
   hipError_t err = hipSuccess;
-#define CALL3(L_, R_, V_, WT_)                                                                                                         \
+#define CALL4(L_, R_, V_, WT_, IN_)                                                                                                    \
   do {                                                                                                                                 \
     if (lds > 65536)                                                                                                                   \
-      err = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_gemm_kernel<L_, R_, V_, WT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
-    if (err == hipSuccess) hipLaunchKernelGGL((spmm_gemm_kernel<L_, R_, V_, WT_>), grid, dim3(kBlock), lds, st, a, W, N, how);         \
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(spmm_gemm_kernel<L_, R_, V_, WT_, IN_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+    if (err == hipSuccess) hipLaunchKernelGGL((spmm_gemm_kernel<L_, R_, V_, WT_, IN_>), grid, dim3(kBlock), lds, st, a, W, N, how);    \
   } while (0)
+#define CALL3(L_, R_, V_, WT_) do { if (a.val_first) { CALL4(L_, R_, V_, WT_, true); } else { CALL4(L_, R_, V_, WT_, false); } } while (0)
 #define CALL2(L_, R_, V_) do { if (wt) { CALL3(L_, R_, V_, true); } else { CALL3(L_, R_, V_, false); } } while (0)
 #define CALL(V__, L_)                                                                                                   \
   do {                                                                                                                  \
@@ -582,6 +583,7 @@ hipError_t launch_spmm_gemm(RowsArgs a, const RowsHow &rows, const float *W, int
 #undef CALL
 #undef CALL2
 #undef CALL3
+#undef CALL4
   return err != hipSuccess ? err : hipGetLastError();
 }
 
