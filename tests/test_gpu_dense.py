@@ -61,6 +61,40 @@ def test_gemm_panel_edges(gpu, tf, M, K, N):
             assert np.array_equal(np.isinf(got[~ok]), np.isinf(ref[~ok]))
 
 
+@pytest.mark.parametrize("M,K,N", [(20480, 4, 65), (20479, 4, 65), (20481, 31, 66), (24001, 33, 65), (24000, 51, 96), (20495, 64, 97), (50000, 65, 128),
+                                   (30001, 128, 128), (20485, 161, 72), (21000, 213, 128), (21001, 214, 129), (20500, 300, 100), (20483, 426, 65),
+                                   (20482, 427, 65), (49152, 64, 33), (49151, 64, 33), (49161, 96, 48), (49999, 130, 64), (50003, 427, 40),
+                                   (49153, 853, 36), (49154, 854, 36), (262145, 67, 35)])
+@pytest.mark.parametrize("w_t", [False, True])
+def test_gemm_on_bf16_cores(gpu, tf, M, K, N, w_t):
+    """Products as sums of bf16 parts, either side of where they begin and of what LDS holds: no further from float64 than fp32 sums, for
+    operands of one size and of many sizes; infinities, NaN and values that bf16 rounds to infinity stay in their rows, and come out
+    as fp32 arithmetic has them."""
+    say(f"gemm on bf16 cores {M} x {K} x {N} w_t={w_t}")
+    rng = np.random.default_rng(M + 3 * K + 5 * N)
+    W = rng.uniform(-0.2, 0.2, (K, N)).astype(np.float32)
+    Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if w_t else W)
+    flags = C_TRANSPOSED if w_t else 0
+    big = np.float32(3.4e38)  # rounds to infinity in bf16
+    for spread in (0.0, 20.0):
+        X = (rng.uniform(-1, 1, (M, K)) * np.exp2(rng.uniform(-spread, spread, (M, K)))).astype(np.float32)
+        X[1, K - 1], X[M - 1, 0], X[M // 2, 0], X[M - 2, K // 2] = np.inf, np.nan, big, -np.inf
+        odd = np.zeros(M, bool)
+        odd[[1, M - 1, M // 2, M - 2]] = True
+        Xd, Y = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(np.full((M, N), 7.0, np.float32))
+        assert tf.lib().tf_gemm_ex(Xd.h, Wd.h, Y.h, None, flags, None) == 0
+        tf.device_synchronize()
+        got = Y.to_numpy()
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = X.astype(np.float64) @ W.astype(np.float64)
+            size = np.abs(X[~odd]).astype(np.float64) @ np.abs(W).astype(np.float64)
+        # K roundings of partial sums, each below the sum of magnitudes
+        assert np.all(np.abs(got[~odd] - want[~odd]) <= (K + 8) * 2.0 ** -24 * size)
+        assert np.array_equal(np.isnan(got[odd]), np.isnan(want[odd]))
+        assert np.array_equal(np.sign(got[[1, M - 2]]), np.sign(want[[1, M - 2]])) and np.all(np.isinf(got[[1, M - 2]]))
+        assert np.all(np.abs(got[M // 2] - want[M // 2]) <= (K + 8) * 2.0 ** -24 * np.abs(want[M // 2]).max())
+
+
 @pytest.mark.parametrize("K,N", [(129, 33), (64, 100), (18, 128)])
 def test_gemm_of_listed_rows(gpu, tf, K, N):
     """The rows an R-MAT graph reads, gathered by the product itself and stored in the order of their reads."""

@@ -109,7 +109,6 @@ hipError_t launch_fused_gemm_spmm(const TileDesc *, int, const int *, const floa
 hipError_t launch_fused_gemm_spmm_stream(const TileDesc *, int, const int *, const int *, const int *,
                                          const float *, const float *, int, int, int, const int *,
                                          const float *, float *, float *, int, int, hipStream_t, int relu_in = 0);
-hipError_t launch_gemm(const float *, const float *, float *, const int *, int, int, int, int, hipStream_t, int y_by_position = 0);
 hipError_t launch_fill(float *, size_t, float, hipStream_t);
 hipError_t launch_pad(const float *, int, int, float *, int, int, hipStream_t);
 hipError_t launch_transpose_pad(const float *, int, int, int, int, float *, int, int, hipStream_t);
@@ -906,14 +905,6 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
   return tf::run_remainder(A, s, tf::Remainder{d->inter, s->opts.N, s->opts.N, s->M, D->d, acc, 0}, false, st);
 }
 
-// W as the row GEMM takes it: row-major K x N with N a multiple of 32 up to 256, K of 8, small enough for LDS.  Its 32-row
-// blocks on two wavefronts per SIMD are the faster kernel from 1,024 rows per compute unit on, the other one balances fewer better (us,
-// 64 x 128 / 128 x 64 / 128 x 128, this one and launch_gemm_any: 100,000 rows 34 25 52 and 26 24 42, 131,072 rows 30 26 46 and 28 26 44, 262,144 rows
-// 52 46 82 and 55 50 82).
-static bool row_gemm_takes(long long rows, int K, int N, int compute_units) {
-  return rows >= 1024LL * compute_units && K % 8 == 0 && N % 32 == 0 && N <= 256 && (long long)K * N * 4 <= 131072;
-}
-
 // What a GeMM-SpMM pass reads and writes: B (M x K), C (K x N, or N x K with c_t) and D (L x N).
 struct GemmPass {
   const float *B, *C;
@@ -949,15 +940,15 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
     const int n_plain = (int)s->plain_rows.size();
     const int placed = s->t_pos.empty() ? 0 : 1;  // the intermediate's rows stored in the order of the list
     const bool all = n_plain == s->M && s->plain_hot == 0 && !placed;
-    const bool row_gemm = !g.c_t && ldt == g.N && row_gemm_takes(n_plain, g.K, g.N, s->opts.compute_units);
     auto gemm = [&](int first, int count) {
       const int *rows = all ? nullptr : d->plain_rows + first;
       float *Y = d->inter + (placed ? (size_t)first * ldt : 0);
-      return row_gemm ? tf::launch_gemm(g.B, g.C, Y, rows, count, g.K, g.N, s->opts.compute_units, st, placed)
-                      : tf::launch_gemm_any(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, tf::GemmOut(), s->opts.compute_units, st);
+      tf::GemmOut how;
+      how.of_rows = n_plain;
+      return tf::launch_gemm_any(g.B, g.K, g.C, g.c_t, Y, ldt, rows, !placed, count, g.K, g.N, how, s->opts.compute_units, st);
     };
     if (overlap) {
-      TF_PHASE(s, "gemm_rows_kernel (hot rows)", st, gemm(0, s->plain_hot));
+      TF_PHASE(s, "dense product (hot rows)", st, gemm(0, s->plain_hot));
       // the regrouped values (of the hot and of the cold segments) before the fork: the cold segments run on
       // this stream and are not ordered after anything the side stream does until the join
       if (tf_status rc2 = tf::ensure_segment_values(A, s, st)) return rc2;
@@ -965,9 +956,9 @@ static tf_status gemm_spmm_pass(const tf_csr *A, tf_schedule *s, const GemmPass 
       TF_HIP(hipStreamWaitEvent(d->side, d->fork, 0));
       if (tf_status rc2 = tf::run_hot_segments(s, rem, d->side)) return rc2;
       TF_HIP(hipEventRecord(d->join, d->side));
-      if (n_plain > s->plain_hot) TF_PHASE(s, "gemm_rows_kernel (other rows)", st, gemm(s->plain_hot, n_plain - s->plain_hot));
+      if (n_plain > s->plain_hot) TF_PHASE(s, "dense product (other rows)", st, gemm(s->plain_hot, n_plain - s->plain_hot));
     } else {
-      TF_PHASE(s, row_gemm ? "gemm_rows_kernel" : "gemm_panel_kernel", st, gemm(0, n_plain));
+      TF_PHASE(s, "dense product", st, gemm(0, n_plain));
     }
   }
   return tf::run_remainder(A, s, rem, overlap && !s->plain_rows.empty(), st);
@@ -1017,17 +1008,11 @@ static tf_status gemm_spmm_impl(const tf_csr *A, const tf_dense *B, const tf_den
       }
       rc = tf::run_remainder(A, rows, tf::Remainder{B->d, K, K, B->M, d->inter, 0, 0, tf::inter_streams(s)}, false, st);
       if (rc) return rc;
-      if (!c_t && !acc && !relu && row_gemm_takes(s->L, K, N, cus))
-        TF_PHASE(rows, "gemm_rows_kernel", st, tf::launch_gemm(d->inter, C->d, D->d, nullptr, s->L, K, N, cus, st, 0));
-      else
-        TF_PHASE(rows, "gemm_panel_kernel", st, tf::launch_gemm_any(d->inter, K, C->d, c_t, D->d, N, nullptr, 0, s->L, K, N, how, cus, st));
+      TF_PHASE(rows, "dense product", st, tf::launch_gemm_any(d->inter, K, C->d, c_t, D->d, N, nullptr, 0, s->L, K, N, how, cus, st));
       return TF_OK;
     }
     const int ldt = tf::inter_ld(s);
-    if (!c_t && ldt == N && row_gemm_takes(s->M, K, N, cus))
-      TF_PHASE(rows, "gemm_rows_kernel", st, tf::launch_gemm(B->d, C->d, d->inter, nullptr, s->M, K, N, cus, st, 0));
-    else
-      TF_PHASE(rows, "gemm_panel_kernel", st, tf::launch_gemm_any(B->d, K, C->d, c_t, d->inter, ldt, nullptr, 0, s->M, K, N, tf::GemmOut(), cus, st));
+    TF_PHASE(rows, "dense product", st, tf::launch_gemm_any(B->d, K, C->d, c_t, d->inter, ldt, nullptr, 0, s->M, K, N, tf::GemmOut(), cus, st));
     return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, relu}, false, st);
   }
   if (tf::untiled(s)) return gemm_spmm_pass(A, s, GemmPass{B->d, C->d, c_t, s->user_K, s->user_N, D->d, acc, 0, relu}, flags, st);
@@ -1230,13 +1215,9 @@ extern "C" tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *
     return fail(TF_EINVAL, "tf_gemm: shapes X %d x %d, W %d x %d%s, Y %d x %d", X->M, X->N, W->M, W->N, w_t ? " (transposed)" : "", Y->M, Y->N);
   if (mask && (mask->M != M || mask->N != N)) return fail(TF_EINVAL, "tf_gemm: mask is %d x %d, Y is %d x %d", mask->M, mask->N, M, N);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (!w_t && !mask && row_gemm_takes(M, K, N, tf::default_compute_units()))
-    TF_HIP(tf::launch_gemm(X->d, W->d, Y->d, nullptr, M, K, N, tf::default_compute_units(), st, 0));
-  else {
-    tf::GemmOut how;
-    how.mask = mask ? mask->d : nullptr;
-    TF_HIP(tf::launch_gemm_any(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, how, tf::default_compute_units(), st));
-  }
+  tf::GemmOut how;
+  how.mask = mask ? mask->d : nullptr;
+  TF_HIP(tf::launch_gemm_any(X->d, K, W->d, w_t ? 1 : 0, Y->d, N, nullptr, 0, M, K, N, how, tf::default_compute_units(), st));
   return TF_OK;
 }
 

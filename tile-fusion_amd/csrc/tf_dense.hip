@@ -291,35 +291,273 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
   }
 }
 
+// ---------------------------------------------------------------------------------
+// The same on the bf16 matrix cores (split8 in tf_device.h), for W whose three bf16 parts fit LDS: a step is 32 values of k, W's parts lie
+// in LDS as the matrix cores take them (a lane's eight values of a column in one 16-byte read), X's are made in registers on
+// the way.  Bound: X and Y from HBM behind some 8 us until the first product (262,144 x 128 x 128 63 us, 4.3 TB/s; gemm_panel_kernel 81, waiting for
+// the fp32 cores), and the board's power: the same on operands that are all the same number runs at 5.2 TB/s.  Where W takes two panels the parts
+// of X are made twice: 200,000 x 256 x 128 99 us, 60 at the rate of a copy.
+// ---------------------------------------------------------------------------------
+// Eight wavefronts per compute unit: more of them in flight read memory more slowly (100,000 x 300 x 64: 41.5 us, twelve 41.8, six 42.3).
+constexpr int kSplitWaves = 8;
+constexpr long long split_lds(int K, int columns) { return ((long long)K + 31) / 32 * columns * 192; }
+
+template <int V, int Q, bool WT, int OUT, int A>
+__global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
+                                                                   float *__restrict__ Y, int ldy, const int *__restrict__ rows,
+                                                                   int y_by_row, int n_rows, int K, int N,
+                                                                   const GemmOut out_how) {
+  extern __shared__ __align__(16) bf8 wparts[];  // [step][tile][part][lane]
+  constexpr int P = 16 * V * Q, T = V * Q;
+  const int waves = blockDim.x / 64, wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
+  const int panel0 = blockIdx.y * P, S = (K + 31) / 32, G = (S + A - 1) / A;
+  // Blocks in turn over the workgroups, so that what is being read is one stretch of memory and not a place per wavefront (reads alone,
+  // 131,072 rows of 1 KB that no cache holds: 34.5 against 38.9 us).
+  const int n_blocks = (n_rows + 15) / 16, stride = gridDim.x * waves, b0 = wave * gridDim.x + blockIdx.x;
+  auto column = [&](int n) { return OUT == kAnyOut ? min(panel0 + n, N - 1) : min(panel0 + n - n % V, N - V) + n % V; };  // of W
+  f4v x[A][2];  // a lane's eight values of the next A steps
+  auto row_index = [&](int b) __attribute__((always_inline)) {
+    const int q = min(b * 16 + j, n_rows - 1);
+    if constexpr (OUT == kPlain || OUT == kMasked) return q;
+    else if constexpr (OUT == kListed) return rows[q];
+    else return rows ? rows[q] : q;
+  };
+  auto load = [&](const float *xp, int s, f4v (&o)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w) o[w] = *reinterpret_cast<const f4u *>(xp + min(32 * s + 8 * h + 4 * w, K - 4));
+  };
+  // W's parts into LDS: a column's eight values of k per item, U items' loads on their way at a time, the first of them in front of
+  // the first rows of X (loads return in order, and all workgroups' first rows are a burst of 16 MB).
+  constexpr int U = 8;
+  const int items = S * T * 64;
+  f4v v[U][2];
+  auto load_items = [&](int it0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = it0 + u * (int)blockDim.x;
+      if (it >= items) break;  // (whole wavefronts: the items are a multiple of 64)
+      const int jj = it % 16, hh = it / 16 % 4, t = it / 64 % T, s = it / (64 * T), k0 = 32 * s + 8 * hh;
+      const int c = column(16 * V * (t / V) + V * jj + t % V);
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const int kk = k0 + 4 * w;
+        if (kk + 4 <= K) {
+          if constexpr (WT) v[u][w] = *reinterpret_cast<const f4u *>(W + (size_t)c * K + kk);
+          else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[u][w][i] = W[(size_t)(kk + i) * N + c];
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[u][w][i] = kk + i < K ? W[WT ? (size_t)c * K + kk + i : (size_t)(kk + i) * N + c] : 0.f;
+        }
+      }
+    }
+  };
+  auto put_items = [&](int it0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = it0 + u * (int)blockDim.x;
+      if (it >= items) break;
+      const split4 p = split8(v[u][0], v[u][1]);
+      bf8 *at = wparts + (size_t)(it / 64) * 192 + it % 64;
+      at[0] = p.h;
+      at[64] = p.m;
+      at[128] = p.l;
+    }
+  };
+  load_items(threadIdx.x);
+  const float *xp = X;
+  int next_row = 0;  // of this lane in the block after the next one to begin
+  if (b0 < n_blocks) {
+    xp = X + (size_t)row_index(b0) * ldx;
+    next_row = row_index(b0 + stride);
+#pragma unroll
+    for (int u = 0; u < A; ++u) load(xp, u, x[u]);
+  }
+  put_items(threadIdx.x);
+  for (int it0 = threadIdx.x + U * blockDim.x; it0 < items; it0 += U * blockDim.x) {
+    load_items(it0);
+    put_items(it0);
+  }
+  __syncthreads();
+  acc4 big[T], small[T];
+  const bf8 *wl = wparts + lane;
+  auto multiply = [&](int s, const split4 &a) __attribute__((always_inline)) {
+    const bf8 *w = wl + (size_t)s * (T * 192);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const bf8 wh = w[t * 192], wm = w[t * 192 + 64], wlo = w[t * 192 + 128];
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, wh, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wlo, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.u, wm, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, wh, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wm, small[t], 0, 0, 0);
+      big[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wh, big[t], 0, 0, 0);
+    }
+  };
+  // Where K is no multiple of four, one lane group's last values lie d places behind those that were loaded.  (W's parts are zero where k
+  // is past K.)
+  int d[2];
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const int at = 32 * (S - 1) + 8 * h + 4 * w;
+    d[w] = at < K ? at - min(at, K - 4) : 0;
+  }
+  // A step: its values become parts, whereupon their registers take the values A steps on, of this block or the next.
+  auto step = [&](int s, f4v (&o)[2], const float *from, int ahead) __attribute__((always_inline)) {
+    if (s == S - 1 && K % 4 != 0) {
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        o[w] = d[w] & 1 ? f4v{o[w][1], o[w][2], o[w][3], 0.f} : o[w];
+        o[w] = d[w] & 2 ? f4v{o[w][2], o[w][3], 0.f, 0.f} : o[w];
+      }
+    }
+    const split4 a = split8(o[0], o[1]);
+    load(from, ahead, o);
+    __builtin_amdgcn_sched_barrier(0);  // (the requests stay in front of the products)
+    if (s < S) multiply(s, a);
+  };
+  for (int b = b0; b < n_blocks; b += stride) {
+    const float *xn = X + (size_t)next_row * ldx;
+    next_row = row_index(b + 2 * stride);
+    int y_row[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int x = min(b * 16 + 4 * h + r, n_rows - 1);
+      if constexpr (OUT == kListed) y_row[r] = rows[x]; else y_row[r] = x;
+      if (OUT == kListed && !y_by_row) y_row[r] = x;
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      big[t] = 0.f;
+      small[t] = 0.f;
+    }
+    for (int g = 0; g < G; ++g) {
+      const bool more = g + 1 < G;
+#pragma unroll
+      for (int u = 0; u < A; ++u) step(g * A + u, x[u], more ? xp : xn, more ? (g + 1) * A + u : u);
+    }
+    float finite = 0.f;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        big[t][r] += small[t][r] * (1.f / kSplitScale);
+        finite = __builtin_fmaf(big[t][r], 0.f, finite);
+      }
+    if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for bf16
+#pragma unroll
+      for (int t = 0; t < T; ++t) big[t] = 0.f;
+#pragma unroll 1
+      for (int k0 = 0; k0 < K; k0 += 4) {
+        const int k = min(k0 + h, K - 1);
+        const float xv = k0 + h < K ? xp[k] : 0.f;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const int c = column(16 * V * (t / V) + V * j + t % V);
+          const float w = k0 + h < K ? W[WT ? (size_t)c * K + k : (size_t)k * N + c] : 0.f;
+          big[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, w, big[t], 0, 0, 0);
+        }
+      }
+    }
+    xp = xn;
+    if constexpr (OUT == kAnyOut) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int x = b * 16 + 4 * h + r;
+        if (x >= n_rows) continue;
+        const size_t row = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const int c = panel0 + 16 * V * q + V * j;
+          cvec<V> out;
+#pragma unroll
+          for (int v = 0; v < V; ++v) out.v[v] = big[q * V + v][r];
+          gemm_store<V>(Y, row + c, out, N - c, out_how);
+        }
+      }
+    } else {
+      size_t at[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) at[r] = (size_t)y_row[r] * ldy;
+      cvec<V> m[4][Q];
+      if constexpr (OUT == kMasked) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) m[r][q] = *reinterpret_cast<const cvec<V> *>(out_how.mask + at[r] + min(panel0 + 16 * V * q + V * j, N - V));
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          cvec<V> out;
+#pragma unroll
+          for (int v = 0; v < V; ++v) out.v[v] = OUT == kMasked && m[r][q].v[v] <= 0.f ? 0.f : big[q * V + v][r];
+          *reinterpret_cast<cvec<V> *>(Y + at[r] + min(panel0 + 16 * V * q + V * j, N - V)) = out;
+        }
+    }
+  }
+}
+
 // X: n_rows x K, row stride ldx (or the rows of X that `rows` lists); Y: row q of it at q * ldy, or at rows[q] * ldy when
 // y_by_row is set.  wt: W is N x K.
 hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, float *Y, int ldy, const int *rows, int y_by_row,
                            int n_rows, int K, int N, const GemmOut &how, int compute_units, hipStream_t st) {
   if (n_rows <= 0) return hipSuccess;
-  // Which kernel (us, this one / one 16-row tile per wavefront, at 8,000 / 16,000 / 30,000 rows): copying W to LDS
-  // takes some 4 us before the first product, the other kernel reads it from L2 for every row tile, by single values where W is
-  // K x N.  128 x 128 9.3 / 8.1 (K x N: 9.3 / 11.6), 11.0 / 13.8, 16.8 / 23; 64 x 64 5.0 / 4.6 (5.0 / 5.7), 5.0 / 6.0, 6.7 / 9.0; 500 x 32, 30,000 rows
-  // 17.6 / 20.8; 40 x 7 6.7 / 4.2.  Widths are cut into panels that fit LDS (X is read once per panel).
-  const long long lds_k = (long long)(K + 15) / 16 * 16 * 4;  // bytes per column
-  int unit = N <= 16 ? 16 : N <= 32 ? 32 : N <= 64 ? 64 : N <= 96 ? 96 : 128;
-  if (N > 128) {  // equal panels
-    const int n_panels = (N + 127) / 128, w = (N + n_panels - 1) / n_panels;
-    unit = w <= 96 ? 96 : 128;
-  }
-  while (unit > 16 && lds_k * unit > 163840) unit = unit == 96 ? 64 : unit / 2;
+  // Which kernel.  Copying W to LDS takes some 4 us before the first product; gemm_direct_kernel reads it from L2 for every row tile, by
+  // single values where W is K x N (us, gemm_panel_kernel / gemm_direct_kernel, at 8,000 / 16,000 / 30,000 rows: 128 x 128 9.3 / 8.1 (K x N: 9.3 / 11.6),
+  // 11.0 / 13.8, 16.8 / 23; 64 x 64 5.0 / 4.6 (5.0 / 5.7), 5.0 / 6.0, 6.7 / 9.0; 500 x 32, 30,000 rows 17.6 / 20.8; 40 x 7 6.7 / 4.2).
+  // The bf16 cores pay where the fp32 ones were what a product waited for: beyond 64 columns from 80 rows per compute unit on, where splitting W no
+  // longer counts, for 33 to 64 columns where there are more rows and K is not small (us, operands in no cache, gemm_panel_kernel /
+  // gemm_split_kernel with W N x K: 12,500 rows 300 x 64 10.5 / 12.9; 24,000 rows 64 x 128 11.9 / 10.1, 128 x 128 17.2 / 14.4, 128 x 64 10.0 / 10.1,
+  // 300 x 128 32.2 / 23.1; 50,000 rows 128 x 64 15.4 / 15.1, 32 x 64 8.6 / 8.3; 100,000 rows 32 x 64 12.0 / 12.4, 64 x 64 16.4 / 15.2, 128 x 64 25.0 / 20.5,
+  // 300 x 64 51.4 / 41.4, 128 x 128 43.6 / 30.3, 300 x 128 88.3 / 67.1; 262,144 rows 128 x 40 47.2 / 38.0, 128 x 128 81 / 63; 200,000 rows
+  // 256 x 128 119 / 99, two panels; 60,000 rows 300 x 300 172 / 93, five; but 150,000 rows 512 x 128 173 / 194, four panels of 32).
+  // Widths are cut into equal panels that fit LDS; X is read once per panel, by compute units of the same XCD at about the same time.
+  const int all_rows = std::max(n_rows, how.of_rows);
+  const bool on_bf16 = (N > 64 ? all_rows >= 80LL * compute_units : N > 32 && K >= 64 && all_rows >= 192LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
+  const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
+  const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
+  int unit = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;
+  auto lds_of = [&](int columns) { return on_bf16 ? split_lds(K, columns) : ((long long)K + 15) / 16 * 16 * 4 * columns; };
+  while (unit > 16 && lds_of(unit) > kMaxLds) unit = unit == 96 ? 64 : unit / 2;
   const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 80LL * compute_units : (wt ? 48LL : 24LL) * compute_units;
-  if (n_rows >= from && lds_k * unit <= 163840 && K >= 4) {
-    const int panels = (N + unit - 1) / unit, lds = (int)(lds_k * unit), n_blocks = (n_rows + 15) / 16;
-    const int waves = n_blocks >= 16 * compute_units ? 16 : n_blocks >= 8 * compute_units ? 8 : 4;
-    const dim3 grid(std::max(1, std::min(compute_units / std::min(panels, 2), (n_blocks + waves - 1) / waves)), panels);
+  if (all_rows >= from && lds_of(unit) <= kMaxLds && K >= 4) {
+    const int panels = (N + unit - 1) / unit, lds = (int)lds_of(unit), n_blocks = (n_rows + 15) / 16;
+    // workgroups per panel: a multiple of 8, so that a row block's panels are on one XCD
+    const int across = on_bf16 ? std::max(8, compute_units / panels / 8 * 8) : compute_units / std::min(panels, 2);
+    int waves = n_blocks >= 16 * compute_units ? 16 : n_blocks >= 8 * compute_units ? 8 : 4;
+    // steps of k in flight: the number that goes into K's without a rest, or nearly (131,072 x 300 x 64: 45 us with five, 52 with four)
+    int ahead = 2;
+    if (on_bf16) {
+      waves = std::max(4, std::min(kSplitWaves, (n_blocks + across - 1) / across));
+      const int steps = (K + 31) / 32;
+      for (int n : {3, 4, 5})
+        if ((steps + n - 1) / n * n <= (steps + ahead - 1) / ahead * ahead && steps > ahead) ahead = n;
+    }
+    const dim3 grid(std::max(1, std::min(across, (n_blocks + waves - 1) / waves)), panels);
     hipError_t err = hipSuccess;
     const int out = how.accumulate || how.relu || N < 4 || (rows && how.mask) ? kAnyOut : rows ? kListed : how.mask ? kMasked : kPlain;
-#define CALLP3(V_, Q_, WT_, OUT_)                                                                                              \
+#define CALLP4(...)                                                                                                            \
   do {                                                                                                                         \
     if (lds > 65536)                                                                                                           \
-      err = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_panel_kernel<V_, Q_, WT_, OUT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(__VA_ARGS__), hipFuncAttributeMaxDynamicSharedMemorySize, lds);  \
     if (err == hipSuccess)                                                                                                     \
-      hipLaunchKernelGGL((gemm_panel_kernel<V_, Q_, WT_, OUT_>), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how); \
+      hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(64 * waves), lds, st, X, ldx, W, Y, ldy, rows, y_by_row, n_rows, K, N, how); \
+  } while (0)
+#define CALLP3(V_, Q_, WT_, OUT_)                                                                                              \
+  do {                                                                                                                         \
+    if (!on_bf16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_>); }                                                            \
+    else if constexpr (V_ * Q_ >= 2) {                                                                                         \
+      if (V_ * Q_ == 2 || ahead == 4) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 4>); }                                     \
+      else if constexpr (V_ * Q_ > 2) {                                                                                        \
+        if (ahead == 5) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 5>); }                                                   \
+        else if (ahead == 3) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 3>); }                                              \
+        else { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 2>); }                                                              \
+      }                                                                                                                        \
+    }                                                                                                                          \
   } while (0)
 #define CALLP2(V_, Q_, WT_)                                                                                                    \
   do { if (out == kPlain) { CALLP3(V_, Q_, WT_, kPlain); } else if (out == kMasked) { CALLP3(V_, Q_, WT_, kMasked); } else if (out == kListed) { CALLP3(V_, Q_, WT_, kListed); } else { CALLP3(V_, Q_, WT_, kAnyOut); } } while (0)
@@ -334,6 +572,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 #undef CALLP
 #undef CALLP2
 #undef CALLP3
+#undef CALLP4
     return err != hipSuccess ? err : hipGetLastError();
   }
   // Column blocks per wavefront: as many as the width has (up to four: X is then read once per 64 columns), fewer

@@ -88,6 +88,7 @@ struct GemmOut {
   const float *mask = nullptr;  // of Y's shape: 0 where it is zero or less (the derivative of a ReLU whose output it is)
   int accumulate = 0;           // Y += the product
   int relu = 0;
+  int of_rows = 0;              // rows of the whole product where it comes in parts: all are computed by the same kernel (0: its own)
 };
 
 // How launch_weight_grad cuts Y = G^T X (tf_dense.hip).

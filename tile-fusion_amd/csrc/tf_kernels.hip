@@ -669,259 +669,7 @@ __global__ __launch_bounds__(kBlock) void fused_gemm_spmm_kernel(
   }
 }
 
-// Row-list GEMM  Y[r,:] = X[r,:K] * W  for r = rows[q] (or r = q when rows is null):
-// intermediate rows that no tile fuses, and tf_gemm, for many rows (row_gemm_takes in tf_api.cpp).  Persistent: W (K x N) is copied to
-// LDS once per workgroup, then every wavefront walks its own 32-row blocks with no
-// barrier at all; the rows of X for the next 32 values of k are already in flight
-// (16 bytes per lane and load, see tile_gemm for the k permutation) while the MFMAs of
-// the current ones issue.
 constexpr int kGemmBlock = 512;
-
-template <int NB> struct alignas((NB == 1 || NB == 2 || NB == 4) ? 4 * NB : (NB == 8 ? 16 : 4)) wvec { float v[NB]; };
-
-// Column block nb of a wavefront's 32 x (32 NB) output tile holds the columns NB j + nb, j = 0 .. 31 (not
-// 32 nb + j): W then sits in LDS as it is in memory, row-major, the NB values a lane feeds to the NB MFMAs of
-// one k step are adjacent (one LDS read of 4 NB bytes per k step), and a lane ends up with NB consecutive
-// columns of each of its output rows, which leave with one store (16 bytes when NB = 4; a row of the tile
-// is 32 such stores side by side).  The reads for the next eight values of k are issued before the MFMAs
-// of the current eight.
-template <int NB>
-__device__ __forceinline__ void mfma_step8(const fvec<4> &a, const wvec<NB> (&bw)[4], v16f (&acc)[NB]) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-      acc[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[t], bw[t].v[nb], acc[nb], 0, 0, 0);
-}
-
-// Copies W (K x N, row-major) into LDS as it is: 16 bytes per load, eight loads in flight per thread.
-template <int NB>
-__device__ __forceinline__ void stage_weights(const float *__restrict__ W, int K, float *wlds) {
-  constexpr int N = NB * 32;
-  const int n4 = K * N / 4;
-  const fvec<4> *src = reinterpret_cast<const fvec<4> *>(W);
-  fvec<4> *dst = reinterpret_cast<fvec<4> *>(wlds);
-  for (int i0 = threadIdx.x; i0 < n4; i0 += 8 * kGemmBlock) {
-    fvec<4> v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + u * kGemmBlock;
-      v[u] = src[i < n4 ? i : i0];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + u * kGemmBlock;
-      if (i < n4) dst[i] = v[u];
-    }
-  }
-}
-
-constexpr int kGemmSeg = 16;  // row blocks whose row numbers a wavefront keeps in LDS at a time
-
-// G4C > 0: K = 32 G4C is known when the kernel is built, and a block's MFMAs, the requests for the operands
-// three groups ahead and the reads of W one step ahead are one stretch of code without a branch: a wavefront
-// issues in order, so address arithmetic, a wait for a row number or a branch between two MFMAs leaves the
-// pipe without work from this wavefront (39,000 -> 33,500 cycles per block and wavefront for K = 128, of
-// which the block's 256 MFMAs of the two wavefronts of a SIMD take 32,800).
-// YPOS (row lists only): the result of list position q goes to row q of Y instead of row rows[q] -- the rows of the
-// result stored side by side in the order of the list.
-template <int NB, bool LIST, int G4C, bool YPOS = false>
-__global__ __launch_bounds__(kGemmBlock) void gemm_rows_kernel(const float *__restrict__ X,
-                                                               const float *__restrict__ W,
-                                                               float *__restrict__ Y,
-                                                               const int *__restrict__ rows, int n_rows,
-                                                               int K) {
-  extern __shared__ __align__(16) float wlds[];
-  constexpr int N = NB * 32;
-  stage_weights<NB>(W, K, wlds);
-  __syncthreads();
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int h = lane / 32, j = lane % 32;
-  const int total_waves = gridDim.x * (kGemmBlock / 64);
-  const int nrb = (n_rows + 31) / 32;
-  const int steps = K / 8;  // 8-wide k steps; this lane's rows of W in step s are 8s + 4h + t
-  const int G4 = (steps + 3) / 4;  // groups of four steps (32 values of k): the unit the A operand is fetched in
-  const wvec<NB> *wl = reinterpret_cast<const wvec<NB> *>(wlds) + (4 * h) * 32 + j;
-  // this wavefront's slice of LDS behind W: the row numbers of the blocks it is working on (row
-  // lists only).  Reading them from LDS keeps the row list out of the chain of global loads, so
-  // the A operands requested ahead are never waited for early.
-  int *ridx = reinterpret_cast<int *>(wlds + K * N) + wave * (kGemmSeg * 32);
-  // every wavefront walks one contiguous run of row blocks; run lengths differ by at most one
-  // and the longer runs are spread evenly over the compute units
-  const int gw = blockIdx.x * (kGemmBlock / 64) + wave;
-  // When the blocks do not divide among the wavefronts, the odd ones are cut into their NB column blocks
-  // and those are dealt out instead: a wavefront with one more whole block than the others would set
-  // the kernel's time (200,000 rows are 6,250 blocks for 2,048 wavefronts: four blocks against three
-  // and a quarter).  Not when the odd blocks are so many that a wavefront would get all columns anyway.
-  const int whole = nrb / total_waves, odd = nrb - whole * total_waves;
-  const int tail_per_wave = (odd * NB + total_waves - 1) / total_waves;
-  const bool split_tail = odd > 0 && tail_per_wave < NB;
-  const int run0 = split_tail ? gw * whole : (int)((long long)gw * nrb / total_waves);
-  const int run_end = split_tail ? run0 + whole : (int)((long long)(gw + 1) * nrb / total_waves);
-  if (split_tail) {
-    const int n_tail = odd * NB;
-    for (int t = gw * tail_per_wave; t < min(n_tail, (gw + 1) * tail_per_wave); ++t) {
-      const int rb = whole * total_waves + t / NB, nb = t % NB;
-      const int pos = min(rb * 32 + j, n_rows - 1);
-      const float *p = X + (size_t)(LIST ? rows[pos] : pos) * K + 4 * h;
-      v16f acc1;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc1[r] = 0.f;
-      const float *wt = wlds + ((4 * h) * 32 + j) * NB + nb;  // W[k][NB j + nb] sits at (k*32 + j)*NB + nb
-      fvec<4> a = *reinterpret_cast<const fvec<4> *>(p);
-      for (int st = 0; st < steps; ++st) {
-        const fvec<4> an = *reinterpret_cast<const fvec<4> *>(p + 8 * min(st + 1, steps - 1));
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[u], wt[(size_t)(8 * st + u) * 32 * NB], acc1, 0, 0, 0);
-        a = an;
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int x = rb * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-        if (x < n_rows) Y[(size_t)(LIST && !YPOS ? rows[x] : x) * N + NB * j + nb] = acc1[r];
-      }
-    }
-  }
-  for (int rb0 = run0; rb0 < run_end; rb0 += kGemmSeg) {
-    const int rb_end = min(run_end, rb0 + kGemmSeg);
-    if constexpr (LIST) {
-      for (int x = lane; x < (rb_end - rb0) * 32; x += 64) ridx[x] = rows[min(rb0 * 32 + x, n_rows - 1)];
-    }
-    const int total_groups = (rb_end - rb0) * G4;
-    // row (of X and Y) behind position x of this segment
-    auto row_at = [&](int x) { return LIST ? ridx[x] : min(rb0 * 32 + x, n_rows - 1); };
-    // ... and the row of Y it is stored to
-    auto yrow_at = [&](int x) { return LIST && !YPOS ? ridx[x] : min(rb0 * 32 + x, n_rows - 1); };
-    if constexpr (G4C > 0) {
-      static_assert(G4C >= 4 && G4C % 4 == 0, "four operand sets in turn, a block starts with the first");
-      const int nblk = rb_end - rb0;
-      auto operand_row = [&](int b) { return X + (size_t)row_at(min(b, nblk - 1) * 32 + j) * K + 4 * h; };
-      const float *pc = operand_row(0);
-      fvec<4> set[4][4];
-#pragma unroll
-      for (int q = 0; q < 3; ++q)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) set[q][u] = load4(pc + q * 32 + 8 * u);
-      wvec<NB> bw[4], bn[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) bw[t] = wl[t * 32];
-      // accumulator register r of block b, all NB column blocks, into its row of Y
-      auto store_row = [&](const v16f (&acc)[NB], int b, int r) __attribute__((always_inline)) {
-        wvec<NB> out;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) out.v[nb] = acc[nb][r];
-        *reinterpret_cast<wvec<NB> *>(Y + (size_t)yrow_at(b * 32 + 8 * (r / 4) + 4 * h + (r % 4)) * N + NB * j) = out;
-      };
-      for (int b = 0; b < nblk; ++b) {
-        const float *pn = operand_row(b + 1);
-        v16f acc[NB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
-#pragma unroll
-        for (int g = 0; g < G4C; ++g) {
-          const float *src = g + 3 < G4C ? pc + (g + 3) * 32 : pn + (g + 3 - G4C) * 32;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) set[(g + 3) % 4][u] = load4(src + 8 * u);
-          __builtin_amdgcn_sched_barrier(0);  // the requests stay here: the scheduler would move them to the block's end
-#pragma unroll
-          for (int t2 = 0; t2 < 4; t2 += 2) {
-            const int st = 4 * g + t2;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bn[t] = wl[(8 * (st + 1) + t) * 32];
-            mfma_step8<NB>(set[g % 4][t2], bw, acc);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bw[t] = wl[(8 * ((st + 2) % (4 * G4C)) + t) * 32];
-            mfma_step8<NB>(set[g % 4][t2 + 1], bn, acc);
-          }
-        }
-        if ((rb0 + b + 1) * 32 <= n_rows) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) store_row(acc, b, r);
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if ((rb0 + b) * 32 + 8 * (r / 4) + 4 * h + (r % 4) < n_rows) store_row(acc, b, r);
-        }
-        pc = pn;
-      }
-      continue;
-    }
-    // A operand of group gi (block rb0 + gi / G4, steps 4 (gi % G4) ..): four 16-byte loads per lane,
-    // always issued (block and k clamped to existing ones, the surplus is never used) so that the
-    // loads of later groups stay in flight while earlier ones are consumed.
-    auto load_group = [&](int gi, fvec<4> (&c)[4]) {
-      const int g = min(gi, total_groups - 1);
-      const int s0 = (g % G4) * 4;
-      const float *p = X + (size_t)row_at((g / G4) * 32 + j) * K + s0 * 8 + 4 * h;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) c[u] = *reinterpret_cast<const fvec<4> *>(p + 8 * min(u, steps - 1 - s0));
-    };
-    // three register sets, used in turn: a group's operands are requested two groups ahead
-    fvec<4> set0[4], set1[4], set2[4];
-    load_group(0, set0);
-    load_group(1, set1);
-    v16f acc[NB];
-    auto run_group = [&](int gi, const fvec<4> (&c)[4]) {
-      const int g = gi % G4, blk = gi / G4, s0 = 4 * g;
-      if (g == 0) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
-      }
-      wvec<NB> bw[4], bn[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) bw[t] = wl[(8 * s0 + t) * 32];
-      {
-        const int sn = min(s0 + 1, steps - 1);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) bn[t] = wl[(8 * sn + t) * 32];
-        mfma_step8<NB>(c[0], bw, acc);
-      }
-      if (s0 + 1 < steps) {
-        const int sn = min(s0 + 2, steps - 1);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) bw[t] = wl[(8 * sn + t) * 32];
-        mfma_step8<NB>(c[1], bn, acc);
-      }
-      if (s0 + 2 < steps) {
-        const int sn = min(s0 + 3, steps - 1);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) bn[t] = wl[(8 * sn + t) * 32];
-        mfma_step8<NB>(c[2], bw, acc);
-      }
-      if (s0 + 3 < steps) mfma_step8<NB>(c[3], bn, acc);
-      if (g == G4 - 1) {
-        // accumulator register r of column block nb of lane (h, j) holds output row 8*(r/4) + 4*h + r%4, column NB j + nb
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int x = blk * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-          if (rb0 * 32 + x < n_rows) {
-            wvec<NB> out;
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) out.v[nb] = acc[nb][r];
-            *reinterpret_cast<wvec<NB> *>(Y + (size_t)yrow_at(x) * N + NB * j) = out;
-          }
-        }
-      }
-    };
-    for (int gi = 0; gi < total_groups; gi += 3) {
-      load_group(gi + 2, set2);
-      run_group(gi, set0);
-      if (gi + 1 < total_groups) {
-        load_group(gi + 3, set0);
-        run_group(gi + 1, set1);
-      }
-      if (gi + 2 < total_groups) {
-        load_group(gi + 4, set1);
-        run_group(gi + 2, set2);
-      }
-    }
-  }
-}
 
 // Fused GeMM-SpMM tile kernel with W in registers.  v_mfma_f32_16x16x4_f32: a wavefront
 // owns 16 output columns (CPW such column blocks when N > 128) and keeps its K x 16 slice of
@@ -1957,42 +1705,6 @@ hipError_t launch_fused_gemm_spmm_stream(const TileDesc *tiles, int n_tiles, con
 #undef CALL2
 #undef CALL3
 #undef CALL4
-  return err != hipSuccess ? err : hipGetLastError();
-}
-
-hipError_t launch_gemm(const float *X, const float *W, float *Y, const int *rows, int n_rows, int K,
-                       int N, int compute_units, hipStream_t st, int y_by_position) {
-  if (n_rows <= 0) return hipSuccess;
-  if ((y_by_position && !rows) || (long long)K * N * 4 > 131072) return hipErrorInvalidValue;
-  const int NB = N / 32;
-  hipError_t err = hipSuccess;
-  const int w_bytes = K * N * 4;
-  // W resident in LDS: persistent workgroups, as many per compute unit as the LDS allows
-  const int per_cu = 1;  // register use (accumulators + both operand pipelines) allows one 8-wave workgroup
-  const int nrb = (n_rows + 31) / 32;
-  const int grid = std::max(1, std::min(compute_units * per_cu, (nrb + kGemmBlock / 64 - 1) / (kGemmBlock / 64)));
-  const int lds = w_bytes + (rows ? (kGemmBlock / 64) * kGemmSeg * 32 * 4 : 0);  // + the wavefronts' row numbers
-#define CALL3(NB_, LIST_, G4C_, YPOS_)                                                              \
-  err = allow_lds(gemm_rows_kernel<NB_, LIST_, G4C_, YPOS_>, lds);                                  \
-  if (err == hipSuccess)                                                                            \
-    hipLaunchKernelGGL((gemm_rows_kernel<NB_, LIST_, G4C_, YPOS_>), dim3(grid), dim3(kGemmBlock), lds, st, X, W, Y, \
-                       rows, n_rows, K)
-  // K = 128 and 256 with up to 128 columns have kernels of their own (K built in)
-#define CALL2(NB_, LIST_, YPOS_)                        \
-  do {                                                  \
-    if constexpr (NB_ <= 4) {                           \
-      if (K == 128) { CALL3(NB_, LIST_, 4, YPOS_); }    \
-      else if (K == 256) { CALL3(NB_, LIST_, 8, YPOS_); } \
-      else { CALL3(NB_, LIST_, 0, YPOS_); }             \
-    } else {                                            \
-      CALL3(NB_, LIST_, 0, YPOS_);                      \
-    }                                                   \
-  } while (0)
-#define CALL(NB_) do { if (rows && y_by_position) { CALL2(NB_, true, true); } else if (rows) { CALL2(NB_, true, false); } else { CALL2(NB_, false, false); } } while (0)
-  TF_DISPATCH_NB(NB, CALL);
-#undef CALL
-#undef CALL2
-#undef CALL3
   return err != hipSuccess ? err : hipGetLastError();
 }
 
