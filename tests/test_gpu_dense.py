@@ -95,6 +95,37 @@ def test_gemm_on_bf16_cores(gpu, tf, M, K, N, w_t):
         assert np.all(np.abs(got[M // 2] - want[M // 2]) <= (K + 8) * 2.0 ** -24 * np.abs(want[M // 2]).max())
 
 
+@pytest.mark.parametrize("K,N", [(128, 128), (120, 96), (64, 64), (40, 32), (136, 32), (256, 64), (256, 128)])
+def test_streamed_runs_on_bf16_cores(gpu, tf, K, N):
+    """Banded rows whose intermediate never leaves LDS: within fp32's rounding of float64, values of many sizes, and what is not finite
+    stays with the rows that read it."""
+    say(f"streamed runs {K} x {N}")
+    rng = np.random.default_rng(K + N)
+    M, width, n = 26001, 24, 7
+    cols = np.clip(np.arange(M)[:, None] + np.sort(np.argsort(rng.random((M, width)), axis=1)[:, :n], axis=1) - width // 2, 0, M - 1)
+    A = sp.csr_matrix((rng.uniform(-1, 1, M * n).astype(np.float32), cols.ravel(), np.arange(M + 1) * n), shape=(M, M))
+    A.sum_duplicates()
+    A.sort_indices()
+    B = (rng.uniform(-1, 1, (M, K)) * np.exp2(rng.uniform(-20, 20, (M, K)))).astype(np.float32)
+    W = rng.uniform(-0.2, 0.2, (K, N)).astype(np.float32)
+    B[0, K - 1], B[M - 1, 0], B[M // 2, 5] = np.inf, np.nan, 3.4e38
+    read = np.zeros(M, bool)
+    read[[0, M - 1, M // 2]] = True
+    odd = (A != 0).astype(np.float32) @ read.astype(np.float32) > 0
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K, lds_budget_bytes=163840)  # (a given budget: tiles, never two products)
+    assert S.info()["streamed"] == 1
+    D, Bd, Wd = tf.DenseMatrix(M, N), tf.DenseMatrix.from_numpy(B), tf.DenseMatrix.from_numpy(W)
+    tf.gemm_spmm(Ah.to_device(), Bd, Wd, D, S)
+    tf.device_synchronize()
+    got = D.to_numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = A.astype(np.float64) @ (B.astype(np.float64) @ W.astype(np.float64))
+    size = abs(A).astype(np.float64) @ (np.where(np.isfinite(B), np.abs(B), 0).astype(np.float64) @ np.abs(W).astype(np.float64))
+    assert np.all(np.abs(got[~odd] - want[~odd]) <= (K + n + 8) * 2.0 ** -24 * size[~odd])
+    assert np.array_equal(np.isnan(got[odd]), np.isnan(want[odd])) and not odd.all() and odd.sum() >= 3
+
+
 @pytest.mark.parametrize("K,N", [(129, 33), (64, 100), (18, 128)])
 def test_gemm_of_listed_rows(gpu, tf, K, N):
     """The rows an R-MAT graph reads, gathered by the product itself and stored in the order of their reads."""

@@ -359,7 +359,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
     for (int u = 0; u < U; ++u) {
       const int it = it0 + u * (int)blockDim.x;
       if (it >= items) break;
-      const split4 p = split8(v[u][0], v[u][1]);
+      const split3<bf8> p = split8(v[u][0], v[u][1]);
       bf8 *at = wparts + (size_t)(it / 64) * 192 + it % 64;
       at[0] = p.h;
       at[64] = p.m;
@@ -383,14 +383,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
   __syncthreads();
   acc4 big[T], small[T];
   const bf8 *wl = wparts + lane;
-  auto multiply = [&](int s, const split4 &a) __attribute__((always_inline)) {
+  auto multiply = [&](int s, const split3<bf8> &a) __attribute__((always_inline)) {
     const bf8 *w = wl + (size_t)s * (T * 192);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const bf8 wh = w[t * 192], wm = w[t * 192 + 64], wlo = w[t * 192 + 128];
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, wh, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wlo, small[t], 0, 0, 0);
-      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.u, wm, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, wm, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, wh, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wm, small[t], 0, 0, 0);
       big[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wh, big[t], 0, 0, 0);
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
         o[w] = d[w] & 2 ? f4v{o[w][2], o[w][3], 0.f, 0.f} : o[w];
       }
     }
-    const split4 a = split8(o[0], o[1]);
+    const split3<bf8> a = split8(o[0], o[1]);
     load(from, ahead, o);
     __builtin_amdgcn_sched_barrier(0);  // (the requests stay in front of the products)
     if (s < S) multiply(s, a);
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
     for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        big[t][r] += small[t][r] * (1.f / kSplitScale);
+        big[t][r] = (big[t][r] + small[t][r]) * kSplitOut;
         finite = __builtin_fmaf(big[t][r], 0.f, finite);
       }
     if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for bf16

@@ -198,27 +198,33 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 //
 // A float is the sum of three bf16 of eight significant bits each, x = h + m + l, every difference exact.  The product of two such
 // sums without the three terms below 2^-26 of it (m l, l m, l l) is six bf16 products, which v_mfma_f32_16x16x32_bf16 adds up in fp32 in 6 x 16
-// cycles per 32 values of k; v_mfma_f32_16x16x4_f32 takes 8 x 32.  h h goes to one accumulator, the five small terms, 2^8 times
-// too large, to another: the large sum is then rounded once per 32 values of k and not per four, and m and l keep their bits down to
-// where h alone is a normal bf16 (the cores take denormal bf16 for zero).  Relative error against 64 bits, values in [0, 1) times values
-// in [-0.2, 0.2), K = 32 / 64 / 128 / 256 / 512, this and fp32 MFMA: 0.36 / 0.47 / 0.62 / 0.86 / 1.05 and 1.0 / 1.6 / 2.2 / 3.0 / 3.7 e-7.
-// Infinities, NaN and what overflows bf16 make the sums NaN or infinite: the caller looks for those and computes such a block
-// again on the fp32 cores.
+// cycles per 32 values of k; v_mfma_f32_16x16x4_f32 takes 8 x 32.  Relative error against 64 bits, values in [0, 1) times values in [-0.2, 0.2),
+// K = 32 / 64 / 128 / 256 / 512, in e-7: fp32 cores 1.0 / 1.6 / 2.2 / 3.0 / 3.7, this in one accumulator 0.37 / 1.1 / 1.7 / 2.4 / 3.0, with
+// h h in one and the five small terms in another 0.36 / 0.47 / 0.62 / 0.86 / 1.05 (the large sum is then rounded once per 32 values of k).
+// The cores take denormal bf16 for zero: both operands are made 2^20 times larger on the way in, so that the parts of every
+// normal float are normal, and sums 2^-40 times smaller on the way out.  Infinities, NaN and sums beyond 2^88 come out infinite or NaN: the
+// caller looks for those and computes such a block again on the fp32 cores.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-struct split3 { bf8 h, m, l; };        // x = h + (m + l) / 256
-struct split4 { bf8 h, m, l, u; };     // ... and u = m / 256
-constexpr float kSplitScale = 256.f;
+typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+constexpr float kSplitIn = 0x1p20f, kSplitOut = 0x1p-40f;
+template <class T> struct split3 { T h, m, l; };
 
-__device__ __forceinline__ split4 split8(const f4v &lo, const f4v &hi) {
-  split4 o;
+__device__ __forceinline__ void split(float v, __bf16 &h, __bf16 &m, __bf16 &l) {
+  const float x = v * kSplitIn;
+  h = (__bf16)x;
+  const float r = x - (float)h;
+  m = (__bf16)r;
+  l = (__bf16)(r - (float)m);
+}
+__device__ __forceinline__ split3<bf8> split8(const f4v &lo, const f4v &hi) {
+  split3<bf8> o;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float x = i < 4 ? lo[i % 4] : hi[i % 4];
-    o.h[i] = (__bf16)x;
-    const float r = x - (float)o.h[i], r8 = r * kSplitScale;
-    o.u[i] = (__bf16)r;
-    o.m[i] = (__bf16)r8;
-    o.l[i] = (__bf16)(r8 - (float)o.m[i]);
+    __bf16 h, m, l;
+    split(i < 4 ? lo[i % 4] : hi[i % 4], h, m, l);
+    o.h[i] = h;
+    o.m[i] = m;
+    o.l[i] = l;
   }
   return o;
 }

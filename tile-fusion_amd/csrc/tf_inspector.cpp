@@ -234,7 +234,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
   // ... and stream: one workgroup per compute unit walks a long run of rows and keeps the last
   // ring_rows intermediate rows in LDS (a power of two, at least 256: 64 rows being written,
   // 64 of alignment slack and a reach of 128 or more).
-  const int stream_fixed = 2 * 64 * 36 * 4 + ((o.K <= 128 && o.N <= 128) ? 8 : 4) * 64 * 8 + (1024 + 4) * 4;  // X staging + consumer scratch + step table (<= 1024 steps)
+  const int stream_fixed = tf::kStreamStageBytes + ((o.K <= 128 && o.N <= 128) ? 8 : 4) * 64 * 8;  // X staging + consumer scratch
   auto ring_for = [&](int budget) {
     int r = 0;
     for (int c = 256; c <= 4096 && stream_fixed + (long long)c * (o.N + 4) * 4 <= budget; c *= 2) r = c;

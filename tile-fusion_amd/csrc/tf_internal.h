@@ -14,6 +14,8 @@
 namespace tf {
 
 constexpr int kMaxLds = 163840;  // LDS per workgroup on gfx950
+// Streamed GeMM-SpMM runs: two buffers of 64 x 32 values of B, each as three bf16 parts.
+constexpr int kStreamStageBytes = 24576;
 
 // One fused tile = one workgroup.  The workgroup computes intermediate rows
 // [prod_begin, prod_end) into LDS, stores rows [wb_begin, wb_end) of them to the

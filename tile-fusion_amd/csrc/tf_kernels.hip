@@ -862,8 +862,8 @@ __global__ __launch_bounds__(kGemmBlock) void fused_gemm_spmm_regw_kernel(
 // Streaming fused GeMM-SpMM kernel.  A workgroup walks one long run of intermediate rows,
 // 64 at a time, and keeps only the last `ring_rows` of them in LDS (a ring: row r sits in
 // slot (r - prod_begin) % ring_rows).  Eight producer wavefronts compute the next 64 rows on
-// MFMA exactly as in the tile kernel above (W in registers, X through the staging buffers)
-// while NCW consumer wavefronts compute the fused rows whose last column was produced in
+// the bf16 matrix cores (split8 in tf_device.h: a wavefront keeps the three parts of its 16 columns of W in registers, X becomes parts
+// on its way through the staging buffers, once for all wavefronts) while NCW consumer wavefronts compute the fused rows whose last column was produced in
 // the step before -- the schedule lists them step by step -- so the MFMA pipe and the
 // VALU/LDS gather work overlap all the time, W is loaded once per run and no row is computed
 // twice inside a run.  Both kinds of wavefront meet at one barrier per 32 values of k
@@ -877,7 +877,13 @@ __global__ __launch_bounds__(kGemmBlock) void fused_gemm_spmm_regw_kernel(
 // first LPR entries half a step ahead, both unconditionally (clamped to existing records).  The entries are turned
 // into (byte offset into the ring, value) pairs in a small per-group LDS area and walked in
 // CSR order with broadcast reads.
+// What bounds it: fp32 MFMAs and the consumers' FMAs share the vector pipe of a SIMD, so their times added up; the six bf16 products take 0.4
+// of the MFMA time and run beside FMAs (us, 262,144 rows of 16 in a band of 32, operands in no cache, fp32 producers / these: K = N = 128 132 / 115,
+// 256 x 128 215 / 178, 128 x 96 125 / 108, 64 x 128 125 / 111, 256 x 64 154 / 144, 128 x 64 90 / 85, 64 x 32 58 / 58).  Now the consumers: a row's
+// entries, one LDS read and four FMAs each, between two barriers.  The five small terms go to the same accumulators as the large one here
+// (registers): still closer to 64 bits than fp32 products (1.7 and 2.2e-7 at K = 128).
 constexpr int kStreamProducers = 8;   // wavefronts
+static_assert(kStreamStageBytes == 2 * 3 * kXRows * kXChunk * 2, "two buffers of three bf16 parts");
 
 template <int KS, int CPW, int LPR, int NCW, bool ACC>
 __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm_stream_kernel(
@@ -894,11 +900,10 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
   const int ld = N + kSlabPad;
   const int P = t.prod_end - t.prod_begin;
   const int S = (P + kXRows - 1) / kXRows;  // production steps
-  float *xbuf = lds;
-  float *ring = lds + kXStageFloats;
+  bf8 *xbuf = reinterpret_cast<bf8 *>(lds);
+  float *ring = lds + kStreamStageBytes / 4;
   const int ring_mask = ring_rows - 1;
-  int *sp = reinterpret_cast<int *>(ring + ring_rows * ld) + NCW * 128;  // S + 2 offsets into fused_rec
-  for (int x = threadIdx.x; x < S + 2; x += (NW + NCW) * 64) sp[x] = step_ptr[step_begin[blockIdx.x] + x];
+  const int *__restrict__ sp = step_ptr + step_begin[blockIdx.x];  // S + 2 offsets into fused_rec
 
   if (wave < NW) {
     // ---- producers -------------------------------------------------------------------
@@ -925,35 +930,54 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
       }
       return r;
     };
-    float *const xdst = xbuf + sr * kXLd + sk;
+    // Three parts of the unit in the order in which the matrix cores take them: row tile, k / 8, row, eight values of k.  (The rows of k / 8 = g
+    // in the order r ^ 4 g: the four that a row's threads write to lie in different banks.)
+    char *const xdst = reinterpret_cast<char *>(xbuf) + ((sr / 16 * 4 + sk / 8) * 16 + (sr % 16 ^ sk / 8 * 4)) * 16 + sk % 8 * 2;
+    auto put_unit = [&](int buf, const fvec<4> &x) {
+      split3<bf4> p;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        __bf16 hi, mid, lo;
+        split(x.v[c], hi, mid, lo);
+        p.h[c] = hi;
+        p.m[c] = mid;
+        p.l[c] = lo;
+      }
+      char *at = xdst + buf * (kStreamStageBytes / 2);
+      *reinterpret_cast<bf4 *>(at) = p.h;
+      *reinterpret_cast<bf4 *>(at + 4096) = p.m;
+      *reinterpret_cast<bf4 *>(at + 8192) = p.l;
+    };
     const int ld4 = ld * 4;
     char *const ring_lane = reinterpret_cast<char *>(ring) + ((16 * rg + 4 * h) * ld + 16 * cb0 + j) * 4;
-    {
-      const fvec<4> first = chunk_unit(0);
-      *reinterpret_cast<fvec<4> *>(xdst) = unit_or_zero(first, 0);
-    }
+    // W, the first unit and a step's worth of units behind it: one trip to memory for all
+    f4v wv[CPW][NKC][2];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+      for (int kc = 0; kc < NKC; ++kc)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int cb = cb0 + NW * c, k = 32 * kc + 8 * h + i;
+          wv[c][kc][i / 4][i % 4] = (cb < CB && k < K) ? W[(size_t)k * N + 16 * cb + j] : 0.f;
+        }
+    const fvec<4> first = chunk_unit(0);
     fvec<4> xs[NKC];  // xs[k]: the unit of the next interval k of a step that is not in LDS yet
 #pragma unroll
     for (int k = 0; k < NKC; ++k) xs[(k + 1) % NKC] = chunk_unit(k + 1);
-    float w[CPW][KS * 4];
+    split3<bf8> w[CPW][NKC];
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      const int cb = cb0 + NW * c;
+    for (int c = 0; c < CPW; ++c)
 #pragma unroll
-      for (int m = 0; m < KS; ++m)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int k = 16 * m + 4 * h + u;
-          w[c][4 * m + u] = (cb < CB && k < K) ? W[(size_t)k * N + 16 * cb + j] : 0.f;
-        }
-    }
-    // W has landed before the loop starts.  (Otherwise the first MFMA of every step waits for "everything
+      for (int kc = 0; kc < NKC; ++kc) w[c][kc] = split8(wv[c][kc][0], wv[c][kc][1]);
+    put_unit(0, unit_or_zero(first, 0));
+    // W has landed before the loop starts.  (Otherwise the first product of every step waits for "everything
     // requested before this point" -- the compiler cannot tell the loads of W, long done, from the staging
     // unit requested a moment ago, and a step would begin by waiting out a full trip to memory.)
 #pragma unroll
     for (int c = 0; c < CPW; ++c)
 #pragma unroll
-      for (int i = 0; i < KS * 4; ++i) asm volatile("" : : "v"(w[c][i]));
+      for (int kc = 0; kc < NKC; ++kc) asm volatile("" : : "v"(w[c][kc].h), "v"(w[c][kc].m), "v"(w[c][kc].l));
     lds_barrier();
     for (int q = 0; q < S; ++q) {
       v4f acc[CPW][4];
@@ -964,32 +988,68 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc) {
         const int ch = q * NKC + kc;
-        const float *xb = xbuf + (kc & 1) * (kXRows * kXLd);
+        const bf8 *xb = xbuf + (kc & 1) * (kStreamStageBytes / 32) + (16 * h + (j ^ 4 * h));
+        // The unit of the next interval goes to the other buffer, its register takes the unit of the same interval of the next step; in front
+        // of the products, which may then run on past the barrier.
+        put_unit((kc + 1) & 1, unit_or_zero(xs[(kc + 1) % NKC], (kc + 1) % NKC));
+        xs[(kc + 1) % NKC] = chunk_unit(ch + 1 + NKC);
         if (cb0 < CB && kc * kXChunk < K) {  // uniform
+          constexpr int PAIR = RG > 1 ? 2 : 1;  // row tiles multiplied side by side
 #pragma unroll
-          for (int m2 = 0; m2 < 2; ++m2) {
-            fvec<4> a[4];
+          for (int b0 = 0; b0 < 4; b0 += PAIR)
+            if (b0 * RG < 4) {
+              split3<bf8> x[PAIR];
+#pragma unroll
+              for (int u = 0; u < PAIR; ++u)
+                if ((b0 + u) * RG < 4) {
+                  const bf8 *p = xb + (rg + RG * (b0 + u)) * 64;
+                  x[u] = split3<bf8>{p[0], p[256], p[512]};
+                }
+#pragma unroll
+              for (int c = 0; c < CPW; ++c) {
+                const split3<bf8> &wp = w[c][kc];
+                auto add = [&](bf8 split3<bf8>::*xpart, bf8 split3<bf8>::*wpart) __attribute__((always_inline)) {
+#pragma unroll
+                  for (int u = 0; u < PAIR; ++u)
+                    if ((b0 + u) * RG < 4) acc[c][b0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u].*xpart, wp.*wpart, acc[c][b0 + u], 0, 0, 0);
+                };
+                add(&split3<bf8>::l, &split3<bf8>::h);
+                add(&split3<bf8>::h, &split3<bf8>::l);
+                add(&split3<bf8>::m, &split3<bf8>::m);
+                add(&split3<bf8>::m, &split3<bf8>::h);
+                add(&split3<bf8>::h, &split3<bf8>::m);
+                add(&split3<bf8>::h, &split3<bf8>::h);
+              }
+            }
+        }
+        if (kc == NKC - 1 && cb0 < CB) {
+          float finite = 0.f;
+#pragma unroll
+          for (int c = 0; c < CPW; ++c)
 #pragma unroll
             for (int bi = 0; bi < 4; ++bi)
-              if (bi * RG < 4)
-                a[bi] = *reinterpret_cast<const fvec<4> *>(xb + (16 * (rg + RG * bi) + j) * kXLd + 16 * m2 + 4 * h);
+              if (bi * RG < 4) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+                for (int r = 0; r < 4; ++r) {
+                  acc[c][bi][r] *= kSplitOut;
+                  finite = __builtin_fmaf(acc[c][bi][r], 0.f, finite);
+                }
+              }
+          if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for bf16: on the fp32 cores
+#pragma unroll
+            for (int c = 0; c < CPW; ++c)
 #pragma unroll
               for (int bi = 0; bi < 4; ++bi)
                 if (bi * RG < 4) {
-#pragma unroll
-                  for (int c = 0; c < CPW; ++c)
-                    acc[c][bi] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[bi].v[u], w[c][4 * (2 * kc + m2) + u],
-                                                                      acc[c][bi], 0, 0, 0);
+                  const float *row = B + (size_t)(t.prod_begin + min(q * kXRows + 16 * (rg + RG * bi) + j, P - 1)) * K;
+                  const int col = min(16 * (cb0 + NW * c) + j, N - 1);
+                  v4f s = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                  for (int k = h; k < K; k += 4)
+                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(relu_in ? fmaxf(row[k], 0.f) : row[k], W[(size_t)k * N + col], s, 0, 0, 0);
+                  acc[c][bi] = s;
                 }
           }
-        }
-        // the unit of the next interval goes to the other buffer, its register takes the unit
-        // of the same interval of the next step
-        *reinterpret_cast<fvec<4> *>(xdst + ((kc + 1) & 1) * (kXRows * kXLd)) = unit_or_zero(xs[(kc + 1) % NKC], (kc + 1) % NKC);
-        xs[(kc + 1) % NKC] = chunk_unit(ch + 1 + NKC);
-        if (kc == NKC - 1 && cb0 < CB) {
           // last interval of the step: the 64 new rows go into the ring (and to HBM where the
           // remainder reads them) before the barrier that lets the consumers at them
           const int row0 = t.prod_begin + q * kXRows;
@@ -1045,7 +1105,7 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
   const bool ok = coff < N;
   int2 *scratch = reinterpret_cast<int2 *>(ring + ring_rows * ld) + cg * LPR;
   const char *rbase = reinterpret_cast<const char *>(ring) + (ok ? coff : 0) * 4;
-  lds_barrier();  // step table visible (the producers' first staging unit too)
+  lds_barrier();  // (the producers' first staging unit is in LDS)
   const int sp_first = sp[0], sp_last = sp[S + 1];
   // Rows of a step [c0, c0 + len) handled in its interval kc: an even share.
   auto share = [&](int c0, int len, int kc, int &b, int &e) {
@@ -1105,8 +1165,11 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
 #pragma unroll
     for (int r = 0; r < RPI; ++r) load_entries(rec[kc][r], pc[kc][r], pa[kc][r]);
   int s0 = sp_first, s1 = sp[1];  // rows of step q are [s0, s1)
+  int spv = sp[min(lane, S + 1)];  // 64 of the steps' offsets, one a lane (a scalar load would be waited for by the next LDS read)
   for (int q = 0; q < S; ++q) {
-    const int s2 = q + 1 < S ? sp[q + 2] : s1;  // rows of the next production step: [s1, s2)
+    const int at = min(q + 2, S);
+    if ((at & 63) == 0 && at == q + 2) spv = sp[min(at + lane, S + 1)];
+    const int s2 = __builtin_amdgcn_readlane(spv, at & 63);  // rows of the next production step: [s1, s2)
 #pragma unroll
     for (int kc = 0; kc < NKC; ++kc) {
       int4 cur[RPI];
