@@ -158,6 +158,31 @@ def test_weight_gradient(gpu, tf, M, N, K):
     assert rel(Y.to_numpy(), G.astype(np.float64).T @ X.astype(np.float64)) <= 1e-5
 
 
+@pytest.mark.parametrize("M,N,K", [(4097, 1, 1), (4100, 3, 2), (4128, 17, 48), (4129, 33, 49), (5000, 49, 65), (9999, 64, 64), (33000, 100, 20), (150001, 7, 129)])
+def test_weight_gradient_on_bf16_cores(gpu, tf, M, N, K):
+    """Every width of tile, last blocks of any number of rows: within fp32's rounding of float64 for values of many sizes; what is not
+    finite stays in its row and column of the result."""
+    say(f"weight gradient on bf16 cores {M} rows, {N} x {K}")
+    rng = np.random.default_rng(M + N + K)
+    G, X = ((rng.uniform(-1, 1, (M, w)) * np.exp2(rng.uniform(-8, 8, (M, w)))).astype(np.float32) for w in (N, K))
+    lib = tf.lib()
+    ws = tf.DenseMatrix(1, max(1, lib.tf_weight_grad_workspace(M, N, K) // 4))
+    for odd in (False, True):
+        if odd:
+            G[M - 1, N - 1], X[M // 2, K - 1] = np.inf, np.nan
+        Gd, Xd, Y = tf.DenseMatrix.from_numpy(G), tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(np.full((N, K), np.nan, np.float32))
+        assert lib.tf_weight_grad(Gd.h, Xd.h, Y.h, C.c_void_p(ws.device_ptr()), None) == 0
+        tf.device_synchronize()
+        got = Y.to_numpy()
+        with np.errstate(invalid="ignore"):
+            want = G.astype(np.float64).T @ X.astype(np.float64)
+        ok = np.isfinite(want)
+        size = np.abs(np.where(np.isfinite(G), G, 0)).astype(np.float64).T @ np.abs(np.where(np.isfinite(X), X, 0)).astype(np.float64)
+        # fewer than 300 roundings of sums on the way of any term, each below the sum of magnitudes
+        assert np.all(np.abs(got[ok] - want[ok]) <= 300 * 2.0 ** -24 * size[ok])
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and ok.all() == (not odd)
+
+
 @pytest.mark.parametrize("N", [1, 3, 4, 7, 16, 40, 64, 100, 128, 257])
 @pytest.mark.parametrize("relu", [False, True])
 def test_scheduled_row_product(gpu, tf, N, relu):

@@ -368,9 +368,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
   };
   load_items(threadIdx.x);
   const float *xp = X;
-  int next_row = 0;  // of this lane in the block after the next one to begin
+  int row = 0, next_row = 0;  // of this lane in the block to begin next and in the one behind it
   if (b0 < n_blocks) {
-    xp = X + (size_t)row_index(b0) * ldx;
+    row = row_index(b0);
+    xp = X + (size_t)row * ldx;
     next_row = row_index(b0 + stride);
 #pragma unroll
     for (int u = 0; u < A; ++u) load(xp, u, x[u]);
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
     d[w] = at < K ? at - min(at, K - 4) : 0;
   }
   // A step: its values become parts, whereupon their registers take the values A steps on, of this block or the next.
-  auto step = [&](int s, f4v (&o)[2], const float *from, int ahead) __attribute__((always_inline)) {
+  auto step = [&](int s, f4v (&o)[2], const float *from, int ahead, float in_scale) __attribute__((always_inline)) {
     if (s == S - 1 && K % 4 != 0) {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
@@ -413,20 +414,24 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
         o[w] = d[w] & 2 ? f4v{o[w][2], o[w][3], 0.f, 0.f} : o[w];
       }
     }
-    const split3<bf8> a = split8(o[0], o[1]);
+    const split3<bf8> a = split8(o[0], o[1], in_scale);
     load(from, ahead, o);
     __builtin_amdgcn_sched_barrier(0);  // (the requests stay in front of the products)
     if (s < S) multiply(s, a);
   };
   for (int b = b0; b < n_blocks; b += stride) {
     const float *xn = X + (size_t)next_row * ldx;
+    const float in_scale = row & 1 ? -kSplitIn : kSplitIn;
+    row = next_row;
     next_row = row_index(b + 2 * stride);
     int y_row[4];
+    float out_scale[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int x = min(b * 16 + 4 * h + r, n_rows - 1);
-      if constexpr (OUT == kListed) y_row[r] = rows[x]; else y_row[r] = x;
-      if (OUT == kListed && !y_by_row) y_row[r] = x;
+      const int of = OUT == kPlain || OUT == kMasked ? x : OUT == kListed || rows ? rows[x] : x;
+      y_row[r] = OUT == kListed && y_by_row ? of : x;
+      out_scale[r] = of & 1 ? -kSplitOut : kSplitOut;
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -436,14 +441,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
     for (int g = 0; g < G; ++g) {
       const bool more = g + 1 < G;
 #pragma unroll
-      for (int u = 0; u < A; ++u) step(g * A + u, x[u], more ? xp : xn, more ? (g + 1) * A + u : u);
+      for (int u = 0; u < A; ++u) step(g * A + u, x[u], more ? xp : xn, more ? (g + 1) * A + u : u, in_scale);
     }
     float finite = 0.f;
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        big[t][r] = (big[t][r] + small[t][r]) * kSplitOut;
+        big[t][r] = (big[t][r] + small[t][r]) * out_scale[r];
         finite = __builtin_fmaf(big[t][r], 0.f, finite);
       }
     if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for bf16
@@ -467,14 +472,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
       for (int r = 0; r < 4; ++r) {
         const int x = b * 16 + 4 * h + r;
         if (x >= n_rows) continue;
-        const size_t row = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
+        const size_t y = (size_t)(rows && y_by_row ? rows[x] : x) * ldy;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
           const int c = panel0 + 16 * V * q + V * j;
           cvec<V> out;
 #pragma unroll
           for (int v = 0; v < V; ++v) out.v[v] = big[q * V + v][r];
-          gemm_store<V>(Y, row + c, out, N - c, out_how);
+          gemm_store<V>(Y, y + c, out, N - c, out_how);
         }
       }
     } else {
@@ -596,72 +601,113 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 }
 
 // ---------------------------------------------------------------------------------
-// Y[n, k] = sum over m < M of G[m, n] * X[m, k]: the gradient of a layer's weights.  Both operands are read once, in
-// whole rows; a wavefront holds a 32 NB x 32 KB tile of Y (v_mfma_f32_32x32x2_f32: lane (j, h) supplies row m + h of
-// both operands) and sums its share of the rows, the four wavefronts of a workgroup are added through LDS, and
-// weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.  Column NB j + nb of G belongs to
-// column block nb (and KB j + kb of X to kb), so that a lane loads adjacent columns; a lane whose columns would
-// reach past the last one works on the last NB (KB) instead, which writes some values of Y twice, the same.
-// Bound: the rows of X and G from HBM, or fp32 MFMA when 2 N K / 4 (N + K) exceeds 31 FLOP per byte.
+// Y[n, k] = sum over m < M of G[m, n] * X[m, k]: the gradient of a layer's weights, on the bf16 matrix cores (split8 in tf_device.h).  A
+// wavefront holds a 16 NB x 16 KB tile of Y and takes 32 rows of both operands at a time, in whole lines: lane (j, h) loads the columns
+// NB j .. of G and KB j .. of X in the rows 8 h .. 8 h + 7, which are what its part of a 16 x 16 x 32 product wants of each of
+// the NB (KB) column blocks.  The next rows are requested as soon as these have become parts.  The wavefronts of a launch take blocks of
+// rows in turn; a workgroup's four are added through LDS, and weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.
+// A lane whose columns would reach past the last one works on the last NB (KB) instead, which writes some values of Y twice, the same.
+// Bound: the rows of X and G from HBM, 16 KB a wavefront in flight, behind some 10 us for two launches and the sums at the end (us, operands in no
+// cache, both launches, fp32 cores on 64 x 160 tiles / this: 14,000 rows 32 x 69 18.2 / 9.5, 35,000 rows 64 x 128 26.1 / 22.5, 100,000 rows 64 x 128 36.6 / 33.0,
+// 20 x 100 26.6 / 22.8, 131,072 rows 64 x 300 75 / 66, 40 x 64 28.3 / 24.4, 262,144 rows 128 x 128 109 / 98; error against 64 bits at 100,000 rows
+// 1.7e-7 / 1.0e-7).
 // ---------------------------------------------------------------------------------
-constexpr int kWgUnroll = 4;  // pairs of rows in flight per wavefront
+constexpr int kWgRows = 32;       // rows of a block
 constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel
 
 template <int NB, int KB>
 __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__restrict__ G, int N, const float *__restrict__ X,
-                                                             int K, int M, int rows_per_group, int k_chunks,
-                                                             float *__restrict__ partial) {
+                                                             int K, int M, int k_chunks, float *__restrict__ partial) {
   constexpr int T = NB * KB;
-  __shared__ acc16 red[2][T][64];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 32, h = lane / 32;
+  __shared__ acc4 red[2][T][64];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
   const int nc = blockIdx.y / k_chunks, kc = blockIdx.y % k_chunks;
-  const float *gp = G + min(nc * 32 * NB + NB * j, N - NB);
-  const float *xp = X + min(kc * 32 * KB + KB * j, K - KB);
-  const int m_end = min(M, (int)(blockIdx.x + 1) * rows_per_group);
-  acc16 acc[NB][KB];
+  const float *gp = G + min(nc * 16 * NB + NB * j, N - NB);
+  const float *xp = X + min(kc * 16 * KB + KB * j, K - KB);
+  const int n_blocks = (M + kWgRows - 1) / kWgRows, stride = 4 * gridDim.x, b0 = 4 * blockIdx.x + wave;
+  acc4 acc[NB][KB];
 #pragma unroll
   for (int a = 0; a < NB; ++a)
 #pragma unroll
     for (int b = 0; b < KB; ++b) acc[a][b] = 0.f;
-  struct operands { cvec<NB> g[kWgUnroll]; cvec<KB> x[kWgUnroll]; };
-  auto load = [&](int m0) __attribute__((always_inline)) {
-    operands o;
+  cvec<NB> g[8];
+  cvec<KB> x[8];
+  auto load_g = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kWgUnroll; ++u) {
-      const size_t m = min(m0 + 2 * u + h, M - 1);
-      o.g[u] = *reinterpret_cast<const cvec<NB> *>(gp + m * N);
-      o.x[u] = *reinterpret_cast<const cvec<KB> *>(xp + m * K);
-    }
-    return o;
+    for (int i = 0; i < 8; ++i) g[i] = *reinterpret_cast<const cvec<NB> *>(gp + (size_t)min(kWgRows * b + 8 * h + i, M - 1) * N);
   };
-  auto multiply = [&](const operands &o) __attribute__((always_inline)) {
+  auto load_x = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kWgUnroll; ++u)
-#pragma unroll
-      for (int a = 0; a < NB; ++a)
-#pragma unroll
-        for (int b = 0; b < KB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(o.g[u].v[a], o.x[u].v[b], acc[a][b], 0, 0, 0);
+    for (int i = 0; i < 8; ++i) x[i] = *reinterpret_cast<const cvec<KB> *>(xp + (size_t)min(kWgRows * b + 8 * h + i, M - 1) * K);
   };
-  constexpr int S = 2 * kWgUnroll;  // rows per step
-  int m = blockIdx.x * rows_per_group + wave * S;
-  if (m < m_end) {
-    operands cur = load(m);
-    for (; m + S <= m_end; m += 4 * S) {
-      const operands nxt = load(m + 4 * S < m_end ? m + 4 * S : m);
-      multiply(cur);
-      cur = nxt;
-    }
-    if (m < m_end) {  // rows past the group's last one are zeros in both operands
+  if (b0 < n_blocks) {
+    load_g(b0);
+    load_x(b0);
+  }
+  for (int b = b0; b < n_blocks; b += stride) {
+    if (kWgRows * (b + 1) > M) {  // rows past the last one are zeros in both operands
 #pragma unroll
-      for (int u = 0; u < kWgUnroll; ++u)
-        if (m + 2 * u + h >= m_end) {
+      for (int i = 0; i < 8; ++i)
+        if (kWgRows * b + 8 * h + i >= M) {
 #pragma unroll
-          for (int a = 0; a < NB; ++a) cur.g[u].v[a] = 0.f;
+          for (int a = 0; a < NB; ++a) g[i].v[a] = 0.f;
 #pragma unroll
-          for (int b = 0; b < KB; ++b) cur.x[u].v[b] = 0.f;
+          for (int c = 0; c < KB; ++c) x[i].v[c] = 0.f;
         }
-      multiply(cur);
     }
+    const float sign = b & 1 ? -1.f : 1.f;
+    split3<bf8> gs[NB], xs[KB];
+#pragma unroll
+    for (int a = 0; a < NB; ++a) gs[a] = split8(f4v{g[0].v[a], g[1].v[a], g[2].v[a], g[3].v[a]}, f4v{g[4].v[a], g[5].v[a], g[6].v[a], g[7].v[a]}, sign * kSplitIn);
+    load_g(b + stride);
+#pragma unroll
+    for (int c = 0; c < KB; ++c) xs[c] = split8(f4v{x[0].v[c], x[1].v[c], x[2].v[c], x[3].v[c]}, f4v{x[4].v[c], x[5].v[c], x[6].v[c], x[7].v[c]});
+    load_x(b + stride);
+    __builtin_amdgcn_sched_barrier(0);  // (the requests stay in front of the products)
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int c = 0; c < KB; ++c) {
+        acc4 s = 0.f;  // (the block's own sum: the long sum is rounded once per 32 rows)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].h, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].l, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].m, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].h, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].m, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].h, s, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[a][c][r] = __builtin_fmaf(sign, s[r], acc[a][c][r]);
+      }
+  }
+  float finite = 0.f;
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int c = 0; c < KB; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        acc[a][c][r] *= kSplitOut;
+        finite = __builtin_fmaf(acc[a][c][r], 0.f, finite);
+      }
+  if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for the parts: on the fp32 cores
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+      for (int c = 0; c < KB; ++c) acc[a][c] = 0.f;
+#pragma unroll 1
+    for (int b = b0; b < n_blocks; b += stride)
+#pragma unroll 1
+      for (int m0 = kWgRows * b; m0 < min(kWgRows * (b + 1), M); m0 += 4) {
+        const size_t m = min(m0 + h, M - 1);
+        const float in = m0 + h < M ? 1.f : 0.f;
+        cvec<NB> gv = *reinterpret_cast<const cvec<NB> *>(gp + m * N);
+        cvec<KB> xv = *reinterpret_cast<const cvec<KB> *>(xp + m * K);
+#pragma unroll
+        for (int a = 0; a < NB; ++a)
+#pragma unroll
+          for (int c = 0; c < KB; ++c)
+            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(in != 0.f ? gv.v[a] : 0.f, in != 0.f ? xv.v[c] : 0.f, acc[a][c], 0, 0, 0);
+      }
   }
 #pragma unroll
   for (int half = 2; half >= 1; half /= 2) {
@@ -669,53 +715,56 @@ __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__rest
 #pragma unroll
       for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int b = 0; b < KB; ++b) red[wave - half][a * KB + b][lane] = acc[a][b];
+        for (int c = 0; c < KB; ++c) red[wave - half][a * KB + c][lane] = acc[a][c];
     }
     __syncthreads();
     if (wave < half) {
 #pragma unroll
       for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int b = 0; b < KB; ++b) acc[a][b] += red[wave][a * KB + b][lane];
+        for (int c = 0; c < KB; ++c) acc[a][c] += red[wave][a * KB + c][lane];
     }
     __syncthreads();
   }
   if (wave == 0) {  // partial[group][chunk][tile][register][lane]
-    float *out = partial + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * (T * 1024) + lane;
+    float *out = partial + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * (T * 256) + lane;
 #pragma unroll
     for (int a = 0; a < NB; ++a)
 #pragma unroll
-      for (int b = 0; b < KB; ++b)
+      for (int c = 0; c < KB; ++c)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[((a * KB + b) * 16 + r) * 64] = acc[a][b][r];
+        for (int r = 0; r < 4; ++r) out[((a * KB + c) * 4 + r) * 64] = acc[a][c][r];
   }
 }
 
-// Adds the groups' tiles: one workgroup per register of a tile, the groups dealt to its four wavefronts.
+// Adds the groups' tiles: one workgroup per register of a tile, the groups dealt to its four wavefronts, eight loads of each in flight (four: 10 us
+// for 256 groups of 64 x 128).
 __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float *__restrict__ partial, int groups, int chunks,
                                                                  int k_chunks, int NB, int KB, int N, int K,
                                                                  float *__restrict__ Y) {
   __shared__ float red[3][64];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 32, h = lane / 32;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
   const int T = NB * KB, chunk = blockIdx.y, reg = blockIdx.x;
-  const float *p = partial + (size_t)chunk * (T * 1024) + reg * 64 + lane;
-  const size_t stride = (size_t)chunks * (T * 1024);
+  const float *p = partial + (size_t)chunk * (T * 256) + reg * 64 + lane;
+  const size_t stride = (size_t)chunks * (T * 256);
   float s = 0.f;
-  int g = wave;
-  for (; g + 12 < groups; g += 16) {
-    const float a = p[(size_t)g * stride], b = p[(size_t)(g + 4) * stride], c = p[(size_t)(g + 8) * stride], d = p[(size_t)(g + 12) * stride];
-    s += (a + b) + (c + d);
+  for (int g = wave; g < groups; g += 32) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(g + 4 * u, groups - 1) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = g + 4 * u < groups ? v[u] : 0.f;
+    s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   }
-  for (; g < groups; g += 4) s += p[(size_t)g * stride];
   if (wave > 0) red[wave - 1][lane] = s;
   __syncthreads();
   if (wave > 0) return;
   s += red[0][lane];
   s += red[1][lane];
   s += red[2][lane];
-  const int r = reg % 16, kb = (reg / 16) % KB, nb = reg / 16 / KB;
-  const int i = 8 * (r / 4) + 4 * h + r % 4;  // row of the 32 x 32 block that register r of lane (j, h) holds
-  const int n = min(chunk / k_chunks * 32 * NB + NB * i, N - NB) + nb, k = min(chunk % k_chunks * 32 * KB + KB * j, K - KB) + kb;
+  const int r = reg % 4, kb = (reg / 4) % KB, nb = reg / 4 / KB;
+  const int i = 4 * h + r;  // row of the 16 x 16 block that register r of lane (j, h) holds
+  const int n = min(chunk / k_chunks * 16 * NB + NB * i, N - NB) + nb, k = min(chunk % k_chunks * 16 * KB + KB * j, K - KB) + kb;
   Y[(size_t)n * K + k] = s;
 }
 
@@ -772,19 +821,21 @@ WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
   p.few = M <= kWgFewRows && ((N + 15) / 16) * ((K + 15) / 16) <= 2 * compute_units && std::max(N, K) <= 16384;
   p.partial_floats = 0;
   if (p.few) return p;
-  p.nb = N > 32 ? 2 : 1;
-  p.n_chunks = (N + 32 * p.nb - 1) / (32 * p.nb);
-  // the width of X in the fewest chunks of at most 160 columns, evenly (300 = 2 x 160, 128 = 1 x 128, 500 = 4 x 128)
-  p.k_chunks = (K + 159) / 160;
-  p.kb = std::max(1, std::min(5, (K + 32 * p.k_chunks - 1) / (32 * p.k_chunks)));
-  if (p.kb > K) p.kb = 1;
-  p.k_chunks = (K + 32 * p.kb - 1) / (32 * p.kb);
+  // chunks of up to 64 columns of both, evenly (300 = 5 x 64, 128 = 2 x 64, 40 = 48)
+  auto cut = [](int width, int &chunks, int &blocks) {
+    chunks = (width + 63) / 64;
+    blocks = std::min(width, ((width + chunks - 1) / chunks + 15) / 16);
+    chunks = (width + 16 * blocks - 1) / (16 * blocks);
+  };
+  cut(N, p.n_chunks, p.nb);
+  cut(K, p.k_chunks, p.kb);
   const int chunks = p.n_chunks * p.k_chunks;
-  // two workgroups per compute unit; a group has 32 rows or more (one step of its four wavefronts)
-  const int want = std::max(1, 2 * compute_units / chunks);
-  p.rows_per_group = std::max(32, (((M + want - 1) / want) + 31) / 32 * 32);
-  p.groups = (M + p.rows_per_group - 1) / p.rows_per_group;
-  p.partial_floats = (size_t)p.groups * chunks * p.nb * p.kb * 1024;
+  // two workgroups per compute unit; a wavefront has a block of rows or more
+  const int blocks = (M + kWgRows - 1) / kWgRows;
+  // (a multiple of 8: the chunks of a block of rows on one XCD, whose L2 has the other operand and the lines two chunks share)
+  p.groups = std::max(1, std::min(std::max(1, 2 * compute_units / chunks), (blocks + 3) / 4));
+  if (p.groups > 8) p.groups = p.groups / 8 * 8;
+  p.partial_floats = (size_t)p.groups * chunks * p.nb * p.kb * 256;
   return p;
 }
 
@@ -796,21 +847,14 @@ hipError_t launch_weight_grad(const WeightGradPlan &p, const float *G, int N, co
   }
   const int chunks = p.n_chunks * p.k_chunks;
   const dim3 grid(p.groups, chunks);
-#define CALL2(NB_, KB_) \
-  hipLaunchKernelGGL((weight_grad_kernel<NB_, KB_>), grid, dim3(256), 0, st, G, N, X, K, M, p.rows_per_group, p.k_chunks, partial)
-#define CALL(NB_)                                                                  \
-  do {                                                                             \
-    switch (p.kb) {                                                                \
-      case 1: CALL2(NB_, 1); break; case 2: CALL2(NB_, 2); break; case 3: CALL2(NB_, 3); break; \
-      case 4: CALL2(NB_, 4); break; default: CALL2(NB_, 5); break;                 \
-    }                                                                              \
-  } while (0)
-  if (p.nb == 2) CALL(2); else CALL(1);
+#define CALL2(NB_, KB_) hipLaunchKernelGGL((weight_grad_kernel<NB_, KB_>), grid, dim3(256), 0, st, G, N, X, K, M, p.k_chunks, partial)
+#define CALL(NB_) do { switch (p.kb) { case 1: CALL2(NB_, 1); break; case 2: CALL2(NB_, 2); break; case 3: CALL2(NB_, 3); break; default: CALL2(NB_, 4); } } while (0)
+  switch (p.nb) { case 1: CALL(1); break; case 2: CALL(2); break; case 3: CALL(3); break; default: CALL(4); }
 #undef CALL
 #undef CALL2
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3(p.nb * p.kb * 16, chunks), dim3(256), 0, st, partial, p.groups, chunks, p.k_chunks,
+  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3(p.nb * p.kb * 4, chunks), dim3(256), 0, st, partial, p.groups, chunks, p.k_chunks,
                      p.nb, p.kb, N, K, Y);
   return hipGetLastError();
 }

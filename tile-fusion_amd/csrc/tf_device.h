@@ -204,24 +204,26 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 // The cores take denormal bf16 for zero: both operands are made 2^20 times larger on the way in, so that the parts of every
 // normal float are normal, and sums 2^-40 times smaller on the way out.  Infinities, NaN and sums beyond 2^88 come out infinite or NaN: the
 // caller looks for those and computes such a block again on the fp32 cores.
+// What the cores cut off when they align products is always cut downwards, some 4e-9 of a sum: nothing in one result, but 2e-7 in a
+// weight gradient over 3,000 blocks of rows with as many terms of either sign.  Callers therefore scale rows of odd number, or every other block of them, by -2^20.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
 constexpr float kSplitIn = 0x1p20f, kSplitOut = 0x1p-40f;
 template <class T> struct split3 { T h, m, l; };
 
-__device__ __forceinline__ void split(float v, __bf16 &h, __bf16 &m, __bf16 &l) {
-  const float x = v * kSplitIn;
+__device__ __forceinline__ void split(float v, __bf16 &h, __bf16 &m, __bf16 &l, float scale = kSplitIn) {
+  const float x = v * scale;
   h = (__bf16)x;
   const float r = x - (float)h;
   m = (__bf16)r;
   l = (__bf16)(r - (float)m);
 }
-__device__ __forceinline__ split3<bf8> split8(const f4v &lo, const f4v &hi) {
+__device__ __forceinline__ split3<bf8> split8(const f4v &lo, const f4v &hi, float scale = kSplitIn) {
   split3<bf8> o;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     __bf16 h, m, l;
-    split(i < 4 ? lo[i % 4] : hi[i % 4], h, m, l);
+    split(i < 4 ? lo[i % 4] : hi[i % 4], h, m, l, scale);
     o.h[i] = h;
     o.m[i] = m;
     o.l[i] = l;

@@ -96,7 +96,7 @@ struct GemmOut {
 // How launch_weight_grad cuts Y = G^T X (tf_dense.hip).
 struct WeightGradPlan {
   bool few;  // in one launch, without a workspace; the cuts below are not set
-  int nb, kb, n_chunks, k_chunks, rows_per_group, groups;
+  int nb, kb, n_chunks, k_chunks, groups;
   size_t partial_floats;
 };
 

@@ -938,7 +938,7 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         __bf16 hi, mid, lo;
-        split(x.v[c], hi, mid, lo);
+        split(x.v[c], hi, mid, lo, sr / 16 % 2 ? -kSplitIn : kSplitIn);
         p.h[c] = hi;
         p.m[c] = mid;
         p.l[c] = lo;
@@ -1031,7 +1031,7 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
               if (bi * RG < 4) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                  acc[c][bi][r] *= kSplitOut;
+                  acc[c][bi][r] *= (rg + RG * bi) % 2 ? -kSplitOut : kSplitOut;
                   finite = __builtin_fmaf(acc[c][bi][r], 0.f, finite);
                 }
               }
