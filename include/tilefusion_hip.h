@@ -482,6 +482,9 @@ tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *Y, const tf
  * tf_weight_grad_workspace(M, N, K) bytes (null where that is 0), in use until the call's work on `stream` is done. */
 tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream);
 size_t tf_weight_grad_workspace(int M, int N, int K);
+/* Two of them in the launches of one: Y1 = G1^T X1 and Y2 = G2^T X2, the same bits as two calls, each with a workspace of its own. */
+tf_status tf_weight_grad_pair(const tf_dense *G1, const tf_dense *X1, tf_dense *Y1, float *workspace1, const tf_dense *G2, const tf_dense *X2,
+                              tf_dense *Y2, float *workspace2, void *stream);
 
 /* D = A * (B * C), A and B sparse, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the

@@ -183,6 +183,32 @@ def test_weight_gradient_on_bf16_cores(gpu, tf, M, N, K):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and ok.all() == (not odd)
 
 
+@pytest.mark.parametrize("M1,M2", [(100, 100), (3072, 3072), (3073, 3073), (20001, 20001), (3000, 5000), (5000, 3000)])
+def test_two_weight_gradients_in_one_call(gpu, tf, M1, M2):
+    """Sharing their launches changes no bit of either, of few rows and of many (and of one and the other)."""
+    say(f"two weight gradients {M1} {M2}")
+    rng = np.random.default_rng(M1 + M2)
+    lib = tf.lib()
+    alone, pair = [], []
+    for M, N, K in ((M1, 32, 69), (M2, 7, 130)):
+        Gd, Xd = (tf.DenseMatrix.from_numpy(rng.uniform(-1, 1, (M, w)).astype(np.float32)) for w in (N, K))
+        ws = tf.DenseMatrix(1, max(1, lib.tf_weight_grad_workspace(M, N, K) // 4))
+        Y = [tf.DenseMatrix.from_numpy(np.full((N, K), np.nan, np.float32)) for _ in range(2)]
+        assert lib.tf_weight_grad(Gd.h, Xd.h, Y[0].h, C.c_void_p(ws.device_ptr()), None) == 0
+        alone.append((Y[0], Gd, Xd, ws))
+        pair.append((Gd, Xd, Y[1], ws))
+    args = [a for g, x, y, ws in pair for a in (g.h, x.h, y.h, C.c_void_p(ws.device_ptr()))]
+    tf.device_synchronize()
+    assert lib.tf_weight_grad_pair(*args, None) == 0
+    tf.device_synchronize()
+    for (want, G, X, _), (_, _, got, _) in zip(alone, pair):
+        assert np.array_equal(got.to_numpy(), want.to_numpy())
+        assert rel(got.to_numpy(), G.to_numpy().astype(np.float64).T @ X.to_numpy().astype(np.float64)) <= 1e-5
+    for bad in range(8):  # every operand is checked before either product runs
+        if bad % 4 != 3:
+            assert lib.tf_weight_grad_pair(*[None if i == bad else a for i, a in enumerate(args)], None) != 0
+
+
 @pytest.mark.parametrize("N", [1, 3, 4, 7, 16, 40, 64, 100, 128, 257])
 @pytest.mark.parametrize("relu", [False, True])
 def test_scheduled_row_product(gpu, tf, N, relu):

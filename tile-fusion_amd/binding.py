@@ -132,6 +132,7 @@ SIGNATURES = {
     "tf_gemm": (C.c_int, [_VP, _VP, _VP, _VP]),
     "tf_gemm_ex": (C.c_int, [_VP, _VP, _VP, _VP, C.c_uint, _VP]),
     "tf_weight_grad": (C.c_int, [_VP, _VP, _VP, _VP, _VP]),
+    "tf_weight_grad_pair": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP]),
     "tf_weight_grad_workspace": (C.c_size_t, [C.c_int, C.c_int, C.c_int]),
     "tf_calibrate_issue": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float)]),
 }

@@ -96,8 +96,8 @@ hipError_t launch_fused_spmm_spmm_window64(const TileDesc *, const int *, int, c
 hipError_t launch_spmm_rows(RowsArgs, const RowsHow &, hipStream_t);
 hipError_t launch_spmm_gemm(RowsArgs, const RowsHow &, const float *, int, int, const GemmOut &, hipStream_t);
 hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int, const int *, int, int, int, int, const GemmOut &, int, hipStream_t);
-WeightGradPlan plan_weight_grad(int, int, int, int);
-hipError_t launch_weight_grad(const WeightGradPlan &, const float *, int, const float *, int, int, float *, float *, hipStream_t);
+WeightGradTask plan_weight_grad(int, int, int, int);
+hipError_t launch_weight_grads(const WeightGradTask &, const WeightGradTask *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
 hipError_t launch_march_fill(const int *, const int *, const float *, const float *, int *, size_t, hipStream_t);
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
@@ -1223,15 +1223,34 @@ extern "C" tf_status tf_gemm_ex(const tf_dense *X, const tf_dense *W, tf_dense *
 
 extern "C" size_t tf_weight_grad_workspace(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return tf::plan_weight_grad(M, N, K, tf::default_compute_units()).partial_floats * sizeof(float);
+  return tf::plan_weight_grad(M, N, K, tf::default_compute_units()).partial_floats() * sizeof(float);
+}
+
+static tf_status weight_grad_task(const char *who, const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, tf::WeightGradTask *t) {
+  if (!G || !X || !Y) return fail(TF_EINVAL, "%s: null argument", who);
+  if (G->M != X->M || Y->M != G->N || Y->N != X->N)
+    return fail(TF_EINVAL, "%s: shapes G %d x %d, X %d x %d, Y %d x %d", who, G->M, G->N, X->M, X->N, Y->M, Y->N);
+  *t = tf::plan_weight_grad(G->M, G->N, X->N, tf::default_compute_units());
+  if (t->partial_floats() && !workspace) return fail(TF_EINVAL, "%s: %zu bytes of workspace needed", who, t->partial_floats() * sizeof(float));
+  t->G = G->d;
+  t->X = X->d;
+  t->Y = Y->d;
+  t->partial = workspace;
+  return TF_OK;
 }
 
 extern "C" tf_status tf_weight_grad(const tf_dense *G, const tf_dense *X, tf_dense *Y, float *workspace, void *stream) {
-  if (!G || !X || !Y) return fail(TF_EINVAL, "tf_weight_grad: null argument");
-  if (G->M != X->M || Y->M != G->N || Y->N != X->N)
-    return fail(TF_EINVAL, "tf_weight_grad: shapes G %d x %d, X %d x %d, Y %d x %d", G->M, G->N, X->M, X->N, Y->M, Y->N);
-  const tf::WeightGradPlan p = tf::plan_weight_grad(G->M, G->N, X->N, tf::default_compute_units());
-  if (p.partial_floats && !workspace) return fail(TF_EINVAL, "tf_weight_grad: %zu bytes of workspace needed", p.partial_floats * sizeof(float));
-  TF_HIP(tf::launch_weight_grad(p, G->d, G->N, X->d, X->N, G->M, workspace, Y->d, static_cast<hipStream_t>(stream)));
+  tf::WeightGradTask t;
+  if (tf_status rc = weight_grad_task("tf_weight_grad", G, X, Y, workspace, &t)) return rc;
+  TF_HIP(tf::launch_weight_grads(t, nullptr, static_cast<hipStream_t>(stream)));
+  return TF_OK;
+}
+
+extern "C" tf_status tf_weight_grad_pair(const tf_dense *G1, const tf_dense *X1, tf_dense *Y1, float *workspace1, const tf_dense *G2, const tf_dense *X2,
+                                         tf_dense *Y2, float *workspace2, void *stream) {
+  tf::WeightGradTask a, b;
+  if (tf_status rc = weight_grad_task("tf_weight_grad_pair", G1, X1, Y1, workspace1, &a)) return rc;
+  if (tf_status rc = weight_grad_task("tf_weight_grad_pair", G2, X2, Y2, workspace2, &b)) return rc;
+  TF_HIP(tf::launch_weight_grads(a, &b, static_cast<hipStream_t>(stream)));
   return TF_OK;
 }

@@ -613,18 +613,18 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // 1.7e-7 / 1.0e-7).
 // ---------------------------------------------------------------------------------
 constexpr int kWgRows = 32;       // rows of a block
-constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel
+constexpr int kWgFewRows = 3072;  // up to here in one launch, weight_grad_few_kernel
 
 template <int NB, int KB>
-__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__restrict__ G, int N, const float *__restrict__ X,
-                                                             int K, int M, int k_chunks, float *__restrict__ partial) {
+__device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int group, int chunk, acc4 (*red)[64]) {
   constexpr int T = NB * KB;
-  __shared__ acc4 red[2][T][64];
+  const float *__restrict__ G = t.G, *__restrict__ X = t.X;
+  const int N = t.N, K = t.K, M = t.M;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
-  const int nc = blockIdx.y / k_chunks, kc = blockIdx.y % k_chunks;
+  const int nc = chunk / t.k_chunks, kc = chunk % t.k_chunks;
   const float *gp = G + min(nc * 16 * NB + NB * j, N - NB);
   const float *xp = X + min(kc * 16 * KB + KB * j, K - KB);
-  const int n_blocks = (M + kWgRows - 1) / kWgRows, stride = 4 * gridDim.x, b0 = 4 * blockIdx.x + wave;
+  const int n_blocks = (M + kWgRows - 1) / kWgRows, stride = 4 * t.groups, b0 = 4 * group + wave;
   acc4 acc[NB][KB];
 #pragma unroll
   for (int a = 0; a < NB; ++a)
@@ -715,19 +715,19 @@ __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__rest
 #pragma unroll
       for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int c = 0; c < KB; ++c) red[wave - half][a * KB + c][lane] = acc[a][c];
+        for (int c = 0; c < KB; ++c) red[(wave - half) * T + a * KB + c][lane] = acc[a][c];
     }
     __syncthreads();
     if (wave < half) {
 #pragma unroll
       for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int c = 0; c < KB; ++c) acc[a][c] += red[wave][a * KB + c][lane];
+        for (int c = 0; c < KB; ++c) acc[a][c] += red[wave * T + a * KB + c][lane];
     }
     __syncthreads();
   }
   if (wave == 0) {  // partial[group][chunk][tile][register][lane]
-    float *out = partial + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * (T * 256) + lane;
+    float *out = t.partial + ((size_t)group * (t.n_chunks * t.k_chunks) + chunk) * (T * 256) + lane;
 #pragma unroll
     for (int a = 0; a < NB; ++a)
 #pragma unroll
@@ -737,15 +737,32 @@ __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const float *__rest
   }
 }
 
+// Two gradients a launch: the workgroups from first_blocks on work on the second, whose rows come in while the first one's sums are added up.  (A
+// training step of two layers on 13,800 nodes, 69 -> 32 -> 6: 17.7 us in four launches, 11.4 in two.)
+__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
+  __shared__ acc4 red[2 * 16][64];
+  const bool other = (int)blockIdx.x >= first_blocks;
+  const WeightGradTask &t = other ? second : first;
+  const int at = other ? blockIdx.x - first_blocks : blockIdx.x, group = at % t.groups, chunk = at / t.groups;
+#define TILE(NB_, KB_) case NB_ * 8 + KB_: weight_grad_tile<NB_, KB_>(t, group, chunk, red); break
+  switch (t.nb * 8 + t.kb) {
+    TILE(1, 1); TILE(1, 2); TILE(1, 3); TILE(1, 4); TILE(2, 1); TILE(2, 2); TILE(2, 3); TILE(2, 4);
+    TILE(3, 1); TILE(3, 2); TILE(3, 3); TILE(3, 4); TILE(4, 1); TILE(4, 2); TILE(4, 3); TILE(4, 4);
+  }
+#undef TILE
+}
+
 // Adds the groups' tiles: one workgroup per register of a tile, the groups dealt to its four wavefronts, eight loads of each in flight (four: 10 us
 // for 256 groups of 64 x 128).
-__global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float *__restrict__ partial, int groups, int chunks,
-                                                                 int k_chunks, int NB, int KB, int N, int K,
-                                                                 float *__restrict__ Y) {
+__global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
+  const bool other = (int)blockIdx.x >= first_blocks;
+  const WeightGradTask &t = other ? second : first;
+  const int at = other ? blockIdx.x - first_blocks : blockIdx.x, NB = t.nb, KB = t.kb, N = t.N, K = t.K, groups = t.groups, k_chunks = t.k_chunks;
+  const int chunks = t.n_chunks * k_chunks;
   __shared__ float red[3][64];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
-  const int T = NB * KB, chunk = blockIdx.y, reg = blockIdx.x;
-  const float *p = partial + (size_t)chunk * (T * 256) + reg * 64 + lane;
+  const int T = NB * KB, chunk = at / (4 * T), reg = at % (4 * T);
+  const float *p = t.partial + (size_t)chunk * (T * 256) + reg * 64 + lane;
   const size_t stride = (size_t)chunks * (T * 256);
   float s = 0.f;
   for (int g = wave; g < groups; g += 32) {
@@ -765,20 +782,23 @@ __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float *__
   const int r = reg % 4, kb = (reg / 4) % KB, nb = reg / 4 / KB;
   const int i = 4 * h + r;  // row of the 16 x 16 block that register r of lane (j, h) holds
   const int n = min(chunk / k_chunks * 16 * NB + NB * i, N - NB) + nb, k = min(chunk % k_chunks * 16 * KB + KB * j, K - KB) + kb;
-  Y[(size_t)n * K + k] = s;
+  t.Y[(size_t)n * K + k] = s;
 }
 
 // The same for few rows in one launch: a workgroup of sixteen wavefronts per 16 x 16 tile of Y (v_mfma_f32_16x16x4_f32, so that
 // there are tiles enough) and no partial sums in memory.  What counts is the chain of loads: a wavefront keeps sixteen steps of four
-// rows in flight, eight being multiplied and the next eight on their way.  Two launches / this one, us: 7 x 32,
-// 1,000 rows 6.3 / 3.8, 4,096 7.2 / 8.0, 8,192 9.8 / 14; 32 x 500, 3,000 rows 12.0 / 9.0; 128 x 512, 4,096 rows 20.9 / 11.2 -- and a launch less for
-// the host, which is what a small model waits for.
-__global__ __launch_bounds__(1024, 4) void weight_grad_few_kernel(const float *__restrict__ G, int N, const float *__restrict__ X, int K, int M,
-                                                                  int k_tiles, float *__restrict__ Y) {
+// rows in flight, eight being multiplied and the next eight on their way.  This / weight_grad_kernel and its sums, us: 16 x 40, 1,000 rows 5.8 / 7.4,
+// 64 x 100, 2,000 rows 8.7 / 10.1, 7 x 32, 3,000 rows 8.0 / 7.0, 32 x 500, 3,000 rows 12.2 / 9.1, 32 x 100, 4,096 rows 14.3 / 7.9 -- and a launch less for
+// the host, 3.5 us, which is what a small model waits for.
+__global__ __launch_bounds__(1024, 4) void weight_grad_few_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
   constexpr int W = 16, U = 8;
   __shared__ float red[W][4][64];
+  const bool other = (int)blockIdx.x >= first_blocks;
+  const WeightGradTask &t = other ? second : first;
+  const float *__restrict__ G = t.G, *__restrict__ X = t.X;
+  const int at = other ? blockIdx.x - first_blocks : blockIdx.x, N = t.N, K = t.K, M = t.M;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
-  const int n0 = blockIdx.x / k_tiles * 16, k0 = blockIdx.x % k_tiles * 16;
+  const int n0 = at / t.k_chunks * 16, k0 = at % t.k_chunks * 16;
   // rows past the last one lie past the end of both buffers: their loads return zeros
   const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(G), 0, M * N * 4, 0x00020000),
                                xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(X), 0, M * K * 4, 0x00020000);
@@ -811,16 +831,22 @@ __global__ __launch_bounds__(1024, 4) void weight_grad_few_kernel(const float *_
 #pragma unroll
   for (int w = 1; w < W; ++w) s += red[w][wave][lane];
   const int n = n0 + 4 * h + wave, k = k0 + j;
-  if (n < N && k < K) Y[(size_t)n * K + k] = s;
+  if (n < N && k < K) t.Y[(size_t)n * K + k] = s;
 }
 
-// How launch_weight_grad cuts the product: chunks of Y, groups of rows.
-WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
-  WeightGradPlan p;
+// How launch_weight_grads cuts a product: chunks of Y, groups of rows.
+WeightGradTask plan_weight_grad(int M, int N, int K, int compute_units) {
+  WeightGradTask p;
+  p.M = M;
+  p.N = N;
+  p.K = K;
   // (some more tiles than compute units; 32-bit offsets, with a thousand rows past the end)
   p.few = M <= kWgFewRows && ((N + 15) / 16) * ((K + 15) / 16) <= 2 * compute_units && std::max(N, K) <= 16384;
-  p.partial_floats = 0;
-  if (p.few) return p;
+  if (p.few) {
+    p.n_chunks = (N + 15) / 16;
+    p.k_chunks = (K + 15) / 16;
+    return p;
+  }
   // chunks of up to 64 columns of both, evenly (300 = 5 x 64, 128 = 2 x 64, 40 = 48)
   auto cut = [](int width, int &chunks, int &blocks) {
     chunks = (width + 63) / 64;
@@ -829,33 +855,32 @@ WeightGradPlan plan_weight_grad(int M, int N, int K, int compute_units) {
   };
   cut(N, p.n_chunks, p.nb);
   cut(K, p.k_chunks, p.kb);
-  const int chunks = p.n_chunks * p.k_chunks;
   // two workgroups per compute unit; a wavefront has a block of rows or more
-  const int blocks = (M + kWgRows - 1) / kWgRows;
   // (a multiple of 8: the chunks of a block of rows on one XCD, whose L2 has the other operand and the lines two chunks share)
+  const int chunks = p.n_chunks * p.k_chunks, blocks = (M + kWgRows - 1) / kWgRows;
   p.groups = std::max(1, std::min(std::max(1, 2 * compute_units / chunks), (blocks + 3) / 4));
   if (p.groups > 8) p.groups = p.groups / 8 * 8;
-  p.partial_floats = (size_t)p.groups * chunks * p.nb * p.kb * 256;
   return p;
 }
 
-hipError_t launch_weight_grad(const WeightGradPlan &p, const float *G, int N, const float *X, int K, int M, float *partial, float *Y, hipStream_t st) {
-  if (p.few) {
-    const int k_tiles = (K + 15) / 16, n_tiles = (N + 15) / 16;
-    hipLaunchKernelGGL(weight_grad_few_kernel, dim3(k_tiles * n_tiles), dim3(1024), 0, st, G, N, X, K, M, k_tiles, Y);
+// One gradient, or (second not null) two that share their launches where both are of few rows, or both are not.
+hipError_t launch_weight_grads(const WeightGradTask &first, const WeightGradTask *second, hipStream_t st) {
+  if (second && second->few != first.few) {
+    const hipError_t err = launch_weight_grads(first, nullptr, st);
+    return err != hipSuccess ? err : launch_weight_grads(*second, nullptr, st);
+  }
+  const WeightGradTask none;
+  const WeightGradTask &b = second ? *second : none;
+  const int first_blocks = first.blocks(), blocks = first_blocks + (second ? b.blocks() : 0);
+  if (first.few) {
+    hipLaunchKernelGGL(weight_grad_few_kernel, dim3(blocks), dim3(1024), 0, st, first, b, first_blocks);
     return hipGetLastError();
   }
-  const int chunks = p.n_chunks * p.k_chunks;
-  const dim3 grid(p.groups, chunks);
-#define CALL2(NB_, KB_) hipLaunchKernelGGL((weight_grad_kernel<NB_, KB_>), grid, dim3(256), 0, st, G, N, X, K, M, p.k_chunks, partial)
-#define CALL(NB_) do { switch (p.kb) { case 1: CALL2(NB_, 1); break; case 2: CALL2(NB_, 2); break; case 3: CALL2(NB_, 3); break; default: CALL2(NB_, 4); } } while (0)
-  switch (p.nb) { case 1: CALL(1); break; case 2: CALL(2); break; case 3: CALL(3); break; default: CALL(4); }
-#undef CALL
-#undef CALL2
-  hipError_t err = hipGetLastError();
+  hipLaunchKernelGGL(weight_grad_kernel, dim3(blocks), dim3(256), 0, st, first, b, first_blocks);
+  const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3(p.nb * p.kb * 4, chunks), dim3(256), 0, st, partial, p.groups, chunks, p.k_chunks,
-                     p.nb, p.kb, N, K, Y);
+  auto registers = [](const WeightGradTask &t) { return t.nb * t.kb * 4 * t.n_chunks * t.k_chunks; };
+  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3(registers(first) + (second ? registers(b) : 0)), dim3(256), 0, st, first, b, registers(first));
   return hipGetLastError();
 }
 

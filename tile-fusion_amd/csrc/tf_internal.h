@@ -93,11 +93,15 @@ struct GemmOut {
   int of_rows = 0;              // rows of the whole product where it comes in parts: all are computed by the same kernel (0: its own)
 };
 
-// How launch_weight_grad cuts Y = G^T X (tf_dense.hip).
-struct WeightGradPlan {
-  bool few;  // in one launch, without a workspace; the cuts below are not set
-  int nb, kb, n_chunks, k_chunks, groups;
-  size_t partial_floats;
+// Y = G^T X, G M x N and X M x K, and how launch_weight_grads cuts it (tf_dense.hip).
+struct WeightGradTask {
+  const float *G = nullptr, *X = nullptr;
+  float *Y = nullptr, *partial = nullptr;
+  int M = 0, N = 0, K = 0;
+  int few = 0;  // in one launch, without a workspace; of the cuts below only k_chunks is set
+  int nb = 0, kb = 0, n_chunks = 0, k_chunks = 0, groups = 0;
+  int blocks() const { return few ? n_chunks * k_chunks : groups * n_chunks * k_chunks; }  // workgroups
+  size_t partial_floats() const { return few ? 0 : (size_t)blocks() * nb * kb * 256; }
 };
 
 struct DeviceSchedule;  // device copies + workspace, defined in tf_api.cpp

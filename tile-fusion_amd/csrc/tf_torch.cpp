@@ -308,16 +308,31 @@ Tensor gemm(const Tensor &t, const Tensor &w_, const Tensor *mask) {
 }
 
 // t^T * x: the gradient of a layer's weights (out x in), t = A^T times the gradient of the layer's output
-Tensor weight_grad(const Tensor &t, const Tensor &x_) {
-  const Tensor x = f32(x_);
+struct WeightGrad {
+  Tensor t, x, out, ws;
+  WeightGrad(const Tensor &t_, const Tensor &x_) : t(t_), x(f32(x_)) {
+    const int M = (int)t.size(0), N = (int)t.size(1), K = (int)x.size(1);
+    out = at::empty({N, K}, t.options());
+    const int64_t floats = (int64_t)(tf_weight_grad_workspace(M, N, K) / sizeof(float));
+    if (floats > 0) ws = at::empty({floats}, t.options());
+  }
+  float *workspace() const { return ws.defined() ? ws.data_ptr<float>() : nullptr; }
+};
+Tensor weight_grad(const Tensor &t, const Tensor &x) {
   c10::OptionalDeviceGuard guard(t.device());
-  const int M = (int)t.size(0), N = (int)t.size(1), K = (int)x.size(1);
-  Tensor out = at::empty({N, K}, t.options());
-  const int64_t floats = (int64_t)(tf_weight_grad_workspace(M, N, K) / sizeof(float));
-  const Tensor ws = floats > 0 ? at::empty({floats}, t.options()) : Tensor();
-  Dense tb(t), xb(x), ob(out);
-  check(tf_weight_grad(tb, xb, ob, floats > 0 ? ws.data_ptr<float>() : nullptr, stream_of(t)));
-  return out;
+  const WeightGrad w(t, x);
+  Dense tb(w.t), xb(w.x), ob(w.out);
+  check(tf_weight_grad(tb, xb, ob, w.workspace(), stream_of(t)));
+  return w.out;
+}
+// both layers' at once
+void weight_grads(const Tensor &t1, const Tensor &x1, const Tensor &t2, const Tensor &x2, Tensor *g1, Tensor *g2) {
+  c10::OptionalDeviceGuard guard(t1.device());
+  const WeightGrad a(t1, x1), b(t2, x2);
+  Dense ta(a.t), xa(a.x), oa(a.out), tb(b.t), xb(b.x), ob(b.out);
+  check(tf_weight_grad_pair(ta, xa, oa, a.workspace(), tb, xb, ob, b.workspace(), stream_of(t1)));
+  *g1 = a.out;
+  *g2 = b.out;
 }
 
 // ---- autograd ------------------------------------------------------------------------------------
@@ -376,6 +391,12 @@ struct TwoLayers : public torch::autograd::Function<TwoLayers> {
     const AdjacencyPtr at = transpose_of(held(ctx->saved_data["adj"]));
     Tensor gx, g1, g2;
     const Tensor T = spmm(*at, grads[0]);
+    if (want_1 && want_2) {
+      const Tensor T1 = spmm(*at, gemm(T, w2, &hidden));
+      if (want_x) gx = gemm(T1, w1, nullptr);
+      weight_grads(T1, x, T, hidden, &g1, &g2);
+      return {Tensor(), gx, g1, g2};
+    }
     if (want_2) g2 = weight_grad(T, hidden);
     if (want_x || want_1) layer_gradients(at, gemm(T, w2, &hidden), x, w1, want_x, want_1, &gx, &g1);
     return {Tensor(), gx, g1, g2};
