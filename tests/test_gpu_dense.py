@@ -344,6 +344,37 @@ def test_layer_in_one_launch(gpu, tf, M, K, N, listed):
         assert rel(D.to_numpy(), np.maximum(ref, 0) if flags & RELU else ref) <= 1e-5, flags
 
 
+@pytest.mark.parametrize("M,K,N,one", [(19999, 32, 97, True), (20000, 32, 97, False), (20000, 31, 97, True), (20001, 128, 128, False), (23999, 64, 96, True),
+                                       (29999, 64, 96, True), (30000, 64, 96, False), (30000, 65, 97, False), (30001, 44, 65, True), (30003, 32, 65, False)])
+def test_layer_beyond_64_columns(gpu, tf, M, K, N, one):
+    """One launch or two, on either side of the row counts and widths between them: the same sums, a value that is not finite included."""
+    say(f"beyond 64 columns M={M} {K}x{N}")
+    rng = np.random.default_rng(M + K + N)
+    A = sp.csr_matrix(tf.workloads.erdos_renyi_gcn(M, 4.0, seed=5), dtype=np.float32)
+    X, W, D0 = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    S.set_profiling(True)
+    for bad in (None, np.inf, np.nan):
+        if bad is not None:
+            X[M // 2, K - 1] = bad
+        with np.errstate(invalid="ignore"):
+            want = A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))
+        for flags in (0, C_TRANSPOSED, 1, RELU):
+            Wd = tf.DenseMatrix.from_numpy(np.ascontiguousarray(W.T) if flags & C_TRANSPOSED else W)
+            D = tf.DenseMatrix.from_numpy(D0)
+            Xd = tf.DenseMatrix.from_numpy(X)
+            assert tf.lib().tf_gemm_spmm(Ah.to_device().h, Xd.h, Wd.h, D.h, S.h, flags, None) == 0
+            tf.device_synchronize()
+            assert ("spmm_gemm_kernel" in [n for n, _ in S.profile()]) == one
+            ref = want + D0 if flags & 1 else want
+            got, fine = D.to_numpy(), np.isfinite(ref).all(axis=1)  # a row that reads the value is not finite anywhere
+            if bad is not None and not flags & RELU:
+                assert not fine.all() and not np.isfinite(got[~fine]).any()
+            # K products and the row's entries, each rounded once, in single precision
+            assert rel(got[fine], np.maximum(ref, 0)[fine] if flags & RELU else ref[fine]) <= 1e-6, flags
+
+
 @pytest.mark.parametrize("M,K,N", [(500, 2544, 1273), (500, 2545, 1273), (500, 3000, 2000), (60, 6001, 3001)])
 def test_layer_of_few_rows_and_wide_features(gpu, tf, M, K, N):
     """Up to the K whose rows fill LDS in one launch, and beyond it."""

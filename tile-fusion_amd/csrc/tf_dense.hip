@@ -522,10 +522,11 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   // gemm_split_kernel with W N x K: 12,500 rows 300 x 64 10.5 / 12.9; 24,000 rows 64 x 128 11.9 / 10.1, 128 x 128 17.2 / 14.4, 128 x 64 10.0 / 10.1,
   // 300 x 128 32.2 / 23.1; 50,000 rows 128 x 64 15.4 / 15.1, 32 x 64 8.6 / 8.3; 100,000 rows 32 x 64 12.0 / 12.4, 64 x 64 16.4 / 15.2, 128 x 64 25.0 / 20.5,
   // 300 x 64 51.4 / 41.4, 128 x 128 43.6 / 30.3, 300 x 128 88.3 / 67.1; 262,144 rows 128 x 40 47.2 / 38.0, 128 x 128 81 / 63; 200,000 rows
-  // 256 x 128 119 / 99, two panels; 60,000 rows 300 x 300 172 / 93, five; but 150,000 rows 512 x 128 173 / 194, four panels of 32).
+  // 256 x 128 119 / 99, two panels; 60,000 rows 300 x 300 172 / 93, five; but 150,000 rows 512 x 128 173 / 194, four panels of 32;
+  // 60,000 rows 8 x 66 8.5 / 9.0, 16 x 96 8.5 / 9.3, 24 x 96 10.1 / 9.7, 24 x 128 12.4 / 11.0, 180,000 rows 24 x 128 31.9 / 26.1: a step takes 32 k).
   // Widths are cut into equal panels that fit LDS; X is read once per panel, by compute units of the same XCD at about the same time.
   const int all_rows = std::max(n_rows, how.of_rows);
-  const bool on_bf16 = (N > 64 ? all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K >= 64 && all_rows >= 150LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
+  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K >= 64 && all_rows >= 150LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
   const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
   const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
   int unit = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;

@@ -118,6 +118,12 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    20,000 rows 64 x 64 10.2 / 20.1, 128 x 128 30 / 36, 200 x 128 47 / 43, 100 x 16 14.0 / 11.9.  With more rows the intermediate's
 //    trip does, as long as W's trips from L2 do not: 200,000 rows 64 x 64 93 / 113, 700 x 700 grid 30 x 30 52 / 78, 64 x 64
 //    127 / 136, 128 x 128 408 / 316; streamed tiles stay the faster way at 64 x 64 (262,144-row band 79 / 60).
+//    Beyond 64 columns the dense product of a launch of its own runs on the bf16 cores and this one's does not, so from 20,000 rows on
+//    (65 to 96 columns: 30,000) only what would be A (B C) otherwise stays in one launch, and gathers of less than 32 columns (one launch
+//    / two; 16,000 rows of 10 entries 64 x 128 16.9 / 15.5, 140 x 143 grid 14.8 / 15.6, 128 x 128 23.6 / 22.2; 21,000 rows of 10
+//    32 x 128 17.7 / 14.5, 128 x 128 32.7 / 27.1; 100,000 rows of 5 32 x 128 37.4 / 29.0, 64 x 128 62 / 45, 64 x 96 52 / 42, 48 x 66
+//    44 / 51, 16 x 96 23.0 / 23.3; 150 x 150 grid 64 x 96 15.1 / 14.3; 180 x 180 16.9 / 16.4, 64 x 128 20.6 / 18.9, 32 x 128 14.4 /
+//    15.0, 16 x 96 9.0 / 11.5; 250 x 250 64 x 128 32.5 / 24.6).
 //  * as (A B) C in two launches where K is two thirds of N or less: the gathers are K columns wide instead of N.  K = 32, N = 128: 700 x 700
 //    grid 219 us -> 118 us (136 in one launch), 262,144 rows of 16 in a band of 32 (streamed tiles) 86 -> 64 us.
 //  * as A (B C) where tiles need padded copies of B or column panels of D (262,144-row band, 250 x 32: 327 us, as two
@@ -139,8 +145,9 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     const bool padded = K != S->opts.K || N != S->opts.N, partly = (long long)S->fused_ids.size() * 8 < 7LL * S->L;
     const bool streamed = tiled && S->gemm_stream && !padded && !partly;
     S->one_launch = tf::spmm_gemm_fits(S->L, K, N) &&
-                    (M < 24000 ? (K <= 128 && (K <= 2 * N || M < 10000)) || (K <= 2 * N && work <= 2000000)
-                               : K <= 64 && K <= N && (N <= 64 || M <= 150000) && !(streamed && K > 32));
+                    (M < (N <= 96 ? 24000 : 20000) ? (K <= 128 && (K <= 2 * N || M < 10000)) || (K <= 2 * N && work <= 2000000)
+                                                   : K <= 64 && K <= N && (N <= 64 || (M <= 150000 && (K < 32 || 3 * K > 2 * N || (N <= 96 && M < 30000)))) &&
+                                                         !(streamed && K > 32));
     S->spmm_first = S->one_launch || 3LL * K <= 2LL * N;
     want = S->spmm_first || (tiled && (padded || !S->gemm_regw || partly || !S->gemm_stream));
     if (S->one_launch) {  // hub rows known before any list is made (see below)
