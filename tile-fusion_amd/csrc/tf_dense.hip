@@ -408,6 +408,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
   // A step: its values become parts, whereupon their registers take the values A steps on, of this block or the next.
   auto step = [&](int s, f4v (&o)[2], const float *from, int ahead, float in_scale) __attribute__((always_inline)) {
     if (s == S - 1 && K % 4 != 0) {
+      asm volatile("");  // (a branch: as selects these were 24 of a step's 138 vector instructions, 84 with split8's pairs)
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
         o[w] = d[w] & 1 ? f4v{o[w][1], o[w][2], o[w][3], 0.f} : o[w];

@@ -934,15 +934,7 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
     // in the order r ^ 4 g: the four that a row's threads write to lie in different banks.)
     char *const xdst = reinterpret_cast<char *>(xbuf) + ((sr / 16 * 4 + sk / 8) * 16 + (sr % 16 ^ sk / 8 * 4)) * 16 + sk % 8 * 2;
     auto put_unit = [&](int buf, const fvec<4> &x) {
-      split3<bf4> p;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        __bf16 hi, mid, lo;
-        split(x.v[c], hi, mid, lo, sr / 16 % 2 ? -kSplitIn : kSplitIn);
-        p.h[c] = hi;
-        p.m[c] = mid;
-        p.l[c] = lo;
-      }
+      const split3<bf4> p = split4(x.v[0], x.v[1], x.v[2], x.v[3], sr / 16 % 2 ? -kSplitIn : kSplitIn);
       char *at = xdst + buf * (kStreamStageBytes / 2);
       *reinterpret_cast<bf4 *>(at) = p.h;
       *reinterpret_cast<bf4 *>(at + 4096) = p.m;
