@@ -64,7 +64,8 @@ def test_gemm_panel_edges(gpu, tf, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(18432, 4, 65), (18431, 4, 65), (18433, 31, 66), (24001, 33, 65), (24000, 51, 96), (18447, 64, 97), (50000, 65, 128),
                                    (30001, 128, 128), (18437, 161, 72), (18439, 213, 128), (10241, 214, 129), (10239, 214, 129), (10240, 300, 100),
                                    (10243, 426, 65), (18434, 427, 65), (38400, 64, 33), (38399, 64, 33), (38409, 96, 48), (49999, 130, 64),
-                                   (38403, 427, 40), (38401, 853, 36), (38402, 854, 36), (262145, 67, 35)])
+                                   (38403, 427, 40), (38401, 853, 36), (38402, 854, 36), (262145, 67, 35),
+                                   (18434, 16, 70), (18435, 17, 70), (38405, 48, 33), (38405, 49, 33), (38401, 63, 64)])
 @pytest.mark.parametrize("w_t", [False, True])
 def test_gemm_on_bf16_cores(gpu, tf, M, K, N, w_t):
     """Products as sums of bf16 parts, either side of where they begin and of what LDS holds: no further from float64 than fp32 sums, for

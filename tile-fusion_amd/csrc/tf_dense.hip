@@ -516,7 +516,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   // single values where W is K x N (us, gemm_panel_kernel / gemm_direct_kernel, at 8,000 / 16,000 / 30,000 rows: 128 x 128 9.3 / 8.1 (K x N: 9.3 / 11.6),
   // 11.0 / 13.8, 16.8 / 23; 64 x 64 5.0 / 4.6 (5.0 / 5.7), 5.0 / 6.0, 6.7 / 9.0; 500 x 32, 30,000 rows 17.6 / 20.8; 40 x 7 6.7 / 4.2).
   // The bf16 cores pay where the fp32 ones were what a product waited for: beyond 64 columns from 72 rows per compute unit on, where splitting W no
-  // longer counts (40 where gemm_panel_kernel has more than 213 values of k for each), for 33 to 64 columns from 150 on where K is not small (us,
+  // longer counts (40 where gemm_panel_kernel has more than 213 values of k for each), for 33 to 64 columns from 150 on where K is beyond 48 (us,
   // operands in L2 and the Infinity Cache, gemm_panel_kernel / gemm_split_kernel: 13,000 rows 128 x 128 10.8 / 11.1, 300 x 128 19.2 / 16.6, 128 x 64
   // 7.5 / 7.8; 16,000 rows 128 x 128 10.8 / 11.0, 20,000 rows 128 x 128 16.2 / 13.3, 300 x 128 31.5 / 19.7, 64 x 100 10.7 / 8.9; 30,000 rows 128 x 64
   // 10.5 / 9.8, 64 x 64 7.8 / 8.1; 40,000 rows 64 x 64 9.1 / 8.3, 128 x 64 13.9 / 12.1; operands in no cache, gemm_panel_kernel /
@@ -524,10 +524,11 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   // 300 x 128 32.2 / 23.1; 50,000 rows 128 x 64 15.4 / 15.1, 32 x 64 8.6 / 8.3; 100,000 rows 32 x 64 12.0 / 12.4, 64 x 64 16.4 / 15.2, 128 x 64 25.0 / 20.5,
   // 300 x 64 51.4 / 41.4, 128 x 128 43.6 / 30.3, 300 x 128 88.3 / 67.1; 262,144 rows 128 x 40 47.2 / 38.0, 128 x 128 81 / 63; 200,000 rows
   // 256 x 128 119 / 99, two panels; 60,000 rows 300 x 300 172 / 93, five; but 150,000 rows 512 x 128 173 / 194, four panels of 32;
-  // 60,000 rows 8 x 66 8.5 / 9.0, 16 x 96 8.5 / 9.3, 24 x 96 10.1 / 9.7, 24 x 128 12.4 / 11.0, 180,000 rows 24 x 128 31.9 / 26.1: a step takes 32 k).
+  // 60,000 rows 8 x 66 8.5 / 9.0, 16 x 96 8.5 / 9.3, 24 x 96 10.1 / 9.7, 24 x 128 12.4 / 11.0, 180,000 rows 24 x 128 31.9 / 26.1: a step takes 32 k;
+  // 131,072 rows 40 x 64 16.6 / 18.0, 48 x 64 17.0 / 17.1, 60 x 64 20.0 / 17.8, 60 x 40 19.1 / 15.9, 40,000 rows 60 x 64 10.4 / 8.9).
   // Widths are cut into equal panels that fit LDS; X is read once per panel, by compute units of the same XCD at about the same time.
   const int all_rows = std::max(n_rows, how.of_rows);
-  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K >= 64 && all_rows >= 150LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
+  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K > 48 && all_rows >= 150LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
   const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
   const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
   int unit = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;
