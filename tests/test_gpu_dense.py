@@ -96,6 +96,50 @@ def test_gemm_on_bf16_cores(gpu, tf, M, K, N, w_t):
         assert np.all(np.abs(got[M // 2] - want[M // 2]) <= (K + 8) * 2.0 ** -24 * np.abs(want[M // 2]).max())
 
 
+def few_values(rng, M, K, q):
+    """Rows of q values at random places (all K where q is K), the rest zeros: what bag-of-words features are."""
+    X = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    if q < K:
+        keep = np.zeros((M, K), bool)
+        np.put_along_axis(keep, np.argsort(rng.random((M, K)), axis=1)[:, :q], True, 1)
+        X[~keep] = 0
+    return X
+
+
+def fp32_sums(X, W):
+    """X W as a chain of fp32 fmas, each rounded to nearest."""
+    s = np.zeros((X.shape[0], W.shape[1]), np.float32)
+    for k in range(X.shape[1]):
+        s = (s + X[:, k:k + 1].astype(np.float64) * W[k].astype(np.float64)).astype(np.float32)
+    return s
+
+
+def no_further_than_fp32(got, X, W, q):
+    """The error against float64 over the sum of magnitudes: its root mean square is at most that of fp32 sums; one product is rounded once, and sums of more
+    lose less than 2^-23 of themselves with every further value and are rounded once at the end.  (2^-6 for what is left out and for second roundings.)"""
+    def error(y, X):
+        size = np.abs(X).astype(np.float64) @ np.abs(W).astype(np.float64)
+        e = np.abs(y - X.astype(np.float64) @ W.astype(np.float64)) / np.maximum(size, 1e-300)
+        return e[size > 0]
+    e, part = error(got, X), slice(0, 6000)
+    fp32 = error(fp32_sums(X[part], W), X[part])
+    print(f"  {q} values: largest {e.max():.3g} ({fp32.max():.3g}), rms {np.sqrt((e ** 2).mean()):.4g} ({np.sqrt((fp32 ** 2).mean()):.4g})", flush=True)
+    assert np.sqrt((e ** 2).mean()) <= 1.02 * np.sqrt((fp32 ** 2).mean())  # (two samples of some 400,000 values or more: 0.3 %)
+    assert e.max() <= (2 * q - 1) * 2.0 ** -24 * (1 + 2.0 ** -6)
+
+
+@pytest.mark.parametrize("M,K,N", [(18433, 128, 128), (40000, 64, 64), (30000, 301, 100)])
+@pytest.mark.parametrize("q", [1, 2, 3, 4, 8, 64])
+def test_gemm_of_few_features_a_row(gpu, tf, M, K, N, q):
+    say(f"gemm of rows of few features {M} x {K} x {N}, {q} a row")
+    rng = np.random.default_rng(M + K + q)
+    X, W = few_values(rng, M, K, q), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    Xd, Wd, Y = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(W), tf.DenseMatrix(M, N)
+    assert tf.lib().tf_gemm_ex(Xd.h, Wd.h, Y.h, None, 0, None) == 0
+    tf.device_synchronize()
+    no_further_than_fp32(Y.to_numpy(), X, W, q)
+
+
 @pytest.mark.parametrize("K,N", [(128, 128), (120, 96), (64, 64), (40, 32), (136, 32), (256, 64), (256, 128)])
 def test_streamed_runs_on_bf16_cores(gpu, tf, K, N):
     """Banded rows whose intermediate never leaves LDS: within fp32's rounding of float64, values of many sizes, and what is not finite

@@ -389,6 +389,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const bf8 wh = w[t * 192], wm = w[t * 192 + 64], wlo = w[t * 192 + 128];
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, wm, small[t], 0, 0, 0);
+      small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, wlo, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, wh, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, wlo, small[t], 0, 0, 0);
       small[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, wm, small[t], 0, 0, 0);
@@ -675,6 +677,8 @@ __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int gr
 #pragma unroll
       for (int c = 0; c < KB; ++c) {
         acc4 s = 0.f;  // (the block's own sum: the long sum is rounded once per 32 rows)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].m, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].l, s, 0, 0, 0);
         s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].h, s, 0, 0, 0);
         s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].l, s, 0, 0, 0);
         s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].m, s, 0, 0, 0);

@@ -196,11 +196,14 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 
 // ---- fp32 products on the bf16 matrix cores ----
 //
-// A float is the sum of three bf16 of eight significant bits each, x = h + m + l, every difference exact.  The product of two such
-// sums without the three terms below 2^-26 of it (m l, l m, l l) is six bf16 products, which v_mfma_f32_16x16x32_bf16 adds up in fp32 in 6 x 16
-// cycles per 32 values of k; v_mfma_f32_16x16x4_f32 takes 8 x 32.  Relative error against 64 bits, values in [0, 1) times values in [-0.2, 0.2),
-// K = 32 / 64 / 128 / 256 / 512, in e-7: fp32 cores 1.0 / 1.6 / 2.2 / 3.0 / 3.7, this in one accumulator 0.37 / 1.1 / 1.7 / 2.4 / 3.0, with
-// h h in one and the five small terms in another 0.36 / 0.47 / 0.62 / 0.86 / 1.05 (the large sum is then rounded once per 32 values of k).
+// A float is the sum of three bf16 of eight significant bits each, x = h + m + l, every difference exact: m is below 2^-8 of x, l below 2^-16.
+// The product of two such sums without l l, below 2^-32 of it, is eight bf16 products, which v_mfma_f32_16x16x32_bf16 adds up in fp32 in
+// 8 x 16 cycles per 32 values of k; v_mfma_f32_16x16x4_f32 takes 8 x 32.  (m l and l m reach 4.9e-8 of a product together: without them a row with one
+// value that is not zero came out up to 1.1e-7 off where a rounded product is 6.0e-8 off.)  h h is added up in one accumulator and the seven small terms
+// in another: the cores cut sums off instead of rounding them, and the large sum is then cut once per 32 values of k, and not at all
+// while it has 24 bits.  Root mean square of the error over the sum of magnitudes, values in [-1, 1], K = 128, in e-8, for 1 / 2 / 4 / 8 / 128 values
+// that are not zero: fp32 cores 2.53 / 2.54 / 2.53 / 2.48 / 2.40, this 2.53 / 2.09 / 1.64 / 1.26 / 0.70; largest of five million 6.0 / 11.3 / 17 / 22 / 30 and
+// 6.0 / 15.0 / 14 / 15 / 9.
 // The cores take denormal bf16 for zero: both operands are made 2^20 times larger on the way in, so that the parts of every
 // normal float are normal, and sums 2^-40 times smaller on the way out.  Infinities, NaN and sums beyond 2^88 come out infinite or NaN: the
 // caller looks for those and computes such a block again on the fp32 cores.

@@ -1005,6 +1005,8 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
                   for (int u = 0; u < PAIR; ++u)
                     if ((b0 + u) * RG < 4) acc[c][b0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u].*xpart, wp.*wpart, acc[c][b0 + u], 0, 0, 0);
                 };
+                add(&split3<bf8>::l, &split3<bf8>::m);
+                add(&split3<bf8>::m, &split3<bf8>::l);
                 add(&split3<bf8>::l, &split3<bf8>::h);
                 add(&split3<bf8>::h, &split3<bf8>::l);
                 add(&split3<bf8>::m, &split3<bf8>::m);
