@@ -228,6 +228,30 @@ def test_weight_gradient_on_bf16_cores(gpu, tf, M, N, K):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and ok.all() == (not odd)
 
 
+@pytest.mark.parametrize("M,N,K", [(5000, 64, 100), (40000, 40, 128)])
+@pytest.mark.parametrize("q", [1, 2, 4, 8, 64])
+def test_weight_gradient_of_rare_features(gpu, tf, M, N, K, q):
+    """Columns of X of q values in all: no further from float64 than rounded fp32 products added up in fp32."""
+    say(f"weight gradient of rare features {M} rows, {N} x {K}, {q} a column")
+    rng = np.random.default_rng(M + q)
+    G, X = rng.uniform(-1, 1, (M, N)).astype(np.float32), np.ascontiguousarray(few_values(rng, K, M, q).T)
+    lib = tf.lib()
+    ws = tf.DenseMatrix(1, max(1, lib.tf_weight_grad_workspace(M, N, K) // 4))
+    Gd, Xd, Y = tf.DenseMatrix.from_numpy(G), tf.DenseMatrix.from_numpy(X), tf.DenseMatrix(N, K)
+    assert lib.tf_weight_grad(Gd.h, Xd.h, Y.h, C.c_void_p(ws.device_ptr()), None) == 0
+    tf.device_synchronize()
+    rows = np.stack([np.flatnonzero(X[:, k]) for k in range(K)])                             # K x q
+    products = G[rows].astype(np.float64) * X[rows, np.arange(K)[:, None]][:, :, None]       # K x q x N
+    want, size = products.sum(1).T, np.abs(products).sum(1).T
+    fp32 = np.zeros((K, N), np.float32)
+    for p in np.moveaxis(products.astype(np.float32), 1, 0):
+        fp32 += p
+    e, ref = np.abs(Y.to_numpy() - want) / size, np.abs(fp32.T - want) / size
+    say(f"  largest {e.max():.3g} ({ref.max():.3g}), rms {np.sqrt((e ** 2).mean()):.4g} ({np.sqrt((ref ** 2).mean()):.4g})")
+    assert e.max() <= q * 2.0 ** -24 * (1 + 2.0 ** -6)  # every product and every sum rounded once
+    assert np.sqrt((e ** 2).mean()) <= 1.05 * np.sqrt((ref ** 2).mean())  # (of some 6,000 values each: 1.3 %)
+
+
 @pytest.mark.parametrize("M1,M2", [(100, 100), (3072, 3072), (3073, 3073), (20001, 20001), (3000, 5000), (5000, 3000)])
 def test_two_weight_gradients_in_one_call(gpu, tf, M1, M2):
     """Sharing their launches changes no bit of either, of few rows and of many (and of one and the other)."""

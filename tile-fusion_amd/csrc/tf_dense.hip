@@ -676,17 +676,18 @@ __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int gr
     for (int a = 0; a < NB; ++a)
 #pragma unroll
       for (int c = 0; c < KB; ++c) {
-        acc4 s = 0.f;  // (the block's own sum: the long sum is rounded once per 32 rows)
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].m, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].l, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].h, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].l, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].m, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].h, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].m, s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].h, s, 0, 0, 0);
+        // The block's own sums, the large terms by themselves: h h of a few rows is exact, and what is left is rounded to nearest here, once per 32 rows.
+        acc4 small = 0.f;
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].m, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].l, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].l, xs[c].h, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].l, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].m, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].m, xs[c].h, small, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].m, small, 0, 0, 0);
+        const acc4 big = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gs[a].h, xs[c].h, acc4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[a][c][r] = __builtin_fmaf(sign, s[r], acc[a][c][r]);
+        for (int r = 0; r < 4; ++r) acc[a][c][r] = __builtin_fmaf(sign, big[r] + small[r], acc[a][c][r]);
       }
   }
   float finite = 0.f;
