@@ -164,12 +164,57 @@ static int hubs_and_columns() {
   return bad;
 }
 
+// Streamed GeMM-SpMM runs: the last lane group's reads of a row's entries end inside the LDS that the kernel is launched with, and every
+// quarter (half) of a group's slots is read by the lane of a quad that it is passed on from.
+static int streamed_entries() {
+  int bad = 0, streamed = 0;
+  const int M = 30000;
+  std::vector<int> p(M + 1), i;
+  for (int r = 0; r < M; ++r) {
+    for (int c = r > 2 ? r - 3 : 0; c <= r + 3 && c < M; ++c) i.push_back(c);
+    p[r + 1] = (int)i.size();
+  }
+  for (int N : {32, 64, 96, 128})
+    for (int K : {8, 64, 128, 136, 256})
+      for (int budget : {65536, 102400, 163840}) {
+        tf_inspect_opts o{};
+        o.struct_size = sizeof(o);
+        o.op = TF_OP_GEMM_SPMM;
+        o.K = K;
+        o.N = N;
+        o.lds_budget_bytes = budget;
+        tf_schedule *s = nullptr;
+        if (tf_inspect(M, M, p.data(), i.data(), &o, &s)) { printf("%s\n", tf::g_err); return 1; }
+        if (s->gemm_stream) {
+          ++streamed;
+          const int lanes = N <= 32 ? 8 : N <= 64 ? 16 : 32, consumers = K <= 128 ? 8 : 4;
+          const long long scratch = tf::kStreamStageBytes + (long long)s->ring_rows * (N + 4) * 4;
+          for (int g = 0; g < consumers * 64 / lanes; ++g)
+            for (int l = 0; l < lanes; ++l) {
+              const int q = tf::stream_quarter(l, lanes);
+              for (int c = 0; c < lanes; c += 16) {
+                const int slot = c + 4 * q + 3;  // of the group's
+                if (slot >= lanes || scratch + 8LL * (g * lanes + slot + 1) > s->lds_bytes) {
+                  printf("N %d K %d budget %d: lane %d of group %d reads slot %d, LDS ends at %d\n", N, K, budget, l, g, slot, s->lds_bytes);
+                  ++bad;
+                }
+              }
+              if (4 * (l & 3) < lanes && q != (l & 3)) { printf("lane %d of %d reads quarter %d\n", l, lanes, q); ++bad; }
+            }
+        }
+        tf_schedule_free(s);
+      }
+  if (streamed < 20) { printf("%d streamed\n", streamed); ++bad; }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
     const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
                   : !strcmp(argv[k], "partial_sums") ? partial_sums()
-                  : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns() : 1;
+                  : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns()
+                  : !strcmp(argv[k], "streamed_entries") ? streamed_entries() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

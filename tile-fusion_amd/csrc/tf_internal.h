@@ -16,6 +16,9 @@ namespace tf {
 constexpr int kMaxLds = 163840;  // LDS per workgroup on gfx950
 // Streamed GeMM-SpMM runs: two buffers of 64 x 32 values of B, each as three bf16 parts.
 constexpr int kStreamStageBytes = 24576;
+// ... and a row's entries, as many slots as a group of `lanes` lanes (8, 16 or 32) has.  Lane l reads four slots from base + 4 stream_quarter(l): of each
+// sixteen entries its quad's lanes hold a quarter each, of a group's eight two lanes the same half.
+constexpr int stream_quarter(int l, int lanes) { return l & 3 & (lanes / 4 - 1); }
 
 // One fused tile = one workgroup.  The workgroup computes intermediate rows
 // [prod_begin, prod_end) into LDS, stores rows [wb_begin, wb_end) of them to the

@@ -1129,7 +1129,7 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
       const int cnt = min(LPR, rec.z - rec.y - u * LPR);
       if (u == 0 || cnt > 0) {
         scratch[glane] = make_int2(((c[u] - t.prod_begin) & ring_mask) * (ld * 4), __float_as_int(a[u]));
-        acc = lds_row_dot_quad(scratch, 0, cnt, rbase, glane & 3, acc);  // (reads up to 3 pairs past the row's: never used)
+        acc = lds_row_dot_quad(scratch, 0, cnt, rbase, stream_quarter(glane, LPR), acc);  // (slots past the row's are read and not used)
       }
     }
     if (ok) store_streaming<4>(dst, acc);
