@@ -171,6 +171,25 @@ def test_streamed_runs_on_bf16_cores(gpu, tf, K, N):
     assert np.array_equal(np.isnan(got[odd]), np.isnan(want[odd])) and not odd.all() and odd.sum() >= 3
 
 
+@pytest.mark.parametrize("K,N", [(128, 128), (120, 96), (64, 64), (40, 32), (128, 64), (64, 96), (256, 64), (256, 128), (200, 32), (136, 96)])
+@pytest.mark.parametrize("q", [1, 2, 4, 8, 64])
+def test_streamed_runs_of_few_features_a_row(gpu, tf, K, N, q):
+    """The rows of the intermediate themselves (A is the identity)."""
+    if q > K:
+        pytest.skip("fewer features")
+    say(f"streamed runs of few features a row {K} x {N}, {q} a row")
+    M = 25000
+    rng = np.random.default_rng(K + N + q)
+    X, W = few_values(rng, M, K, q), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    Ah = tf.CsrMatrix.from_scipy(sp.identity(M, dtype=np.float32, format="csr"))
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K, lds_budget_bytes=163840)
+    assert S.info()["streamed"] == 1
+    D, Xd, Wd = tf.DenseMatrix(M, N), tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(W)
+    tf.gemm_spmm(Ah.to_device(), Xd, Wd, D, S)
+    tf.device_synchronize()
+    no_further_than_fp32(D.to_numpy(), X, W, q)
+
+
 @pytest.mark.parametrize("K,N", [(129, 33), (64, 100), (18, 128)])
 def test_gemm_of_listed_rows(gpu, tf, K, N):
     """The rows an R-MAT graph reads, gathered by the product itself and stored in the order of their reads."""

@@ -880,8 +880,7 @@ __global__ __launch_bounds__(kGemmBlock) void fused_gemm_spmm_regw_kernel(
 // What bounds it: fp32 MFMAs and the consumers' FMAs share the vector pipe of a SIMD, so their times added up; the six bf16 products take 0.4
 // of the MFMA time and run beside FMAs (us, 262,144 rows of 16 in a band of 32, operands in no cache, fp32 producers / these: K = N = 128 132 / 115,
 // 256 x 128 215 / 178, 128 x 96 125 / 108, 64 x 128 125 / 111, 256 x 64 154 / 144, 128 x 64 90 / 85, 64 x 32 58 / 58).  Now the consumers: a row's
-// entries, one LDS read and four FMAs each, between two barriers.  The five small terms go to the same accumulators as the large one here
-// (registers): still closer to 64 bits than fp32 products (1.7 and 2.2e-7 at K = 128).
+// entries, one LDS read and four FMAs each, between two barriers.
 constexpr int kStreamProducers = 8;   // wavefronts
 static_assert(kStreamStageBytes == 2 * 3 * kXRows * kXChunk * 2, "two buffers of three bf16 parts");
 
@@ -912,18 +911,25 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
     constexpr int RG = CPW == 1 ? (LPR == 8 ? 4 : LPR == 16 ? 2 : 1) : 1;
     const int cb0 = RG > 1 ? wave % (NW / RG) : wave;
     const int rg = RG > 1 ? wave / (NW / RG) : 0;
-    const int sr = threadIdx.x / 8, sk = (threadIdx.x % 8) * 4;
+    // What is multiplied in one interval: SR rows by SK values of k, TB row tiles a wavefront, each with an accumulator for the large terms and one for the
+    // small ones.  Where a wavefront has a column block to itself a step's 64 rows are two halves, one after the other, so that the accumulators
+    // take the registers of four tiles and not of eight.
+    constexpr int SR = RG == 1 ? 32 : kXRows, SK = kXRows * kXChunk / SR, TB = SR / 16 / RG;
+    constexpr int KI = KS * 16 / SK;  // intervals over K for the same rows
+    static_assert(KI * (kXRows / SR) == NKC && TB >= 1, "a step is NKC intervals");
+    constexpr int AH = NKC;  // intervals whose units are on their way
+    const int sr = threadIdx.x / (SK / 4), sk = threadIdx.x % (SK / 4) * 4;
     // Always a load (of the last row / the last values of k when past the end, zeroed when it
     // is stored to LDS): a load under a condition would have to land before the next barrier.
     auto chunk_unit = [&](int ch) -> fvec<4> {
-      const int q = min(ch / NKC, S - 1), k = min((ch % NKC) * kXChunk + sk, K - 4);
-      const int row = t.prod_begin + min(q * kXRows + sr, P - 1);
+      const int q = min(ch / NKC, S - 1), k = min(ch % KI * SK + sk, K - 4);
+      const int row = t.prod_begin + min(q * kXRows + ch % NKC / KI * SR + sr, P - 1);
       return load_streaming4(B + (size_t)row * K + k);
     };
     // relu_in: B is a layer's output before its activation, max(x, 0) is applied here on its way to the MFMAs
     // (the second layer of tf_gcn_two_layers: saves a pass over the hidden layer)
     auto unit_or_zero = [&](const fvec<4> &x, int kc) -> fvec<4> {
-      fvec<4> r = kc * kXChunk + sk < K ? x : vzero<4>();
+      fvec<4> r = kc % KI * SK + sk < K ? x : vzero<4>();
       if (relu_in) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) r.v[c] = fmaxf(r.v[c], 0.f);
@@ -931,8 +937,9 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
       return r;
     };
     // Three parts of the unit in the order in which the matrix cores take them: row tile, k / 8, row, eight values of k.  (The rows of k / 8 = g
-    // in the order r ^ 4 g: the four that a row's threads write to lie in different banks.)
-    char *const xdst = reinterpret_cast<char *>(xbuf) + ((sr / 16 * 4 + sk / 8) * 16 + (sr % 16 ^ sk / 8 * 4)) * 16 + sk % 8 * 2;
+    // in the order r ^ 16 g / (SK / 8): those that a row's threads write to lie in different banks.)
+    constexpr int KG = SK / 8;
+    char *const xdst = reinterpret_cast<char *>(xbuf) + ((sr / 16 * KG + sk / 8) * 16 + (sr % 16 ^ sk / 8 * (16 / KG))) * 16 + sk % 8 * 2;
     auto put_unit = [&](int buf, const fvec<4> &x) {
       const split3<bf4> p = split4(x.v[0], x.v[1], x.v[2], x.v[3], sr / 16 % 2 ? -kSplitIn : kSplitIn);
       char *at = xdst + buf * (kStreamStageBytes / 2);
@@ -954,9 +961,9 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
           wv[c][kc][i / 4][i % 4] = (cb < CB && k < K) ? W[(size_t)k * N + 16 * cb + j] : 0.f;
         }
     const fvec<4> first = chunk_unit(0);
-    fvec<4> xs[NKC];  // xs[k]: the unit of the next interval k of a step that is not in LDS yet
+    fvec<4> xs[AH];  // xs[k % AH]: the unit of the next interval k of a step that is not in LDS yet
 #pragma unroll
-    for (int k = 0; k < NKC; ++k) xs[(k + 1) % NKC] = chunk_unit(k + 1);
+    for (int k = 0; k < AH; ++k) xs[(k + 1) % AH] = chunk_unit(k + 1);
     split3<bf8> w[CPW][NKC];
 #pragma unroll
     for (int c = 0; c < CPW; ++c)
@@ -972,80 +979,81 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
       for (int kc = 0; kc < NKC; ++kc) asm volatile("" : : "v"(w[c][kc].h), "v"(w[c][kc].m), "v"(w[c][kc].l));
     lds_barrier();
     for (int q = 0; q < S; ++q) {
-      v4f acc[CPW][4];
-#pragma unroll
-      for (int c = 0; c < CPW; ++c)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[c][b] = v4f{0.f, 0.f, 0.f, 0.f};
+      v4f big[CPW][TB], small[CPW][TB];
 #pragma unroll
       for (int kc = 0; kc < NKC; ++kc) {
-        const int ch = q * NKC + kc;
-        const bf8 *xb = xbuf + (kc & 1) * (kStreamStageBytes / 32) + (16 * h + (j ^ 4 * h));
+        const int ch = q * NKC + kc, half = kc / KI;
         // The unit of the next interval goes to the other buffer, its register takes the unit of the same interval of the next step; in front
         // of the products, which may then run on past the barrier.
-        put_unit((kc + 1) & 1, unit_or_zero(xs[(kc + 1) % NKC], (kc + 1) % NKC));
-        xs[(kc + 1) % NKC] = chunk_unit(ch + 1 + NKC);
-        if (cb0 < CB && kc * kXChunk < K) {  // uniform
-          constexpr int PAIR = RG > 1 ? 2 : 1;  // row tiles multiplied side by side
+        put_unit((kc + 1) & 1, unit_or_zero(xs[(kc + 1) % AH], (kc + 1) % NKC));
+        xs[(kc + 1) % AH] = chunk_unit(ch + 1 + AH);
+        if (kc % KI == 0) {
 #pragma unroll
-          for (int b0 = 0; b0 < 4; b0 += PAIR)
-            if (b0 * RG < 4) {
+          for (int c = 0; c < CPW; ++c)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) big[c][b] = small[c][b] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int sub = 0; sub < SK / 32; ++sub) {
+          const int k32 = kc % KI * (SK / 32) + sub;
+          if (cb0 < CB && 32 * k32 < K) {  // uniform
+            const int g = 4 * sub + h;
+            const bf8 *xb = xbuf + (kc & 1) * (kStreamStageBytes / 32) + 16 * g + (j ^ g * (16 / KG));
+            constexpr int PAIR = RG > 1 && KS <= 4 ? TB : 1;  // row tiles multiplied side by side
+#pragma unroll
+            for (int b0 = 0; b0 < TB; b0 += PAIR) {
               split3<bf8> x[PAIR];
 #pragma unroll
-              for (int u = 0; u < PAIR; ++u)
-                if ((b0 + u) * RG < 4) {
-                  const bf8 *p = xb + (rg + RG * (b0 + u)) * 64;
-                  x[u] = split3<bf8>{p[0], p[256], p[512]};
-                }
+              for (int u = 0; u < PAIR; ++u) {
+                const bf8 *p = xb + (rg + RG * (b0 + u)) * (KG * 16);
+                x[u] = split3<bf8>{p[0], p[256], p[512]};
+              }
 #pragma unroll
               for (int c = 0; c < CPW; ++c) {
-                const split3<bf8> &wp = w[c][kc];
-                auto add = [&](bf8 split3<bf8>::*xpart, bf8 split3<bf8>::*wpart) __attribute__((always_inline)) {
+                const split3<bf8> &wp = w[c][k32];
+                auto add = [&](v4f (&to)[TB], bf8 split3<bf8>::*xpart, bf8 split3<bf8>::*wpart) __attribute__((always_inline)) {
 #pragma unroll
-                  for (int u = 0; u < PAIR; ++u)
-                    if ((b0 + u) * RG < 4) acc[c][b0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u].*xpart, wp.*wpart, acc[c][b0 + u], 0, 0, 0);
+                  for (int u = 0; u < PAIR; ++u) to[b0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u].*xpart, wp.*wpart, to[b0 + u], 0, 0, 0);
                 };
-                add(&split3<bf8>::l, &split3<bf8>::m);
-                add(&split3<bf8>::m, &split3<bf8>::l);
-                add(&split3<bf8>::l, &split3<bf8>::h);
-                add(&split3<bf8>::h, &split3<bf8>::l);
-                add(&split3<bf8>::m, &split3<bf8>::m);
-                add(&split3<bf8>::m, &split3<bf8>::h);
-                add(&split3<bf8>::h, &split3<bf8>::m);
-                add(&split3<bf8>::h, &split3<bf8>::h);
+                add(small[c], &split3<bf8>::l, &split3<bf8>::m);
+                add(small[c], &split3<bf8>::m, &split3<bf8>::l);
+                add(small[c], &split3<bf8>::l, &split3<bf8>::h);
+                add(small[c], &split3<bf8>::h, &split3<bf8>::l);
+                add(small[c], &split3<bf8>::m, &split3<bf8>::m);
+                add(small[c], &split3<bf8>::m, &split3<bf8>::h);
+                add(small[c], &split3<bf8>::h, &split3<bf8>::m);
+                add(big[c], &split3<bf8>::h, &split3<bf8>::h);
               }
             }
+          }
         }
-        if (kc == NKC - 1 && cb0 < CB) {
+        if (kc % KI == KI - 1 && cb0 < CB) {
           float finite = 0.f;
 #pragma unroll
           for (int c = 0; c < CPW; ++c)
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-              if (bi * RG < 4) {
+            for (int b = 0; b < TB; ++b)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  acc[c][bi][r] *= (rg + RG * bi) % 2 ? -kSplitOut : kSplitOut;
-                  finite = __builtin_fmaf(acc[c][bi][r], 0.f, finite);
-                }
+              for (int r = 0; r < 4; ++r) {
+                big[c][b][r] = (big[c][b][r] + small[c][b][r]) * ((rg + RG * b) % 2 ? -kSplitOut : kSplitOut);
+                finite = __builtin_fmaf(big[c][b][r], 0.f, finite);
               }
           if (__ballot(finite != 0.f)) {  // (NaN) infinities or NaN in the operands, or too large for bf16: on the fp32 cores
 #pragma unroll
             for (int c = 0; c < CPW; ++c)
 #pragma unroll
-              for (int bi = 0; bi < 4; ++bi)
-                if (bi * RG < 4) {
-                  const float *row = B + (size_t)(t.prod_begin + min(q * kXRows + 16 * (rg + RG * bi) + j, P - 1)) * K;
-                  const int col = min(16 * (cb0 + NW * c) + j, N - 1);
-                  v4f s = v4f{0.f, 0.f, 0.f, 0.f};
+              for (int b = 0; b < TB; ++b) {
+                const float *row = B + (size_t)(t.prod_begin + min(q * kXRows + SR * half + 16 * (rg + RG * b) + j, P - 1)) * K;
+                const int col = min(16 * (cb0 + NW * c) + j, N - 1);
+                v4f s = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-                  for (int k = h; k < K; k += 4)
-                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(relu_in ? fmaxf(row[k], 0.f) : row[k], W[(size_t)k * N + col], s, 0, 0, 0);
-                  acc[c][bi] = s;
-                }
+                for (int k = h; k < K; k += 4)
+                  s = __builtin_amdgcn_mfma_f32_16x16x4f32(relu_in ? fmaxf(row[k], 0.f) : row[k], W[(size_t)k * N + col], s, 0, 0, 0);
+                big[c][b] = s;
+              }
           }
-          // last interval of the step: the 64 new rows go into the ring (and to HBM where the
-          // remainder reads them) before the barrier that lets the consumers at them
+          // last interval of these rows: they go into the ring (and to HBM where the remainder reads them)
+          // before the barrier that lets the consumers at them, the step's last
           const int row0 = t.prod_begin + q * kXRows;
           const bool plain = (q + 1) * kXRows <= P && (row0 + kXRows <= t.wb_begin || row0 >= t.wb_end);
           if (plain) {
@@ -1054,31 +1062,27 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
             // slot is reduced; everything else is this lane's fixed place in the step plus a multiple of a row.
             char *base = ring_lane + ((q * kXRows) & ring_mask) * ld4;
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-              if (bi * RG < 4) {
+            for (int b = 0; b < TB; ++b)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+              for (int r = 0; r < 4; ++r)
 #pragma unroll
-                  for (int c = 0; c < CPW; ++c)
-                    *reinterpret_cast<float *>(base + (16 * RG * bi + r) * ld4 + 64 * NW * c) = acc[c][bi][r];
-              }
+                for (int c = 0; c < CPW; ++c)
+                  *reinterpret_cast<float *>(base + (SR * half + 16 * RG * b + r) * ld4 + 64 * NW * c) = big[c][b][r];
           } else {
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-              if (bi * RG < 4) {
+            for (int b = 0; b < TB; ++b)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  const int lr = q * kXRows + 16 * (rg + RG * bi) + 4 * h + r;
-                  if (lr < P) {
-                    const int row = t.prod_begin + lr;
-                    const bool wb = row >= t.wb_begin && row < t.wb_end;
+              for (int r = 0; r < 4; ++r) {
+                const int lr = q * kXRows + SR * half + 16 * (rg + RG * b) + 4 * h + r;
+                if (lr < P) {
+                  const int row = t.prod_begin + lr;
+                  const bool wb = row >= t.wb_begin && row < t.wb_end;
 #pragma unroll
-                    for (int c = 0; c < CPW; ++c) {
-                      const int col = 16 * (cb0 + NW * c) + j;
-                      if (col < N) {
-                        ring[(lr & ring_mask) * ld + col] = acc[c][bi][r];
-                        if (wb) T[(size_t)row * N + col] = acc[c][bi][r];
-                      }
+                  for (int c = 0; c < CPW; ++c) {
+                    const int col = 16 * (cb0 + NW * c) + j;
+                    if (col < N) {
+                      ring[(lr & ring_mask) * ld + col] = big[c][b][r];
+                      if (wb) T[(size_t)row * N + col] = big[c][b][r];
                     }
                   }
                 }
