@@ -870,17 +870,16 @@ __global__ __launch_bounds__(kGemmBlock) void fused_gemm_spmm_regw_kernel(
 // (the staging rhythm: KS/2 intervals per step, the ones past K empty); the consumers spread
 // a step's rows evenly over those intervals.
 // Nothing that is still in flight is ever moved between registers: a producer thread keeps
-// one staging register per interval of a step (a whole step of X in flight), the barriers
+// one staging unit per interval (four intervals of X in flight, two where a step has no more), the barriers
 // wait for LDS traffic only, and a consumer lane group
 // keeps one register set per interval of a step -- the (row, first entry, end) record of the
 // row it will compute in the same interval of the next step is requested a step ahead, its
 // first LPR entries half a step ahead, both unconditionally (clamped to existing records).  The entries are turned
 // into (byte offset into the ring, value) pairs in a small per-group LDS area and walked in
 // CSR order with broadcast reads.
-// What bounds it: fp32 MFMAs and the consumers' FMAs share the vector pipe of a SIMD, so their times added up; the six bf16 products take 0.4
-// of the MFMA time and run beside FMAs (us, 262,144 rows of 16 in a band of 32, operands in no cache, fp32 producers / these: K = N = 128 132 / 115,
-// 256 x 128 215 / 178, 128 x 96 125 / 108, 64 x 128 125 / 111, 256 x 64 154 / 144, 128 x 64 90 / 85, 64 x 32 58 / 58).  Now the consumers: a row's
-// entries, one LDS read and four FMAs each, between two barriers.
+// What bounds it: fp32 MFMAs and the consumers' FMAs share the vector pipe of a SIMD, so their times added up; the eight bf16 products take half
+// of the MFMA time and run beside FMAs (us, 262,144 rows of 16 in a band of 32, fp32 producers / these: K = N = 128 131 / 114, 256 x 128 215 / 170,
+// 160 x 128 170 / 139, 256 x 64 154 / 131, 128 x 64 88 / 84).  Now the consumers: a row's entries, one LDS read and four FMAs each, between two barriers.
 constexpr int kStreamProducers = 8;   // wavefronts
 static_assert(kStreamStageBytes == 2 * 3 * kXRows * kXChunk * 2, "two buffers of three bf16 parts");
 
@@ -913,11 +912,13 @@ __global__ __launch_bounds__((kStreamProducers + NCW) * 64) void fused_gemm_spmm
     const int rg = RG > 1 ? wave / (NW / RG) : 0;
     // What is multiplied in one interval: SR rows by SK values of k, TB row tiles a wavefront, each with an accumulator for the large terms and one for the
     // small ones.  Where a wavefront has a column block to itself a step's 64 rows are two halves, one after the other, so that the accumulators
-    // take the registers of four tiles and not of eight.
-    constexpr int SR = RG == 1 ? 32 : kXRows, SK = kXRows * kXChunk / SR, TB = SR / 16 / RG;
+    // take the registers of four tiles and not of eight; where K is beyond 128, and W's parts take 96 registers, one tile at a time.  (With two
+    // and eight intervals of X in flight these kernels kept 13 to 30 registers in scratch memory: us, 262,144 rows of 16, 256 x 128 214 / 170, 256 x 64
+    // 166 / 131, 160 x 128 193 / 139.)
+    constexpr int SR = KS > 8 ? 16 * RG : RG == 1 ? 32 : kXRows, SK = kXRows * kXChunk / SR, TB = SR / 16 / RG;
     constexpr int KI = KS * 16 / SK;  // intervals over K for the same rows
     static_assert(KI * (kXRows / SR) == NKC && TB >= 1, "a step is NKC intervals");
-    constexpr int AH = NKC;  // intervals whose units are on their way
+    constexpr int AH = NKC < 4 ? NKC : 4;  // intervals whose units are on their way
     const int sr = threadIdx.x / (SK / 4), sk = threadIdx.x % (SK / 4) * 4;
     // Always a load (of the last row / the last values of k when past the end, zeroed when it
     // is stored to LDS): a load under a condition would have to land before the next barrier.
