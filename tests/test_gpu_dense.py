@@ -140,6 +140,43 @@ def test_gemm_of_few_features_a_row(gpu, tf, M, K, N, q):
     no_further_than_fp32(Y.to_numpy(), X, W, q)
 
 
+@pytest.mark.parametrize("small", [-148, -140, -125, -110])
+@pytest.mark.parametrize("what", ["gemm", "gemm weights", "streamed", "weight gradient"])
+def test_small_operands_on_bf16_cores(gpu, tf, what, small):
+    """Values of 2^small, denormal ones among them, times values whose products are normal floats: as precise as any others; and times values that leave
+    the results denormal, to their last place."""
+    say(f"small operands {what} 2^{small}")
+    rng = np.random.default_rng(-small)
+    M, K, N = 25000, 96, 72
+    lib = tf.lib()
+    for other in (35, -4):
+        # sums and differences of the smallest floats: what counts is kept whole by the first rounding, to fp32
+        tiny = lambda m, n: (rng.uniform(-1, 1, (m, n)) * 2.0 ** small).astype(np.float32)
+        X = tiny(M, K) if what != "gemm weights" else rng.uniform(-1, 1, (M, K)).astype(np.float32) * np.float32(2.0 ** other)
+        if what == "weight gradient":
+            G, Y = (rng.uniform(-1, 1, (M, N)) * 2.0 ** other).astype(np.float32), tf.DenseMatrix(N, K)
+            ws = tf.DenseMatrix(1, max(1, lib.tf_weight_grad_workspace(M, N, K) // 4))
+            Gd, Xd = tf.DenseMatrix.from_numpy(G), tf.DenseMatrix.from_numpy(X)
+            assert lib.tf_weight_grad(Gd.h, Xd.h, Y.h, C.c_void_p(ws.device_ptr()), None) == 0
+            a, b, terms = G.T, X, 300
+        else:
+            W = tiny(K, N) if what == "gemm weights" else (rng.uniform(-1, 1, (K, N)) * 2.0 ** other).astype(np.float32)
+            Xd, Wd, Y = tf.DenseMatrix.from_numpy(X), tf.DenseMatrix.from_numpy(W), tf.DenseMatrix(M, N)
+            if what == "streamed":
+                Ah = tf.CsrMatrix.from_scipy(sp.identity(M, dtype=np.float32, format="csr"))
+                S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K, lds_budget_bytes=163840)
+                assert S.info()["streamed"] == 1
+                tf.gemm_spmm(Ah.to_device(), Xd, Wd, Y, S)
+            else:
+                assert lib.tf_gemm_ex(Xd.h, Wd.h, Y.h, None, 0, None) == 0
+            a, b, terms = X, W, K + 8
+        tf.device_synchronize()
+        a, b = a.astype(np.float64), b.astype(np.float64)
+        # roundings of sums, each below the sum of magnitudes, or half a place of the smallest float where a group's sum is denormal
+        bound = terms * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 600 * 2.0 ** -150
+        assert np.all(np.abs(Y.to_numpy() - a @ b) <= bound), (what, small, other)
+
+
 @pytest.mark.parametrize("K,N", [(128, 128), (120, 96), (64, 64), (40, 32), (136, 32), (256, 64), (256, 128)])
 def test_streamed_runs_on_bf16_cores(gpu, tf, K, N):
     """Banded rows whose intermediate never leaves LDS: within fp32's rounding of float64, values of many sizes, and what is not finite
@@ -175,8 +212,7 @@ def test_streamed_runs_on_bf16_cores(gpu, tf, K, N):
 @pytest.mark.parametrize("q", [1, 2, 4, 8, 64])
 def test_streamed_runs_of_few_features_a_row(gpu, tf, K, N, q):
     """The rows of the intermediate themselves (A is the identity)."""
-    if q > K:
-        pytest.skip("fewer features")
+    q = min(q, K)
     say(f"streamed runs of few features a row {K} x {N}, {q} a row")
     M = 25000
     rng = np.random.default_rng(K + N + q)

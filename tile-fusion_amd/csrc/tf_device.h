@@ -204,9 +204,10 @@ typedef float acc4 __attribute__((ext_vector_type(4)));
 // while it has 24 bits.  Root mean square of the error over the sum of magnitudes, values in [-1, 1], K = 128, in e-8, for 1 / 2 / 4 / 8 / 128 values
 // that are not zero: fp32 cores 2.53 / 2.54 / 2.53 / 2.48 / 2.40, this 2.53 / 2.09 / 1.64 / 1.26 / 0.70; largest of five million 6.0 / 11.3 / 17 / 22 / 30 and
 // 6.0 / 15.0 / 14 / 15 / 9.
-// The cores take denormal bf16 for zero: both operands are made 2^20 times larger on the way in, so that the parts of every
-// normal float are normal, and sums 2^-40 times smaller on the way out.  Infinities, NaN and sums beyond 2^88 come out infinite or NaN: the
-// caller looks for those and computes such a block again on the fp32 cores.
+// bf16 has no bits below 2^-133 where floats end at 2^-149: both operands are made 2^20 times larger on the way in, which leaves every part of every float
+// whole, and sums 2^-40 times smaller on the way out.  (Parts may be denormal: the cores take them as they are.  Operands of 2^-148 times 2^35 come out
+// as precise as any others.)  Infinities, NaN, operands beyond 2^107 and sums beyond 2^87 come out infinite or NaN: the caller looks for those and
+// computes such a block again on the fp32 cores.
 // What the cores cut off when they align products is always cut downwards, some 4e-9 of a sum: nothing in one result, but 2e-7 in a
 // weight gradient over 3,000 blocks of rows with as many terms of either sign.  Callers therefore scale rows of odd number, or every other block of them, by -2^20.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
