@@ -307,6 +307,35 @@ def test_weight_gradient_of_rare_features(gpu, tf, M, N, K, q):
     assert np.sqrt((e ** 2).mean()) <= 1.05 * np.sqrt((ref ** 2).mean())  # (of some 6,000 values each: 1.3 %)
 
 
+@pytest.mark.parametrize("what,M,K,N", [("gemm", 18437, 300, 65), ("gemm", 18437, 300, 67), ("gemm", 18437, 257, 130), ("gemm", 18437, 300, 68), ("gradient", 9000, 193, 40),
+                                        ("gradient", 9000, 40, 195), ("gradient", 9000, 194, 129), ("gradient", 3073, 70, 65)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 1e38])
+def test_columns_of_other_panels_keep_their_bits(gpu, tf, what, M, K, N, bad):
+    """A value in the last column that takes its panel (chunk) to the fp32 cores changes nothing in the panels before it, also where
+    the last one is narrower than what a lane works on."""
+    say(f"panels {what} {M} x {K} x {N} {bad}")
+    rng = np.random.default_rng(M + K + N)
+    lib = tf.lib()
+    X, W, G = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    got = []
+    for value in (0.5, bad, bad):
+        W[0, N - 1] = G[M // 2, N - 1] = value
+        Xd, Wd, Gd = (tf.DenseMatrix.from_numpy(a) for a in (X, W, G))
+        if what == "gemm":
+            Y = tf.DenseMatrix(M, N)
+            assert lib.tf_gemm_ex(Xd.h, Wd.h, Y.h, None, 0, None) == 0
+        else:
+            Y, ws = tf.DenseMatrix(N, K), tf.DenseMatrix(1, lib.tf_weight_grad_workspace(M, N, K) // 4)
+            assert lib.tf_weight_grad(Gd.h, Xd.h, Y.h, C.c_void_p(ws.device_ptr()), None) == 0
+        tf.device_synchronize()
+        got.append(Y.to_numpy() if what == "gemm" else Y.to_numpy().T)
+    panel = 64 if what == "gemm" else 16 * -(-(-(-N // -(-N // 64))) // 16)  # (gradients: chunks of up to 64 columns, evenly)
+    before = (N - 1) // panel * panel
+    assert before > 0 or N <= 64
+    assert np.array_equal(got[0][:, :before], got[1][:, :before])
+    assert np.array_equal(got[1], got[2], equal_nan=True)
+
+
 @pytest.mark.parametrize("M1,M2", [(100, 100), (3072, 3072), (3073, 3073), (20001, 20001), (3000, 5000), (5000, 3000)])
 def test_two_weight_gradients_in_one_call(gpu, tf, M1, M2):
     """Sharing their launches changes no bit of either, of few rows and of many (and of one and the other)."""

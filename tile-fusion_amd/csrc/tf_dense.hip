@@ -552,7 +552,11 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     }
     const dim3 grid(std::max(1, std::min(across, (n_blocks + waves - 1) / waves)), panels);
     hipError_t err = hipSuccess;
-    const int out = how.accumulate || how.relu || N < 4 || (rows && how.mask) ? kAnyOut : rows ? kListed : how.mask ? kMasked : kPlain;
+    // (a last panel of less than a lane's columns must not store the one before it: the two may differ in their last bits, where one of them went
+    // over to the fp32 cores)
+    const int lane_columns = unit == 16 ? 1 : unit % 64 ? 2 : 4;
+    const bool narrow_last = on_bf16 && panels > 1 && N - (panels - 1) * unit < lane_columns;
+    const int out = how.accumulate || how.relu || N < 4 || narrow_last || (rows && how.mask) ? kAnyOut : rows ? kListed : how.mask ? kMasked : kPlain;
 #define CALLP4(...)                                                                                                            \
   do {                                                                                                                         \
     if (lds > 65536)                                                                                                           \
@@ -614,7 +618,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // NB j .. of G and KB j .. of X in the rows 8 h .. 8 h + 7, which are what its part of a 16 x 16 x 32 product wants of each of
 // the NB (KB) column blocks.  The next rows are requested as soon as these have become parts.  The wavefronts of a launch take blocks of
 // rows in turn; a workgroup's four are added through LDS, and weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.
-// A lane whose columns would reach past the last one works on the last NB (KB) instead, which writes some values of Y twice, the same.
+// A lane whose columns would reach past the last one works on the last NB (KB) instead: some values of Y are computed twice.
 // Bound: the rows of X and G from HBM, 16 KB a wavefront in flight, behind some 10 us for two launches and the sums at the end (us, operands in no
 // cache, both launches, fp32 cores on 64 x 160 tiles / this: 14,000 rows 32 x 69 18.2 / 9.5, 35,000 rows 64 x 128 26.1 / 22.5, 100,000 rows 64 x 128 36.6 / 33.0,
 // 20 x 100 26.6 / 22.8, 131,072 rows 64 x 300 75 / 66, 40 x 64 28.3 / 24.4, 262,144 rows 128 x 128 109 / 98; error against 64 bits at 100,000 rows
@@ -792,8 +796,10 @@ __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const WeightGra
   s += red[2][lane];
   const int r = reg % 4, kb = (reg / 4) % KB, nb = reg / 4 / KB;
   const int i = 4 * h + r;  // row of the 16 x 16 block that register r of lane (j, h) holds
-  const int n = min(chunk / k_chunks * 16 * NB + NB * i, N - NB) + nb, k = min(chunk % k_chunks * 16 * KB + KB * j, K - KB) + kb;
-  t.Y[(size_t)n * K + k] = s;
+  const int n0 = chunk / k_chunks * 16 * NB, k0 = chunk % k_chunks * 16 * KB;
+  const int n = min(n0 + NB * i, N - NB) + nb, k = min(k0 + KB * j, K - KB) + kb;
+  // (what lies in front of the chunk is stored by the one it belongs to: the two may differ in their last bits, where one of them went over to the fp32 cores)
+  if (n >= n0 && k >= k0) t.Y[(size_t)n * K + k] = s;
 }
 
 // The same for few rows in one launch: a workgroup of sixteen wavefronts per 16 x 16 tile of Y (v_mfma_f32_16x16x4_f32, so that
