@@ -37,7 +37,7 @@ def test_gemm_of_any_shape(gpu, tf, M, K, N, w_t):
 
 
 @pytest.mark.parametrize("M,K,N", [(13001, 4, 33), (12999, 17, 64), (20481, 18, 17), (13007, 19, 129), (13001, 66, 97), (262145, 131, 35), (40000, 100, 100),
-                                   (13000, 5, 257)])
+                                   (13000, 5, 257), (262145, 8, 32), (262144, 16, 64), (262143, 15, 33), (66000, 17, 40), (20479, 16, 31), (20480, 4, 17)])
 def test_gemm_panel_edges(gpu, tf, M, K, N):
     """W in LDS: steps of k that end after one to four values, a last lane whose columns overlap its neighbour's, rows and panels
     that end early; non-finite values beside the edges stay where they are."""

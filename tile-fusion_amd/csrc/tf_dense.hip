@@ -119,15 +119,19 @@ __global__ __launch_bounds__(256) void gemm_direct_kernel(const float *__restric
 
 // ---------------------------------------------------------------------------------
 // The same product for many rows: W (a panel of 16 V Q columns of it) in LDS, once per workgroup, row-major and padded with zeros
-// to whole steps of k and whole panels, whichever way it is stored; every wavefront walks its own run of 16-row blocks
-// with no barrier, its rows of X requested a group of kGemmAhead steps ahead (the first group before W is staged).
+// to whole steps of k and whole panels, whichever way it is stored; every wavefront takes 16-row blocks
+// with no barrier, its rows of X requested a group of A steps ahead (the first group before W is staged).
 // Column block (v, q) of lane j is column 16 V q + V j + v: a lane reads V adjacent values of W per k and stores V adjacent columns of
 // Y, sixteen lanes side by side.  Sixteen wavefronts per compute unit (up to 128 registers each), so that a SIMD has
 // three others to feed its matrix core while one waits: 131,072 x 300 x 64 takes 54 us (139 us with
 // every row tile reading W from L2; 33 us and 39 us for a padded copy of X in 32-row blocks).
+// The wavefronts take blocks in turn, so that what is read and written is one stretch of memory; with K of 16 or less a group is the one step there is.
+// (us, 262,144 rows, a kernel of 32-row MFMAs that took such rows before this one / a run of blocks for each wavefront / in turn / and one step:
+// 8 x 32 12.7 / 13.7 / 13.0 / 11.9, 64 x 32 24.5 / 24.7 / 20.5, 8 x 64 17.7 / 20.2 / 19.0 / 18.0, 16 x 64 20.8 / 23.0 / 19.9 / 18.7, 8 x 128 29.5 / 35.8 / 33.4 / 30.2,
+// 16 x 128 32.2 / 42.0 / 35.9 / 31.2, 128 x 32 40.5 / 40.7 / 34.2; 1,000,000 rows 16 x 128 124 / 140 / 140 / 118; 16,000 rows 128 x 128 12.0 / 11.9 / 11.4.)
 // Bound: X and Y from HBM for up to 64 columns, fp32 MFMA beyond.
 // ---------------------------------------------------------------------------------
-constexpr int kGemmAhead = 4;  // steps of 16 values of k per group of operands
+constexpr int kGemmAhead = 4;  // A: steps of 16 values of k per group of operands
 
 // Rows in order and values as they are; with zeros where the mask is zero or less; rows of a list, values as they are; all else.
 enum { kPlain, kMasked, kListed, kAnyOut };
@@ -137,21 +141,20 @@ enum { kPlain, kMasked, kListed, kAnyOut };
 // V columns reach past the last one works on the last V, and the last step's values of k past K are cleared in registers.
 // (Conditions around them, us: 262,144 x 64 x 64 37, 128 x 64 58, 64 x 128 61; without 29, 50, 55;
 // 30,000 x 300 x 64 23.0, 100 x 83 15.8; without 18.3, 13.1.)
-template <int V, int Q, bool WT, int OUT>
+template <int V, int Q, bool WT, int OUT, int A>
 __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restrict__ X, int ldx, const float *__restrict__ W,
                                                           float *__restrict__ Y, int ldy, const int *__restrict__ rows,
                                                           int y_by_row, int n_rows, int K, int N,
                                                           const GemmOut out_how) {
   extern __shared__ __align__(16) float wlds[];
-  constexpr int P = 16 * V * Q, A = kGemmAhead;  // columns of the panel
+  constexpr int P = 16 * V * Q;  // columns of the panel
   const int waves = blockDim.x / 64, wave = threadIdx.x / 64, lane = threadIdx.x % 64, j = lane % 16, h = lane / 16;
   const int panel0 = blockIdx.y * P, S = (K + 15) / 16, G = (S + A - 1) / A;
-  const int n_blocks = (n_rows + 15) / 16, total_waves = gridDim.x * waves, gw = blockIdx.x * waves + wave;
-  const int b0 = (int)((long long)gw * n_blocks / total_waves), b1 = (int)((long long)(gw + 1) * n_blocks / total_waves);
+  const int n_blocks = (n_rows + 15) / 16, stride = gridDim.x * waves, b0 = wave * gridDim.x + blockIdx.x;
   auto column = [&](int n) { return OUT == kAnyOut ? min(panel0 + n, N - 1) : min(panel0 + n - n % V, N - V) + n % V; };  // of W
   struct operands { f4v a[A]; };
   auto row_index = [&](int b) __attribute__((always_inline)) {
-    const int q = min(min(b, b1 - 1) * 16 + j, n_rows - 1);
+    const int q = min(b * 16 + j, n_rows - 1);
     if constexpr (OUT == kPlain || OUT == kMasked) return q;
     else if constexpr (OUT == kListed) return rows[q];
     else return rows ? rows[q] : q;
@@ -165,9 +168,9 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
   const float *xp = X;
   operands cur;
   int next_row = 0;  // of this lane in the block after the next one to begin
-  if (b0 < b1) {
+  if (b0 < n_blocks) {
     xp = X + (size_t)row_index(b0) * ldx;
-    next_row = row_index(b0 + 1);
+    next_row = row_index(b0 + stride);
     cur = load(xp, 0);
   }
   // W into LDS: a column's sixteen values of one step per thread and item, all requested before the first is stored
@@ -232,9 +235,9 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
       step(s, v);
     }
   };
-  for (int b = b0; b < b1; ++b) {
+  for (int b = b0; b < n_blocks; b += stride) {
     const float *xn = X + (size_t)next_row * ldx;
-    next_row = row_index(b + 2);
+    next_row = row_index(b + 2 * stride);
     int y_row[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -566,7 +569,8 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   } while (0)
 #define CALLP3(V_, Q_, WT_, OUT_)                                                                                              \
   do {                                                                                                                         \
-    if (!on_bf16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_>); }                                                            \
+    if (!on_bf16 && K <= 16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, 1>); }                                              \
+    else if (!on_bf16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, kGemmAhead>); }                                           \
     else if constexpr (V_ * Q_ >= 2) {                                                                                         \
       if (V_ * Q_ == 2 || ahead == 4) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 4>); }                                     \
       else if constexpr (V_ * Q_ > 2) {                                                                                        \
