@@ -65,12 +65,14 @@ def test_gemm_panel_edges(gpu, tf, M, K, N):
                                    (30001, 128, 128), (18437, 161, 72), (18439, 213, 128), (10241, 214, 129), (10239, 214, 129), (10240, 300, 100),
                                    (10243, 426, 65), (18434, 427, 65), (38400, 64, 33), (38399, 64, 33), (38409, 96, 48), (49999, 130, 64),
                                    (38403, 427, 40), (38401, 853, 36), (38402, 854, 36), (262145, 67, 35),
-                                   (18434, 16, 70), (18435, 17, 70), (38405, 48, 33), (38405, 49, 33), (38401, 63, 64)])
+                                   (18434, 16, 70), (18435, 17, 70), (38405, 48, 33), (38405, 49, 33), (38401, 63, 64),
+                                   (18433, 192, 128), (18433, 193, 128), (18435, 256, 96), (18435, 257, 96), (18434, 416, 68), (18434, 417, 68),
+                                   (18434, 415, 126), (38403, 416, 33), (38403, 416, 64), (38401, 417, 36)])
 @pytest.mark.parametrize("w_t", [False, True])
 def test_gemm_on_bf16_cores(gpu, tf, M, K, N, w_t):
-    """Products as sums of bf16 parts, either side of where they begin and of what LDS holds: no further from float64 than fp32 sums, for
-    operands of one size and of many sizes; infinities, NaN and values that bf16 rounds to infinity stay in their rows, and come out
-    as fp32 arithmetic has them."""
+    """Products as sums of bf16 parts, either side of where they begin and of what LDS holds (192 values of k for a panel of 128 columns, 256 for 96, 416 for
+    64): within the bound of fp32 sums around float64, for operands of one size and of many sizes; infinities, NaN and values that bf16
+    rounds to infinity stay in their rows, and come out as fp32 arithmetic has them."""
     say(f"gemm on bf16 cores {M} x {K} x {N} w_t={w_t}")
     rng = np.random.default_rng(M + 3 * K + 5 * N)
     W = rng.uniform(-0.2, 0.2, (K, N)).astype(np.float32)

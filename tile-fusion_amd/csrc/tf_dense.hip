@@ -520,25 +520,23 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   // Which kernel.  Copying W to LDS takes some 4 us before the first product; gemm_direct_kernel reads it from L2 for every row tile, by
   // single values where W is K x N (us, gemm_panel_kernel / gemm_direct_kernel, at 8,000 / 16,000 / 30,000 rows: 128 x 128 9.3 / 8.1 (K x N: 9.3 / 11.6),
   // 11.0 / 13.8, 16.8 / 23; 64 x 64 5.0 / 4.6 (5.0 / 5.7), 5.0 / 6.0, 6.7 / 9.0; 500 x 32, 30,000 rows 17.6 / 20.8; 40 x 7 6.7 / 4.2).
-  // The bf16 cores pay where the fp32 ones were what a product waited for: beyond 64 columns from 72 rows per compute unit on, where splitting W no
-  // longer counts (40 where gemm_panel_kernel has more than 213 values of k for each), for 33 to 64 columns from 150 on where K is beyond 48 (us,
-  // operands in L2 and the Infinity Cache, gemm_panel_kernel / gemm_split_kernel: 13,000 rows 128 x 128 10.8 / 11.1, 300 x 128 19.2 / 16.6, 128 x 64
-  // 7.5 / 7.8; 16,000 rows 128 x 128 10.8 / 11.0, 20,000 rows 128 x 128 16.2 / 13.3, 300 x 128 31.5 / 19.7, 64 x 100 10.7 / 8.9; 30,000 rows 128 x 64
-  // 10.5 / 9.8, 64 x 64 7.8 / 8.1; 40,000 rows 64 x 64 9.1 / 8.3, 128 x 64 13.9 / 12.1; operands in no cache, gemm_panel_kernel /
-  // gemm_split_kernel with W N x K: 12,500 rows 300 x 64 10.5 / 12.9; 24,000 rows 64 x 128 11.9 / 10.1, 128 x 128 17.2 / 14.4, 128 x 64 10.0 / 10.1,
-  // 300 x 128 32.2 / 23.1; 50,000 rows 128 x 64 15.4 / 15.1, 32 x 64 8.6 / 8.3; 100,000 rows 32 x 64 12.0 / 12.4, 64 x 64 16.4 / 15.2, 128 x 64 25.0 / 20.5,
-  // 300 x 64 51.4 / 41.4, 128 x 128 43.6 / 30.3, 300 x 128 88.3 / 67.1; 262,144 rows 128 x 40 47.2 / 38.0, 128 x 128 81 / 63; 200,000 rows
-  // 256 x 128 119 / 99, two panels; 60,000 rows 300 x 300 172 / 93, five; but 150,000 rows 512 x 128 173 / 194, four panels of 32;
-  // 60,000 rows 8 x 66 8.5 / 9.0, 16 x 96 8.5 / 9.3, 24 x 96 10.1 / 9.7, 24 x 128 12.4 / 11.0, 180,000 rows 24 x 128 31.9 / 26.1: a step takes 32 k;
-  // 131,072 rows 40 x 64 16.6 / 18.0, 48 x 64 17.0 / 17.1, 60 x 64 20.0 / 17.8, 60 x 40 19.1 / 15.9, 40,000 rows 60 x 64 10.4 / 8.9).
+  // The bf16 cores pay where the fp32 ones are what a product waits for and panels of 64 columns fit LDS (up to 416 values of k): beyond 64 columns from 72
+  // rows per compute unit on, where splitting W no longer counts (40 beyond 213 values of k, where a row block is a long chain of fp32
+  // products), for 33 to 64 columns from 150 on where K is beyond 48 (us, gemm_panel_kernel / gemm_split_kernel, W as it is stored in turn: 10,240 rows
+  // 192 x 128 13.8 / 16.8, 213 x 128 16.3 / 14.2, 14,000 rows 200 x 128 16.3 / 14.7, 213 x 96 14.4 / 15.3, 300 x 128 20.8 / 18.5; 18,432 rows 20 x 128 7.9 / 8.6, 32 x 128 8.1 / 7.4, 64 x 128 11.0 / 9.0, 128 x 128 16.2 / 14.9;
+  // 20,000 rows 200 x 128 24.4 / 17.8; 30,000 rows 128 x 128 17.3 / 16.7; 60,000 rows 24 x 96 10.9 / 10.3, 128 x 128 26.6 / 23.9; 180,000 rows 24 x 128
+  // 28.2 / 26.5; 38,400 rows 64 x 64 9.1 / 9.1, 128 x 64 12.9 / 13.5, 300 x 64 23.6 / 23.4; 40,000 rows 60 x 64 9.9 / 8.8; 60,000 rows 64 x 64 11.0 / 10.6;
+  // 100,000 rows 49 x 64 15.3 / 15.1, 128 x 64 23.7 / 21.4, 300 x 64 47.7 / 40.5; 131,072 rows 60 x 40 18.4 / 15.5; 262,144 rows 64 x 64 28.1 / 27.0, 128 x 40
+  // 45.0 / 39.4; five panels, 60,000 rows 300 x 300 169 / 93.  Panels of 32, where X is split for each: 40,000 rows 500 x 64 34.5 / 36.0, 100,000 rows
+  // 73 / 77, 262,144 rows 165 / 181, 100,000 rows 832 x 48 108 / 122, 150,000 rows 512 x 128 173 / 194).
   // Widths are cut into equal panels that fit LDS; X is read once per panel, by compute units of the same XCD at about the same time.
   const int all_rows = std::max(n_rows, how.of_rows);
-  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K > 48 && all_rows >= 150LL * compute_units) && split_lds(K, N > 64 ? 64 : 32) <= kMaxLds;
+  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K > 48 && all_rows >= 150LL * compute_units) && split_lds(K, 64) <= kMaxLds;
   const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
   const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
   int unit = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;
   auto lds_of = [&](int columns) { return on_bf16 ? split_lds(K, columns) : ((long long)K + 15) / 16 * 16 * 4 * columns; };
-  while (unit > 16 && lds_of(unit) > kMaxLds) unit = unit == 96 ? 64 : unit / 2;
+  while (unit > (on_bf16 ? 64 : 16) && lds_of(unit) > kMaxLds) unit = unit == 96 ? 64 : unit / 2;
   const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 80LL * compute_units : (wt ? 48LL : 24LL) * compute_units;
   if (all_rows >= from && lds_of(unit) <= kMaxLds && K >= 4) {
     const int panels = (N + unit - 1) / unit, lds = (int)lds_of(unit), n_blocks = (n_rows + 15) / 16;
@@ -571,13 +569,11 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   do {                                                                                                                         \
     if (!on_bf16 && K <= 16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, 1>); }                                              \
     else if (!on_bf16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, kGemmAhead>); }                                           \
-    else if constexpr (V_ * Q_ >= 2) {                                                                                         \
-      if (V_ * Q_ == 2 || ahead == 4) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 4>); }                                     \
-      else if constexpr (V_ * Q_ > 2) {                                                                                        \
-        if (ahead == 5) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 5>); }                                                   \
-        else if (ahead == 3) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 3>); }                                              \
-        else { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 2>); }                                                              \
-      }                                                                                                                        \
+    else if constexpr (V_ * Q_ >= 4) {                                                                                         \
+      if (ahead == 4) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 4>); }                                                     \
+      else if (ahead == 5) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 5>); }                                                \
+      else if (ahead == 3) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 3>); }                                                \
+      else { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 2>); }                                                                \
     }                                                                                                                          \
   } while (0)
 #define CALLP2(V_, Q_, WT_)                                                                                                    \
