@@ -245,6 +245,32 @@ def test_gemm_of_listed_rows(gpu, tf, K, N):
     assert rel(D.to_numpy(), A.astype(np.float64) @ (X.astype(np.float64) @ W.astype(np.float64))) <= 1e-5
 
 
+@pytest.mark.parametrize("K,N", [(131, 101), (257, 70), (80, 97)])
+def test_gemm_of_listed_rows_on_bf16_cores(gpu, tf, K, N):
+    """The same with rows enough for the bf16 cores: every read row of a larger graph, K and N no multiples of four, one row that is not finite."""
+    say(f"gemm of many listed rows {K} x {N}")
+    rng = np.random.default_rng(K * N)
+    A = tf.workloads.rmat(16, 8 << 16, seed=5)
+    M = A.shape[0]
+    read = np.flatnonzero(np.bincount(A.indices, minlength=M))
+    assert 72 * 256 <= read.size < M  # (rows that nothing reads: the product takes a list)
+    B, W = rng.uniform(-1, 1, (M, K)).astype(np.float32), rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    row = read[read.size // 2]
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, op=tf.OP_GEMM_SPMM, N=N, K=K)
+    Bf = B.astype(np.float64)
+    for bad in (None, np.inf):
+        if bad is not None:
+            B[row, K - 1] = bad
+        D, Bd, Wd = tf.DenseMatrix(M, N), tf.DenseMatrix.from_numpy(B), tf.DenseMatrix.from_numpy(W)
+        tf.gemm_spmm(Ah.to_device(), Bd, Wd, D, S)
+        tf.device_synchronize()
+        got, want = D.to_numpy(), A.astype(np.float64) @ (Bf @ W.astype(np.float64))
+        hit = np.asarray((A[:, [row]] != 0).todense()).ravel() if bad is not None else np.zeros(M, bool)
+        assert rel(got[~hit], want[~hit]) <= 1e-6  # (K products and a row's entries, each rounded once)
+        assert not np.isfinite(got[hit]).any() and (bad is None or hit.any())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 7, 5), (33, 32, 128), (3000, 7, 32), (3000, 32, 500), (10000, 64, 300), (5001, 33, 161),
                                    (100000, 64, 128), (20011, 130, 31), (64, 300, 97), (4096, 65, 33), (4097, 31, 30)])
 def test_weight_gradient(gpu, tf, M, N, K):

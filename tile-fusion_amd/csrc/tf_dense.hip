@@ -531,12 +531,21 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
   // 73 / 77, 262,144 rows 165 / 181, 100,000 rows 832 x 48 108 / 122, 150,000 rows 512 x 128 173 / 194).
   // Widths are cut into equal panels that fit LDS; X is read once per panel, by compute units of the same XCD at about the same time.
   const int all_rows = std::max(n_rows, how.of_rows);
-  const bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K > 48 && all_rows >= 150LL * compute_units) && split_lds(K, 64) <= kMaxLds;
-  const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
-  const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
-  int unit = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;
+  bool on_bf16 = (N > 64 ? K > 16 && all_rows >= (K > 213 ? 40LL : 72LL) * compute_units : N > 32 && K > 48 && all_rows >= 150LL * compute_units) && split_lds(K, 64) <= kMaxLds;
   auto lds_of = [&](int columns) { return on_bf16 ? split_lds(K, columns) : ((long long)K + 15) / 16 * 16 * 4 * columns; };
-  while (unit > (on_bf16 ? 64 : 16) && lds_of(unit) > kMaxLds) unit = unit == 96 ? 64 : unit / 2;
+  auto panel_width = [&]() {
+    const int most = on_bf16 ? 128 : N <= 16 ? 16 : N <= 32 ? 32 : 128;
+    const int panels0 = (N + most - 1) / most, w0 = (N + panels0 - 1) / panels0;
+    int w = w0 <= 16 ? 16 : w0 <= 32 ? 32 : w0 <= 64 ? 64 : w0 <= 96 ? 96 : 128;
+    while (w > (on_bf16 ? 64 : 16) && lds_of(w) > kMaxLds) w = w == 96 ? 64 : w / 2;
+    return w;
+  };
+  int unit = panel_width();
+  // (65 to 67 columns, of 257 values of k and more, are one panel of 96 on the fp32 cores, 60,000 rows 300 x 65 45 us, and one of 64 and the rest on the others, 51)
+  if (on_bf16 && N > unit && N - unit < 4) {
+    on_bf16 = false;
+    unit = panel_width();
+  }
   const long long from = N <= 16 ? LLONG_MAX : N <= 32 ? 80LL * compute_units : (wt ? 48LL : 24LL) * compute_units;
   if (all_rows >= from && lds_of(unit) <= kMaxLds && K >= 4) {
     const int panels = (N + unit - 1) / unit, lds = (int)lds_of(unit), n_blocks = (n_rows + 15) / 16;
