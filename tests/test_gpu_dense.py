@@ -336,7 +336,7 @@ def test_weight_gradient_of_rare_features(gpu, tf, M, N, K, q):
 
 
 @pytest.mark.parametrize("what,M,K,N", [("gemm", 18437, 300, 65), ("gemm", 18437, 300, 67), ("gemm", 18437, 257, 130), ("gemm", 18437, 300, 68), ("gradient", 9000, 193, 40),
-                                        ("gradient", 9000, 40, 195), ("gradient", 9000, 194, 129), ("gradient", 3073, 70, 65)])
+                                        ("gradient", 9000, 40, 195), ("gradient", 9000, 194, 129), ("gradient", 4097, 70, 65)])
 @pytest.mark.parametrize("bad", [np.inf, np.nan, 1e38])
 def test_columns_of_other_panels_keep_their_bits(gpu, tf, what, M, K, N, bad):
     """A value in the last column that takes its panel (chunk) to the fp32 cores changes nothing in the panels before it, also where
@@ -364,7 +364,7 @@ def test_columns_of_other_panels_keep_their_bits(gpu, tf, what, M, K, N, bad):
     assert np.array_equal(got[1], got[2], equal_nan=True)
 
 
-@pytest.mark.parametrize("M1,M2", [(100, 100), (3072, 3072), (3073, 3073), (20001, 20001), (3000, 5000), (5000, 3000)])
+@pytest.mark.parametrize("M1,M2", [(100, 100), (3072, 3072), (3073, 3073), (4096, 4096), (4097, 4097), (20001, 20001), (3000, 5000), (5000, 3000), (4096, 4097)])
 def test_two_weight_gradients_in_one_call(gpu, tf, M1, M2):
     """Sharing their launches changes no bit of either, of few rows and of many (and of one and the other)."""
     say(f"two weight gradients {M1} {M2}")

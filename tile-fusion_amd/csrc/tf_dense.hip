@@ -634,7 +634,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // 1.7e-7 / 1.0e-7).
 // ---------------------------------------------------------------------------------
 constexpr int kWgRows = 32;       // rows of a block
-constexpr int kWgFewRows = 3072;  // up to here in one launch, weight_grad_few_kernel
+constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel
 
 template <int NB, int KB>
 __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int group, int chunk, acc4 (*red)[64]) {
@@ -814,8 +814,9 @@ __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const WeightGra
 // The same for few rows in one launch: a workgroup of sixteen wavefronts per 16 x 16 tile of Y (v_mfma_f32_16x16x4_f32, so that
 // there are tiles enough) and no partial sums in memory.  What counts is the chain of loads: a wavefront keeps sixteen steps of four
 // rows in flight, eight being multiplied and the next eight on their way.  This / weight_grad_kernel and its sums, us: 16 x 40, 1,000 rows 5.8 / 7.4,
-// 64 x 100, 2,000 rows 8.7 / 10.1, 7 x 32, 3,000 rows 8.0 / 7.0, 32 x 500, 3,000 rows 12.2 / 9.1, 32 x 100, 4,096 rows 14.3 / 7.9 -- and a launch less for
-// the host, 3.5 us, which is what a small model waits for.
+// 64 x 100, 2,000 rows 8.7 / 10.1, 7 x 32, 3,000 rows 8.0 / 7.0, 32 x 500, 3,000 rows 12.2 / 9.1, 32 x 100, 4,096 rows 14.3 / 7.9 -- and a launch and a
+// workspace less for the host, which is what a small model waits for: 4,096 nodes, layer 100 -> 32 forward and backward 74 us (two launches 80), 512 -> 128 73
+// (76), two layers 100 -> 32 -> 7 90 (94), 500 -> 64 -> 40 87 (93).
 __global__ __launch_bounds__(1024, 4) void weight_grad_few_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
   constexpr int W = 16, U = 8;
   __shared__ float red[W][4][64];
