@@ -300,6 +300,9 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 // the way.  Bound: X and Y from HBM behind some 8 us until the first product (262,144 x 128 x 128 63 us, 4.3 TB/s; gemm_panel_kernel 81, waiting for
 // the fp32 cores), and the board's power: the same on operands that are all the same number runs at 5.2 TB/s.  Where W takes two panels the parts
 // of X are made twice: 200,000 x 256 x 128 99 us, 60 at the rate of a copy.
+// What is not finite: a row of X costs its block a second pass on the fp32 cores (100,000 x 128 x 128 39.4 -> 39.6 us, 131,072 x 300 x 64 51.8 -> 58.7; with
+// one load at a time 36 -> 63 and 52 -> 91), a value in W one for every block: 79 and 125 us, 335 where W is N x K (176, 345, 415; a product on
+// the fp32 cores alone 45 and 57).
 // ---------------------------------------------------------------------------------
 // Eight wavefronts per compute unit: more of them in flight read memory more slowly (100,000 x 300 x 64: 41.5 us, twelve 41.8, six 42.3).
 constexpr int kSplitWaves = 8;
@@ -461,14 +464,23 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_split_kernel(const floa
 #pragma unroll
       for (int t = 0; t < T; ++t) big[t] = 0.f;
 #pragma unroll 1
-      for (int k0 = 0; k0 < K; k0 += 4) {
-        const int k = min(k0 + h, K - 1);
-        const float xv = k0 + h < K ? xp[k] : 0.f;
+      for (int k0 = 0; k0 < K; k0 += 16) {  // lane (j, h): values 4 h + u of sixteen in product u, all on their way at once
+        float xv[4], wv[4][T];
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-          const int c = column(16 * V * (t / V) + V * j + t % V);
-          const float w = k0 + h < K ? W[WT ? (size_t)c * K + k : (size_t)k * N + c] : 0.f;
-          big[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, w, big[t], 0, 0, 0);
+        for (int u = 0; u < 4; ++u) {
+          const int k = min(k0 + 4 * h + u, K - 1);
+          xv[u] = xp[k];
+#pragma unroll
+          for (int t = 0; t < T; ++t) {
+            const int c = column(16 * V * (t / V) + V * j + t % V);
+            wv[u][t] = W[WT ? (size_t)c * K + k : (size_t)k * N + c];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const bool in = k0 + 4 * h + u < K;
+#pragma unroll
+          for (int t = 0; t < T; ++t) big[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xv[u] : 0.f, in ? wv[u][t] : 0.f, big[t], 0, 0, 0);
         }
       }
     }

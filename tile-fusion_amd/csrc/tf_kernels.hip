@@ -880,6 +880,8 @@ __global__ __launch_bounds__(kGemmBlock) void fused_gemm_spmm_regw_kernel(
 // What bounds it: fp32 MFMAs and the consumers' FMAs share the vector pipe of a SIMD, so their times added up; the eight bf16 products take half
 // of the MFMA time and run beside FMAs (us, 262,144 rows of 16 in a band of 32, fp32 producers / these: K = N = 128 131 / 114, 256 x 128 215 / 170,
 // 160 x 128 170 / 139, 256 x 64 154 / 131, 128 x 64 88 / 84).  Now the consumers: a row's entries, one LDS read and four FMAs each, between two barriers.
+// A row of B that is not finite costs nothing that shows; W with such a value, which every product meets, 128 x 128 127 -> 424 us.  (Four loads at a time there:
+// 330 us, but 107 -> 110 where all is finite.)
 constexpr int kStreamProducers = 8;   // wavefronts
 static_assert(kStreamStageBytes == 2 * 3 * kXRows * kXChunk * 2, "two buffers of three bf16 parts");
 
