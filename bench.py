@@ -273,14 +273,14 @@ def check_result(cfg, got, max_rows=1 << 17, W2=None):
 
 def kernel_names(info, op_is_gemm, unfused):
     if unfused:
-        return "gemm_split_kernel + spmm_rows_kernel"
+        return "dense product + spmm_rows_kernel"
     if not op_is_gemm:
         return ("fused_spmm_spmm_march_kernel" if info["marched"] else
                 "fused_spmm_spmm_window64_kernel" if info["wide_strips"] else
                 "fused_spmm_spmm_window_kernel" if info["windowed"] else
                 "fused_spmm_spmm_kernel" if info["n_fused_rows"] else "spmm_rows_kernel (twice)")
     if info["n_fused_rows"] == 0:
-        return "gemm_split_kernel + spmm_rows_kernel" + (" (+ long-row segments)" if info["n_long_rows"] else "")
+        return "dense product + spmm_rows_kernel" + (" (+ long-row segments)" if info["n_long_rows"] else "")
     return ("fused_gemm_spmm_stream_kernel" if info["streamed"] else
             "fused_gemm_spmm_regw_kernel" if info["register_weights"] else "fused_gemm_spmm_kernel")
 

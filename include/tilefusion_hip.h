@@ -473,7 +473,12 @@ tf_status tf_spmm(const tf_csr *A, const tf_dense *X, tf_dense *Y, unsigned flag
  * among workgroups, so that a graph with hub rows does not wait for the one lane group that has the longest (R-MAT, 2^17
  * nodes, N = 64: 1.23 ms without, 0.06 ms with).  Asynchronous on `stream`, one call at a time per schedule. */
 tf_status tf_spmm_scheduled(const tf_csr *A, const tf_dense *X, tf_dense *Y, tf_schedule *schedule, unsigned flags, void *stream);
-/* Y = X * W   (the cblas_sgemm call at fusion/gcn/GCN_Layer_MKL_Forward_Utils.h:1144), any shape. */
+/* Y = X * W   (the cblas_sgemm call at fusion/gcn/GCN_Layer_MKL_Forward_Utils.h:1144), any shape.
+ * Large dense products, here and inside tf_gemm_spmm and tf_weight_grad, run on the bf16 matrix cores, every float as the sum of three bf16: as
+ * close to exact sums as fp32 arithmetic (root mean square), the same bits on every call.  But a row's last bits depend on where it stands: equal
+ * rows of X at an even and an odd place may differ in them, and a value that is not finite (or a sum beyond 2^87) takes the sixteen rows
+ * around it -- one in W all rows -- to the fp32 cores, whose last bits are others.  Values that are not finite come out where fp32 arithmetic
+ * has them and nowhere else. */
 tf_status tf_gemm(const tf_dense *X, const tf_dense *W, tf_dense *Y, void *stream);
 /* The same with W stored N x K (TF_C_TRANSPOSED), and with Y = 0 wherever `mask` (of Y's shape, may be null) is zero
  * or less: the step back through a ReLU whose output is `mask`. */

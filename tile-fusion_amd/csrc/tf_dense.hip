@@ -297,9 +297,10 @@ __global__ __launch_bounds__(1024) void gemm_panel_kernel(const float *__restric
 // ---------------------------------------------------------------------------------
 // The same on the bf16 matrix cores (split8 in tf_device.h), for W whose three bf16 parts fit LDS: a step is 32 values of k, W's parts lie
 // in LDS as the matrix cores take them (a lane's eight values of a column in one 16-byte read), X's are made in registers on
-// the way.  Bound: X and Y from HBM behind some 8 us until the first product (262,144 x 128 x 128 63 us, 4.3 TB/s; gemm_panel_kernel 81, waiting for
-// the fp32 cores), and the board's power: the same on operands that are all the same number runs at 5.2 TB/s.  Where W takes two panels the parts
-// of X are made twice: 200,000 x 256 x 128 99 us, 60 at the rate of a copy.
+// the way.  Bound: X and Y from HBM behind some 8 us until the first product (262,144 x 128 x 128 84 us in turn with other
+// operands, gemm_panel_kernel 98, waiting for the fp32 cores; 63 and 81 with six products on a cooler board), and the board's power: the same on operands that are all the
+// same number runs at 5.2 TB/s, and two tiles' products side by side change nothing.  Where W takes two panels the parts of X are made twice:
+// 200,000 x 256 x 128 106 us, 60 at the rate of a copy.
 // What is not finite: a row of X costs its block a second pass on the fp32 cores (100,000 x 128 x 128 39.4 -> 39.6 us, 131,072 x 300 x 64 51.8 -> 58.7; with
 // one load at a time 36 -> 63 and 52 -> 91), a value in W one for every block: 79 and 125 us, 335 where W is N x K (176, 345, 415; a product on
 // the fp32 cores alone 45 and 57).
@@ -641,9 +642,9 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // rows in turn; a workgroup's four are added through LDS, and weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.
 // A lane whose columns would reach past the last one works on the last NB (KB) instead: some values of Y are computed twice.
 // Bound: the rows of X and G from HBM, 16 KB a wavefront in flight, behind some 10 us for two launches and the sums at the end (us, operands in no
-// cache, both launches, fp32 cores on 64 x 160 tiles / this: 14,000 rows 32 x 69 18.2 / 9.5, 35,000 rows 64 x 128 26.1 / 22.5, 100,000 rows 64 x 128 36.6 / 33.0,
-// 20 x 100 26.6 / 22.8, 131,072 rows 64 x 300 75 / 66, 40 x 64 28.3 / 24.4, 262,144 rows 128 x 128 109 / 98; error against 64 bits at 100,000 rows
-// 1.7e-7 / 1.0e-7).
+// cache, both launches, fp32 cores on 64 x 160 tiles / this: 14,000 rows 32 x 69 18.0 / 10.3, 35,000 rows 64 x 128 25.7 / 22.8, 100,000 rows 64 x 128 36.3 / 32.0,
+// 20 x 100 25.9 / 24.1, 131,072 rows 64 x 300 75 / 66, 40 x 64 28.1 / 26.0, 262,144 rows 128 x 128 105 / 94; relative error against 64 bits at 100,000 rows
+// 1.8e-7 / 1.0e-7).
 // ---------------------------------------------------------------------------------
 constexpr int kWgRows = 32;       // rows of a block
 constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel

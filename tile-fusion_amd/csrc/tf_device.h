@@ -217,7 +217,7 @@ template <class T> struct split3 { T h, m, l; };
 
 // Two floats at a time, their parts read back out of the pair of bf16: 26 VALU instructions for four floats.  (Left to itself the compiler converts
 // every value once for the pair and once for the difference: 34.  131,072 rows 300 x 64 34.2 -> 32.3 us, a weight gradient of 300 x 64 and 64 x 40
-// over them 66.0 -> 56.6, 1,049,157 rows 128 x 128 219 -> 211, together with the branch for K's last values in gemm_split_kernel.)
+// over them 66.0 -> 56.6, 1,049,157 rows 128 x 128 219 -> 211, all in six products, together with the branch for K's last values in gemm_split_kernel.)
 __device__ __forceinline__ void split2(float v0, float v1, float scale, unsigned &h, unsigned &m, unsigned &l) {
   typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
   typedef float f2 __attribute__((ext_vector_type(2)));

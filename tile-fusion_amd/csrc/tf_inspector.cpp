@@ -122,8 +122,10 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    (65 to 96 columns: 30,000) only what would be A (B C) otherwise stays in one launch, and gathers of less than 32 columns (one launch
 //    / two; 16,000 rows of 10 entries 64 x 128 16.9 / 15.5, 140 x 143 grid 14.8 / 15.6, 128 x 128 23.6 / 22.2; 21,000 rows of 10
 //    32 x 128 17.7 / 14.5, 128 x 128 32.7 / 27.1; 100,000 rows of 5 32 x 128 37.4 / 29.0, 64 x 128 62 / 45, 64 x 96 52 / 42, 48 x 66
-//    44 / 51, 16 x 96 23.0 / 23.3; 150 x 150 grid 64 x 96 15.1 / 14.3; 180 x 180 16.9 / 16.4, 64 x 128 20.6 / 18.9, 32 x 128 14.4 /
-//    15.0, 16 x 96 9.0 / 11.5; 250 x 250 64 x 128 32.5 / 24.6).
+//    44 / 51, 16 x 96 23.0 / 23.3; 150 x 150 grid 64 x 96 15.1 / 14.3, 32 x 128 14.4 / 12.6; 180 x 180 16 x 96 9.0 / 11.5, 64 x 96 17.2 / 14.7, 64 x 128
+//    20.3 / 17.0; 250 x 250 32 x 96 17.7 / 15.9, 32 x 128 21.1 / 18.1, 64 x 128 32.5 / 24.6.  At 32,400 rows of a grid, which is a whole number of turns
+//    for one launch's workgroups, gathers of 32 columns lose: 32 x 128 14.7 / 14.9, 32 x 96 11.9 / 12.7; as many rows of an Erdos-Renyi graph 16.9 / 14.9
+//    and 14.4 / 13.0).
 //  * as (A B) C in two launches where K is two thirds of N or less: the gathers are K columns wide instead of N.  K = 32, N = 128: 700 x 700
 //    grid 219 us -> 118 us (136 in one launch), 262,144 rows of 16 in a band of 32 (streamed tiles) 86 -> 64 us.
 //  * as A (B C) where tiles need padded copies of B or column panels of D (262,144-row band, 250 x 32: 327 us, as two
@@ -489,7 +491,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       int own = user->tile_rows > 0 ? std::max(user->tile_rows, 64)
                                      : std::max(ceil_div(M, o.compute_units), 128);  // one run per compute unit: a run
       // count that leaves compute units idle costs more than short runs do (32,768 rows: 29 us in 256 runs of 128, 43 us in 128 of 256)
-      own = std::min(own, 1000 * 64 - 2 * ring_rows);  // a run's step table holds 1024 steps
+      // at most 1,024 steps a run, as tf_schedule_validate asks: some 65,000 rows, of which a run's start and halo are less than a hundredth
+      own = std::min(own, 1000 * 64 - 2 * ring_rows);
       const int qspan = ring_rows / 64 - 2;
       // What the consumer wavefronts of the kernel take per step without falling behind, and
       // the longest row a lane group holds in registers.
