@@ -565,13 +565,15 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     // workgroups per panel: a multiple of 8, so that a row block's panels are on one XCD
     const int across = on_bf16 ? std::max(8, compute_units / panels / 8 * 8) : compute_units / std::min(panels, 2);
     int waves = n_blocks >= 16 * compute_units ? 16 : n_blocks >= 8 * compute_units ? 8 : 4;
-    // steps of k in flight: the number that goes into K's without a rest, or nearly (131,072 x 300 x 64: 45 us with five, 52 with four)
+    // steps of k in flight: two, where three or five do not leave less of a rest of K's (us with two / three / four / five: 60,000 x 128 x 64 14.3 /
+    // 15.9 / 15.9 / 16.0, 131,072 x 64 x 64 16.2 / 17.2 / 19.0 / 20.4, 300 x 64 48.5 / 51 / 50.5 / 48.6, 262,144 x 128 x 128 69.6 / 74.5 / 72 / 72.6, 30,000 x 300 x 128
+    // 26.9 / 28.1 / 28.6 / 28.2; three steps of K, 100,000 x 96 x 128 29.2 / 27.7 / 28.8 / 29.4; five, 100,000 x 160 x 64 26.6 / 25.8 / 29.5 / 24.8)
     int ahead = 2;
     if (on_bf16) {
       waves = std::max(4, std::min(kSplitWaves, (n_blocks + across - 1) / across));
       const int steps = (K + 31) / 32;
-      for (int n : {3, 4, 5})
-        if ((steps + n - 1) / n * n <= (steps + ahead - 1) / ahead * ahead && steps > ahead) ahead = n;
+      for (int n : {3, 5})
+        if ((steps + n - 1) / n * n < (steps + ahead - 1) / ahead * ahead) ahead = n;
     }
     const dim3 grid(std::max(1, std::min(across, (n_blocks + waves - 1) / waves)), panels);
     hipError_t err = hipSuccess;
@@ -592,8 +594,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
     if (!on_bf16 && K <= 16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, 1>); }                                              \
     else if (!on_bf16) { CALLP4(gemm_panel_kernel<V_, Q_, WT_, OUT_, kGemmAhead>); }                                           \
     else if constexpr (V_ * Q_ >= 4) {                                                                                         \
-      if (ahead == 4) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 4>); }                                                     \
-      else if (ahead == 5) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 5>); }                                                \
+      if (ahead == 5) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 5>); }                                                \
       else if (ahead == 3) { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 3>); }                                                \
       else { CALLP4(gemm_split_kernel<V_, Q_, WT_, OUT_, 2>); }                                                                \
     }                                                                                                                          \
