@@ -1,0 +1,97 @@
+"""Runs over a grid whose 27-point stencil both matrices are (csrc/tf_box.hip): the oracle's bits at the edges of its
+tiles, strips and planes, and where C holds infinities and NaN; patterns that are nearly the stencil stay with the general runs."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from test_gpu_march import box_stencil, march
+from test_gpu_parity import oracle_spmm_spmm, say
+
+
+# (x, y, z): one and two points more than a column, two planes, one column, fewer lines than a run takes; columns of C: a strip's edges, ragged
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,N", [((9, 31, 12), 64), ((25, 13, 9), 64), ((13, 26, 12), 128), ((30, 40, 2), 64), ((2, 200, 20), 64), ((200, 2, 23), 192),
+                                    ((24, 12, 13), 64), ((48, 47, 50), 37), ((47, 48, 50), 65), ((48, 50, 47), 49)])
+def test_box_bit_exact(gpu, tf, orc, dims, N):
+    say(f"box {dims} N={N}")
+    A = box_stencil(*dims, True, seed=31)
+    B = A.copy()
+    B.data = np.random.default_rng(32).uniform(-1, 1, B.nnz).astype(np.float32)
+    Cd = tf.workloads.uniform((A.shape[0], N), 33)
+    D0 = tf.workloads.uniform((A.shape[0], N), 34)
+    want = oracle_spmm_spmm(orc, A, B, Cd)
+    Ah, Bh = tf.CsrMatrix.from_scipy(A), tf.CsrMatrix.from_scipy(B)
+    for kw in (dict(), dict(compute_units=7)):
+        S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, march=1 if N % 64 == 0 else 0, **kw)
+        S.validate()
+        info = S.info()
+        assert info["marched"] == 1 and info["march_tile_x"] in (8, 12) and info["march_tile_y"] <= 6, info
+        if N % 64 and kw:
+            continue  # (few compute units: more turns of the runs than two products take)
+        for acc in (False, True):
+            D = tf.DenseMatrix(A.shape[0], N, D0) if acc else tf.DenseMatrix(A.shape[0], N)
+            if not acc:
+                D.fill(float("nan"))
+            tf.spmm_spmm(Ah, Bh, tf.DenseMatrix.from_numpy(Cd), D, S, accumulate=acc)
+            tf.device_synchronize()
+            assert np.array_equal(D.to_numpy(), D0 + want if acc else want), (dims, N, kw, acc)
+
+
+@pytest.mark.gpu
+def test_box_keeps_infinities_where_they_are(gpu, tf, orc):
+    """A row of C that is not finite reaches the rows of D within two points of it and no others, at corners and across tiles too."""
+    say("box with infinities and NaN")
+    nx, ny, nz = 20, 13, 14
+    A = box_stencil(nx, ny, nz, True, seed=35)
+    Cd = tf.workloads.uniform((A.shape[0], 64), 36)
+    hit = [0, nx - 1, nx * ny * (nz - 1), (5 * ny + 6) * nx + 12, (7 * ny + 12) * nx + 7]
+    Cd[hit] = np.array([np.inf, -np.inf, np.nan, np.inf, np.nan], np.float32)[:, None]
+    with np.errstate(invalid="ignore"):
+        want = oracle_spmm_spmm(orc, A, A, Cd)
+    got, _ = march(tf, A, A, Cd)
+    assert np.array_equal(got, want, equal_nan=True)
+    reach = np.zeros(A.shape[0], bool)
+    for h in hit:
+        p, q = np.arange(A.shape[0]), h
+        reach |= (abs(p % nx - q % nx) <= 2) & (abs(p // nx % ny - q // nx % ny) <= 2) & (abs(p // nx // ny - q // nx // ny) <= 2)
+    assert np.isfinite(got[~reach]).all()
+
+
+def test_box_only_where_the_pattern_is_the_stencil(tf):
+    """An entry moved, missing or out of order, two patterns of different grids, a wrong grid hint: not this kernel's runs (its columns are 8 or 12
+    by at most 6 points, the general runs' of 27 points 8 by 5 or 4 unless told otherwise) or refused by the validator."""
+    A = box_stencil(24, 20, 18, True, seed=39)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=64, inner=Ah, march=1)
+    S.validate()
+    slots = S.info()["march_slots"]
+    for kind in ("moved", "swapped", "missing", "other"):
+        B = A.copy()
+        mid = B.indptr[(9 * 20 + 10) * 24 + 12]
+        if kind == "moved":
+            B.indices[mid] -= 1
+        elif kind == "swapped":
+            B.indices[mid], B.indices[mid + 1] = B.indices[mid + 1], B.indices[mid]
+        elif kind == "missing":
+            B.data[mid + 3] = 0
+            B.eliminate_zeros()
+        else:
+            B = box_stencil(20, 24, 18, True, seed=39)
+        Bh = tf.CsrMatrix.from_scipy(sp.csr_matrix((B.data, B.indices, B.indptr), shape=B.shape))
+        for outer, inner in ((Bh, Bh), (Ah, Bh), (Bh, Ah)):
+            if kind == "other" and outer is inner:
+                continue
+            try:
+                T = tf.inspector(outer, 1, op=tf.OP_SPMM_SPMM, N=64, inner=inner, march=1)
+                T.validate()
+                assert T.info()["march_slots"] != slots, kind
+            except tf.TileFusionError as e:
+                assert e.status == -5, (kind, str(e))
+        S._inner = Bh
+        with pytest.raises(tf.TileFusionError):
+            S.validate(Bh)
+    S._inner = Ah
+    assert tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=64, inner=Ah, grid=(20, 24, 18)).info()["march_slots"] != slots
+    with pytest.raises(tf.TileFusionError):   # (whole strips, as ever, for who insists on marching runs)
+        tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=48, inner=Ah, march=1)
+    assert tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=64, inner=Ah, march=-1).info()["marched"] == 0

@@ -99,6 +99,7 @@ hipError_t launch_gemm_any(const float *, int, const float *, int, float *, int,
 WeightGradTask plan_weight_grad(int, int, int, int);
 hipError_t launch_weight_grads(const WeightGradTask &, const WeightGradTask *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
+hipError_t launch_fused_box(BoxArgs, int, hipStream_t);
 hipError_t launch_march_fill(const int *, const int *, const float *, const float *, int *, size_t, hipStream_t);
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
                                         const float *, float *, float *, int, int, int, int, int, int, int, hipStream_t);
@@ -244,6 +245,7 @@ static tf_status ensure_device(tf_schedule *s) {
   if (s->two_passes) {  // (the lists are the other schedule's)
     parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
     parts.list(s->l2_tiles, &d->l2_tiles);
+  } else if (s->box) {  // (no lists)
   } else if (s->march) {  // nothing but the run lists is needed on the device
     parts.list(s->march_runs, &d->m_runs);
     parts.list(s->march_row_ptr, &d->m_row_ptr);
@@ -840,6 +842,13 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     }
     if (rc) return rc;
     return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, 0}, false, st);
+  }
+  if (s->box) {
+    tf::BoxArgs a = s->box_runs;
+    a.Ax = A->x; a.Bx = B->x; a.C = C->d; a.D = D->d;
+    a.val_bytes = (unsigned)A->nnz * 4;
+    TF_PHASE(s, "fused_box_kernel", st, tf::launch_fused_box(a, acc, st));
+    return TF_OK;
   }
   if (s->march) {
     // The values in the order of the runs' ELL rows (the reference's reordered adjacency,

@@ -110,6 +110,9 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 13 us, 110,592 rows 34 / 28 us,
 //    216,000 rows 48 / 50 us (N = 128: 97 / 121), 2^21 rows 341 / 610 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
 //    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
+//    Runs over a grid's whole 27-point stencil have a kernel of their own (us, its runs / two products): N = 64, 16^3 points 18 / 8, 32^3 25 / 22,
+//    40^3 31 / 39, 64^3 87 / 136, 96^3 174 / 560; 64^3, N = 16 84 / 59, 32 85 / 86, 37 94 / 124, 96 150 / 240.  Their expected time, a sum over
+//    runs and planes (build_box), against 5 + M (0.11 + 0.0063 N) / 1000, which is within a tenth of two products on up to 64^3 points.
 //
 // GeMM-SpMM:
 //  * as (A B) C in one launch (spmm_gemm_kernel) where no row has its sum from several workgroups and K is narrow.  Under 24,000
@@ -163,7 +166,8 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     }
     if (S->spmm_first) N = K;
   } else if (S->march)
-    want = given.march == 0 && (S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
+    want = given.march == 0 && (S->box ? S->box_us > 5 + S->M * (0.11e-3 + 6.3e-6 * S->opts.N)
+                                       : S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
   else
     want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;
   if (!want) return TF_OK;
@@ -462,7 +466,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 
     // ---- marching runs (stencils on 3D grids: no range of consecutive rows holds a row's dependences) ----
     if (!windowed && have_inner && o.march >= 0) {
-      if (tf::build_march(S, M, Ap, Ai, o.inner_Ap, o.inner_Ai, o, given)) {
+      if (tf::build_box(S, M, Ap, Ai, o.inner_Ap, o.inner_Ai, o, given) || tf::build_march(S, M, Ap, Ai, o.inner_Ap, o.inner_Ai, o, given)) {
         if (tf_status rc = choose_two_passes(S, given, Ap, Ai)) { tf_schedule_free(S); return rc; }
         *out = S;
         return TF_OK;
@@ -1374,7 +1378,7 @@ extern "C" tf_status tf_schedule_validate_inner(const tf_schedule *s, int L, int
         tf_pattern_hash(L, Ap, Ai) != s->pattern_hash)
       return tf::fail(TF_ESCHEDULE, "the schedule's runs were built from another inner pattern");
     if (tf_status rc = validate_two_passes(s, L, M, Ap, Ai)) return rc;
-    return tf::validate_march(s, M, Ap, Ai, inner_Ap, inner_Ai);
+    return s->box ? tf::validate_box(s, M, Ap, Ai, inner_Ap, inner_Ai) : tf::validate_march(s, M, Ap, Ai, inner_Ap, inner_Ai);
   }
   if (tf_status rc = tf_schedule_validate(s, L, M, Ap, Ai)) return rc;
   if (!s->windowed) return TF_OK;

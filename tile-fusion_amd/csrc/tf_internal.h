@@ -107,6 +107,19 @@ struct WeightGradTask {
   size_t partial_floats() const { return few ? 0 : (size_t)blocks() * nb * kb * 256; }
 };
 
+// Runs over the 27-point stencil (tf_box.hip): columns of 2 q x by points.  LDS holds two planes of C with two points around the
+// column and two of the intermediate with one.
+constexpr int kBoxBlock = 1024, kBoxMaxY = 6;
+constexpr int box_lds(int q, int by) { return 512 * ((2 * q + 4) * (by + 4) + (2 * q + 2) * (by + 2)) + 16 * 108 * (2 * q + 1); }
+struct BoxArgs {
+  int nx = 0, ny = 0, nz = 0, N = 0;
+  int q = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x and y, planes a run, strips of 64 columns
+  int per_xcd = 0;                                               // set by the launcher
+  unsigned val_bytes = 0;                                        // of Ax and of Bx
+  const float *Ax = nullptr, *Bx = nullptr, *C = nullptr;
+  float *D = nullptr;
+};
+
 struct DeviceSchedule;  // device copies + workspace, defined in tf_api.cpp
 
 // Marching runs: LDS layout and list format shared by the inspector, the validator and the kernel.
@@ -226,6 +239,10 @@ struct tf_schedule {
   std::vector<int> march_ell_off;    // [march_ell_stride(march_width) per ELL row] LDS byte offset of the row read (the zero row for padding)
   std::vector<int> march_ell_src;    // ... and where its value comes from: index into B's values, or into A's
                                      // with kMarchSrcA set; -1 for padding (value 0)
+  // Runs over a grid whose 27-point stencil both patterns are: marching runs of a kernel of their own, without any of the lists above.
+  bool box = false;
+  tf::BoxArgs box_runs;
+  double box_us = 0;  // what they are expected to take
   // Two-layer tiles (GeMM-SpMM schedules of a square matrix with K and N of 32, 64 or 128, when every tile's two
   // halos fit LDS): what tf_gcn_two_layers runs when this is the second layer's schedule.  l2_lds_bytes: the LDS
   // of the fullest tile (slab A in front, slab B -- X staging, then the hidden rows -- behind it).
@@ -267,6 +284,10 @@ template <class T> tf_status emit_out(const char *who, T *out, T &full, size_t m
 bool build_march(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi,
                  const tf_inspect_opts &o, const tf_inspect_opts &given);
 tf_status validate_march(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi);
+// The same for runs over a 27-point stencil.
+bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi,
+               const tf_inspect_opts &o, const tf_inspect_opts &given);
+tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi);
 void release_device_schedule(DeviceSchedule *d);
 int default_compute_units();
 

@@ -16,6 +16,7 @@
 // schedule slow or impossible, never wrong.
 #include <algorithm>
 #include <climits>
+#include <cstdlib>
 #include <cstring>
 #include <iterator>
 #include <map>
@@ -480,6 +481,138 @@ tf_status validate_march(const tf_schedule *s, int M, const int *Ap, const int *
   if (expect_iter != n_iters) return fail(TF_ESCHEDULE, "marching schedule: iterations left over");
   for (int i = 0; i < M; ++i)
     if (done[i] != 1) return fail(TF_ESCHEDULE, "second-op row %d scheduled %d times", i, done[i]);
+  return TF_OK;
+}
+
+// ---- runs over the 27-point stencil of a grid ------------------------------------------------------------------
+//
+// The kernel (tf_box.hip) computes from a row's grid point where its entries lie and which rows they name, so it needs no lists -- and a
+// pattern that is exactly this one.  Any N.
+namespace {
+
+// The nx x ny x nz grid (two points or more each way, x fastest) on which every row's columns are its point's neighbours
+// within one step in every direction, itself among them, ascending.
+bool box_grid(int M, const int *Ap, const int *Ai, int grid[3]) {
+  if (M < 8 || Ap[1] - Ap[0] != 8) return false;  // row 0: 0, 1, nx, nx + 1, and the same in the next plane
+  const int nx = Ai[2], plane = Ai[4];
+  if (nx < 2 || plane < 2 * nx || plane % nx != 0 || M % plane != 0 || M / plane < 2) return false;
+  const int ny = plane / nx, nz = M / plane;
+  if ((long long)Ap[M] != (3LL * nx - 2) * (3LL * ny - 2) * (3LL * nz - 2)) return false;
+  const int *col = Ai;
+  int row = 0;
+  for (int z = 0; z < nz; ++z)
+    for (int y = 0; y < ny; ++y)
+      for (int x = 0; x < nx; ++x, ++row) {
+        if (Ai + Ap[row] != col) return false;
+        for (int c = std::max(z - 1, 0); c <= std::min(z + 1, nz - 1); ++c)
+          for (int b = std::max(y - 1, 0); b <= std::min(y + 1, ny - 1); ++b)
+            for (int a = std::max(x - 1, 0); a <= std::min(x + 1, nx - 1); ++a)
+              if (*col++ != (c * ny + b) * nx + a) return false;
+      }
+  grid[0] = nx; grid[1] = ny; grid[2] = nz;
+  return true;
+}
+
+constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+}  // namespace
+
+bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi, const tf_inspect_opts &o, const tf_inspect_opts &given) {
+  if (S->L != M || o.inner_cols != M || Ap[M] >= (1 << 29) || Bp[M] != Ap[M]) return false;
+  if (given.march_tile_x > 0 || given.march_tile_y > 0) return false;  // (the general runs take any column)
+  if (given.march > 0 && o.N % 64 != 0) return false;                  // (who insists on marching runs has been told that they take whole strips)
+  int grid[3], inner[3];
+  if (!box_grid(M, Ap, Ai, grid)) return false;
+  if (!(Bp == Ap && Bi == Ai) && (!box_grid(M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner))) return false;
+  if ((given.grid_nx > 0 || given.grid_ny > 0 || given.grid_nz > 0) && (given.grid_nx != grid[0] || given.grid_ny != grid[1] || given.grid_nz != grid[2])) return false;
+  const int nx = grid[0], ny = grid[1], nz = grid[2];
+  if ((long long)nx * ny * o.N * 4 >= UINT_MAX) return false;  // the kernel's offsets in a plane of C
+  // Shape and planes of a run: the least time of the device's turns.  A step takes a compute unit the same time whatever its lines (0.05 us times
+  // 7 q + 12: 2.0 and 2.7 us measured for q = 4 and 6), and a run takes six steps more than the planes it owns.
+  BoxArgs best;
+  const int strips = ceil_div(o.N, 64);
+  S->box_us = 1e30;
+  for (const int q : {4, 6}) {
+    const int tx = ceil_div(nx, 2 * q), ty = ceil_div(ny, kBoxMaxY);
+    for (int cuts = 1; cuts <= nz; ++cuts) {
+      const int zlen = ceil_div(nz, cuts);
+      if (cuts > 1 && zlen == ceil_div(nz, cuts - 1)) continue;
+      const long long runs = (long long)tx * ty * ceil_div(nz, zlen) * strips;
+      if (runs > (1 << 24)) break;
+      const double us = 8 + 0.05 * (7 * q + 12) * (double)((runs + o.compute_units - 1) / o.compute_units) * (zlen + 6);
+      if (us < S->box_us) {
+        S->box_us = us;
+        best.q = q; best.by = ceil_div(ny, ty); best.tx = tx; best.ty = ty; best.zlen = zlen; best.n_runs = (int)runs;
+      }
+    }
+  }
+  if (best.q == 0) return false;
+  best.nx = nx; best.ny = ny; best.nz = nz; best.N = o.N; best.strips = strips;
+  S->march = S->box = true;
+  S->box_runs = best;
+  std::copy(grid, grid + 3, S->march_grid);
+  S->march_tile[0] = 2 * best.q; S->march_tile[1] = best.by;
+  S->lds_bytes = box_lds(best.q, best.by);
+  S->march_slots = S->slab_rows = S->lds_bytes / kMarchRowBytes;
+  S->march_width = 27;
+  S->fused_nnz = S->inner_nnz = Ap[M];
+  S->inner_hash = Bp == Ap && Bi == Ai ? S->pattern_hash : tf_pattern_hash(M, Bp, Bi);
+  S->march_declined = TF_MARCH_BUILT;
+  // MultiDimensionalSet-layout view: one partition per run (all its strips), its points as first-op ids and again as second-op ids
+  S->n_producer_rows = 0;
+  S->fused_ids.reserve(M); S->id.reserve(2 * (size_t)M); S->type.reserve(2 * (size_t)M);
+  S->ptr2.assign(1, 0);
+  for (int z0 = 0; z0 < nz; z0 += best.zlen)
+    for (int y0 = 0; y0 < ny; y0 += best.by)
+      for (int x0 = 0; x0 < nx; x0 += 2 * best.q) {
+        const int x1 = std::min(nx, x0 + 2 * best.q), y1 = std::min(ny, y0 + best.by), z1 = std::min(nz, z0 + best.zlen);
+        TileDesc t{};
+        t.cons_begin = (int)S->fused_ids.size();
+        for (int z = z0; z < z1; ++z)
+          for (int y = y0; y < y1; ++y)
+            for (int x = x0; x < x1; ++x) S->fused_ids.push_back((z * ny + y) * nx + x);
+        t.cons_end = (int)S->fused_ids.size();
+        t.own_begin = t.prod_begin = t.wb_begin = t.wb_end = S->fused_ids[t.cons_begin];
+        t.own_end = t.prod_end = S->fused_ids.back() + 1;
+        S->n_producer_rows += (long long)(std::min(nx, x1 + 1) - std::max(0, x0 - 1)) * (std::min(ny, y1 + 1) - std::max(0, y0 - 1)) * (std::min(nz, z1 + 1) - std::max(0, z0 - 1));
+        for (int type = 0; type < 2; ++type) {
+          S->id.insert(S->id.end(), S->fused_ids.begin() + t.cons_begin, S->fused_ids.begin() + t.cons_end);
+          S->type.insert(S->type.end(), (size_t)(t.cons_end - t.cons_begin), type);
+          S->ker_begin.push_back((int)S->id.size());
+        }
+        S->ptr2.push_back((int)S->id.size());
+        for (const int v : {t.prod_begin, t.prod_end, t.own_begin, t.own_end}) S->tile_range.push_back(v);
+        S->writeback.push_back(t.own_begin); S->writeback.push_back(t.own_begin);
+        S->tiles.push_back(t);
+      }
+  S->launch_tiles = S->tiles;
+  const int nt = (int)S->tiles.size();
+  S->ptr1 = {0, nt, nt};
+  return true;
+}
+
+// That both patterns are the grid's, that the runs fit LDS and own every point once, as the kernel deals them.
+tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi) {
+  const BoxArgs &b = s->box_runs;
+  int grid[3], inner[3];
+  if (!box_grid(M, Ap, Ai, grid) || !box_grid(M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner) || grid[0] != b.nx || grid[1] != b.ny || grid[2] != b.nz)
+    return fail(TF_ESCHEDULE, "runs over a %d x %d x %d grid: the patterns are not its 27-point stencil", b.nx, b.ny, b.nz);
+  if (b.N != s->opts.N || b.strips != ceil_div(b.N, 64) || b.by < 1 || b.by > kBoxMaxY || s->lds_bytes != box_lds(b.q, b.by) || s->lds_bytes > kMaxLds)
+    return fail(TF_ESCHEDULE, "runs over a grid: %d columns, %d lines, %d bytes of LDS", b.N, b.by, s->lds_bytes);
+  const int cuts = b.zlen > 0 ? ceil_div(b.nz, b.zlen) : 0;
+  if (cuts < 1 || b.q < 1 || b.tx != ceil_div(b.nx, 2 * b.q) || b.ty != ceil_div(b.ny, b.by) || (long long)b.tx * b.ty * cuts * b.strips != b.n_runs ||
+      s->tiles.size() != (size_t)b.tx * b.ty * cuts)
+    return fail(TF_ESCHEDULE, "runs over a grid: %d runs of %d planes do not cover it", b.n_runs, b.zlen);
+  std::vector<char> done(M, 0);
+  for (size_t r = 0; r < s->tiles.size(); ++r) {
+    const TileDesc &t = s->tiles[r];
+    for (int q = t.cons_begin; q < t.cons_end; ++q) {
+      const int i = s->fused_ids[q], x = i % b.nx, y = i / b.nx % b.ny, z = i / b.nx / b.ny;
+      if (i < 0 || i >= M || done[i]++ || (size_t)((z / b.zlen * b.ty + y / b.by) * b.tx + x / (2 * b.q)) != r)
+        return fail(TF_ESCHEDULE, "runs over a grid: row %d is not run %zu's, or twice there", i, r);
+    }
+  }
+  if (s->fused_ids.size() != (size_t)M) return fail(TF_ESCHEDULE, "runs over a grid: %zu of %d rows", s->fused_ids.size(), M);
   return TF_OK;
 }
 
