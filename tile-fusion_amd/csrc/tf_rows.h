@@ -31,9 +31,13 @@ inline RowShape row_shape(int N, int accumulate) {
 // 41.8 / 42.7).
 // The last slice's last lane may not reach back into the slice before it where Y is added to: workgroups of two XCDs would both
 // add to those columns, and one that loads after the other has stored adds twice.  (N = 97 .. 99: whole rows.)
+// A few long rows' chunks beside them, which take all columns slice by slice, do not matter, many do (Erdos-Renyi with some rows of more than 32
+// entries, N = 128, whole rows / slices, two products: 20,000 rows 38.9 / 29.0, 28,334 rows of 16 56.8 / 40.0, 50,000 rows of 17 118 / 88; N = 64, 60,000 rows
+// 65.8 / 58.1; a layer forward and backward, 100 -> 128, 60,000 rows 216 / 194; power-law graphs, a tenth of whose rows are long: 2^14 nodes, 96 -> 128 34 / 36,
+// 2^16 50 / 54).
 constexpr int kSliceCols = 32;
 inline int slices_for(const RowsArgs &a) {
-  if (a.ldx % 32 != 0 || (reinterpret_cast<uintptr_t>(a.X) & 127u)) return 1;
+  if (a.ldx % 32 != 0 || (reinterpret_cast<uintptr_t>(a.X) & 127u) || (long long)a.n_chunks * 256 > a.n_rows) return 1;
   const long long bytes = (long long)a.x_rows * a.ldx * 4;
   int slices = 1;
   if (a.N > 96 && a.N <= 128 && a.x_rows >= 16000 && bytes <= (64LL << 20)) slices = 4;

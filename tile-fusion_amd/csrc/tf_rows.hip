@@ -525,7 +525,7 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   if (a.n_rows <= 0 && a.n_chunks <= 0) return hipSuccess;
   RowShape s = row_shape(a.N, a.accumulate);
   a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
-  a.slices = s.V == 4 && !how.flagged && a.n_chunks == 0 && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
+  a.slices = s.V == 4 && !how.flagged && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
   if (a.slices > 1) s.LPR = kSliceCols / 4;
   const int G = kBlock / s.LPR;
   a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
