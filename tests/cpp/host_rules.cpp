@@ -58,6 +58,44 @@ static int column_owners() {
   return bad;
 }
 
+// The same for sweep_rows_kernel: a lane group takes a slice's columns in one go, X is within the 32 bits of its offsets, and the limit is behind it
+// after the steps.
+static int sweep_columns() {
+  int bad = 0, shapes[3] = {};
+  for (int N = 1; N <= 140; ++N)
+    for (long long rows : {1000LL, 29000LL, 30000LL, 60000LL, 90000LL, 125000LL, 300000LL, 1000000LL, 17000000LL})
+      for (int ldx : {N, (N + 31) / 32 * 32})
+        for (int off : {0, 16})
+          for (int accumulate : {0, 1})
+            for (int mean : {5, 6, 40}) {
+              tf::RowsArgs a;
+              tf::RowsHow how;
+              a.X = reinterpret_cast<const float *>((uintptr_t)4096 + off);
+              a.ldx = ldx; a.N = N; a.n_rows = (int)rows; a.x_rows = (unsigned)rows; a.accumulate = accumulate;
+              how.spread_entries = rows * mean;
+              const tf::SweepShape s = tf::sweep_for(a, how);
+              if (s.LPR == 0) continue;
+              ++shapes[s.slices / 2];
+              std::vector<int> owners(N, 0);
+              for (int slice = 0; slice < s.slices; ++slice) {
+                std::vector<char> mine(N, 0);
+                for (int lane = 0; lane < s.LPR; ++lane) {
+                  const int col = slice * s.LPR * 4 + lane * 4;
+                  if (col >= N) continue;
+                  for (int u = 0; u < 4; ++u) mine[tf::clamp_col<4>(col, N) + u] = 1;
+                }
+                for (int c = 0; c < N; ++c) owners[c] += mine[c];
+              }
+              bool ok = (s.LPR == 4 || s.LPR == 8 || s.LPR == 16 || s.LPR == 32) && s.LPR * 4 * s.slices >= N && 8 % s.slices == 0 && mean >= 6;
+              for (int c = 0; c < N; ++c) ok = ok && owners[c] >= 1 && (!accumulate || owners[c] == 1);
+              const unsigned long long bytes = (unsigned long long)rows * ldx * 4, step = bytes / s.steps + 1;
+              ok = ok && bytes <= 0x80000000ull && s.steps >= mean && step * s.steps >= bytes && step * s.steps < 0xffffffffull;
+              if (!ok) { printf("N %d ldx %d rows %lld accumulate %d: %d lanes, %d slices, %d steps\n", N, ldx, rows, accumulate, s.LPR, s.slices, s.steps); ++bad; }
+            }
+  for (int n : shapes) bad += n == 0;
+  return bad;
+}
+
 // Layers that run in one launch: the rows of A B that a workgroup holds fit its LDS, at every K; wider ones are inspected into something
 // else and accepted all the same.
 static int one_launch_fits() {
@@ -211,7 +249,7 @@ static int streamed_entries() {
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
-    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
+    const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "sweep_columns") ? sweep_columns() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
                   : !strcmp(argv[k], "partial_sums") ? partial_sums()
                   : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns()
                   : !strcmp(argv[k], "streamed_entries") ? streamed_entries() : 1;

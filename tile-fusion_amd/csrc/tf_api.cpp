@@ -414,6 +414,7 @@ static tf_status remainder_rows(const tf_csr *A, tf_schedule *s, const Remainder
   a.X = r.T; a.ldx = r.ldt; a.x_rows = r.rows; a.Y = r.D; a.ldy = ldd; a.N = N;
   a.accumulate = r.accumulate; a.relu = r.relu; a.streaming = r.streaming;
   how.xcd_chunk_rows = s->row_deal;
+  how.spread_entries = s->rem_sweep ? A->nnz : 0;
   a.zero_rows = d->zero_rows;
   a.n_zero = r.accumulate && !r.relu ? 0 : (int)s->zero_rows.size();  // (D += 0 needs nothing)
   a.chunks = d->long_chunks;

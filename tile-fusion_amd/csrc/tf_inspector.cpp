@@ -640,14 +640,48 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // inside a group), and a group is worked on, like a short row, by the XCD of its partition;
     // entries outside all partitions ("cold") go to all XCDs as before.  Groups are cut into
     // segments of at most 64 entries; a row's segments are added up in a fixed order.
+    auto scattered = [&] {  // (some 8,192 rows are looked at)
+      const size_t n = S->rem_rows.size(), step = n / 8192 + 1;
+      double far = 0;
+      long long entries = 0;
+      for (size_t q = 0; q < n; q += step) {
+        const int i = S->rem_rows[q];
+        for (int k = Ap[i]; k < Ap[i + 1]; ++k) far += std::abs(Ai[k] - (double)i * M / L);
+        entries += Ap[i + 1] - Ap[i];
+      }
+      return far * 8 > (double)M * entries;
+    };
+    // Rows of some entries each, spread over all columns with none read much more than the others (an Erdos-Renyi graph): the row product
+    // takes them in the matrix' own order and lets all rows in flight read the same part of X (sweep_rows_kernel), without a list.
+    auto for_sweep = [&] {
+      if ((int)(S->rem_rows.size() + S->long_rows.size()) != L || S->rem_rows.empty() || !tf::sweep_fits(M, o.N, L, nnz)) return false;
+      if (user->long_row_nnz > 0 || user->long_row_partition > 0 || given.reorder_adjacency > 0 || given.place_intermediate > 0 || given.short_row_hot_bytes > 0 ||
+          o.xcd_chunk_rows != 0)
+        return false;
+      for (const auto &lr : S->long_rows)
+        if (Ap[lr.row + 1] - Ap[lr.row] > kWholeRowMax) return false;
+      if (!scattered()) return false;
+      // The most-read eighth of the columns takes less than a quarter of the reads: summed up from the most-read ones down.
+      std::vector<int> reads(M, 0), of_count(256, 0);
+      for (long long k = 0; k < nnz; ++k) ++reads[Ai[k]];
+      for (int r : reads) ++of_count[std::min(r, 255)];
+      long long left = M / 8, taken = 0;
+      for (int c = 255; c >= 0 && left > 0; --c) {
+        const long long cols = std::min<long long>(left, of_count[c]);
+        taken += cols * c;
+        left -= cols;
+      }
+      return of_count[255] == 0 && 4 * taken < nnz;
+    };
+    const bool sweep = for_sweep();
     std::vector<signed char> part;  // per intermediate row: its hot partition, or -1 (empty without long_part)
     {
       long long long_nnz = 0;
       for (const auto &lr : S->long_rows) long_nnz += Ap[lr.row + 1] - Ap[lr.row];
       // (narrower rows are not worth partial sums of their own: 2^20 nodes, N = 32 / 48 / 64, chunks 242 / 432 / 550 us, partitions
       // 294 / 438 / 472)
-      const bool want = o.long_row_partition > 0 ||
-                        (o.long_row_partition == 0 && long_nnz >= (1 << 20) && (long long)M * o.N * 4 > (64LL << 20) && o.N >= 56);
+      const bool want = !sweep && (o.long_row_partition > 0 ||
+                                   (o.long_row_partition == 0 && long_nnz >= (1 << 20) && (long long)M * o.N * 4 > (64LL << 20) && o.N >= 56));
       // (three times an L2's 4 MB measured best on the R-MAT graph: 2.68 ms per step with 4 MB, 2.54 with 12 or
       // 16 MB, 2.60 with 32 MB -- the reads inside a partition are skewed too, and its hottest rows are what stays)
       const int part_rows = std::max(64, (o.hot_partition_bytes > 0 ? o.hot_partition_bytes : (12 << 20)) / (o.N * 4));
@@ -658,7 +692,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       // themselves.  R-MAT graphs, rows of up to 32 / 64 / 128 entries kept whole: 2^16 nodes, N = 8 / 64, 25.9 / 25.8 / 36.7 and 37.4 / 36.1 / 38.3 us,
       // 2^17 nodes 37 / 40.7 / 47.3 and 56 / 52.9 / 52.4, 2^18 nodes 64 / 61 / 70 and 107 / 104 / 96, 2^20 nodes 196 / 194 / 178 and
       // 555 / 556 / 555 (N = 32: 279 / 270 / 242).
-      const int whole = want ? 64 : L >= 200000 && o.N >= 16 ? kWholeRowMax : L >= 100000 && o.N >= 48 ? 64 : 32;
+      const int whole = sweep ? kWholeRowMax : want ? 64 : L >= 200000 && o.N >= 16 ? kWholeRowMax : L >= 100000 && o.N >= 48 ? 64 : 32;
       if (user->long_row_nnz <= 0 && whole > o.long_row_nnz && S->long_chunks.size() < (size_t)INT_MAX) {
         std::vector<tf::LongRow> keep_rows;
         std::vector<tf::LongChunk> keep_chunks;
@@ -804,23 +838,12 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         const int len = Ap[i + 1] - Ap[i];
         return len <= 8 ? 0 : len <= 32 ? 1 : len <= 128 ? 2 : len <= 512 ? 3 : 4;
       };
-      auto scattered = [&] {  // (some 8,192 rows are looked at)
-        const size_t n = S->rem_rows.size(), step = n / 8192 + 1;
-        double far = 0;
-        long long entries = 0;
-        for (size_t q = 0; q < n; q += step) {
-          const int i = S->rem_rows[q];
-          for (int k = Ap[i]; k < Ap[i + 1]; ++k) far += std::abs(Ai[k] - (double)i * M / L);
-          entries += Ap[i + 1] - Ap[i];
-        }
-        return far * 8 > (double)M * entries;
-      };
       // Rows without entries, when they are many (half of the nodes of an R-MAT graph are isolated), leave the list: a row of
       // zeros needs no lane group of its own and no row pointers, the row kernels clear it beside their other work.
       {
         size_t n_empty = 0;
         for (int i : S->rem_rows) n_empty += Ap[i + 1] == Ap[i];
-        if (n_empty >= 4096 && n_empty * 8 >= S->rem_rows.size() && n_empty < S->rem_rows.size()) {
+        if (!sweep && n_empty >= 4096 && n_empty * 8 >= S->rem_rows.size() && n_empty < S->rem_rows.size()) {
           std::vector<int> keep;
           keep.reserve(S->rem_rows.size() - n_empty);
           S->zero_rows.reserve(n_empty);
@@ -833,8 +856,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       // (a product of all rows whose rows are nearly all of one class -- a stencil and its boundary -- stays in order too: the
       // list costs its rows an indirection and the entries a copy; 27 points, 40^3, N = 16: 21.1 us through a list, 19.1 without)
       const size_t most = *std::max_element(in_class, in_class + 5);
-      const bool far = scattered();
-      if (!((int)S->rem_rows.size() == L && most * 8 >= S->rem_rows.size() * 7)) {
+      const bool far = sweep || scattered();
+      if (!sweep && !((int)S->rem_rows.size() == L && most * 8 >= S->rem_rows.size() * 7)) {
         if (far) {
           std::vector<int> at(o.long_row_nnz + 2, 0);  // (no remainder row is longer)
           const std::vector<int> rows(S->rem_rows);
@@ -855,6 +878,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       // to the XCDs in turn / a run each: 7 points, 60^3, N = 32, 44 / 30 us, 30 x 40 x 50, N = 64, 30.5 / 18; 27 points, 24^3, N = 32, 13.1 / 10.8, 60^3
       // 85 / 75; 5 points, 900^2, N = 32, 120 / 95.  Past 100 MB of X the runs' planes outgrow the Infinity Cache together, and turns of
       // 512 rows are better: 7 points, 110^3, N = 32, 293 / 252 / 231 in turns.
+      S->rem_sweep = sweep && S->rem_identity;
       S->row_deal = o.xcd_chunk_rows;
       if (S->rem_identity && !far && o.xcd_chunk_rows == 0) {
         constexpr int kXcds = 8;

@@ -82,9 +82,12 @@ struct RowsArgs {
   unsigned *arrived = nullptr;
   unsigned chunk_blocks = 0;          // set by the launcher
   int n_blocks = 0, per_xcd = 0, slices = 1;  // set by the launcher
+  int sweep_steps = 0;                        // ... for sweep_rows_kernel: steps in which its window passes over X,
+  unsigned sweep_bytes = 0;                   // and by how much in each
 };
 struct RowsHow {
   int xcd_chunk_rows = 0;   // how row blocks are dealt to the XCDs (tf_inspect_opts.xcd_chunk_rows)
+  long long spread_entries = 0;  // of all rows where their columns are spread over X alike, rising in each row (0: they are not, or nobody knows)
   int flagged = 0;          // columns carry the "cold" mark
 };
 
@@ -184,6 +187,7 @@ struct tf_schedule {
   std::vector<int> rem_rows;        // remainder rows handled one row per lane group, ordered by
                                     // length class so that a workgroup's rows cost about the same
   bool rem_identity = false;        // rem_rows is 0..L-1 in order
+  bool rem_sweep = false;           // ... whose columns are spread over all alike (RowsHow::spread_entries)
   std::vector<int> zero_rows;       // second-op rows without entries, when many: their rows of D are cleared by a
                                     // fill kernel instead of taking a lane group each in the row kernel
   // When the list is not the identity, its rows are also kept as a CSR of their own in list order

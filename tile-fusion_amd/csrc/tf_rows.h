@@ -1,6 +1,7 @@
 // How the row kernels (tf_rows.hip) deal a row's columns to lanes and XCDs.  Host rules without a HIP header, so that a
 // test can enumerate which lane stores which column.
 #pragma once
+#include <algorithm>
 #include <climits>
 
 #include "tf_internal.h"
@@ -44,6 +45,41 @@ inline int slices_for(const RowsArgs &a) {
   else if (a.N > 48 && a.N <= 64 && a.compact && !a.val_first && a.x_rows >= 24000 && bytes <= (40LL << 20)) slices = 2;
   if (a.accumulate && a.N - 4 < (slices - 1) * kSliceCols) slices = 1;
   return slices;
+}
+
+// sweep_rows_kernel: rows of some entries each, spread over an X that no L2 holds and the Infinity Cache does.  Erdos-Renyi graphs, one product,
+// the other kernel / this one (us; a layer's two products with values read in place in brackets): N = 64, 60,000 rows of 11 20.3 / 20.8
+// (47.2 / 41.8), 100,000 38.2 / 34.1 (83 / 69), 200,000 82.9 / 77.7 (177 / 156); N = 128, 30,000 rows 15.7 / 18.0 (34.6 / 35.7), 60,000 38.5 / 38.4 (88 / 77),
+// 100,000 77.5 / 67.0 (173 / 137), 200,000 168 / 156 (344 / 315), 400,000 335 / 334 (690 / 656); N = 32, 200,000 rows 42.4 / 40.4 (95 / 83); N = 16,
+// 250,000 rows 44.1 / 36.9 (106 / 78).  Not below 15 MB of X (36,000 rows of 13, N = 100: 21.3 / 23.2), where it outgrows the Infinity Cache (10^6 rows of
+// 9, N = 64: 355 / 359), for fewer than 5.5 entries a row (200,000 rows of 4, N = 64: 35.8 / 37.2), or where a row is three quarters of a lane group
+// (120,000 rows, N = 80: 68 / 70).
+constexpr int kSweepRows = 4, kSweepEntries = 16;
+constexpr bool sweep_fits(long long x_rows, int N, long long rows, long long entries) {
+  return N >= 4 && (N <= 64 || (N > 96 && N <= 128)) && x_rows * N * 4 >= 15000000 && x_rows * N * 4 <= (256ll << 20) && 2 * entries >= 11 * rows;
+}
+// Lanes a row takes, column slices, and the steps in which the limit passes over X.  Slices as above where rows start at a line, of 64 columns where four
+// of 32 do not pay: as long as an XCD's slice is small enough that most of it is read by more than one row in flight (N = 128, whole rows / two slices / four:
+// 60,000 rows 45 / 38.4 / 38.8, 100,000 78 / 69.5 / 67, 200,000 162 / 156 / 164; N = 64, whole / two, 100,000 36.5 / 34.1, 200,000 79.5 / 77.7,
+// 400,000 168 / 185).  More steps than entries, or rows that have two close together fall behind (steps per entry 1 / 1.5 / 2: N = 64, 60,000 rows
+// 20.2 / 20.8 / 22.6, 100,000 35.6 / 34.1 / 36.6, 200,000 85 / 80 / 78).
+struct SweepShape { int LPR = 0, slices = 1, steps = 0; };
+inline SweepShape sweep_for(const RowsArgs &a, const RowsHow &how) {
+  SweepShape s;
+  const long long bytes = (long long)a.x_rows * a.ldx * 4;
+  if (how.spread_entries <= 0 || how.flagged || how.xcd_chunk_rows != 0 || a.n_chunks > 0 || a.rows || a.n_zero > 0 ||
+      !sweep_fits(a.x_rows, a.N, a.n_rows, how.spread_entries) || bytes > 0x80000000ll)
+    return s;
+  s.LPR = a.N <= 16 ? 4 : row_shape(a.N, 0).LPR;
+  if (a.ldx % 32 == 0 && !(reinterpret_cast<uintptr_t>(a.X) & 127u)) {
+    if (a.N > 96 && bytes > (40 << 20) && bytes <= (64 << 20)) s.LPR = 8, s.slices = 4;
+    else if (a.N > 96) s.LPR = 16, s.slices = 2;
+    else if (a.N > 48 && bytes <= (64 << 20)) s.LPR = 8, s.slices = 2;
+    // (as in slices_for)
+    if (a.accumulate && a.N - 4 < (s.slices - 1) * s.LPR * 4) s.LPR = row_shape(a.N, 0).LPR, s.slices = 1;
+  }
+  s.steps = (int)((bytes > (32 << 20) ? 4 : 3) * how.spread_entries / (2 * a.n_rows)) + 1;
+  return s;
 }
 
 // spmm_gemm_kernel: rows of A X a workgroup holds in LDS, and the LDS they take (K columns in steps of 16, four floats behind

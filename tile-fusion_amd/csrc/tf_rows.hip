@@ -317,6 +317,103 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(const RowsArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
+// The same for rows whose columns rise and are spread over an X that no L2 holds: all rows in flight read the same stretch of X at the
+// same time.  A lane group owns kSweepRows rows and takes at most one entry of each per step, if its column lies in front of a
+// limit that rises with the steps; every XCD's workgroups (of one column slice where there are slices) start together and take steps of the same
+// length, so that more of an XCD's gathers hit what another row has just fetched.  Bound: the lines that come from the Infinity Cache once
+// per XCD and generation of workgroups, then L2 (100,000 rows of 11, N = 128: 67 us, 563 MB gathered; 77.5 in spmm_rows_kernel).  Nothing depends on the timing but time: entries are added in the row's order.
+// Four rows a group are what 64 registers hold, of eight wavefronts per SIMD; eight rows and half the wavefronts read the same at N = 64 (36.1 / 34.2 us)
+// and 4 % faster at 128.  Each lane group keeps kSweepEntries entries of each row in LDS, behind them a mark that lies in front of no limit, and refills when its
+// wavefront has used all of them up.
+// ---------------------------------------------------------------------------------
+constexpr unsigned kSweepEnd = 0xffffffffu;
+template <int LPR>
+__global__ __launch_bounds__(kBlock, LPR == 4 ? 4 : 8) void sweep_rows_kernel(const RowsArgs a) {
+  constexpr int G = kBlock / LPR, R = kSweepRows, E = kSweepEntries;
+  __shared__ uint2 pairs[G][R][E + 1];  // byte offset in X and value
+  const int group = threadIdx.x / LPR, glane = threadIdx.x % LPR;
+  asm volatile("" ::"s"(a.Ap), "s"(a.Ai), "s"(a.Ax), "s"(a.X), "s"(a.Y), "s"(a.ldx), "s"(a.ldy), "s"(a.N), "s"(a.n_rows), "s"(a.accumulate),
+               "s"(a.streaming), "s"(a.relu), "s"(a.slices), "s"(a.sweep_steps), "s"(a.sweep_bytes));
+  const int xcd = blockIdx.x % kXcds, b = blockIdx.x / kXcds * (kXcds / a.slices) + xcd / a.slices;
+  const int c_begin = xcd % a.slices * (LPR * 4);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X), 0, (int)(a.x_rows * a.ldx * 4u), 0x00020000);
+  const int q0 = (b * G + group) * R, n = min(max(a.n_rows - q0, 0), R);  // (a group without rows stays with its wavefront)
+  const int col = c_begin + glane * 4, coff = clamp_col<4>(col, a.N);
+  const bool ok = col < a.N;
+  int at[R + 1];  // the rows' next entries to go to LDS, and their end
+#pragma unroll
+  for (int r = 0; r <= R; ++r) at[r] = n > 0 ? a.Ap[q0 + min(r, n)] : 0;
+  int len[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) len[r] = at[r + 1] - at[r];
+  fvec<4> acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    acc[r] = vzero<4>();
+    if (a.accumulate && ok && r < n) acc[r] = load_any<4>(a.Y + (size_t)(q0 + r) * a.ldy + coff);
+  }
+  unsigned limit = a.sweep_bytes;
+  int steps = a.sweep_steps;
+  for (;;) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int k0 = 0; k0 <= E; k0 += LPR) {
+        const int k = k0 + glane;
+        uint2 e = {kSweepEnd, 0u};
+        if (k < E && k < len[r]) {
+          e.x = (unsigned)a.Ai[at[r] + k] * (a.ldx * 4u);
+          e.y = __float_as_uint(a.Ax[at[r] + k]);
+        }
+        if (k <= E) pairs[group][r][k] = e;
+      }
+    // (a lane group reads what its own lanes have written: of one wavefront, in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    int k[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) k[r] = 0;
+    for (;;) {
+      f4 x[R];
+      float v[R];
+      bool left = false;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint2 e = pairs[group][r][k[r]];
+        const bool take = e.x < limit;  // (never the mark)
+        left |= e.x != kSweepEnd;
+        x[r] = buffer_gather(xr, take ? e.x + coff * 4u : 0x80000000u);  // (past the end of X: zeros, without a memory access)
+        v[r] = take ? __uint_as_float(e.y) : 0.f;
+        k[r] += take;
+      }
+      if (!__ballot(left)) break;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[r].v[u] = __builtin_fmaf(v[r], x[r][u], acc[r].v[u]);
+      limit = --steps > 0 ? limit + a.sweep_bytes : kSweepEnd;
+    }
+    bool more = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      at[r] += E;
+      len[r] -= E;
+      more |= len[r] > 0;
+    }
+    if (!__ballot(more)) break;
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r < n && ok) {
+      if (a.relu) relu_of<4>(acc[r]);
+      store_any<4>(a.Y + (size_t)(q0 + r) * a.ldy + coff, acc[r], a.streaming);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------
 // Y = (A X) W in one launch: the rows of A X, K columns wide, are gathered as in spmm_rows_kernel into LDS, R of them a
 // workgroup, and multiplied by W (K x N, or N x K with WT) on v_mfma_f32_16x16x4_f32; neither intermediate nor second
 // launch.  In the product a wavefront owns 16 rows and 16 V columns (column V j + v of its panel is column block v's lane j).
@@ -527,6 +624,19 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
   a.slices = s.V == 4 && !how.flagged && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
   if (a.slices > 1) s.LPR = kSliceCols / 4;
+  const SweepShape sweep = s.V == 4 ? sweep_for(a, how) : SweepShape{};
+  if (sweep.LPR > 0) {
+    const int rows = kBlock / sweep.LPR * kSweepRows, per = kXcds / sweep.slices;
+    a.slices = sweep.slices;
+    a.n_blocks = (a.n_rows + rows - 1) / rows;
+    a.sweep_steps = sweep.steps;
+    a.sweep_bytes = (unsigned)((unsigned long long)a.x_rows * a.ldx * 4 / sweep.steps + 1);
+    const dim3 grid((a.n_blocks + per - 1) / per * kXcds);
+#define CALLS(L_) hipLaunchKernelGGL((sweep_rows_kernel<L_>), grid, dim3(kBlock), 0, st, a)
+    if (sweep.LPR == 4) CALLS(4); else if (sweep.LPR == 8) CALLS(8); else if (sweep.LPR == 16) CALLS(16); else CALLS(32);
+#undef CALLS
+    return hipGetLastError();
+  }
   const int G = kBlock / s.LPR;
   a.n_blocks = (std::max(a.n_rows, 0) + G - 1) / G;
   const int blocks = deal_to_xcds(a, how.xcd_chunk_rows, G);
