@@ -100,6 +100,7 @@ WeightGradTask plan_weight_grad(int, int, int, int);
 hipError_t launch_weight_grads(const WeightGradTask &, const WeightGradTask *, hipStream_t);
 hipError_t launch_gather_values(const int *, const float *, float *, int, hipStream_t);
 hipError_t launch_fused_box(BoxArgs, int, hipStream_t);
+hipError_t launch_fused_star(BoxArgs, int, hipStream_t);
 hipError_t launch_march_fill(const int *, const int *, const float *, const float *, int *, size_t, hipStream_t);
 hipError_t launch_fused_spmm_spmm_march(const int *, int, const int *, const int *, const int *, const int *, const int *,
                                         const float *, float *, float *, int, int, int, int, int, int, int, hipStream_t);
@@ -848,7 +849,8 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     tf::BoxArgs a = s->box_runs;
     a.Ax = A->x; a.Bx = B->x; a.C = C->d; a.D = D->d;
     a.val_bytes = (unsigned)A->nnz * 4;
-    TF_PHASE(s, "fused_box_kernel", st, tf::launch_fused_box(a, acc, st));
+    if (a.star) TF_PHASE(s, "fused_star_kernel", st, tf::launch_fused_star(a, acc, st));
+    else TF_PHASE(s, "fused_box_kernel", st, tf::launch_fused_box(a, acc, st));
     return TF_OK;
   }
   if (s->march) {

@@ -113,6 +113,9 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    Runs over a grid's whole 27-point stencil have a kernel of their own (us, its runs / two products): N = 64, 16^3 points 18 / 8, 32^3 25 / 22,
 //    40^3 31 / 39, 64^3 87 / 136, 96^3 174 / 560; 64^3, N = 16 84 / 59, 32 85 / 86, 37 94 / 124, 96 150 / 240.  Their expected time, a sum over
 //    runs and planes (build_box), against 5 + M (0.11 + 0.0063 N) / 1000, which is within a tenth of two products on up to 64^3 points.
+//    So have runs over its whole 7-point stencil (us, its runs / two products / the other runs): N = 64, 24^3 points 11.3 / 8.6, 32^3 11.3 / 11.5, 40^3 15.9 /
+//    18.6, 64^3 34 / 59 / 49, 96^3 114 / 294 / 181, 128^3 230 / 619 / 290; N = 128, 32^3 14.5 / 18.9, 64^3 60 / 136 / 97; 128^3, N = 32 130 / 352, 100 728 / 1,120; 90 x 70
+//    x 80, N = 36 70 / 103; against 4 + M (N, in whole lines) 0.0034 / 1000.  Any N of a multiple of four.
 //
 // GeMM-SpMM:
 //  * as (A B) C in one launch (spmm_gemm_kernel) where no row has its sum from several workgroups and K is narrow.  Under 24,000
@@ -166,7 +169,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     }
     if (S->spmm_first) N = K;
   } else if (S->march)
-    want = given.march == 0 && (S->box ? S->box_us > 5 + S->M * (0.11e-3 + 6.3e-6 * S->opts.N)
+    want = given.march == 0 && (S->box ? S->box_us > S->box_other_us
                                        : S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
   else
     want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;

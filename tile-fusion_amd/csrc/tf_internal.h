@@ -114,9 +114,14 @@ struct WeightGradTask {
 // column and two of the intermediate with one.
 constexpr int kBoxBlock = 1024, kBoxMaxY = 6;
 constexpr int box_lds(int q, int by) { return 512 * ((2 * q + 4) * (by + 4) + (2 * q + 2) * (by + 2)) + 16 * 108 * (2 * q + 1); }
+// Runs over the 7-point stencil (tf_star.hip): columns of 16 by up to 8 points, 32 columns of C wide.  LDS holds two planes of C with two points around
+// the column and two of the intermediate in the same places, lines of 20 points of 128 bytes, and a line that what nobody wants is read from.
+constexpr int kStarX = 16, kStarMaxY = 8, kStarLine = (kStarX + 4) * 128, kStarBlock = 768;
+constexpr int star_lds(int by) { return kStarLine * (2 * ((by + 4) + (by + 2)) + 1); }
 struct BoxArgs {
+  int star = 0;  // the 7-point stencil instead of the 27-point one
   int nx = 0, ny = 0, nz = 0, N = 0;
-  int q = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x and y, planes a run, strips of 64 columns
+  int q = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x and y, planes a run, strips of 64 columns (star: 32)
   int per_xcd = 0;                                               // set by the launcher
   unsigned val_bytes = 0;                                        // of Ax and of Bx
   const float *Ax = nullptr, *Bx = nullptr, *C = nullptr;
@@ -246,7 +251,7 @@ struct tf_schedule {
   // Runs over a grid whose 27-point stencil both patterns are: marching runs of a kernel of their own, without any of the lists above.
   bool box = false;
   tf::BoxArgs box_runs;
-  double box_us = 0;  // what they are expected to take
+  double box_us = 0, box_other_us = 0;  // what they are expected to take, and two products
   // Two-layer tiles (GeMM-SpMM schedules of a square matrix with K and N of 32, 64 or 128, when every tile's two
   // halos fit LDS): what tf_gcn_two_layers runs when this is the second layer's schedule.  l2_lds_bytes: the LDS
   // of the fullest tile (slab A in front, slab B -- X staging, then the hidden rows -- behind it).

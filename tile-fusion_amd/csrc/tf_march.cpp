@@ -513,33 +513,69 @@ bool box_grid(int M, const int *Ap, const int *Ai, int grid[3]) {
   return true;
 }
 
+// The same for its neighbours along the axes.
+bool star_grid(int M, const int *Ap, const int *Ai, int grid[3]) {
+  if (M < 8 || Ap[1] - Ap[0] != 4) return false;  // row 0: 0, 1, nx, and the first of the next plane
+  const int nx = Ai[2], plane = Ai[3];
+  if (nx < 2 || plane < 2 * nx || plane % nx != 0 || M % plane != 0 || M / plane < 2) return false;
+  const int ny = plane / nx, nz = M / plane;
+  if ((long long)Ap[M] != 7LL * M - 2LL * plane - 2LL * nx * nz - 2LL * ny * nz) return false;
+  const int *col = Ai;
+  int row = 0;
+  for (int z = 0; z < nz; ++z)
+    for (int y = 0; y < ny; ++y)
+      for (int x = 0; x < nx; ++x, ++row) {
+        if (Ai + Ap[row] != col) return false;
+        if ((z > 0 && *col++ != row - plane) || (y > 0 && *col++ != row - nx) || (x > 0 && *col++ != row - 1) || *col++ != row ||
+            (x < nx - 1 && *col++ != row + 1) || (y < ny - 1 && *col++ != row + nx) || (z < nz - 1 && *col++ != row + plane))
+          return false;
+      }
+  grid[0] = nx; grid[1] = ny; grid[2] = nz;
+  return true;
+}
+
+bool stencil_grid(int star, int M, const int *Ap, const int *Ai, int grid[3]) { return star ? star_grid(M, Ap, Ai, grid) : box_grid(M, Ap, Ai, grid); }
+
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
+constexpr int strip_cols(const BoxArgs &b) { return b.star ? 32 : 64; }
+constexpr int column_x(const BoxArgs &b) { return b.star ? kStarX : 2 * b.q; }
+constexpr int runs_lds(const BoxArgs &b) { return b.star ? star_lds(b.by) : box_lds(b.q, b.by); }
 
 }  // namespace
 
 bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi, const tf_inspect_opts &o, const tf_inspect_opts &given) {
   if (S->L != M || o.inner_cols != M || Ap[M] >= (1 << 29) || Bp[M] != Ap[M]) return false;
-  if (given.march_tile_x > 0 || given.march_tile_y > 0) return false;  // (the general runs take any column)
   if (given.march > 0 && o.N % 64 != 0) return false;                  // (who insists on marching runs has been told that they take whole strips)
   int grid[3], inner[3];
-  if (!box_grid(M, Ap, Ai, grid)) return false;
-  if (!(Bp == Ap && Bi == Ai) && (!box_grid(M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner))) return false;
+  const bool star = o.N % 4 == 0 && star_grid(M, Ap, Ai, grid);
+  if (!star && !box_grid(M, Ap, Ai, grid)) return false;
+  // (the general runs take any column; who insists on marching runs over a 7-point stencil gets these where the column asked for is theirs)
+  const bool tile_given = given.march_tile_x > 0 || given.march_tile_y > 0, star_tile = given.march_tile_x == kStarX && given.march_tile_y <= kStarMaxY;
+  if (star ? !(tile_given ? star_tile : given.march == 0) : tile_given) return false;
+  const int most_y = star ? given.march_tile_y > 0 ? given.march_tile_y : kStarMaxY : kBoxMaxY;
+  if (!(Bp == Ap && Bi == Ai) && (!stencil_grid(star, M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner))) return false;
   if ((given.grid_nx > 0 || given.grid_ny > 0 || given.grid_nz > 0) && (given.grid_nx != grid[0] || given.grid_ny != grid[1] || given.grid_nz != grid[2])) return false;
   const int nx = grid[0], ny = grid[1], nz = grid[2];
-  if ((long long)nx * ny * o.N * 4 >= UINT_MAX) return false;  // the kernel's offsets in a plane of C
+  if ((long long)nx * ny * o.N * 4 >= (star ? 0x80000000LL : (long long)UINT_MAX)) return false;  // the kernel's offsets in a plane of C
   // Shape and planes of a run: the least time of the device's turns.  A step takes a compute unit the same time whatever its lines (0.05 us times
   // 7 q + 12: 2.0 and 2.7 us measured for q = 4 and 6), and a run takes six steps more than the planes it owns.
+  // (star: columns of 16 by 8, four steps more than planes, each the longer the less of C and D the caches hold: N = 64, 40^3 points 1.0 us, 64^3 1.4, 128^3 1.9)
+  const double star_step = 1.1 + 0.8 * std::min(1.0, 8.0 * M * o.N / 4e8);
   BoxArgs best;
-  const int strips = ceil_div(o.N, 64);
+  best.star = star;
+  const int strips = ceil_div(o.N, strip_cols(best));
   S->box_us = 1e30;
   for (const int q : {4, 6}) {
-    const int tx = ceil_div(nx, 2 * q), ty = ceil_div(ny, kBoxMaxY);
+    if (star && q == 6) break;
+    const int tx = ceil_div(nx, star ? kStarX : 2 * q), ty = ceil_div(ny, most_y);
     for (int cuts = 1; cuts <= nz; ++cuts) {
       const int zlen = ceil_div(nz, cuts);
       if (cuts > 1 && zlen == ceil_div(nz, cuts - 1)) continue;
       const long long runs = (long long)tx * ty * ceil_div(nz, zlen) * strips;
       if (runs > (1 << 24)) break;
-      const double us = 8 + 0.05 * (7 * q + 12) * (double)((runs + o.compute_units - 1) / o.compute_units) * (zlen + 6);
+      if (star && zlen > kMarchMaxIter) continue;  // (longer runs have little to gain, and fewer to even out a turn)
+      const double turns = (double)((runs + o.compute_units - 1) / o.compute_units);
+      const double us = star ? 8 + star_step * turns * (zlen + 4) : 8 + 0.05 * (7 * q + 12) * turns * (zlen + 6);
       if (us < S->box_us) {
         S->box_us = us;
         best.q = q; best.by = ceil_div(ny, ty); best.tx = tx; best.ty = ty; best.zlen = zlen; best.n_runs = (int)runs;
@@ -547,14 +583,16 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
     }
   }
   if (best.q == 0) return false;
+  S->box_other_us = star ? 4 + M * 3.4e-6 * (o.N > 32 ? strips * 32 : o.N) : 5 + M * (0.11e-3 + 6.3e-6 * o.N);
+  if (star && o.N % 64 != 0 && S->box_us > S->box_other_us) return false;  // (no runs at all: two products)
   best.nx = nx; best.ny = ny; best.nz = nz; best.N = o.N; best.strips = strips;
   S->march = S->box = true;
   S->box_runs = best;
   std::copy(grid, grid + 3, S->march_grid);
-  S->march_tile[0] = 2 * best.q; S->march_tile[1] = best.by;
-  S->lds_bytes = box_lds(best.q, best.by);
+  S->march_tile[0] = column_x(best); S->march_tile[1] = best.by;
+  S->lds_bytes = runs_lds(best);
   S->march_slots = S->slab_rows = S->lds_bytes / kMarchRowBytes;
-  S->march_width = 27;
+  S->march_width = star ? 7 : 27;
   S->fused_nnz = S->inner_nnz = Ap[M];
   S->inner_hash = Bp == Ap && Bi == Ai ? S->pattern_hash : tf_pattern_hash(M, Bp, Bi);
   S->march_declined = TF_MARCH_BUILT;
@@ -564,8 +602,8 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->ptr2.assign(1, 0);
   for (int z0 = 0; z0 < nz; z0 += best.zlen)
     for (int y0 = 0; y0 < ny; y0 += best.by)
-      for (int x0 = 0; x0 < nx; x0 += 2 * best.q) {
-        const int x1 = std::min(nx, x0 + 2 * best.q), y1 = std::min(ny, y0 + best.by), z1 = std::min(nz, z0 + best.zlen);
+      for (int x0 = 0; x0 < nx; x0 += column_x(best)) {
+        const int x1 = std::min(nx, x0 + column_x(best)), y1 = std::min(ny, y0 + best.by), z1 = std::min(nz, z0 + best.zlen);
         TileDesc t{};
         t.cons_begin = (int)S->fused_ids.size();
         for (int z = z0; z < z1; ++z)
@@ -595,12 +633,12 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
 tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi) {
   const BoxArgs &b = s->box_runs;
   int grid[3], inner[3];
-  if (!box_grid(M, Ap, Ai, grid) || !box_grid(M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner) || grid[0] != b.nx || grid[1] != b.ny || grid[2] != b.nz)
-    return fail(TF_ESCHEDULE, "runs over a %d x %d x %d grid: the patterns are not its 27-point stencil", b.nx, b.ny, b.nz);
-  if (b.N != s->opts.N || b.strips != ceil_div(b.N, 64) || b.by < 1 || b.by > kBoxMaxY || s->lds_bytes != box_lds(b.q, b.by) || s->lds_bytes > kMaxLds)
+  if (!stencil_grid(b.star, M, Ap, Ai, grid) || !stencil_grid(b.star, M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner) || grid[0] != b.nx || grid[1] != b.ny || grid[2] != b.nz)
+    return fail(TF_ESCHEDULE, "runs over a %d x %d x %d grid: the patterns are not its %d-point stencil", b.nx, b.ny, b.nz, b.star ? 7 : 27);
+  if (b.N != s->opts.N || (b.star && b.N % 4 != 0) || b.strips != ceil_div(b.N, strip_cols(b)) || b.by < 1 || b.by > (b.star ? kStarMaxY : kBoxMaxY) || s->lds_bytes != runs_lds(b) || s->lds_bytes > kMaxLds)
     return fail(TF_ESCHEDULE, "runs over a grid: %d columns, %d lines, %d bytes of LDS", b.N, b.by, s->lds_bytes);
   const int cuts = b.zlen > 0 ? ceil_div(b.nz, b.zlen) : 0;
-  if (cuts < 1 || b.q < 1 || b.tx != ceil_div(b.nx, 2 * b.q) || b.ty != ceil_div(b.ny, b.by) || (long long)b.tx * b.ty * cuts * b.strips != b.n_runs ||
+  if (cuts < 1 || b.q < 1 || b.tx != ceil_div(b.nx, column_x(b)) || b.ty != ceil_div(b.ny, b.by) || (long long)b.tx * b.ty * cuts * b.strips != b.n_runs ||
       s->tiles.size() != (size_t)b.tx * b.ty * cuts)
     return fail(TF_ESCHEDULE, "runs over a grid: %d runs of %d planes do not cover it", b.n_runs, b.zlen);
   std::vector<char> done(M, 0);
@@ -608,7 +646,7 @@ tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai
     const TileDesc &t = s->tiles[r];
     for (int q = t.cons_begin; q < t.cons_end; ++q) {
       const int i = s->fused_ids[q], x = i % b.nx, y = i / b.nx % b.ny, z = i / b.nx / b.ny;
-      if (i < 0 || i >= M || done[i]++ || (size_t)((z / b.zlen * b.ty + y / b.by) * b.tx + x / (2 * b.q)) != r)
+      if (i < 0 || i >= M || done[i]++ || (size_t)((z / b.zlen * b.ty + y / b.by) * b.tx + x / column_x(b)) != r)
         return fail(TF_ESCHEDULE, "runs over a grid: row %d is not run %zu's, or twice there", i, r);
     }
   }
