@@ -311,6 +311,12 @@ def test_weight_gradient_on_bf16_cores(gpu, tf, M, N, K):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and ok.all() == (not odd)
 
 
+# workgroups of eight wavefronts from 2,048 blocks of 32 rows on (256 compute units), of four below
+@pytest.mark.parametrize("M,N,K", [(65504, 17, 130), (65505, 17, 130), (65537, 64, 48), (70001, 130, 257), (131071, 2, 3)])
+def test_weight_gradient_of_many_rows(gpu, tf, M, N, K):
+    test_weight_gradient_on_bf16_cores(gpu, tf, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(5000, 64, 100), (40000, 40, 128)])
 @pytest.mark.parametrize("q", [1, 2, 4, 8, 64])
 def test_weight_gradient_of_rare_features(gpu, tf, M, N, K, q):
@@ -388,6 +394,12 @@ def test_two_weight_gradients_in_one_call(gpu, tf, M1, M2):
     for bad in range(8):  # every operand is checked before either product runs
         if bad % 4 != 3:
             assert lib.tf_weight_grad_pair(*[None if i == bad else a for i, a in enumerate(args)], None) != 0
+
+
+@pytest.mark.parametrize("M1,M2", [(65505, 65505), (65504, 65505), (66000, 4096)])
+def test_two_weight_gradients_of_many_rows_in_one_call(gpu, tf, M1, M2):
+    test_two_weight_gradients_in_one_call(gpu, tf, M1, M2)
+
 
 
 @pytest.mark.parametrize("N", [1, 3, 4, 7, 16, 40, 64, 100, 128, 257])

@@ -640,7 +640,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 // wavefront holds a 16 NB x 16 KB tile of Y and takes 32 rows of both operands at a time, in whole lines: lane (j, h) loads the columns
 // NB j .. of G and KB j .. of X in the rows 8 h .. 8 h + 7, which are what its part of a 16 x 16 x 32 product wants of each of
 // the NB (KB) column blocks.  The next rows are requested as soon as these have become parts.  The wavefronts of a launch take blocks of
-// rows in turn; a workgroup's four are added through LDS, and weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.
+// rows in turn; a workgroup's four or eight are added through LDS, and weight_grad_reduce_kernel adds the workgroups' tiles -- all in a fixed order.
 // A lane whose columns would reach past the last one works on the last NB (KB) instead: some values of Y are computed twice.
 // Bound: the rows of X and G from HBM, 16 KB a wavefront in flight, behind some 10 us for two launches and the sums at the end (us, operands in no
 // cache, both launches, fp32 cores on 64 x 160 tiles / this: 14,000 rows 32 x 69 18.0 / 10.3, 35,000 rows 64 x 128 25.7 / 22.8, 100,000 rows 64 x 128 36.3 / 32.0,
@@ -650,7 +650,7 @@ hipError_t launch_gemm_any(const float *X, int ldx, const float *W, int wt, floa
 constexpr int kWgRows = 32;       // rows of a block
 constexpr int kWgFewRows = 4096;  // up to here in one launch, weight_grad_few_kernel
 
-template <int NB, int KB>
+template <int NB, int KB, int WAVES>
 __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int group, int chunk, acc4 (*red)[64]) {
   constexpr int T = NB * KB;
   const float *__restrict__ G = t.G, *__restrict__ X = t.X;
@@ -659,7 +659,7 @@ __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int gr
   const int nc = chunk / t.k_chunks, kc = chunk % t.k_chunks;
   const float *gp = G + min(nc * 16 * NB + NB * j, N - NB);
   const float *xp = X + min(kc * 16 * KB + KB * j, K - KB);
-  const int n_blocks = (M + kWgRows - 1) / kWgRows, stride = 4 * t.groups, b0 = 4 * group + wave;
+  const int n_blocks = (M + kWgRows - 1) / kWgRows, stride = WAVES * t.groups, b0 = WAVES * group + wave;
   acc4 acc[NB][KB];
 #pragma unroll
   for (int a = 0; a < NB; ++a)
@@ -748,7 +748,7 @@ __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int gr
       }
   }
 #pragma unroll
-  for (int half = 2; half >= 1; half /= 2) {
+  for (int half = WAVES / 2; half >= 1; half /= 2) {
     if (wave >= half && wave < 2 * half) {
 #pragma unroll
       for (int a = 0; a < NB; ++a)
@@ -777,12 +777,13 @@ __device__ __forceinline__ void weight_grad_tile(const WeightGradTask &t, int gr
 
 // Two gradients a launch: the workgroups from first_blocks on work on the second, whose rows come in while the first one's sums are added up.  (A
 // training step of two layers on 13,800 nodes, 69 -> 32 -> 6: 17.7 us in four launches, 11.4 in two.)
-__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
-  __shared__ acc4 red[2 * 16][64];
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void weight_grad_kernel(const WeightGradTask first, const WeightGradTask second, int first_blocks) {
+  __shared__ acc4 red[WAVES / 2 * 16][64];
   const bool other = (int)blockIdx.x >= first_blocks;
   const WeightGradTask &t = other ? second : first;
   const int at = other ? blockIdx.x - first_blocks : blockIdx.x, group = at % t.groups, chunk = at / t.groups;
-#define TILE(NB_, KB_) case NB_ * 8 + KB_: weight_grad_tile<NB_, KB_>(t, group, chunk, red); break
+#define TILE(NB_, KB_) case NB_ * 8 + KB_: weight_grad_tile<NB_, KB_, WAVES>(t, group, chunk, red); break
   switch (t.nb * 8 + t.kb) {
     TILE(1, 1); TILE(1, 2); TILE(1, 3); TILE(1, 4); TILE(2, 1); TILE(2, 2); TILE(2, 3); TILE(2, 4);
     TILE(3, 1); TILE(3, 2); TILE(3, 3); TILE(3, 4); TILE(4, 1); TILE(4, 2); TILE(4, 3); TILE(4, 4);
@@ -896,17 +897,20 @@ WeightGradTask plan_weight_grad(int M, int N, int K, int compute_units) {
   };
   cut(N, p.n_chunks, p.nb);
   cut(K, p.k_chunks, p.kb);
-  // two workgroups per compute unit; a wavefront has a block of rows or more
+  // eight wavefronts per compute unit, of a block of rows or more each
   // (a multiple of 8: the chunks of a block of rows on one XCD, whose L2 has the other operand and the lines two chunks share)
   const int chunks = p.n_chunks * p.k_chunks, blocks = (M + kWgRows - 1) / kWgRows;
-  p.groups = std::max(1, std::min(std::max(1, 2 * compute_units / chunks), (blocks + 3) / 4));
+  // Eight wavefronts a workgroup halve the sums that go through memory, where every wavefront of the device has a block of rows all the same (two groups
+  // of four / one of eight, both launches: 100,000 rows 64 x 128 30.1 / 27.8 us, a layer 145 / 141; 131,072 rows 64 x 300 and 40 x 64 73 / 70, the step 291 / 287).
+  p.waves = blocks >= 8 * compute_units ? 8 : 4;
+  p.groups = std::max(1, std::min(std::max(1, 8 / p.waves * compute_units / chunks), (blocks + p.waves - 1) / p.waves));
   if (p.groups > 8) p.groups = p.groups / 8 * 8;
   return p;
 }
 
 // One gradient, or (second not null) two that share their launches where both are of few rows, or both are not.
 hipError_t launch_weight_grads(const WeightGradTask &first, const WeightGradTask *second, hipStream_t st) {
-  if (second && second->few != first.few) {
+  if (second && (second->few != first.few || second->waves != first.waves)) {
     const hipError_t err = launch_weight_grads(first, nullptr, st);
     return err != hipSuccess ? err : launch_weight_grads(*second, nullptr, st);
   }
@@ -917,7 +921,8 @@ hipError_t launch_weight_grads(const WeightGradTask &first, const WeightGradTask
     hipLaunchKernelGGL(weight_grad_few_kernel, dim3(blocks), dim3(1024), 0, st, first, b, first_blocks);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(weight_grad_kernel, dim3(blocks), dim3(256), 0, st, first, b, first_blocks);
+  if (first.waves == 8) hipLaunchKernelGGL(weight_grad_kernel<8>, dim3(blocks), dim3(512), 0, st, first, b, first_blocks);
+  else hipLaunchKernelGGL(weight_grad_kernel<4>, dim3(blocks), dim3(256), 0, st, first, b, first_blocks);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   auto registers = [](const WeightGradTask &t) { return t.nb * t.kb * 4 * t.n_chunks * t.k_chunks; };

@@ -105,7 +105,7 @@ struct WeightGradTask {
   float *Y = nullptr, *partial = nullptr;
   int M = 0, N = 0, K = 0;
   int few = 0;  // in one launch, without a workspace; of the cuts below only k_chunks is set
-  int nb = 0, kb = 0, n_chunks = 0, k_chunks = 0, groups = 0;
+  int nb = 0, kb = 0, n_chunks = 0, k_chunks = 0, groups = 0, waves = 0;  // waves: of a workgroup
   int blocks() const { return few ? n_chunks * k_chunks : groups * n_chunks * k_chunks; }  // workgroups
   size_t partial_floats() const { return few ? 0 : (size_t)blocks() * nb * kb * 256; }
 };
