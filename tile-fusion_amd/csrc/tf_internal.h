@@ -118,10 +118,13 @@ constexpr int box_lds(int q, int by) { return 512 * ((2 * q + 4) * (by + 4) + (2
 // the column and two of the intermediate in the same places, lines of 20 points of 128 bytes, and a line that what nobody wants is read from.
 constexpr int kStarX = 16, kStarMaxY = 8, kStarLine = (kStarX + 4) * 128, kStarBlock = 768;
 constexpr int star_lds(int by) { return kStarLine * (2 * ((by + 4) + (by + 2)) + 1); }
+// ... and over the 5-point stencil of a 2D grid, which is its one with a line for a plane: columns of up to 94 points of a line.
+constexpr int kFlatX = 94, kFlatBlock = (kFlatX + 2) / 2 * 8, kFlatLine = (kFlatX + 6) * 128, kFlatRuns = 2;  // runs a compute unit holds
+constexpr int flat_lds() { return kFlatLine * 4; }
 struct BoxArgs {
-  int star = 0;  // the 7-point stencil instead of the 27-point one
+  int star = 0;  // the 7-point (ny = 1: 5-point) stencil instead of the 27-point one
   int nx = 0, ny = 0, nz = 0, N = 0;
-  int q = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x and y, planes a run, strips of 64 columns (star: 32)
+  int q = 0, bx = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x (bx points) and y, planes a run, strips of 64 columns (star: 32)
   int per_xcd = 0;                                               // set by the launcher
   unsigned val_bytes = 0;                                        // of Ax and of Bx
   const float *Ax = nullptr, *Bx = nullptr, *C = nullptr;

@@ -534,12 +534,30 @@ bool star_grid(int M, const int *Ap, const int *Ai, int grid[3]) {
   return true;
 }
 
-bool stencil_grid(int star, int M, const int *Ap, const int *Ai, int grid[3]) { return star ? star_grid(M, Ap, Ai, grid) : box_grid(M, Ap, Ai, grid); }
+// The same of a 2D grid of lines of nx points: planes of one line.
+bool flat_grid(int M, const int *Ap, const int *Ai, int grid[3]) {
+  if (M < 4 || Ap[1] - Ap[0] != 3) return false;  // row 0: 0, 1, nx
+  const int nx = Ai[2];
+  if (nx < 2 || M % nx != 0 || M / nx < 2) return false;
+  const int nz = M / nx;
+  if ((long long)Ap[M] != 5LL * M - 2LL * nx - 2LL * nz) return false;
+  const int *col = Ai;
+  int row = 0;
+  for (int z = 0; z < nz; ++z)
+    for (int x = 0; x < nx; ++x, ++row) {
+      if (Ai + Ap[row] != col) return false;
+      if ((z > 0 && *col++ != row - nx) || (x > 0 && *col++ != row - 1) || *col++ != row || (x < nx - 1 && *col++ != row + 1) || (z < nz - 1 && *col++ != row + nx)) return false;
+    }
+  grid[0] = nx; grid[1] = 1; grid[2] = nz;
+  return true;
+}
+
+bool stencil_grid(int star, int M, const int *Ap, const int *Ai, int grid[3]) { return star ? star_grid(M, Ap, Ai, grid) || flat_grid(M, Ap, Ai, grid) : box_grid(M, Ap, Ai, grid); }
 
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 constexpr int strip_cols(const BoxArgs &b) { return b.star ? 32 : 64; }
-constexpr int column_x(const BoxArgs &b) { return b.star ? kStarX : 2 * b.q; }
-constexpr int runs_lds(const BoxArgs &b) { return b.star ? star_lds(b.by) : box_lds(b.q, b.by); }
+constexpr int column_x(const BoxArgs &b) { return b.bx; }
+constexpr int runs_lds(const BoxArgs &b) { return !b.star ? box_lds(b.q, b.by) : b.ny == 1 ? flat_lds() : star_lds(b.by); }
 
 }  // namespace
 
@@ -547,10 +565,10 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   if (S->L != M || o.inner_cols != M || Ap[M] >= (1 << 29) || Bp[M] != Ap[M]) return false;
   if (given.march > 0 && o.N % 64 != 0) return false;                  // (who insists on marching runs has been told that they take whole strips)
   int grid[3], inner[3];
-  const bool star = o.N % 4 == 0 && star_grid(M, Ap, Ai, grid);
+  const bool star = o.N % 4 == 0 && stencil_grid(true, M, Ap, Ai, grid), flat = star && grid[1] == 1;
   if (!star && !box_grid(M, Ap, Ai, grid)) return false;
   // (the general runs take any column; who insists on marching runs over a 7-point stencil gets these where the column asked for is theirs)
-  const bool tile_given = given.march_tile_x > 0 || given.march_tile_y > 0, star_tile = given.march_tile_x == kStarX && given.march_tile_y <= kStarMaxY;
+  const bool tile_given = given.march_tile_x > 0 || given.march_tile_y > 0, star_tile = given.march_tile_x == (flat ? kFlatX : kStarX) && given.march_tile_y <= (flat ? 1 : kStarMaxY);
   if (star ? !(tile_given ? star_tile : given.march == 0) : tile_given) return false;
   const int most_y = star ? given.march_tile_y > 0 ? given.march_tile_y : kStarMaxY : kBoxMaxY;
   if (!(Bp == Ap && Bi == Ai) && (!stencil_grid(star, M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner))) return false;
@@ -567,18 +585,20 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->box_us = 1e30;
   for (const int q : {4, 6}) {
     if (star && q == 6) break;
-    const int tx = ceil_div(nx, star ? kStarX : 2 * q), ty = ceil_div(ny, most_y);
+    const int bx = flat ? (ceil_div(nx, ceil_div(nx, kFlatX)) + 1) / 2 * 2 : star ? kStarX : 2 * q;  // (flat: even ones, pairs of points)
+    const int tx = ceil_div(nx, bx), ty = ceil_div(ny, most_y);
     for (int cuts = 1; cuts <= nz; ++cuts) {
       const int zlen = ceil_div(nz, cuts);
       if (cuts > 1 && zlen == ceil_div(nz, cuts - 1)) continue;
       const long long runs = (long long)tx * ty * ceil_div(nz, zlen) * strips;
       if (runs > (1 << 24)) break;
       if (star && zlen > kMarchMaxIter) continue;  // (longer runs have little to gain, and fewer to even out a turn)
-      const double turns = (double)((runs + o.compute_units - 1) / o.compute_units);
+      const int at_once = o.compute_units * (flat ? kFlatRuns : 1);
+      const double turns = (double)((runs + at_once - 1) / at_once);
       const double us = star ? 8 + star_step * turns * (zlen + 4) : 8 + 0.05 * (7 * q + 12) * turns * (zlen + 6);
       if (us < S->box_us) {
         S->box_us = us;
-        best.q = q; best.by = ceil_div(ny, ty); best.tx = tx; best.ty = ty; best.zlen = zlen; best.n_runs = (int)runs;
+        best.q = q; best.bx = bx; best.by = ceil_div(ny, ty); best.tx = tx; best.ty = ty; best.zlen = zlen; best.n_runs = (int)runs;
       }
     }
   }
@@ -592,7 +612,7 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->march_tile[0] = column_x(best); S->march_tile[1] = best.by;
   S->lds_bytes = runs_lds(best);
   S->march_slots = S->slab_rows = S->lds_bytes / kMarchRowBytes;
-  S->march_width = star ? 7 : 27;
+  S->march_width = flat ? 5 : star ? 7 : 27;
   S->fused_nnz = S->inner_nnz = Ap[M];
   S->inner_hash = Bp == Ap && Bi == Ai ? S->pattern_hash : tf_pattern_hash(M, Bp, Bi);
   S->march_declined = TF_MARCH_BUILT;
@@ -634,7 +654,7 @@ tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai
   const BoxArgs &b = s->box_runs;
   int grid[3], inner[3];
   if (!stencil_grid(b.star, M, Ap, Ai, grid) || !stencil_grid(b.star, M, Bp, Bi, inner) || !std::equal(grid, grid + 3, inner) || grid[0] != b.nx || grid[1] != b.ny || grid[2] != b.nz)
-    return fail(TF_ESCHEDULE, "runs over a %d x %d x %d grid: the patterns are not its %d-point stencil", b.nx, b.ny, b.nz, b.star ? 7 : 27);
+    return fail(TF_ESCHEDULE, "runs over a %d x %d x %d grid: the patterns are not its %d-point stencil", b.nx, b.ny, b.nz, !b.star ? 27 : b.ny == 1 ? 5 : 7);
   if (b.N != s->opts.N || (b.star && b.N % 4 != 0) || b.strips != ceil_div(b.N, strip_cols(b)) || b.by < 1 || b.by > (b.star ? kStarMaxY : kBoxMaxY) || s->lds_bytes != runs_lds(b) || s->lds_bytes > kMaxLds)
     return fail(TF_ESCHEDULE, "runs over a grid: %d columns, %d lines, %d bytes of LDS", b.N, b.by, s->lds_bytes);
   const int cuts = b.zlen > 0 ? ceil_div(b.nz, b.zlen) : 0;

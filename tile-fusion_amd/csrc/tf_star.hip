@@ -1,5 +1,5 @@
-// Fused SpMM-SpMM on the 7-point stencil of a 3D grid (gfx950): D = A (B C), A and B the pattern in which every grid point reads itself
-// and its neighbours along the axes, x fastest (checked against the matrices by the inspector: build_box in tf_march.cpp).  Any values.
+// Fused SpMM-SpMM on the 7-point stencil of a 3D grid and the 5-point one of a 2D grid (gfx950): D = A (B C), A and B the pattern in which every grid
+// point reads itself and its neighbours along the axes, x fastest (checked against the matrices by the inspector: build_box in tf_march.cpp).  Any values.
 // The reference's answer to such patterns is tiling with redundancy (fusion/src/SpMM_SpMM.cpp:984-1057).
 #include <hip/hip_runtime.h>
 #include <cstdlib>
@@ -30,14 +30,15 @@ template <int L> __device__ __forceinline__ void fma_quad(float val, const f4 &x
 
 // A row's values: lane l of a quad holds the ones of the neighbours l and 4 + l of (-z, -y, -x, itself, +x, +y, +z), zero for a neighbour that is not there.
 struct StarRow { float lo, hi; };
+template <bool FLAT>
 __device__ __forceinline__ f4 star_sum(const StarRow &v, const f4 &mz, const f4 &my, const f4 &mx, const f4 &own, const f4 &px, const f4 &py, const f4 &pz) {
   float acc[4] = {0.f, 0.f, 0.f, 0.f};  // in the order of the row's entries
   fma_quad<0>(v.lo, mz, acc);
-  fma_quad<1>(v.lo, my, acc);
+  if constexpr (!FLAT) fma_quad<1>(v.lo, my, acc);
   fma_quad<2>(v.lo, mx, acc);
   fma_quad<3>(v.lo, own, acc);
   fma_quad<0>(v.hi, px, acc);
-  fma_quad<1>(v.hi, py, acc);
+  if constexpr (!FLAT) fma_quad<1>(v.hi, py, acc);
   fma_quad<2>(v.hi, pz, acc);
   return f4{acc[0], acc[1], acc[2], acc[3]};
 }
@@ -90,38 +91,42 @@ struct StarPlace {
 // 16 by 8 points of 32 columns: the intermediate 1.4 times and C's planes 1.8 times the column, where 8 by 8 of 64 columns are 1.5 and 2.1, in
 // as much of LDS.  Plain stores of D take 262 instead of 254.  Each sum is made in the order of the row's entries, so results carry
 // the reference's bits; what is outside the grid is zero, with zeros for values.
+// FLAT: a 2D grid, its lines for planes; a column is up to 94 points of a line, and two workgroups share a compute unit.  (1000 x 1000 points, us, here / as
+// two products: N = 64 120 / 310, 100 302 / 537, 128 236 / 576; 900 x 900, N = 32 46 / 90.)
 // LDS rows of 128 bytes: two lane groups of a read, two points apart, would meet in the same banks; rows 2 and 3 of every four change places.
-template <bool ACC, bool SAME>
-__global__ __launch_bounds__(kStarBlock) void fused_star_kernel(const BoxArgs a) {
+template <bool ACC, bool SAME, bool FLAT>
+__global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_kernel(const BoxArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int run = xcd_contiguous(blockIdx.x, a.per_xcd);
   if (run >= a.n_runs) return;
-  constexpr int LINE = kStarX + 4, PAIRS = (kStarX + 2) / 2;
+  constexpr int LINE = FLAT ? kFlatX + 6 : kStarX + 4, PAIRS = FLAT ? (kFlatX + 2) / 2 : (kStarX + 2) / 2, UP = FLAT ? 0 : LINE * 128;  // UP: bytes from a line to the next
   const int c0 = run % a.strips * 32, r1 = run / a.strips, r2 = r1 / a.tx;
-  const int x0 = r1 % a.tx * kStarX, y0 = r2 % a.ty * a.by, z0 = r2 / a.ty * a.zlen, z1 = min(a.nz, z0 + a.zlen);
+  const int bx = FLAT ? a.bx : kStarX, x0 = r1 % a.tx * bx, y0 = r2 % a.ty * a.by, z0 = r2 / a.ty * a.zlen, z1 = min(a.nz, z0 + a.zlen);
   if (z0 >= z1) return;
   const int nx = a.nx, ny = a.ny, nz = a.nz, N = a.N, by = a.by, plane = nx * ny, per_plane = 7 * plane - 2 * nx - 2 * ny;
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
-  const unsigned c_bytes = kStarLine * (by + 4), t_bytes = kStarLine * (by + 2), t_at = 2 * c_bytes - kStarLine;  // (of the intermediate lines 1 .. by + 2 only)
+  const unsigned c_bytes = FLAT ? kFlatLine : kStarLine * (by + 4), t_bytes = FLAT ? kFlatLine : kStarLine * (by + 2);
+  const unsigned t_at = 2 * c_bytes - UP;  // (of the intermediate lines 1 .. by + 2 only)
   const int group = threadIdx.x / 8, gl = threadIdx.x % 8, l = gl % 4, col = c0 + gl * 4;
-  const int line = group / PAIRS, pair = group % PAIRS, x = x0 - 1 + 2 * pair, y = y0 - 1 + line;
-  const bool t_on = line < by + 2, col_ok = col < N;
+  const int line = FLAT ? 0 : group / PAIRS, pair = FLAT ? group : group % PAIRS, x = x0 - 1 + 2 * pair, y = FLAT ? 0 : y0 - 1 + line;
+  const bool t_on = FLAT ? 2 * pair < bx + 2 : line < by + 2, col_ok = col < N;
   auto row_at = [&](int i) __attribute__((always_inline)) { return lds0 + (unsigned)((i ^ (i >> 1 & 1)) * 128 + gl * 16); };
-  const int i0 = (t_on ? line + 1 : 1) * LINE + 1 + 2 * pair;
+  const int i0 = (FLAT ? 0 : t_on ? line + 1 : 1) * LINE + 1 + 2 * pair;
   const unsigned at_mx = row_at(i0 - 1), at_0 = row_at(i0), at_1 = row_at(i0 + 1), at_px = row_at(i0 + 2);
 
   // the group's point around those of the intermediate: the lines before and behind, then the ends of the others
-  const int around = 2 * (LINE - 2) + 2 * (by + 2), e = group - 2 * (LINE - 2);
-  const int ri = e < -(LINE - 2) ? group + 1 : e < 0 ? (by + 3) * LINE + 1 + group - (LINE - 2) : (1 + e / 2) * LINE + (e & 1) * (LINE - 1);
+  const int around = FLAT ? 2 : 2 * (LINE - 2) + 2 * (by + 2), e = group - 2 * (LINE - 2);
+  const int ri = FLAT ? (group == 0 ? 0 : bx + 3) : e < -(LINE - 2) ? group + 1 : e < 0 ? (by + 3) * LINE + 1 + group - (LINE - 2) : (1 + e / 2) * LINE + (e & 1) * (LINE - 1);
   const bool r_on = group < around;
   const unsigned at_r = row_at(ri);
 
   auto source = [&](int px, int py, bool on) __attribute__((always_inline)) -> unsigned {
     return on && col_ok && px >= 0 && px < nx && py >= 0 && py < ny ? 4u * (((unsigned)py * nx + px) * N + col) : kNowhere;
   };
-  const unsigned from0 = source(x, y, t_on), from1 = source(x + 1, y, t_on), from_r = source(x0 - 2 + ri % LINE, y0 - 2 + ri / LINE, r_on);
+  const unsigned from0 = source(x, y, t_on), from1 = source(x + 1, y, t_on), from_r = source(x0 - 2 + ri % LINE, FLAT ? 0 : y0 - 2 + ri / LINE, r_on);
   const bool in_0 = t_on && x >= 0 && x < nx && y >= 0 && y < ny, in_1 = t_on && x + 1 >= 0 && x + 1 < nx && y >= 0 && y < ny;
-  const bool d_line = line >= 1 && line <= by && y < ny && col_ok, d_0 = d_line && pair > 0 && x < nx, d_1 = d_line && pair < PAIRS - 1 && x + 1 < nx;
+  const bool d_line = (FLAT || (line >= 1 && line <= by)) && y < ny && col_ok;
+  const bool d_0 = d_line && pair > 0 && x < min(nx, x0 + bx), d_1 = d_line && x + 1 < min(nx, x0 + bx);
   const int plane_bytes = (int)((unsigned)plane * N * 4u);
   auto c_plane = [&](int z) __attribute__((always_inline)) {  // (a buffer of nothing outside the grid and the run)
     const bool there = z >= 0 && z < nz && z <= z1 + 1;
@@ -173,8 +178,8 @@ __global__ __launch_bounds__(kStarBlock) void fused_star_kernel(const BoxArgs a)
     }
     f4 t[2] = {0.f, 0.f};
     if (z <= t_last) {
-      const f4 s0 = star_sum(vb[B][0], c[M][0], lds_read4(at_0 + c_now - kStarLine), lds_read4(at_mx + c_now), c[O][0], c[O][1], lds_read4(at_0 + c_now + kStarLine), c[U][0]);
-      const f4 s1 = star_sum(vb[B][1], c[M][1], lds_read4(at_1 + c_now - kStarLine), c[O][0], c[O][1], lds_read4(at_px + c_now), lds_read4(at_1 + c_now + kStarLine), c[U][1]);
+      const f4 s0 = star_sum<FLAT>(vb[B][0], c[M][0], lds_read4(at_0 + c_now - UP), lds_read4(at_mx + c_now), c[O][0], c[O][1], lds_read4(at_0 + c_now + UP), c[U][0]);
+      const f4 s1 = star_sum<FLAT>(vb[B][1], c[M][1], lds_read4(at_1 + c_now - UP), c[O][0], c[O][1], lds_read4(at_px + c_now), lds_read4(at_1 + c_now + UP), c[U][1]);
       t[0] = in_0 ? s0 : f4(0.f);
       t[1] = in_1 ? s1 : f4(0.f);
     }
@@ -192,8 +197,8 @@ __global__ __launch_bounds__(kStarBlock) void fused_star_kernel(const BoxArgs a)
     if (r_on) lds_write4(at_r + c_next, r[B]);
     r[B] = load(c_plane(z + 3), from_r);
     if (z - 1 >= z0 && t_on) {
-      const f4 d0 = star_sum(va[B][0], t2[0], lds_read4(at_0 + t_back - kStarLine), lds_read4(at_mx + t_back), t1[0], t1[1], lds_read4(at_0 + t_back + kStarLine), t[0]);
-      const f4 d1 = star_sum(va[B][1], t2[1], lds_read4(at_1 + t_back - kStarLine), t1[0], t1[1], lds_read4(at_px + t_back), lds_read4(at_1 + t_back + kStarLine), t[1]);
+      const f4 d0 = star_sum<FLAT>(va[B][0], t2[0], lds_read4(at_0 + t_back - UP), lds_read4(at_mx + t_back), t1[0], t1[1], lds_read4(at_0 + t_back + UP), t[0]);
+      const f4 d1 = star_sum<FLAT>(va[B][1], t2[1], lds_read4(at_1 + t_back - UP), t1[0], t1[1], lds_read4(at_px + t_back), lds_read4(at_1 + t_back + UP), t[1]);
       f4 *out = reinterpret_cast<f4 *>(a.D + (((size_t)(z - 1) * ny + y) * nx + x) * N + col);
       f4 *out1 = reinterpret_cast<f4 *>(a.D + (((size_t)(z - 1) * ny + y) * nx + x + 1) * N + col);
       if (d_0) __builtin_nontemporal_store(ACC ? *out + d0 : d0, out);
@@ -220,18 +225,21 @@ __global__ __launch_bounds__(kStarBlock) void fused_star_kernel(const BoxArgs a)
 
 hipError_t launch_fused_star(BoxArgs a, int accumulate, hipStream_t st) {
   static const bool remap = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
-  const int lds = star_lds(a.by);
-  if (a.by < 1 || a.by > kStarMaxY || a.N % 4 != 0 || a.n_runs <= 0) return hipErrorInvalidValue;
+  const bool flat = a.ny == 1;
+  const int lds = flat ? flat_lds() : star_lds(a.by), block = flat ? kFlatBlock : kStarBlock;
+  if (a.by < 1 || a.by > kStarMaxY || a.bx < 1 || a.bx > (flat ? kFlatX : kStarX) || a.N % 4 != 0 || a.n_runs <= 0) return hipErrorInvalidValue;
   a.per_xcd = remap ? (a.n_runs + kXcds - 1) / kXcds : 0;
   const dim3 grid((a.n_runs + kXcds - 1) / kXcds * kXcds);
-#define CALL(ACC_, SAME_)                                                                                                                            \
-  do {                                                                                                                                               \
-    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fused_star_kernel<ACC_, SAME_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
-    if (err != hipSuccess) return err;                                                                                                               \
-    hipLaunchKernelGGL((fused_star_kernel<ACC_, SAME_>), grid, dim3(kStarBlock), lds, st, a);                                                         \
+#define CALL(ACC_, SAME_, FLAT_)                                                                                                                             \
+  do {                                                                                                                                                      \
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fused_star_kernel<ACC_, SAME_, FLAT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+    if (err != hipSuccess) return err;                                                                                                                      \
+    hipLaunchKernelGGL((fused_star_kernel<ACC_, SAME_, FLAT_>), grid, dim3(block), lds, st, a);                                                              \
   } while (0)
-  if (a.Ax == a.Bx) { if (accumulate) CALL(true, true); else CALL(false, true); }
-  else { if (accumulate) CALL(true, false); else CALL(false, false); }
+#define CALL2(ACC_, SAME_) do { if (flat) CALL(ACC_, SAME_, true); else CALL(ACC_, SAME_, false); } while (0)
+  if (a.Ax == a.Bx) { if (accumulate) CALL2(true, true); else CALL2(false, true); }
+  else { if (accumulate) CALL2(true, false); else CALL2(false, false); }
+#undef CALL2
 #undef CALL
   return hipGetLastError();
 }
