@@ -391,7 +391,8 @@ def run_config(tf, cfg, idx, steps, warmup, args):
         "working_set_vs_llc": round(operand_bytes / LLC_BYTES, 2),
         "rel_err_vs_f64": err, "rows_checked": rows_checked,
         "kernels": kernels, "kernel": ("fused_gcn2_kernel" if args.two_layers == "fuse" else "2 x " + kernel_names(info, gemm, False) + " + relu_kernel")
-        if (gemm and args.two_layers) else kernel_names(info, gemm, args.unfused),
+        if (gemm and args.two_layers) else
+        kernels[0]["name"] if info["marched"] and not args.unfused and len(kernels) == 1 else kernel_names(info, gemm, args.unfused),
         "schedule": {"lds_bytes": info["lds_bytes"], "windowed": bool(info["windowed"]), "wide_strips": bool(info["wide_strips"]),
                      "streamed": bool(info["streamed"]), "marched": bool(info["marched"]), "tiles": info["n_tiles"], "fused_rows": info["n_fused_rows"],
                      "remainder_rows": info["n_remainder_rows"], "long_rows": info["n_long_rows"],
