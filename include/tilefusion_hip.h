@@ -252,7 +252,10 @@ typedef struct {
      7-point-like stencil (row-to-column distances 1, nx, nx*ny).  The grid only deals rows to runs:
      what a run loads, recomputes and keeps is derived from the patterns and checked by
      tf_schedule_validate_inner, so a wrong grid cannot give wrong results.  march_tile_x/y: 0 = the
-     largest column whose rows fit LDS (8 x 8 on a 7-point stencil). */
+     largest column whose rows fit LDS (8 x 8 on a 7-point stencil).
+     Where both patterns are a grid's whole 27-, 7- or (2D) 5-point stencil the runs have kernels of their own, for any N (7 and
+     5 points: multiples of 4), unless march = 1 is given with other widths than multiples of 64; over 7 and 5 points with
+     march = 1 only where march_tile_x/y name a column of theirs (16 x 8 or less, 94 x 1). */
   int march;
   int grid_nx, grid_ny, grid_nz;
   int march_tile_x, march_tile_y;

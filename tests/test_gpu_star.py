@@ -8,11 +8,12 @@ from test_gpu_parity import oracle_spmm_spmm, say
 
 
 # (x, y, z): a column and one or two points more, two planes, three, two points wide, lines that do not divide; columns of C: a strip, its edges, four
-# columns behind it; y = 1: lines of one column, one point more, two and three of them, two lines.  (Small grids of widths that are no strips of 64 go to two products: the larger ones are those that do not.)
+# columns behind it; y = 1: lines of one column, one point more, two and three of them, two lines,
+# and a D of more than 320 MB whose rows are no whole lines.  (Small grids of widths that are no strips of 64 go to two products: the larger ones are those that do not.)
 @pytest.mark.gpu
 @pytest.mark.parametrize("dims,N", [((16, 8, 9), 64), ((17, 9, 12), 64), ((18, 10, 2), 64), ((33, 17, 3), 128), ((2, 150, 6), 64), ((150, 2, 6), 64),
                                     ((290, 2, 5), 192), ((31, 23, 40), 64), ((90, 80, 70), 60), ((63, 61, 67), 100), ((110, 100, 60), 32), ((96, 40, 70), 96),
-                                    ((94, 1, 20), 64), ((95, 1, 41), 64), ((93, 1, 50), 128), ((189, 1, 33), 192), ((2500, 1, 2), 64), ((700, 1, 300), 36), ((501, 1, 400), 100)])
+                                    ((94, 1, 20), 64), ((95, 1, 41), 64), ((93, 1, 50), 128), ((189, 1, 33), 192), ((2500, 1, 2), 64), ((700, 1, 300), 36), ((501, 1, 400), 100), ((1003, 1, 850), 100)])
 def test_star_bit_exact(gpu, tf, orc, dims, N):
     say(f"star {dims} N={N}")
     A = stencil_3d(*dims, seed=61)

@@ -114,7 +114,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    40^3 31 / 39, 64^3 87 / 136, 96^3 174 / 560; 64^3, N = 16 84 / 59, 32 85 / 86, 37 94 / 124, 96 150 / 240.  Their expected time, a sum over
 //    runs and planes (build_box), against 5 + M (0.11 + 0.0063 N) / 1000, which is within a tenth of two products on up to 64^3 points.
 //    So have runs over its whole 7-point stencil (us, its runs / two products / the other runs): N = 64, 24^3 points 11.3 / 8.6, 32^3 11.3 / 11.5, 40^3 15.9 /
-//    18.6, 64^3 34 / 59 / 49, 96^3 114 / 294 / 181, 128^3 230 / 619 / 290; N = 128, 32^3 14.5 / 18.9, 64^3 60 / 136 / 97; 128^3, N = 32 130 / 352, 100 728 / 1,120; 90 x 70
+//    18.6, 64^3 34 / 59 / 49, 96^3 114 / 294 / 181, 128^3 230 / 619 / 290; N = 128, 32^3 14.5 / 18.9, 64^3 60 / 136 / 97; 128^3, N = 32 130 / 352, 100 642 / 1,120; 90 x 70
 //    x 80, N = 36 70 / 103; against 4 + M (N, in whole lines) 0.0034 / 1000.  Any N of a multiple of four.  And over the 5-point stencil of a 2D grid whose
 //    lines no window holds: N = 64, 400 x 100 13.8 / 12.8, 300^2 19.3 / 23.3 / 28.4, 500^2 34 / 53 / 44, 1024 x 200 29 / 44 / 44, 700^2 54 / 141 / 90, 1000^2
 //    120 / 310 / 162; 250^2, N = 48 15.6 / 16.4, 600 x 500, N = 36 37 / 58.

@@ -125,7 +125,7 @@ struct BoxArgs {
   int star = 0;  // the 7-point (ny = 1: 5-point) stencil instead of the 27-point one
   int nx = 0, ny = 0, nz = 0, N = 0;
   int q = 0, bx = 0, by = 0, tx = 0, ty = 0, zlen = 0, strips = 0, n_runs = 0;  // columns in x (bx points) and y, planes a run, strips of 64 columns (star: 32)
-  int per_xcd = 0;                                               // set by the launcher
+  int per_xcd = 0, streaming = 1;                                // set by the launcher
   unsigned val_bytes = 0;                                        // of Ax and of Bx
   const float *Ax = nullptr, *Bx = nullptr, *C = nullptr;
   float *D = nullptr;

@@ -89,10 +89,10 @@ struct StarPlace {
 // intermediate to the one that makes D (128^3 points, N = 64: 230 us, 254 with a load for each).  Bound: HBM, at the rate of a copy for C, D and the values
 // (235 us at 5.1 TB/s; gathering runs over lists 290, two products 619); on 64^3 points, N = 64, 34 us (49, 59), the steps themselves, 1.4 us each.
 // 16 by 8 points of 32 columns: the intermediate 1.4 times and C's planes 1.8 times the column, where 8 by 8 of 64 columns are 1.5 and 2.1, in
-// as much of LDS.  Plain stores of D take 262 instead of 254.  Each sum is made in the order of the row's entries, so results carry
+// as much of LDS.  Each sum is made in the order of the row's entries, so results carry
 // the reference's bits; what is outside the grid is zero, with zeros for values.
 // FLAT: a 2D grid, its lines for planes; a column is up to 94 points of a line, and two workgroups share a compute unit.  (1000 x 1000 points, us, here / as
-// two products: N = 64 120 / 310, 100 302 / 537, 128 236 / 576; 900 x 900, N = 32 46 / 90.)
+// two products: N = 64 120 / 310, 100 259 / 537, 128 236 / 576; 900 x 900, N = 32 46 / 90.)
 // LDS rows of 128 bytes: two lane groups of a read, two points apart, would meet in the same banks; rows 2 and 3 of every four change places.
 template <bool ACC, bool SAME, bool FLAT>
 __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_kernel(const BoxArgs a) {
@@ -136,6 +136,10 @@ __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     const u4 v = __builtin_amdgcn_raw_buffer_load_b128(from, (int)at, 0, 0);
     return f4{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
+  };
+  auto store = [&](f4 *to, const f4 &v) __attribute__((always_inline)) {  // (written out: the compiler makes one store of the two branches and drops the hint)
+    if (a.streaming) asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(to), "v"(v) : "memory");
+    else *to = v;
   };
   const __amdgpu_buffer_rsrc_t av = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.Ax), 0, (int)a.val_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t bv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.Bx), 0, (int)a.val_bytes, 0x00020000);
@@ -201,8 +205,8 @@ __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_
       const f4 d1 = star_sum<FLAT>(va[B][1], t2[1], lds_read4(at_1 + t_back - UP), t1[0], t1[1], lds_read4(at_px + t_back), lds_read4(at_1 + t_back + UP), t[1]);
       f4 *out = reinterpret_cast<f4 *>(a.D + (((size_t)(z - 1) * ny + y) * nx + x) * N + col);
       f4 *out1 = reinterpret_cast<f4 *>(a.D + (((size_t)(z - 1) * ny + y) * nx + x + 1) * N + col);
-      if (d_0) __builtin_nontemporal_store(ACC ? *out + d0 : d0, out);
-      if (d_1) __builtin_nontemporal_store(ACC ? *out1 + d1 : d1, out1);
+      if (d_0) store(out, ACC ? *out + d0 : d0);
+      if (d_1) store(out1, ACC ? *out1 + d1 : d1);
     }
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -229,6 +233,9 @@ hipError_t launch_fused_star(BoxArgs a, int accumulate, hipStream_t st) {
   const int lds = flat ? flat_lds() : star_lds(a.by), block = flat ? kFlatBlock : kStarBlock;
   if (a.by < 1 || a.by > kStarMaxY || a.bx < 1 || a.bx > (flat ? kFlatX : kStarX) || a.N % 4 != 0 || a.n_runs <= 0) return hipErrorInvalidValue;
   a.per_xcd = remap ? (a.n_runs + kXcds - 1) / kXcds : 0;
+  // Streaming stores but where strips share lines of a D that the Infinity Cache does not hold, which would go to memory in parts (us, streaming / plain:
+  // N = 100, 128^3 points 719 / 642, 1000 x 1000 302 / 259, 64^3 63.1 / 61.8; N = 84, 96^3 201 / 206; N = 48, 64^3 34.4 / 35.7; whole lines, 128^3, N = 64 254 / 262).
+  a.streaming = a.N % 32 == 0 || (long long)a.nx * a.ny * a.nz * a.N * 4 <= (320ll << 20);
   const dim3 grid((a.n_runs + kXcds - 1) / kXcds * kXcds);
 #define CALL(ACC_, SAME_, FLAT_)                                                                                                                             \
   do {                                                                                                                                                      \
