@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
-from test_gpu_march import box_stencil, march
+from test_gpu_march import box_stencil, march, stencil_3d
 from test_gpu_parity import oracle_spmm_spmm, say
 
 
@@ -25,9 +25,10 @@ def test_box_bit_exact(gpu, tf, orc, dims, N):
         S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, march=1 if N % 64 == 0 else 0, **kw)
         S.validate()
         info = S.info()
-        assert info["marched"] == 1 and info["march_tile_x"] in (8, 12) and info["march_tile_y"] <= 6, info
         if N % 64 and kw:
-            continue  # (few compute units: more turns of the runs than two products take)
+            assert info["marched"] == 0  # (few compute units: more turns of the runs than two products take)
+            continue
+        assert info["marched"] == 1 and info["march_tile_x"] in (8, 12) and info["march_tile_y"] <= 6, info
         for acc in (False, True):
             D = tf.DenseMatrix(A.shape[0], N, D0) if acc else tf.DenseMatrix(A.shape[0], N)
             if not acc:
@@ -95,3 +96,20 @@ def test_box_only_where_the_pattern_is_the_stencil(tf):
     with pytest.raises(tf.TileFusionError):   # (whole strips, as ever, for who insists on marching runs)
         tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=48, inner=Ah, march=1)
     assert tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=64, inner=Ah, march=-1).info()["marched"] == 0
+
+
+@pytest.mark.parametrize("dims,N,points", [((16, 16, 16), 37, 27), ((12, 13, 14), 20, 27), ((16, 16, 16), 36, 7), ((300, 1, 30), 36, 5), ((2, 9, 11), 50, 27)])
+def test_two_products_are_nothing_else(tf, dims, N, points):
+    """A grid's stencil in a width that whole strips do not divide, on so few points that two products are faster: no runs are reported, and A's
+    pattern alone validates the schedule."""
+    A = box_stencil(*dims, True, seed=71) if points == 27 else stencil_3d(*dims, seed=71)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, strip_cols=64, compute_units=256)
+    info = S.info()
+    assert info["marched"] == 0 and info["march_tile_x"] == 0, info
+    if not info["windowed"]:
+        assert info["march_declined"] == 2
+    S.validate()
+    S._inner = None
+    if not info["windowed"]:
+        S.validate()

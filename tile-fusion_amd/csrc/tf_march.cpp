@@ -559,6 +559,13 @@ constexpr int strip_cols(const BoxArgs &b) { return b.star ? 32 : 64; }
 constexpr int column_x(const BoxArgs &b) { return b.bx; }
 constexpr int runs_lds(const BoxArgs &b) { return !b.star ? box_lds(b.q, b.by) : b.ny == 1 ? flat_lds() : star_lds(b.by); }
 
+// Whether build_march makes runs of its lists over a grid's whole stencil too: whole strips, offsets and lists of 32 bits (some 2.7 ELL rows of 256 bytes a
+// point of 27), a grid that is given or that detect_grid finds.
+bool general_runs_take(const BoxArgs &b, int M, const tf_inspect_opts &given) {
+  return b.N % 64 == 0 && M < (1 << 24) && (long long)M * b.N * 4 < (1LL << 32) && (b.star || M < 6000000) &&
+         (given.grid_nx > 0 || (!b.star ? b.nx >= 3 : b.ny > 1 || b.nx >= 16));
+}
+
 }  // namespace
 
 bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi, const tf_inspect_opts &o, const tf_inspect_opts &given) {
@@ -604,8 +611,9 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   }
   if (best.q == 0) return false;
   S->box_other_us = star ? 4 + M * 3.4e-6 * (o.N > 32 ? strips * 32 : o.N) : 5 + M * (0.11e-3 + 6.3e-6 * o.N);
-  if (star && o.N % 64 != 0 && S->box_us > S->box_other_us) return false;  // (no runs at all: two products)
   best.nx = nx; best.ny = ny; best.nz = nz; best.N = o.N; best.strips = strips;
+  // Where two products are faster and only these runs could march, the schedule is one of two products and nothing else, which any inner matrix will do for.
+  if (given.march == 0 && !general_runs_take(best, M, given) && S->box_us > S->box_other_us) return false;
   S->march = S->box = true;
   S->box_runs = best;
   std::copy(grid, grid + 3, S->march_grid);
