@@ -113,3 +113,28 @@ def test_two_products_are_nothing_else(tf, dims, N, points):
     S._inner = None
     if not info["windowed"]:
         S.validate()
+
+
+def beside_two_products(tf, points, N):
+    """A grid's whole stencil and the schedule of its runs in a width that only they take."""
+    A = box_stencil(40, 41, 39, True, seed=72) if points == 27 else stencil_3d(40, 41, 39, seed=72) if points == 7 else stencil_3d(300, 1, 310, seed=72)
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, compute_units=256)
+    assert S.info()["marched"] == 1
+    return A, Ah, S
+
+
+def one_entry_moved(tf, A):
+    i = A.shape[0] // 2
+    B = sp.csr_matrix((A.data, A.indices.copy(), A.indptr), shape=A.shape)
+    B.indices[B.indptr[i]] -= 1
+    return B, tf.CsrMatrix(B.shape[0], B.shape[1], B.indptr, B.indices, B.data)
+
+
+@pytest.mark.parametrize("points,N", [(27, 61), (27, 100), (7, 100), (5, 60)])
+def test_the_outer_pattern_alone_validates(tf, points, N):
+    """Runs that stand in for two products are validated against A's pattern, as two products are; another pattern is not A's."""
+    A, Ah, S = beside_two_products(tf, points, N)
+    assert tf.lib().tf_schedule_validate(S.h, Ah.M, Ah.N, Ah._pp, Ah._pi) == 0
+    _, Bh = one_entry_moved(tf, A)
+    assert tf.lib().tf_schedule_validate(S.h, Bh.M, Bh.N, Bh._pp, Bh._pi) == -4

@@ -1190,6 +1190,7 @@ extern "C" tf_status tf_schedule_validate(const tf_schedule *s, int L, int M, co
   if (L != s->L || M != s->M || Ap[L] != s->nnz)
     return tf::fail(TF_ESCHEDULE, "schedule was built for %d x %d with %lld entries, got %d x %d with %d",
                     s->L, s->M, s->nnz, L, M, Ap[L]);
+  if (s->box_beside) return tf::validate_box(s, M, Ap, Ai, Ap, Ai);
   if (s->march)
     return tf::fail(TF_EINVAL, "tf_schedule_validate: marching runs are checked against both patterns: use tf_schedule_validate_inner");
   if (tf_status rc = validate_two_passes(s, L, M, Ap, Ai)) return rc;

@@ -251,8 +251,9 @@ struct tf_schedule {
   std::vector<int> march_ell_off;    // [march_ell_stride(march_width) per ELL row] LDS byte offset of the row read (the zero row for padding)
   std::vector<int> march_ell_src;    // ... and where its value comes from: index into B's values, or into A's
                                      // with kMarchSrcA set; -1 for padding (value 0)
-  // Runs over a grid whose 27-point stencil both patterns are: marching runs of a kernel of their own, without any of the lists above.
+  // Runs over a grid whose 27-, 7- or 5-point stencil both patterns are: marching runs of a kernel of their own, without any of the lists above.
   bool box = false;
+  bool box_beside = false;  // ... that stand in for two products: the schedule is as good for A's pattern alone
   tf::BoxArgs box_runs;
   double box_us = 0, box_other_us = 0;  // what they are expected to take, and two products
   // Two-layer tiles (GeMM-SpMM schedules of a square matrix with K and N of 32, 64 or 128, when every tile's two

@@ -612,9 +612,12 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   if (best.q == 0) return false;
   S->box_other_us = star ? 4 + M * 3.4e-6 * (o.N > 32 ? strips * 32 : o.N) : 5 + M * (0.11e-3 + 6.3e-6 * o.N);
   best.nx = nx; best.ny = ny; best.nz = nz; best.N = o.N; best.strips = strips;
-  // Where two products are faster and only these runs could march, the schedule is one of two products and nothing else, which any inner matrix will do for.
-  if (given.march == 0 && !general_runs_take(best, M, given) && S->box_us > S->box_other_us) return false;
+  // Where only these runs could march nobody has asked for runs: a schedule of two products, which these are taken in place of.  Where two products are faster
+  // it is nothing else.
+  const bool beside = given.march == 0 && !general_runs_take(best, M, given);
+  if (beside && S->box_us > S->box_other_us) return false;
   S->march = S->box = true;
+  S->box_beside = beside;
   S->box_runs = best;
   std::copy(grid, grid + 3, S->march_grid);
   S->march_tile[0] = column_x(best); S->march_tile[1] = best.by;
