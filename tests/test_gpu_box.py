@@ -138,3 +138,51 @@ def test_the_outer_pattern_alone_validates(tf, points, N):
     assert tf.lib().tf_schedule_validate(S.h, Ah.M, Ah.N, Ah._pp, Ah._pi) == 0
     _, Bh = one_entry_moved(tf, A)
     assert tf.lib().tf_schedule_validate(S.h, Bh.M, Bh.N, Bh._pp, Bh._pi) == -4
+
+
+def other_inners(tf, A):
+    """Inner matrices of A's shape and entry count, with an entry more, and with other columns."""
+    M = A.shape[0]
+    moved = one_entry_moved(tf, A)[0]
+    more = sp.csr_matrix(A + sp.csr_matrix((np.ones(1, np.float32), ([3], [M - 1])), shape=A.shape))
+    wide = sp.random(M, 500, density=6 / 500, format="csr", random_state=73, dtype=np.float32)
+    for B in (moved, more, wide):
+        B.indices = B.indices.astype(np.int32)
+        B.indptr = B.indptr.astype(np.int32)
+    return moved, more, wide
+
+
+@pytest.mark.parametrize("points,N", [(27, 61), (7, 100), (5, 60)])
+def test_other_inner_patterns_validate(tf, points, N):
+    A, Ah, S = beside_two_products(tf, points, N)
+    for B in other_inners(tf, A):
+        S._inner = tf.CsrMatrix(B.shape[0], B.shape[1], B.indptr, B.indices, B.data)
+        S.validate()
+    S._inner = None
+    S.validate()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("points,N", [(27, 61), (27, 100), (7, 100), (5, 60)])
+def test_other_inner_matrices(gpu, tf, orc, points, N):
+    """A schedule whose runs stand in for two products takes any inner matrix, and with the one it was made for it runs them, before and after."""
+    say(f"other inner matrices on {points} points N={N}")
+    A, Ah, S = beside_two_products(tf, points, N)
+    S.set_profiling(True)
+    runs = "fused_box_kernel" if points == 27 else "fused_star_kernel"
+    for B in (A, *other_inners(tf, A), A):
+        Bh = Ah if B is A else tf.CsrMatrix(B.shape[0], B.shape[1], B.indptr, B.indices, B.data)
+        Cd = tf.workloads.uniform((B.shape[1], N), 74)
+        D0 = tf.workloads.uniform((A.shape[0], N), 75)
+        want = oracle_spmm_spmm(orc, A, B, Cd)
+        for acc in (False, True):
+            D = tf.DenseMatrix(A.shape[0], N, D0)
+            tf.spmm_spmm(Ah, Bh, tf.DenseMatrix.from_numpy(Cd), D, S, accumulate=acc)
+            tf.device_synchronize()
+            names = [n for n, _ in S.profile()]
+            assert (names == [runs]) == (B is A) and len(names) == (1 if B is A else 2), names
+            if not acc:
+                assert np.array_equal(D.to_numpy(), want)
+            else:  # (the runs add a whole sum to D; the rows' sums start at D: 27 roundings more of the magnitudes there are)
+                size = abs(A.astype(np.float64)) @ abs(B.astype(np.float64) @ Cd) + abs(D0)
+                assert (abs(D.to_numpy() - (want + D0.astype(np.float64))) <= 2 * 28 * 2.0 ** -24 * size).all()

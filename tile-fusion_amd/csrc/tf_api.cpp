@@ -218,7 +218,7 @@ static bool untiled(const tf_schedule *s) { return s->opts.op == TF_OP_GEMM_SPMM
 // Floats from one row of the intermediate to the next: a multiple of 4, so that every lane's columns of a row are one
 // aligned load, and whole cache lines where the row kernel then works in column slices (slices_for in tf_rows.hip).
 static int inter_ld(const tf_schedule *s) {
-  if (!untiled(s) && !s->two_passes) return s->opts.N;
+  if (!untiled(s) && !s->two_passes && !s->box) return s->opts.N;
   const int N = s->user_N;
   return N > 96 && N < 128 && s->M >= 16000 && s->M <= 131072 ? 128 : (N + 3) / 4 * 4;
 }
@@ -246,7 +246,8 @@ static tf_status ensure_device(tf_schedule *s) {
   if (s->two_passes) {  // (the lists are the other schedule's)
     parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
     parts.list(s->l2_tiles, &d->l2_tiles);
-  } else if (s->box) {  // (no lists)
+  } else if (s->box) {  // no lists; the calls that the runs are not for are two products
+    if (s->box_beside) parts.reserve((size_t)s->M * inter_ld(s), &d->inter);
   } else if (s->march) {  // nothing but the run lists is needed on the device
     parts.list(s->march_runs, &d->m_runs);
     parts.list(s->march_row_ptr, &d->m_row_ptr);
@@ -808,6 +809,22 @@ static tf::RowsArgs all_rows(const tf_csr *A, const float *X, float *Y, int N) {
   return a;
 }
 
+// What runs over a stencil are not for, in the schedule's stead: both products row by row through an intermediate in HBM, the same sums in the same order.
+static tf_status box_as_two_products(const tf_csr *A, const tf_csr *B, const tf_dense *C, tf_dense *D, tf_schedule *s, int acc, hipStream_t st) {
+  tf::DeviceSchedule *d = s->dev;
+  const int N = s->opts.N, ldt = tf::inter_ld(s);
+  tf::RowsArgs first = all_rows(B, C->d, d->inter, N), second = all_rows(A, d->inter, D->d, N);
+  first.ldy = second.ldx = ldt;
+  first.streaming = tf::inter_streams(s);
+  second.streaming = 1;
+  second.accumulate = acc;
+  tf::RowsHow how;
+  how.xcd_chunk_rows = s->row_deal;
+  TF_PHASE(s, "spmm_rows_kernel (intermediate rows)", st, tf::launch_spmm_rows(first, tf::RowsHow(), st));
+  TF_PHASE(s, "spmm_rows_kernel (second-op rows)", st, tf::launch_spmm_rows(second, how, st));
+  return TF_OK;
+}
+
 extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_dense *C, tf_dense *D,
                                   tf_schedule *s, unsigned flags, void *stream) {
   tf_status rc = check_common("tf_spmm_spmm", A, C, D, s, TF_OP_SPMM_SPMM);
@@ -822,7 +839,8 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
   tf::DeviceSchedule *d = s->dev;
   d->prof_n = 0;
   const int n_launch = (int)s->launch_tiles.size();
-  if (s->march && (B->nnz != s->inner_nnz || B->N != s->opts.inner_cols || (B->hash && B->hash != s->inner_hash)))
+  const bool other_inner = s->march && (B->nnz != s->inner_nnz || B->N != s->opts.inner_cols || (B->hash && B->hash != s->inner_hash));
+  if (other_inner && !s->box_beside)
     return fail(TF_ESCHEDULE, "tf_spmm_spmm: the schedule's runs were built on another inner pattern than B's");
   if (s->two_passes) {
     tf_schedule *rows = s->two_passes;
@@ -845,6 +863,7 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     if (rc) return rc;
     return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, 0}, false, st);
   }
+  if (other_inner) return box_as_two_products(A, B, C, D, s, acc, st);
   if (s->box) {
     tf::BoxArgs a = s->box_runs;
     a.Ax = A->x; a.Bx = B->x; a.C = C->d; a.D = D->d;

@@ -97,6 +97,18 @@ extern "C" uint64_t tf_pattern_hash(int M, const int *Ap, const int *Ai) {
   return h ? h : 1;
 }
 
+// A product of all rows in order, of a matrix with locality: one contiguous run of rows per XCD, so that a row of X is
+// gathered into one L2, not into all eight -- where no XCD's run has much more work than the others'.  Two products, workgroups dealt
+// to the XCDs in turn / a run each: 7 points, 60^3, N = 32, 44 / 30 us, 30 x 40 x 50, N = 64, 30.5 / 18; 27 points, 24^3, N = 32, 13.1 / 10.8, 60^3
+// 85 / 75; 5 points, 900^2, N = 32, 120 / 95.  Past 100 MB of X the runs' planes outgrow the Infinity Cache together, and turns of
+// 512 rows are better: 7 points, 110^3, N = 32, 293 / 252 / 231 in turns.
+int tf::rows_in_order_deal(int L, int M, int N, const int *Ap) {
+  constexpr int kXcds = 8;
+  long long most_work = 0;
+  for (int x = 0; x < kXcds; ++x) most_work = std::max<long long>(most_work, Ap[(x + 1LL) * L / kXcds] - Ap[(long long)x * L / kXcds]);
+  return most_work * kXcds * 100 <= 115LL * Ap[L] ? (long long)M * N * 4 <= (100LL << 20) ? -1 : 512 : 0;
+}
+
 enum { kTiles, kRows, kRowsOfChecked };
 constexpr int kWholeRowMax = 128;  // rows of more entries are cut up, whatever the widths and row counts (unless the caller says otherwise)
 static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out);
@@ -878,19 +890,8 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       }
       S->rem_identity = (int)S->rem_rows.size() == L;
       for (int q = 0; q < L && S->rem_identity; ++q) S->rem_identity = (S->rem_rows[q] == q);
-      // A product of all rows in order, of a matrix with locality: one contiguous run of rows per XCD, so that a row of X is
-      // gathered into one L2, not into all eight -- where no XCD's run has much more work than the others'.  Two products, workgroups dealt
-      // to the XCDs in turn / a run each: 7 points, 60^3, N = 32, 44 / 30 us, 30 x 40 x 50, N = 64, 30.5 / 18; 27 points, 24^3, N = 32, 13.1 / 10.8, 60^3
-      // 85 / 75; 5 points, 900^2, N = 32, 120 / 95.  Past 100 MB of X the runs' planes outgrow the Infinity Cache together, and turns of
-      // 512 rows are better: 7 points, 110^3, N = 32, 293 / 252 / 231 in turns.
       S->rem_sweep = sweep && S->rem_identity;
-      S->row_deal = o.xcd_chunk_rows;
-      if (S->rem_identity && !far && o.xcd_chunk_rows == 0) {
-        constexpr int kXcds = 8;
-        long long most_work = 0;
-        for (int x = 0; x < kXcds; ++x) most_work = std::max<long long>(most_work, Ap[(x + 1LL) * L / kXcds] - Ap[(long long)x * L / kXcds]);
-        if (most_work * kXcds * 100 <= 115LL * nnz) S->row_deal = (long long)M * o.N * 4 <= (100LL << 20) ? -1 : 512;
-      }
+      S->row_deal = S->rem_identity && !far && o.xcd_chunk_rows == 0 ? tf::rows_in_order_deal(L, M, o.N, Ap) : o.xcd_chunk_rows;
       // Reordered adjacency (createReorderedAdj, GCN_Single_Layer_SP_Demo_Utils.h:618-653): a list that is
       // not simply all rows in order gets its rows stored side by side in list order, so that a
       // workgroup reads one stretch of columns and values instead of one stretch per row.
@@ -1140,7 +1141,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   }
   long long ws = 0;
   if (s->march) ws += (long long)s->march_ell_off.size() * 16;  // ELL rows with values, their offsets and sources
-  if (s->n_writeback_rows > 0 || s->two_passes) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
+  if (s->n_writeback_rows > 0 || s->two_passes || s->box_beside) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
   if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C
@@ -1401,7 +1402,7 @@ extern "C" tf_status tf_schedule_validate(const tf_schedule *s, int L, int M, co
 // holds every row its producer rows read, and that window, slab and tables fit the tile's LDS.
 extern "C" tf_status tf_schedule_validate_inner(const tf_schedule *s, int L, int M, const int *Ap, const int *Ai,
                                                 const int *inner_Ap, const int *inner_Ai, int inner_cols) {
-  if (s && s->march) {
+  if (s && s->march && !s->box_beside) {
     if (!Ap || !inner_Ap || L != s->L || M != s->M || L != M || Ap[L] != s->nnz)
       return tf::fail(TF_ESCHEDULE, "tf_schedule_validate_inner: the schedule's runs were built for other patterns");
     if (inner_cols != s->opts.inner_cols || inner_Ap[M] != s->inner_nnz || tf_pattern_hash(M, inner_Ap, inner_Ai) != s->inner_hash ||

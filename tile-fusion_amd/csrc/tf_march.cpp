@@ -618,6 +618,7 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   if (beside && S->box_us > S->box_other_us) return false;
   S->march = S->box = true;
   S->box_beside = beside;
+  S->row_deal = rows_in_order_deal(M, M, o.N, Ap);
   S->box_runs = best;
   std::copy(grid, grid + 3, S->march_grid);
   S->march_tile[0] = column_x(best); S->march_tile[1] = best.by;
