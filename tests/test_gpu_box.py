@@ -117,7 +117,7 @@ def test_two_products_are_nothing_else(tf, dims, N, points):
 
 def beside_two_products(tf, points, N):
     """A grid's whole stencil and the schedule of its runs in a width that only they take."""
-    A = box_stencil(40, 41, 39, True, seed=72) if points == 27 else stencil_3d(40, 41, 39, seed=72) if points == 7 else stencil_3d(300, 1, 310, seed=72)
+    A = box_stencil(40, 41, 39, True, seed=72) if points == 27 else stencil_3d(48, 47, 50, seed=72) if points == 7 else stencil_3d(300, 1, 310, seed=72)
     Ah = tf.CsrMatrix.from_scipy(A)
     S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, compute_units=256)
     assert S.info()["marched"] == 1
@@ -186,3 +186,33 @@ def test_other_inner_matrices(gpu, tf, orc, points, N):
             else:  # (the runs add a whole sum to D; the rows' sums start at D: 27 roundings more of the magnitudes there are)
                 size = abs(A.astype(np.float64)) @ abs(B.astype(np.float64) @ Cd) + abs(D0)
                 assert (abs(D.to_numpy() - (want + D0.astype(np.float64))) <= 2 * 28 * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("points,N", [(27, 61), (27, 64), (7, 100), (7, 64), (5, 60), (5, 64)])
+def test_wrapped_inner_matrices_of_unknown_pattern(gpu, tf, orc, points, N):
+    """A wrapped inner matrix without a hash may have any pattern with A's count of entries: the runs, which go by their own pattern, are not for it.
+    With the hash of the inner pattern, or on A's own row pointers and columns, they are."""
+    say(f"wrapped inner matrices on {points} points N={N}")
+    A, Ah, S = beside_two_products(tf, points, N)
+    S.set_profiling(True)
+    other = one_entry_moved(tf, A)[0]
+    Cd = tf.workloads.uniform((A.shape[0], N), 76)
+    Ch = tf.DenseMatrix.from_numpy(Cd)
+    D = tf.DenseMatrix(A.shape[0], N)
+
+    def wrap(B, hash=0, like=None):
+        own = [tf.DenseMatrix.from_numpy(np.ascontiguousarray(x).view(np.float32).reshape(1, -1)) for x in (B.indptr, B.indices, B.data)]
+        own[:2] = like or own[:2]
+        return tf.CsrMatrix.wrap_device(tf.CsrMatrix.from_scipy(B), *(x.device_ptr() for x in own), hash), own
+
+    Aw, A_dev = wrap(A)
+    values = A.copy()
+    values.data = np.random.default_rng(77).uniform(-1, 1, A.nnz).astype(np.float32)
+    for outer, (inner, _keep), B, by_runs in ((Ah, wrap(other), other, False), (Ah, wrap(values), values, False), (Ah, wrap(values, tf.pattern_hash(A)), values, True),
+                                              (Aw, (Aw, None), A, True), (Aw, wrap(values, like=A_dev[:2]), values, True)):
+        D.fill(float("nan"))
+        tf.spmm_spmm(outer, inner, Ch, D, S)
+        tf.device_synchronize()
+        assert np.array_equal(D.to_numpy(), oracle_spmm_spmm(orc, A, B, Cd))
+        assert (len(S.profile()) == 1) == by_runs, S.profile()

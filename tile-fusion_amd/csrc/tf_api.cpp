@@ -247,7 +247,7 @@ static tf_status ensure_device(tf_schedule *s) {
     parts.reserve(s->spmm_first ? (size_t)s->L * s->user_K : (size_t)s->M * inter_ld(s), &d->inter);
     parts.list(s->l2_tiles, &d->l2_tiles);
   } else if (s->box) {  // no lists; the calls that the runs are not for are two products
-    if (s->box_beside) parts.reserve((size_t)s->M * inter_ld(s), &d->inter);
+    if (s->box_room) parts.reserve((size_t)s->M * inter_ld(s), &d->inter);
   } else if (s->march) {  // nothing but the run lists is needed on the device
     parts.list(s->march_runs, &d->m_runs);
     parts.list(s->march_row_ptr, &d->m_row_ptr);
@@ -863,8 +863,10 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
     if (rc) return rc;
     return tf::run_remainder(A, rows, tf::Remainder{d->inter, ldt, N, s->M, D->d, acc, 0}, false, st);
   }
-  if (other_inner) return box_as_two_products(A, B, C, D, s, acc, st);
   if (s->box) {
+    // (a wrapped matrix without a hash may have any pattern; who has runs that always were runs has given B the inner one)
+    const bool unknown_inner = s->box_room && !B->hash && !(B->p == A->p && B->i == A->i);
+    if (other_inner || unknown_inner) return box_as_two_products(A, B, C, D, s, acc, st);
     tf::BoxArgs a = s->box_runs;
     a.Ax = A->x; a.Bx = B->x; a.C = C->d; a.D = D->d;
     a.val_bytes = (unsigned)A->nnz * 4;

@@ -109,6 +109,11 @@ int tf::rows_in_order_deal(int L, int M, int N, const int *Ap) {
   return most_work * kXcds * 100 <= 115LL * Ap[L] ? (long long)M * N * 4 <= (100LL << 20) ? -1 : 512 : 0;
 }
 
+// (above choose_two_passes: runs of lists with few rows to march over)
+bool tf::march_as_two_products(const tf_schedule *S) {
+  return S->march_width <= kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20);
+}
+
 enum { kTiles, kRows, kRowsOfChecked };
 constexpr int kWholeRowMax = 128;  // rows of more entries are cut up, whatever the widths and row counts (unless the caller says otherwise)
 static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out);
@@ -183,8 +188,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
     }
     if (S->spmm_first) N = K;
   } else if (S->march)
-    want = given.march == 0 && (S->box ? S->box_us > S->box_other_us
-                                       : S->march_width <= tf::kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20));
+    want = given.march == 0 && (S->box ? S->box_us > S->box_other_us : tf::march_as_two_products(S));
   else
     want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;
   if (!want) return TF_OK;
@@ -1141,7 +1145,7 @@ extern "C" tf_status tf_schedule_get_info(const tf_schedule *s, tf_schedule_info
   }
   long long ws = 0;
   if (s->march) ws += (long long)s->march_ell_off.size() * 16;  // ELL rows with values, their offsets and sources
-  if (s->n_writeback_rows > 0 || s->two_passes || s->box_beside) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
+  if (s->n_writeback_rows > 0 || s->two_passes || s->box_room) ws += std::max((long long)s->M * s->opts.N, (long long)s->L * (s->spmm_first ? s->user_K : 0)) * 4;
   ws += (long long)s->long_chunks.size() * s->opts.N * 4;
   if (s->long_part) ws += ((long long)s->seg_ptr.size() - 1) * s->opts.N * 4 + (long long)s->seg_src.size() * 4;  // partial sums, regrouped values
   if (s->user_K != s->opts.K) ws += ((long long)s->M + s->opts.N) * s->opts.K * 4;  // padded copies of B and C

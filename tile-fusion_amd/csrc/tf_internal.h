@@ -254,6 +254,7 @@ struct tf_schedule {
   // Runs over a grid whose 27-, 7- or 5-point stencil both patterns are: marching runs of a kernel of their own, without any of the lists above.
   bool box = false;
   bool box_beside = false;  // ... that stand in for two products: the schedule is as good for A's pattern alone, with any inner matrix
+  bool box_room = false;    // ... or stand where the runs of lists would be two products: with room for an intermediate, for calls they are not for
   tf::BoxArgs box_runs;
   double box_us = 0, box_other_us = 0;  // what they are expected to take, and two products
   // Two-layer tiles (GeMM-SpMM schedules of a square matrix with K and N of 32, 64 or 128, when every tile's two
@@ -301,6 +302,7 @@ tf_status validate_march(const tf_schedule *s, int M, const int *Ap, const int *
 bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi,
                const tf_inspect_opts &o, const tf_inspect_opts &given);
 tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi);
+bool march_as_two_products(const tf_schedule *S);
 int rows_in_order_deal(int L, int M, int N, const int *Ap);
 void release_device_schedule(DeviceSchedule *d);
 int default_compute_units();

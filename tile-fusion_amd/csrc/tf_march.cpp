@@ -625,6 +625,7 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->lds_bytes = runs_lds(best);
   S->march_slots = S->slab_rows = S->lds_bytes / kMarchRowBytes;
   S->march_width = flat ? 5 : star ? 7 : 27;
+  S->box_room = beside || (given.march == 0 && march_as_two_products(S));
   S->fused_nnz = S->inner_nnz = Ap[M];
   S->inner_hash = Bp == Ap && Bi == Ai ? S->pattern_hash : tf_pattern_hash(M, Bp, Bi);
   S->march_declined = TF_MARCH_BUILT;
