@@ -433,6 +433,8 @@ enum {
  * matrix "A" and the outer one "B", the README and this ABI name them the other way
  * round).  A is L x M, B is M x Kc, C is Kc x N, D is L x N.  The schedule must come
  * from tf_inspect on A's pattern with op = TF_OP_SPMM_SPMM and the same N.
+ * C and D are two buffers.  (One may be the other, or overlap it, where the schedule runs two products or runs over a grid's whole
+ * stencil; tiles and the other marching runs read C while D is stored, unchecked.)
  * Asynchronous on `stream`.  One call at a time per schedule (it owns the workspace). */
 tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_dense *C, tf_dense *D,
                        tf_schedule *schedule, unsigned flags, void *stream);

@@ -216,3 +216,31 @@ def test_wrapped_inner_matrices_of_unknown_pattern(gpu, tf, orc, points, N):
         tf.device_synchronize()
         assert np.array_equal(D.to_numpy(), oracle_spmm_spmm(orc, A, B, Cd))
         assert (len(S.profile()) == 1) == by_runs, S.profile()
+
+
+# (whole strips on grids that were two products before there were runs for them, and larger ones, which make their intermediate then)
+@pytest.mark.gpu
+@pytest.mark.parametrize("points,dims,N", [(27, (40, 41, 39), 61), (27, (40, 41, 39), 64), (7, (48, 47, 50), 100), (7, (48, 47, 50), 64), (5, (300, 1, 310), 60), (7, (60, 55, 60), 64)])
+def test_in_place(gpu, tf, orc, points, dims, N):
+    """D in C's memory, all of it or a part: what C holds before the call is multiplied."""
+    say(f"in place on {points} points {dims} N={N}")
+    A = box_stencil(*dims, True, seed=78) if points == 27 else stencil_3d(*dims, seed=78)
+    M = A.shape[0]
+    Ah = tf.CsrMatrix.from_scipy(A)
+    S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, compute_units=256)
+    S.set_profiling(True)
+    Cd = tf.workloads.uniform((M, N), 79)
+    want = oracle_spmm_spmm(orc, A, A, Cd)
+    both = tf.DenseMatrix(M + 8, N)  # C from row 0 or 8 on, D from row 8 on (rows of 240 bytes and more, in whole 16 bytes after four of them)
+    for first in (0, 8):
+        C = tf.DenseMatrix.wrap_device(M, N, both.device_ptr() + first * N * 4)
+        D = tf.DenseMatrix.wrap_device(M, N, both.device_ptr() + 8 * N * 4)
+        C.copy_from(tf.DenseMatrix.from_numpy(Cd))
+        tf.spmm_spmm(Ah, Ah, C, D, S)
+        tf.device_synchronize()
+        assert np.array_equal(D.to_numpy(), want), (first, S.profile())
+        assert len(S.profile()) == 2
+    D = tf.DenseMatrix(M, N)
+    tf.spmm_spmm(Ah, Ah, tf.DenseMatrix.from_numpy(Cd), D, S)
+    tf.device_synchronize()
+    assert np.array_equal(D.to_numpy(), want) and len(S.profile()) == 1

@@ -51,6 +51,7 @@ struct DeviceSchedule {
   unsigned *arrived = nullptr;   // per row of several chunks: how many of them are done
   LongRow *seg_groups = nullptr;
   float *inter = nullptr;    // M x N intermediate, only if some tile writes back
+  float *spare = nullptr;    // ... one of its own, for runs over a stencil that are asked once for what they are not for
   float *partial = nullptr;  // n_long_chunks (or segments) x N
   int *seg_ptr = nullptr, *seg_src = nullptr, *seg_col = nullptr, *lrow_seg = nullptr;  // column-partitioned long rows
   float *seg_val = nullptr;  // A's values in the order of the regrouped entries
@@ -163,7 +164,7 @@ int default_compute_units() {
 
 void release_device_schedule(DeviceSchedule *d) {
   if (!d) return;
-  (void)hipFree(d->arena); (void)hipFree(d->hidden);
+  (void)hipFree(d->arena); (void)hipFree(d->hidden); (void)hipFree(d->spare);
   if (d->side) (void)hipStreamDestroy(d->side);
   if (d->fork) (void)hipEventDestroy(d->fork);
   if (d->join) (void)hipEventDestroy(d->join);
@@ -813,6 +814,10 @@ static tf::RowsArgs all_rows(const tf_csr *A, const float *X, float *Y, int N) {
 static tf_status box_as_two_products(const tf_csr *A, const tf_csr *B, const tf_dense *C, tf_dense *D, tf_schedule *s, int acc, hipStream_t st) {
   tf::DeviceSchedule *d = s->dev;
   const int N = s->opts.N, ldt = tf::inter_ld(s);
+  if (!d->inter) {
+    TF_HIP(hipMalloc(reinterpret_cast<void **>(&d->spare), (size_t)s->M * ldt * sizeof(float)));
+    d->inter = d->spare;
+  }
   tf::RowsArgs first = all_rows(B, C->d, d->inter, N), second = all_rows(A, d->inter, D->d, N);
   first.ldy = second.ldx = ldt;
   first.streaming = tf::inter_streams(s);
@@ -866,7 +871,9 @@ extern "C" tf_status tf_spmm_spmm(const tf_csr *A, const tf_csr *B, const tf_den
   if (s->box) {
     // (a wrapped matrix without a hash may have any pattern; who has runs that always were runs has given B the inner one)
     const bool unknown_inner = s->box_room && !B->hash && !(B->p == A->p && B->i == A->i);
-    if (other_inner || unknown_inner) return box_as_two_products(A, B, C, D, s, acc, st);
+    // (a run reads what is around its points in C while others store theirs in D; two products have read C when D is stored)
+    const bool in_place = D->d < C->d + (size_t)C->M * C->N && C->d < D->d + (size_t)D->M * D->N;
+    if (other_inner || unknown_inner || in_place) return box_as_two_products(A, B, C, D, s, acc, st);
     tf::BoxArgs a = s->box_runs;
     a.Ax = A->x; a.Bx = B->x; a.C = C->d; a.D = D->d;
     a.val_bytes = (unsigned)A->nnz * 4;
