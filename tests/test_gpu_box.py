@@ -244,3 +244,16 @@ def test_in_place(gpu, tf, orc, points, dims, N):
     tf.spmm_spmm(Ah, Ah, tf.DenseMatrix.from_numpy(Cd), D, S)
     tf.device_synchronize()
     assert np.array_equal(D.to_numpy(), want) and len(S.profile()) == 1
+
+
+@pytest.mark.parametrize("points,N", [(27, 61), (27, 100), (7, 100), (5, 60)])
+def test_options_that_shape_tiles_get_tiles(tf, points, N):
+    """Runs that stand in for two products do so where nothing is asked of the tiles; a budget of LDS, a tile's rows or halo and what becomes of long rows
+    shape the schedule as before."""
+    A, Ah, _ = beside_two_products(tf, points, N)
+    for kw in (dict(lds_budget_bytes=65536), dict(tile_rows=700), dict(max_redundancy=1.0), dict(long_row_nnz=8), dict(long_row_partition=-1)):
+        S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, compute_units=256, **kw)
+        info = S.info()
+        assert info["marched"] == 0 and info["lds_bytes"] <= kw.get("lds_budget_bytes", 81920), (kw, info)
+        assert info["n_producer_rows"] == A.shape[0] or "max_redundancy" not in kw, info
+        S.validate()

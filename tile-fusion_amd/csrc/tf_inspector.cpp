@@ -109,6 +109,11 @@ int tf::rows_in_order_deal(int L, int M, int N, const int *Ap) {
   return most_work * kXcds * 100 <= 115LL * Ap[L] ? (long long)M * N * 4 <= (100LL << 20) ? -1 : 512 : 0;
 }
 
+// Who sets the size of tiles, their halo or what becomes of long rows gets tiles made so, not two products or runs in their place.
+bool tf::asks_for_tiles(const tf_inspect_opts &given) {
+  return given.tile_rows > 0 || given.lds_budget_bytes > 0 || given.max_redundancy > 0.f || given.long_row_nnz > 0 || given.long_row_partition != 0;
+}
+
 // (above choose_two_passes: runs of lists with few rows to march over)
 bool tf::march_as_two_products(const tf_schedule *S) {
   return S->march_width <= kMarchW ? S->M < 150000 : (long long)S->M * S->opts.N * 4 < (192LL << 20);
@@ -190,7 +195,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
   } else if (S->march)
     want = given.march == 0 && (S->box ? S->box_us > S->box_other_us : tf::march_as_two_products(S));
   else
-    want = given.tile_rows <= 0 && given.lds_budget_bytes <= 0 && given.max_redundancy <= 0.f && given.long_row_nnz <= 0 && given.long_row_partition == 0;
+    want = !tf::asks_for_tiles(given);
   if (!want) return TF_OK;
   tf_inspect_opts o{};
   o.struct_size = sizeof(o);

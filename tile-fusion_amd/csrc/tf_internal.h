@@ -302,6 +302,7 @@ tf_status validate_march(const tf_schedule *s, int M, const int *Ap, const int *
 bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi,
                const tf_inspect_opts &o, const tf_inspect_opts &given);
 tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai, const int *Bp, const int *Bi);
+bool asks_for_tiles(const tf_inspect_opts &given);
 bool march_as_two_products(const tf_schedule *S);
 int rows_in_order_deal(int L, int M, int N, const int *Ap);
 void release_device_schedule(DeviceSchedule *d);

@@ -615,7 +615,7 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   // Where only these runs could march nobody has asked for runs: a schedule of two products, which these are taken in place of.  Where two products are faster
   // it is nothing else.
   const bool beside = given.march == 0 && !general_runs_take(best, M, given);
-  if (beside && S->box_us > S->box_other_us) return false;
+  if (beside && (S->box_us > S->box_other_us || asks_for_tiles(given))) return false;
   S->march = S->box = true;
   S->box_beside = beside;
   S->row_deal = rows_in_order_deal(M, M, o.N, Ap);
