@@ -141,15 +141,19 @@ __global__ __launch_bounds__(kBoxBlock) void fused_box_kernel(const BoxArgs a) {
     if (z >= nz || z > z1 + 1) return;
     const float *base = a.C + (size_t)z * nx * ny * N;
     const unsigned to = lds0 + (z & 1) * c_bytes + wave * (POINTS * ROW);
-    // (written out: for loads into LDS that it knows of the compiler has every later read of LDS wait)
+    // (written out: for loads into LDS that it knows of the compiler has every later read of LDS wait.  Nobody else counts the states that must pass
+    // before the load reads its base, which may come from a lane of a register (five), and m0 (one).)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (m0 named as overwritten: of a reserved register worth a warning)
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const unsigned f = WIDE ? from[WIDE ? i : 0] : source(i);
       if (f != ~0u) {
-        if constexpr (WIDE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + i * (WAVES * POINTS * ROW)), "v"(f), "s"(base) : "memory");
-        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to + i * (WAVES * POINTS * ROW)), "v"(f), "s"(base) : "memory");
+        if constexpr (WIDE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to + i * (WAVES * POINTS * ROW)), "v"(f), "s"(base) : "memory", "m0");
+        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2" ::"s"(to + i * (WAVES * POINTS * ROW)), "v"(f), "s"(base) : "memory", "m0");
       }
     }
+#pragma clang diagnostic pop
   };
 
   // acc[q][i]: the sum of point q's row in plane z - 1 + i of the three that read plane z

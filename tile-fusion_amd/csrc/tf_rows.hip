@@ -39,8 +39,9 @@ template <int V> __device__ __forceinline__ void store_any(float *p, const fvec<
 #pragma unroll
     for (int u = 0; u < V; ++u) x[u] = v.v[u];
   }
-  // (written out: the compiler makes one store of the two branches and drops the hint)
-  if (streaming && V == 4) asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(p), "v"(x) : "memory");
+  // (written out: the compiler makes one store of the two branches and drops the hint; the state that must pass before the registers of
+  // sixteen bytes are written is then ours too)
+  if (streaming && V == 4) asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 0" ::"v"(p), "v"(x) : "memory");
   else if (streaming && V == 1) asm volatile("global_store_dword %0, %1, off nt" ::"v"(p), "v"(x) : "memory");
   else *reinterpret_cast<typename at4<V>::type *>(p) = x;
 }

@@ -137,8 +137,9 @@ __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_
     const u4 v = __builtin_amdgcn_raw_buffer_load_b128(from, (int)at, 0, 0);
     return f4{__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
   };
-  auto store = [&](f4 *to, const f4 &v) __attribute__((always_inline)) {  // (written out: the compiler makes one store of the two branches and drops the hint)
-    if (a.streaming) asm volatile("global_store_dwordx4 %0, %1, off nt" ::"v"(to), "v"(v) : "memory");
+  // (written out: the compiler makes one store of the two branches and drops the hint; the state that must pass before its registers are written is then ours too)
+  auto store = [&](f4 *to, const f4 &v) __attribute__((always_inline)) {
+    if (a.streaming) asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 0" ::"v"(to), "v"(v) : "memory");
     else *to = v;
   };
   const __amdgpu_buffer_rsrc_t av = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.Ax), 0, (int)a.val_bytes, 0x00020000);
