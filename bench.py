@@ -271,16 +271,18 @@ def check_result(cfg, got, max_rows=1 << 17, W2=None):
     return err, (L if rows is None else int(rows.size))
 
 
-def kernel_names(info, op_is_gemm, unfused):
+def kernel_names(info, op_is_gemm, unfused, launches=()):
+    """What a step runs.  launches: its profile's names; which of the row kernels takes a product's rows is in there only."""
+    rows = "sweep_rows_kernel" if any(n.startswith("sweep_rows_kernel") for n in launches) else "spmm_rows_kernel"
     if unfused:
         return "dense product + spmm_rows_kernel"
     if not op_is_gemm:
         return ("fused_spmm_spmm_march_kernel" if info["marched"] else
                 "fused_spmm_spmm_window64_kernel" if info["wide_strips"] else
                 "fused_spmm_spmm_window_kernel" if info["windowed"] else
-                "fused_spmm_spmm_kernel" if info["n_fused_rows"] else "spmm_rows_kernel (twice)")
+                "fused_spmm_spmm_kernel" if info["n_fused_rows"] else rows + " (twice)")
     if info["n_fused_rows"] == 0:
-        return "dense product + spmm_rows_kernel" + (" (+ long-row segments)" if info["n_long_rows"] else "")
+        return "dense product + " + rows + (" (+ long-row segments)" if info["n_long_rows"] else "")
     return ("fused_gemm_spmm_stream_kernel" if info["streamed"] else
             "fused_gemm_spmm_regw_kernel" if info["register_weights"] else "fused_gemm_spmm_kernel")
 
@@ -345,6 +347,7 @@ def run_config(tf, cfg, idx, steps, warmup, args):
         step(st)
         kernels = [{"name": n, "ms": round(ms, 5)} for n, ms in S.profile()]
         S.set_profiling(False)
+    names = [k["name"] for k in kernels]
 
     err, rows_checked = (None, 0)
     if not args.no_check:
@@ -390,9 +393,9 @@ def run_config(tf, cfg, idx, steps, warmup, args):
         "gather": {"gathered_bytes": int(gathered), "l2_gather_TBps": L2_GATHER_TBS, "frac": round(t_gather / dev_s, 4)} if gathered else None,
         "working_set_vs_llc": round(operand_bytes / LLC_BYTES, 2),
         "rel_err_vs_f64": err, "rows_checked": rows_checked,
-        "kernels": kernels, "kernel": ("fused_gcn2_kernel" if args.two_layers == "fuse" else "2 x " + kernel_names(info, gemm, False) + " + relu_kernel")
+        "kernels": kernels, "kernel": ("fused_gcn2_kernel" if args.two_layers == "fuse" else "2 x " + kernel_names(info, gemm, False, names) + " + relu_kernel")
         if (gemm and args.two_layers) else
-        kernels[0]["name"] if info["marched"] and not args.unfused and len(kernels) == 1 else kernel_names(info, gemm, args.unfused),
+        names[0] if info["marched"] and len(names) == 1 else kernel_names(info, gemm, args.unfused, names),
         "schedule": {"lds_bytes": info["lds_bytes"], "windowed": bool(info["windowed"]), "wide_strips": bool(info["wide_strips"]),
                      "streamed": bool(info["streamed"]), "marched": bool(info["marched"]), "tiles": info["n_tiles"], "fused_rows": info["n_fused_rows"],
                      "remainder_rows": info["n_remainder_rows"], "long_rows": info["n_long_rows"],

@@ -38,9 +38,11 @@ def test_spread_rows(gpu, tf, orc, rows, N):
     want = oracle_spmm_spmm(orc, A, A, Cd)
     Ch = tf.DenseMatrix.from_numpy(Cd)
     D = tf.DenseMatrix(rows, N)
+    S.set_profiling(True)
     tf.spmm_spmm(Ah, Ah, Ch, D, S)
     tf.device_synchronize()
     assert np.array_equal(D.to_numpy(), want)
+    assert [n for n, _ in S.profile()] == ["sweep_rows_kernel"] * 2
     D0 = tf.workloads.uniform((rows, N), 53)
     D = tf.DenseMatrix(rows, N, D0)
     tf.spmm_spmm(Ah, Ah, Ch, D, S, accumulate=True)

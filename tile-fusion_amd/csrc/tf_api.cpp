@@ -10,6 +10,7 @@
 #include <new>
 
 #include "tf_internal.h"
+#include "tf_rows.h"
 
 // ---- handles ---------------------------------------------------------------------
 
@@ -466,7 +467,8 @@ static tf_status run_remainder(const tf_csr *A, tf_schedule *s, const Remainder 
   if (tf_status rc = remainder_rows(A, s, r, st, a, how)) return rc;
   // one launch, the long rows' workgroups first
   if (a.n_rows > 0 || a.n_chunks > 0)
-    TF_PHASE(s, a.n_chunks > 0 ? "spmm_rows_kernel (short and long remainder rows)" : "spmm_rows_kernel (short remainder rows)", st, launch_spmm_rows(a, how, st));
+    TF_PHASE(s, sweep_for(a, how).LPR > 0 ? "sweep_rows_kernel" : a.n_chunks > 0 ? "spmm_rows_kernel (short and long remainder rows)" : "spmm_rows_kernel (short remainder rows)", st,
+             launch_spmm_rows(a, how, st));
   if (s->long_part) {
     const int n_hot = 8 * s->seg_per_xcd, n_seg = (int)s->seg_ptr.size() - 1;
     if (!hot_on_side) {

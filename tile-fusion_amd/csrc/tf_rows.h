@@ -67,7 +67,7 @@ struct SweepShape { int LPR = 0, slices = 1, steps = 0; };
 inline SweepShape sweep_for(const RowsArgs &a, const RowsHow &how) {
   SweepShape s;
   const long long bytes = (long long)a.x_rows * a.ldx * 4;
-  if (how.spread_entries <= 0 || how.flagged || how.xcd_chunk_rows != 0 || a.n_chunks > 0 || a.rows || a.n_zero > 0 ||
+  if (row_shape(a.N, a.accumulate).V != 4 || how.spread_entries <= 0 || how.flagged || how.xcd_chunk_rows != 0 || a.n_chunks > 0 || a.rows || a.n_zero > 0 ||
       !sweep_fits(a.x_rows, a.N, a.n_rows, how.spread_entries) || bytes > 0x80000000ll)
     return s;
   s.LPR = a.N <= 16 ? 4 : row_shape(a.N, 0).LPR;

@@ -625,7 +625,7 @@ hipError_t launch_spmm_rows(RowsArgs a, const RowsHow &how, hipStream_t st) {
   a.chunk_blocks = (a.n_chunks + kXcds - 1) / kXcds * kXcds;
   a.slices = s.V == 4 && !how.flagged && how.xcd_chunk_rows == 0 ? slices_for(a) : 1;
   if (a.slices > 1) s.LPR = kSliceCols / 4;
-  const SweepShape sweep = s.V == 4 ? sweep_for(a, how) : SweepShape{};
+  const SweepShape sweep = sweep_for(a, how);
   if (sweep.LPR > 0) {
     const int rows = kBlock / sweep.LPR * kSweepRows, per = kXcds / sweep.slices;
     a.slices = sweep.slices;
