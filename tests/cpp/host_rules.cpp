@@ -93,6 +93,10 @@ static int sweep_columns() {
               if (!ok) { printf("N %d ldx %d rows %lld accumulate %d: %d lanes, %d slices, %d steps\n", N, ldx, rows, accumulate, s.LPR, s.slices, s.steps); ++bad; }
             }
   for (int n : shapes) bad += n == 0;
+  // 128 columns: four slices of the other kernel up to 20 MB of X
+  for (long long rows : {30000LL, 39000LL, 39104LL, 46000LL})
+    for (int mean : {6, 11, 17})
+      if (tf::sweep_fits(rows, 128, rows, rows * mean) != (rows > 39062)) { printf("%lld rows of %d, N 128\n", rows, mean); ++bad; }
   return bad;
 }
 

@@ -9,10 +9,10 @@ from test_gpu_parity import oracle_spmm_spmm, say
 pytestmark = pytest.mark.gpu
 
 
-# rows: a little more than 15 MB of X for the width, at the edges of a workgroup's rows; N: every number of lanes, slices of 32 and of 64 columns, rows
+# rows: a little more than 15 MB of X for the width (20 for 128), at the edges of a workgroup's rows; N: every number of lanes, slices of 32 and of 64 columns, rows
 # that do not start at a line, a last lane that reaches back (97: into the slice before it).  Row lengths around the 16 entries that
 # are kept in LDS, none, and as many as a row in one piece may have; one row reads one column many times, one reads the last columns only.
-@pytest.mark.parametrize("rows,N", [(29312, 128), (84001, 128), (38703, 97), (37502, 100), (58602, 64), (76531, 49), (113641, 33), (117249, 32),
+@pytest.mark.parametrize("rows,N", [(39104, 128), (84001, 128), (38703, 97), (37502, 100), (58602, 64), (76531, 49), (113641, 33), (117249, 32),
                                     (220601, 17), (234385, 16), (340910, 11), (140001, 128)])
 def test_spread_rows(gpu, tf, orc, rows, N):
     say(f"spread rows, {rows} rows, N={N}")

@@ -49,14 +49,17 @@ inline int slices_for(const RowsArgs &a) {
 
 // sweep_rows_kernel: rows of some entries each, spread over an X that no L2 holds and the Infinity Cache does.  Erdos-Renyi graphs, one product,
 // the other kernel / this one (us; a layer's two products with values read in place in brackets): N = 64, 60,000 rows of 11 20.3 / 20.8
-// (47.2 / 41.8), 100,000 38.2 / 34.1 (83 / 69), 200,000 82.9 / 77.7 (177 / 156); N = 128, 30,000 rows 15.7 / 18.0 (34.6 / 35.7), 60,000 38.5 / 38.4 (88 / 77),
+// (47.2 / 41.8), 100,000 38.2 / 34.1 (83 / 69), 200,000 82.9 / 77.7 (177 / 156); N = 128, 60,000 38.5 / 38.4 (88 / 77),
 // 100,000 77.5 / 67.0 (173 / 137), 200,000 168 / 156 (344 / 315), 400,000 335 / 334 (690 / 656); N = 32, 200,000 rows 42.4 / 40.4 (95 / 83); N = 16,
 // 250,000 rows 44.1 / 36.9 (106 / 78).  Not below 15 MB of X (36,000 rows of 13, N = 100: 21.3 / 23.2), where it outgrows the Infinity Cache (10^6 rows of
 // 9, N = 64: 355 / 359), for fewer than 5.5 entries a row (200,000 rows of 4, N = 64: 35.8 / 37.2), or where a row is three quarters of a lane group
-// (120,000 rows, N = 80: 68 / 70).
+// (120,000 rows, N = 80: 68 / 70).  Four slices of whole lines of 128 columns hold out longer, up to 20 MB (two products, kept values, rows of 6 / 9 / 11 / 17:
+// 30,000 rows 24.2 / 28.5 / 31.8 / 43.4 against 27.6 / 33.8 / 37.3 / 53.2, 34,000 26.8 / 32.4 / 36.4 / 50.3 against 29.8 / 34.6 / 39.4 / 56.2, 38,000 30.0 / 36.9 / 41.6 /
+// 57.9 against 32.2 / 37.9 / 41.6 / 59.7, 42,000 33.5 / 42.0 / 47.5 / 67.7 against 35.5 / 42.9 / 49.1 / 70.8, 46,000 37.3 / 47.2 / 54.2 / 76.5 against 37.9 / 45.9 / 50.6 / 71.1; a layer
+// of 64 -> 128, values read in place, rows of 17: 30,000 rows 77.3 against 79.3, 34,000 89.9 against 89.0, 42,000 106 against 103.5).
 constexpr int kSweepRows = 4, kSweepEntries = 16;
 constexpr bool sweep_fits(long long x_rows, int N, long long rows, long long entries) {
-  return N >= 4 && (N <= 64 || (N > 96 && N <= 128)) && x_rows * N * 4 >= 15000000 && x_rows * N * 4 <= (256ll << 20) && 2 * entries >= 11 * rows;
+  return N >= 4 && (N <= 64 || (N > 96 && N <= 128)) && x_rows * N * 4 >= (N == 128 ? 20000000 : 15000000) && x_rows * N * 4 <= (256ll << 20) && 2 * entries >= 11 * rows;
 }
 // Lanes a row takes, column slices, and the steps in which the limit passes over X.  Slices as above where rows start at a line, of 64 columns where four
 // of 32 do not pay: as long as an XCD's slice is small enough that most of it is read by more than one row in flight (N = 128, whole rows / two slices / four:
