@@ -250,13 +250,43 @@ static int streamed_entries() {
   return bad;
 }
 
+// Graphs whose reads are spread alike take the sweep, in one product as in two; one column that is read 255 times or more and they do not, whatever
+// a byte makes of its count.
+static int even_reads() {
+  int bad = 0;
+  const int M = 60000, mean = 11;
+  for (int often : {0, 254, 255, 256, 257, 300, 512, 767, 1024, 60000}) {
+    std::vector<int> p(1, 0), i;
+    unsigned long long at = 1;
+    for (int r = 0; r < M; ++r) {
+      for (int k = 0; k < mean; ++k) {
+        at = at * 6364136223846793005ull + 1442695040888963407ull;
+        i.push_back(1 + (int)((at >> 33) % (M - 1)));
+      }
+      if (r < often) i.push_back(0);
+      p.push_back((int)i.size());
+    }
+    tf_inspect_opts o{};
+    o.struct_size = sizeof(o);
+    o.op = TF_OP_SPMM_SPMM;
+    o.N = 64;
+    tf_schedule *s = nullptr, *rows = nullptr;
+    if (tf_inspect(M, M, p.data(), i.data(), &o, &s) || tf_inspect_spmm(M, M, p.data(), i.data(), 64, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
+    if (!s->two_passes || s->two_passes->rem_sweep != (often < 255) || rows->rem_sweep != (often < 255)) { printf("a column read %d times\n", often); ++bad; }
+    tf_schedule_free(s);
+    tf_schedule_free(rows);
+  }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
     const int b = !strcmp(argv[k], "column_owners") ? column_owners() : !strcmp(argv[k], "sweep_columns") ? sweep_columns() : !strcmp(argv[k], "one_launch_fits") ? one_launch_fits()
                   : !strcmp(argv[k], "partial_sums") ? partial_sums()
                   : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns()
-                  : !strcmp(argv[k], "streamed_entries") ? streamed_entries() : 1;
+                  : !strcmp(argv[k], "streamed_entries") ? streamed_entries()
+                  : !strcmp(argv[k], "even_reads") ? even_reads() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

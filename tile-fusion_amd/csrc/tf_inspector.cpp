@@ -121,7 +121,7 @@ bool tf::march_as_two_products(const tf_schedule *S) {
 
 enum { kTiles, kRows, kRowsOfChecked };
 constexpr int kWholeRowMax = 128;  // rows of more entries are cut up, whatever the widths and row counts (unless the caller says otherwise)
-static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out);
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out, int reads_even = -1);
 
 // Which SpMM-SpMM schedules the executor runs as two row products instead of in their tiles, when the caller has not asked
 // for tiles of its own.
@@ -205,7 +205,7 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
   o.xcd_chunk_rows = given.xcd_chunk_rows;
   o.reorder_adjacency = given.reorder_adjacency;
   o.pattern_hash = S->pattern_hash;
-  if (tf_status rc = inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes)) return rc;
+  if (tf_status rc = inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes, S->reads_even)) return rc;
   const tf_schedule *rows = S->two_passes;
   if (S->one_launch && (!rows->long_chunks.empty() || rows->long_part || rows->rem_flagged)) {
     // hub rows: another order of the products, or the schedule's own (a GEMM of the rows that are read, placed by reads)
@@ -215,15 +215,16 @@ static tf_status choose_two_passes(tf_schedule *S, const tf_inspect_opts &given,
       tf_schedule_free(S->two_passes);
       S->two_passes = nullptr;
       o.N = S->user_N;  // (the lists and the room for partial sums are for the width that is gathered)
-      if (!S->launch_tiles.empty()) return inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes);
+      if (!S->launch_tiles.empty()) return inspect(S->L, S->M, Ap, Ai, &o, kRowsOfChecked, &S->two_passes, S->reads_even);
     }
   }
   return TF_OK;
 }
 
 // kRows: a schedule for one product Y = A X (tf_inspect_spmm): no tiles, every row in the remainder lists.  kRowsOfChecked: the same of a
-// pattern that an inspection under way has checked (a pass over the entries less: 2.5 of 14.5 ms at 100,000 rows of 16).
-static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out) {
+// pattern that an inspection under way has checked (a pass over the entries less: 2.5 of 14.5 ms at 100,000 rows of 16).  reads_even: what is known of the
+// pattern (tf_schedule).
+static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_inspect_opts *user, int what, tf_schedule **out, int reads_even) {
   const bool rows_only = what != kTiles;
   if (!out) return tf::fail(TF_EINVAL, "tf_inspect: out is null");
   *out = nullptr;
@@ -344,6 +345,7 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     S->user_K = user_K;
     S->user_N = user_N;
     S->rows_only = rows_only;
+    S->reads_even = reads_even;
     S->n_panels = n_panels;
     S->gemm_regw = gemm_regw;
     S->gemm_stream = gemm_stream;
@@ -640,12 +642,13 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // Remainder: rows not fused; long ones are cut into chunks of up to chunk_nnz entries, each
     // worked on by a whole workgroup.
     const int chunk_nnz = std::max(o.long_row_nnz, 1024);
-    std::vector<char> need(M, 0);
+    std::vector<unsigned char> need(M, 0);  // by how many entries, up to 255
+    auto read_by = [of = need.data()](int c) { of[c] += of[c] != 255; };
     if (rows_only) S->rem_rows.reserve(L);
     for (int i = 0; i < L; ++i) {
       if (fused[i]) { S->fused_nnz += Ap[i + 1] - Ap[i]; continue; }
       if (!rows_only)
-        for (int k = Ap[i]; k < Ap[i + 1]; ++k) need[Ai[k]] = 1;
+        for (int k = Ap[i]; k < Ap[i + 1]; ++k) read_by(Ai[k]);
       const int len = Ap[i + 1] - Ap[i];
       if (len > o.long_row_nnz) {
         tf::LongRow lr{i, (int)S->long_chunks.size(), 0, 0};
@@ -687,17 +690,21 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       for (const auto &lr : S->long_rows)
         if (Ap[lr.row + 1] - Ap[lr.row] > kWholeRowMax) return false;
       if (!scattered()) return false;
-      // The most-read eighth of the columns takes less than a quarter of the reads: summed up from the most-read ones down.
-      std::vector<int> reads(M, 0), of_count(256, 0);
-      for (long long k = 0; k < nnz; ++k) ++reads[Ai[k]];
-      for (int r : reads) ++of_count[std::min(r, 255)];
-      long long left = M / 8, taken = 0;
-      for (int c = 255; c >= 0 && left > 0; --c) {
-        const long long cols = std::min<long long>(left, of_count[c]);
-        taken += cols * c;
-        left -= cols;
+      // The most-read eighth of the columns takes less than a quarter of the reads, and none 255 or more: summed up from the most-read ones down.  (Once for a
+      // schedule and its two products, whose rows are all counted above: 50,000 rows of 13 would take 0.8 of 6 ms for each.)
+      if (S->reads_even < 0) {
+        if (rows_only) std::for_each(Ai, Ai + nnz, read_by);
+        std::vector<int> of_count(256, 0);
+        for (int r : need) ++of_count[r];
+        long long left = M / 8, taken = 0;
+        for (int c = 255; c >= 0 && left > 0; --c) {
+          const long long cols = std::min<long long>(left, of_count[c]);
+          taken += cols * c;
+          left -= cols;
+        }
+        S->reads_even = of_count[255] == 0 && 4 * taken < nnz;
       }
-      return of_count[255] == 0 && 4 * taken < nnz;
+      return S->reads_even == 1;
     };
     const bool sweep = for_sweep();
     std::vector<signed char> part;  // per intermediate row: its hot partition, or -1 (empty without long_part)

@@ -196,6 +196,7 @@ struct tf_schedule {
                                     // length class so that a workgroup's rows cost about the same
   bool rem_identity = false;        // rem_rows is 0..L-1 in order
   bool rem_sweep = false;           // ... whose columns are spread over all alike (RowsHow::spread_entries)
+  int reads_even = -1;              // no column of A is read much more often than the others (-1: not counted)
   std::vector<int> zero_rows;       // second-op rows without entries, when many: their rows of D are cleared by a
                                     // fill kernel instead of taking a lane group each in the row kernel
   // When the list is not the identity, its rows are also kept as a CSR of their own in list order
