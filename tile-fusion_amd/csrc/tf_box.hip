@@ -3,7 +3,6 @@
 // tf_march.cpp).  Any values.  The reference's answer to such patterns is tiling with redundancy (fusion/src/SpMM_SpMM.cpp:984-1057).
 #include <hip/hip_runtime.h>
 #include <algorithm>
-#include <cstdlib>
 #include <utility>
 
 #include "tf_internal.h"
@@ -235,11 +234,10 @@ __global__ __launch_bounds__(kBoxBlock) void fused_box_kernel(const BoxArgs a) {
 }
 
 hipError_t launch_fused_box(BoxArgs a, int accumulate, hipStream_t st) {
-  static const bool remap = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
   const int lds = box_lds(a.q, a.by);
   if (a.by < 1 || a.by > kBoxMaxY || lds > kMaxLds || a.n_runs <= 0) return hipErrorInvalidValue;
-  a.per_xcd = remap ? (a.n_runs + kXcds - 1) / kXcds : 0;
-  const dim3 grid((a.n_runs + kXcds - 1) / kXcds * kXcds);
+  a.per_xcd = per_xcd_of(a.n_runs);
+  const dim3 grid(grid_of(a.n_runs));
   const bool wide = a.N % 4 == 0;  // a load of four floats into LDS wants 16 bytes' alignment (operands have it: tf_dense_wrap_device)
   hipError_t err = hipErrorInvalidValue;
 #define CALL3(Q_, ACC_, WIDE_)                                                                                                                        \

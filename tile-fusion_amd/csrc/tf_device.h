@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <climits>
+#include <cstdlib>
 
 #include "tf_internal.h"
 
@@ -72,6 +73,15 @@ __device__ __forceinline__ int xcd_contiguous(int bid, int bpc) {
   const int xcd = bid % kXcds, s = bid / kXcds;
   return ((s / bpc) * kXcds + xcd) * bpc + (s % bpc);
 }
+
+// Work items per XCD for xcd_contiguous; 0 (identity mapping) when the environment variable
+// TF_XCD_REMAP is set to 0.  The grid is sized grid_of(n) either way.
+inline bool xcd_remap_on() {
+  static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
+  return on;
+}
+inline int per_xcd_of(int n) { return xcd_remap_on() ? (n + kXcds - 1) / kXcds : 0; }
+inline int grid_of(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every
 // global load and store of the wavefront, which would cut off the loads a kernel issues

@@ -1570,15 +1570,6 @@ Shape pick_shape(int N) {
   return {V, LPR};
 }
 
-// Work items per XCD for xcd_contiguous; 0 (identity mapping) when the environment variable
-// TF_XCD_REMAP is set to 0.  The grid is sized grid_of(n) either way.
-inline bool xcd_remap_on() {
-  static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
-  return on;
-}
-inline int per_xcd_of(int n) { return xcd_remap_on() ? (n + kXcds - 1) / kXcds : 0; }
-inline int grid_of(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
-
 template <class F> hipError_t allow_lds(F kernel, int bytes) {
   if (bytes <= 65536) return hipSuccess;
   return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),

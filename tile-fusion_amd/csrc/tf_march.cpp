@@ -556,7 +556,6 @@ bool stencil_grid(int star, int M, const int *Ap, const int *Ai, int grid[3]) { 
 
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 constexpr int strip_cols(const BoxArgs &b) { return b.star ? 32 : 64; }
-constexpr int column_x(const BoxArgs &b) { return b.bx; }
 constexpr int runs_lds(const BoxArgs &b) { return !b.star ? box_lds(b.q, b.by) : b.ny == 1 ? flat_lds() : star_lds(b.by); }
 
 // Whether build_march makes runs of its lists over a grid's whole stencil too: whole strips, offsets and lists of 32 bits (some 2.7 ELL rows of 256 bytes a
@@ -621,7 +620,7 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->row_deal = rows_in_order_deal(M, M, o.N, Ap);
   S->box_runs = best;
   std::copy(grid, grid + 3, S->march_grid);
-  S->march_tile[0] = column_x(best); S->march_tile[1] = best.by;
+  S->march_tile[0] = best.bx; S->march_tile[1] = best.by;
   S->lds_bytes = runs_lds(best);
   S->march_slots = S->slab_rows = S->lds_bytes / kMarchRowBytes;
   S->march_width = flat ? 5 : star ? 7 : 27;
@@ -635,8 +634,8 @@ bool build_box(tf_schedule *S, int M, const int *Ap, const int *Ai, const int *B
   S->ptr2.assign(1, 0);
   for (int z0 = 0; z0 < nz; z0 += best.zlen)
     for (int y0 = 0; y0 < ny; y0 += best.by)
-      for (int x0 = 0; x0 < nx; x0 += column_x(best)) {
-        const int x1 = std::min(nx, x0 + column_x(best)), y1 = std::min(ny, y0 + best.by), z1 = std::min(nz, z0 + best.zlen);
+      for (int x0 = 0; x0 < nx; x0 += best.bx) {
+        const int x1 = std::min(nx, x0 + best.bx), y1 = std::min(ny, y0 + best.by), z1 = std::min(nz, z0 + best.zlen);
         TileDesc t{};
         t.cons_begin = (int)S->fused_ids.size();
         for (int z = z0; z < z1; ++z)
@@ -671,7 +670,7 @@ tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai
   if (b.N != s->opts.N || (b.star && b.N % 4 != 0) || b.strips != ceil_div(b.N, strip_cols(b)) || b.by < 1 || b.by > (b.star ? kStarMaxY : kBoxMaxY) || s->lds_bytes != runs_lds(b) || s->lds_bytes > kMaxLds)
     return fail(TF_ESCHEDULE, "runs over a grid: %d columns, %d lines, %d bytes of LDS", b.N, b.by, s->lds_bytes);
   const int cuts = b.zlen > 0 ? ceil_div(b.nz, b.zlen) : 0;
-  if (cuts < 1 || b.q < 1 || b.tx != ceil_div(b.nx, column_x(b)) || b.ty != ceil_div(b.ny, b.by) || (long long)b.tx * b.ty * cuts * b.strips != b.n_runs ||
+  if (cuts < 1 || b.q < 1 || b.tx != ceil_div(b.nx, b.bx) || b.ty != ceil_div(b.ny, b.by) || (long long)b.tx * b.ty * cuts * b.strips != b.n_runs ||
       s->tiles.size() != (size_t)b.tx * b.ty * cuts)
     return fail(TF_ESCHEDULE, "runs over a grid: %d runs of %d planes do not cover it", b.n_runs, b.zlen);
   std::vector<char> done(M, 0);
@@ -679,7 +678,7 @@ tf_status validate_box(const tf_schedule *s, int M, const int *Ap, const int *Ai
     const TileDesc &t = s->tiles[r];
     for (int q = t.cons_begin; q < t.cons_end; ++q) {
       const int i = s->fused_ids[q], x = i % b.nx, y = i / b.nx % b.ny, z = i / b.nx / b.ny;
-      if (i < 0 || i >= M || done[i]++ || (size_t)((z / b.zlen * b.ty + y / b.by) * b.tx + x / column_x(b)) != r)
+      if (i < 0 || i >= M || done[i]++ || (size_t)((z / b.zlen * b.ty + y / b.by) * b.tx + x / b.bx) != r)
         return fail(TF_ESCHEDULE, "runs over a grid: row %d is not run %zu's, or twice there", i, r);
     }
   }

@@ -6,7 +6,6 @@
 // the number of rows in flight.
 #include <hip/hip_runtime.h>
 #include <algorithm>
-#include <cstdlib>
 #include <utility>
 
 #include "tf_internal.h"
@@ -593,11 +592,6 @@ __global__ __launch_bounds__(kSegBlock) void long_seg_reduce_kernel(const LongRo
 // ---- launchers ----------------------------------------------------------------------
 
 namespace {
-
-inline bool xcd_remap_on() {
-  static const bool on = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
-  return on;
-}
 
 // How a.n_blocks workgroups of `rows` rows are dealt to the XCDs -- 0: workgroup b takes block b; > 0: chunks of rows per XCD turn;
 // < 0: one contiguous run per XCD -- and the workgroups to launch for it.

@@ -2,7 +2,6 @@
 // point reads itself and its neighbours along the axes, x fastest (checked against the matrices by the inspector: build_box in tf_march.cpp).  Any values.
 // The reference's answer to such patterns is tiling with redundancy (fusion/src/SpMM_SpMM.cpp:984-1057).
 #include <hip/hip_runtime.h>
-#include <cstdlib>
 
 #include "tf_internal.h"
 #include "tf_device.h"
@@ -229,15 +228,14 @@ __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_
 }
 
 hipError_t launch_fused_star(BoxArgs a, int accumulate, hipStream_t st) {
-  static const bool remap = [] { const char *e = getenv("TF_XCD_REMAP"); return !(e && e[0] == '0'); }();
   const bool flat = a.ny == 1;
   const int lds = flat ? flat_lds() : star_lds(a.by), block = flat ? kFlatBlock : kStarBlock;
   if (a.by < 1 || a.by > kStarMaxY || a.bx < 1 || a.bx > (flat ? kFlatX : kStarX) || a.N % 4 != 0 || a.n_runs <= 0) return hipErrorInvalidValue;
-  a.per_xcd = remap ? (a.n_runs + kXcds - 1) / kXcds : 0;
+  a.per_xcd = per_xcd_of(a.n_runs);
   // Streaming stores but where strips share lines of a D that the Infinity Cache does not hold, which would go to memory in parts (us, streaming / plain:
   // N = 100, 128^3 points 719 / 642, 1000 x 1000 302 / 259, 64^3 63.1 / 61.8; N = 84, 96^3 201 / 206; N = 48, 64^3 34.4 / 35.7; whole lines, 128^3, N = 64 254 / 262).
   a.streaming = a.N % 32 == 0 || (long long)a.nx * a.ny * a.nz * a.N * 4 <= (320ll << 20);
-  const dim3 grid((a.n_runs + kXcds - 1) / kXcds * kXcds);
+  const dim3 grid(grid_of(a.n_runs));
 #define CALL(ACC_, SAME_, FLAT_)                                                                                                                             \
   do {                                                                                                                                                      \
     const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fused_star_kernel<ACC_, SAME_, FLAT_>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
