@@ -257,3 +257,28 @@ def test_options_that_shape_tiles_get_tiles(tf, points, N):
         assert info["marched"] == 0 and info["lds_bytes"] <= kw.get("lds_budget_bytes", 81920), (kw, info)
         assert info["n_producer_rows"] == A.shape[0] or "max_redundancy" not in kw, info
         S.validate()
+
+
+# (N: one strip of part of its columns, a whole and half of one, one and a bit; the grid's edges off the columns' both ways)
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,N", [((61, 59, 47), 36), ((61, 59, 47), 60), ((48, 47, 50), 96), ((47, 48, 50), 100), ((60, 62, 49), 44), ((61, 59, 47), 132)])
+def test_box_sixteen_byte_loads_of_part_of_a_strip(gpu, tf, orc, dims, N):
+    """Widths of whole sixteen bytes that are no whole strips: the form that loads four columns at once, some of its lanes with nothing to load."""
+    say(f"box {dims} N={N}")
+    A = box_stencil(*dims, True, seed=41)
+    B = A.copy()
+    B.data = np.random.default_rng(42).uniform(-1, 1, B.nnz).astype(np.float32)
+    Cd = tf.workloads.uniform((A.shape[0], N), 43)
+    D0 = tf.workloads.uniform((A.shape[0], N), 44)
+    want = oracle_spmm_spmm(orc, A, B, Cd)
+    Ah, Bh = tf.CsrMatrix.from_scipy(A), tf.CsrMatrix.from_scipy(B)
+    S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, compute_units=256)
+    S.set_profiling(True)
+    for acc in (False, True):
+        D = tf.DenseMatrix(A.shape[0], N, D0) if acc else tf.DenseMatrix(A.shape[0], N)
+        if not acc:
+            D.fill(float("nan"))
+        tf.spmm_spmm(Ah, Bh, tf.DenseMatrix.from_numpy(Cd), D, S, accumulate=acc)
+        tf.device_synchronize()
+        assert np.array_equal(D.to_numpy(), D0 + want if acc else want), (dims, N, acc)
+        assert [n for n, _ in S.profile()] == ["fused_box_kernel"]

@@ -195,3 +195,34 @@ def test_march_wide_accumulate_other_values_and_flat_grid(gpu, tf, orc):
     got, info = march(tf, F, F, Cf)
     assert np.array_equal(got, oracle_spmm_spmm(orc, F, F, Cf)), info
 
+
+
+# 27 points and a pattern that is not wholly their stencil's, or a column that is given: runs of lists, rows of up to 27 entries
+@pytest.mark.parametrize("dims,N,whole", [((12, 12, 12), 64, True), ((20, 17, 9), 128, True), ((24, 24, 24), 64, False), ((9, 14, 31), 192, False)])
+def test_march_lists_of_27_points_bit_exact(gpu, tf, orc, dims, N, whole):
+    say(f"march lists of 27 points {dims} whole={whole} N={N}")
+    A = box_stencil(*dims, True, seed=51)
+    if not whole:
+        A.data[A.indptr[A.shape[0] // 2] + 3] = 0
+        A.eliminate_zeros()
+    B = A.copy()
+    B.data = np.random.default_rng(52).uniform(-1, 1, B.nnz).astype(np.float32)
+    Cd = tf.workloads.uniform((A.shape[0], N), 53)
+    D0 = tf.workloads.uniform((A.shape[0], N), 54)
+    Ah, Bh = tf.CsrMatrix.from_scipy(A), tf.CsrMatrix.from_scipy(B)
+    for kw in (dict(), dict(compute_units=16)):
+        if whole:
+            kw["march_tile"] = (8, 4)
+        S = tf.inspector(Ah, 1, op=tf.OP_SPMM_SPMM, N=N, inner=Ah, march=1, **kw)
+        S.validate()
+        S.set_profiling(True)
+        for inner, want in ((Ah, oracle_spmm_spmm(orc, A, A, Cd)), (Bh, oracle_spmm_spmm(orc, A, B, Cd))):
+            for acc in (False, True):
+                D = tf.DenseMatrix(A.shape[0], N, D0)
+                tf.spmm_spmm(Ah, inner, tf.DenseMatrix.from_numpy(Cd), D, S, accumulate=acc)
+                tf.device_synchronize()
+                if not acc:
+                    assert np.array_equal(D.to_numpy(), want), (dims, N, kw)
+                else:
+                    assert orc.rel_err(D.to_numpy(), want.astype(np.float64) + D0) <= 1e-6
+                assert any(n.startswith("fused_spmm_spmm_march_kernel") for n, _ in S.profile()), S.profile()

@@ -8,6 +8,8 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
+from test_gpu_spread import spread
+
 torch = pytest.importorskip("torch")
 ops_mod = importlib.import_module("tile-fusion_amd.torch_ops")
 TOL = 1e-4
@@ -300,3 +302,32 @@ def test_captured_calls_on_two_streams(gpu, tf):
                 assert torch.equal(t, want)
             assert torch.equal(call(), want)
             torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,K,H,N", [(62001, 48, 64, 64), (45000, 100, 96, 100)])
+def test_layers_on_graphs_without_locality(gpu, n, K, H, N):
+    """Graphs large enough for sweep_rows_kernel (test_gpu_spread.py): a layer forward and backward, and two layers with a ReLU between, forward also
+    after the values have changed."""
+    print(f"sw_gcn spread layers n={n} {K} -> {H} -> {N}", flush=True)
+    A = spread(n, n, 9, 64)
+    g = torch.Generator().manual_seed(65)
+    x0, w1, w2 = torch.rand(n, K, generator=g), torch.rand(H, K, generator=g) - 0.5, torch.rand(N, H, generator=g) - 0.5
+    go = torch.rand(n, H, generator=g) - 0.5
+    adj = csr_tensor(A, "cuda")
+    for step in range(2):
+        B = A.astype(np.float64)
+        B.data = B.data * (1 + step)
+        adj.values().data.copy_(torch.tensor(A.data * np.float32(1 + step)))
+        xd, w1d, w2d, god = (t.double().numpy() for t in (x0, w1, w2, go))
+        one = B @ (xd @ w1d.T)
+        x, w = x0.cuda().requires_grad_(), w1.cuda().requires_grad_()
+        out = torch.ops.sw_gcn.fusedGeMMSpMM_vt_ro(adj, x, w, torch.ops.sw_gcn.inspect_vt_ro(adj, K, H, 500000, 8), 8, 0)
+        assert rel_err(out, one) <= TOL, step
+        if step == 0:  # (the transpose is made again after changes that a version counter shows)
+            out.backward(go.cuda())
+            back = B.T @ god
+            assert rel_err(x.grad, back @ w1d) <= TOL and rel_err(w.grad, back.T @ xd) <= TOL
+        with torch.no_grad():
+            two = torch.ops.sw_gcn.fusedGCN(adj, x0.cuda(), w1.cuda(), w2.cuda(), 8)
+        assert rel_err(two, B @ (np.maximum(one, 0) @ w2d.T)) <= TOL, step
