@@ -97,8 +97,8 @@ template <int Q> struct BoxValues {
 // v_mfma_f32_4x4x1 does: four values, broadcast from the block of lanes that the instruction names, times the value of each lane, added to four registers,
 // each sum rounded once as by a fused multiply-add (5 million random ones, denormals and infinities among them, have fmaf's bits) -- a row's entries come in
 // the order of its columns, so results carry the reference's bits.  The fourth register is left over; three fused multiply-adds in 8.8 cycles are still
-// more than v_fmac_f32 with a DPP broadcast makes (4.6 each).  96^3 points, N = 64: 174 us, against 533 in gathering runs and 560 as two products;
-// on DPP in this arrangement 216.  What is left: the matrix cores are busy 0.43 of the time, other VALU work and their power take as much again;
+// more than v_fmac_f32 with a DPP broadcast makes (4.6 each).  96^3 points, N = 64: 164 us (174 on another card), against 533 in gathering runs and 550 as two products;
+// on DPP in this arrangement 216.  What is left, of 174: the matrix cores are busy 0.43 of the time, other VALU work and their power take as much again;
 // without any loads it takes 127, without the sums 150.  (A plane of C ahead of time into L2: nothing gained.  Each row's values in three parts, as the
 // planes ask for them, 180.  Lines of seven points: registers spill, 424.)
 template <int Q, bool ACC, bool WIDE>

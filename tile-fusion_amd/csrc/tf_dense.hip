@@ -901,7 +901,8 @@ WeightGradTask plan_weight_grad(int M, int N, int K, int compute_units) {
   // (a multiple of 8: the chunks of a block of rows on one XCD, whose L2 has the other operand and the lines two chunks share)
   const int chunks = p.n_chunks * p.k_chunks, blocks = (M + kWgRows - 1) / kWgRows;
   // Eight wavefronts a workgroup halve the sums that go through memory, where every wavefront of the device has a block of rows all the same (two groups
-  // of four / one of eight, both launches: 100,000 rows 64 x 128 30.1 / 27.8 us, a layer 145 / 141; 131,072 rows 64 x 300 and 40 x 64 73 / 70, the step 291 / 287).
+  // of four / one of eight, both launches: 100,000 rows 64 x 128 30.1 / 27.8 us, a layer 145 / 141; 131,072 rows 64 x 300 and 40 x 64 73 / 70, of a step of 280 that runs
+  // differ by as much).
   p.waves = blocks >= 8 * compute_units ? 8 : 4;
   p.groups = std::max(1, std::min(std::max(1, 8 / p.waves * compute_units / chunks), (blocks + p.waves - 1) / p.waves));
   if (p.groups > 8) p.groups = p.groups / 8 * 8;

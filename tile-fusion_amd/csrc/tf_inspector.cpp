@@ -132,14 +132,17 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
 //    needs 256 runs.  Rows of up to 8 entries, N = 64, runs / two products: 40,000 rows 25 / 13 us, 110,592 rows 34 / 28 us,
 //    216,000 rows 48 / 50 us (N = 128: 97 / 121), 2^21 rows 341 / 610 us.  Wider rows (27 points): 64,000 rows 70 / 46 us, 512,000 rows 327 / 294 us and (N = 128)
 //    623 / 654 us, 884,736 rows 548 / 550 us: the runs win once C and the intermediate outgrow the 256 MB Infinity Cache.
-//    Runs over a grid's whole 27-point stencil have a kernel of their own (us, its runs / two products): N = 64, 16^3 points 18 / 8, 32^3 25 / 22,
-//    40^3 31 / 39, 64^3 87 / 136, 96^3 174 / 560; 64^3, N = 16 84 / 59, 32 85 / 86, 37 94 / 124, 96 150 / 240.  Their expected time, a sum over
-//    runs and planes (build_box), against 5 + M (0.11 + 0.0063 N) / 1000, which is within a tenth of two products on up to 64^3 points.
-//    So have runs over its whole 7-point stencil (us, its runs / two products / the other runs): N = 64, 24^3 points 11.3 / 8.6, 32^3 11.3 / 11.5, 40^3 15.9 /
-//    18.6, 64^3 34 / 59 / 49, 96^3 114 / 294 / 181, 128^3 230 / 619 / 290; N = 128, 32^3 14.5 / 18.9, 64^3 60 / 136 / 97; 128^3, N = 32 130 / 352, 100 642 / 1,120; 90 x 70
-//    x 80, N = 36 70 / 103; against 4 + M (N, in whole lines) 0.0034 / 1000.  Any N of a multiple of four.  And over the 5-point stencil of a 2D grid whose
-//    lines no window holds: N = 64, 400 x 100 13.8 / 12.8, 300^2 19.3 / 23.3 / 28.4, 500^2 34 / 53 / 44, 1024 x 200 29 / 44 / 44, 700^2 54 / 141 / 90, 1000^2
-//    120 / 310 / 162; 250^2, N = 48 15.6 / 16.4, 600 x 500, N = 36 37 / 58.
+//    Runs over a grid's whole 27-point stencil have a kernel of their own (us, its runs / two products): N = 64, 16^3 points 17.6 / 8.8, 32^3 23.4 / 20.3,
+//    40^3 28 / 34, 64^3 81 / 118, 96^3 164 / 550, 128^3 399 / 1,260; 64^3, N = 16 81 / 56, 32 81 / 80, 37 90 / 115, 96 141 / 228; 96^3, N = 16 151 / 221.  Their expected
+//    time, a sum over runs and planes (build_box), against 5 + M (0.11 + 0.0063 N) / 1000, which is within a fifth of two products on up to 64^3 points.
+//    So have runs over its whole 7-point stencil (us, its runs / two products / the other runs): N = 64, 24^3 points 10.8 / 8.7, 32^3 10.9 / 11.2, 40^3 15.2 /
+//    17.9, 64^3 33 / 56 / 49, 96^3 107 / 279 / 181, 128^3 221 / 604 / 290; N = 128, 32^3 14.1 / 18.3, 64^3 56 / 128 / 97; 128^3, N = 32 123 / 338, 100 643 / 1,115; 90 x 70
+//    x 80, N = 36 66 / 88; against 4 + M (N, in whole lines from 32 on) 0.0034 / 1000.  Any N of a multiple of four.  That is what two products take while the Infinity
+//    Cache holds C and the intermediate and rows are whole half lines (64^3, N = 16 18 for 21, 32 33 for 34, 64 61 for 56), and a quarter to a third less than beyond it
+//    (128^3, N = 32 232 for 338, 64 460 for 604) or with rows across lines (64^3, N = 20 22 for 31): there some grids of fewer than 32 columns stay two
+//    products that the runs would take less for (128^3, N = 16 100 / 181, 64^3, N = 20 20 / 31), none the other way (96^3, N = 16 54 / 53).
+//    And over the 5-point stencil of a 2D grid whose lines no window holds: N = 64, 400 x 100 13.6 / 12.7, 300^2 19.0 / 22.4 / 28.4, 500^2 34 / 50 / 44, 1024 x 200
+//    28 / 42 / 44, 700^2 52 / 138 / 90, 1000^2 118 / 292 / 162; 250^2, N = 48 15.5 / 15.5, 600 x 500, N = 36 37 / 55; 1000^2, N = 16 51 / 55, 20 51 / 96.
 //
 // GeMM-SpMM:
 //  * as (A B) C in one launch (spmm_gemm_kernel) where no row has its sum from several workgroups and K is narrow.  Under 24,000

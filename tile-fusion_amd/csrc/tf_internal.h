@@ -121,6 +121,7 @@ constexpr int star_lds(int by) { return kStarLine * (2 * ((by + 4) + (by + 2)) +
 // ... and over the 5-point stencil of a 2D grid, which is its one with a line for a plane: columns of up to 94 points of a line.
 constexpr int kFlatX = 94, kFlatBlock = (kFlatX + 2) / 2 * 8, kFlatLine = (kFlatX + 6) * 128, kFlatRuns = 2;  // runs a compute unit holds
 constexpr int flat_lds() { return kFlatLine * 4; }
+// What either kernel of such runs is launched with.
 struct BoxArgs {
   int star = 0;  // the 7-point (ny = 1: 5-point) stencil instead of the 27-point one
   int nx = 0, ny = 0, nz = 0, N = 0;

@@ -85,13 +85,14 @@ struct StarPlace {
 // intermediate of the planes z - 1, z, z + 1 of C, and plane z - 1 of D likewise, while plane z + 1 of C goes to LDS and planes z + 2 and
 // z + 3 are on their way to registers; one barrier a step.  The points around those of the intermediate pass through a register to LDS.
 // No lists: a row's place among the values follows from its point; where A and B are one matrix a row's values are kept from the step that makes the
-// intermediate to the one that makes D (128^3 points, N = 64: 230 us, 254 with a load for each).  Bound: HBM, at the rate of a copy for C, D and the values
-// (235 us at 5.1 TB/s; gathering runs over lists 290, two products 619); on 64^3 points, N = 64, 34 us (49, 59), the steps themselves, 1.4 us each.
+// intermediate to the one that makes D (128^3 points, N = 64: 221 us, 250 with a load for each).  Bound: HBM, 1.26 GB at 5.7 TB/s, more than a plain copy's 5.0
+// (gathering runs over lists 290, two products 604; the clocks that launches in close order leave make it 260); on 64^3 points, N = 64, 33 us (49, 56), the steps
+// themselves, 1.4 us each.
 // 16 by 8 points of 32 columns: the intermediate 1.4 times and C's planes 1.8 times the column, where 8 by 8 of 64 columns are 1.5 and 2.1, in
 // as much of LDS.  Each sum is made in the order of the row's entries, so results carry
 // the reference's bits; what is outside the grid is zero, with zeros for values.
 // FLAT: a 2D grid, its lines for planes; a column is up to 94 points of a line, and two workgroups share a compute unit.  (1000 x 1000 points, us, here / as
-// two products: N = 64 120 / 310, 100 259 / 537, 128 236 / 576; 900 x 900, N = 32 46 / 90.)
+// two products: N = 64 118 / 292, 100 259 / 522, 128 222 / 556; 900 x 900, N = 32 45 / 82.)
 // LDS rows of 128 bytes: two lane groups of a read, two points apart, would meet in the same banks; rows 2 and 3 of every four change places.
 template <bool ACC, bool SAME, bool FLAT>
 __global__ __launch_bounds__(FLAT ? kFlatBlock : kStarBlock, 3) void fused_star_kernel(const BoxArgs a) {
@@ -233,7 +234,8 @@ hipError_t launch_fused_star(BoxArgs a, int accumulate, hipStream_t st) {
   if (a.by < 1 || a.by > kStarMaxY || a.bx < 1 || a.bx > (flat ? kFlatX : kStarX) || a.N % 4 != 0 || a.n_runs <= 0) return hipErrorInvalidValue;
   a.per_xcd = per_xcd_of(a.n_runs);
   // Streaming stores but where strips share lines of a D that the Infinity Cache does not hold, which would go to memory in parts (us, streaming / plain:
-  // N = 100, 128^3 points 719 / 642, 1000 x 1000 302 / 259, 64^3 63.1 / 61.8; N = 84, 96^3 201 / 206; N = 48, 64^3 34.4 / 35.7; whole lines, 128^3, N = 64 254 / 262).
+  // N = 100, 128^3 points 718 / 642, 1000 x 1000 302 / 259, 64^3 55.5 / 56.7; N = 84, 96^3 201 / 204; N = 48, 64^3 32.0 / 33.3; whole lines, N = 64, 128^3 220 / 229, 96^3
+  // 107 / 121, 1000 x 1000 118 / 120.  On the wrong side by 3 and 4 %: 128^3, N = 48 241 / 249, N = 32 122 / 117).
   a.streaming = a.N % 32 == 0 || (long long)a.nx * a.ny * a.nz * a.N * 4 <= (320ll << 20);
   const dim3 grid(grid_of(a.n_runs));
 #define CALL(ACC_, SAME_, FLAT_)                                                                                                                             \
