@@ -1,8 +1,10 @@
 // Rules of dispatch, checked on the host: which lane of which workgroup stores which column, what fits LDS.  Compiled with the host
 // sources by tests/test_host_rules.py; each argument names a check; exits 0 when all of them hold.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <vector>
 #include "tf_internal.h"
 #include "tf_rows.h"
@@ -251,31 +253,35 @@ static int streamed_entries() {
 }
 
 // Graphs whose reads are spread alike take the sweep, in one product as in two; one column that is read 255 times or more and they do not, whatever
-// a byte makes of its count.
+// a byte makes of its count.  Nor do rows whose columns are in no order, or fall.
 static int even_reads() {
   int bad = 0;
   const int M = 60000, mean = 11;
-  for (int often : {0, 254, 255, 256, 257, 300, 512, 767, 1024, 60000}) {
-    std::vector<int> p(1, 0), i;
-    unsigned long long at = 1;
-    for (int r = 0; r < M; ++r) {
-      for (int k = 0; k < mean; ++k) {
-        at = at * 6364136223846793005ull + 1442695040888963407ull;
-        i.push_back(1 + (int)((at >> 33) % (M - 1)));
+  for (int order = 0; order < 3; ++order)
+    for (int often : {0, 254, 255, 256, 257, 300, 512, 767, 1024, 60000}) {
+      std::vector<int> p(1, 0), i;
+      unsigned long long at = 1;
+      for (int r = 0; r < M; ++r) {
+        for (int k = 0; k < mean; ++k) {
+          at = at * 6364136223846793005ull + 1442695040888963407ull;
+          i.push_back(1 + (int)((at >> 33) % (M - 1)));
+        }
+        if (r < often) i.push_back(0);
+        if (order == 0) std::sort(i.begin() + p.back(), i.end());
+        if (order == 1) std::sort(i.begin() + p.back(), i.end(), std::greater<int>());
+        p.push_back((int)i.size());
       }
-      if (r < often) i.push_back(0);
-      p.push_back((int)i.size());
+      const bool sweeps = often < 255 && order == 0;
+      tf_inspect_opts o{};
+      o.struct_size = sizeof(o);
+      o.op = TF_OP_SPMM_SPMM;
+      o.N = 64;
+      tf_schedule *s = nullptr, *rows = nullptr;
+      if (tf_inspect(M, M, p.data(), i.data(), &o, &s) || tf_inspect_spmm(M, M, p.data(), i.data(), 64, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
+      if (!s->two_passes || s->two_passes->rem_sweep != sweeps || rows->rem_sweep != sweeps) { printf("order %d, a column read %d times\n", order, often); ++bad; }
+      tf_schedule_free(s);
+      tf_schedule_free(rows);
     }
-    tf_inspect_opts o{};
-    o.struct_size = sizeof(o);
-    o.op = TF_OP_SPMM_SPMM;
-    o.N = 64;
-    tf_schedule *s = nullptr, *rows = nullptr;
-    if (tf_inspect(M, M, p.data(), i.data(), &o, &s) || tf_inspect_spmm(M, M, p.data(), i.data(), 64, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
-    if (!s->two_passes || s->two_passes->rem_sweep != (often < 255) || rows->rem_sweep != (often < 255)) { printf("a column read %d times\n", often); ++bad; }
-    tf_schedule_free(s);
-    tf_schedule_free(rows);
-  }
   return bad;
 }
 

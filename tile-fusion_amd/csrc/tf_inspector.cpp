@@ -672,14 +672,18 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
     // inside a group), and a group is worked on, like a short row, by the XCD of its partition;
     // entries outside all partitions ("cold") go to all XCDs as before.  Groups are cut into
     // segments of at most 64 entries; a row's segments are added up in a fixed order.
+    size_t looked = 0, unordered = 0;  // of the rows that are looked at, those whose columns do not rise
     auto scattered = [&] {  // (some 8,192 rows are looked at)
       const size_t n = S->rem_rows.size(), step = n / 8192 + 1;
       double far = 0;
       long long entries = 0;
+      looked = unordered = 0;
       for (size_t q = 0; q < n; q += step) {
         const int i = S->rem_rows[q];
         for (int k = Ap[i]; k < Ap[i + 1]; ++k) far += std::abs(Ai[k] - (double)i * M / L);
         entries += Ap[i + 1] - Ap[i];
+        ++looked;
+        unordered += !std::is_sorted(Ai + Ap[i], Ai + Ap[i + 1]);
       }
       return far * 8 > (double)M * entries;
     };
@@ -692,7 +696,9 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
         return false;
       for (const auto &lr : S->long_rows)
         if (Ap[lr.row + 1] - Ap[lr.row] > kWholeRowMax) return false;
-      if (!scattered()) return false;
+      // Rows in no order wait with nearly all of their entries for the limit's last step (two products, in the other kernel / in this one / rows that rise: 100,000 rows of 11,
+      // N = 64, 79 / 98 / 68, 50,001 of 13, N = 100, 78 / 110 / 71, 160,000 of 17, N = 32, 101 / 119 / 77).
+      if (!scattered() || unordered * 64 > looked) return false;
       // The most-read eighth of the columns takes less than a quarter of the reads, and none 255 or more: summed up from the most-read ones down.  (Once for a
       // schedule and its two products, whose rows are all counted above: 50,000 rows of 13 would take 0.8 of 6 ms for each.)
       if (S->reads_even < 0) {
