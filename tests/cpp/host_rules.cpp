@@ -285,6 +285,37 @@ static int even_reads() {
   return bad;
 }
 
+// Far from the diagonal is not spread: rows that read where their neighbours in the order do, in blocks elsewhere, along another diagonal or in a part of their
+// entries, have what a sweep would bring together.
+static int rows_with_neighbours() {
+  int bad = 0;
+  const int M = 60000, mean = 11;
+  unsigned long long at = 1;
+  auto any = [&](int n) {
+    at = at * 6364136223846793005ull + 1442695040888963407ull;
+    return (int)((at >> 33) % n);
+  };
+  struct Kind { const char *name; int local, block, fields; bool sweep; };  // of 100 entries so many near the diagonal, blocks so large elsewhere, fields
+  for (const Kind &kind : {Kind{"any", 0, M, 0, true}, Kind{"a quarter near", 25, M, 0, true}, Kind{"two thirds near", 67, M, 0, false}, Kind{"blocks of a sixth", 0, M / 6, 0, false},
+                           Kind{"halves", 0, M / 2, 0, false}, Kind{"half near", 50, M, 0, true},
+                           Kind{"blocks of 200", 0, 200, 0, false}, Kind{"two fields", 0, M, 2, false}, Kind{"three fields", 0, M, 3, false}}) {
+    std::vector<int> p(1, 0), i;
+    for (int r = 0; r < M; ++r) {
+      const int base = (r / kind.block + M / kind.block / 2) % (M / kind.block) * kind.block;
+      for (int k = 0; k < mean; ++k)
+        i.push_back(kind.fields ? (r + M / kind.fields * (k % kind.fields) + k / kind.fields * 3) % M
+                    : any(100) < kind.local ? std::min(M - 1, std::max(0, r + any(33) - 16)) : base + any(kind.block));
+      std::sort(i.begin() + p.back(), i.end());
+      p.push_back((int)i.size());
+    }
+    tf_schedule *rows = nullptr;
+    if (tf_inspect_spmm(M, M, p.data(), i.data(), 64, 0, &rows)) { printf("%s\n", tf::g_err); return 1; }
+    if (rows->rem_sweep != kind.sweep) { printf("%s\n", kind.name); ++bad; }
+    tf_schedule_free(rows);
+  }
+  return bad;
+}
+
 int main(int argc, char **argv) {
   int bad = 0;
   for (int k = 1; k < argc; ++k) {
@@ -292,7 +323,8 @@ int main(int argc, char **argv) {
                   : !strcmp(argv[k], "partial_sums") ? partial_sums()
                   : !strcmp(argv[k], "hubs_and_columns") ? hubs_and_columns()
                   : !strcmp(argv[k], "streamed_entries") ? streamed_entries()
-                  : !strcmp(argv[k], "even_reads") ? even_reads() : 1;
+                  : !strcmp(argv[k], "even_reads") ? even_reads()
+                  : !strcmp(argv[k], "rows_with_neighbours") ? rows_with_neighbours() : 1;
     printf("%s: bad %d\n", argv[k], b);
     bad += b;
   }

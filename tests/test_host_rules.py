@@ -24,7 +24,7 @@ def host_rules(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["column_owners", "sweep_columns", "one_launch_fits", "partial_sums", "hubs_and_columns", "streamed_entries", "even_reads"])
+@pytest.mark.parametrize("check", ["column_owners", "sweep_columns", "one_launch_fits", "partial_sums", "hubs_and_columns", "streamed_entries", "even_reads", "rows_with_neighbours"])
 def test_rule(host_rules, check):
     r = subprocess.run([host_rules, check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout[-3000:]

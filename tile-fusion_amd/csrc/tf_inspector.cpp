@@ -699,6 +699,28 @@ static tf_status inspect(int L, int M, const int *Ap, const int *Ai, const tf_in
       // Rows in no order wait with nearly all of their entries for the limit's last step (two products, in the other kernel / in this one / rows that rise: 100,000 rows of 11,
       // N = 64, 79 / 98 / 68, 50,001 of 13, N = 100, 78 / 110 / 71, 160,000 of 17, N = 32, 101 / 119 / 77).
       if (!scattered() || unordered * 64 > looked) return false;
+      // Nor does it pay where rows in flight read the same part of X anyway, far from the diagonal as it may be: where three fifths of a row's columns have one of the row
+      // before it nearby, within an eighth of the distance between a row's columns, or a row's columns reach over less than three quarters of what columns drawn from all of X
+      // do.  Two products of rows of 11, us, in the other kernel / this one: blocks of 200 columns elsewhere (all nearby), 100,000 rows, N = 64 53 / 57, 128 70 / 102, of
+      // 20,000 (0.72) 57 / 63 and 81 / 112; two fields of a 300 x 300 grid's 5 points, N = 32 53 / 57, 64 99 / 103; of columns spread over all a share near the diagonal,
+      // 0.65 (0.66), 100,000 rows 52 / 59 and 96 / 109; a half (0.55), 61 / 60 and 113 / 114, 160,000 rows, N = 32 50 / 47, 128 222 / 175; a quarter (0.38), 100,000 rows 74 / 63 and
+      // 138 / 122.  The two halves of a bipartite graph (0.40, reach 0.5), N = 64 71 / 65, 100 130 / 142, 128 117 / 132.
+      {
+        const size_t n = S->rem_rows.size(), step = n / 1024 + 1;
+        long long nearby = 0, entries = 0;
+        double reach = 0, rows = 0;
+        for (size_t q = 0; q + 1 < n; q += step) {
+          const int *before = Ai + Ap[S->rem_rows[q]], *end = Ai + Ap[S->rem_rows[q] + 1], *from = Ai + Ap[S->rem_rows[q + 1]], *to = Ai + Ap[S->rem_rows[q + 1] + 1];
+          const long long apart = M / (4 * (end - before) + 1);
+          if (end - before > 1) {
+            const auto least_most = std::minmax_element(before, end);
+            reach += ((double)*least_most.second - *least_most.first) * (end - before + 1) / (end - before - 1);
+            rows += 1;
+          }
+          for (; from != to; ++from, ++entries) nearby += std::any_of(before, end, [&](int c) { return std::abs((long long)c - *from) * 2 <= apart; });
+        }
+        if (5 * nearby > 3 * entries || 4 * reach < 3 * rows * M) return false;
+      }
       // The most-read eighth of the columns takes less than a quarter of the reads, and none 255 or more: summed up from the most-read ones down.  (Once for a
       // schedule and its two products, whose rows are all counted above: 50,000 rows of 13 would take 0.8 of 6 ms for each.)
       if (S->reads_even < 0) {
